@@ -274,8 +274,8 @@ __device__ __forceinline__ bool wave_product_tiles(floatx4 (&acc)[2][NT], const 
                                                    const half8* wlds, const half_t* a0, const half_t* a1, int wave,
                                                    int lane, int nks_total, int ks_wave, int rotation, const Poll& poll,
                                                    Prefetch&& prefetch) {
-    static_assert(KS % 8 == 0, "whole chunks");
-    constexpr int CKT = CKO ? CKO : ((KS >= 16) ? 8 : 4);
+    constexpr int CKT = CKO ? CKO : ((KS >= 16) ? 8 : (KS >= 8) ? 4 : 2);
+    static_assert(KS % CKT == 0, "whole chunks");
     constexpr int NCHK = KS / CKT;      // chunks per tile
     constexpr int NCH = 2 * NCHK;
     static_assert(NBUF >= 2 && NBUF <= NCH, "register sets: one feeds the MFMAs, the others are in flight");
@@ -407,7 +407,7 @@ __device__ __forceinline__ bool wave_product(floatx4 (&acc)[2][NT], const half8 
                                              const half8* wlds, const half8* wfrag_wave, const half_t* a0,
                                              const half_t* a1, int wave, int lane, int nks_total,
                                              int ks_wave, int rotation, const Poll& poll, Prefetch&& prefetch) {
-    if constexpr (RESIDENT && (KS % 4 == 0)) {
+    if constexpr (RESIDENT) {
         // Loads and MFMAs are unconditional: k-steps beyond the real contraction length fetch a
         // clamped (finite) address and meet all-zero weight fragments.  Chunks of CK k-steps (2*CK
         // fragments) alternate between two register sets: one is in flight while the other feeds the
@@ -416,6 +416,7 @@ __device__ __forceinline__ bool wave_product(floatx4 (&acc)[2][NT], const half8 
         // kernel that waits on a trip through memory takes more, of shorter chunks (CKO) where registers are short:
         // five sets of 2 k-steps keep as much in flight as three sets of 4 and take 5/6 of the registers).
         constexpr int CK = CKO ? CKO : ((KS >= 16) ? 4 : 2);
+        static_assert(KS % CK == 0, "whole chunks");
         constexpr int NCH = KS / CK;
         constexpr int D = NBUF - 1;   // chunks requested ahead of the one being multiplied
         half8 fa[NBUF][CK], fb[NBUF][CK];
@@ -859,7 +860,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
     constexpr int JB = 4 * NT;    // hidden units of this slice
     constexpr int NC = 16 * NT;   // gate columns of this slice (i,f,g,o blocks of JB)
     constexpr int PLD = NC + kPartPad;
-    constexpr bool SPLIT = RESIDENT && MT == 2 && JB >= 32 && (KS % 8 == 0);
+    constexpr bool SPLIT = RESIDENT && MT == 2 && JB >= 32;
     // cell updates per thread: the slice's units of one batch row are shared by GPR threads; 32 rows x 8 threads,
     // or 16 rows x 16 threads (per phase, or when a block has one row tile) where the slice is wide enough for 2 units each
     constexpr int GPR = (SPLIT || (MT == 1 && JB >= 32)) ? 16 : 8;
@@ -948,7 +949,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
                 ahead = wave_product_tiles<NT, KS, 0, NPH * UPT / 2, kFwdBufs, false, 0, DS>(acc, wreg, nullptr, a0, a1, wave, lane, nks_total, ks_wave, rotation, poll,
                                                              [&]() { prefetch(t, rb); });
             else
-                ahead = wave_product<NT, KS, RESIDENT, 0, UPT / 2, MT, DEEP ? 4 : 2, DEEP ? 2 : 0, DEEP, DS && !DEEP>(acc, wreg, nullptr, wfrag_wave, a0, a1, wave, lane, nks_total,
+                ahead = wave_product<NT, KS, RESIDENT, 0, UPT / 2, MT, DEEP ? 4 : 2, DEEP ? 2 : (KS == 12) ? 4 : 0, DEEP, DS && !DEEP>(acc, wreg, nullptr, wfrag_wave, a0, a1, wave, lane, nks_total,
                                                                ks_wave, rotation, poll, [&]() { prefetch(t, rb); });
             if constexpr (DS) first_request.learn(ahead);
             clk.lap(0);
@@ -1085,7 +1086,7 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
     constexpr int JB = 4 * NT;
     constexpr int NC = 16 * NT;
     constexpr int PLD = NC + kPartPad;
-    static_assert(JB == 32 && KS == 4, "slices of 32 units; four k-steps per wave");
+    static_assert(JB == 32 && (KS == 2 || KS == 4), "slices of 32 units; a register set per k-step");
     extern __shared__ __attribute__((aligned(16))) float part_all[];  // [2][NW][16][PLD]
     __shared__ int lds_abort;
     __shared__ int lds_role[2];
@@ -1346,7 +1347,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
     // dG_t, then rows 16..31, and fetch and multiply tile by tile, so the second half of a step's cell updates and its
     // cache stores run while the peers are already in the first half of their next product (measured at 1024 units
     // and 256 rows: 4.85 -> 4.5 us per step; without waiting for producers at all the step takes 4.2).
-    constexpr bool SPLIT = RESIDENT && MT == 2 && JB >= 32 && (KS % 8 == 0);
+    constexpr bool SPLIT = RESIDENT && MT == 2 && JB >= 32;
     constexpr int GPR = (SPLIT || (MT == 1 && JB >= 32)) ? 16 : 8;   // threads per batch row (as in the forward kernel)
     constexpr int UPT = JB / GPR;
     constexpr int NPH = SPLIT ? 2 : 1;   // pointwise phases per step
@@ -1453,7 +1454,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
                     ahead = wave_product_tiles<NT, KS, KL, NPF, 4, false, 4, DS>(acc, wreg, wlds, a0, a1, wave, lane, nks_total, ks_wave, rotation, poll,
                                                            [&]() { prefetch(t, rb); });
                 else
-                    ahead = wave_product<NT, KS, RESIDENT, KL, NPF, MT, 2, 0, false, DS>(acc, wreg, wlds, wfrag_wave, a0, a1, wave, lane, nks_total,
+                    ahead = wave_product<NT, KS, RESIDENT, KL, NPF, MT, 2, (KS == 8) ? 4 : 0, false, DS>(acc, wreg, wlds, wfrag_wave, a0, a1, wave, lane, nks_total,
                                                               ks_wave, rotation, poll, [&]() { prefetch(t, rb); });
                 if constexpr (DS) first_request.learn(ahead);
                 clk.lap(0);
@@ -2324,10 +2325,10 @@ static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
                         });
 }
 
-template <bool DS>
+template <int KS, bool DS>
 static hipError_t run_fwd_il(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     constexpr int NT = 8, NW = 8;
-    auto kernel = rec_fwd_il_kernel<NT, 4, DS>;
+    auto kernel = rec_fwd_il_kernel<NT, KS, DS>;
     if (L.nw != NW || L.nt != NT || L.mt != 2 || !L.resident) return hipErrorInvalidValue;
     const size_t lds = size_t(2) * NW * 16 * (16 * NT + kPartPad) * sizeof(float);
     hipError_t e = raise_lds(kernel, lds);
@@ -2345,23 +2346,42 @@ static hipError_t run_fwd_il(const RecLayout& L, const RecFwdArgs& a, hipStream_
                         });
 }
 
+template <int NT, int KS, int MT>
+static hipError_t run_fwd_ds(const RecLayout& L, const RecFwdArgs& a, bool ds, hipStream_t stream, StepGraphCache* graphs) {
+    return ds ? run_fwd<NT, KS, true, MT, true>(L, a, stream, graphs) : run_fwd<NT, KS, true, MT, false>(L, a, stream, graphs);
+}
+
 hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     if (a.T <= 0 || a.B <= 0 || a.t1 <= a.t0) return hipSuccess;
     if (a.Hp % 32 != 0 || a.Hp % L.jb != 0 || a.t0 < 0 || a.t1 > a.T) return hipErrorInvalidValue;
     // device-scope stores into the exchange ring: a persistent launch whose groups span XCDs
     const bool ds = L.persistent && !L.xcd_local;
     if (!L.resident) return run_fwd<8, 1, false, 2, false>(L, a, stream, graphs);
-    if (L.nw == 8)   // eight waves: the interleaved kernel, 32-row blocks
-        return ds ? run_fwd_il<true>(L, a, stream, graphs) : run_fwd_il<false>(L, a, stream, graphs);
+    const int ks = rec_fwd_ks(L, a.Hp);
+    if (L.nw == 8) {   // eight waves: the interleaved kernel, 32-row blocks
+        if (ks <= 2) return ds ? run_fwd_il<2, true>(L, a, stream, graphs) : run_fwd_il<2, false>(L, a, stream, graphs);
+        return ds ? run_fwd_il<4, true>(L, a, stream, graphs) : run_fwd_il<4, false>(L, a, stream, graphs);
+    }
     if (L.nt == 8) {
-        if (L.mt == 1) return ds ? run_fwd<8, 8, true, 1, true>(L, a, stream, graphs) : run_fwd<8, 8, true, 1, false>(L, a, stream, graphs);
-        return ds ? run_fwd<8, 8, true, 2, true>(L, a, stream, graphs) : run_fwd<8, 8, true, 2, false>(L, a, stream, graphs);
+        // A kernel is unrolled for KS k-steps per wave and multiplies all of them, the ones past the contraction by zero
+        // weights: one built for 1024 units spends the same time per step at 256.  So there is one per 256 units (with
+        // two row tiles, where the product is the smaller part, per 512).  Measured, us per step, forward / backward, one kernel for all
+        // -> this: 256 units and 8 rows 1.76 / 2.44 -> 1.50 / 1.82, 512 and 64 rows 1.84 / 2.90 -> 1.64 / 2.16, 672
+        // and 20 rows 1.91 / 2.97 -> 1.74 / 2.54, 1536 and 48 rows 3.18 / 6.74 -> 2.90 / 5.73.
+        if (L.mt == 1) {
+            if (ks <= 2) return run_fwd_ds<8, 2, 1>(L, a, ds, stream, graphs);
+            if (ks <= 4) return run_fwd_ds<8, 4, 1>(L, a, ds, stream, graphs);
+            if (ks <= 6) return run_fwd_ds<8, 6, 1>(L, a, ds, stream, graphs);
+            return run_fwd_ds<8, 8, 1>(L, a, ds, stream, graphs);
+        }
+        if (ks <= 4) return run_fwd_ds<8, 4, 2>(L, a, ds, stream, graphs);
+        return run_fwd_ds<8, 8, 2>(L, a, ds, stream, graphs);
     }
     if (L.nt == 4) {
-        if (L.mt == 1) return ds ? run_fwd<4, 16, true, 1, true>(L, a, stream, graphs) : run_fwd<4, 16, true, 1, false>(L, a, stream, graphs);
-        if (!ds) return run_fwd<4, 16, true, 2, false>(L, a, stream, graphs);
-        const bool several_blocks = L.nrb >= 2 * L.ng;   // every workgroup takes at least two row blocks per step
-        return several_blocks ? run_fwd<4, 16, true, 2, true, true>(L, a, stream, graphs) : run_fwd<4, 16, true, 2, true>(L, a, stream, graphs);
+        if (L.mt == 1) return ks <= 12 ? run_fwd_ds<4, 12, 1>(L, a, ds, stream, graphs) : run_fwd_ds<4, 16, 1>(L, a, ds, stream, graphs);
+        if (!ds || L.nrb < 2 * L.ng) return ks <= 12 ? run_fwd_ds<4, 12, 2>(L, a, ds, stream, graphs) : run_fwd_ds<4, 16, 2>(L, a, ds, stream, graphs);
+        // every workgroup takes at least two row blocks per step
+        return ks <= 12 ? run_fwd<4, 12, true, 2, true, true>(L, a, stream, graphs) : run_fwd<4, 16, true, 2, true, true>(L, a, stream, graphs);
     }
     return hipErrorInvalidValue;
 }
@@ -2386,6 +2406,11 @@ static hipError_t run_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
                             }
                             return hipSuccess;
                         });
+}
+
+template <int NT, int KS, int KL, int MT>
+static hipError_t run_bwd_ds(const RecLayout& L, const RecBwdArgs& a, bool ds, hipStream_t stream, StepGraphCache* graphs) {
+    return ds ? run_bwd<NT, KS, true, KL, MT, true>(L, a, stream, graphs) : run_bwd<NT, KS, true, KL, MT, false>(L, a, stream, graphs);
 }
 
 template <int MT, int KQ, int NM, int KS, bool LOCAL>
@@ -2425,13 +2450,20 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
     }
     const bool ds = L.persistent && !L.xcd_local;   // (as in launch_rec_fwd)
     if (!L.resident) return run_bwd<2, 1, false, 0, 2, false>(L, a, stream, graphs);
+    const int ks = rec_bwd_ks(L, a.Hp);
     if (L.nt == 2) {
-        if (L.mt == 1) return ds ? run_bwd<2, 32, true, 8, 1, true>(L, a, stream, graphs) : run_bwd<2, 32, true, 8, 1, false>(L, a, stream, graphs);
-        return ds ? run_bwd<2, 32, true, 8, 2, true>(L, a, stream, graphs) : run_bwd<2, 32, true, 8, 2, false>(L, a, stream, graphs);
+        if (L.mt == 1) {
+            if (ks <= 8) return run_bwd_ds<2, 8, 0, 1>(L, a, ds, stream, graphs);
+            if (ks <= 16) return run_bwd_ds<2, 16, 0, 1>(L, a, ds, stream, graphs);
+            if (ks <= 24) return run_bwd_ds<2, 24, 0, 1>(L, a, ds, stream, graphs);
+            return run_bwd_ds<2, 32, 8, 1>(L, a, ds, stream, graphs);
+        }
+        if (ks <= 16) return run_bwd_ds<2, 16, 0, 2>(L, a, ds, stream, graphs);
+        return run_bwd_ds<2, 32, 8, 2>(L, a, ds, stream, graphs);
     }
     if (L.nt == 1) {
-        if (L.mt == 1) return ds ? run_bwd<1, 64, true, 24, 1, true>(L, a, stream, graphs) : run_bwd<1, 64, true, 24, 1, false>(L, a, stream, graphs);
-        return ds ? run_bwd<1, 64, true, 24, 2, true>(L, a, stream, graphs) : run_bwd<1, 64, true, 24, 2, false>(L, a, stream, graphs);
+        if (L.mt == 1) return ks <= 48 ? run_bwd_ds<1, 48, 12, 1>(L, a, ds, stream, graphs) : run_bwd_ds<1, 64, 24, 1>(L, a, ds, stream, graphs);
+        return ks <= 48 ? run_bwd_ds<1, 48, 12, 2>(L, a, ds, stream, graphs) : run_bwd_ds<1, 64, 24, 2>(L, a, ds, stream, graphs);
     }
     return hipErrorInvalidValue;
 }

@@ -1,0 +1,21 @@
+"""Kernels and launch choices that a rule picks by size, each at the sizes where the rule or the kernel could go wrong
+(both sides of a boundary, remainders, the smallest and the largest of a range), against the CPU oracle."""
+import pytest
+
+from helpers import check_against, make_problem
+from test_core_gpu import oracle_reference, run_core
+
+pytestmark = pytest.mark.gpu
+
+
+# hidden sizes on both sides of every step of the contraction the recurrence kernels are built for; the batch decides
+# between 16-row blocks (few rows), 32-row blocks (200 rows of 513 units) and the eight-wave kernel (300 rows of 512)
+@pytest.mark.parametrize("B,H", [(3, 128), (17, 256), (5, 257), (40, 512), (300, 512), (200, 513), (9, 700), (33, 769), (2, 1024),
+                                 (20, 1100), (40, 1536), (7, 1537)])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_recurrence_kernels_by_contraction_length(B, H, stepwise):
+    p = make_problem(5, B, 24, H, seed=B * 10000 + H)
+    ref, _ = oracle_reference(p)
+    got, info = run_core(p, stepwise=stepwise)
+    assert info["fallbacks"] == 0
+    check_against(ref, got, label=f"B={B} H={H} stepwise={stepwise}")
