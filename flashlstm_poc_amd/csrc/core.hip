@@ -781,12 +781,11 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, floa
     const half_t* Hop = p->Y.as<half_t>();
     const int n_ih = dW_ih ? d.Ip : 0, n_hh = dW_hh ? d.Hp : 0, ncols = n_ih + n_hh;
     if (ncols > 0) {
-        // automatic: what the kernel's own schedule makes fastest (gemm_tn_auto_splits), at least four 64-row slabs
-        // per split
+        // automatic: what the kernels' schedules make fastest (gemm_tn_plan_splits), at least two 64-row slabs per split
         int want = p->opt_dw_splits > 0 ? p->opt_dw_splits : p->eff_dw;
         if (want <= 0) {
-            const size_t cap = TB / 256 < 64 ? TB / 256 : 64;
-            want = gemm_tn_auto_splits(4 * d.Hp, n_ih ? n_ih : n_hh, n_ih ? n_hh : 0, int(TB), cap < 1 ? 1 : int(cap));
+            const size_t cap = TB / 128 < 64 ? TB / 128 : 64;
+            want = gemm_tn_plan_splits(4 * d.Hp, n_ih ? n_ih : n_hh, n_ih ? n_hh : 0, int(TB), cap < 1 ? 1 : int(cap));
         }
         if (want > 64) want = 64;
         const int splits = gemm_effective_splits(int(TB), want);
@@ -1151,8 +1150,8 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
     // 2) split-K count of the weight-gradient GEMM around what the schedule model picks
     p->opt_stepwise = best.step_f && best.step_b; p->opt_mt_f = best.mt_f; p->opt_mt_b = best.mt_b;
     replan(p);
-    const size_t cap = TB / 256 < 64 ? TB / 256 : 64;
-    const int rule = gemm_tn_auto_splits(4 * d.Hp, d.Ip, d.Hp, int(TB), cap < 1 ? 1 : int(cap));
+    const size_t cap = TB / 128 < 64 ? TB / 128 : 64;
+    const int rule = gemm_tn_plan_splits(4 * d.Hp, d.Ip, d.Hp, int(TB), cap < 1 ? 1 : int(cap));
     int last_eff = -1;
     for (int cand : {rule / 2, rule, rule + 1, rule * 2, rule * 4}) {
         if (cand < 1 || cand > 64) continue;

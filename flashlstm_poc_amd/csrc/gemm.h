@@ -36,4 +36,14 @@ int gemm_effective_splits(int K, int wanted);
 // side by side when N2 > 0), at most max_splits.
 int gemm_tn_auto_splits(int M, int N1, int N2, int K, int max_splits);
 
+// The kernels for products that do not fill the chip with 256 x 256 tiles (gemm_tile.hip): the tile size the launchers
+// above take for a product (64, 128 or 256), and the split count for it (a TN product with fp32 partials).
+int gemm_nt_tile_size(int M, int N, int K);
+int gemm_tn_tile_size(int M, int N1, int N2, int K, int splits);
+int gemm_tn_plan_splits(int M, int N1, int N2, int K, int max_splits);
+hipError_t launch_gemm_nt_tile(const GemmNT& g, int tile, hipStream_t stream);
+hipError_t launch_gemm_tn_tile(const GemmNT& g, int tile, int splits, int slabs_per_split, hipStream_t stream);
+// blocks of 32 tiles of 256 x 256 that the large kernels deal to the XCDs for an M x (N1 + N2) product
+long gemm_blocks_of_32(int M, int N1, int N2);
+
 }  // namespace flstm_hip

@@ -683,6 +683,10 @@ hipError_t launch_gemm_nt(const GemmNT& g, hipStream_t stream) {
         // ones must read as zero.  Callers use gemm_effective_splits() to avoid this path.
         return hipErrorInvalidValue;
     }
+    if (splits == 1) {
+        const int tile = gemm_nt_tile_size(g.M, g.N, g.K);
+        if (tile != BM) return launch_gemm_nt_tile(g, tile, stream);
+    }
     const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
     const TileOrder order = make_order(tiles_m, tiles_n, splits);
     // (set before every launch: the call is cheap, needs no process-wide flag and holds for whichever device is current)
@@ -709,18 +713,27 @@ hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream) {
     // (a copy addresses a slab's 64 k-rows with 32-bit byte offsets from the slab's first row)
     if (g.lda >= (size_t(1) << 22) || g.ldb >= (size_t(1) << 22) || (g.B2 && g.ldb2 >= (size_t(1) << 22)))
         return hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tn_stream),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(kLdsBytesStream));
-    if (e != hipSuccess) return e;
     const int nslab = (g.K + BK - 1) / BK;
     const int slabs_per_split = (nslab + splits - 1) / splits;
     if (g.B2 && (g.C32 == nullptr || g.N1 <= 0 || g.N1 >= g.N || g.N1 % 8 != 0 || g.ldb2 % 8 != 0)) return hipErrorInvalidValue;
+    if (g.C32) {
+        const int tile = gemm_tn_tile_size(g.M, g.B2 ? g.N1 : g.N, g.B2 ? g.N - g.N1 : 0, g.K, splits);
+        if (tile != BM) return launch_gemm_tn_tile(g, tile, splits, slabs_per_split, stream);
+    }
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tn_stream),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(kLdsBytesStream));
+    if (e != hipSuccess) return e;
     const int tiles_m = (g.M + BM - 1) / BM;
     const int tiles_n = g.B2 ? (g.N1 + BN - 1) / BN + (g.N - g.N1 + BN - 1) / BN : (g.N + BN - 1) / BN;
     const TileOrder order = make_order(tiles_m, tiles_n, splits);
     hipLaunchKernelGGL(gemm_tn_stream, dim3(256), dim3(kThreads), kLdsBytesStream, stream, g, order,
                        slabs_per_split);
     return hipGetLastError();
+}
+
+long gemm_blocks_of_32(int M, int N1, int N2) {
+    const TileOrder o = make_order((M + BM - 1) / BM, (N1 + BN - 1) / BN + (N2 > 0 ? (N2 + BN - 1) / BN : 0), 1);
+    return long(o.nsm) * o.nsn;
 }
 
 // Split count for a TN product with fp32 partials, from the way the kernel schedules it: blocks of 32 tiles x splits
