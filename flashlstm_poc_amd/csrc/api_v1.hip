@@ -19,7 +19,6 @@ namespace {
 struct V1Impl {
     lstm_compute_precision_t precision;
     size_t batch, input_size, hidden_size;
-    int proj_chunk;
     lstm_execution_mode_t mode;
     flstm_core_plan* plan;   // null when any dimension is zero
     hipStream_t stream;
@@ -42,6 +41,7 @@ extern "C" int lstm_create_buffers(lstm_compute_precision_t precision, size_t se
                                    size_t input_size, size_t hidden_size, int input_proj_chunk_size,
                                    lstm_buffers* buffers) {
     (void)seq_len;  // buffers are sized by the first forward and grow on demand
+    (void)input_proj_chunk_size;  // the projection is one product over the sequence (core.hip, forward_project)
     if (!buffers) return kInvalid;
     buffers->impl = nullptr;
     if (precision != LSTM_COMPUTE_PRECISION_FP16_ACC32 && precision != LSTM_COMPUTE_PRECISION_FP16_ACC16)
@@ -52,7 +52,6 @@ extern "C" int lstm_create_buffers(lstm_compute_precision_t precision, size_t se
     impl->batch = batch;
     impl->input_size = input_size;
     impl->hidden_size = hidden_size;
-    impl->proj_chunk = input_proj_chunk_size;
     impl->mode = LSTM_EXECUTION_MODE_IMMEDIATE;
     impl->plan = nullptr;
     impl->stream = nullptr;
@@ -62,7 +61,6 @@ extern "C" int lstm_create_buffers(lstm_compute_precision_t precision, size_t se
     if (!empty) {
         int rc = flstm_core_create(batch, input_size, hidden_size, &impl->plan);
         if (rc) { destroy_impl(impl); return rc; }
-        flstm_core_set_option(impl->plan, "proj_chunk", input_proj_chunk_size);
     }
     hipError_t e = hipStreamCreateWithFlags(&impl->stream, hipStreamNonBlocking);
     if (e != hipSuccess) { destroy_impl(impl); return int(e); }

@@ -477,9 +477,9 @@ size_t rebuild_start_state(Entry& e, const Streams& st, size_t j, size_t W, size
     check(hipMemcpyAsync(e.ck_c.p, static_cast<const char*>(cache.c_ptr) + k * BH * (c32 ? 4 : 2), BH * (c32 ? 4 : 2),
                          hipMemcpyHostToDevice, st.cs), "c checkpoint upload");
     if (h32) copy_state(static_cast<float*>(e.carry_h.p), e.ck_h.p, BH, st.cs);
-    else check(flstm_hip::unpad_from_half(static_cast<const half_t*>(e.ck_h.p), H, B, int(H), e.carry_h.p, 1, st.cs), "h checkpoint");
+    else check(flstm_hip::gather_from_half(static_cast<const half_t*>(e.ck_h.p), H, B, int(H), e.carry_h.p, 1, B, 0, st.cs), "h checkpoint");
     if (c32) copy_state(static_cast<float*>(e.carry_c.p), e.ck_c.p, BH, st.cs);
-    else check(flstm_hip::unpad_from_half(static_cast<const half_t*>(e.ck_c.p), H, B, int(H), e.carry_c.p, 1, st.cs), "c checkpoint");
+    else check(flstm_hip::gather_from_half(static_cast<const half_t*>(e.ck_c.p), H, B, int(H), e.carry_c.p, 1, B, 0, st.cs), "c checkpoint");
     size_t cur = t_ck;
     while (cur < target) {
         const size_t end = (cur / W + 1) * W < target ? (cur / W + 1) * W : target;   // stop at every window start

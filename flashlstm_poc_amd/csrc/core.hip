@@ -67,20 +67,17 @@ struct DevBuf {
     static DevBuf view(void* ptr, size_t n) { DevBuf b; b.p = ptr; b.bytes = n; b.borrowed = true; return b; }
 };
 
-struct PhaseTimer {
-    hipEvent_t ev[8] = {};
-    bool ok = false;
-    hipError_t init() {
-        for (auto& e : ev) { hipError_t r = hipEventCreate(&e); if (r != hipSuccess) return r; }
-        ok = true;
-        return hipSuccess;
-    }
-    void destroy() { if (ok) for (auto& e : ev) (void)hipEventDestroy(e); ok = false; }
-};
-
 }  // namespace
 
 constexpr int kFirstHold = 8, kMaxHold = 1024;
+
+// The plan's status block on the device: word 0 the status, words 1 and 2 the delay hints of the two recurrences, the
+// time stamps of a pass, and sets of seat counters: every recurrence launch needs eight zeroed ones, so a pass that
+// launches several (ranges of steps, windows of rows) takes the sets its setup has zeroed one after the other.
+constexpr size_t kStampsOffset = 64, kSeatsOffset = 256;
+constexpr int kSeatSets = 64;
+constexpr size_t kStatusBytes = kSeatsOffset + size_t(kSeatSets) * 8 * sizeof(unsigned);
+static_assert(kStampsOffset + kStampCount * sizeof(long long) <= kSeatsOffset, "stamps fit in front of the seats");
 
 struct flstm_core_plan {
     int device = 0;
@@ -90,7 +87,7 @@ struct flstm_core_plan {
     RecLayout Lf{}, Lb{};
     int ks_f = 0, ks_b = 0;
     // options
-    int opt_stepwise = 0, opt_proj_chunk = 0, opt_spin_limit = 1 << 30, opt_spin_ms = 250, opt_dw_splits = 0, opt_accumulate = 0;
+    int opt_stepwise = 0, opt_spin_limit = 1 << 30, opt_spin_ms = 250, opt_dw_splits = 0, opt_accumulate = 0;
     // A persistent launch that gave up (its workgroups were not all running at once, or not spread over the XCDs
     // as expected) demotes that direction to step-wise launches for `hold` passes; then the persistent kernel is
     // tried again.  Every further give-up doubles the hold (at most kMaxHold passes).
@@ -109,12 +106,13 @@ struct flstm_core_plan {
     int eff_mt_f = 0, eff_mt_b = 0, eff_step_f = 0, eff_step_b = 0, eff_dw = 0, eff_two_d = -1;
     bool two_d_explicit = false;   // option "bwd_two_d" (or its environment variable) was given: a tuned value does not replace it
     size_t eff_T = 0;
-    int opt_cooperative = 1;
+    int opt_cooperative = 0;
     StepGraphCache graphs_f, graphs_b;   // captured step-wise launches (only used where the persistent kernels are not)
     int opt_graphs = 1;
     int opt_two_d = 1;   // backward recurrence for 2048 hidden units, two-way split: 0 never, 1 where it is faster, 2 wherever it can run
     int opt_waves_f = 0;   // wavefronts per workgroup of the forward recurrence: 0 = by size, 4, 8 (the weights are packed for it)
-    int* status_host = nullptr;   // pinned: the device status word lands here with the end-of-pass copy
+    HostStatus* status_host = nullptr;   // pinned: the last launch of a pass leaves the status word and the stamps here
+    int seat_sets_left = 0;              // zeroed sets of seat counters in the status block
     int inject_stall = 0;         // test hook: treat the next N passes as if their launches had given up
     // weights
     DevBuf wih_p, wih_t, wfrag_f, wfrag_b, wfrag_b2, bias_p;
@@ -125,16 +123,13 @@ struct flstm_core_plan {
     bool have_cache = false;
     // pass in progress (begin / steps / end)
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
-             half_t* y_direct = nullptr; bool seats_clean = false; } fw;   // y_direct: the recurrence writes the caller's y itself
-    // (seats_clean: the pass's setup has zeroed the seat counters for the first recurrence launch that follows it)
+             half_t* y_direct = nullptr; } fw;   // y_direct: the recurrence writes the caller's y itself
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
-             float S = 1.f, dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false;
-             bool seats_clean = false; } bw;
+             float S = 1.f, dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
     // backward scratch
     DevBuf dYp, dG, dHn, dC, dH0, db_part, dw_part, prof, part_b;
     int opt_profile = 0, wall_khz = 100000;
     long long prof_f[8] = {}, prof_b[8] = {};
-    PhaseTimer tm;
     float ms_fwd[3] = {-1, -1, -1}, ms_bwd[4] = {-1, -1, -1, -1};
 };
 
@@ -176,28 +171,50 @@ void use_tuned(flstm_core_plan* p, size_t T) {
     }
 }
 
-// The status word of the recurrence kernels travels to pinned host memory behind the pass's last kernel, so the
-// wait that ends the pass anyway is also the one that makes it readable: no second round trip to the device.
-int enqueue_status_copy(flstm_core_plan* p, hipStream_t s) {
-    FL_TRY(hipMemcpyAsync(p->status_host, p->status.p, sizeof(int), hipMemcpyDeviceToHost, s));
+long long* stamps_of(const flstm_core_plan* p) { return reinterpret_cast<long long*>(p->status.as<char>() + kStampsOffset); }
+
+// The last launch of a pass: it leaves the status word of the recurrence kernels and the stamps in pinned host memory,
+// so the wait that ends the pass anyway is also the one that makes them readable: no second round trip to the device.
+int publish_with(flstm_core_plan* p, OpList& last, int stamp, hipStream_t s) {
+    last.status = p->status.as<int>();
+    last.stamps = stamps_of(p);
+    last.stamp = stamp;
+    last.publish = p->status_host;
+    FL_TRY(run_ops(last, s));
+    return 0;
+}
+int wait_stream(hipStream_t s) {
+    FL_TRY(hipStreamSynchronize(s));
+    persistent_stream_idle(s);
     return 0;
 }
 // after the stream has been waited for: the status of the pass; a non-zero one is cleared on the device
-int take_status(flstm_core_plan* p, bool fwd, hipStream_t s, int* out) {
-    *out = *static_cast<volatile int*>(p->status_host);
+int take_status(flstm_core_plan* p, hipStream_t s, int* out) {
+    *out = *static_cast<volatile int*>(&p->status_host->status);
     if (*out != 0) FL_TRY(fill_zero(p->status.p, sizeof(int), s));
-    (void)fwd;
     if (*out == 0 && p->inject_stall > 0) {   // (2 in a row: the step-wise repeat of a pass fails too, i.e. the call does)
         p->inject_stall--;
         *out = 1;
     }
     return 0;
 }
-int wait_status(flstm_core_plan* p, bool fwd, hipStream_t s, int* out) {
-    int rc = enqueue_status_copy(p, s);
+int wait_status(flstm_core_plan* p, OpList& last, int stamp, hipStream_t s, int* out) {
+    int rc = publish_with(p, last, stamp, s);
     if (rc) return rc;
-    FL_TRY(hipStreamSynchronize(s));
-    return take_status(p, fwd, s, out);
+    rc = wait_stream(s);
+    if (rc) return rc;
+    return take_status(p, s, out);
+}
+
+// Eight zeroed seat counters for the next recurrence launch.
+int next_seats(flstm_core_plan* p, unsigned** out, hipStream_t s) {
+    char* const first = p->status.as<char>() + kSeatsOffset;
+    if (p->seat_sets_left <= 0) {
+        FL_TRY(fill_zero(first, size_t(kSeatSets) * 8 * sizeof(unsigned), s));
+        p->seat_sets_left = kSeatSets;
+    }
+    *out = reinterpret_cast<unsigned*>(first) + size_t(--p->seat_sets_left) * 8;
+    return 0;
 }
 
 // A persistent launch gave up: step-wise launches for the next `hold` passes of that direction.
@@ -216,10 +233,10 @@ void pass_done(flstm_core_plan* p, bool fwd) {
     if (hold > 0 && --hold == 0) replan(p);
 }
 
-float elapsed(hipEvent_t a, hipEvent_t b) {
-    float ms = -1.f;
-    if (hipEventElapsedTime(&ms, a, b) != hipSuccess) return -1.f;
-    return ms;
+// milliseconds between two stamps of the pass that has just been waited for (-1: not both there)
+float elapsed(const flstm_core_plan* p, int from, int to) {
+    const long long a = p->status_host->stamps[from], b = p->status_host->stamps[to];
+    return (a > 0 && b >= a) ? float(double(b - a) / p->wall_khz) : -1.f;
 }
 
 }  // namespace
@@ -251,27 +268,20 @@ extern "C" int flstm_core_create(size_t batch, size_t input_size, size_t hidden_
     p->d.H = int(hidden_size);
     p->d.Ip = int(round_up(input_size, 64));
     p->d.Hp = int(round_up(hidden_size, 32));
-    // Persistent launches are cooperative launches (co-residency of the whole grid is then a condition of the launch
-    // instead of an assumption) -- except under a rocprofiler-sdk tool: with rocprofv3 attached, a process that has
-    // made a cooperative launch takes a segmentation fault inside the tool when it exits (results and traces are
-    // complete by then; seen with ROCm 7.2), so plain launches are used there.  FLASHLSTM_COOPERATIVE_LAUNCH=0/1
-    // or the option "cooperative" decides explicitly.
+    // Persistent launches go through the gate of launch_persistent; FLASHLSTM_COOPERATIVE_LAUNCH=1 or the option
+    // "cooperative" sends them through hipLaunchCooperativeKernel instead (not under a rocprofiler-sdk tool: with rocprofv3
+    // attached, a process that has made a cooperative launch takes a segmentation fault inside the tool when it exits).
     {
-        const char* preload = getenv("LD_PRELOAD");
-        const bool profiled = (preload && strstr(preload, "rocprofiler")) || getenv("ROCPROFILER_REGISTER_LIBRARY") ||
-                              getenv("ROCP_TOOL_LIBRARIES") || getenv("ROCPROF_OUTPUT_PATH");
-        p->opt_cooperative = profiled ? 0 : 1;
         if (const char* v = getenv("FLASHLSTM_COOPERATIVE_LAUNCH")) p->opt_cooperative = atoi(v) != 0;
         if (const char* v = getenv("FLASHLSTM_STEP_GRAPHS")) p->opt_graphs = atoi(v) != 0;
         if (const char* v = getenv("FLASHLSTM_BWD_TWO_D")) { p->opt_two_d = atoi(v) < 0 ? 0 : (atoi(v) > 2 ? 2 : atoi(v)); p->two_d_explicit = true; }
         if (const char* v = getenv("FLASHLSTM_WAVES_FWD")) p->opt_waves_f = (atoi(v) == 4 || atoi(v) == 8) ? atoi(v) : 0;
     }
     replan(p);
-    e = p->status.reserve(64);
-    if (e == hipSuccess) e = hipMemset(p->status.p, 0, 64);
-    if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&p->status_host), 64, hipHostMallocDefault);
-    if (e == hipSuccess) p->status_host[0] = 0;
-    if (e == hipSuccess) e = p->tm.init();
+    e = p->status.reserve(kStatusBytes);
+    if (e == hipSuccess) e = hipMemset(p->status.p, 0, kStatusBytes);
+    if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&p->status_host), sizeof(HostStatus), hipHostMallocDefault);
+    if (e == hipSuccess) memset(p->status_host, 0, sizeof(HostStatus));
     if (e != hipSuccess) { flstm_core_destroy(p); return int(e); }
     *out = p;
     return 0;
@@ -283,7 +293,6 @@ extern "C" int flstm_core_destroy(flstm_core_plan* p) {
                       &p->status, &p->xch_f, &p->xch_b, &p->dYp, &p->dG, &p->dHn, &p->dC,
                       &p->dH0, &p->db_part, &p->dw_part, &p->prof})
         b->release();
-    p->tm.destroy();
     if (p->status_host) (void)hipHostFree(p->status_host);
     delete p;
     return 0;
@@ -292,7 +301,7 @@ extern "C" int flstm_core_destroy(flstm_core_plan* p) {
 extern "C" int flstm_core_set_option(flstm_core_plan* p, const char* name, long value) {
     if (!p || !name) return FLSTM_E_INVALID;
     if (!strcmp(name, "stepwise")) { p->opt_stepwise = value != 0; replan(p); return 0; }
-    if (!strcmp(name, "proj_chunk")) { p->opt_proj_chunk = int(value); return 0; }
+    if (!strcmp(name, "proj_chunk")) return 0;   // (accepted; the projection is one product: forward_project)
     if (!strcmp(name, "spin_limit")) { if (value < 0) return FLSTM_E_INVALID; p->opt_spin_limit = int(value); return 0; }
     if (!strcmp(name, "spin_ms")) { if (value < 1 || value > 60000) return FLSTM_E_INVALID; p->opt_spin_ms = int(value); return 0; }
     if (!strcmp(name, "profile")) {
@@ -420,61 +429,72 @@ namespace {
 
 // Forward pass in three parts so that a caller can feed it in ranges of steps: setup (state rows, exchange
 // ring), any number of step ranges in order (x rows -> projection -> recurrence), and the status check.
+bool x_in_place(const flstm_core_plan* p, flstm_dtype x_dtype) { return x_dtype == FLSTM_F16 && p->d.I == p->d.Ip; }
+
+// (whole_x: the operand of all steps is made here; a pass fed in ranges has not got x yet)
 int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0,
-                  const void* c0, flstm_dtype state_dtype, hipStream_t s) {
+                  const void* c0, flstm_dtype state_dtype, bool whole_x, hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     p->fw.T = T; p->fw.x = x; p->fw.x_dtype = x_dtype; p->fw.open = true;
-    if (!(x_dtype == FLSTM_F16 && d.I == d.Ip)) FL_TRY(p->X16.reserve(TB * d.Ip * sizeof(half_t)));
+    if (!x_in_place(p, x_dtype)) FL_TRY(p->X16.reserve(TB * d.Ip * sizeof(half_t)));
     FL_TRY(p->G.reserve(TB * 4 * d.Hp * sizeof(half_t)));
     FL_TRY(p->Y.reserve((TB + d.B) * d.Hp * sizeof(half_t)));
     FL_TRY(p->C.reserve((TB + d.B) * d.Hp * sizeof(float)));
     const size_t xslot = exchange_slot_halfs(d.B, d.Hp);
     FL_TRY(p->xch_f.reserve(4 * xslot * sizeof(half_t)));
-    // One launch: the initial state rows (a null h0 / c0 reads as zeros), the exchange ring -- slot 0 zero (h0 goes in
-    // below; rows past B stay zero), slots 1 to 3 the 'unwritten' pattern --, the seat counters and the phase counters.
-    PrepList prep;
-    prep.to_half(h0, state_dtype == FLSTM_F32, size_t(d.B), d.H, size_t(d.H), 1.f, p->Y.as<half_t>(), size_t(d.B), size_t(d.Hp));
-    prep.to_float(c0, state_dtype == FLSTM_F32, size_t(d.B), d.H, 1.f, p->C.as<float>(), size_t(d.Hp));
-    prep.fill(p->xch_f.p, xslot * sizeof(half_t), 0u);
+    // One launch: the initial state rows (a null h0 / c0 reads as zeros), the exchange ring -- slot 0 holds h0 (rows past B
+    // zero), slots 1 to 3 the 'unwritten' pattern --, the seat and phase counters, and (whole passes) the fp16 operand
+    // made of x.
+    OpList prep;
+    const int f32 = state_dtype == FLSTM_F32;
+    prep.to_half(h0, f32, size_t(d.B), d.H, size_t(d.H), 1.f, p->Y.as<half_t>(), size_t(d.B), size_t(d.Hp));
+    prep.to_float(c0, f32, size_t(d.B), d.H, 1.f, p->C.as<float>(), size_t(d.Hp));
+    prep.to_exchange(h0, f32, size_t(d.B), d.H, d.Hp, p->xch_f.as<half_t>());
     prep.fill(p->xch_f.as<half_t>() + xslot, 3 * xslot * sizeof(half_t), 0xFFFFFFFFu);
-    prep.fill(p->status.as<unsigned>() + 8, 8 * sizeof(unsigned), 0u);
+    prep.fill(p->status.as<char>() + kSeatsOffset, kStatusBytes - kSeatsOffset, 0u);
+    if (p->static_call) prep.fill(p->status.p, kStampsOffset, 0u);   // (a borrowed status block holds whatever the last call left)
     if (p->opt_profile) prep.fill(p->prof.p, 8 * sizeof(long long), 0u);
-    FL_TRY(run_prep(prep, s));
-    p->fw.seats_clean = true;
-    FL_TRY(to_exchange_layout(p->Y.as<half_t>(), d.B, d.Hp, size_t(d.Hp), p->xch_f.as<half_t>(), s));
+    if (whole_x && !x_in_place(p, x_dtype))
+        prep.to_half(x, x_dtype == FLSTM_F32, TB, d.I, size_t(d.I), 1.f, p->X16.as<half_t>(), TB, size_t(d.Ip));
+    prep.stamps = stamps_of(p);
+    prep.stamp = kStampFwdStart;
+    FL_TRY(run_ops(prep, s));
+    p->seat_sets_left = kSeatSets;
     return 0;
 }
 
 // x rows of steps [t0, t0+n) -> fp16 operand -> x-projection (+ bias) in G
-int forward_project(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
+int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, hipStream_t s) {
     const Dims& d = p->d;
     const half_t* A = nullptr;   // first row of step t0
     size_t lda = 0;
-    if (p->fw.x_dtype == FLSTM_F16 && d.I == d.Ip) {
+    if (x_in_place(p, p->fw.x_dtype)) {
         A = static_cast<const half_t*>(p->fw.x) + t0 * d.B * d.I;
         lda = size_t(d.I);
     } else {
         const size_t esz = p->fw.x_dtype == FLSTM_F32 ? 4 : 2;
         const char* src = static_cast<const char*>(p->fw.x) + t0 * d.B * d.I * esz;
         half_t* dst = p->X16.as<half_t>() + t0 * d.B * d.Ip;
-        FL_TRY(convert_pad(src, p->fw.x_dtype == FLSTM_F32, n * d.B, d.I, size_t(d.I), 1.f, dst, n * d.B, size_t(d.Ip), s));
+        if (!converted) {
+            OpList conv;
+            conv.to_half(src, p->fw.x_dtype == FLSTM_F32, n * d.B, d.I, size_t(d.I), 1.f, dst, n * d.B, size_t(d.Ip));
+            FL_TRY(run_ops(conv, s));
+        }
         A = dst;
         lda = size_t(d.Ip);
     }
-    // hoisted input projection, optionally in chunks of time steps
-    size_t chunk_steps = (p->opt_proj_chunk <= 0 || size_t(p->opt_proj_chunk) > n) ? n : size_t(p->opt_proj_chunk);
-    for (size_t c0 = 0; c0 < n; c0 += chunk_steps) {
-        const size_t steps = (c0 + chunk_steps <= n) ? chunk_steps : n - c0;
-        GemmNT g{};
-        g.A = A + c0 * d.B * lda; g.lda = lda;
-        g.B = p->wih_p.as<half_t>(); g.ldb = size_t(d.Ip);
-        g.M = int(steps * d.B); g.N = 4 * d.Hp; g.K = d.Ip;
-        g.C16 = p->G.as<half_t>() + (t0 + c0) * d.B * 4 * d.Hp; g.C32 = nullptr; g.ldc = size_t(4) * d.Hp;
-        g.alpha = 1.f; g.splits = 1; g.split_stride = 0;
-        g.bias = p->bias_p.as<float>();   // b_ih + b_hh, packed gate order: the recurrence reads x-projection + bias
-        FL_TRY(launch_gemm_nt(g, s));
-    }
+    // The hoisted input projection, one product over all steps.  Cutting it into chunks of time steps (the reference's
+    // projchunksz, option "proj_chunk") saves no memory here, where the gate rows of the whole pass are kept, and changes
+    // no result; chunks of 64 steps of 32 rows at 1024 units took 32 launches of 24.5 us where one product takes 410 us.
+    GemmNT g{};
+    g.A = A; g.lda = lda;
+    g.B = p->wih_p.as<half_t>(); g.ldb = size_t(d.Ip);
+    g.M = int(n * d.B); g.N = 4 * d.Hp; g.K = d.Ip;
+    g.C16 = p->G.as<half_t>() + t0 * d.B * 4 * d.Hp; g.C32 = nullptr; g.ldc = size_t(4) * d.Hp;
+    g.alpha = 1.f; g.splits = 1; g.split_stride = 0;
+    g.bias = p->bias_p.as<float>();   // b_ih + b_hh, packed gate order: the recurrence reads x-projection + bias
+    FL_TRY(launch_gemm_nt(g, s));
     return 0;
 }
 
@@ -486,10 +506,10 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     a.y_out = p->fw.y_direct;
     a.X = p->xch_f.as<half_t>(); a.x_slot = exchange_slot_halfs(d.B, d.Hp);
     a.status = p->status.as<int>();
-    a.seats = p->status.as<unsigned>() + 8;
-    a.delay_hint = p->status.as<int>() + 1;   // (the status block: word 0 status, 1 / 2 delay hints, 8..15 seats)
-    if (!p->fw.seats_clean) FL_TRY(fill_zero(a.seats, 8 * sizeof(unsigned), s));
-    p->fw.seats_clean = false;
+    a.delay_hint = p->status.as<int>() + 1;
+    a.stamps = stamps_of(p) + kStampFwdRec;
+    int rc = next_seats(p, &a.seats, s);
+    if (rc) return rc;
     a.B = d.B; a.Hp = d.Hp; a.T = int(p->fw.T); a.t0 = int(t0); a.t1 = int(t0 + n);
     a.spin_limit = p->opt_spin_limit;
     a.spin_ticks = (long long)p->opt_spin_ms * p->wall_khz;
@@ -511,16 +531,17 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
 
 int forward_once(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0,
                  const void* c0, flstm_dtype state_dtype, hipStream_t s) {
-    int rc = forward_setup(p, T, x, x_dtype, h0, c0, state_dtype, s);
+    int rc = forward_setup(p, T, x, x_dtype, h0, c0, state_dtype, true, s);
     if (rc) return rc;
-    FL_TRY(hipEventRecord(p->tm.ev[0], s));
-    rc = forward_project(p, 0, T, s);
+    rc = forward_project(p, 0, T, true, s);
     if (rc) return rc;
-    FL_TRY(hipEventRecord(p->tm.ev[1], s));
-    rc = forward_recur(p, 0, T, s);
-    if (rc) return rc;
-    FL_TRY(hipEventRecord(p->tm.ev[2], s));
-    return 0;
+    return forward_recur(p, 0, T, s);
+}
+
+void final_states(const flstm_core_plan* p, size_t TB, void* hy, void* cy, flstm_dtype dtype, OpList& out) {
+    const Dims& d = p->d;
+    out.unpad(p->Y.as<half_t>() + TB * d.Hp, 0, size_t(d.Hp), size_t(d.B), d.H, 1.f, hy, dtype == FLSTM_F32);
+    out.unpad(p->C.as<float>() + TB * d.Hp, 1, size_t(d.Hp), size_t(d.B), d.H, 1.f, cy, dtype == FLSTM_F32);
 }
 
 // One whole forward pass: projection, recurrence, outputs, one wait, status.  The outputs are written behind the
@@ -542,14 +563,12 @@ int forward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtyp
         int rc = forward_once(p, T, x, x_dtype, h0, c0, state_dtype, s);
         p->fw.y_direct = nullptr;
         if (rc) return rc;
+        OpList out;   // outputs and final states, one launch
         if (!y_direct)
-            FL_TRY(unpad_from_half(p->Y.as<half_t>() + size_t(d.B) * d.Hp, size_t(d.Hp), TB, d.H, y, y_dtype == FLSTM_F32, s));
-        PrepList out;   // final states, one launch
-        out.unpad(p->Y.as<half_t>() + TB * d.Hp, 0, size_t(d.Hp), size_t(d.B), d.H, 1.f, hy, out_state_dtype == FLSTM_F32);
-        out.unpad(p->C.as<float>() + TB * d.Hp, 1, size_t(d.Hp), size_t(d.B), d.H, 1.f, cy, out_state_dtype == FLSTM_F32);
-        FL_TRY(run_prep(out, s));
+            out.unpad(p->Y.as<half_t>() + size_t(d.B) * d.Hp, 0, size_t(d.Hp), TB, d.H, 1.f, y, y_dtype == FLSTM_F32);
+        final_states(p, TB, hy, cy, out_state_dtype, out);
         int st = 0;
-        rc = wait_status(p, true, s, &st);
+        rc = wait_status(p, out, kStampFwdEnd, s, &st);
         if (rc) return rc;
         if (st == 0) break;
         if (!p->Lf.persistent || attempt > 0) return FLSTM_E_STALLED;
@@ -557,9 +576,9 @@ int forward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtyp
     }
     pass_done(p, true);
     if (p->opt_profile) FL_TRY(hipMemcpy(p->prof_f, p->prof.p, sizeof(p->prof_f), hipMemcpyDeviceToHost));
-    p->ms_fwd[0] = elapsed(p->tm.ev[0], p->tm.ev[1]);
-    p->ms_fwd[1] = elapsed(p->tm.ev[1], p->tm.ev[2]);
-    p->ms_fwd[2] = elapsed(p->tm.ev[0], p->tm.ev[2]);
+    p->ms_fwd[0] = elapsed(p, kStampFwdStart, kStampFwdRec);
+    p->ms_fwd[1] = elapsed(p, kStampFwdRec, kStampFwdRecEnd);
+    p->ms_fwd[2] = elapsed(p, kStampFwdStart, kStampFwdRecEnd);
     p->fw.open = false;
     return 0;
 }
@@ -607,9 +626,8 @@ extern "C" int flstm_core_forward_static(flstm_core_plan* p, size_t T, const voi
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     // the same buffers forward_setup() sizes, carved out of the static array instead of allocated
-    const bool x_in_place = (x_dtype == FLSTM_F16 && d.I == d.Ip);
-    const size_t need[6] = {256,
-                            x_in_place ? 0 : TB * d.Ip * sizeof(half_t),
+    const size_t need[6] = {kStatusBytes,
+                            x_in_place(p, x_dtype) ? 0 : TB * d.Ip * sizeof(half_t),
                             TB * 4 * d.Hp * sizeof(half_t),
                             (TB + d.B) * d.Hp * sizeof(half_t),
                             (TB + d.B) * d.Hp * sizeof(float),
@@ -623,12 +641,12 @@ extern "C" int flstm_core_forward_static(flstm_core_plan* p, size_t T, const voi
     for (int i = 0; i < 6; ++i) { saved[i] = *slot[i]; *slot[i] = DevBuf::view(b + off[i], need[i]); }
     const bool had_cache = p->have_cache;
     p->have_cache = false;   // (the plan's own caches are untouched, but no pass may use the borrowed ones later)
-    // status word and seat counters start at zero; the array keeps whatever the last call left
-    rc = int(fill_zero(p->status.p, 64, s));
-    p->static_call = true;   // (step-wise launches, if the pass comes to them, are plain launches: a graph capture allocates)
-    if (rc == 0)
-        rc = forward_pass(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, s);
+    // (the setup clears the status block: the array keeps whatever the last call left; step-wise launches, if the
+    // pass comes to them, are plain launches: a graph capture allocates)
+    p->static_call = true;
+    rc = forward_pass(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, s);
     p->static_call = false;
+    p->seat_sets_left = 0;
     p->fw.open = false;   // (also when the pass failed: the next call must not find a pass in progress)
     for (int i = 0; i < 6; ++i) *slot[i] = saved[i];
     p->have_cache = had_cache;
@@ -640,7 +658,7 @@ namespace {
 // Backward recurrence in parts, like the forward pass: setup, step ranges from the end of the sequence towards
 // its start (dY rows -> BPTT steps -> dX rows), and the weight-gradient GEMMs over the whole sequence.
 int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_dtype, const void* d_hn,
-                   const void* d_cn, flstm_dtype dstate_dtype, float S, void* dx, flstm_dtype dx_dtype,
+                   const void* d_cn, flstm_dtype dstate_dtype, float S, void* dx, flstm_dtype dx_dtype, bool whole_dy,
                    hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
@@ -666,8 +684,8 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     FL_TRY(p->xch_b.reserve(dg_slots * xslot * sizeof(half_t)));
     // One launch (see forward_setup): the dG ring 'unwritten', the ring of partial sums in its starting parities, the
     // scaled state gradients, the bias-gradient partials, the seat counters, the phase counters.
-    static_assert(kRecBwdPartSlots + 6 <= 10, "PrepList holds ten operations");
-    PrepList prep;
+    static_assert(kRecBwdPartSlots + 7 <= kMaxOps, "what an OpList holds");
+    OpList prep;
     prep.fill(p->xch_b.p, dg_slots * xslot * sizeof(half_t), 0xFFFFFFFFu);
     if (p->Lb.two_d) {
         const size_t pslot = rec_bwd_part_slot_floats(p->Lb) * sizeof(float);
@@ -678,24 +696,30 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     prep.to_float(d_hn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, S, p->dHn.as<float>(), size_t(d.Hp));
     prep.to_float(d_cn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, S, p->dC.as<float>(), size_t(d.Hp));
     prep.fill(p->db_part.p, size_t(p->Lb.ng) * 4 * d.Hp * sizeof(float), 0u);
-    prep.fill(p->status.as<unsigned>() + 8, 8 * sizeof(unsigned), 0u);
+    prep.fill(p->status.as<char>() + kSeatsOffset, kStatusBytes - kSeatsOffset, 0u);
     if (p->opt_profile) prep.fill(p->prof.as<long long>() + 8, 8 * sizeof(long long), 0u);
-    FL_TRY(run_prep(prep, s));
-    p->bw.seats_clean = true;
+    if (whole_dy && p->bw.dYk != dY)
+        prep.to_half(dY, dy_dtype == FLSTM_F32, TB, d.H, size_t(d.H), S, p->dYp.as<half_t>(), TB, size_t(d.Hp));
+    prep.stamps = stamps_of(p);
+    prep.stamp = kStampBwdStart;
+    FL_TRY(run_ops(prep, s));
+    p->seat_sets_left = kSeatSets;
     return 0;
 }
 
 // steps t_hi .. t_lo (t_lo = -1 includes the closing dh0 product); dY rows of these steps are converted first
 // when the caller's dY cannot be used in place
-int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
+int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hipStream_t s) {
     const Dims& d = p->d;
     const long lo = t_lo < 0 ? 0 : t_lo;
-    if (p->bw.dYk != p->bw.dY && t_hi >= lo) {
+    if (!converted && p->bw.dYk != p->bw.dY && t_hi >= lo) {
         const size_t esz = p->bw.dy_dtype == FLSTM_F32 ? 4 : 2;
         const size_t rows = size_t(t_hi - lo + 1) * d.B;
         const char* src = static_cast<const char*>(p->bw.dY) + size_t(lo) * d.B * d.H * esz;
         half_t* dst = p->dYp.as<half_t>() + size_t(lo) * d.B * d.Hp;
-        FL_TRY(convert_pad(src, p->bw.dy_dtype == FLSTM_F32, rows, d.H, size_t(d.H), p->bw.S, dst, rows, size_t(d.Hp), s));
+        OpList conv;
+        conv.to_half(src, p->bw.dy_dtype == FLSTM_F32, rows, d.H, size_t(d.H), p->bw.S, dst, rows, size_t(d.Hp));
+        FL_TRY(run_ops(conv, s));
     }
     RecBwdArgs a{};
     a.wfrag = p->wfrag_b.as<half8>();
@@ -709,8 +733,8 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
     }
     a.db_part = p->db_part.as<float>();
     a.status = p->status.as<int>();
-    a.seats = p->status.as<unsigned>() + 8;
     a.delay_hint = p->status.as<int>() + 2;
+    a.stamp_end = stamps_of(p) + kStampBwdRecEnd;
     a.B = d.B; a.Hp = d.Hp; a.T = int(p->bw.T); a.dy_scale = p->bw.dy_scale;
     a.t_hi = int(t_hi); a.t_lo = int(t_lo);
     a.spin_limit = p->opt_spin_limit;
@@ -723,8 +747,8 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
     for (int b_lo = 0; b_lo < d.B; b_lo += win) {
         a.b_lo = b_lo;
         a.b_hi = b_lo + win < d.B ? b_lo + win : d.B;
-        if (!p->bw.seats_clean) FL_TRY(fill_zero(a.seats, 8 * sizeof(unsigned), s));
-        p->bw.seats_clean = false;
+        int rc = next_seats(p, &a.seats, s);
+        if (rc) return rc;
         if (win < d.B) {
             const size_t pslot = a.p_slot * sizeof(float);
             const int first_T = t_hi >= long(p->bw.T) - 1 ? int(p->bw.T) : int(t_hi) + 2;   // (its first product step is first_T - 2)
@@ -758,13 +782,9 @@ int backward_dx(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
 int backward_rec_once(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_dtype, const void* d_hn,
                       const void* d_cn, flstm_dtype dstate_dtype, float S, void* dx, flstm_dtype dx_dtype,
                       hipStream_t s) {
-    int rc = backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, S, dx, dx_dtype, s);
+    int rc = backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, S, dx, dx_dtype, true, s);
     if (rc) return rc;
-    FL_TRY(hipEventRecord(p->tm.ev[3], s));
-    rc = backward_recur(p, long(T) - 1, -1, s);
-    if (rc) return rc;
-    FL_TRY(hipEventRecord(p->tm.ev[4], s));
-    return 0;
+    return backward_recur(p, long(T) - 1, -1, true, s);
 }
 
 // dW_ih = dG^T * X and dW_hh = dG^T * H_prev over the whole sequence, bias gradient and state gradients
@@ -780,6 +800,8 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, floa
     const half_t* Xop = direct ? static_cast<const half_t*>(x) : p->X16.as<half_t>();
     const half_t* Hop = p->Y.as<half_t>();
     const int n_ih = dW_ih ? d.Ip : 0, n_hh = dW_hh ? d.Hp : 0, ncols = n_ih + n_hh;
+    const bool accumulate = p->opt_accumulate != 0;
+    OpList out;   // gradients into the caller's layout, one launch
     if (ncols > 0) {
         // automatic: what the kernels' schedules make fastest (gemm_tn_plan_splits), at least two 64-row slabs per split
         int want = p->opt_dw_splits > 0 ? p->opt_dw_splits : p->eff_dw;
@@ -802,21 +824,18 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, floa
         }
         g.C16 = nullptr; g.C32 = p->dw_part.as<float>(); g.ldc = size_t(ncols);
         g.alpha = 1.f; g.splits = splits; g.split_stride = per;
+        g.stamp = stamps_of(p) + kStampBwdDw;
         FL_TRY(launch_gemm_tn(g, s));
-        FL_TRY(reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), 0, n_ih, d.I, invS, p->opt_accumulate != 0, dW_ih, s));
-        FL_TRY(reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), n_ih, n_hh, d.H, invS, p->opt_accumulate != 0, dW_hh, s));
+        out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), 0, d.I, invS, accumulate, dW_ih);
+        out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), n_ih, d.H, invS, accumulate, dW_hh);
     }
-    FL_TRY(hipEventRecord(p->tm.ev[6], s));
-    if (db_ih || db_hh)
-        FL_TRY(reduce_db(d, p->db_part.as<float>(), p->Lb.ng, invS, p->opt_accumulate != 0, db_ih, db_hh, s));
-    PrepList out;   // state gradients, one launch
+    out.reduce_db(d, p->db_part.as<float>(), p->Lb.ng, invS, accumulate, db_ih, db_hh);
     out.unpad(p->dH0.as<float>(), 1, size_t(d.Hp), size_t(d.B), d.H, invS, dh0, 1);
     out.unpad(p->dC.as<float>(), 1, size_t(d.Hp), size_t(d.B), d.H, invS, dc0, 1);
-    FL_TRY(run_prep(out, s));
-    FL_TRY(hipEventRecord(p->tm.ev[7], s));
-    int rc = enqueue_status_copy(p, s);
+    int rc = publish_with(p, out, kStampBwdEnd, s);
     if (rc) return rc;
-    FL_TRY(hipStreamSynchronize(s));
+    rc = wait_stream(s);
+    if (rc) return rc;
     p->bw.open = false;
     return 0;
 }
@@ -852,16 +871,16 @@ extern "C" int flstm_core_backward(flstm_core_plan* p, size_t T, const void* x, 
         if (rc) return rc;
         int st = 0;
         if (p->opt_accumulate) {
-            rc = wait_status(p, false, s, &st);
+            OpList nothing;
+            rc = wait_status(p, nothing, -1, s, &st);
             if (rc) return rc;
         }
         if (st == 0) {
             rc = backward_dx(p, long(T) - 1, 0, s);
             if (rc) return rc;
-            FL_TRY(hipEventRecord(p->tm.ev[5], s));
             rc = backward_finish(p, x, x_dtype, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
             if (rc) return rc;
-            rc = take_status(p, false, s, &st);
+            rc = take_status(p, s, &st);
             if (rc) return rc;
             if (st == 0) break;
         }
@@ -871,10 +890,11 @@ extern "C" int flstm_core_backward(flstm_core_plan* p, size_t T, const void* x, 
     pass_done(p, false);
     if (p->opt_profile)
         FL_TRY(hipMemcpy(p->prof_b, p->prof.as<long long>() + 8, sizeof(p->prof_b), hipMemcpyDeviceToHost));
-    p->ms_bwd[0] = elapsed(p->tm.ev[3], p->tm.ev[4]);
-    p->ms_bwd[1] = elapsed(p->tm.ev[4], p->tm.ev[5]);
-    p->ms_bwd[2] = elapsed(p->tm.ev[5], p->tm.ev[6]);
-    p->ms_bwd[3] = elapsed(p->tm.ev[3], p->tm.ev[7]);
+    const int dw_start = (dW_ih || dW_hh) ? kStampBwdDw : kStampBwdEnd;   // (without that product the dX one ends with the pass)
+    p->ms_bwd[0] = elapsed(p, kStampBwdStart, kStampBwdRecEnd);
+    p->ms_bwd[1] = elapsed(p, kStampBwdRecEnd, dw_start);
+    p->ms_bwd[2] = elapsed(p, dw_start, kStampBwdEnd);
+    p->ms_bwd[3] = elapsed(p, kStampBwdStart, kStampBwdEnd);
     return 0;
 }
 
@@ -888,14 +908,14 @@ extern "C" int flstm_core_forward_begin(flstm_core_plan* p, size_t T, const void
     p->have_cache = false;
     for (float& m : p->ms_fwd) m = -1.f;
     use_tuned(p, T);
-    return forward_setup(p, T, x, x_dtype, h0, c0, state_dtype, static_cast<hipStream_t>(stream));
+    return forward_setup(p, T, x, x_dtype, h0, c0, state_dtype, false, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int flstm_core_forward_steps(flstm_core_plan* p, size_t t0, size_t nsteps, void* stream) {
     if (!p || !p->fw.open || t0 + nsteps > p->fw.T) return FLSTM_E_INVALID;
     if (nsteps == 0) return 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int rc = forward_project(p, t0, nsteps, s);
+    int rc = forward_project(p, t0, nsteps, false, s);
     if (rc) return rc;
     return forward_recur(p, t0, nsteps, s);
 }
@@ -907,12 +927,10 @@ extern "C" int flstm_core_forward_end(flstm_core_plan* p, void* hy, void* cy, fl
     const Dims& d = p->d;
     const size_t TB = p->fw.T * size_t(d.B);
     p->fw.open = false;
-    FL_TRY(unpad_from_half(p->Y.as<half_t>() + TB * d.Hp, size_t(d.Hp), size_t(d.B), d.H, hy,
-                           out_state_dtype == FLSTM_F32, s));
-    FL_TRY(unpad_from_float(p->C.as<float>() + TB * d.Hp, size_t(d.Hp), size_t(d.B), d.H, 1.f, cy,
-                            out_state_dtype == FLSTM_F32, s));
+    OpList out;
+    final_states(p, TB, hy, cy, out_state_dtype, out);
     int st = 0;
-    int rc = wait_status(p, true, s, &st);
+    int rc = wait_status(p, out, kStampFwdEnd, s, &st);
     if (rc) return rc;
     if (st != 0) {   // a persistent launch gave up: the caller repeats the pass through flstm_core_forward
         if (p->Lf.persistent) demote(p, true);
@@ -931,7 +949,7 @@ extern "C" int flstm_core_backward_begin(flstm_core_plan* p, size_t T, const voi
     for (float& m : p->ms_bwd) m = -1.f;
     const float S = grad_scale > 0.f ? grad_scale : 1.f;
     use_tuned(p, T);
-    return backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, S, dx, dx_dtype, static_cast<hipStream_t>(stream));
+    return backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, S, dx, dx_dtype, false, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int flstm_core_backward_steps(flstm_core_plan* p, size_t t_hi, size_t nsteps, void* stream) {
@@ -939,7 +957,7 @@ extern "C" int flstm_core_backward_steps(flstm_core_plan* p, size_t t_hi, size_t
     hipStream_t s = static_cast<hipStream_t>(stream);
     const long lo = long(t_hi) - long(nsteps) + 1;
     // the range that reaches step 0 also runs the closing product for dh0
-    int rc = backward_recur(p, long(t_hi), lo == 0 ? -1 : lo, s);
+    int rc = backward_recur(p, long(t_hi), lo == 0 ? -1 : lo, false, s);
     if (rc == int(hipErrorCooperativeLaunchTooLarge) && p->Lb.persistent && !p->refused_bwd) {
         // the grid cannot be co-resident: step-wise from now on; the rings of this pass were laid out for the persistent
         // kernel, so the caller repeats the pass (as after a launch that gave up)
@@ -961,7 +979,8 @@ extern "C" int flstm_core_backward_end(flstm_core_plan* p, const void* x, flstm_
     hipStream_t s = static_cast<hipStream_t>(stream);
     // the caller's gradients may be accumulated into: the status of the recurrence is checked before they are touched
     int st = 0;
-    int rc = wait_status(p, false, s, &st);
+    OpList nothing;
+    int rc = wait_status(p, nothing, -1, s, &st);
     if (rc) return rc;
     if (st != 0) {   // the caller repeats the pass through flstm_core_backward
         p->bw.open = false;

@@ -20,6 +20,8 @@ struct GemmNT {
     // [N1, N) from B2 (N - N1 columns, row pitch ldb2): one launch forms A^T * [B | B2] and reads A once.  N1 must
     // be a multiple of 8; output tiles never straddle the seam (each side is tiled on its own).
     const half_t* B2; size_t ldb2; int N1;
+    // optional: workgroup 0 leaves the time it started here (ticks of the constant-rate clock)
+    long long* stamp;
 };
 
 // Enqueue on `stream`. Returns hipSuccess or the launch error.

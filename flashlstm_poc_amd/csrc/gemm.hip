@@ -217,6 +217,7 @@ __global__ __launch_bounds__(kThreads) void gemm_nt_stream(GemmNT g, TileOrder o
 
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    if (g.stamp && blockIdx.x == 0 && tid == 0) *g.stamp = wall_clock64();
     const int wm = wave / kWavesN, wn = wave % kWavesN;
     const int rounds = order.per_xcd;
 
@@ -444,6 +445,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_stream(GemmNT g, TileOrder o
 
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    if (g.stamp && blockIdx.x == 0 && tid == 0) *g.stamp = wall_clock64();
     const int wm = wave / kWavesN, wn = wave % kWavesN;
     const int rounds = order.per_xcd;
     const int nslab_total = (g.K + BK - 1) / BK;

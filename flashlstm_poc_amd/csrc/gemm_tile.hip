@@ -139,6 +139,7 @@ __global__ __launch_bounds__(kTileThreads) void gemm_nt_tile(GemmNT g, int tiles
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    if (g.stamp && blockIdx.x == 0 && tid == 0) *g.stamp = wall_clock64();
     int tm, tn;
     tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * TM, n0 = tn * TM, nk = g.K / BK;
@@ -237,6 +238,7 @@ __global__ __launch_bounds__(kTileThreads) void gemm_tn_tile(GemmNT g, int tiles
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    if (g.stamp && blockIdx.x == 0 && tid == 0) *g.stamp = wall_clock64();
     int tm, tn;
     tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int tiles_n1 = g.B2 ? (g.N1 + TM - 1) / TM : (1 << 30);

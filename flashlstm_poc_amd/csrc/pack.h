@@ -23,41 +23,6 @@ hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, hal
 hipError_t pack_wfrag_bwd2d(const Dims& d, const float* w_hh, half8* out, int kq, hipStream_t s);
 hipError_t pack_bias(const Dims& d, const float* b_ih, const float* b_hh, float* bias_p, hipStream_t s);
 
-// rows x cols (ld_in, fp32 when in_f32 else fp16) -> fp16 [rows_out][ld_out], zero padded.
-// Replaces src/kernels.cu:5-43 (populate_activations_kernel).
-hipError_t convert_pad(const void* in, int in_f32, size_t rows, int cols, size_t ld_in, float scale,
-                       half_t* out, size_t rows_out, size_t ld_out, hipStream_t s);
-// fp16/fp32 (rows x cols) -> fp32 [rows][ld_out] zero padded, scaled; null input -> zeros.
-hipError_t convert_pad_f32(const void* in, int in_f32, size_t rows, int cols, float scale, float* out,
-                           size_t ld_out, hipStream_t s);
-// padded internals -> caller tensors: out[r][c] = scale * in[r][c], c < cols.
-hipError_t unpad_from_half(const half_t* in, size_t ld_in, size_t rows, int cols, void* out, int out_f32,
-                           hipStream_t s);
-hipError_t unpad_from_float(const float* in, size_t ld_in, size_t rows, int cols, float scale, void* out,
-                            int out_f32, hipStream_t s);
-
-// Row-block gather: output row r is input row (r / rows_per_block) * block_stride + r % rows_per_block.
-// Used to pull the pre-step states at every R-th step out of the state arrays (the h/c checkpoints
-// of flashlstm_v2/src/lstm_forward.cu:727-783).
-hipError_t gather_from_half(const half_t* in, size_t ld_in, size_t rows, int cols, void* out, int out_f32,
-                            size_t rows_per_block, size_t block_stride, hipStream_t s);
-hipError_t gather_from_float(const float* in, size_t ld_in, size_t rows, int cols, float scale, void* out,
-                             int out_f32, size_t rows_per_block, size_t block_stride, hipStream_t s);
-
-// out[c][r] = in[r][c] for r < rows, c < cols; out rows are ld_out long, columns [rows, ld_out) are
-// zeroed; output rows [cols, cols_out) are zeroed as well.
-hipError_t transpose_pad(const void* in, int in_f32, size_t rows, int cols, size_t ld_in, half_t* out,
-                         int cols_out, size_t ld_out, hipStream_t s);
-
-// Sums columns [col0, col0 + ncols) of the split-K partials [splits][4Hp][ld] (packed gate rows) into dst
-// [4H][out_cols] (PyTorch row order, the first out_cols of those columns), times `scale`; `accumulate` adds to dst
-// instead of overwriting it (the beta=1 accumulation over chunks of flashlstm_v2/src/lstm_backward.cu:1112-1142).
-hipError_t reduce_dw(const Dims& d, const float* partial, int splits, size_t ld, int col0, int ncols, int out_cols,
-                     float scale, bool accumulate, float* dst, hipStream_t s);
-// db_part [ng][4Hp] packed -> db_ih == db_hh (4H), times scale (flashlstm_v2/src/lstm_backward.cu:1218-1231).
-hipError_t reduce_db(const Dims& d, const float* db_part, int ng, float scale, bool accumulate, float* db_ih,
-                     float* db_hh, hipStream_t s);
-
 // dst[r][c] (pitch ldc) = sum over z < splits of partial[z * per + r * cols + c]: split-K partials of a plain GEMM.
 hipError_t reduce_partials(const float* partial, int splits, size_t per, int rows, int cols, size_t ldc, float* dst,
                            hipStream_t s);
@@ -69,50 +34,70 @@ hipError_t checksum_add(const void* p, size_t bytes, u64 salt, u64* out, hipStre
 
 hipError_t fill_zero(void* p, size_t bytes, hipStream_t s);
 
-// Up to ten of the small operations above in ONE launch: a pass starts with half a dozen of them (state rows, rings,
-// counters), each a few microseconds of kernel plus a launch gap of its own when issued one by one.
-struct PrepOp {
-    enum Kind : int { kNone = 0, kFill = 1, kToHalf = 2, kToFloat = 3, kUnpad = 4 };
-    int kind = kNone;
-    int in_f32 = 0, out_f32 = 0;
+// The layout operations around the GEMMs and the recurrence, up to kMaxOps of them in ONE launch.  A pass starts with
+// half a dozen of them (state rows, rings, counters, operand conversion) and ends with as many (outputs, final states,
+// gradient reductions); each is a few microseconds of kernel plus a launch of its own when issued one by one.
+constexpr int kMaxOps = 12;
+struct LayoutOp {
+    enum Kind : int { kFill = 1, kToHalf, kToFloat, kUnpad, kToExchange, kReduceDw, kReduceDb };
+    int kind = 0;
+    int in_f32 = 0, out_f32 = 0, vec = 1;   // vec: elements per work item (8 or 4 where alignment allows, else 1)
     void* dst = nullptr;
-    const void* src = nullptr;   // kToHalf / kToFloat: null reads as zeros
-    size_t n = 0;                // kFill: 32-bit words; kToHalf / kToFloat: rows_out * ld_out elements; kUnpad: rows * cols
-    unsigned word = 0;           // kFill
-    size_t rows = 0, ld_in = 0, ld_out = 1;
+    void* dst2 = nullptr;
+    const void* src = nullptr;              // null reads as zeros (kToHalf, kToFloat, kToExchange)
+    size_t n = 0;                           // work items
+    size_t rows = 0, ld_in = 0, ld_out = 1; // elements
+    size_t rows_per_block = 0, block_stride = 0;
     int cols = 0;
+    unsigned word = 0;                      // kFill
     float scale = 1.f;
+    int splits = 0, H = 0, accumulate = 0;  // kReduceDw, kReduceDb
+    size_t per = 0;
+    unsigned first_block = 0, blocks = 0;   // set by run_ops
 };
-struct PrepList {
+// Time stamps and status of a pass.  Device side: word 0 of `status` is the recurrence's status, `stamps` hold ticks of
+// the constant-rate clock.  A list with `publish` set copies both to pinned host memory, so that the wait that ends the
+// pass is also the one that makes them readable: no copy command and no second round trip.
+enum Stamp : int { kStampFwdStart, kStampFwdRec, kStampFwdRecEnd, kStampBwdStart, kStampBwdRecEnd, kStampBwdDw, kStampBwdEnd, kStampFwdEnd, kStampCount };
+struct HostStatus {
+    int status;
+    int pad[15];
+    long long stamps[kStampCount];
+};
+struct OpList {
     int count = 0;
-    PrepOp op[10];
-    void fill(void* p, size_t bytes, unsigned word) {
-        if (bytes == 0) return;
-        PrepOp& o = op[count++];
-        o.kind = PrepOp::kFill; o.dst = p; o.n = bytes / 4; o.word = word;
-    }
-    // the operations of convert_pad() and convert_pad_f32()
-    void to_half(const void* in, int in_f32, size_t rows, int cols, size_t ld_in, float scale, half_t* out, size_t rows_out, size_t ld_out) {
-        if (rows_out * ld_out == 0) return;
-        PrepOp& o = op[count++];
-        o.kind = PrepOp::kToHalf; o.in_f32 = in_f32; o.dst = out; o.src = in; o.n = rows_out * ld_out;
-        o.rows = rows; o.cols = cols; o.ld_in = ld_in; o.ld_out = ld_out; o.scale = scale;
-    }
-    void to_float(const void* in, int in_f32, size_t rows, int cols, float scale, float* out, size_t ld_out) {
-        if (rows * ld_out == 0) return;
-        PrepOp& o = op[count++];
-        o.kind = PrepOp::kToFloat; o.in_f32 = in_f32; o.dst = out; o.src = in; o.n = rows * ld_out;
-        o.rows = rows; o.cols = cols; o.ld_in = size_t(cols); o.ld_out = ld_out; o.scale = scale;
-    }
-    // the operation of unpad_from_half() / unpad_from_float(): out[r][c] = scale * in[r][c], c < cols; a null `out` adds nothing
-    void unpad(const void* in, int in_f32, size_t ld_in, size_t rows, int cols, float scale, void* out, int out_f32) {
-        if (out == nullptr || rows * size_t(cols) == 0) return;
-        PrepOp& o = op[count++];
-        o.kind = PrepOp::kUnpad; o.in_f32 = in_f32; o.out_f32 = out_f32; o.dst = out; o.src = in; o.n = rows * size_t(cols);
-        o.rows = rows; o.cols = cols; o.ld_in = ld_in; o.ld_out = size_t(cols); o.scale = scale;
-    }
+    int stamp = -1;                   // which stamp block 0 writes when it is done (-1: none)
+    const int* status = nullptr;      // device status word (with `publish`)
+    long long* stamps = nullptr;
+    HostStatus* publish = nullptr;
+    LayoutOp op[kMaxOps];
+
+    void fill(void* p, size_t bytes, unsigned word);   // bytes: a multiple of 4
+    // rows x cols (pitch ld_in, fp32 when in_f32 else fp16; null reads as zeros), times `scale`, -> fp16 [rows_out][ld_out], zero padded
+    void to_half(const void* in, int in_f32, size_t rows, int cols, size_t ld_in, float scale, half_t* out, size_t rows_out, size_t ld_out);
+    // ... -> fp32 [rows][ld_out], zero padded (the input's pitch is cols)
+    void to_float(const void* in, int in_f32, size_t rows, int cols, float scale, float* out, size_t ld_out);
+    // padded internals -> caller tensors: out[r][c] = scale * in[row(r)][c], c < cols, with
+    // row(r) = (r / rows_per_block) * block_stride + r % rows_per_block (rows_per_block = 0: row(r) = r): a gather of row
+    // blocks pulls the states at every R-th step out of the state arrays.  A null `out` adds nothing.
+    void unpad(const void* in, int in_f32, size_t ld_in, size_t rows, int cols, float scale, void* out, int out_f32,
+               size_t rows_per_block = 0, size_t block_stride = 0);
+    // rows x cols (pitch cols; null reads as zeros) -> a whole slot of an exchange ring (fragment-major, rows padded to 32, kcols
+    // columns), zero elsewhere
+    void to_exchange(const void* in, int in_f32, size_t rows, int cols, int kcols, half_t* slot);
+    // Sums columns [col0, col0 + out_cols) of the split-K partials [splits][4Hp][ld] (packed gate rows) into dst
+    // [4H][out_cols] (PyTorch row order), times `scale`; `accumulate` adds to dst instead of overwriting it (the beta=1
+    // accumulation over chunks of flashlstm_v2/src/lstm_backward.cu:1112-1142).  A null dst adds nothing.
+    void reduce_dw(const Dims& d, const float* partial, int splits, size_t ld, int col0, int out_cols, float scale, bool accumulate, float* dst);
+    // db_part [ng][4Hp] packed -> db_ih == db_hh (4H), times scale (flashlstm_v2/src/lstm_backward.cu:1218-1231)
+    void reduce_db(const Dims& d, const float* db_part, int ng, float scale, bool accumulate, float* db_ih, float* db_hh);
 };
-hipError_t run_prep(const PrepList& list, hipStream_t s);
+hipError_t run_ops(OpList& list, hipStream_t s);
+// one operation as a launch of its own
+hipError_t gather_from_half(const half_t* in, size_t ld_in, size_t rows, int cols, void* out, int out_f32,
+                            size_t rows_per_block, size_t block_stride, hipStream_t s);
+hipError_t gather_from_float(const float* in, size_t ld_in, size_t rows, int cols, float scale, void* out, int out_f32,
+                             size_t rows_per_block, size_t block_stride, hipStream_t s);
 // fp16 values spread over (-amp, amp) from a hash of the index (operands for timing runs)
 hipError_t fill_noise(half_t* p, size_t n, unsigned seed, float amp, hipStream_t s);
 // Fills a buffer (multiple of 4 bytes) with one 32-bit pattern; a kernel, so it may be captured in a graph.

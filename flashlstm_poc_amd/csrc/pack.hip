@@ -121,131 +121,196 @@ __global__ void pack_bias_kernel(Dims d, const float* __restrict__ b_ih, const f
     out[q] = row >= 0 ? b_ih[row] + b_hh[row] : 0.f;
 }
 
-template <typename TIn>
-__global__ void convert_pad_kernel(const TIn* __restrict__ in, size_t rows, int cols, size_t ld_in,
-                                   float scale, half_t* __restrict__ out, size_t rows_out, size_t ld_out) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    if (idx >= rows_out * ld_out) return;
-    const size_t r = idx / ld_out;
-    const int c = int(idx % ld_out);
-    float v = 0.f;
-    if (r < rows && c < cols) v = scale * (float)in[r * ld_in + c];
-    out[idx] = (half_t)v;
-}
-
-template <typename TIn>
-__global__ void convert_pad_f32_kernel(const TIn* __restrict__ in, size_t rows, int cols, float scale,
-                                       float* __restrict__ out, size_t ld_out) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    if (idx >= rows * ld_out) return;
-    const size_t r = idx / ld_out;
-    const int c = int(idx % ld_out);
-    float v = 0.f;
-    if (in != nullptr && c < cols) v = scale * (float)in[r * cols + c];
-    out[idx] = v;
-}
-
-// Output row r comes from input row (r / rows_per_block) * block_stride + r % rows_per_block.
-template <typename TIn, typename TOut>
-__global__ void unpad_kernel(const TIn* __restrict__ in, size_t ld_in, size_t rows, int cols, float scale,
-                             TOut* __restrict__ out, size_t rows_per_block, size_t block_stride) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    if (idx >= rows * size_t(cols)) return;
-    const size_t r = idx / cols;
-    const int c = int(idx % cols);
-    const size_t rin = (r / rows_per_block) * block_stride + r % rows_per_block;
-    out[idx] = (TOut)(scale * (float)in[rin * ld_in + c]);
-}
-
-// 64x64 tile transpose through LDS.
-template <typename TIn>
-__global__ void transpose_pad_kernel(const TIn* __restrict__ in, size_t rows, int cols, size_t ld_in,
-                                     half_t* __restrict__ out, int cols_out, size_t ld_out) {
-    __shared__ half_t tile[64][66];
-    const size_t r0 = size_t(blockIdx.x) * 64;
-    const int c0 = blockIdx.y * 64;
-    const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;  // 4 rows of 64 threads
-    for (int i = ty; i < 64; i += 4) {
-        const size_t r = r0 + i;
-        const int c = c0 + tx;
-        float v = 0.f;
-        if (r < rows && c < cols) v = (float)in[r * ld_in + c];
-        tile[i][tx] = (half_t)v;
-    }
-    __syncthreads();
-    for (int i = ty; i < 64; i += 4) {
-        const int c = c0 + i;       // output row
-        const size_t r = r0 + tx;   // output column
-        if (c < cols_out && r < ld_out) out[size_t(c) * ld_out + r] = tile[tx][i];
-    }
-}
-
-// columns [col0, col0 + ncols) of partial [splits][4Hp][ld] with packed gate rows -> dst [4H][out_cols] in PyTorch
-// row order
-__global__ void reduce_dw_kernel(Dims d, const float* __restrict__ partial, int splits, size_t ld, int col0, int ncols,
-                                 int out_cols, float scale, int accumulate, float* __restrict__ dst) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    if (idx >= size_t(4) * d.Hp * ncols) return;
-    const int q = int(idx / ncols), n = int(idx % ncols);
-    const int row = torch_row(q, d.H);
-    if (row < 0 || n >= out_cols) return;
-    const size_t per = size_t(4) * d.Hp * ld, src = size_t(q) * ld + col0 + n;
-    float s = 0.f;
-    for (int z = 0; z < splits; ++z) s += partial[size_t(z) * per + src];
-    float* out = dst + size_t(row) * out_cols + n;
-    *out = accumulate ? *out + scale * s : scale * s;
-}
-
-__global__ void reduce_db_kernel(Dims d, const float* __restrict__ db_part, int ng, float scale, int accumulate,
-                                 float* __restrict__ db_ih, float* __restrict__ db_hh) {
-    const int q = blockIdx.x * kT + threadIdx.x;
-    if (q >= 4 * d.Hp) return;
-    const int row = torch_row(q, d.H);
-    if (row < 0) return;
-    float s = 0.f;
-    for (int g = 0; g < ng; ++g) s += db_part[size_t(g) * 4 * d.Hp + q];
-    s *= scale;
-    if (db_ih) db_ih[row] = accumulate ? db_ih[row] + s : s;
-    if (db_hh && db_hh != db_ih) db_hh[row] = accumulate ? db_hh[row] + s : s;
-}
-
-// flat 16-byte copy (both ends 16-byte aligned, n16 chunks)
-__global__ void copy16_kernel(const uint4* __restrict__ in, uint4* __restrict__ out, size_t n16) {
-    const size_t stride = size_t(gridDim.x) * kT;
-    for (size_t i = size_t(blockIdx.x) * kT + threadIdx.x; i < n16; i += stride) out[i] = in[i];
-}
-
 __global__ void fill_words_kernel(unsigned* p, size_t words, unsigned value) {
     const size_t stride = size_t(gridDim.x) * kT;
     for (size_t i = size_t(blockIdx.x) * kT + threadIdx.x; i < words; i += stride) p[i] = value;
 }
 
-// blockIdx.y selects the operation, the blocks of a row walk it with a grid stride
-__global__ void prep_kernel(PrepList list) {
-    const PrepOp& o = list.op[blockIdx.y];
-    const size_t stride = size_t(gridDim.x) * kT;
-    const size_t first = size_t(blockIdx.x) * kT + threadIdx.x;
-    if (o.kind == PrepOp::kFill) {
-        unsigned* p = static_cast<unsigned*>(o.dst);
-        for (size_t i = first; i < o.n; i += stride) p[i] = o.word;
-    } else if (o.kind == PrepOp::kToHalf || o.kind == PrepOp::kToFloat) {
-        for (size_t i = first; i < o.n; i += stride) {
-            const size_t r = i / o.ld_out;
-            const int c = int(i % o.ld_out);
-            float v = 0.f;
-            if (o.src != nullptr && r < o.rows && c < o.cols) {
-                const size_t at = r * o.ld_in + c;
-                v = o.scale * (o.in_f32 ? static_cast<const float*>(o.src)[at] : (float)static_cast<const half_t*>(o.src)[at]);
-            }
-            if (o.kind == PrepOp::kToHalf) static_cast<half_t*>(o.dst)[i] = (half_t)v;
-            else static_cast<float*>(o.dst)[i] = v;
+// Index arithmetic of the operations in 32 bits where the counts allow: a 64-bit division is a hundred instructions,
+// more than the memory traffic of the 16 bytes it addresses.
+__device__ __forceinline__ void split_index(size_t i, size_t width, size_t& r, size_t& c) {
+    if ((i | width) >> 32) { r = i / width; c = i % width; }
+    else { const unsigned q = unsigned(i) / unsigned(width); r = q; c = unsigned(i) - q * unsigned(width); }
+}
+
+template <int V>
+__device__ __forceinline__ void load_floats(const void* src, size_t at, int in_f32, float (&v)[V]) {
+    if constexpr (V == 8) {
+        if (in_f32) {
+            const floatx4* p = reinterpret_cast<const floatx4*>(static_cast<const float*>(src) + at);
+            const floatx4 a = p[0], b = p[1];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
+        } else {
+            const half8 h = ld_half8(static_cast<const half_t*>(src) + at);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = (float)h[e];
         }
-    } else if (o.kind == PrepOp::kUnpad) {
-        for (size_t i = first; i < o.n; i += stride) {
-            const size_t at = (i / o.cols) * o.ld_in + i % o.cols;
-            const float v = o.scale * (o.in_f32 ? static_cast<const float*>(o.src)[at] : (float)static_cast<const half_t*>(o.src)[at]);
-            if (o.out_f32) static_cast<float*>(o.dst)[i] = v;
-            else static_cast<half_t*>(o.dst)[i] = (half_t)v;
+    } else {
+        v[0] = in_f32 ? static_cast<const float*>(src)[at] : (float)static_cast<const half_t*>(src)[at];
+    }
+}
+template <int V>
+__device__ __forceinline__ void store_values(void* dst, size_t at, int out_f32, const float (&v)[V]) {
+    if constexpr (V == 8) {
+        if (out_f32) {
+            floatx4* p = reinterpret_cast<floatx4*>(static_cast<float*>(dst) + at);
+            p[0] = floatx4{v[0], v[1], v[2], v[3]};
+            p[1] = floatx4{v[4], v[5], v[6], v[7]};
+        } else {
+            half8 h;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) h[e] = (half_t)v[e];
+            st_half8(static_cast<half_t*>(dst) + at, h);
+        }
+    } else {
+        if (out_f32) static_cast<float*>(dst)[at] = v[0];
+        else static_cast<half_t*>(dst)[at] = (half_t)v[0];
+    }
+}
+
+// kToHalf / kToFloat: V consecutive elements of an output row (V = 8: ld_out is a multiple of 8)
+template <int V>
+__device__ __forceinline__ void op_convert(const LayoutOp& o, size_t first, size_t stride) {
+    const int out_f32 = o.kind == LayoutOp::kToFloat;
+    const bool aligned = (o.ld_in % V == 0) && (reinterpret_cast<uintptr_t>(o.src) % 16 == 0);   // whole 16-byte loads
+    for (size_t i = first; i < o.n; i += stride) {
+        size_t r, c;
+        split_index(i, o.ld_out / V, r, c);
+        c *= V;
+        float v[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = 0.f;
+        if (o.src != nullptr && r < o.rows) {
+            const size_t at = r * o.ld_in + c;
+            if (aligned && c + V <= size_t(o.cols)) {
+                load_floats<V>(o.src, at, o.in_f32, v);
+            } else {
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+                    if (c + e < size_t(o.cols)) { float one[1]; load_floats<1>(o.src, at + e, o.in_f32, one); v[e] = one[0]; }
+            }
+#pragma unroll
+            for (int e = 0; e < V; ++e) v[e] *= o.scale;
+        }
+        store_values<V>(o.dst, r * o.ld_out + c, out_f32, v);
+    }
+}
+
+// kUnpad: V consecutive elements of an output row (V = 8: both pitches multiples of 8, both bases 16-byte aligned)
+template <int V>
+__device__ __forceinline__ void op_unpad(const LayoutOp& o, size_t first, size_t stride) {
+    for (size_t i = first; i < o.n; i += stride) {
+        size_t r, c;
+        split_index(i, size_t(o.cols) / V, r, c);
+        size_t rin = r;
+        if (o.rows_per_block) {
+            size_t blk, rest;
+            split_index(r, o.rows_per_block, blk, rest);
+            rin = blk * o.block_stride + rest;
+        }
+        float v[V];
+        load_floats<V>(o.src, rin * o.ld_in + c * V, o.in_f32, v);
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] *= o.scale;
+        store_values<V>(o.dst, i * V, o.out_f32, v);
+    }
+}
+
+// kReduceDw: V consecutive columns of a gradient row (V = 4: pitches and first column multiples of 4).  The partials of an element are
+// added in the order of the splits.
+template <int V>
+__device__ __forceinline__ void op_reduce_dw(const LayoutOp& o, size_t first, size_t stride) {
+    const float* partial = static_cast<const float*>(o.src);
+    float* dst = static_cast<float*>(o.dst);
+    for (size_t i = first; i < o.n; i += stride) {
+        size_t row, c;
+        split_index(i, size_t(o.cols) / V, row, c);
+        c *= V;
+        const unsigned gate = unsigned(row) / unsigned(o.H), j = unsigned(row) % unsigned(o.H);
+        const size_t at = (size_t(4) * j + gate) * o.ld_in + c;
+        float s[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) s[e] = 0.f;
+        for (int z = 0; z < o.splits; ++z) {
+            const float* p = partial + size_t(z) * o.per + at;
+            if constexpr (V == 4) {
+                const floatx4 q = *reinterpret_cast<const floatx4*>(p);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] += q[e];
+            } else {
+                s[0] += p[0];
+            }
+        }
+        float* out = dst + row * size_t(o.cols) + c;
+#pragma unroll
+        for (int e = 0; e < V; ++e) out[e] = o.accumulate ? out[e] + o.scale * s[e] : o.scale * s[e];
+    }
+}
+
+// Blocks [first_block, first_block + blocks) of the grid walk an operation with a grid stride.  All of it is memory
+// traffic or launch latency: eight elements per thread in 16-byte accesses where the pitches allow (fp32 sequence of
+// 65536 x 1024 from fp16 rows: 2.1 TB/s with one element per thread and 64-bit index arithmetic).
+__global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
+    int which = 0;
+    while (which + 1 < list.count && blockIdx.x >= list.op[which + 1].first_block) ++which;
+    if (list.count > 0) {
+        const LayoutOp& o = list.op[which];
+        const size_t stride = size_t(o.blocks) * kT;
+        const size_t first = size_t(blockIdx.x - o.first_block) * kT + threadIdx.x;
+        if (o.kind == LayoutOp::kFill) {
+            if (o.vec == 4) {
+                uint4* p = static_cast<uint4*>(o.dst);
+                for (size_t i = first; i < o.n; i += stride) p[i] = uint4{o.word, o.word, o.word, o.word};
+            } else {
+                unsigned* p = static_cast<unsigned*>(o.dst);
+                for (size_t i = first; i < o.n; i += stride) p[i] = o.word;
+            }
+        } else if (o.kind == LayoutOp::kToHalf || o.kind == LayoutOp::kToFloat) {
+            if (o.vec == 8) op_convert<8>(o, first, stride);
+            else op_convert<1>(o, first, stride);
+        } else if (o.kind == LayoutOp::kUnpad) {
+            if (o.vec == 8) op_unpad<8>(o, first, stride);
+            else op_unpad<1>(o, first, stride);
+        } else if (o.kind == LayoutOp::kToExchange) {
+            // item i = eight halfs of one lane: [16-row tile][32-wide k-step][lane] (recurrent.hip, xch_offset)
+            const unsigned nks = unsigned(o.ld_out) / 32;
+            for (size_t i = first; i < o.n; i += stride) {
+                const unsigned lane = unsigned(i) % 64, ks = (unsigned(i) / 64) % nks, tile = unsigned(i) / 64 / nks;
+                const size_t r = size_t(tile) * 16 + lane % 16;
+                const unsigned k = ks * 32 + (lane / 16) * 8;
+                half8 h{};
+                if (o.src != nullptr && r < o.rows) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (k + e < unsigned(o.cols)) { float one[1]; load_floats<1>(o.src, r * o.cols + k + e, o.in_f32, one); h[e] = (half_t)one[0]; }
+                }
+                st_half8(static_cast<half_t*>(o.dst) + i * 8, h);
+            }
+        } else if (o.kind == LayoutOp::kReduceDw) {
+            if (o.vec == 4) op_reduce_dw<4>(o, first, stride);
+            else op_reduce_dw<1>(o, first, stride);
+        } else if (o.kind == LayoutOp::kReduceDb) {
+            const float* part = static_cast<const float*>(o.src);
+            float *db_ih = static_cast<float*>(o.dst), *db_hh = static_cast<float*>(o.dst2);
+            for (size_t q = first; q < o.n; q += stride) {
+                const int row = torch_row(int(q), o.H);
+                if (row < 0) continue;
+                float s = 0.f;
+                for (int g = 0; g < o.splits; ++g) s += part[size_t(g) * o.n + q];
+                s *= o.scale;
+                if (db_ih) db_ih[row] = o.accumulate ? db_ih[row] + s : s;
+                if (db_hh && db_hh != db_ih) db_hh[row] = o.accumulate ? db_hh[row] + s : s;
+            }
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0 && list.stamps) {
+        const long long now = wall_clock64();
+        if (list.stamp >= 0) list.stamps[list.stamp] = now;
+        if (list.publish) {   // (what earlier launches left: this launch writes neither the status nor the other stamps)
+            __hip_atomic_store(&list.publish->status, *list.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            for (int i = 0; i < kStampCount; ++i)
+                __hip_atomic_store(&list.publish->stamps[i], i == list.stamp ? now : list.stamps[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 }
@@ -279,105 +344,104 @@ hipError_t pack_bias(const Dims& d, const float* b_ih, const float* b_hh, float*
     return hipGetLastError();
 }
 
-hipError_t convert_pad(const void* in, int in_f32, size_t rows, int cols, size_t ld_in, float scale,
-                       half_t* out, size_t rows_out, size_t ld_out, hipStream_t s) {
-    const size_t n = rows_out * ld_out;
-    if (n == 0) return hipSuccess;
-    if (in_f32)
-        hipLaunchKernelGGL(convert_pad_kernel<float>, dim3(grid_for(n)), dim3(kT), 0, s,
-                           static_cast<const float*>(in), rows, cols, ld_in, scale, out, rows_out, ld_out);
-    else
-        hipLaunchKernelGGL(convert_pad_kernel<half_t>, dim3(grid_for(n)), dim3(kT), 0, s,
-                           static_cast<const half_t*>(in), rows, cols, ld_in, scale, out, rows_out, ld_out);
-    return hipGetLastError();
+namespace {
+
+// a work item's elements: 8 where rows and bases allow 16-byte accesses
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+
+void OpList::fill(void* p, size_t bytes, unsigned w) {
+    if (bytes == 0) return;
+    LayoutOp& o = op[count++];
+    o.kind = LayoutOp::kFill; o.dst = p; o.word = w;
+    o.vec = (aligned16(p) && bytes % 16 == 0) ? 4 : 1;
+    o.n = bytes / 4 / o.vec;
 }
 
-hipError_t convert_pad_f32(const void* in, int in_f32, size_t rows, int cols, float scale, float* out,
-                           size_t ld_out, hipStream_t s) {
-    const size_t n = rows * ld_out;
-    if (n == 0) return hipSuccess;
-    if (in_f32)
-        hipLaunchKernelGGL(convert_pad_f32_kernel<float>, dim3(grid_for(n)), dim3(kT), 0, s,
-                           static_cast<const float*>(in), rows, cols, scale, out, ld_out);
-    else
-        hipLaunchKernelGGL(convert_pad_f32_kernel<half_t>, dim3(grid_for(n)), dim3(kT), 0, s,
-                           static_cast<const half_t*>(in), rows, cols, scale, out, ld_out);
+void OpList::to_half(const void* in, int in_f32, size_t rows, int cols, size_t ld_in, float scale, half_t* out, size_t rows_out, size_t ld_out) {
+    if (rows_out * ld_out == 0) return;
+    LayoutOp& o = op[count++];
+    o.kind = LayoutOp::kToHalf; o.in_f32 = in_f32; o.dst = out; o.src = in;
+    o.vec = (ld_out % 8 == 0 && aligned16(out)) ? 8 : 1;
+    o.n = rows_out * ld_out / o.vec;
+    o.rows = rows; o.cols = cols; o.ld_in = ld_in; o.ld_out = ld_out; o.scale = scale;
+}
+
+void OpList::to_float(const void* in, int in_f32, size_t rows, int cols, float scale, float* out, size_t ld_out) {
+    if (rows * ld_out == 0) return;
+    LayoutOp& o = op[count++];
+    o.kind = LayoutOp::kToFloat; o.in_f32 = in_f32; o.dst = out; o.src = in;
+    o.vec = (ld_out % 8 == 0 && aligned16(out)) ? 8 : 1;
+    o.n = rows * ld_out / o.vec;
+    o.rows = rows; o.cols = cols; o.ld_in = size_t(cols); o.ld_out = ld_out; o.scale = scale;
+}
+
+void OpList::unpad(const void* in, int in_f32, size_t ld_in, size_t rows, int cols, float scale, void* out, int out_f32,
+                   size_t rows_per_block, size_t block_stride) {
+    if (out == nullptr || rows * size_t(cols) == 0) return;
+    LayoutOp& o = op[count++];
+    o.kind = LayoutOp::kUnpad; o.in_f32 = in_f32; o.out_f32 = out_f32; o.dst = out; o.src = in;
+    o.vec = (cols % 8 == 0 && ld_in % 8 == 0 && aligned16(in) && aligned16(out)) ? 8 : 1;
+    o.n = rows * size_t(cols) / o.vec;
+    o.rows = rows; o.cols = cols; o.ld_in = ld_in; o.scale = scale;
+    o.rows_per_block = rows_per_block >= rows ? 0 : rows_per_block; o.block_stride = block_stride;
+}
+
+void OpList::to_exchange(const void* in, int in_f32, size_t rows, int cols, int kcols, half_t* slot) {
+    LayoutOp& o = op[count++];
+    o.kind = LayoutOp::kToExchange; o.in_f32 = in_f32; o.dst = slot; o.src = in;
+    o.n = exchange_slot_halfs(int(rows), kcols) / 8;
+    o.rows = rows; o.cols = cols; o.ld_out = size_t(kcols);
+}
+
+void OpList::reduce_dw(const Dims& d, const float* partial, int splits, size_t ld, int col0, int out_cols, float scale,
+                       bool accumulate, float* dst) {
+    if (dst == nullptr || out_cols <= 0) return;
+    LayoutOp& o = op[count++];
+    o.kind = LayoutOp::kReduceDw; o.src = partial + col0; o.dst = dst;
+    o.vec = (out_cols % 4 == 0 && ld % 4 == 0 && col0 % 4 == 0 && aligned16(dst)) ? 4 : 1;
+    o.n = size_t(4) * d.H * out_cols / o.vec;
+    o.cols = out_cols; o.ld_in = ld; o.splits = splits; o.per = size_t(4) * d.Hp * ld; o.H = d.H; o.scale = scale;
+    o.accumulate = accumulate ? 1 : 0;
+}
+
+void OpList::reduce_db(const Dims& d, const float* db_part, int ng, float scale, bool accumulate, float* db_ih, float* db_hh) {
+    if (!db_ih && !db_hh) return;
+    LayoutOp& o = op[count++];
+    o.kind = LayoutOp::kReduceDb; o.src = db_part; o.dst = db_ih; o.dst2 = db_hh;
+    o.n = size_t(4) * d.Hp; o.splits = ng; o.H = d.H; o.scale = scale; o.accumulate = accumulate ? 1 : 0;
+}
+
+hipError_t run_ops(OpList& list, hipStream_t s) {
+    if (list.count > kMaxOps) return hipErrorInvalidValue;
+    if (list.count <= 0 && !list.publish) return hipSuccess;
+    unsigned total = 0;
+    for (int i = 0; i < list.count; ++i) {
+        LayoutOp& o = list.op[i];
+        size_t blocks = (o.n + kT - 1) / kT;
+        if (blocks > 4096) blocks = 4096;   // (more work than that is walked with the grid stride)
+        if (blocks < 1) blocks = 1;
+        o.first_block = total;
+        o.blocks = unsigned(blocks);
+        total += o.blocks;
+    }
+    hipLaunchKernelGGL(layout_ops_kernel, dim3(total ? total : 1), dim3(kT), 0, s, list);
     return hipGetLastError();
 }
 
 hipError_t gather_from_half(const half_t* in, size_t ld_in, size_t rows, int cols, void* out, int out_f32,
                             size_t rows_per_block, size_t block_stride, hipStream_t s) {
-    const size_t n = rows * size_t(cols);
-    if (n == 0 || out == nullptr) return hipSuccess;
-    // unpadded fp16 rows that are contiguous on both sides: a flat vector copy
-    if (!out_f32 && size_t(cols) == ld_in && rows_per_block >= rows && (n * sizeof(half_t)) % 16 == 0 &&
-        reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
-        const size_t n16 = n * sizeof(half_t) / 16;
-        size_t blocks = (n16 + kT - 1) / kT;
-        if (blocks > 8192) blocks = 8192;
-        hipLaunchKernelGGL(copy16_kernel, dim3(unsigned(blocks)), dim3(kT), 0, s, reinterpret_cast<const uint4*>(in),
-                           static_cast<uint4*>(out), n16);
-        return hipGetLastError();
-    }
-    if (out_f32)
-        hipLaunchKernelGGL((unpad_kernel<half_t, float>), dim3(grid_for(n)), dim3(kT), 0, s, in, ld_in, rows,
-                           cols, 1.f, static_cast<float*>(out), rows_per_block, block_stride);
-    else
-        hipLaunchKernelGGL((unpad_kernel<half_t, half_t>), dim3(grid_for(n)), dim3(kT), 0, s, in, ld_in, rows,
-                           cols, 1.f, static_cast<half_t*>(out), rows_per_block, block_stride);
-    return hipGetLastError();
+    OpList list;
+    list.unpad(in, 0, ld_in, rows, cols, 1.f, out, out_f32, rows_per_block, block_stride);
+    return run_ops(list, s);
 }
 
-hipError_t gather_from_float(const float* in, size_t ld_in, size_t rows, int cols, float scale, void* out,
-                             int out_f32, size_t rows_per_block, size_t block_stride, hipStream_t s) {
-    const size_t n = rows * size_t(cols);
-    if (n == 0 || out == nullptr) return hipSuccess;
-    if (out_f32)
-        hipLaunchKernelGGL((unpad_kernel<float, float>), dim3(grid_for(n)), dim3(kT), 0, s, in, ld_in, rows,
-                           cols, scale, static_cast<float*>(out), rows_per_block, block_stride);
-    else
-        hipLaunchKernelGGL((unpad_kernel<float, half_t>), dim3(grid_for(n)), dim3(kT), 0, s, in, ld_in, rows,
-                           cols, scale, static_cast<half_t*>(out), rows_per_block, block_stride);
-    return hipGetLastError();
-}
-
-hipError_t unpad_from_half(const half_t* in, size_t ld_in, size_t rows, int cols, void* out, int out_f32,
-                           hipStream_t s) {
-    return gather_from_half(in, ld_in, rows, cols, out, out_f32, rows ? rows : 1, 0, s);
-}
-
-hipError_t unpad_from_float(const float* in, size_t ld_in, size_t rows, int cols, float scale, void* out,
-                            int out_f32, hipStream_t s) {
-    return gather_from_float(in, ld_in, rows, cols, scale, out, out_f32, rows ? rows : 1, 0, s);
-}
-
-hipError_t transpose_pad(const void* in, int in_f32, size_t rows, int cols, size_t ld_in, half_t* out,
-                         int cols_out, size_t ld_out, hipStream_t s) {
-    if (cols_out == 0 || ld_out == 0) return hipSuccess;
-    dim3 grid(unsigned(ceil_div(ld_out, 64)), unsigned(ceil_div(size_t(cols_out), 64)));
-    if (in_f32)
-        hipLaunchKernelGGL(transpose_pad_kernel<float>, grid, dim3(kT), 0, s, static_cast<const float*>(in),
-                           rows, cols, ld_in, out, cols_out, ld_out);
-    else
-        hipLaunchKernelGGL(transpose_pad_kernel<half_t>, grid, dim3(kT), 0, s, static_cast<const half_t*>(in),
-                           rows, cols, ld_in, out, cols_out, ld_out);
-    return hipGetLastError();
-}
-
-hipError_t reduce_dw(const Dims& d, const float* partial, int splits, size_t ld, int col0, int ncols, int out_cols,
-                     float scale, bool accumulate, float* dst, hipStream_t s) {
-    if (dst == nullptr) return hipSuccess;
-    const size_t n = size_t(4) * d.Hp * ncols;
-    hipLaunchKernelGGL(reduce_dw_kernel, dim3(grid_for(n)), dim3(kT), 0, s, d, partial, splits, ld, col0, ncols,
-                       out_cols, scale, int(accumulate), dst);
-    return hipGetLastError();
-}
-
-hipError_t reduce_db(const Dims& d, const float* db_part, int ng, float scale, bool accumulate, float* db_ih,
-                     float* db_hh, hipStream_t s) {
-    hipLaunchKernelGGL(reduce_db_kernel, dim3(grid_for(size_t(4) * d.Hp)), dim3(kT), 0, s, d, db_part, ng,
-                       scale, int(accumulate), db_ih, db_hh);
-    return hipGetLastError();
+hipError_t gather_from_float(const float* in, size_t ld_in, size_t rows, int cols, float scale, void* out, int out_f32,
+                             size_t rows_per_block, size_t block_stride, hipStream_t s) {
+    OpList list;
+    list.unpad(in, 1, ld_in, rows, cols, scale, out, out_f32, rows_per_block, block_stride);
+    return run_ops(list, s);
 }
 
 __global__ void reduce_partials_kernel(const float* __restrict__ partial, int splits, size_t per, int rows, int cols,
@@ -399,23 +463,38 @@ hipError_t reduce_partials(const float* partial, int splits, size_t per, int row
 
 // Position-weighted sum of the 16-bit units of a buffer, added to *out: any changed, moved or swapped element
 // changes the sum (up to a 2^-64 accident); the order of the additions does not matter, so atomics may be used.
-__global__ void checksum_kernel(const unsigned short* __restrict__ p, size_t n, u64 salt, u64* out) {
+// Eight units per thread and 16-byte load (one 2-byte load per thread and iteration read 16 MiB at 160 GB/s, 104 us).
+__device__ __forceinline__ u64 checksum_unit(unsigned v16, size_t i, u64 salt) {
+    u64 v = (u64(v16) + 1u) * (2 * (i + salt) + 1) * 0x9E3779B97F4A7C15ull;
+    v ^= v >> 29;
+    return v * 0xBF58476D1CE4E5B9ull;
+}
+__global__ __launch_bounds__(kT) void checksum_kernel(const unsigned short* __restrict__ p, size_t n, u64 salt, u64* out) {
+    __shared__ u64 wave_sum[kT / 64];
     u64 acc = 0;
-    const size_t stride = size_t(gridDim.x) * blockDim.x;
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-        u64 v = (u64(p[i]) + 1u) * (2 * (i + salt) + 1) * 0x9E3779B97F4A7C15ull;
-        v ^= v >> 29;
-        acc += v * 0xBF58476D1CE4E5B9ull;
+    const size_t stride = size_t(gridDim.x) * blockDim.x, first = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const size_t n8 = (reinterpret_cast<uintptr_t>(p) % 16 == 0) ? n / 8 : 0;
+    for (size_t i = first; i < n8; i += stride) {
+        const uint4 q = reinterpret_cast<const uint4*>(p)[i];
+        const unsigned w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc += checksum_unit((w[e / 2] >> (16 * (e % 2))) & 0xffffu, i * 8 + e, salt);
     }
+    for (size_t i = n8 * 8 + first; i < n; i += stride) acc += checksum_unit(p[i], i, salt);
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if (threadIdx.x % 64 == 0 && acc != 0) atomicAdd(reinterpret_cast<unsigned long long*>(out), acc);
+    if (threadIdx.x % 64 == 0) wave_sum[threadIdx.x / 64] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kT / 64; ++w) acc += wave_sum[w];
+        atomicAdd(reinterpret_cast<unsigned long long*>(out), acc);
+    }
 }
 
 hipError_t checksum_add(const void* p, size_t bytes, u64 salt, u64* out, hipStream_t s) {
     if (p == nullptr || bytes < 2) return hipSuccess;
     const size_t n = bytes / 2;   // every tensor of this library is made of 2- or 4-byte elements
-    int blocks = grid_for(n);
-    if (blocks > 2048) blocks = 2048;
+    int blocks = grid_for(ceil_div(n, 8));
+    if (blocks > 512) blocks = 512;
     hipLaunchKernelGGL(checksum_kernel, dim3(blocks), dim3(kT), 0, s, static_cast<const unsigned short*>(p), n, salt, out);
     return hipGetLastError();
 }
@@ -426,17 +505,6 @@ hipError_t fill_words(void* p, size_t bytes, unsigned value, hipStream_t s) {
     int blocks = grid_for(words);
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(fill_words_kernel, dim3(blocks), dim3(kT), 0, s, static_cast<unsigned*>(p), words, value);
-    return hipGetLastError();
-}
-
-hipError_t run_prep(const PrepList& list, hipStream_t s) {
-    if (list.count <= 0) return hipSuccess;
-    size_t most = 0;
-    for (int i = 0; i < list.count; ++i) most = list.op[i].n > most ? list.op[i].n : most;
-    size_t blocks = (most + kT - 1) / kT;
-    if (blocks > 256) blocks = 256;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(prep_kernel, dim3(unsigned(blocks), unsigned(list.count)), dim3(kT), 0, s, list);
     return hipGetLastError();
 }
 

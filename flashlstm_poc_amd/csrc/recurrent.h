@@ -20,7 +20,9 @@ struct RecLayout {
     int persistent;  // 1: one launch walks all steps, 0: one launch per step
     int resident;    // 1: weight fragments live in registers for the whole launch
     int grid;        // workgroups per launch
-    int cooperative; // host side: 1 = persistent launches go through hipLaunchCooperativeKernel (set by the plan)
+    int cooperative; // host side: 1 = persistent launches go through hipLaunchCooperativeKernel (set by the plan), 0 = through
+                     // launch_persistent's own gate
+    int num_cus;     // of the device the layout was made for
     int rot_div;     // k-step rotation (rec_kstep_rotation): slices rot_div apart run on the same XCD
     int two_d;       // backward, 2048 hidden units: workgroups split the product over output columns AND the contraction
                      // (32 column slices x kq contraction slices, partial sums exchanged inside an XCD); nt, jb, nh
@@ -52,6 +54,7 @@ struct RecFwdArgs {
     int* status;         // 0 ok, 1 spin limit hit, 2 workgroup not on the expected XCD
     int B, Hp, T;
     int t0, t1;          // steps [t0, t1) of the sequence are run by this call (state and ring carry over)
+    long long* stamps;   // optional [2]: when the pass's first launch started and its last one ended (workgroup of group 0, slice 0)
     int spin_limit;      // reloads of a fragment chunk that still shows the 'unwritten' pattern before giving up
     long long spin_ticks;   // the same bound as time: ticks of the device's constant-rate wall clock
     long long* prof;     // optional [8] cycle counters of workgroup 0 per phase (null = off)
@@ -84,6 +87,7 @@ struct RecBwdArgs {
                          // every array keeps its full-batch strides, the rings are indexed by the row in the batch)
     float dy_scale;      // factor applied to dY on load (the loss scale, or 1 when dY is pre-scaled)
     int t_hi, t_lo;      // steps t_hi down to t_lo are run by this call; t_lo = -1 adds the closing dh0 product
+    long long* stamp_end;   // optional: when the last launch of the pass ended (workgroup of group 0, slice 0)
     int spin_limit;
     long long spin_ticks;
     long long* prof;     // optional [8] cycle counters of workgroup 0 per phase (null = off)
@@ -167,12 +171,13 @@ int rec_bwd_ring_rows(const RecLayout& L, int B);
 
 // Halfs in one slot of an exchange ring for a [rows][cols] operand (rows padded to 32).
 size_t exchange_slot_halfs(int rows, int cols);
-// Row-major [rows][cols] (cols % 32 == 0) -> fragment-major exchange layout.
-hipError_t to_exchange_layout(const half_t* in, int rows, int cols, size_t ld, half_t* out, hipStream_t s);
-
 // Number of k-steps (32 wide) every wave holds for a layout (sizes the fragment arrays).
 int rec_fwd_ks(const RecLayout& L, int Hp);
 int rec_bwd_ks(const RecLayout& L, int Hp);
+
+// To be called once a stream that persistent launches went to has been waited for: launches on other streams no longer
+// need to be ordered behind it (launch_persistent).
+void persistent_stream_idle(hipStream_t stream);
 
 // Runs steps [t0, t1). Persistent layouts use one launch; otherwise one launch per step.
 hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs = nullptr);

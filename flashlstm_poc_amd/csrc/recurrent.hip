@@ -34,7 +34,9 @@
 //  * Fallback.  The same kernels launched once per step (no waits, kernel boundaries order
 //    memory) serve shapes whose weights do not fit on chip, and are the safe path after a failed
 //    persistent launch.
+#include <atomic>
 #include <cstring>
+#include <mutex>
 #include <type_traits>
 
 #include "recurrent.h"
@@ -925,6 +927,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
             if (rb_count == 2 && row_used && b2 < p.B) ld_f32_now(p.C + (size_t(t_begin) * p.B + b2) * p.Hp + j, creg2[ph]);
         }
     }
+    if (p.stamps && t_begin == p.t0 && hs == 0 && g == 0 && tid == 0) p.stamps[0] = wall_clock64();
     __syncthreads();
     loads_landed();
     clk.start();
@@ -1044,6 +1047,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
         }
     }
     if constexpr (DS) first_request.leave(p.delay_hint);
+    if (p.stamps && hs == 0 && g == 0 && tid == 0) p.stamps[1] = wall_clock64();
     clk.flush();
 }
 
@@ -1149,6 +1153,7 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
             creg[tl] = v[0];
         }
     }
+    if (p.stamps && t_begin == p.t0 && hs == 0 && g == 0 && tid == 0) p.stamps[0] = wall_clock64();
     request_xp(t_begin, g, std::integral_constant<int, 0>{});
     __syncthreads();
     loads_landed();
@@ -1330,6 +1335,7 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
         }
     }
     clk.lap(2);
+    if (p.stamps && hs == 0 && g == 0 && tid == 0) p.stamps[1] = wall_clock64();
     clk.flush();
 }
 
@@ -1579,6 +1585,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
             if constexpr (MT == 1 && GPR == 8) __syncthreads();   // (waves without cells to update: as in the forward kernel)
         }
     }
+    if (p.stamp_end && hs == 0 && g == 0 && tid == 0) *p.stamp_end = wall_clock64();
     clk.flush();
     // single-step launches leave dc in memory for the next launch
     if (dc_in_regs && t_last >= 0) {
@@ -2016,6 +2023,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd2d_kernel(RecBwdArgs p, RecLa
         // together, as in the forward kernel)
         if constexpr (MT == 1) __syncthreads();
     }
+    if (p.stamp_end && s == 0 && q == 0 && g == 0 && tid == 0) *p.stamp_end = wall_clock64();
     clk.flush();
     if (t_last >= 0) {   // a launch that stops before the closing pass leaves dc in memory for the next one
 #pragma unroll
@@ -2045,53 +2053,80 @@ __global__ __launch_bounds__(kThreads) void rec_bwd2d_kernel(RecBwdArgs p, RecLa
     }
 }
 
-// rows x cols row-major (ld) -> fragment-major exchange layout (one thread per pair of halfs)
-__global__ void to_exchange_layout_kernel(const half_t* __restrict__ in, int rows, int cols, size_t ld,
-                                          half_t* __restrict__ out, int nks) {
-    const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const size_t pairs = size_t(rows) * (cols / 2);
-    if (idx >= pairs) return;
-    const int r = int(idx / (cols / 2)), k = int(idx % (cols / 2)) * 2;
-    *reinterpret_cast<unsigned*>(out + xch_offset(r, k, nks)) = *reinterpret_cast<const unsigned*>(in + size_t(r) * ld + k);
-}
-
-// (set before every launch: the call is cheap, needs no process-wide flag and holds for whichever device is current)
+// Per kernel and device, once: the dynamic LDS limit is raised and the workgroups of it a CU can hold are looked up.
+constexpr int kMaxDevices = 64;
 template <typename K>
-hipError_t raise_lds(K kernel, size_t bytes) {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
+hipError_t prepare_kernel(K kernel, size_t lds, int threads, std::atomic<int>* per_cu /*[kMaxDevices]*/, int* device) {
+    hipError_t e = hipGetDevice(device);
+    if (e != hipSuccess) return e;
+    if (*device < 0 || *device >= kMaxDevices) return hipErrorInvalidDevice;
+    if (per_cu[*device].load(std::memory_order_acquire) != 0) return hipSuccess;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    if (e != hipSuccess) return e;
+    int n = 0;
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds);
+    if (e != hipSuccess) return e;
+    per_cu[*device].store(n > 0 ? n : -1, std::memory_order_release);
+    return hipSuccess;
 }
 
-// A persistent launch needs all its workgroups running at once: they wait for each other's data.  The cooperative
-// launch makes that a condition of the launch (the runtime refuses a grid that cannot be co-resident and does not
-// run it beside another kernel); where the runtime has no cooperative launch the ordinary one is used, and the
-// bounded waits inside the kernel cover the case that some workgroup is late.
+// A persistent launch needs all its workgroups running at once: they wait for each other's data.  Two of them side by
+// side on one device (two plans, two streams) could each get half of the CUs and wait for the rest, so launches to
+// different streams are put one behind the other here; launches to one stream are in order anyway.  Only when a launch
+// meets another stream's pass in flight does that cost anything (an event).  hipLaunchCooperativeKernel gives the same
+// guarantee by sending every such kernel through a queue of its own, with a signal from the caller's queue to it and one
+// back: 20 us per launch, 40 of the 400 us of a training pass over 64 steps of 256 units.
+struct PersistentGate {
+    std::mutex mutex;
+    hipStream_t stream = nullptr;   // where the last launch went
+    bool in_flight = false;         // ... and it has not been waited for yet
+    hipEvent_t event = nullptr;
+};
+PersistentGate g_gate[kMaxDevices];
+
+// A grid that cannot be co-resident is exactly what a persistent launch must not be given: nothing is launched then
+// (hipErrorCooperativeLaunchTooLarge) and the caller runs the pass step-wise.  Workgroups of OTHER kernels can still keep
+// some of the grid waiting; the bounded waits inside the kernels cover that.
 template <typename K, typename A>
 hipError_t launch_persistent(K kernel, int grid, size_t lds, hipStream_t stream, A a, RecLayout L, int t_a, int t_b,
-                             int ks_wave, int threads = kThreads) {
+                             int ks_wave, int workgroups_per_cu, int device, int threads = kThreads) {
     if (L.cooperative) {
         void* params[] = {&a, &L, &t_a, &t_b, &ks_wave};
         hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(grid), dim3(threads), params,
                                                   unsigned(lds), stream);
         if (e == hipSuccess) return hipSuccess;
         (void)hipGetLastError();
-        // A grid the runtime says cannot be co-resident is exactly what a persistent launch must not be given: nothing
-        // is launched, and the caller runs the pass step-wise.  Any other refusal (no cooperative launch on this
-        // runtime) falls back to the plain launch, whose bounded waits cover a late workgroup.
         if (e == hipErrorCooperativeLaunchTooLarge) return e;
+        // (any other refusal: no cooperative launch on this runtime)
+    }
+    if (workgroups_per_cu < 1 || grid > workgroups_per_cu * L.num_cus) return hipErrorCooperativeLaunchTooLarge;
+    PersistentGate& gate = g_gate[device];
+    std::lock_guard<std::mutex> lock(gate.mutex);
+    if (gate.in_flight && gate.stream != stream) {
+        hipError_t e = hipSuccess;
+        if (!gate.event) e = hipEventCreateWithFlags(&gate.event, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(gate.event, gate.stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(stream, gate.event, 0);
+        if (e != hipSuccess) {   // (the other stream is gone: nothing of it can be running once the device is idle)
+            (void)hipGetLastError();
+            e = hipDeviceSynchronize();
+            if (e != hipSuccess) return e;
+        }
     }
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, a, L, t_a, t_b, ks_wave);
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) { gate.stream = stream; gate.in_flight = true; }
+    return e;
 }
 
 }  // namespace
 
-hipError_t to_exchange_layout(const half_t* in, int rows, int cols, size_t ld, half_t* out, hipStream_t s) {
-    if (rows <= 0 || cols <= 0) return hipSuccess;
-    if (cols % 32 != 0) return hipErrorInvalidValue;
-    const size_t pairs = size_t(rows) * (cols / 2);
-    hipLaunchKernelGGL(to_exchange_layout_kernel, dim3(unsigned((pairs + 255) / 256)), dim3(256), 0, s, in, rows, cols,
-                       ld, out, cols / 32);
-    return hipGetLastError();
+void persistent_stream_idle(hipStream_t stream) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return;
+    PersistentGate& gate = g_gate[device];
+    std::lock_guard<std::mutex> lock(gate.mutex);
+    if (gate.stream == stream) gate.in_flight = false;
 }
 
 size_t exchange_slot_halfs(int rows, int cols) { return round_up(size_t(rows), 32) * size_t(cols); }
@@ -2151,6 +2186,7 @@ static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_s
 
 RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt, int waves) {
     RecLayout L{};
+    L.num_cus = num_cus;
     bool fits = true;
     if (Hp <= 1024) L.nt = 8;
     else if (Hp <= 2048) L.nt = 4;
@@ -2163,6 +2199,7 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
 
 RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt, int two_d) {
     RecLayout L{};
+    L.num_cus = num_cus;
     bool fits = true;
     if (Hp <= 1024) L.nt = 2;
     else if (Hp <= 2048) L.nt = 1;
@@ -2310,10 +2347,12 @@ static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
     auto kernel = rec_fwd_kernel<NT, KS, RES, MT, DS, DEEP>;
     if (L.nw != NW) return hipErrorInvalidValue;   // (the weight fragments are packed for L.nw waves)
     const size_t lds = size_t(2) * NW * kRows * (16 * NT + kPartPad) * sizeof(float);
-    hipError_t e = raise_lds(kernel, lds);
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
     if (e != hipSuccess) return e;
     const int ks_wave = rec_fwd_ks(L, a.Hp);
-    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t0, a.t1, ks_wave, NW * kWave);
+    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
                         [&]() -> hipError_t {
                             for (int t = a.t0; t < a.t1; ++t) {
@@ -2331,10 +2370,12 @@ static hipError_t run_fwd_il(const RecLayout& L, const RecFwdArgs& a, hipStream_
     auto kernel = rec_fwd_il_kernel<NT, KS, DS>;
     if (L.nw != NW || L.nt != NT || L.mt != 2 || !L.resident) return hipErrorInvalidValue;
     const size_t lds = size_t(2) * NW * 16 * (16 * NT + kPartPad) * sizeof(float);
-    hipError_t e = raise_lds(kernel, lds);
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
     if (e != hipSuccess) return e;
     const int ks_wave = rec_fwd_ks(L, a.Hp);
-    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t0, a.t1, ks_wave, NW * kWave);
+    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
                         [&]() -> hipError_t {
                             for (int t = a.t0; t < a.t1; ++t) {
@@ -2393,10 +2434,12 @@ static hipError_t run_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
     if (L.nw != NW) return hipErrorInvalidValue;   // (the weight fragments are packed for L.nw waves)
     static_assert(size_t(2) * NW * kRows * (16 * NT + kPartPad) >= size_t(NW * kWave) * 8 * NT, "db reduction reuses the partial-sum area");
     const size_t lds = size_t(2) * NW * kRows * (16 * NT + kPartPad) * sizeof(float) + size_t(NW) * KL * NT * kWave * sizeof(half8);
-    hipError_t e = raise_lds(kernel, lds);
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
     if (e != hipSuccess) return e;
     const int ks_wave = rec_bwd_ks(L, a.Hp);
-    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, ks_wave, NW * kWave);
+    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, ks_wave, per_cu[device].load(), device, NW * kWave);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t_hi, a.t_lo, a.t_hi - a.t_lo + 1,
                         stream, [&]() -> hipError_t {
                             for (int t = a.t_hi; t >= a.t_lo; --t) {
@@ -2418,9 +2461,11 @@ static hipError_t run_bwd2d(const RecLayout& L, const RecBwdArgs& a, hipStream_t
     auto kernel = rec_bwd2d_kernel<MT, KQ, NM, KS, LOCAL>;
     constexpr int KL = (KS == 16) ? 5 : 0;   // k-steps per wave whose weights live in LDS (as in the kernel)
     const size_t lds = size_t(2) * 4 * kRows * (64 + kPartPad) * sizeof(float) + size_t(4) * KL * 4 * kWave * sizeof(half8);
-    hipError_t e = raise_lds(kernel, lds);
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, lds, kThreads, per_cu, &device);
     if (e != hipSuccess) return e;
-    return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0);
+    return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
 }
 
 hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {

@@ -41,17 +41,17 @@ int flstm_core_create(size_t batch, size_t input_size, size_t hidden_size, flstm
 int flstm_core_destroy(flstm_core_plan* plan);
 
 /* Options: "stepwise" (1 = one launch per time step instead of the persistent kernels),
- * "proj_chunk" (time steps per input-projection GEMM, <=0 = whole sequence; results do not depend
- * on it), "spin_limit" / "spin_ms" (reloads of a not-yet-written operand, and milliseconds spent on them, before a
+ * "proj_chunk" (accepted for the reference's interface; the input projection is one product whatever it says), "spin_limit" / "spin_ms" (reloads of a not-yet-written operand, and milliseconds spent on them, before a
  * waiting workgroup of a persistent launch gives up; default 2^30 reloads / 250 ms; 0 reloads = give up at the first
  * operand found unwritten), "dw_splits" (split-K slices of
  * the weight-gradient GEMM, 0 = automatic), "accumulate_grads" (1 = the backward pass adds dW_ih, dW_hh, db_ih
  * and db_hh to what the caller's buffers hold instead of overwriting them: a sequence processed as several
  * consecutive segments, last segment first, each segment's dh0 / dc0 fed to the next call as d_hn / d_cn),
  * "row_tiles_fwd" / "row_tiles_bwd" (16-row tiles per row block of that recurrence: 1, 2, or 0 = automatic),
- * "cooperative" (1: persistent launches are cooperative launches, so that co-residency of the whole grid is a
- * condition of the launch; 0: plain launches; default 1, but 0 when a rocprofiler-sdk tool is attached -- a process
- * that made a cooperative launch faults inside that tool at exit -- and FLASHLSTM_COOPERATIVE_LAUNCH overrides),
+ * "cooperative" (0, the default: persistent launches are plain launches whose grid is checked to be co-resident, and
+ * launches to different streams of a device are put one behind the other; 1: hipLaunchCooperativeKernel, which costs
+ * 20 us more per launch -- and a process that made a cooperative launch faults inside an attached rocprofiler-sdk tool
+ * at exit; FLASHLSTM_COOPERATIVE_LAUNCH sets the default),
  * "step_graphs" (1, the default: where a pass runs as one launch per time step -- weights that do not fit on chip, a
  * demoted direction, "stepwise" -- the launches of a range of steps are captured into a hipGraph on first use and
  * replayed afterwards, when the stream allows capture; 0 = plain launches; FLASHLSTM_STEP_GRAPHS sets the default),
