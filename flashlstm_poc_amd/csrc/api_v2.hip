@@ -40,6 +40,7 @@
 
 #include "../../include/flashlstm/lstm_core.h"
 #include "../../include/flashlstm_v2/lstm.hpp"
+#include "core_internal.h"
 #include "instrument.h"
 #include "pack.h"
 
@@ -82,18 +83,23 @@ struct Entry {
     Buf x_dev, y_dev, dy_dev, dx_dev, ck_h, ck_c;
     Buf carry_h, carry_c, carry_dh, carry_dc;   // fp32 (B, H): state / state gradient between windows
     Buf sum_dev;                                // one 64-bit checksum accumulator
+    unsigned long long* sum_host = nullptr;     // pinned: where it is copied to
     Buf starts;                                 // fp32 [window][h, c][B * H]: state at the start of each window
+    size_t held_is_within_budget = 0;           // the most these buffers have held that was found within the device's budget
     std::vector<char> start_known;              // which entries of `starts` hold the current sequence's states
     ForwardKey last;
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
-    std::vector<hipEvent_t> chunk_in, chunk_out;   // one pair per chunk of a streamed pass
-    void need_chunk_events(size_t n) {
-        while (chunk_in.size() < n) {
-            hipEvent_t a = nullptr, b = nullptr;
-            check(hipEventCreateWithFlags(&a, hipEventDisableTiming), "hipEventCreate");
-            check(hipEventCreateWithFlags(&b, hipEventDisableTiming), "hipEventCreate");
-            chunk_in.push_back(a);
-            chunk_out.push_back(b);
+    std::vector<hipEvent_t> chunk_in, dy_in, chunk_out;   // one of each per chunk of a streamed pass
+    std::vector<size_t> chunks;                    // first step of each chunk of the window in progress, and its end
+    size_t nchunks() const { return chunks.size() - 1; }
+    void cut_into_chunks(std::vector<size_t> starts) {
+        chunks = std::move(starts);
+        while (chunk_in.size() < nchunks()) {
+            for (std::vector<hipEvent_t>* list : {&dy_in, &chunk_out, &chunk_in}) {
+                hipEvent_t ev = nullptr;
+                check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
+                list->push_back(ev);
+            }
         }
     }
     size_t device_bytes() const {
@@ -109,9 +115,11 @@ struct Entry {
         for (Buf* b : {&x_dev, &y_dev, &dy_dev, &dx_dev, &ck_h, &ck_c, &carry_h, &carry_c, &carry_dh, &carry_dc, &starts,
                        &sum_dev})
             b->release();
+        if (sum_host) (void)hipHostFree(sum_host);
         if (ev_in) (void)hipEventDestroy(ev_in);
         if (ev_out) (void)hipEventDestroy(ev_out);
         for (hipEvent_t ev : chunk_in) (void)hipEventDestroy(ev);
+        for (hipEvent_t ev : dy_in) (void)hipEventDestroy(ev);
         for (hipEvent_t ev : chunk_out) (void)hipEventDestroy(ev);
     }
 };
@@ -124,6 +132,7 @@ constexpr size_t kMaxEntries = 4;
 // in bytes as well as in count: shapes other than the one in use are dropped, least recently used first, while
 // they hold more than FLASHLSTM_V2_REGISTRY_MB together (default: a quarter of the device's memory).
 void trim_registry() {
+    if (g_entries.size() < 2) return;
     size_t cap = 0;
     if (const char* v = getenv("FLASHLSTM_V2_REGISTRY_MB")) cap = size_t(atol(v) > 0 ? atol(v) : 0) << 20;
     if (cap == 0) {
@@ -154,6 +163,7 @@ Entry& entry_for(size_t B, size_t I, size_t H) {
     Entry& e = g_entries.front();
     e.B = B; e.I = I; e.H = H; e.device = dev;
     check_core(flstm_core_create(B, I, H, &e.plan), "flstm_core_create");
+    check(hipHostMalloc(reinterpret_cast<void**>(&e.sum_host), sizeof(*e.sum_host), hipHostMallocDefault), "hipHostMalloc");
     check(hipEventCreateWithFlags(&e.ev_in, hipEventDisableTiming), "hipEventCreate");
     check(hipEventCreateWithFlags(&e.ev_out, hipEventDisableTiming), "hipEventCreate");
     trim_registry();
@@ -178,8 +188,9 @@ unsigned long long fingerprint(const void* p, size_t bytes) {
 }
 
 // Checksum over the full contents of the device tensors a pass depends on (computed on the device, 8 bytes come
-// back): weights or initial states updated in place between forward and backward change it.
-unsigned long long device_print(Entry& e, hipStream_t s, const float* w_ih, const float* w_hh, const float* b_ih,
+// back): weights or initial states updated in place between forward and backward change it.  Enqueued here, readable
+// (read_device_print) once the stream has been waited for.
+void enqueue_device_print(Entry& e, hipStream_t s, const float* w_ih, const float* w_hh, const float* b_ih,
                                 const float* b_hh, const __half* h0, const __half* c0) {
     using flstm_hip::checksum_add;
     const size_t G = 4 * e.H;
@@ -192,11 +203,11 @@ unsigned long long device_print(Entry& e, hipStream_t s, const float* w_ih, cons
     check(checksum_add(b_hh, G * sizeof(float), 0x4000000000ull, acc, s), "checksum");
     check(checksum_add(h0, e.B * e.H * sizeof(half_t), 0x5000000000ull, acc, s), "checksum");
     check(checksum_add(c0, e.B * e.H * sizeof(half_t), 0x6000000000ull, acc, s), "checksum");
-    unsigned long long host = 0;
-    check(hipMemcpyAsync(&host, acc, sizeof(host), hipMemcpyDeviceToHost, s), "checksum");
-    check(hipStreamSynchronize(s), "checksum");
+    check(hipMemcpyAsync(e.sum_host, acc, sizeof(*e.sum_host), hipMemcpyDeviceToHost, s), "checksum");
+}
+unsigned long long read_device_print(const Entry& e, const float* b_ih, const float* b_hh, const __half* h0, const __half* c0) {
     // which of the optional tensors are present is part of the identity
-    return host ^ (b_ih ? 1ull : 0) ^ (b_hh ? 2ull : 0) ^ (h0 ? 4ull : 0) ^ (c0 ? 8ull : 0);
+    return *static_cast<volatile unsigned long long*>(e.sum_host) ^ (b_ih ? 1ull : 0) ^ (b_hh ? 2ull : 0) ^ (h0 ? 4ull : 0) ^ (c0 ? 8ull : 0);
 }
 
 void validate_common(size_t R, hipStream_t c, hipStream_t h2d, hipStream_t d2h) {
@@ -205,10 +216,32 @@ void validate_common(size_t R, hipStream_t c, hipStream_t h2d, hipStream_t d2h) 
         throw std::runtime_error("compute, h2d and d2h streams must be pairwise distinct");
 }
 
-size_t chunk_steps_for(size_t T) {
-    const char* v = getenv("FLASHLSTM_V2_CHUNK_STEPS");   // read per call: cheap, and tests switch it
-    const long env = v ? atol(v) : 64L;
-    return (env <= 0 || size_t(env) > T) ? T : size_t(env);
+// The steps at which the chunks of a window of T steps start, and T at the end.  FLASHLSTM_V2_CHUNK_STEPS sets one
+// length for all (0 = whole window; read per call: cheap, and tests switch it).  Otherwise chunks are 128 steps, so that
+// the projection and dX products fill the chip (64 steps of 32 rows at 1024 units: 25 and 35 us, 128 steps: 32 and 45),
+// but short at both ends of the window: nothing can run before the first chunk is up, and nothing hides the last one's way
+// down.
+std::vector<size_t> chunk_starts(size_t T) {
+    std::vector<size_t> at{0};
+    if (const char* v = getenv("FLASHLSTM_V2_CHUNK_STEPS")) {
+        const long env = atol(v);
+        const size_t c = (env <= 0 || size_t(env) > T) ? T : size_t(env);
+        while (at.back() < T) at.push_back(at.back() + c < T ? at.back() + c : T);
+        return at;
+    }
+    constexpr size_t kEnds[2] = {32, 64}, kMiddle = 128;
+    size_t left = T;
+    std::vector<size_t> tail;
+    for (size_t len : kEnds) {   // a piece at either end while there is room
+        if (left <= 2 * len) break;
+        at.push_back(at.back() + len);
+        tail.push_back(len);
+        left -= 2 * len;
+    }
+    const size_t pieces = (left + kMiddle - 1) / kMiddle;
+    for (size_t i = 0; i < pieces; ++i) at.push_back(at.back() + left / pieces + (i < left % pieces ? 1 : 0));
+    for (size_t i = tail.size(); i-- > 0;) at.push_back(at.back() + tail[i]);
+    return at;
 }
 
 // rows [row0, row0+rows) of a device matrix with pitch ld (elements of esz bytes, `cols` used) -> packed host rows
@@ -232,7 +265,7 @@ void sync_all(const Streams& st) {
 // against a budget of FLASHLSTM_V2_DEVICE_BUDGET_MB (default: 70 % of the device's memory, and no more than
 // 85 % of what is free now plus what this shape's buffers already hold).  FLASHLSTM_V2_WINDOW_STEPS forces a
 // value.  Read per call: cheap, and tests switch them.
-size_t window_steps_for(const Entry& e, size_t T) {
+size_t window_steps_for(Entry& e, size_t T) {
     const size_t B = e.B, I = e.I, H = e.H;
     if (const char* v = getenv("FLASHLSTM_V2_WINDOW_STEPS")) {
         const long w = atol(v);
@@ -243,17 +276,23 @@ size_t window_steps_for(const Entry& e, size_t T) {
     size_t budget = 0;
     if (const char* v = getenv("FLASHLSTM_V2_DEVICE_BUDGET_MB")) budget = size_t(atol(v) > 0 ? atol(v) : 0) << 20;
     if (budget == 0) {
-        size_t free_b = 0, total_b = 0;
-        check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
         size_t held = size_t(flstm_core_get_info(e.plan, "device_bytes") > 0 ? flstm_core_get_info(e.plan, "device_bytes") : 0);
         for (const Buf* b : {&e.x_dev, &e.y_dev, &e.dy_dev, &e.dx_dev}) held += b->bytes;
+        // a sequence that what is already held has room for needs no look at the device's memory (the call asks the
+        // driver)
+        if (e.held_is_within_budget >= held && per_step * T <= held / 20 * 17) return T;
+        size_t free_b = 0, total_b = 0;
+        check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        if (held <= total_b / 10 * 7) e.held_is_within_budget = held;
         budget = total_b / 10 * 7;
         if (budget > (free_b + held) / 20 * 17) budget = (free_b + held) / 20 * 17;
     }
     size_t w = budget / per_step;
     if (w >= T) return T;
-    const size_t c = chunk_steps_for(T);
-    if (w > c) w -= w % c;   // whole chunks
+    if (const char* v = getenv("FLASHLSTM_V2_CHUNK_STEPS")) {   // whole chunks
+        const size_t c = atol(v) > 0 ? size_t(atol(v)) : T;
+        if (w > c) w -= w % c;
+    }
     return w ? w : 1;
 }
 
@@ -269,39 +308,98 @@ CachePtrs cache_ptrs(Entry& e) {
     return cp;
 }
 
+// Device-visible address of `bytes` of pinned host memory, or null (pageable memory, or not known to the runtime).
+void* device_address(const void* host, size_t bytes) {
+    if (!host || !bytes) return nullptr;
+    void* first = nullptr;
+    for (const char* at : {static_cast<const char*>(host), static_cast<const char*>(host) + bytes - 1}) {
+        hipPointerAttribute_t attr{};
+        if (hipPointerGetAttributes(&attr, at) != hipSuccess || attr.type != hipMemoryTypeHost || !attr.devicePointer) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (!first) first = attr.devicePointer;
+        else if (static_cast<char*>(attr.devicePointer) - static_cast<char*>(first) != ptrdiff_t(bytes - 1)) return nullptr;
+    }
+    return first;
+}
+
+// The checkpoints of a pass: entry k = state before step k * R.
+struct Checkpoints {
+    size_t t0 = 0, R = 1;              // first step of the window in the sequence, interval
+    flstm::GateCacheHost host{nullptr, nullptr};
+    bool h32 = true, c32 = true;
+    void *h_dev = nullptr, *c_dev = nullptr;   // device-visible addresses of the host arrays (null: not pinned)
+    // entries whose step lies in steps [lo, hi) of the window
+    void range(size_t lo, size_t hi, size_t& k0, size_t& k1) const { k0 = (t0 + lo + R - 1) / R; k1 = (t0 + hi + R - 1) / R; }
+    bool wanted() const { return host.h_ptr || host.c_ptr; }
+};
+
+void upload_x(Entry& e, const Streams& st, const __half* x_host, size_t k) {
+    const size_t t0 = e.chunks[k], m = e.chunks[k + 1] - t0, row = e.B * e.I * sizeof(half_t);
+    check(hipMemcpyAsync(static_cast<char*>(e.x_dev.p) + t0 * row, reinterpret_cast<const char*>(x_host) + t0 * row, m * row,
+                         hipMemcpyHostToDevice, st.h2d), "x upload");
+    check(hipEventRecord(e.chunk_in[k], st.h2d), "hipEventRecord");
+}
+// The first chunks of a window go up before anything else is enqueued: packing and checksums run meanwhile.
+constexpr size_t kChunksAhead = 2;
+void begin_x_upload(Entry& e, const Streams& st, size_t n, const __half* x_host) {
+    e.x_dev.reserve(n * e.B * e.I * sizeof(half_t));
+    e.cut_into_chunks(chunk_starts(n));
+    for (size_t k = 0; k < kChunksAhead && k < e.nchunks(); ++k) upload_x(e, st, x_host, k);
+}
+
+void write_checkpoints(Entry& e, const Streams& st, const CachePtrs& cp, size_t lo, size_t hi, const Checkpoints& ck);
+
 // Forward pass over the n steps of one window, from the state (h_in, c_in) of `state_dtype`: x rows up, chunk
-// by chunk, projection + recurrence behind them, y rows down.  Leaves the window's caches in the plan (row
-// block 0 of the state arrays = the state the window started from) and x in e.x_dev; writes the final state
-// to (hy, cy) in `out_dtype` when they are given.  The compute stream is idle when it returns.
-CachePtrs forward_window(Entry& e, const Streams& st, size_t n, const __half* x_host, const void* h_in,
-                         const void* c_in, flstm_dtype state_dtype, __half* y_host, void* hy, void* cy,
-                         flstm_dtype out_dtype) {
-    const size_t B = e.B, I = e.I, H = e.H;
-    e.x_dev.reserve(n * B * I * sizeof(half_t));
+// by chunk (begin_x_upload has been called), projection + recurrence behind them, y rows and checkpoints down.  Leaves
+// the window's caches in the plan (row block 0 of the state arrays = the state the window started from) and x in e.x_dev;
+// writes the final state to (hy, cy) in `out_dtype` when they are given.  The compute stream is idle when it returns.
+// The rows of chunk k go down beside the recurrence of chunk k + 1, made by workgroups of that launch which have no part
+// in it (core_copy_beside), where there are such and the host memory is pinned; else as copies on the d2h stream.
+void forward_window(Entry& e, const Streams& st, size_t n, const __half* x_host, const void* h_in, const void* c_in,
+                    flstm_dtype state_dtype, __half* y_host, const Checkpoints& ck, void* hy, void* cy, flstm_dtype out_dtype) {
+    const size_t B = e.B, H = e.H;
     check_core(flstm_core_forward_begin(e.plan, n, e.x_dev.p, FLSTM_F16, h_in, c_in, state_dtype, st.cs),
                "flstm_core_forward_begin");
     CachePtrs cp = cache_ptrs(e);
-    const size_t C = chunk_steps_for(n), nchunks = (n + C - 1) / C;
-    e.need_chunk_events(nchunks);
-    auto upload = [&](size_t k) {
-        const size_t t0 = k * C, m = (t0 + C <= n) ? C : n - t0;
-        check(hipMemcpyAsync(static_cast<char*>(e.x_dev.p) + t0 * B * I * sizeof(half_t),
-                             reinterpret_cast<const char*>(x_host) + t0 * B * I * sizeof(half_t), m * B * I * sizeof(half_t),
-                             hipMemcpyHostToDevice, st.h2d), "x upload");
-        check(hipEventRecord(e.chunk_in[k], st.h2d), "hipEventRecord");
+    const size_t nchunks = e.nchunks();
+    char* const y_dev = static_cast<char*>(device_address(y_host, n * B * H * sizeof(half_t)));
+    const bool pinned = (!y_host || y_dev) && (!ck.host.h_ptr || ck.h_dev) && (!ck.host.c_ptr || ck.c_dev);
+    // y rows and checkpoints of steps [lo, hi), as copies beside the launch that comes next
+    auto offer = [&](size_t lo, size_t hi) -> bool {
+        if (!pinned) return false;
+        flstm_hip::OpList list;
+        if (y_host)   // h_t of step t is row block t+1 of the state cache
+            list.unpad(cp.h + (lo + 1) * B * cp.ldh, 0, cp.ldh, (hi - lo) * B, int(H), 1.f, y_dev + lo * B * H * sizeof(half_t), 0);
+        size_t k0, k1;
+        ck.range(lo, hi, k0, k1);
+        if (k1 > k0) {
+            const size_t rows = (k1 - k0) * B, row0 = (k0 * ck.R - ck.t0) * B;
+            if (ck.host.h_ptr) list.unpad(cp.h + row0 * cp.ldh, 0, cp.ldh, rows, int(H), 1.f, static_cast<char*>(ck.h_dev) + k0 * B * H * (ck.h32 ? 4 : 2), ck.h32, B, ck.R * B);
+            if (ck.host.c_ptr) list.unpad(cp.c + row0 * cp.ldc, 1, cp.ldc, rows, int(H), 1.f, static_cast<char*>(ck.c_dev) + k0 * B * H * (ck.c32 ? 4 : 2), ck.c32, B, ck.R * B);
+        }
+        return list.count == 0 || flstm_hip::core_copy_beside(e.plan, true, list);
     };
-    upload(0);
+    auto download = [&](size_t k, size_t lo, size_t hi) {   // ... on the d2h stream, behind what the compute stream has been given so far
+        if (!y_host) return;
+        check(hipEventRecord(e.chunk_out[k], st.cs), "hipEventRecord");
+        check(hipStreamWaitEvent(st.d2h, e.chunk_out[k], 0), "hipStreamWaitEvent");
+        download_rows(y_host, cp.h + B * cp.ldh, cp.ldh, H, sizeof(half_t), lo * B, (hi - lo) * B, st.d2h);
+    };
+    size_t ck_from = 0;   // checkpoints before this step are on their way
     for (size_t k = 0; k < nchunks; ++k) {
-        const size_t t0 = k * C, m = (t0 + C <= n) ? C : n - t0;
-        if (k + 1 < nchunks) upload(k + 1);
+        const size_t t0 = e.chunks[k], m = e.chunks[k + 1] - t0;
+        if (k + kChunksAhead < nchunks) upload_x(e, st, x_host, k + kChunksAhead);
+        if (k > 0) {
+            const size_t before = e.chunks[k - 1];
+            if (offer(before, t0)) { if (ck_from == before) ck_from = t0; }
+            else download(k - 1, before, t0);
+        }
         check(hipStreamWaitEvent(st.cs, e.chunk_in[k], 0), "hipStreamWaitEvent");
         check_core(flstm_core_forward_steps(e.plan, t0, m, st.cs), "flstm_core_forward_steps");
-        check(hipEventRecord(e.chunk_out[k], st.cs), "hipEventRecord");
-        if (y_host) {   // h_t of step t is row block t+1 of the state cache
-            check(hipStreamWaitEvent(st.d2h, e.chunk_out[k], 0), "hipStreamWaitEvent");
-            download_rows(y_host, cp.h + B * cp.ldh, cp.ldh, H, sizeof(half_t), t0 * B, m * B, st.d2h);
-        }
     }
+    download(nchunks - 1, e.chunks[nchunks - 1], n);
     int rc = flstm_core_forward_end(e.plan, hy, cy, out_dtype, 1, st.cs);
     if (rc == FLSTM_E_STALLED) {
         // a persistent launch gave up: repeat the pass through the entry point that falls back to step-wise launches
@@ -312,40 +410,39 @@ CachePtrs forward_window(Entry& e, const Streams& st, size_t n, const __half* x_
                                       FLSTM_F16, hy, cy, out_dtype, 1, st.cs), "flstm_core_forward");
         if (y_host) check(hipMemcpyAsync(y_host, e.y_dev.p, y_bytes, hipMemcpyDeviceToHost, st.d2h), "y download");
         cp = cache_ptrs(e);
+        ck_from = 0;
     } else {
         check_core(rc, "flstm_core_forward_end");
     }
-    return cp;
+    write_checkpoints(e, st, cp, ck_from, n, ck);
 }
 
-// Checkpoints that fall into the window of steps [t0, t0 + n): entry k = state before step k * R, which is row
-// block k * R - t0 of the window's state arrays.
-void write_checkpoints(Entry& e, const Streams& st, const CachePtrs& cp, size_t t0, size_t n, size_t R,
-                       flstm::GateCacheHost cache, flstm::StreamingLstmOptions opt) {
+// The checkpoints that fall into steps [lo, hi) of the window, gathered from its state arrays and sent down on the d2h
+// stream.
+void write_checkpoints(Entry& e, const Streams& st, const CachePtrs& cp, size_t lo, size_t hi, const Checkpoints& ck) {
     const size_t B = e.B, H = e.H;
-    const size_t k0 = (t0 + R - 1) / R, k1 = (t0 + n + R - 1) / R;   // k * R in [t0, t0 + n)
-    if (k1 <= k0 || (!cache.h_ptr && !cache.c_ptr)) return;
-    const size_t nk = k1 - k0, row0 = (k0 * R - t0) * B;
-    const bool h32 = opt.h_dtype == flstm::GateCacheDType::kFloat32;
-    const bool c32 = opt.c_dtype == flstm::GateCacheDType::kFloat32;
-    const size_t hsz = h32 ? 4 : 2, csz = c32 ? 4 : 2;
-    if (cache.h_ptr) {
+    size_t k0, k1;
+    ck.range(lo, hi, k0, k1);
+    if (k1 <= k0 || !ck.wanted()) return;
+    const size_t nk = k1 - k0, row0 = (k0 * ck.R - ck.t0) * B;
+    const size_t hsz = ck.h32 ? 4 : 2, csz = ck.c32 ? 4 : 2;
+    if (ck.host.h_ptr) {
         e.ck_h.reserve(nk * B * H * hsz);
-        check(flstm_hip::gather_from_half(cp.h + row0 * cp.ldh, cp.ldh, nk * B, int(H), e.ck_h.p, h32, B, R * B, st.cs),
+        check(flstm_hip::gather_from_half(cp.h + row0 * cp.ldh, cp.ldh, nk * B, int(H), e.ck_h.p, ck.h32, B, ck.R * B, st.cs),
               "checkpoint gather");
     }
-    if (cache.c_ptr) {
+    if (ck.host.c_ptr) {
         e.ck_c.reserve(nk * B * H * csz);
-        check(flstm_hip::gather_from_float(cp.c + row0 * cp.ldc, cp.ldc, nk * B, int(H), 1.f, e.ck_c.p, c32, B, R * B,
+        check(flstm_hip::gather_from_float(cp.c + row0 * cp.ldc, cp.ldc, nk * B, int(H), 1.f, e.ck_c.p, ck.c32, B, ck.R * B,
                                            st.cs), "checkpoint gather");
     }
     check(hipEventRecord(e.ev_out, st.cs), "hipEventRecord");
     check(hipStreamWaitEvent(st.d2h, e.ev_out, 0), "hipStreamWaitEvent");
-    if (cache.h_ptr)
-        check(hipMemcpyAsync(static_cast<char*>(cache.h_ptr) + k0 * B * H * hsz, e.ck_h.p, nk * B * H * hsz,
+    if (ck.host.h_ptr)
+        check(hipMemcpyAsync(static_cast<char*>(ck.host.h_ptr) + k0 * B * H * hsz, e.ck_h.p, nk * B * H * hsz,
                              hipMemcpyDeviceToHost, st.d2h), "h checkpoints");
-    if (cache.c_ptr)
-        check(hipMemcpyAsync(static_cast<char*>(cache.c_ptr) + k0 * B * H * csz, e.ck_c.p, nk * B * H * csz,
+    if (ck.host.c_ptr)
+        check(hipMemcpyAsync(static_cast<char*>(ck.host.c_ptr) + k0 * B * H * csz, e.ck_c.p, nk * B * H * csz,
                              hipMemcpyDeviceToHost, st.d2h), "c checkpoints");
 }
 
@@ -363,13 +460,22 @@ void run_forward(Entry& e, size_t T, size_t R, const __half* x_host, const __hal
                  const Streams& st) {
     const size_t B = e.B, I = e.I, H = e.H, BH = B * H;
     e.last.valid = false;
-    check_core(flstm_core_pack_weights(e.plan, w_ih, w_hh, st.cs), "flstm_core_pack_weights");
-    check_core(flstm_core_pack_bias(e.plan, b_ih, b_hh, st.cs), "flstm_core_pack_bias");
     const size_t W = window_steps_for(e, T), nwin = (T + W - 1) / W;
+    begin_x_upload(e, st, W, x_host);
+    check_core(flstm_hip::core_pack_weights_async(e.plan, w_ih, w_hh, st.cs), "flstm_core_pack_weights");
+    check_core(flstm_core_pack_bias(e.plan, b_ih, b_hh, st.cs), "flstm_core_pack_bias");
+    enqueue_device_print(e, st.cs, w_ih, w_hh, b_ih, b_hh, h0, c0);
+    Checkpoints ck;
+    ck.R = R;
+    ck.host = cache;
+    ck.h32 = opt.h_dtype == flstm::GateCacheDType::kFloat32;
+    ck.c32 = opt.c_dtype == flstm::GateCacheDType::kFloat32;
+    const size_t entries = (T + R - 1) / R;
+    ck.h_dev = device_address(cache.h_ptr, entries * BH * (ck.h32 ? 4 : 2));
+    ck.c_dev = device_address(cache.c_ptr, entries * BH * (ck.c32 ? 4 : 2));
     e.start_known.assign(nwin, 0);
     if (nwin == 1) {
-        const CachePtrs cp = forward_window(e, st, T, x_host, h0, c0, FLSTM_F16, y_host, hy, cy, FLSTM_F16);
-        write_checkpoints(e, st, cp, 0, T, R, cache, opt);
+        forward_window(e, st, T, x_host, h0, c0, FLSTM_F16, y_host, ck, hy, cy, FLSTM_F16);
     } else {
         e.carry_h.reserve(BH * sizeof(float));
         e.carry_c.reserve(BH * sizeof(float));
@@ -381,13 +487,13 @@ void run_forward(Entry& e, size_t T, size_t R, const __half* x_host, const __hal
                 copy_state(start_state(e, j, 0), e.carry_h.p, BH, st.cs);
                 copy_state(start_state(e, j, 1), e.carry_c.p, BH, st.cs);
                 e.start_known[j] = 1;
+                begin_x_upload(e, st, n, x_host + t0 * B * I);
             }
-            const CachePtrs cp = forward_window(
-                e, st, n, x_host + t0 * B * I, first ? static_cast<const void*>(h0) : e.carry_h.p,
-                first ? static_cast<const void*>(c0) : e.carry_c.p, first ? FLSTM_F16 : FLSTM_F32,
-                y_host ? y_host + t0 * B * H : nullptr, last ? static_cast<void*>(hy) : e.carry_h.p,
-                last ? static_cast<void*>(cy) : e.carry_c.p, last ? FLSTM_F16 : FLSTM_F32);
-            write_checkpoints(e, st, cp, t0, n, R, cache, opt);
+            ck.t0 = t0;
+            forward_window(e, st, n, x_host + t0 * B * I, first ? static_cast<const void*>(h0) : e.carry_h.p,
+                           first ? static_cast<const void*>(c0) : e.carry_c.p, first ? FLSTM_F16 : FLSTM_F32,
+                           y_host ? y_host + t0 * B * H : nullptr, ck, last ? static_cast<void*>(hy) : e.carry_h.p,
+                           last ? static_cast<void*>(cy) : e.carry_c.p, last ? FLSTM_F16 : FLSTM_F32);
             sync_all(st);   // the next window reuses every buffer
         }
     }
@@ -397,53 +503,65 @@ void run_forward(Entry& e, size_t T, size_t R, const __half* x_host, const __hal
     k.w_ih = w_ih; k.w_hh = w_hh; k.T = T; k.R = R; k.W = W;
     k.x_print = fingerprint(x_host, T * B * I * sizeof(half_t));
     k.y_print = y_host ? fingerprint(y_host, T * B * H * sizeof(half_t)) : 0;
-    k.dev_print = device_print(e, st.cs, w_ih, w_hh, b_ih, b_hh, h0, c0);
+    k.dev_print = read_device_print(e, b_ih, b_hh, h0, c0);
     k.valid = true;
     e.last = k;
 }
 
+// Steps [lo, lo + m) of the k-th chunk of a backward window: from the end of the sequence towards its start.
+void backward_chunk(const Entry& e, size_t k, size_t& lo, size_t& m) {
+    const size_t i = e.nchunks() - 1 - k;
+    lo = e.chunks[i];
+    m = e.chunks[i + 1] - lo;
+}
+void upload_dy(Entry& e, const Streams& st, const __half* dY_host, size_t k) {
+    size_t lo, m;
+    backward_chunk(e, k, lo, m);
+    const size_t row = e.B * e.H * sizeof(half_t);
+    check(hipMemcpyAsync(static_cast<char*>(e.dy_dev.p) + lo * row, reinterpret_cast<const char*>(dY_host) + lo * row, m * row,
+                         hipMemcpyHostToDevice, st.h2d), "dY upload");
+    check(hipEventRecord(e.dy_in[k], st.h2d), "hipEventRecord");
+}
+void begin_dy_upload(Entry& e, const Streams& st, size_t n, const __half* dY_host) {   // (as begin_x_upload)
+    e.dy_dev.reserve(n * e.B * e.H * sizeof(half_t));
+    e.cut_into_chunks(chunk_starts(n));
+    for (size_t k = 0; k < kChunksAhead && k < e.nchunks(); ++k) upload_dy(e, st, dY_host, k);
+}
+void download_dx(Entry& e, const Streams& st, size_t k, __half* dx_host, size_t lo, size_t m) {
+    check(hipEventRecord(e.chunk_out[k], st.cs), "hipEventRecord");
+    check(hipStreamWaitEvent(st.d2h, e.chunk_out[k], 0), "hipStreamWaitEvent");
+    download_rows(dx_host, e.dx_dev.p, e.I, e.I, sizeof(half_t), lo * e.B, m * e.B, st.d2h);
+}
+
 // BPTT over the n steps of the window whose forward caches the plan holds (and whose x rows are in e.x_dev):
-// dY rows up chunk by chunk from the end, BPTT steps + dX behind them, dx rows down; then the weight-gradient
+// (begin_dy_upload has been called) dY rows up chunk by chunk from the end, BPTT steps + dX behind them, dx rows down; then the weight-gradient
 // GEMMs over the window.  (d_hn, d_cn) of `dstate_dtype` is the gradient flowing in at the window's end,
 // (dh0, dc0) the one flowing out at its start (fp32).
 void backward_window(Entry& e, const Streams& st, size_t n, const __half* dY_host, const void* d_hn, const void* d_cn,
                      flstm_dtype dstate_dtype, __half* dx_host, bool accumulate, float* dW_ih, float* dW_hh,
                      float* db_ih, float* db_hh, float* dh0, float* dc0) {
     const size_t B = e.B, I = e.I, H = e.H;
-    const size_t x_bytes = n * B * I * sizeof(half_t), y_bytes = n * B * H * sizeof(half_t);
-    e.dy_dev.reserve(y_bytes);
+    const size_t x_bytes = n * B * I * sizeof(half_t);
     if (dx_host) e.dx_dev.reserve(x_bytes);
     check_core(flstm_core_set_option(e.plan, "accumulate_grads", accumulate ? 1 : 0), "flstm_core_set_option");
     check_core(flstm_core_backward_begin(e.plan, n, e.dy_dev.p, FLSTM_F16, d_hn, d_cn, dstate_dtype, 1.f,
                                          dx_host ? e.dx_dev.p : nullptr, FLSTM_F16, st.cs), "flstm_core_backward_begin");
-    const size_t C = chunk_steps_for(n), nchunks = (n + C - 1) / C;
-    e.need_chunk_events(nchunks);
-    auto chunk_range = [&](size_t k, size_t& lo, size_t& m) {   // chunk k counts from the end; the first one takes the remainder
-        const size_t rem = n % C, first = rem ? rem : C;
-        m = (k == 0) ? first : C;
-        const size_t hi = n - 1 - (k == 0 ? 0 : first + (k - 1) * C);
-        lo = hi + 1 - m;
-    };
-    auto upload = [&](size_t k) {
-        size_t lo, m;
-        chunk_range(k, lo, m);
-        check(hipMemcpyAsync(static_cast<char*>(e.dy_dev.p) + lo * B * H * sizeof(half_t),
-                             reinterpret_cast<const char*>(dY_host) + lo * B * H * sizeof(half_t), m * B * H * sizeof(half_t),
-                             hipMemcpyHostToDevice, st.h2d), "dY upload");
-        check(hipEventRecord(e.chunk_in[k], st.h2d), "hipEventRecord");
-    };
-    upload(0);
+    const size_t nchunks = e.nchunks();
+    char* const dx_pinned = static_cast<char*>(device_address(dx_host, x_bytes));
     for (size_t k = 0; k < nchunks; ++k) {
         size_t lo, m;
-        chunk_range(k, lo, m);
-        if (k + 1 < nchunks) upload(k + 1);
-        check(hipStreamWaitEvent(st.cs, e.chunk_in[k], 0), "hipStreamWaitEvent");
-        check_core(flstm_core_backward_steps(e.plan, lo + m - 1, m, st.cs), "flstm_core_backward_steps");
-        check(hipEventRecord(e.chunk_out[k], st.cs), "hipEventRecord");
-        if (dx_host) {
-            check(hipStreamWaitEvent(st.d2h, e.chunk_out[k], 0), "hipStreamWaitEvent");
-            download_rows(dx_host, e.dx_dev.p, I, I, sizeof(half_t), lo * B, m * B, st.d2h);
+        backward_chunk(e, k, lo, m);
+        if (k + kChunksAhead < nchunks) upload_dy(e, st, dY_host, k + kChunksAhead);
+        if (k > 0 && dx_host) {   // dx rows of the chunk before, beside this one's recurrence (as in forward_window)
+            size_t plo, pm;
+            backward_chunk(e, k - 1, plo, pm);
+            flstm_hip::OpList list;
+            list.unpad(static_cast<const half_t*>(e.dx_dev.p) + plo * B * I, 0, I, pm * B, int(I), 1.f, dx_pinned + plo * B * I * sizeof(half_t), 0);
+            if (!dx_pinned || !flstm_hip::core_copy_beside(e.plan, false, list)) download_dx(e, st, k - 1, dx_host, plo, pm);
         }
+        check(hipStreamWaitEvent(st.cs, e.dy_in[k], 0), "hipStreamWaitEvent");
+        check_core(flstm_core_backward_steps(e.plan, lo + m - 1, m, st.cs), "flstm_core_backward_steps");
+        if (k + 1 == nchunks && dx_host) download_dx(e, st, k, dx_host, lo, m);
     }
     int rc = flstm_core_backward_end(e.plan, e.x_dev.p, FLSTM_F16, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, st.cs);
     if (rc == FLSTM_E_STALLED) {
@@ -483,7 +601,8 @@ size_t rebuild_start_state(Entry& e, const Streams& st, size_t j, size_t W, size
     size_t cur = t_ck;
     while (cur < target) {
         const size_t end = (cur / W + 1) * W < target ? (cur / W + 1) * W : target;   // stop at every window start
-        forward_window(e, st, end - cur, x_host + cur * B * I, e.carry_h.p, e.carry_c.p, FLSTM_F32, nullptr, e.carry_h.p,
+        begin_x_upload(e, st, end - cur, x_host + cur * B * I);
+        forward_window(e, st, end - cur, x_host + cur * B * I, e.carry_h.p, e.carry_c.p, FLSTM_F32, nullptr, Checkpoints{}, e.carry_h.p,
                        e.carry_c.p, FLSTM_F32);
         sync_all(st);
         cur = end;
@@ -546,7 +665,12 @@ void StreamingLstmBackward(size_t T, size_t B, size_t I, size_t H, size_t R, con
                k.cc == cache.c_ptr && k.h0 == h0 && k.c0 == c0 && k.w_ih == w_ih && k.w_hh == w_hh && k.T == T &&
                k.W == W;
     if (hit) hit = (k.x_print == fingerprint(x_host, x_bytes)) && (!y_host || k.y_print == fingerprint(y_host, y_bytes));
-    if (hit) hit = (k.dev_print == device_print(e, cs, w_ih, w_hh, b_ih, b_hh, h0, c0));
+    if (nwin == 1) begin_dy_upload(e, st, T, dY_host);   // (under the checksum, or the forward pass again)
+    if (hit) {
+        enqueue_device_print(e, cs, w_ih, w_hh, b_ih, b_hh, h0, c0);
+        check(hipStreamSynchronize(cs), "checksum");
+        hit = (k.dev_print == read_device_print(e, b_ih, b_hh, h0, c0));
+    }
     const double fwd_flops_per_step = flstm_hip::gemm_flops(4 * H, B, I + H);
     if (nwin == 1) {
         if (!hit) {
@@ -572,9 +696,11 @@ void StreamingLstmBackward(size_t T, size_t B, size_t I, size_t H, size_t R, con
             if (!first && !e.start_known[j])
                 prof.add_total(double(rebuild_start_state(e, st, j, W, R, x_host, cache, opt)) * fwd_flops_per_step);
             // this window's gate cache
+            begin_x_upload(e, st, n, x_host + t0 * B * I);
             forward_window(e, st, n, x_host + t0 * B * I, first ? static_cast<const void*>(h0) : start_state(e, j, 0),
                            first ? static_cast<const void*>(c0) : start_state(e, j, 1), first ? FLSTM_F16 : FLSTM_F32,
-                           nullptr, nullptr, nullptr, FLSTM_F16);
+                           nullptr, Checkpoints{}, nullptr, nullptr, FLSTM_F16);
+            begin_dy_upload(e, st, n, dY_host + t0 * B * H);
             prof.add_total(double(n) * fwd_flops_per_step);
             backward_window(e, st, n, dY_host + t0 * B * H, last ? static_cast<const void*>(d_hn) : e.carry_dh.p,
                             last ? static_cast<const void*>(d_cn) : e.carry_dc.p, last ? FLSTM_F16 : FLSTM_F32,

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/flashlstm/lstm_core.h"
+#include "core_internal.h"
 #include "gemm.h"
 #include "pack.h"
 #include "recurrent.h"
@@ -76,7 +77,8 @@ constexpr int kFirstHold = 8, kMaxHold = 1024;
 // launches several (ranges of steps, windows of rows) takes the sets its setup has zeroed one after the other.
 constexpr size_t kStampsOffset = 64, kSeatsOffset = 256;
 constexpr int kSeatSets = 64;
-constexpr size_t kStatusBytes = kSeatsOffset + size_t(kSeatSets) * 8 * sizeof(unsigned);
+constexpr int kSeatWords = 16;   // eight seat counters, the ticket counter of BesideCopies, padding
+constexpr size_t kStatusBytes = kSeatsOffset + size_t(kSeatSets) * kSeatWords * sizeof(unsigned);
 static_assert(kStampsOffset + kStampCount * sizeof(long long) <= kSeatsOffset, "stamps fit in front of the seats");
 
 struct flstm_core_plan {
@@ -126,6 +128,7 @@ struct flstm_core_plan {
              half_t* y_direct = nullptr; } fw;   // y_direct: the recurrence writes the caller's y itself
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
              float S = 1.f, dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
+    BesideCopies beside_f, beside_b;   // for the next recurrence launch of a pass fed in ranges (core_copy_beside)
     // backward scratch
     DevBuf dYp, dG, dHn, dC, dH0, db_part, dw_part, prof, part_b;
     int opt_profile = 0, wall_khz = 100000;
@@ -210,10 +213,10 @@ int wait_status(flstm_core_plan* p, OpList& last, int stamp, hipStream_t s, int*
 int next_seats(flstm_core_plan* p, unsigned** out, hipStream_t s) {
     char* const first = p->status.as<char>() + kSeatsOffset;
     if (p->seat_sets_left <= 0) {
-        FL_TRY(fill_zero(first, size_t(kSeatSets) * 8 * sizeof(unsigned), s));
+        FL_TRY(fill_zero(first, size_t(kSeatSets) * kSeatWords * sizeof(unsigned), s));
         p->seat_sets_left = kSeatSets;
     }
-    *out = reinterpret_cast<unsigned*>(first) + size_t(--p->seat_sets_left) * 8;
+    *out = reinterpret_cast<unsigned*>(first) + size_t(--p->seat_sets_left) * kSeatWords;
     return 0;
 }
 
@@ -389,8 +392,14 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
 }
 
 extern "C" int flstm_core_pack_weights(flstm_core_plan* p, const float* w_ih, const float* w_hh, void* stream) {
+    const int rc = core_pack_weights_async(p, w_ih, w_hh, static_cast<hipStream_t>(stream));
+    if (rc) return rc;
+    FL_TRY(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+    return 0;
+}
+
+int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, const float* w_hh, hipStream_t s) {
     if (!p || !w_ih || !w_hh) return FLSTM_E_INVALID;
-    hipStream_t s = static_cast<hipStream_t>(stream);
     const Dims& d = p->d;
     FL_TRY(p->wih_p.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
     FL_TRY(p->wih_t.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
@@ -403,7 +412,6 @@ extern "C" int flstm_core_pack_weights(flstm_core_plan* p, const float* w_ih, co
         FL_TRY(p->wfrag_b2.reserve(rec_bwd_two_d_wfrag_bytes(d.Hp)));
         FL_TRY(pack_wfrag_bwd2d(d, w_hh, p->wfrag_b2.as<half8>(), rec_bwd_two_d_kq(d.B, d.Hp), s));
     }
-    FL_TRY(hipStreamSynchronize(s));
     p->weights_packed = true;
     return 0;
 }
@@ -437,6 +445,7 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     p->fw.T = T; p->fw.x = x; p->fw.x_dtype = x_dtype; p->fw.open = true;
+    p->beside_f.count = 0;
     if (!x_in_place(p, x_dtype)) FL_TRY(p->X16.reserve(TB * d.Ip * sizeof(half_t)));
     FL_TRY(p->G.reserve(TB * 4 * d.Hp * sizeof(half_t)));
     FL_TRY(p->Y.reserve((TB + d.B) * d.Hp * sizeof(half_t)));
@@ -498,9 +507,18 @@ int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, hip
     return 0;
 }
 
+// the copies waiting for the next recurrence launch become that launch's
+template <typename Args>
+void take_beside(BesideCopies& waiting, Args& a) {
+    if (waiting.count > 0) { a.beside = waiting; a.beside.ticket = a.seats + 8; }
+    else a.beside.count = 0;   // (a later window of batch rows: the first one has made them)
+    waiting.count = 0;
+}
+
 int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     const Dims& d = p->d;
-    RecFwdArgs a{};
+    RecFwdArgs a;
+    memset(static_cast<void*>(&a), 0, sizeof(a));   // (padding too: the arguments are the key of a captured graph)
     a.wfrag = p->wfrag_f.as<half8>();
     a.Y = p->Y.as<half_t>(); a.G = p->G.as<half_t>(); a.C = p->C.as<float>();
     a.y_out = p->fw.y_direct;
@@ -510,6 +528,7 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     a.stamps = stamps_of(p) + kStampFwdRec;
     int rc = next_seats(p, &a.seats, s);
     if (rc) return rc;
+    take_beside(p->beside_f, a);
     a.B = d.B; a.Hp = d.Hp; a.T = int(p->fw.T); a.t0 = int(t0); a.t1 = int(t0 + n);
     a.spin_limit = p->opt_spin_limit;
     a.spin_ticks = (long long)p->opt_spin_ms * p->wall_khz;
@@ -523,6 +542,10 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
         p->refused_fwd = true;
         p->coop_refusals++;
         replan(p);
+        OpList copies;   // step-wise launches have no workgroups to spare
+        for (int i = 0; i < a.beside.count; ++i) copies.op[copies.count++] = a.beside.op[i];
+        a.beside.count = 0;
+        FL_TRY(run_ops(copies, s));
         e = launch_rec_fwd(p->Lf, a, s, nullptr);
     }
     FL_TRY(e);
@@ -664,6 +687,7 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     const size_t TB = T * size_t(d.B);
     p->bw.T = T; p->bw.dY = dY; p->bw.dy_dtype = dy_dtype; p->bw.S = S; p->bw.dx = dx; p->bw.dx_dtype = dx_dtype;
     p->bw.open = true;
+    p->beside_b.count = 0;
     // (step-wise launches always read a plan-owned copy, so that their captured graph can be replayed)
     if (dy_dtype == FLSTM_F16 && d.H == d.Hp && p->Lb.persistent) {
         p->bw.dYk = static_cast<const half_t*>(dY);
@@ -721,7 +745,8 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
         conv.to_half(src, p->bw.dy_dtype == FLSTM_F32, rows, d.H, size_t(d.H), p->bw.S, dst, rows, size_t(d.Hp));
         FL_TRY(run_ops(conv, s));
     }
-    RecBwdArgs a{};
+    RecBwdArgs a;
+    memset(static_cast<void*>(&a), 0, sizeof(a));   // (as in forward_recur)
     a.wfrag = p->wfrag_b.as<half8>();
     a.G = p->G.as<half_t>(); a.C = p->C.as<float>(); a.dY = p->bw.dYk; a.dG = p->dG.as<half_t>();
     a.dHn = p->dHn.as<float>(); a.dC = p->dC.as<float>(); a.dH0 = p->dH0.as<float>();
@@ -749,6 +774,7 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
         a.b_hi = b_lo + win < d.B ? b_lo + win : d.B;
         int rc = next_seats(p, &a.seats, s);
         if (rc) return rc;
+        take_beside(p->beside_b, a);
         if (win < d.B) {
             const size_t pslot = a.p_slot * sizeof(float);
             const int first_T = t_hi >= long(p->bw.T) - 1 ? int(p->bw.T) : int(t_hi) + 2;   // (its first product step is first_T - 2)
@@ -991,6 +1017,21 @@ extern "C" int flstm_core_backward_end(flstm_core_plan* p, const void* x, flstm_
     if (rc) return rc;
     pass_done(p, false);
     return 0;
+}
+
+bool flstm_hip::core_copy_beside(flstm_core_plan* p, bool forward, const OpList& copies) {
+    // 48 workgroups of 256 threads with one 16-byte load in flight each keep a PCIe link of 57 GB/s busy
+    constexpr int kFewest = 16, kHelpers = 48;
+    const int idle = rec_idle_workgroups(forward ? p->Lf : p->Lb);
+    if (idle < kFewest || copies.count < 1 || copies.count > BesideCopies::kMost) return false;
+    BesideCopies& b = forward ? p->beside_f : p->beside_b;
+    for (int i = 0; i < copies.count; ++i) {
+        if (copies.op[i].kind != LayoutOp::kUnpad) return false;
+        b.op[i] = copies.op[i];
+    }
+    b.count = copies.count;
+    b.helpers = idle < kHelpers ? idle : kHelpers;
+    return true;
 }
 
 extern "C" int flstm_core_cache_ptr(const flstm_core_plan* p, int which, const void** ptr, size_t* ld) {

@@ -1,5 +1,6 @@
 // Layout kernels: weight packing, padded dtype conversion, transposes and output reductions.
 // All are pure HBM-bandwidth work; each thread moves a few elements with coalesced accesses.
+#include "layout_device.h"
 #include "pack.h"
 #include "recurrent.h"
 
@@ -126,49 +127,6 @@ __global__ void fill_words_kernel(unsigned* p, size_t words, unsigned value) {
     for (size_t i = size_t(blockIdx.x) * kT + threadIdx.x; i < words; i += stride) p[i] = value;
 }
 
-// Index arithmetic of the operations in 32 bits where the counts allow: a 64-bit division is a hundred instructions,
-// more than the memory traffic of the 16 bytes it addresses.
-__device__ __forceinline__ void split_index(size_t i, size_t width, size_t& r, size_t& c) {
-    if ((i | width) >> 32) { r = i / width; c = i % width; }
-    else { const unsigned q = unsigned(i) / unsigned(width); r = q; c = unsigned(i) - q * unsigned(width); }
-}
-
-template <int V>
-__device__ __forceinline__ void load_floats(const void* src, size_t at, int in_f32, float (&v)[V]) {
-    if constexpr (V == 8) {
-        if (in_f32) {
-            const floatx4* p = reinterpret_cast<const floatx4*>(static_cast<const float*>(src) + at);
-            const floatx4 a = p[0], b = p[1];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
-        } else {
-            const half8 h = ld_half8(static_cast<const half_t*>(src) + at);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (float)h[e];
-        }
-    } else {
-        v[0] = in_f32 ? static_cast<const float*>(src)[at] : (float)static_cast<const half_t*>(src)[at];
-    }
-}
-template <int V>
-__device__ __forceinline__ void store_values(void* dst, size_t at, int out_f32, const float (&v)[V]) {
-    if constexpr (V == 8) {
-        if (out_f32) {
-            floatx4* p = reinterpret_cast<floatx4*>(static_cast<float*>(dst) + at);
-            p[0] = floatx4{v[0], v[1], v[2], v[3]};
-            p[1] = floatx4{v[4], v[5], v[6], v[7]};
-        } else {
-            half8 h;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) h[e] = (half_t)v[e];
-            st_half8(static_cast<half_t*>(dst) + at, h);
-        }
-    } else {
-        if (out_f32) static_cast<float*>(dst)[at] = v[0];
-        else static_cast<half_t*>(dst)[at] = (half_t)v[0];
-    }
-}
-
 // kToHalf / kToFloat: V consecutive elements of an output row (V = 8: ld_out is a multiple of 8)
 template <int V>
 __device__ __forceinline__ void op_convert(const LayoutOp& o, size_t first, size_t stride) {
@@ -194,26 +152,6 @@ __device__ __forceinline__ void op_convert(const LayoutOp& o, size_t first, size
             for (int e = 0; e < V; ++e) v[e] *= o.scale;
         }
         store_values<V>(o.dst, r * o.ld_out + c, out_f32, v);
-    }
-}
-
-// kUnpad: V consecutive elements of an output row (V = 8: both pitches multiples of 8, both bases 16-byte aligned)
-template <int V>
-__device__ __forceinline__ void op_unpad(const LayoutOp& o, size_t first, size_t stride) {
-    for (size_t i = first; i < o.n; i += stride) {
-        size_t r, c;
-        split_index(i, size_t(o.cols) / V, r, c);
-        size_t rin = r;
-        if (o.rows_per_block) {
-            size_t blk, rest;
-            split_index(r, o.rows_per_block, blk, rest);
-            rin = blk * o.block_stride + rest;
-        }
-        float v[V];
-        load_floats<V>(o.src, rin * o.ld_in + c * V, o.in_f32, v);
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] *= o.scale;
-        store_values<V>(o.dst, i * V, o.out_f32, v);
     }
 }
 
@@ -270,8 +208,7 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
             if (o.vec == 8) op_convert<8>(o, first, stride);
             else op_convert<1>(o, first, stride);
         } else if (o.kind == LayoutOp::kUnpad) {
-            if (o.vec == 8) op_unpad<8>(o, first, stride);
-            else op_unpad<1>(o, first, stride);
+            op_unpad_any(o, first, stride);
         } else if (o.kind == LayoutOp::kToExchange) {
             // item i = eight halfs of one lane: [16-row tile][32-wide k-step][lane] (recurrent.hip, xch_offset)
             const unsigned nks = unsigned(o.ld_out) / 32;
@@ -382,7 +319,9 @@ void OpList::unpad(const void* in, int in_f32, size_t ld_in, size_t rows, int co
     if (out == nullptr || rows * size_t(cols) == 0) return;
     LayoutOp& o = op[count++];
     o.kind = LayoutOp::kUnpad; o.in_f32 = in_f32; o.out_f32 = out_f32; o.dst = out; o.src = in;
-    o.vec = (cols % 8 == 0 && ld_in % 8 == 0 && aligned16(in) && aligned16(out)) ? 8 : 1;
+    o.vec = 1;
+    if (cols % 8 == 0 && ld_in % 8 == 0 && aligned16(in) && aligned16(out)) o.vec = 8;
+    else if (cols % 2 == 0 && ld_in % 2 == 0 && (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 8 == 0) o.vec = 2;
     o.n = rows * size_t(cols) / o.vec;
     o.rows = rows; o.cols = cols; o.ld_in = ld_in; o.scale = scale;
     o.rows_per_block = rows_per_block >= rows ? 0 : rows_per_block; o.block_stride = block_stride;

@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "common.h"
+#include "pack.h"
 
 namespace flstm_hip {
 
@@ -37,6 +38,18 @@ struct RecLayout {
                      // the sizes alone and does not follow mt
 };
 
+// Copies that the idle workgroups of a persistent launch make beside the recurrence (rows that an earlier launch of the
+// pass has finished, on their way to pinned host memory).  A copy kernel on another stream cannot do that: its
+// workgroups sit on CUs that the recurrence's workgroups need as a whole and are waited for, and the runtime's own copy
+// to the host IS such a kernel (64 steps of 32 rows at 1024 units, backward: 190 -> 262 us with one beside it).
+struct BesideCopies {
+    static constexpr int kMost = 3;
+    LayoutOp op[kMost];      // kUnpad operations
+    int count = 0;
+    int helpers = 0;         // idle workgroups that take part
+    unsigned* ticket = nullptr;   // zeroed before the launch
+};
+
 struct RecFwdArgs {
     const half8* wfrag;  // [nh][nw waves][ks][nt][64 lanes] MFMA B-fragments of W_hh (packed gate order)
     half_t* Y;           // [(T+1)*B][Hp]; rows [0,B) = h0, rows [(t+1)B, (t+2)B) = h_t (row-major, for later kernels)
@@ -54,6 +67,7 @@ struct RecFwdArgs {
     int* status;         // 0 ok, 1 spin limit hit, 2 workgroup not on the expected XCD
     int B, Hp, T;
     int t0, t1;          // steps [t0, t1) of the sequence are run by this call (state and ring carry over)
+    BesideCopies beside;
     long long* stamps;   // optional [2]: when the pass's first launch started and its last one ended (workgroup of group 0, slice 0)
     int spin_limit;      // reloads of a fragment chunk that still shows the 'unwritten' pattern before giving up
     long long spin_ticks;   // the same bound as time: ticks of the device's constant-rate wall clock
@@ -87,6 +101,7 @@ struct RecBwdArgs {
                          // every array keeps its full-batch strides, the rings are indexed by the row in the batch)
     float dy_scale;      // factor applied to dY on load (the loss scale, or 1 when dY is pre-scaled)
     int t_hi, t_lo;      // steps t_hi down to t_lo are run by this call; t_lo = -1 adds the closing dh0 product
+    BesideCopies beside;
     long long* stamp_end;   // optional: when the last launch of the pass ended (workgroup of group 0, slice 0)
     int spin_limit;
     long long spin_ticks;
@@ -174,6 +189,9 @@ size_t exchange_slot_halfs(int rows, int cols);
 // Number of k-steps (32 wide) every wave holds for a layout (sizes the fragment arrays).
 int rec_fwd_ks(const RecLayout& L, int Hp);
 int rec_bwd_ks(const RecLayout& L, int Hp);
+
+// Idle workgroups that a launch with this layout can give to BesideCopies (0: step-wise, or every CU has work).
+int rec_idle_workgroups(const RecLayout& L);
 
 // To be called once a stream that persistent launches went to has been waited for: launches on other streams no longer
 // need to be ordered behind it (launch_persistent).

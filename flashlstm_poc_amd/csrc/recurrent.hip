@@ -39,6 +39,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "layout_device.h"
 #include "recurrent.h"
 
 namespace flstm_hip {
@@ -93,6 +94,18 @@ __device__ __forceinline__ Role make_role(int nh, int ng, int gpx, int xcd_local
         r.active = r.g < ng;
     }
     return r;
+}
+
+// What a workgroup without a seat in the recurrence does: its share of the copies handed to the launch.
+__device__ __forceinline__ void copy_beside(const BesideCopies& c, int* lds_ticket) {
+    if (c.count == 0) return;
+    __syncthreads();
+    if (threadIdx.x == 0) *lds_ticket = int(__hip_atomic_fetch_add(c.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    __syncthreads();
+    const int ticket = *lds_ticket;
+    if (ticket >= c.helpers) return;
+    const size_t stride = size_t(c.helpers) * blockDim.x, first = size_t(ticket) * blockDim.x + threadIdx.x;
+    for (int i = 0; i < c.count; ++i) op_unpad_any(c.op[i], first, stride);
 }
 
 // Pattern that marks a not-yet-written pair of halfs in the exchange ring.
@@ -876,7 +889,10 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
 
     if (threadIdx.x == 0) lds_abort = 0;
     const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
-    if (!role.active) return;
+    if (!role.active) {
+        copy_beside(p.beside, lds_role);
+        return;
+    }
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const int hs = role.hs, g = role.g;
     const int rotation = __builtin_amdgcn_readfirstlane(rec_kstep_rotation(hs, L.nh, ks_wave, L.rot_div));
@@ -1097,7 +1113,10 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
 
     if (threadIdx.x == 0) lds_abort = 0;
     const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
-    if (!role.active) return;
+    if (!role.active) {
+        copy_beside(p.beside, lds_role);
+        return;
+    }
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int hs = role.hs, g = role.g;
@@ -1365,7 +1384,10 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
 
     if (threadIdx.x == 0) lds_abort = 0;
     const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
-    if (!role.active) return;
+    if (!role.active) {
+        copy_beside(p.beside, lds_role);
+        return;
+    }
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const int hs = role.hs, g = role.g;
     const int rotation = __builtin_amdgcn_readfirstlane(rec_kstep_rotation(hs, L.nh, ks_wave, L.rot_div));
@@ -2341,6 +2363,18 @@ static hipError_t launch_steps(StepGraphCache* graphs, const void* kernel, const
     return hipGraphLaunch(exec, stream);
 }
 
+int rec_idle_workgroups(const RecLayout& L) {
+    if (!L.persistent || L.two_d) return 0;
+    const int busy = L.ng * L.nh;
+    return busy < L.num_cus ? L.num_cus - busy : 0;
+}
+
+// A launch whose groups sit inside the XCDs always has one workgroup per CU, the others as many as they seat; those
+// get the helpers on top.
+static int grid_with_helpers(const RecLayout& L, const BesideCopies& c) {
+    return (L.xcd_local || c.count == 0) ? L.grid : L.grid + c.helpers;
+}
+
 template <int NT, int KS, bool RES, int MT, bool DS, bool DEEP = false>
 static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     constexpr int NW = 4;
@@ -2352,7 +2386,7 @@ static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
     hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
     if (e != hipSuccess) return e;
     const int ks_wave = rec_fwd_ks(L, a.Hp);
-    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
+    if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
                         [&]() -> hipError_t {
                             for (int t = a.t0; t < a.t1; ++t) {
@@ -2375,7 +2409,7 @@ static hipError_t run_fwd_il(const RecLayout& L, const RecFwdArgs& a, hipStream_
     hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
     if (e != hipSuccess) return e;
     const int ks_wave = rec_fwd_ks(L, a.Hp);
-    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
+    if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
                         [&]() -> hipError_t {
                             for (int t = a.t0; t < a.t1; ++t) {
@@ -2439,7 +2473,7 @@ static hipError_t run_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
     hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
     if (e != hipSuccess) return e;
     const int ks_wave = rec_bwd_ks(L, a.Hp);
-    if (L.persistent) return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, ks_wave, per_cu[device].load(), device, NW * kWave);
+    if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), lds, stream, a, L, a.t_hi, a.t_lo, ks_wave, per_cu[device].load(), device, NW * kWave);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t_hi, a.t_lo, a.t_hi - a.t_lo + 1,
                         stream, [&]() -> hipError_t {
                             for (int t = a.t_hi; t >= a.t_lo; --t) {

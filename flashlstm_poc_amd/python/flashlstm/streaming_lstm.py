@@ -127,6 +127,9 @@ class _StreamingLSTMFunction(torch.autograd.Function):
         ctx.save_for_backward(x_host, h0, c0, weight_ih, weight_hh, bias_ih, bias_hh, y_host, cache_h, cache_c)
         ctx.meta = (T, B, I, H, recompute_interval, h_code, c_code)
         ctx.mark_non_differentiable(cache_h, cache_c)
+        # a gradient nobody has stays None: materialized, those of the checkpoint arrays alone are 64 MiB of zeros on the
+        # host per backward pass (4 of the 22 ms of a pass over 2048 steps of 32 rows at 1024 units)
+        ctx.set_materialize_grads(False)
         return y_host, cache_h, cache_c, hy, cy
 
     @staticmethod
@@ -157,10 +160,10 @@ class _StreamingLSTMFunction(torch.autograd.Function):
         dx_host = torch.empty_like(x_host)
         if not dx_host.is_pinned():
             dx_host = torch.empty(x_host.shape, dtype=torch.float16, pin_memory=True)
-        dW_ih = torch.zeros_like(weight_ih)
-        dW_hh = torch.zeros_like(weight_hh)
-        db_ih = torch.zeros_like(bias_ih)
-        db_hh = torch.zeros_like(bias_hh)
+        dW_ih = torch.empty_like(weight_ih)
+        dW_hh = torch.empty_like(weight_hh)
+        db_ih = torch.empty_like(bias_ih)
+        db_hh = torch.empty_like(bias_hh)
         dh0 = torch.empty((B, H), device="cuda", dtype=torch.float32)
         dc0 = torch.empty_like(dh0)
 
