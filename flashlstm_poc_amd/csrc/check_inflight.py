@@ -1,12 +1,21 @@
 #!/usr/bin/env python3
-"""Static check of gfx950 device assembly for one hazard of hand-issued loads.
+"""Static check of gfx950 device assembly for two hazards of hand-issued loads.
 
 The recurrence kernels request their operand fragments (`global_load_dwordx4 ... sc1`) and the operands they stream
 from memory (`... nt`) in inline assembly and wait for them later with an explicit `s_waitcnt vmcnt(n)`.  The compiler does not know that the destination registers are
 still being written in between; if it copies, reads or reuses them there (a copy at a join of two definitions, a split
 live range) the kernel multiplies garbage.  This script walks the control-flow graph of the assembly from every such
-load and reports any instruction that names a destination register on a path before the first wait for vector memory.
+load and reports any instruction that names a destination register on a path before the first wait that covers it.
+A wait for vector memory covers a load if it leaves no more operations outstanding than were issued after it.
 Branches on flags that the path itself has set to a constant are followed only the way the flag points.
+
+A use that validates what it finds (the comparison with the 'unwritten' pattern) may come after a wait that does not cover
+the newest request: where a reload loop has requested fragments again, the older request into the same registers has
+landed, and what it brought is either the pattern or the data.
+
+The second hazard: a vector-memory instruction must not read a scalar register within five wait states of a vector
+instruction writing it (v_readlane / v_readfirstlane, which is how spilled scalars come back).  The compiler keeps that
+distance for its own instructions and does not look into inline assembly.
 
 usage: check_inflight.py file.s [...]      exit status 1 if a hazard is found
 """
@@ -15,7 +24,12 @@ import sys
 
 # hand-issued loads carry a cache policy the compiler never emits for its own loads of these kernels: sc1 (device
 # scope: the exchanged fragments) or nt (the operands streamed from memory one or two phases ahead)
-LOAD = re.compile(r'^\s+global_load_dword(?:x2|x4)? v\[(\d+):(\d+)\], .*\b(?:sc1|nt)\s*$')
+LOAD = re.compile(r'^\s+global_load_(?:dword|dwordx2|dwordx4|ushort) (?:v\[(\d+):(\d+)\]|v(\d+)), .*\b(?:sc1|nt)\s*$')
+# everything that counts into vmcnt (operations complete in issue order)
+VMEM = re.compile(r'^(?:global|buffer|flat|scratch)_(?:load|store|atomic)')
+SADDR = re.compile(r'^\s+global_load_(?:dword|dwordx2|dwordx4|ushort) \S+ v\d+, s\[(\d+):(\d+)\].*\b(?:sc1|nt)\s*$')
+LANE_TO_SCALAR = re.compile(r'^(?:v_readlane_b32|v_readfirstlane_b32) s(\d+)')
+VMCNT = re.compile(r'vmcnt\((\d+)\)')
 LABEL = re.compile(r'^([.\w$]+):')
 REG = re.compile(r'\bv\[(\d+):(\d+)\]|\bv(\d+)\b')
 
@@ -90,23 +104,27 @@ def check(path):
         m = LOAD.match(l)
         if not m:
             continue
-        a, b = int(m.group(1)), int(m.group(2))
+        a, b = (int(m.group(1)), int(m.group(2))) if m.group(1) else (int(m.group(3)), int(m.group(3)))
         seen = set()
-        stack = step(i, {}, None)
+        # (line, known flags, vcc, operations issued after the load, a wait has been passed)
+        stack = [st + (0, False) for st in step(i, {}, None)]
         while stack:
-            k, known, vcc = stack.pop()
-            key = (k, tuple(sorted(known.items())), vcc)
+            k, known, vcc, younger, waited = stack.pop()
+            key = (k, tuple(sorted(known.items())), vcc, younger, waited)
             if key in seen or k >= len(lines):
                 continue
             seen.add(key)
             t = lines[k].strip()
             if not t or t.startswith(';') or t.startswith('.') or LABEL.match(lines[k]):
-                stack.extend(step(k, known, vcc))
+                stack.extend(st + (younger, waited) for st in step(k, known, vcc))
                 continue
             if t.startswith('s_waitcnt') and 'vmcnt' in t:
-                continue   # the path ends at the first wait for vector memory
+                if younger >= int(VMCNT.search(t).group(1)):
+                    continue   # landed
+                stack.extend(st + (younger, True) for st in step(k, known, vcc))
+                continue
             m2 = LOAD.match(lines[k])
-            if m2 and int(m2.group(1)) == a and int(m2.group(2)) == b:
+            if m2 and int(m2.group(1) or m2.group(3)) == a and int(m2.group(2) or m2.group(3)) == b:
                 continue   # requested again into the same registers (a reload loop)
             code = t.split(';')[0]
             hit = False
@@ -114,15 +132,40 @@ def check(path):
                 lo = int(r.group(1) or r.group(3))
                 hi = int(r.group(2) or r.group(3))
                 if lo <= b and hi >= a:
+                    if waited and re.match(r'v_max3?_u32', code):
+                        hit = True   # (validates what it finds)
+                        break
                     hazards.append((i + 1, a, b, k + 1, code.strip()))
                     hit = True
                     break
             if hit:
                 continue   # (one report per path)
-            stack.extend(step(k, known, vcc))
+            n = min(younger + (1 if VMEM.match(code) else 0), 63)
+            stack.extend(st + (n, waited) for st in step(k, known, vcc))
+    # ---- scalar base written by a vector instruction just before
+    close = []
+    for i, l in enumerate(lines):
+        m = SADDR.match(l)
+        if not m:
+            continue
+        states, k = 0, i - 1
+        while states < 5 and k >= 0:
+            t = lines[k].split(';')[0].strip()
+            if t and not t.startswith('.') and not LABEL.match(lines[k]):
+                if t.startswith('s_nop'):
+                    states += int(t.split()[1], 0) + 1
+                else:
+                    w = LANE_TO_SCALAR.match(t)
+                    if w and int(m.group(1)) <= int(w.group(1)) <= int(m.group(2)):
+                        close.append((path, i + 1, l.strip(), k + 1, t))
+                        break
+                    states += 1
+            k -= 1
+    for h in close[:40]:
+        print('%s: load at line %d (%s) reads a scalar that line %d writes too shortly before: %s' % h)
     for h in hazards[:40]:
         print('%s: load at line %d into v[%d:%d] is in flight when line %d runs: %s' % ((path,) + h))
-    return len(hazards)
+    return len(hazards) + len(close)
 
 
 if __name__ == '__main__':

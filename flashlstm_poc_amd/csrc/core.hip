@@ -270,7 +270,7 @@ extern "C" int flstm_core_create(size_t batch, size_t input_size, size_t hidden_
     p->d.I = int(input_size);
     p->d.H = int(hidden_size);
     p->d.Ip = int(round_up(input_size, 64));
-    p->d.Hp = int(round_up(hidden_size, 32));
+    p->d.Hp = int(round_up(hidden_size, hidden_size > 2048 ? 64 : 32));   // (the wide backward kernel has 64-column slices)
     // Persistent launches go through the gate of launch_persistent; FLASHLSTM_COOPERATIVE_LAUNCH=1 or the option
     // "cooperative" sends them through hipLaunchCooperativeKernel instead (not under a rocprofiler-sdk tool: with rocprofv3
     // attached, a process that has made a cooperative launch takes a segmentation fault inside the tool when it exits).
@@ -406,7 +406,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     FL_TRY(p->wfrag_f.reserve(size_t(p->Lf.nh) * p->Lf.nw * p->ks_f * p->Lf.nt * kWave * sizeof(half8)));
     FL_TRY(p->wfrag_b.reserve(size_t(p->Lb.nh) * p->Lb.nw * p->ks_b * p->Lb.nt * kWave * sizeof(half8)));
     FL_TRY(pack_weights(d, w_ih, w_hh, p->wih_p.as<half_t>(), p->wih_t.as<half_t>(), p->wfrag_f.as<half8>(),
-                        p->ks_f, p->Lf.nt, p->Lf.rot_div, p->Lf.nw, p->wfrag_b.as<half8>(), p->ks_b, p->Lb.nt,
+                        p->ks_f, p->Lf.nt, p->Lf.rot_div, p->Lf.nw, p->Lf.unit_major, p->Lf.wide, p->wfrag_b.as<half8>(), p->ks_b, p->Lb.nt,
                         p->Lb.rot_div, p->Lb.nw, s));
     if (rec_bwd_two_d_possible(d.Hp, p->num_cus)) {   // whether or not the current layout uses them
         FL_TRY(p->wfrag_b2.reserve(rec_bwd_two_d_wfrag_bytes(d.Hp)));

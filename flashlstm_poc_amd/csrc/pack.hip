@@ -34,12 +34,12 @@ __global__ void pack_wih_kernel(Dims d, const float* __restrict__ w_ih, half_t* 
 
 // Forward fragments: B operand of  gates[b][c] += h[b][k] * W_hh[row(c)][k].  The product's columns are local to
 // a workgroup (they only meet the pointwise stage through LDS) and stay gate-major within the slice of JB = 4*NT
-// units: column c = gate * JB + unit.  With eight waves per workgroup (rec_fwd_il_kernel) they are unit-major,
-// column c = 4 * unit + gate: the four accumulation registers of a lane are then the four gates of one unit.
+// units: column c = gate * JB + unit.  In the kernels with one cell per thread (rec_fwd_il_kernel,
+// rec_fwd_wide_kernel) they are unit-major, column c = 4 * unit + gate: the four accumulation registers of a lane are then the four gates of one unit.
 // fragment (hs, wave, ks, n): lane l holds column c = n*16 + l%16 of slice hs,
 // k = (ks*nw + wave)*32 + 8*(l/16) + e, e = 0..7 (nw = wavefronts per workgroup, 4 or 8).
 __global__ void pack_wfrag_fwd_kernel(Dims d, const float* __restrict__ w_hh, half_t* __restrict__ out,
-                                      int ks_wave, int nt, int rot_div, int nw) {
+                                      int ks_wave, int nt, int rot_div, int nw, int unit_major, int wide) {
     const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;  // one half element
     const int nh = d.Hp / (4 * nt);
     const size_t total = size_t(nh) * nw * ks_wave * nt * kWave * 8;
@@ -52,9 +52,10 @@ __global__ void pack_wfrag_fwd_kernel(Dims d, const float* __restrict__ w_hh, ha
     const int wave = int(r % nw); r /= nw;
     const int hs = int(r);
     const int jb = 4 * nt, c = n * 16 + lane % 16;
-    const int gate = (nw == 8) ? c % 4 : c / jb, unit = hs * jb + ((nw == 8) ? c / 4 : c % jb);
-    // (slot ks of slice hs holds a rotated k-step: recurrent.h, rec_kstep_rotation)
-    const int kstep = rec_kstep_of_slot(ks, rec_kstep_rotation(hs, nh, ks_wave, rot_div), ks_wave);
+    const int gate = unit_major ? c % 4 : c / jb, unit = hs * jb + (unit_major ? c / 4 : c % jb);
+    // (slot ks of slice hs holds a rotated k-step: recurrent.h, rec_kstep_rotation, rec_wide_rotation)
+    const int kstep = wide ? (ks ^ rec_wide_rotation(ks, hs / 8, ks_wave))
+                           : rec_kstep_of_slot(ks, rec_kstep_rotation(hs, nh, ks_wave, rot_div), ks_wave);
     const int k = (kstep * nw + wave) * 32 + 8 * (lane / 16) + e;
     out[idx] = (half_t)((unit < d.H && k < d.H) ? w_hh[size_t(gate * d.H + unit) * d.H + k] : 0.f);
 }
@@ -91,9 +92,10 @@ __global__ void pack_wfrag_bwd_kernel(Dims d, const float* __restrict__ w_hh, ha
 // and the eight packed gate rows (4 Hp / kq) q + 32 (4 ks + wave) + 8 (l / 16) .. +7.
 __global__ void pack_wfrag_bwd2d_kernel(Dims d, const float* __restrict__ w_hh, half_t* __restrict__ out, int kq) {
     const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    const size_t total = size_t(4) * d.Hp * d.Hp;
+    const bool wide = d.Hp > 2048;
+    const int ksn = wide ? rec_wide_ks(d.Hp) : d.Hp / (32 * kq);   // k-steps per wave: 4 waves * ksn * 32 = 4 Hp / kq packed gate rows (wide: or more, zeros)
+    const size_t total = size_t(d.Hp / 64) * kq * 4 * ksn * 4 * kWave * 8;
     if (idx >= total) return;
-    const int ksn = d.Hp / (32 * kq);   // k-steps per wave: 4 waves * ksn * 32 = 4 Hp / kq packed gate rows
     size_t r = idx;
     const int e = int(r % 8); r /= 8;
     const int lane = int(r % kWave); r /= kWave;
@@ -104,10 +106,10 @@ __global__ void pack_wfrag_bwd2d_kernel(Dims d, const float* __restrict__ w_hh, 
     const int sl = int(r);
     const int k = sl * 64 + n * 16 + lane % 16;
     // (slot ks of a wave holds the k-step the kernel fetches there: rotated per column slice)
-    const int kstep = rec_kstep_of_slot(ks, rec_bwd2d_rotation(sl, ksn, kq), ksn);
-    const int q = qs * (4 * d.Hp / kq) + (kstep * 4 + wave) * 32 + 8 * (lane / 16) + e;
+    const int kstep = wide ? (ks ^ rec_wide_rotation(ks, sl / 8, ksn)) : rec_kstep_of_slot(ks, rec_bwd2d_rotation(sl, ksn, kq), ksn);
+    const int in_slice = (kstep * 4 + wave) * 32 + 8 * (lane / 16) + e, q = qs * (4 * d.Hp / kq) + in_slice;
     float v = 0.f;
-    if (q < 4 * d.Hp && k < d.H) {
+    if (in_slice < 4 * d.Hp / kq && k < d.H) {
         const int row = torch_row(q, d.H);
         if (row >= 0) v = w_hh[size_t(row) * d.H + k];
     }
@@ -255,13 +257,14 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
 }  // namespace
 
 hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p, half_t* wih_t,
-                        half8* wfrag_fwd, int ks_fwd, int nt_fwd, int rot_div_fwd, int nw_fwd, half8* wfrag_bwd, int ks_bwd,
+                        half8* wfrag_fwd, int ks_fwd, int nt_fwd, int rot_div_fwd, int nw_fwd, int unit_major_fwd, int wide_fwd, half8* wfrag_bwd, int ks_bwd,
                         int nt_bwd, int rot_div_bwd, int nw_bwd, hipStream_t s) {
     const size_t n1 = size_t(4) * d.Hp * d.Ip;
     hipLaunchKernelGGL(pack_wih_kernel, dim3(grid_for(n1)), dim3(kT), 0, s, d, w_ih, wih_p, wih_t);
     const size_t n2 = size_t(d.Hp / (4 * nt_fwd)) * nw_fwd * ks_fwd * nt_fwd * kWave * 8;
     hipLaunchKernelGGL(pack_wfrag_fwd_kernel, dim3(grid_for(n2)), dim3(kT), 0, s, d, w_hh,
-                       reinterpret_cast<half_t*>(wfrag_fwd), ks_fwd, nt_fwd, rot_div_fwd, nw_fwd);
+                       reinterpret_cast<half_t*>(wfrag_fwd), ks_fwd, nt_fwd, rot_div_fwd, nw_fwd,
+                       unit_major_fwd, wide_fwd);
     const size_t n3 = size_t(d.Hp / (16 * nt_bwd)) * nw_bwd * ks_bwd * nt_bwd * kWave * 8;
     hipLaunchKernelGGL(pack_wfrag_bwd_kernel, dim3(grid_for(n3)), dim3(kT), 0, s, d, w_hh,
                        reinterpret_cast<half_t*>(wfrag_bwd), ks_bwd, nt_bwd, rot_div_bwd, nw_bwd);
@@ -270,8 +273,8 @@ hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, hal
 
 hipError_t pack_wfrag_bwd2d(const Dims& d, const float* w_hh, half8* out, int kq, hipStream_t s) {
     // Hp / 64 slices of 64 columns, kq slices of 4 Hp / kq packed gate rows, 8 or 16 k-steps per wave
-    if (!((d.Hp == 2048 && (kq == 4 || kq == 8)) || (d.Hp == 1024 && kq == 2))) return hipErrorInvalidValue;
-    const size_t n = size_t(4) * d.Hp * d.Hp;
+    if (!((d.Hp == 2048 && (kq == 4 || kq == 8)) || (d.Hp == 1024 && kq == 2) || (d.Hp > 2048 && d.Hp % 64 == 0 && kq == 4))) return hipErrorInvalidValue;
+    const size_t n = rec_bwd_two_d_wfrag_bytes(d.Hp) / sizeof(half_t);
     hipLaunchKernelGGL(pack_wfrag_bwd2d_kernel, dim3(grid_for(n)), dim3(kT), 0, s, d, w_hh, reinterpret_cast<half_t*>(out), kq);
     return hipGetLastError();
 }

@@ -7,6 +7,11 @@
 
 namespace flstm_hip {
 
+// k-steps per wave (32 wide) that the kernels for more than 2048 hidden units are built for: 512 units' worth at a time.
+__host__ __device__ inline int rec_wide_ks(int Hp) { return (Hp / 32 + 15) / 16 * 4; }
+// Slot `slot` of a wave holds k-step slot ^ rec_wide_rotation(...) there; r: the slice among those that share an XCD.
+__host__ __device__ inline int rec_wide_rotation(int slot, int r, int ks) { return slot < ks / 8 * 8 ? (r & 7) : (r & 3); }
+
 // How the hidden dimension is cut over workgroups, and how workgroups are tied into groups that
 // exchange h_t (forward) or dG_t (backward) every step.
 struct RecLayout {
@@ -23,6 +28,9 @@ struct RecLayout {
     int grid;        // workgroups per launch
     int cooperative; // host side: 1 = persistent launches go through hipLaunchCooperativeKernel (set by the plan), 0 = through
                      // launch_persistent's own gate
+    int unit_major;  // forward: gate columns of a slice are packed 4 * unit + gate (kernels with one cell per thread), else gate
+                     // blocks of jb units
+    int wide;        // more than 2048 hidden units, weights resident (rec_fwd_wide_kernel, rec_bwd_wide_kernel)
     int num_cus;     // of the device the layout was made for
     int rot_div;     // k-step rotation (rec_kstep_rotation): slices rot_div apart run on the same XCD
     int two_d;       // backward, 2048 hidden units: workgroups split the product over output columns AND the contraction

@@ -215,6 +215,10 @@ __device__ __forceinline__ void wait_frags(half8 (&a)[2]) {
     asm volatile("s_waitcnt vmcnt(%2)" : "+v"(a[0]), "+v"(a[1]) : "n"(N) : "memory");
 }
 template <int N>
+__device__ __forceinline__ void wait_frags(half8 (&a)[1]) {
+    asm volatile("s_waitcnt vmcnt(%1)" : "+v"(a[0]) : "n"(N) : "memory");
+}
+template <int N>
 __device__ __forceinline__ void wait_frags(half8 (&a)[2], half8 (&b)[2]) {
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]) : "n"(N) : "memory");
 }
@@ -1358,6 +1362,571 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
     clk.flush();
 }
 
+// ---------------------------------------------------------------------- more than 2048 hidden units
+// W_hh of 4096 units is 128 MiB.  Streamed from memory every step that is 27 us forward and 90 us backward at 32 rows;
+// the chip holds 128 MiB of registers and 40 MiB of LDS, so up to 4096 units it can stay resident: 512 KiB per workgroup,
+// per wave KS - KL k-steps in registers and KL in LDS.  What is left of the registers (112 of 512) decides the rest.
+// Batch rows are taken in tiles of 16, one after the other (a second tile's accumulators would not fit), one cell per
+// thread.  A tile costs a CU 128 fragment loads of 1 KiB (1 us through its vector-memory path at 4096 units) and 128
+// MFMAs per wave (0.9 us); its exchange through memory hides behind the other tiles of the batch.
+//
+// Slot k of a wave holds k-step k ^ r: the workgroups of an XCD that fetch the same operand start in different places
+// (r differs), so that the XCD as a whole requests different lines instead of many times the same ones, and an address is ONE
+// exclusive-or of a per-lane offset with a constant.  r stays inside groups of eight k-steps (four in a last half group:
+// rec_wide_rotation).
+// Which slots of a wave keep their weights in LDS: every third one from the start, so that a chunk has at most one and the
+// last chunks, with the operands of the cells on their way into registers of their own, have none.
+__host__ __device__ constexpr bool wide_in_lds(int k, int KL) { return k % 3 == 0 && k / 3 < KL; }
+__host__ __device__ constexpr int wide_lds_before(int k, int KL) { return (k + 2) / 3 < KL ? (k + 2) / 3 : KL; }
+
+struct WideOperand {
+    unsigned lane;        // 16 * lane + 1024 * wave: this lane's place in k-step 0 of the wave, in bytes
+    unsigned full, half;  // ... with the rotation of a group of eight / of four
+    unsigned last;        // ... in the last k-step there is (slots past the contraction hold zero weights and fetch that)
+    __device__ __forceinline__ WideOperand(int lane_, int wave, int r, int nks) {
+        lane = unsigned(lane_) * 16u + unsigned(wave) * 1024u;
+        full = lane ^ (unsigned(r & 7) << 12);
+        half = lane ^ (unsigned(r & 3) << 12);
+        last = unsigned(lane_) * 16u + unsigned(nks - 1) * 1024u;
+    }
+};
+
+// Buffers of partial sums [4 waves][16][64 + pad] beside KL k-steps of weights in the 160 KiB of LDS.
+__host__ __device__ constexpr int wide_part_buffers(int KL) { return KL >= 8 ? 1 : 2; }
+
+// acc[n] += the 16 rows of `tile` (fragment-major, the same address in every lane) times this wave's weights: wave_product
+// for these kernels.  Chunks of CK k-steps rotate through NBUF register sets.  LAZY and the reload loop: as there.
+// `prefetch` issues exactly NPF vector loads behind the last fragment load.
+template <int KS, int KL, int NPF, bool LAZY, int CK, int NBUF, typename Prefetch>
+__device__ __forceinline__ bool wide_product(floatx4 (&acc)[2][4], const half8 (&wreg)[KS - KL][4], const half8* wlds,
+                                             const half_t* tile, const WideOperand& op, int lane, const Poll& poll,
+                                             Prefetch&& prefetch) {
+    constexpr int NT = 4, NCH = KS / CK, D = NBUF - 1;   // D chunks in flight while one is multiplied
+    static_assert(KS % 4 == 0 && KL * 3 <= KS - 6, "whole chunks; LDS k-steps end before the last three chunks");
+    half8 f[NBUF][CK];
+    bool check_all = !LAZY, early = false, ahead_of_producers = false;
+    // (opaque: offsets are computed where they are used, not all of them ahead of the step loop in registers that are not there)
+    unsigned full = op.full, half = op.half;
+    asm volatile("" : "+v"(full), "+v"(half));
+    for (;;) {
+    const half_t* base = wave_uniform(tile);
+    auto issue = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < CK; ++k) {
+            const int slot = c * CK + k;
+            unsigned off = (slot < KS / 8 * 8 ? full : half) ^ (unsigned(slot) << 12);
+            if (slot >= (KS % 8 == 0 ? KS - 8 : KS - 4)) off = min(off, op.last);   // (the contraction ends in the last four k-steps of a kernel)
+            ld_frag_async_at(f[c % NBUF][k], off, base);
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < D; ++c) issue(c);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+        const int buf = c % NBUF;
+        if (c + D < NCH) {
+            issue(c + D);
+            if (c + D == NCH - 1) prefetch();
+        }
+        half8 wl[CK][NT];
+#pragma unroll
+        for (int k = 0; k < CK; ++k)
+            if (wide_in_lds(c * CK + k, KL)) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n) wl[k][n] = wlds[(wide_lds_before(c * CK + k, KL) * NT + n) * kWave + lane];
+            }
+        const int last_now = (c + D < NCH - 1) ? c + D : NCH - 1;
+        wait_frags_upto(f[buf], (last_now - c) * CK + (c + D >= NCH - 1 ? NPF : 0));
+        auto unwritten = [&]() -> bool {
+            unsigned m = 0u;
+#pragma unroll
+            for (int k = 0; k < CK; ++k) {
+                const uint4 ua = __builtin_bit_cast(uint4, f[buf][k]);
+                m = max(m, max(max(ua.x, ua.y), max(ua.z, ua.w)));
+            }
+            return __any(m == kUnwritten) != 0;
+        };
+        if (c == 0 || (c <= D && early) || __builtin_expect(check_all, 0)) {
+            if (__builtin_expect(unwritten() && poll.on, 0)) {
+                if (c == 0) early = true;
+                if (c == 0) ahead_of_producers = true;
+                int spins = 0;
+                long long spin_start = 0;
+                do {
+                    if (poll_give_up(poll, spins, spin_start, lane)) break;
+                    issue(c);
+                    if constexpr (!LAZY) {   // (what was requested ahead of it is as stale: wave_product_tiles, REASK)
+#pragma unroll
+                        for (int j = c + 1; j <= last_now; ++j) issue(j);
+                        wait_frags_upto(f[buf], (last_now - c) * CK);
+                    } else {
+                        wait_frags<0>(f[buf]);
+                    }
+                } while (unwritten());
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < CK; ++k)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                half8 w;
+                if (wide_in_lds(c * CK + k, KL)) w = wl[k][n];
+                else w = wreg[c * CK + k - wide_lds_before(c * CK + k, KL)][n];
+                acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, f[buf][k], acc[0][n], 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);   // (chunks stay apart: a scheduler free to move later chunks up runs out of registers)
+    }
+    if (__builtin_expect(check_all || !poll.on || !product_poisoned<1>(acc), 1)) break;
+    check_all = true;
+    // (the wait as in wave_product_tiles.  The copies are made behind it: the registers they go to may be the ones that the
+    // loads of `prefetch` still write.)
+    asm volatile("s_waitcnt vmcnt(0)\n\tv_mov_b32 %0, %2\n\tv_mov_b32 %1, %3" : "=&v"(full), "=&v"(half) : "v"(op.full), "v"(op.half) : "memory");
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[0][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    return ahead_of_producers;
+}
+
+// A wave's weights: slots in registers and in LDS.  What fits the accumulation registers is told to live there (left to
+// itself the register allocator parks it there and copies it back in front of every MFMA: rec_bwd2d_kernel).
+template <int KS, int KL>
+__device__ __forceinline__ void wide_load_weights(half8 (&wreg)[KS - KL][4], half8* wlds, const half8* wfrag_wave, int lane) {
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const half8 w = wfrag_wave[(size_t(k) * 4 + n) * kWave + lane];
+            if (wide_in_lds(k, KL)) wlds[(wide_lds_before(k, KL) * 4 + n) * kWave + lane] = w;
+            else wreg[k - wide_lds_before(k, KL)][n] = w;
+        }
+#pragma unroll
+    for (int k = 0; k < (KS - KL < 15 ? KS - KL : 15); ++k)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) asm volatile("" : "+a"(wreg[k][n]));
+}
+
+// Loads from a scalar base (the same for the whole wave) + 32 bits of offset per lane, in bytes: a 64-bit address per lane
+// and load would take registers that are not there.
+__device__ __forceinline__ void ld_at(uintx2& d, const void* base, unsigned off) {
+    asm volatile("global_load_dwordx2 %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void ld_at(unsigned& d, const void* base, unsigned off) {
+    asm volatile("global_load_dword %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void ld_half_at(unsigned& d, const void* base, unsigned off) {
+    asm volatile("global_load_ushort %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+// past the L1: what this lane, or another CU of the XCD, has stored earlier
+__device__ __forceinline__ void ld_coherent_at(unsigned& d, const void* base, unsigned off) {
+    asm volatile("global_load_dword %0, %1, %2 sc1" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void ld_coherent_at(uintx4& d, const void* base, unsigned off) {
+    asm volatile("global_load_dwordx4 %0, %1, %2 sc1" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+// Phase counters of workgroup 0 (PhaseClock) with everything in LDS.
+struct WideClock {
+    long long* out;
+    __device__ __forceinline__ long long* lds() {
+        __shared__ long long mem[8];   // 0..4 phases, 5 engine clock at the start, 6 wall clock at the start, 7 last lap
+        return mem;
+    }
+    __device__ __forceinline__ void start() {
+        if (out && threadIdx.x == 0) {
+            for (int i = 0; i < 5; ++i) lds()[i] = 0;
+            lds()[6] = lds()[7] = wall_clock64();
+            lds()[5] = clock64();
+        }
+    }
+    __device__ __forceinline__ void lap(int slot) {
+        if (__builtin_expect(out != nullptr, 0)) {
+            if (threadIdx.x == 0) {
+                const long long now = wall_clock64();
+                lds()[slot] += now - lds()[7];
+                lds()[7] = now;
+            }
+        }
+    }
+    __device__ __forceinline__ void flush() {
+        if (out && threadIdx.x == 0) {
+            for (int i = 0; i < 5; ++i) out[i] += lds()[i];
+            out[5] += clock64() - lds()[5];
+            out[6] += wall_clock64() - lds()[6];
+        }
+    }
+};
+// the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
+__device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
+__device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
+__device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
+__device__ __forceinline__ unsigned as_bits(float v) { return __builtin_bit_cast(unsigned, v); }
+
+// Forward: a workgroup owns the 64 gate columns of 16 units over the whole contraction.  Gate columns are packed
+// unit-major, so a thread finds the four gate sums of its cell in one 16-byte LDS read per wave.
+// MANY: several tiles per step.  The operand of a tile is then complete when a workgroup gets to it, and is validated by
+// its effect; the cell state is prefetched with the x-projection, any number of tiles.  With one tile every wave is ahead
+// of its producers: word-by-word checks, first requests held back, the cell state carried in a register.
+template <int KS, int KL, bool MANY>
+__global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, RecLayout L, int t_begin, int t_end, int) {
+    constexpr int NW = 4, NT = 4, JB = 16;
+    constexpr int PLD = 16 * NT + kPartPad;
+    extern __shared__ __attribute__((aligned(16))) float part_all[];  // [2][NW][16][PLD] | weight fragments of KL k-steps
+    __shared__ int lds_abort;
+    __shared__ int lds_role[2];
+    if (threadIdx.x == 0) lds_abort = 0;
+    const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
+    if (!role.active) {
+        copy_beside(p.beside, lds_role);
+        return;
+    }
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+    const int hs = role.hs, g = role.g;
+    const int nks_total = p.Hp / 32;
+    const bool device_scope = L.persistent != 0;
+    const Poll poll{L.persistent != 0, p.spin_limit, p.spin_ticks, p.status, (lds_int_t*)&lds_abort};
+    WideClock clk{(blockIdx.x == 0) ? p.prof : nullptr};
+    int item = 0;
+    FirstRequestDelay first_request;
+    first_request.start_from(p.delay_hint);
+
+    half8 wreg[KS - KL][NT];
+    half8* wlds = reinterpret_cast<half8*>(part_all + 2 * NW * 16 * PLD) + size_t(wave) * KL * NT * kWave;
+    wide_load_weights<KS, KL>(wreg, wlds, p.wfrag + (size_t(hs) * NW + wave) * size_t(KS) * NT * kWave, lane);
+    const WideOperand op(lane, wave, hs / 8, nks_total);
+
+    // this thread's cell of a tile: row r, unit j
+    const int r = tid / JB, u = tid % JB, j = hs * JB + u;
+    const size_t gld = size_t(4) * p.Hp;
+    uintx2 xp;
+    unsigned cp_bits;
+    float carried = 0.f;
+    auto prefetch = [&](int t, int rb) __attribute__((always_inline)) {   // rows past B fetch row B-1 and are not used
+        const unsigned row = unsigned(min(r, p.B - 1 - rb * 16)), cell = row * unsigned(p.Hp) + unsigned(j);
+        const size_t row0 = size_t(t) * p.B + rb * 16;
+        ld_at(xp, p.G + row0 * gld, cell * 8u);
+        // (this thread's own store of the step before; another tile's wait has drained it since)
+        ld_coherent_at(cp_bits, p.C + row0 * p.Hp, cell * 4u);
+    };
+    if (p.stamps && t_begin == p.t0 && hs == 0 && g == 0 && tid == 0) p.stamps[0] = wall_clock64();
+    __syncthreads();
+    loads_landed();
+    clk.start();
+
+    for (int t = t_begin; t < t_end; ++t) {
+        for (int rb = g; rb < L.nrb; rb += L.ng, ++item) {
+            float* part = part_all + size_t(item & 1) * NW * 16 * PLD;
+            const half_t* tile = p.X + size_t(t & 3) * p.x_slot + size_t(rb) * nks_total * 512;   // h_{t-1}, fragment-major
+            half_t* xout = p.X + size_t((t + 1) & 3) * p.x_slot;         // h_t
+            half_t* xnext = p.X + size_t((t + 3) & 3) * p.x_slot;        // will take h_{t+2}: marked unwritten
+            floatx4 acc[2][NT];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[0][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (!MANY) first_request.hold();
+            const bool ahead = wide_product<KS, KL, 2, MANY, 2, 4>(acc, wreg, wlds, tile, op, lane, poll,
+                                                             [&]() __attribute__((always_inline)) { prefetch(t, rb); });
+            if constexpr (!MANY) first_request.learn(ahead);
+            clk.lap(0);
+            spill_partials16<NT>(part, acc, wave, lane, PLD);
+            __syncthreads();
+            if (lds_abort != 0) leave_kernel();
+            clk.lap(1);
+            wait_all_vm();   // x-projection and cell state; and the marks of the step before are in place
+            settle(xp);
+            settle(cp_bits);
+            clk.lap(4);
+            const int b = rb * 16 + r;
+            const bool live = b < p.B;
+            const bool first_of_four = (u % 4) == 0;
+            const unsigned xoff = unsigned(xch_offset(b, j, nks_total));
+            // (every peer has delivered h_{t-1}, so all of them are done reading h_{t-2}: see rec_fwd_kernel)
+            if (first_of_four) store_xch(xnext + xoff, Pack<4>{uintx2{kUnwritten, kUnwritten}}, device_scope);
+            float z[4];
+            unpack_h2(xp.x, z[0], z[1]);
+            unpack_h2(xp.y, z[2], z[3]);
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const floatx4 v = *reinterpret_cast<const floatx4*>(part + (size_t(w) * 16 + r) * PLD + 4 * u);
+                z[0] += v.x; z[1] += v.y; z[2] += v.z; z[3] += v.w;
+            }
+            const float cp = (!MANY && t > t_begin) ? carried : as_float(cp_bits);
+            const float ig = sigmoidf_dev(z[0]), fg = sigmoidf_dev(z[1]), gg = tanhf_dev(z[2]), og = sigmoidf_dev(z[3]);
+            const float cnew = fg * cp + ig * gg;
+            carried = cnew;
+            const float hn = og * tanhf_dev(cnew);
+            // four units of a row into 8 bytes (rows past B travel as zeros)
+            const unsigned hbits = live ? pack_h2(hn, 0.f) : 0u;
+            const unsigned pair = hbits | (quad_xor1(hbits) << 16);   // (in even lanes)
+            const Pack<4> h4{uintx2{pair, quad_xor2(pair)}};
+            if (first_of_four) store_xch(xout + xoff, h4, device_scope);
+            clk.lap(2);
+            // caches for the backward pass: off the critical path
+            if (live) {
+                const size_t row = size_t(t) * p.B + b;
+                p.C[(row + p.B) * p.Hp + j] = cnew;
+                if (first_of_four) {
+                    st_pack(p.Y + (row + p.B) * p.Hp + j, h4);
+                    if (p.y_out) st_pack(p.y_out + row * p.Hp + j, h4);
+                }
+                __builtin_nontemporal_store(uintx2{pack_h2(ig, fg), pack_h2(gg, og)}, reinterpret_cast<uintx2*>(p.G + row * gld + size_t(4) * j));
+            }
+            clk.lap(3);
+        }
+    }
+    if constexpr (!MANY) first_request.leave(p.delay_hint);
+    if (p.stamps && hs == 0 && g == 0 && tid == 0) p.stamps[1] = wall_clock64();
+    clk.flush();
+}
+
+// Backward: the product dh = dG_{t+1} * W_hh is split over 64-column slices s and four slices q of the contraction, as in
+// rec_bwd2d_kernel below (whose two rings and their protocol these are: dG through 8 slots with marks, fp32 partial sums
+// through 3 slots tagged with the parity of the step): a workgroup fetches a quarter of dG_{t+1}, forms a partial product
+// [16 rows][64], sends 16 columns to each of the four workgroups of its slice -- seated in one XCD -- and finishes 16 units.
+// MANY: (step, tile) items form ONE pipeline that does not stop at the end of a step: the product of item m, then the
+// cells of item m-1, whose partial sums have arrived meanwhile.  What the cells of item m-1 need from memory is requested behind
+// the fragment loads of item m, so no load is in flight from one item to the next.  With one tile per step an item's
+// product and cells follow each other.
+template <int KS, int KL, bool MANY>
+__global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, RecLayout L, int t_first, int t_last, int) {
+    constexpr int NW = 4, NT = 4, KQ = 4;
+    constexpr int PLD = 16 * NT + kPartPad;
+    constexpr int kSlots = 8;   // of the dG ring
+    constexpr int kParts = wide_part_buffers(KL);
+    extern __shared__ __attribute__((aligned(16))) float part_all[];  // [kParts][NW][16][PLD] | weight fragments of KL k-steps
+    __shared__ int lds_abort;
+    __shared__ int lds_role[2];
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+    if (tid == 0) {
+        lds_abort = 0;
+        const int xcd = int(xcc_id()) & 7;
+        const unsigned seat = __hip_atomic_fetch_add(p.seats + xcd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (seat >= 32u) __hip_atomic_store(p.status, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lds_role[0] = xcd;
+        lds_role[1] = int(seat);
+    }
+    __syncthreads();
+    if (lds_role[1] >= 32) return;
+    // seats of an XCD: [8 column slices][4 contraction slices]; the slices are dealt over the XCDs
+    const int seat = __builtin_amdgcn_readfirstlane(lds_role[1]), xcd = __builtin_amdgcn_readfirstlane(lds_role[0]);
+    const int q = seat % KQ, s = (seat / KQ) * 8 + xcd;
+    if (s * 64 >= p.Hp) {
+        copy_beside(p.beside, lds_role);
+        return;
+    }
+    const int nks = p.Hp / 8;            // k-steps of the whole contraction: nks / 4 per slice
+    const int nm = L.nrb;
+    const Poll poll{true, p.spin_limit, p.spin_ticks, p.status, (lds_int_t*)&lds_abort};
+    const float S = p.dy_scale;
+    WideClock clk{(blockIdx.x == 0) ? p.prof : nullptr};
+    FirstRequestDelay first_request;
+    first_request.start_from(p.delay_hint);
+
+    half8 wreg[KS - KL][NT];
+    half8* wlds = reinterpret_cast<half8*>(part_all + kParts * NW * 16 * PLD) + size_t(wave) * KL * NT * kWave;
+    wide_load_weights<KS, KL>(wreg, wlds, p.wfrag2 + ((size_t(s) * KQ + q) * NW + wave) * size_t(KS) * NT * kWave, lane);
+    const WideOperand op(lane, wave, seat / KQ, nks / KQ);
+
+    // As a sender a thread sums row r, columns 4c .. 4c+3 of the partial product; as a receiver it collects columns
+    // 4 (c / 4) .. of sender c % 4 for row r and ends up with one of them: the cell (row r, unit j).
+    const int r = tid / 16, c = tid % 16, j = s * 64 + q * 16 + c;
+    const size_t gld = size_t(4) * p.Hp;
+    const unsigned inbox0 = unsigned(s * KQ + q) * unsigned(nm), outbox0 = unsigned(s * KQ + c / 4) * unsigned(nm);
+    const unsigned in_at = (unsigned(c % 4) * 16u + unsigned(r)) * 16u + 4u * unsigned(c / 4);
+    const unsigned out_at = (unsigned(q) * 16u + unsigned(r)) * 16u + 4u * unsigned(c % 4);
+    __shared__ floatx4 db_sum[kThreads];   // bias-gradient sums of this thread's column (in LDS: registers)
+    db_sum[tid] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float dc_carried = 0.f;   // !MANY: the running dc of this thread's cell
+
+    // what the cells of an item need, and their partial sums: six loads
+    uintx2 o_gates;
+    unsigned o_cp, o_cc, o_dy, o_dc;
+    uintx4 o_in;
+    auto part_slot = [&](int t) __attribute__((always_inline)) { return p.P + size_t((t + 3) % kRecBwdPartSlots) * p.p_slot; };
+    auto request_inbox = [&](int t, int rb) __attribute__((always_inline)) {
+        ld_coherent_at(o_in, part_slot(t) + size_t(inbox0 + unsigned(rb)) * 1024u, in_at * 4u);
+    };
+    auto request_ops = [&](int t, int rb) __attribute__((always_inline)) {   // five loads; rows past B fetch row B-1, the closing pass step 0
+        const unsigned row = unsigned(min(r, p.B - 1 - rb * 16)), cell = row * unsigned(p.Hp) + unsigned(j);
+        const size_t row0 = size_t(max(t, 0)) * p.B + rb * 16;
+        ld_at(o_gates, p.G + row0 * gld, cell * 8u);
+        ld_at(o_cp, p.C + row0 * p.Hp, cell * 4u);
+        ld_at(o_cc, p.C + (row0 + p.B) * p.Hp, cell * 4u);
+        ld_half_at(o_dy, p.dY + row0 * p.Hp, cell * 2u);
+        ld_coherent_at(o_dc, p.dC + size_t(rb) * 16 * p.Hp, cell * 4u);
+    };
+    auto settle_ops = [&]() __attribute__((always_inline)) { settle(o_gates); settle(o_cp); settle(o_cc); settle(o_dy); settle(o_dc); };
+    // dh of this thread's cell of (t, rb): the four senders' columns, once they carry this step's parity
+    auto collect = [&](int t, int rb) __attribute__((always_inline)) -> float {
+        const unsigned par = unsigned(t) & 1u;
+        auto stale = [&]() -> bool {
+            const unsigned all1 = o_in.x & o_in.y & o_in.z & o_in.w, any1 = o_in.x | o_in.y | o_in.z | o_in.w;
+            return __any(par ? (all1 & 1u) == 0u : (any1 & 1u) != 0u) != 0;
+        };
+        if (stale()) {
+            int spins = 0;
+            long long spin_start = 0;
+            do {
+                if (poll_give_up(poll, spins, spin_start, lane)) break;
+                request_inbox(t, rb);
+                wait_all_vm();
+                settle(o_in);
+            } while (stale());
+        }
+        const bool hi2 = (lane & 2) != 0, hi1 = (lane & 1) != 0;
+        const float a0 = as_float(hi2 ? o_in.z : o_in.x) + as_float(quad_xor2(hi2 ? o_in.x : o_in.z));
+        const float a1 = as_float(hi2 ? o_in.w : o_in.y) + as_float(quad_xor2(hi2 ? o_in.y : o_in.w));
+        return (hi1 ? a1 : a0) + as_float(quad_xor1(as_bits(hi1 ? a0 : a1)));
+    };
+    auto cell = [&](int t, int rb, float dh, float dc_in) __attribute__((always_inline)) {
+        const int b = rb * 16 + r;
+        const bool live = b < p.B;
+        const unsigned at = unsigned(r) * unsigned(p.Hp) + unsigned(j);   // this cell in the tile's rows of a [..][Hp] array
+        float* const dc_tile = p.dC + size_t(rb) * 16 * p.Hp;
+        if (t < 0) {   // closing pass: gradient wrt h0; dc0 is the running dc
+            if (live) {
+                (p.dH0 + size_t(rb) * 16 * p.Hp)[at] = dh;
+                dc_tile[at] = dc_in;
+            }
+            return;
+        }
+        half_t* xout = p.X + size_t((t + 8) & (kSlots - 1)) * p.x_slot;     // dG_t for everybody
+        half_t* xmark = p.X + size_t((t + 11) & (kSlots - 1)) * p.x_slot;   // dG_{t+3}: read by nobody any more
+        const unsigned off = unsigned(xch_offset(b, 4 * j, nks));
+        store_xch(xmark + off, Pack<4>{uintx2{kUnwritten, kUnwritten}}, true);
+        Pack<4> out{uintx2{0u, 0u}};   // batch rows past B travel as zeros
+        float dc_out = 0.f;
+        if (live) {
+            float gate[4], dy, unused;
+            unpack(Pack<4>{o_gates}, gate);
+            unpack_h2(o_dy & 0xffffu, dy, unused);
+            const float ig = gate[0], fg = gate[1], gg = gate[2], og = gate[3];
+            const float dhu = dh + S * dy;
+            const float tc = tanhf_dev(as_float(o_cc));
+            const float dov = dhu * tc;
+            const float dc = dc_in + dhu * og * (1.f - tc * tc);
+            float da[4];
+            da[0] = dc * gg * ig * (1.f - ig);
+            da[1] = dc * as_float(o_cp) * fg * (1.f - fg);
+            da[2] = dc * ig * (1.f - gg * gg);
+            da[3] = dov * og * (1.f - og);
+            dc_out = dc * fg;
+            out = pack(da);
+            float v[4];   // db sums the values the weight-gradient GEMMs will see (fp16-rounded)
+            unpack(out, v);
+            db_sum[tid] += floatx4{v[0], v[1], v[2], v[3]};
+        }
+        store_xch(xout + off, out, true);
+        if (live) {
+            st_pack(p.dG + (size_t(t) * p.B + rb * 16) * gld + 4u * at, out);
+            if (MANY || t == t_last) dc_tile[at] = dc_out;
+        }
+        dc_carried = dc_out;
+    };
+    // the product of (t, rb), summed over the waves and sent to the workgroups of the slice
+    int item = 0;
+    auto multiply = [&](int t, int rb, auto npf, auto&& prefetch) __attribute__((always_inline)) {
+        float* part = part_all + size_t(kParts == 2 ? item & 1 : 0) * NW * 16 * PLD;
+        const half_t* tile = p.X + size_t((t + 9) & (kSlots - 1)) * p.x_slot + (size_t(rb) * nks + size_t(q) * (nks / KQ)) * 512;   // dG_{t+1}
+        floatx4 acc[2][NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[0][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (!MANY) first_request.hold();
+        const bool ahead = wide_product<KS, KL, decltype(npf)::value, MANY, 2, 4>(acc, wreg, wlds, tile, op, lane, poll, prefetch);
+        if constexpr (!MANY) first_request.learn(ahead);
+        clk.lap(0);
+        if constexpr (kParts == 1) __syncthreads();   // everyone has read the last item's sums
+        spill_partials16<NT>(part, acc, wave, lane, PLD);
+        ++item;
+        __syncthreads();
+        if (lds_abort != 0) leave_kernel();
+        floatx4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) v += *reinterpret_cast<const floatx4*>(part + (size_t(w) * 16 + r) * PLD + 4 * c);
+        uintx4 tagged = __builtin_bit_cast(uintx4, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tagged[e] = (tagged[e] & ~1u) | (unsigned(t) & 1u);
+        // what the loads behind the fragments brought is here, and everything stored so far is acknowledged (the marks of
+        // the items before are in place ahead of what comes next)
+        wait_all_vm();
+        *reinterpret_cast<uintx4*>(part_slot(t) + size_t(outbox0 + unsigned(rb)) * 1024u + out_at) = tagged;
+        clk.lap(1);
+    };
+
+    __syncthreads();
+    loads_landed();
+    clk.start();
+    int t = t_first;
+    if (t >= p.T - 1) {   // the last step of the sequence: dh comes from the caller
+        for (int rb = 0; rb < nm; ++rb) {
+            request_ops(t, rb);
+            unsigned dhn;
+            ld_at(dhn, p.dHn + size_t(rb) * 16 * p.Hp, (unsigned(min(r, p.B - 1 - rb * 16)) * unsigned(p.Hp) + unsigned(j)) * 4u);
+            wait_all_vm();
+            settle_ops();
+            settle(dhn);
+            cell(t, rb, as_float(dhn), as_float(o_dc));
+        }
+        --t;
+    } else if constexpr (!MANY) {
+        request_ops(t, 0);
+        wait_all_vm();
+        settle_ops();
+        dc_carried = as_float(o_dc);
+    }
+    if constexpr (MANY) {
+        bool have_prev = false;
+        int pt = 0, prb = 0;   // the item whose cells are to be done
+        for (; t >= t_last; --t) {
+            for (int rb = 0; rb < nm; ++rb) {
+                // (the first item of a launch requests operands of its own, which nobody uses)
+                const int ot = have_prev ? pt : t, orb = have_prev ? prb : rb;
+                multiply(t, rb, std::integral_constant<int, 6>{}, [&]() __attribute__((always_inline)) { request_ops(ot, orb); request_inbox(ot, orb); });
+                settle_ops();
+                settle(o_in);
+                if (have_prev) {
+                    const float dh = collect(pt, prb);
+                    clk.lap(4);
+                    cell(pt, prb, dh, as_float(o_dc));
+                    clk.lap(2);
+                }
+                have_prev = true;
+                pt = t;
+                prb = rb;
+            }
+        }
+        if (have_prev) {   // the last item's cells
+            request_ops(pt, prb);
+            request_inbox(pt, prb);
+            wait_all_vm();
+            settle_ops();
+            settle(o_in);
+            const float dh = collect(pt, prb);
+            cell(pt, prb, dh, as_float(o_dc));
+        }
+    } else {
+        for (; t >= t_last; --t) {
+            multiply(t, 0, std::integral_constant<int, 5>{}, [&]() __attribute__((always_inline)) { request_ops(t, 0); });
+            settle_ops();
+            request_inbox(t, 0);
+            wait_all_vm();
+            settle(o_in);
+            const float dh = collect(t, 0);
+            clk.lap(4);
+            cell(t, 0, dh, dc_carried);
+            clk.lap(2);
+        }
+        first_request.leave(p.delay_hint);
+    }
+    if (p.stamp_end && s == 0 && q == 0 && tid == 0) *p.stamp_end = wall_clock64();
+    clk.flush();
+    // Bias gradient: fold this launch's sums over the 16 rows (fixed order).
+    __syncthreads();
+    if (tid < 64) {
+        const int col = tid / 4, gt = tid % 4;
+        float sum = 0.f;
+        for (int row = 0; row < 16; ++row) sum += db_sum[row * 16 + col][gt];
+        p.db_part[size_t(4) * (s * 64 + q * 16 + col) + gt] += sum;
+    }
+}
+
 // ----------------------------------------------------------------------------------- backward
 // Gate order and the pointwise derivative follow flashlstm_v2/src/lstm_backward.cu:199-211, except
 // that c_{t-1}, c_t come from the cell-state cache instead of being rebuilt through atanh.
@@ -2153,7 +2722,10 @@ void persistent_stream_idle(hipStream_t stream) {
 
 size_t exchange_slot_halfs(int rows, int cols) { return round_up(size_t(rows), 32) * size_t(cols); }
 
-int rec_fwd_ks(const RecLayout& L, int Hp) { return int(ceil_div(size_t(Hp) / 32, size_t(L.nw))); }
+int rec_fwd_ks(const RecLayout& L, int Hp) {
+    const size_t ks = ceil_div(size_t(Hp) / 32, size_t(L.nw));
+    return int(L.resident && Hp > 2048 ? round_up(ks, 4) : ks);   // (the wide kernels are built for whole groups of four)
+}
 int rec_bwd_ks(const RecLayout& L, int Hp) { return int(ceil_div(size_t(Hp) / 8, size_t(L.nw))); }
 
 // Wavefronts per workgroup of the forward recurrence: eight (rec_fwd_il_kernel: the two row tiles of a 32-row block
@@ -2172,6 +2744,8 @@ int rec_waves(int B, int Hp, int num_cus, int waves) {
     return (!can_16 && one_block_each) ? 8 : 4;
 }
 
+constexpr int kWideMost = 4096;   // hidden units whose W_hh the chip can hold (rec_fwd_wide_kernel)
+
 static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_stepwise, bool fits, int force_mt) {
     L.nh = Hp / L.jb;
     L.resident = fits ? 1 : 0;
@@ -2183,13 +2757,14 @@ static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_s
     const bool can_16 = fits && int(ceil_div(size_t(B), 16)) <= side_by_side;
     L.mt = can_16 ? 1 : 2;
     if (force_mt == 2 || (force_mt == 1 && can_16)) L.mt = force_mt;   // a tuned choice; 16-row blocks only where they fit
+    if (fits && Hp > 2048) L.mt = 1;   // the kernels for more than 2048 units take 16-row tiles one after the other
     if (L.nw == 8) L.mt = 2;   // the eight-wave kernels take 32-row blocks (their two row tiles take turns)
     L.nrb = int(ceil_div(size_t(B), size_t(16 * L.mt)));
     L.xcd_local = 0;
     L.gpx = 0;
     if (!fits || force_stepwise || L.nh > num_cus) {
         L.persistent = 0;
-        L.ng = L.nrb;
+        L.ng = (fits && Hp > 2048) ? 1 : L.nrb;   // (512 KiB of weights per workgroup: loaded once per step, not once per tile)
         L.grid = L.ng * L.nh;
         return;
     }
@@ -2211,11 +2786,13 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.num_cus = num_cus;
     bool fits = true;
     if (Hp <= 1024) L.nt = 8;
-    else if (Hp <= 2048) L.nt = 4;
+    else if (Hp <= kWideMost && Hp / 16 <= num_cus) L.nt = 4;
     else { L.nt = 8; fits = false; }
     L.nw = fits ? rec_waves(B, Hp, num_cus, waves) : 4;
     L.jb = 4 * L.nt;
+    L.unit_major = L.nw == 8 || (fits && Hp > 2048);
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
+    L.wide = fits && Hp > 2048;
     return L;
 }
 
@@ -2235,6 +2812,17 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     // reading in step is what lets the L2 serve one line to many).  A function of the sizes alone: the packed
     // weights depend on it.
     L.rot_div = (L.nh > 32) ? 8 : 0;
+    if (two_d > 0 && !force_stepwise && Hp > 2048 && rec_bwd_two_d_possible(Hp, num_cus)) {   // (rec_bwd_wide_kernel)
+        L.wide = 1;
+        L.persistent = 1;
+        L.two_d = 1;
+        L.kq = 4;
+        L.mt = 1;
+        L.nrb = L.nm = int(ceil_div(size_t(B), 16));
+        L.ng = 1;
+        L.grid = 256;
+        return L;
+    }
     if (two_d > 0 && L.persistent && rec_bwd_two_d_possible(Hp, num_cus)) {
         // 2048 units, more rows than the two-way kernel takes (two passes of 32 rows for each of two groups): batch rows
         // are independent sequences, so the batch is walked in windows of 128 rows, one persistent launch after the
@@ -2276,17 +2864,22 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     return L;
 }
 
-bool rec_bwd_two_d_possible(int Hp, int num_cus) { return (Hp == 2048 || Hp == 1024) && num_cus == 256; }
+bool rec_bwd_two_d_possible(int Hp, int num_cus) {
+    return (Hp == 2048 || Hp == 1024 || (Hp > 2048 && Hp <= kWideMost && Hp % 64 == 0)) && num_cus == 256;
+}
 // Up to two row blocks: 8 slices and one group (with two blocks every workgroup makes two passes per step, and one
 // block's trip through memory hides behind the other's product: 7.0 us per step at 64 rows against 8.0 with 4 slices and
 // two groups of one pass each).  More: 4 slices, two groups.
-int rec_bwd_two_d_kq(int B, int Hp) { return Hp == 1024 ? 2 : (B <= 64 ? 8 : 4); }
+int rec_bwd_two_d_kq(int B, int Hp) { return Hp == 1024 ? 2 : (B <= 64 && Hp == 2048 ? 8 : 4); }
 int rec_bwd_dg_slots(const RecLayout& L) { return L.two_d ? kDgSlots : 4; }
 size_t rec_bwd_part_slot_floats(const RecLayout& L) {
     // [256 workgroups][nm passes][kq senders][rows][64 / kq columns]
     return L.two_d ? size_t(256) * L.nm * 64 * (16 * L.mt) : 0;
 }
-size_t rec_bwd_two_d_wfrag_bytes(int Hp) { return size_t(Hp) * 4 * Hp * sizeof(half_t); }
+size_t rec_bwd_two_d_wfrag_bytes(int Hp) {
+    if (Hp > 2048) return size_t(Hp / 64) * 4 * 4 * rec_wide_ks(Hp) * 4 * kWave * sizeof(half8);
+    return size_t(Hp) * 4 * Hp * sizeof(half_t);
+}
 int rec_bwd_ring_rows(const RecLayout& L, int B) {
     return (L.two_d && L.win_rows) ? int(ceil_div(size_t(B), size_t(L.win_rows))) * L.win_rows : B;
 }
@@ -2364,8 +2957,8 @@ static hipError_t launch_steps(StepGraphCache* graphs, const void* kernel, const
 }
 
 int rec_idle_workgroups(const RecLayout& L) {
-    if (!L.persistent || L.two_d) return 0;
-    const int busy = L.ng * L.nh;
+    if (!L.persistent || (L.two_d && !L.wide)) return 0;
+    const int busy = L.wide && L.two_d ? L.nh * L.jb / 64 * L.kq : L.ng * L.nh;   // (nh, jb: the one-way layout)
     return busy < L.num_cus ? L.num_cus - busy : 0;
 }
 
@@ -2421,6 +3014,34 @@ static hipError_t run_fwd_il(const RecLayout& L, const RecFwdArgs& a, hipStream_
                         });
 }
 
+template <int KS, int KL>
+static hipError_t run_fwd_wide(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
+    constexpr int NW = 4;
+    const int ks_wave = rec_fwd_ks(L, a.Hp);
+    if (L.nw != NW || L.nt != 4 || L.mt != 1 || !L.resident || ks_wave != KS) return hipErrorInvalidValue;
+    const size_t lds = size_t(2) * NW * 16 * (64 + kPartPad) * sizeof(float) + size_t(NW) * KL * 4 * kWave * sizeof(half8);
+    auto launch = [&](auto kernel, std::atomic<int>* per_cu) -> hipError_t {
+        int device = 0;
+        hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
+        if (e != hipSuccess) return e;
+        if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
+        return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
+                            [&]() -> hipError_t {
+                                for (int t = a.t0; t < a.t1; ++t) {
+                                    hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(NW * kWave), lds, stream, a, L, t, t + 1, ks_wave);
+                                    hipError_t le = hipGetLastError();
+                                    if (le != hipSuccess) return le;
+                                }
+                                return hipSuccess;
+                            });
+    };
+    static std::atomic<int> many_per_cu[kMaxDevices], one_per_cu[kMaxDevices];
+    // with one tile per workgroup and step every wave is ahead of its producers: the operand is checked word by word and
+    // the first request held back; with several the operand is complete when a workgroup gets there
+    if (L.nrb > L.ng) return launch(rec_fwd_wide_kernel<KS, KL, true>, many_per_cu);
+    return launch(rec_fwd_wide_kernel<KS, KL, false>, one_per_cu);
+}
+
 template <int NT, int KS, int MT>
 static hipError_t run_fwd_ds(const RecLayout& L, const RecFwdArgs& a, bool ds, hipStream_t stream, StepGraphCache* graphs) {
     return ds ? run_fwd<NT, KS, true, MT, true>(L, a, stream, graphs) : run_fwd<NT, KS, true, MT, false>(L, a, stream, graphs);
@@ -2433,6 +3054,12 @@ hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
     const bool ds = L.persistent && !L.xcd_local;
     if (!L.resident) return run_fwd<8, 1, false, 2, false>(L, a, stream, graphs);
     const int ks = rec_fwd_ks(L, a.Hp);
+    if (a.Hp > 2048) {   // (one kernel per 512 units: all of its k-steps are multiplied)
+        if (ks == 20) return run_fwd_wide<20, 0>(L, a, stream, graphs);
+        if (ks == 24) return run_fwd_wide<24, 2>(L, a, stream, graphs);
+        if (ks == 28) return run_fwd_wide<28, 6>(L, a, stream, graphs);
+        return run_fwd_wide<32, 7>(L, a, stream, graphs);
+    }
     if (L.nw == 8) {   // eight waves: the interleaved kernel, 32-row blocks
         if (ks <= 2) return ds ? run_fwd_il<2, true>(L, a, stream, graphs) : run_fwd_il<2, false>(L, a, stream, graphs);
         return ds ? run_fwd_il<4, true>(L, a, stream, graphs) : run_fwd_il<4, false>(L, a, stream, graphs);
@@ -2502,9 +3129,34 @@ static hipError_t run_bwd2d(const RecLayout& L, const RecBwdArgs& a, hipStream_t
     return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
 }
 
+template <int KS, int KL>
+static hipError_t run_bwd_wide(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream) {
+    const size_t lds = size_t(wide_part_buffers(KL)) * 4 * 16 * (64 + kPartPad) * sizeof(float) + size_t(4) * KL * 4 * kWave * sizeof(half8);
+    auto launch = [&](auto kernel, std::atomic<int>* per_cu) -> hipError_t {
+        int device = 0;
+        hipError_t e = prepare_kernel(kernel, lds, kThreads, per_cu, &device);
+        if (e != hipSuccess) return e;
+        return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
+    };
+    static std::atomic<int> many_per_cu[kMaxDevices], one_per_cu[kMaxDevices];
+    if (L.nrb > 1) return launch(rec_bwd_wide_kernel<KS, KL, true>, many_per_cu);
+    return launch(rec_bwd_wide_kernel<KS, KL, false>, one_per_cu);
+}
+
 hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     if (a.T <= 0 || a.B <= 0 || a.t_hi < a.t_lo) return hipSuccess;
     if (a.Hp % 32 != 0 || a.Hp % L.jb != 0 || a.t_lo < -1 || a.t_hi >= a.T) return hipErrorInvalidValue;
+    if (L.wide) {
+        // what the kernel's indexing assumes
+        if (!L.persistent || !L.two_d || a.Hp % 64 != 0 || a.Hp <= 2048 || a.Hp > kWideMost || L.grid != 256 || L.ng != 1 || L.mt != 1 ||
+            L.nm != L.nrb || L.nrb * 16 < a.B || !a.wfrag2 || !a.P || a.p_slot != rec_bwd_part_slot_floats(L))
+            return hipErrorInvalidValue;
+        const int ks = rec_wide_ks(a.Hp);
+        if (ks == 20) return run_bwd_wide<20, 0>(L, a, stream);
+        if (ks == 24) return run_bwd_wide<24, 2>(L, a, stream);
+        if (ks == 28) return run_bwd_wide<28, 6>(L, a, stream);
+        return run_bwd_wide<32, 8>(L, a, stream);
+    }
     if (L.two_d) {
         // what the kernel's indexing assumes
         const bool local = a.Hp == 1024;

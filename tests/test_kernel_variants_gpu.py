@@ -19,3 +19,14 @@ def test_recurrence_kernels_by_contraction_length(B, H, stepwise):
     got, info = run_core(p, stepwise=stepwise)
     assert info["fallbacks"] == 0
     check_against(ref, got, label=f"B={B} H={H} stepwise={stepwise}")
+
+
+# more hidden units than 2048: one kernel per 512 units of the contraction, batch rows in tiles of 16 (one tile, a partial
+# second one, several), hidden sizes that are a multiple of nothing
+@pytest.mark.parametrize("B,H", [(1, 2049), (16, 2560), (17, 2561), (40, 3072), (3, 3100), (33, 3585), (2, 4096), (18, 4096)])
+def test_recurrence_kernels_for_wide_layers(B, H):
+    p = make_problem(4, B, 24, H, seed=B * 10000 + H)
+    ref, _ = oracle_reference(p)
+    got, info = run_core(p)
+    assert info["fallbacks"] == 0 and info["persistent_fwd"] == 1
+    check_against(ref, got, label=f"B={B} H={H}")
