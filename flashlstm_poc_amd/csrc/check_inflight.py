@@ -9,10 +9,6 @@ load and reports any instruction that names a destination register on a path bef
 A wait for vector memory covers a load if it leaves no more operations outstanding than were issued after it.
 Branches on flags that the path itself has set to a constant are followed only the way the flag points.
 
-A use that validates what it finds (the comparison with the 'unwritten' pattern) may come after a wait that does not cover
-the newest request: where a reload loop has requested fragments again, the older request into the same registers has
-landed, and what it brought is either the pattern or the data.
-
 The second hazard: a vector-memory instruction must not read a scalar register within five wait states of a vector
 instruction writing it (v_readlane / v_readfirstlane, which is how spilled scalars come back).  The compiler keeps that
 distance for its own instructions and does not look into inline assembly.
@@ -34,6 +30,7 @@ LABEL = re.compile(r'^([.\w$]+):')
 REG = re.compile(r'\bv\[(\d+):(\d+)\]|\bv(\d+)\b')
 
 
+HERE = 'every wave has lanes here'   # (every_wave_here() in the sources)
 SPAIR = re.compile(r'^s\[(\d+):(\d+)\]$')
 SREG = re.compile(r'^s(\d+)$')
 
@@ -64,6 +61,8 @@ def check(path):
         if op.startswith('s_cbranch'):
             tgt = label_at.get(ops[0])
             taken = None
+            if op == 's_cbranch_execz' and tgt is not None and i < tgt < i + 60 and any(HERE in l for l in lines[i:tgt]):
+                taken = False
             if op == 's_cbranch_vccnz' and vcc is not None:
                 taken = (vcc == 'nz')
             if op == 's_cbranch_vccz' and vcc is not None:
@@ -106,22 +105,22 @@ def check(path):
             continue
         a, b = (int(m.group(1)), int(m.group(2))) if m.group(1) else (int(m.group(3)), int(m.group(3)))
         seen = set()
-        # (line, known flags, vcc, operations issued after the load, a wait has been passed)
-        stack = [st + (0, False) for st in step(i, {}, None)]
+        # (line, known flags, vcc, operations issued after the load)
+        stack = [st + (0,) for st in step(i, {}, None)]
         while stack:
-            k, known, vcc, younger, waited = stack.pop()
-            key = (k, tuple(sorted(known.items())), vcc, younger, waited)
+            k, known, vcc, younger = stack.pop()
+            key = (k, tuple(sorted(known.items())), vcc, younger)
             if key in seen or k >= len(lines):
                 continue
             seen.add(key)
             t = lines[k].strip()
             if not t or t.startswith(';') or t.startswith('.') or LABEL.match(lines[k]):
-                stack.extend(st + (younger, waited) for st in step(k, known, vcc))
+                stack.extend(st + (younger,) for st in step(k, known, vcc))
                 continue
             if t.startswith('s_waitcnt') and 'vmcnt' in t:
                 if younger >= int(VMCNT.search(t).group(1)):
                     continue   # landed
-                stack.extend(st + (younger, True) for st in step(k, known, vcc))
+                stack.extend(st + (younger,) for st in step(k, known, vcc))
                 continue
             m2 = LOAD.match(lines[k])
             if m2 and int(m2.group(1) or m2.group(3)) == a and int(m2.group(2) or m2.group(3)) == b:
@@ -132,16 +131,13 @@ def check(path):
                 lo = int(r.group(1) or r.group(3))
                 hi = int(r.group(2) or r.group(3))
                 if lo <= b and hi >= a:
-                    if waited and re.match(r'v_max3?_u32', code):
-                        hit = True   # (validates what it finds)
-                        break
                     hazards.append((i + 1, a, b, k + 1, code.strip()))
                     hit = True
                     break
             if hit:
                 continue   # (one report per path)
             n = min(younger + (1 if VMEM.match(code) else 0), 63)
-            stack.extend(st + (n, waited) for st in step(k, known, vcc))
+            stack.extend(st + (n,) for st in step(k, known, vcc))
     # ---- scalar base written by a vector instruction just before
     close = []
     for i, l in enumerate(lines):

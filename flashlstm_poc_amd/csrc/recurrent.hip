@@ -133,6 +133,10 @@ struct Poll {
 // checker of the build (check_inflight.py) cannot tell that the wave is on its way out.
 __device__ __forceinline__ void leave_kernel() { asm volatile("s_endpgm" ::: "memory"); }
 
+// For check_inflight.py: every wave has lanes in the block this stands in, so the branch around it is never taken and the
+// operations in it can be counted on.
+__device__ __forceinline__ void every_wave_here() { asm volatile("; every wave has lanes here"); }
+
 // Said before a step loop: every load issued so far (the weight fragments, the state) has landed.  As an instruction
 // the compiler knows, not inline assembly: otherwise it meets the loop with loads it believes outstanding and puts
 // its own wait for ALL loads in front of the first MFMA of every step, behind the fragments requested ahead.
@@ -374,7 +378,10 @@ __device__ __forceinline__ bool wave_product_tiles(floatx4 (&acc)[2][NT], const 
                     if constexpr (REASK) {
 #pragma unroll
                         for (int j = c + 1; j <= last_issued; ++j) issue(j);
-                        wait_frags_upto(f[buf], (last_issued - c) * CKT);   // (what was in flight before has landed as well)
+                        // (What was in flight before has landed as well, the prefetch included: once that is out, the
+                        // waits of the chunks that follow would allow for operations that are not there, i.e. leave
+                        // fragments in flight into registers that the compiler hands on.  So nothing is left in flight.)
+                        wait_frags_upto(f[buf], last_issued == NCH - 1 ? 0 : (last_issued - c) * CKT);
                     } else {
                         wait_frags<0>(f[buf]);   // (whatever was in flight behind this chunk has landed as well)
                     }
@@ -539,7 +546,7 @@ __device__ __forceinline__ bool wave_product(floatx4 (&acc)[2][NT], const half8 
                         if constexpr (REASK && KS < 64) {
 #pragma unroll
                             for (int j = c + 1; j <= last_now; ++j) issue(j, j % NBUF);
-                            wait_with(last_now - c, false);   // (also what was issued after this chunk the first time)
+                            wait_with(prefetched ? 0 : last_now - c, false);   // (also what was issued after this chunk the first time; as in wave_product_tiles)
                         } else {
                             wait(std::integral_constant<int, 0>{}, buf);
                         }
@@ -1210,7 +1217,7 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
             half_t* xnext = p.X + size_t((pt + 3) & 3) * p.x_slot + size_t(2 * prb + ptl) * tile_halfs;
             // (its x-projection was requested two phases ago, and the wait for the last product's fragments has covered it)
             settle(xp[ptl]);
-            if (even) store_xch(xnext + off_ring, Pack<2>{kUnwritten}, DS);
+            if (even) { every_wave_here(); store_xch(xnext + off_ring, Pack<2>{kUnwritten}, DS); }
             unsigned hbits = 0u;
             if (live) {
                 float z[4];
@@ -1242,13 +1249,14 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
             // the neighbour's half: quad_perm(1, 0, 3, 2) swaps the lanes of a pair
             const unsigned other = unsigned(__builtin_amdgcn_mov_dpp(int(hbits), 0xB1, 0xF, 0xF, true));
             hpair = even ? (hbits | (other << 16)) : (other | (hbits << 16));
-            if (even) store_xch(xout + off_ring, Pack<2>{hpair}, DS);
+            if (even) { every_wave_here(); store_xch(xout + off_ring, Pack<2>{hpair}, DS); }
+        } else {
+            wait_all_vm();   // (no stores behind the fragment loads that the wait below could count)
         }
         clk.lap(2);
         // ---- the fragments: landed once at most the two ring stores issued behind them are outstanding
         // (ONE wait statement names the fragment registers: with one in each branch the compiler joins the two
         // definitions and may copy the registers on the way there, ahead of the wait, while the loads still write them)
-        if (!have_prev) wait_all_vm();
         wait_frags<2>(f);
         auto unwritten = [&]() -> bool {
             unsigned m = 0u;
@@ -1458,7 +1466,7 @@ __device__ __forceinline__ bool wide_product(floatx4 (&acc)[2][4], const half8 (
                     if constexpr (!LAZY) {   // (what was requested ahead of it is as stale: wave_product_tiles, REASK)
 #pragma unroll
                         for (int j = c + 1; j <= last_now; ++j) issue(j);
-                        wait_frags_upto(f[buf], (last_now - c) * CK);
+                        wait_frags_upto(f[buf], c + D >= NCH - 1 ? 0 : (last_now - c) * CK);   // (as in wave_product_tiles)
                     } else {
                         wait_frags<0>(f[buf]);
                     }
@@ -1563,13 +1571,14 @@ __device__ __forceinline__ unsigned as_bits(float v) { return __builtin_bit_cast
 // Forward: a workgroup owns the 64 gate columns of 16 units over the whole contraction.  Gate columns are packed
 // unit-major, so a thread finds the four gate sums of its cell in one 16-byte LDS read per wave.
 // MANY: several tiles per step.  The operand of a tile is then complete when a workgroup gets to it, and is validated by
-// its effect; the cell state is prefetched with the x-projection, any number of tiles.  With one tile every wave is ahead
+// its effect (checked word by word: 32 rows of 4096 units 5.2 -> 5.65 us per step, 128 rows 21.9 -> 23.2); the cell state is prefetched with the x-projection, any number of tiles.  With one tile every wave is ahead
 // of its producers: word-by-word checks, first requests held back, the cell state carried in a register.
-template <int KS, int KL, bool MANY>
+template <int KS, int KL, int NBUF, bool MANY>
 __global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, RecLayout L, int t_begin, int t_end, int) {
     constexpr int NW = 4, NT = 4, JB = 16;
     constexpr int PLD = 16 * NT + kPartPad;
-    extern __shared__ __attribute__((aligned(16))) float part_all[];  // [2][NW][16][PLD] | weight fragments of KL k-steps
+    constexpr int kParts = wide_part_buffers(KL);
+    extern __shared__ __attribute__((aligned(16))) float part_all[];  // [kParts][NW][16][PLD] | weight fragments of KL k-steps
     __shared__ int lds_abort;
     __shared__ int lds_role[2];
     if (threadIdx.x == 0) lds_abort = 0;
@@ -1589,7 +1598,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, Re
     first_request.start_from(p.delay_hint);
 
     half8 wreg[KS - KL][NT];
-    half8* wlds = reinterpret_cast<half8*>(part_all + 2 * NW * 16 * PLD) + size_t(wave) * KL * NT * kWave;
+    half8* wlds = reinterpret_cast<half8*>(part_all + kParts * NW * 16 * PLD) + size_t(wave) * KL * NT * kWave;
     wide_load_weights<KS, KL>(wreg, wlds, p.wfrag + (size_t(hs) * NW + wave) * size_t(KS) * NT * kWave, lane);
     const WideOperand op(lane, wave, hs / 8, nks_total);
 
@@ -1613,7 +1622,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, Re
 
     for (int t = t_begin; t < t_end; ++t) {
         for (int rb = g; rb < L.nrb; rb += L.ng, ++item) {
-            float* part = part_all + size_t(item & 1) * NW * 16 * PLD;
+            float* part = part_all + size_t(kParts == 2 ? item & 1 : 0) * NW * 16 * PLD;
             const half_t* tile = p.X + size_t(t & 3) * p.x_slot + size_t(rb) * nks_total * 512;   // h_{t-1}, fragment-major
             half_t* xout = p.X + size_t((t + 1) & 3) * p.x_slot;         // h_t
             half_t* xnext = p.X + size_t((t + 3) & 3) * p.x_slot;        // will take h_{t+2}: marked unwritten
@@ -1621,10 +1630,11 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, Re
 #pragma unroll
             for (int n = 0; n < NT; ++n) acc[0][n] = floatx4{0.f, 0.f, 0.f, 0.f};
             if constexpr (!MANY) first_request.hold();
-            const bool ahead = wide_product<KS, KL, 2, MANY, 2, 4>(acc, wreg, wlds, tile, op, lane, poll,
+            const bool ahead = wide_product<KS, KL, 2, MANY, 2, NBUF>(acc, wreg, wlds, tile, op, lane, poll,
                                                              [&]() __attribute__((always_inline)) { prefetch(t, rb); });
             if constexpr (!MANY) first_request.learn(ahead);
             clk.lap(0);
+            if constexpr (kParts == 1) __syncthreads();   // everyone has read the last tile's sums
             spill_partials16<NT>(part, acc, wave, lane, PLD);
             __syncthreads();
             if (lds_abort != 0) leave_kernel();
@@ -1680,15 +1690,19 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, Re
 // rec_bwd2d_kernel below (whose two rings and their protocol these are: dG through 8 slots with marks, fp32 partial sums
 // through 3 slots tagged with the parity of the step): a workgroup fetches a quarter of dG_{t+1}, forms a partial product
 // [16 rows][64], sends 16 columns to each of the four workgroups of its slice -- seated in one XCD -- and finishes 16 units.
-// MANY: (step, tile) items form ONE pipeline that does not stop at the end of a step: the product of item m, then the
+// kWidePipe: (step, tile) items form ONE pipeline that does not stop at the end of a step: the product of item m, then the
 // cells of item m-1, whose partial sums have arrived meanwhile.  What the cells of item m-1 need from memory is requested behind
-// the fragment loads of item m, so no load is in flight from one item to the next.  With one tile per step an item's
-// product and cells follow each other.
-template <int KS, int KL, bool MANY>
+// the fragment loads of item m, so no load is in flight from one item to the next.  It takes three tiles: with two, a product
+// follows the cells it depends on at once.  There (kWideTwo) and with one tile (kWideOne) an item's product and cells follow
+// each other: the trip of the partial sums is exposed, the one of dG hides behind the other tile.  Measured at 4096 units,
+// us per step, as a pipeline / one after the other: 32 rows 12.5 / 7.7, 48 rows 9.8 / 11.4, 64 rows 13.1 / 15.0.
+enum : int { kWideOne = 0, kWideTwo = 1, kWidePipe = 2 };
+template <int KS, int KL, int NBUF, int MODE>
 __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, RecLayout L, int t_first, int t_last, int) {
     constexpr int NW = 4, NT = 4, KQ = 4;
     constexpr int PLD = 16 * NT + kPartPad;
     constexpr int kSlots = 8;   // of the dG ring
+    constexpr bool PIPE = MODE == kWidePipe, ONE = MODE == kWideOne;
     constexpr int kParts = wide_part_buffers(KL);
     extern __shared__ __attribute__((aligned(16))) float part_all[];  // [kParts][NW][16][PLD] | weight fragments of KL k-steps
     __shared__ int lds_abort;
@@ -1733,7 +1747,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
     const unsigned out_at = (unsigned(q) * 16u + unsigned(r)) * 16u + 4u * unsigned(c % 4);
     __shared__ floatx4 db_sum[kThreads];   // bias-gradient sums of this thread's column (in LDS: registers)
     db_sum[tid] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float dc_carried = 0.f;   // !MANY: the running dc of this thread's cell
+    float dc_carried = 0.f;   // ONE: the running dc of this thread's cell
 
     // what the cells of an item need, and their partial sums: six loads
     uintx2 o_gates;
@@ -1816,7 +1830,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
         store_xch(xout + off, out, true);
         if (live) {
             st_pack(p.dG + (size_t(t) * p.B + rb * 16) * gld + 4u * at, out);
-            if (MANY || t == t_last) dc_tile[at] = dc_out;
+            if (!ONE || t == t_last) dc_tile[at] = dc_out;
         }
         dc_carried = dc_out;
     };
@@ -1828,9 +1842,9 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
         floatx4 acc[2][NT];
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[0][n] = floatx4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (!MANY) first_request.hold();
-        const bool ahead = wide_product<KS, KL, decltype(npf)::value, MANY, 2, 4>(acc, wreg, wlds, tile, op, lane, poll, prefetch);
-        if constexpr (!MANY) first_request.learn(ahead);
+        if constexpr (ONE) first_request.hold();
+        const bool ahead = wide_product<KS, KL, decltype(npf)::value, PIPE, 2, NBUF>(acc, wreg, wlds, tile, op, lane, poll, prefetch);
+        if constexpr (ONE) first_request.learn(ahead);
         clk.lap(0);
         if constexpr (kParts == 1) __syncthreads();   // everyone has read the last item's sums
         spill_partials16<NT>(part, acc, wave, lane, PLD);
@@ -1865,13 +1879,13 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
             cell(t, rb, as_float(dhn), as_float(o_dc));
         }
         --t;
-    } else if constexpr (!MANY) {
+    } else if constexpr (ONE) {
         request_ops(t, 0);
         wait_all_vm();
         settle_ops();
         dc_carried = as_float(o_dc);
     }
-    if constexpr (MANY) {
+    if constexpr (PIPE) {
         bool have_prev = false;
         int pt = 0, prb = 0;   // the item whose cells are to be done
         for (; t >= t_last; --t) {
@@ -1903,17 +1917,19 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
         }
     } else {
         for (; t >= t_last; --t) {
-            multiply(t, 0, std::integral_constant<int, 5>{}, [&]() __attribute__((always_inline)) { request_ops(t, 0); });
-            settle_ops();
-            request_inbox(t, 0);
-            wait_all_vm();
-            settle(o_in);
-            const float dh = collect(t, 0);
-            clk.lap(4);
-            cell(t, 0, dh, dc_carried);
-            clk.lap(2);
+            for (int rb = 0; rb < (ONE ? 1 : nm); ++rb) {
+                multiply(t, rb, std::integral_constant<int, 5>{}, [&]() __attribute__((always_inline)) { request_ops(t, rb); });
+                settle_ops();
+                request_inbox(t, rb);
+                wait_all_vm();
+                settle(o_in);
+                const float dh = collect(t, rb);
+                clk.lap(4);
+                cell(t, rb, dh, ONE ? dc_carried : as_float(o_dc));
+                clk.lap(2);
+            }
         }
-        first_request.leave(p.delay_hint);
+        if constexpr (ONE) first_request.leave(p.delay_hint);
     }
     if (p.stamp_end && s == 0 && q == 0 && tid == 0) *p.stamp_end = wall_clock64();
     clk.flush();
@@ -2494,7 +2510,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd2d_kernel(RecBwdArgs p, RecLa
 #pragma unroll
         for (int i = 0; i <= NM; ++i) {
             if (i > nmine) break;
-            const bool product = i < nmine, finish = i >= 1;
+            const bool product = i < NM && i < nmine, finish = i >= 1;
             const int rb = g + i * ng, rb_prev = g + (i - 1) * ng;
             uintx4 in0 = {0u, 0u, 0u, 0u}, in1 = {0u, 0u, 0u, 0u};
             // partials of block i-1 in this workgroup's inbox: sender pj % KQ, row pr, 8 columns from 8 * (pj / KQ)
@@ -3014,12 +3030,12 @@ static hipError_t run_fwd_il(const RecLayout& L, const RecFwdArgs& a, hipStream_
                         });
 }
 
-template <int KS, int KL>
+template <int KS, int KL, int NBUF>
 static hipError_t run_fwd_wide(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     constexpr int NW = 4;
     const int ks_wave = rec_fwd_ks(L, a.Hp);
     if (L.nw != NW || L.nt != 4 || L.mt != 1 || !L.resident || ks_wave != KS) return hipErrorInvalidValue;
-    const size_t lds = size_t(2) * NW * 16 * (64 + kPartPad) * sizeof(float) + size_t(NW) * KL * 4 * kWave * sizeof(half8);
+    const size_t lds = size_t(wide_part_buffers(KL)) * NW * 16 * (64 + kPartPad) * sizeof(float) + size_t(NW) * KL * 4 * kWave * sizeof(half8);
     auto launch = [&](auto kernel, std::atomic<int>* per_cu) -> hipError_t {
         int device = 0;
         hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
@@ -3038,8 +3054,8 @@ static hipError_t run_fwd_wide(const RecLayout& L, const RecFwdArgs& a, hipStrea
     static std::atomic<int> many_per_cu[kMaxDevices], one_per_cu[kMaxDevices];
     // with one tile per workgroup and step every wave is ahead of its producers: the operand is checked word by word and
     // the first request held back; with several the operand is complete when a workgroup gets there
-    if (L.nrb > L.ng) return launch(rec_fwd_wide_kernel<KS, KL, true>, many_per_cu);
-    return launch(rec_fwd_wide_kernel<KS, KL, false>, one_per_cu);
+    if (L.nrb > L.ng) return launch(rec_fwd_wide_kernel<KS, KL, NBUF, true>, many_per_cu);
+    return launch(rec_fwd_wide_kernel<KS, KL, NBUF, false>, one_per_cu);
 }
 
 template <int NT, int KS, int MT>
@@ -3055,10 +3071,10 @@ hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
     if (!L.resident) return run_fwd<8, 1, false, 2, false>(L, a, stream, graphs);
     const int ks = rec_fwd_ks(L, a.Hp);
     if (a.Hp > 2048) {   // (one kernel per 512 units: all of its k-steps are multiplied)
-        if (ks == 20) return run_fwd_wide<20, 0>(L, a, stream, graphs);
-        if (ks == 24) return run_fwd_wide<24, 2>(L, a, stream, graphs);
-        if (ks == 28) return run_fwd_wide<28, 6>(L, a, stream, graphs);
-        return run_fwd_wide<32, 7>(L, a, stream, graphs);
+        if (ks == 20) return run_fwd_wide<20, 4, 8>(L, a, stream, graphs);
+        if (ks == 24) return run_fwd_wide<24, 6, 8>(L, a, stream, graphs);
+        if (ks == 28) return run_fwd_wide<28, 7, 7>(L, a, stream, graphs);
+        return run_fwd_wide<32, 8, 5>(L, a, stream, graphs);
     }
     if (L.nw == 8) {   // eight waves: the interleaved kernel, 32-row blocks
         if (ks <= 2) return ds ? run_fwd_il<2, true>(L, a, stream, graphs) : run_fwd_il<2, false>(L, a, stream, graphs);
@@ -3129,7 +3145,7 @@ static hipError_t run_bwd2d(const RecLayout& L, const RecBwdArgs& a, hipStream_t
     return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
 }
 
-template <int KS, int KL>
+template <int KS, int KL, int NBUF>
 static hipError_t run_bwd_wide(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream) {
     const size_t lds = size_t(wide_part_buffers(KL)) * 4 * 16 * (64 + kPartPad) * sizeof(float) + size_t(4) * KL * 4 * kWave * sizeof(half8);
     auto launch = [&](auto kernel, std::atomic<int>* per_cu) -> hipError_t {
@@ -3138,9 +3154,10 @@ static hipError_t run_bwd_wide(const RecLayout& L, const RecBwdArgs& a, hipStrea
         if (e != hipSuccess) return e;
         return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
     };
-    static std::atomic<int> many_per_cu[kMaxDevices], one_per_cu[kMaxDevices];
-    if (L.nrb > 1) return launch(rec_bwd_wide_kernel<KS, KL, true>, many_per_cu);
-    return launch(rec_bwd_wide_kernel<KS, KL, false>, one_per_cu);
+    static std::atomic<int> pipe_per_cu[kMaxDevices], two_per_cu[kMaxDevices], one_per_cu[kMaxDevices];
+    if (L.nrb > 2) return launch(rec_bwd_wide_kernel<KS, KL, NBUF, kWidePipe>, pipe_per_cu);
+    if (L.nrb > 1) return launch(rec_bwd_wide_kernel<KS, KL, NBUF, kWideTwo>, two_per_cu);
+    return launch(rec_bwd_wide_kernel<KS, KL, NBUF, kWideOne>, one_per_cu);
 }
 
 hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
@@ -3152,10 +3169,10 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
             L.nm != L.nrb || L.nrb * 16 < a.B || !a.wfrag2 || !a.P || a.p_slot != rec_bwd_part_slot_floats(L))
             return hipErrorInvalidValue;
         const int ks = rec_wide_ks(a.Hp);
-        if (ks == 20) return run_bwd_wide<20, 0>(L, a, stream);
-        if (ks == 24) return run_bwd_wide<24, 2>(L, a, stream);
-        if (ks == 28) return run_bwd_wide<28, 6>(L, a, stream);
-        return run_bwd_wide<32, 8>(L, a, stream);
+        if (ks == 20) return run_bwd_wide<20, 4, 8>(L, a, stream);
+        if (ks == 24) return run_bwd_wide<24, 6, 8>(L, a, stream);
+        if (ks == 28) return run_bwd_wide<28, 7, 6>(L, a, stream);
+        return run_bwd_wide<32, 8, 4>(L, a, stream);
     }
     if (L.two_d) {
         // what the kernel's indexing assumes
