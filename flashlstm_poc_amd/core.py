@@ -54,6 +54,12 @@ def load_library() -> ctypes.CDLL:
     lib.flstm_core_forward.argtypes = [vp, sz, vp, i32, vp, vp, i32, vp, i32, vp, vp, i32, i32, vp]
     lib.flstm_core_forward_static.argtypes = [vp, sz, vp, i32, vp, vp, i32, vp, i32, vp, vp, i32, vp]
     lib.flstm_core_forward_static.restype = i32
+    lib.flstm_core_pack.argtypes = [vp, vp, vp, vp, vp, vp]
+    lib.flstm_core_absmax.argtypes = [vp, vp, i32, sz, c.POINTER(c.c_float), vp]
+    lib.flstm_stack_forward.argtypes = [vp, i32, sz, vp, i32, vp, vp, i32, vp, i32, vp, vp, vp]
+    lib.flstm_stack_backward.argtypes = [vp, i32, sz, vp, i32, vp, i32, c.c_float, vp, vp, i32, c.c_float, vp, i32] + [vp] * 7
+    for name in ("flstm_core_pack", "flstm_core_absmax", "flstm_stack_forward", "flstm_stack_backward"):
+        getattr(lib, name).restype = i32
     lib.flstm_core_tune.argtypes = [vp, sz, i32, i32, vp]
     lib.flstm_core_tune.restype = i32
     lib.flstm_core_tuned_ms.argtypes = [vp, sz, c.c_char_p]
@@ -180,6 +186,21 @@ class LstmCore:
         return taken
 
     def pack(self, w_ih, w_hh, b_ih=None, b_hh=None) -> None:
+        self._check_parameters(w_ih, w_hh, b_ih, b_hh)
+        rc = self.lib.flstm_core_pack_weights(self._h, w_ih.data_ptr(), w_hh.data_ptr(), self._stream())
+        if rc == 0:
+            rc = self.lib.flstm_core_pack_bias(self._h, _ptr(b_ih), _ptr(b_hh), self._stream())
+        if rc != 0:
+            raise RuntimeError(f"weight packing failed with status {rc}")
+
+    def _pack_enqueue(self, w_ih, w_hh, b_ih, b_hh, stream: int) -> None:
+        """pack() without its wait, for passes that follow on the same stream."""
+        self._check_parameters(w_ih, w_hh, b_ih, b_hh)
+        rc = self.lib.flstm_core_pack(self._h, w_ih.data_ptr(), w_hh.data_ptr(), _ptr(b_ih), _ptr(b_hh), stream)
+        if rc != 0:
+            raise RuntimeError(f"weight packing failed with status {rc}")
+
+    def _check_parameters(self, w_ih, w_hh, b_ih, b_hh) -> None:
         import torch
         for name, t, shape in (("w_ih", w_ih, (4 * self.H, self.I)), ("w_hh", w_hh, (4 * self.H, self.H))):
             if t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous() or tuple(t.shape) != shape:
@@ -187,11 +208,6 @@ class LstmCore:
         for name, t in (("b_ih", b_ih), ("b_hh", b_hh)):
             if t is not None and (t.dtype != torch.float32 or not t.is_cuda or t.numel() != 4 * self.H):
                 raise ValueError(f"{name} must be a CUDA float32 tensor with 4*hidden elements")
-        rc = self.lib.flstm_core_pack_weights(self._h, w_ih.data_ptr(), w_hh.data_ptr(), self._stream())
-        if rc == 0:
-            rc = self.lib.flstm_core_pack_bias(self._h, _ptr(b_ih), _ptr(b_hh), self._stream())
-        if rc != 0:
-            raise RuntimeError(f"weight packing failed with status {rc}")
 
     def forward(self, x, h0=None, c0=None, *, out_dtype=None, save_for_backward: bool = True,
                 want_y: bool = True) -> Tuple:

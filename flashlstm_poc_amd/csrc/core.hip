@@ -72,6 +72,13 @@ struct DevBuf {
 
 constexpr int kFirstHold = 8, kMaxHold = 1024;
 
+// Factors of a backward pass: on dY and on the incoming state gradients as they are read, on dx and on the parameter and
+// initial-state gradients as they are written.
+struct BwdScales {
+    float dy = 1.f, state = 1.f, dx = 1.f, grads = 1.f;
+    static BwdScales loss_scale(float S) { return BwdScales{S, S, 1.f / S, 1.f / S}; }
+};
+
 // The plan's status block on the device: word 0 the status, words 1 and 2 the delay hints of the two recurrences, the
 // time stamps of a pass, and sets of seat counters: every recurrence launch needs eight zeroed ones, so a pass that
 // launches several (ranges of steps, windows of rows) takes the sets its setup has zeroed one after the other.
@@ -127,7 +134,7 @@ struct flstm_core_plan {
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
              half_t* y_direct = nullptr; } fw;   // y_direct: the recurrence writes the caller's y itself
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
-             float S = 1.f, dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
+             BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
     BesideCopies beside_f, beside_b;   // for the next recurrence launch of a pass fed in ranges (core_copy_beside)
     // backward scratch
     DevBuf dYp, dG, dHn, dC, dH0, db_part, dw_part, prof, part_b;
@@ -199,6 +206,11 @@ int take_status(flstm_core_plan* p, hipStream_t s, int* out) {
         p->inject_stall--;
         *out = 1;
     }
+    return 0;
+}
+// a status nobody will look at (the pass is repeated because of another plan's) does not stay behind
+int clear_status(flstm_core_plan* p, hipStream_t s) {
+    if (*static_cast<volatile int*>(&p->status_host->status) != 0) FL_TRY(fill_zero(p->status.p, sizeof(int), s));
     return 0;
 }
 int wait_status(flstm_core_plan* p, OpList& last, int stamp, hipStream_t s, int* out) {
@@ -281,7 +293,7 @@ extern "C" int flstm_core_create(size_t batch, size_t input_size, size_t hidden_
         if (const char* v = getenv("FLASHLSTM_WAVES_FWD")) p->opt_waves_f = (atoi(v) == 4 || atoi(v) == 8) ? atoi(v) : 0;
     }
     replan(p);
-    e = p->status.reserve(kStatusBytes);
+    e = p->status.reserve(kStatusBytes + kAbsmaxBlocks * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(p->status.p, 0, kStatusBytes);
     if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&p->status_host), sizeof(HostStatus), hipHostMallocDefault);
     if (e == hipSuccess) memset(p->status_host, 0, sizeof(HostStatus));
@@ -405,13 +417,21 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     FL_TRY(p->wih_t.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
     FL_TRY(p->wfrag_f.reserve(size_t(p->Lf.nh) * p->Lf.nw * p->ks_f * p->Lf.nt * kWave * sizeof(half8)));
     FL_TRY(p->wfrag_b.reserve(size_t(p->Lb.nh) * p->Lb.nw * p->ks_b * p->Lb.nt * kWave * sizeof(half8)));
-    FL_TRY(pack_weights(d, w_ih, w_hh, p->wih_p.as<half_t>(), p->wih_t.as<half_t>(), p->wfrag_f.as<half8>(),
-                        p->ks_f, p->Lf.nt, p->Lf.rot_div, p->Lf.nw, p->Lf.unit_major, p->Lf.wide, p->wfrag_b.as<half8>(), p->ks_b, p->Lb.nt,
-                        p->Lb.rot_div, p->Lb.nw, s));
+    auto layout = [](const DevBuf& out, const RecLayout& L, int ks) {
+        FragLayout f;
+        f.out = out.as<half8>(); f.ks = ks; f.nt = L.nt; f.rot_div = L.rot_div; f.nw = L.nw; f.unit_major = L.unit_major;
+        return f;
+    };
+    FragLayout fwd = layout(p->wfrag_f, p->Lf, p->ks_f), bwd = layout(p->wfrag_b, p->Lb, p->ks_b), two_d;
+    fwd.wide = p->Lf.wide;
     if (rec_bwd_two_d_possible(d.Hp, p->num_cus)) {   // whether or not the current layout uses them
         FL_TRY(p->wfrag_b2.reserve(rec_bwd_two_d_wfrag_bytes(d.Hp)));
-        FL_TRY(pack_wfrag_bwd2d(d, w_hh, p->wfrag_b2.as<half8>(), rec_bwd_two_d_kq(d.B, d.Hp), s));
+        two_d.out = p->wfrag_b2.as<half8>();
+        two_d.kq = rec_bwd_two_d_kq(d.B, d.Hp);
+        two_d.wide = d.Hp > 2048;
+        two_d.ks = two_d.wide ? rec_wide_ks(d.Hp) : d.Hp / (32 * two_d.kq);
     }
+    FL_TRY(pack_weights(d, w_ih, w_hh, p->wih_p.as<half_t>(), p->wih_t.as<half_t>(), fwd, bwd, two_d, s));
     p->weights_packed = true;
     return 0;
 }
@@ -567,35 +587,38 @@ void final_states(const flstm_core_plan* p, size_t TB, void* hy, void* cy, flstm
     out.unpad(p->C.as<float>() + TB * d.Hp, 1, size_t(d.Hp), size_t(d.B), d.H, 1.f, cy, dtype == FLSTM_F32);
 }
 
-// One whole forward pass: projection, recurrence, outputs, one wait, status.  The outputs are written behind the
-// recurrence without waiting for its status: if the persistent launch gave up, the whole pass is repeated
-// step-wise and overwrites them.
-int forward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
-                 flstm_dtype state_dtype, void* y, flstm_dtype y_dtype, void* hy, void* cy,
-                 flstm_dtype out_state_dtype, hipStream_t s) {
+// One whole forward pass, enqueued: projection, recurrence, outputs, status.  The outputs are written behind the
+// recurrence without waiting for its status: if the persistent launch gave up, the whole pass is repeated step-wise
+// and overwrites them.
+int forward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
+                    flstm_dtype state_dtype, void* y, flstm_dtype y_dtype, void* hy, void* cy,
+                    flstm_dtype out_state_dtype, hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     use_tuned(p, T);
-    for (int attempt = 0;; ++attempt) {
-        // An fp16 output whose rows are the state rows is written by the persistent recurrence itself (no copy
-        // afterwards).  Step-wise launches leave it to the copy: every argument of theirs is then plan-owned, and
-        // the graph they were captured into can be replayed on the next pass.
-        half_t* const y_direct =
-            (y && y_dtype == FLSTM_F16 && d.H == d.Hp && p->Lf.persistent) ? static_cast<half_t*>(y) : nullptr;
-        p->fw.y_direct = y_direct;
-        int rc = forward_once(p, T, x, x_dtype, h0, c0, state_dtype, s);
-        p->fw.y_direct = nullptr;
-        if (rc) return rc;
-        OpList out;   // outputs and final states, one launch
-        if (!y_direct)
-            out.unpad(p->Y.as<half_t>() + size_t(d.B) * d.Hp, 0, size_t(d.Hp), TB, d.H, 1.f, y, y_dtype == FLSTM_F32);
-        final_states(p, TB, hy, cy, out_state_dtype, out);
-        int st = 0;
-        rc = wait_status(p, out, kStampFwdEnd, s, &st);
-        if (rc) return rc;
-        if (st == 0) break;
-        if (!p->Lf.persistent || attempt > 0) return FLSTM_E_STALLED;
-        demote(p, true);   // workgroups not co-resident or not where expected: redo with one launch per step
+    // An fp16 output whose rows are the state rows is written by the persistent recurrence itself (no copy afterwards).
+    // Step-wise launches leave it to the copy: every argument of theirs is then plan-owned, and the graph they were
+    // captured into can be replayed on the next pass.
+    half_t* const y_direct =
+        (y && y_dtype == FLSTM_F16 && d.H == d.Hp && p->Lf.persistent) ? static_cast<half_t*>(y) : nullptr;
+    p->fw.y_direct = y_direct;
+    int rc = forward_once(p, T, x, x_dtype, h0, c0, state_dtype, s);
+    p->fw.y_direct = nullptr;
+    if (rc) return rc;
+    OpList out;   // outputs and final states, one launch
+    if (!y_direct)
+        out.unpad(p->Y.as<half_t>() + size_t(d.B) * d.Hp, 0, size_t(d.Hp), TB, d.H, 1.f, y, y_dtype == FLSTM_F32);
+    final_states(p, TB, hy, cy, out_state_dtype, out);
+    return publish_with(p, out, kStampFwdEnd, s);
+}
+// ... once the stream has been waited for: FLSTM_E_STALLED if it has to be repeated (demoted if it was persistent)
+int forward_conclude(flstm_core_plan* p, hipStream_t s) {
+    int st = 0;
+    int rc = take_status(p, s, &st);
+    if (rc) return rc;
+    if (st != 0) {
+        if (p->Lf.persistent) demote(p, true);   // workgroups not co-resident or not where expected: next time with one launch per step
+        return FLSTM_E_STALLED;
     }
     pass_done(p, true);
     if (p->opt_profile) FL_TRY(hipMemcpy(p->prof_f, p->prof.p, sizeof(p->prof_f), hipMemcpyDeviceToHost));
@@ -604,6 +627,20 @@ int forward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtyp
     p->ms_fwd[2] = elapsed(p, kStampFwdStart, kStampFwdRecEnd);
     p->fw.open = false;
     return 0;
+}
+
+int forward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
+                 flstm_dtype state_dtype, void* y, flstm_dtype y_dtype, void* hy, void* cy,
+                 flstm_dtype out_state_dtype, hipStream_t s) {
+    for (int attempt = 0;; ++attempt) {
+        int rc = forward_enqueue(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, s);
+        if (rc) return rc;
+        rc = wait_stream(s);
+        if (rc) return rc;
+        const bool persistent = p->Lf.persistent != 0;
+        rc = forward_conclude(p, s);
+        if (rc != FLSTM_E_STALLED || !persistent || attempt > 0) return rc;
+    }
 }
 
 }  // namespace
@@ -681,17 +718,17 @@ namespace {
 // Backward recurrence in parts, like the forward pass: setup, step ranges from the end of the sequence towards
 // its start (dY rows -> BPTT steps -> dX rows), and the weight-gradient GEMMs over the whole sequence.
 int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_dtype, const void* d_hn,
-                   const void* d_cn, flstm_dtype dstate_dtype, float S, void* dx, flstm_dtype dx_dtype, bool whole_dy,
-                   hipStream_t s) {
+                   const void* d_cn, flstm_dtype dstate_dtype, const BwdScales& k, void* dx, flstm_dtype dx_dtype,
+                   bool whole_dy, hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
-    p->bw.T = T; p->bw.dY = dY; p->bw.dy_dtype = dy_dtype; p->bw.S = S; p->bw.dx = dx; p->bw.dx_dtype = dx_dtype;
+    p->bw.T = T; p->bw.dY = dY; p->bw.dy_dtype = dy_dtype; p->bw.k = k; p->bw.dx = dx; p->bw.dx_dtype = dx_dtype;
     p->bw.open = true;
     p->beside_b.count = 0;
     // (step-wise launches always read a plan-owned copy, so that their captured graph can be replayed)
     if (dy_dtype == FLSTM_F16 && d.H == d.Hp && p->Lb.persistent) {
         p->bw.dYk = static_cast<const half_t*>(dY);
-        p->bw.dy_scale = S;
+        p->bw.dy_scale = k.dy;
     } else {
         FL_TRY(p->dYp.reserve(TB * d.Hp * sizeof(half_t)));
         p->bw.dYk = p->dYp.as<half_t>();
@@ -714,16 +751,16 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     if (p->Lb.two_d) {
         const size_t pslot = rec_bwd_part_slot_floats(p->Lb) * sizeof(float);
         FL_TRY(p->part_b.reserve(kRecBwdPartSlots * pslot));
-        for (int k = 0; k < kRecBwdPartSlots; ++k)
-            prep.fill(static_cast<char*>(p->part_b.p) + size_t(k) * pslot, pslot, rec_bwd_part_fill(k, int(T)));
+        for (int i = 0; i < kRecBwdPartSlots; ++i)
+            prep.fill(static_cast<char*>(p->part_b.p) + size_t(i) * pslot, pslot, rec_bwd_part_fill(i, int(T)));
     }
-    prep.to_float(d_hn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, S, p->dHn.as<float>(), size_t(d.Hp));
-    prep.to_float(d_cn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, S, p->dC.as<float>(), size_t(d.Hp));
+    prep.to_float(d_hn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, k.state, p->dHn.as<float>(), size_t(d.Hp));
+    prep.to_float(d_cn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, k.state, p->dC.as<float>(), size_t(d.Hp));
     prep.fill(p->db_part.p, size_t(p->Lb.ng) * 4 * d.Hp * sizeof(float), 0u);
     prep.fill(p->status.as<char>() + kSeatsOffset, kStatusBytes - kSeatsOffset, 0u);
     if (p->opt_profile) prep.fill(p->prof.as<long long>() + 8, 8 * sizeof(long long), 0u);
     if (whole_dy && p->bw.dYk != dY)
-        prep.to_half(dY, dy_dtype == FLSTM_F32, TB, d.H, size_t(d.H), S, p->dYp.as<half_t>(), TB, size_t(d.Hp));
+        prep.to_half(dY, dy_dtype == FLSTM_F32, TB, d.H, size_t(d.H), k.dy, p->dYp.as<half_t>(), TB, size_t(d.Hp));
     prep.stamps = stamps_of(p);
     prep.stamp = kStampBwdStart;
     FL_TRY(run_ops(prep, s));
@@ -742,7 +779,7 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
         const char* src = static_cast<const char*>(p->bw.dY) + size_t(lo) * d.B * d.H * esz;
         half_t* dst = p->dYp.as<half_t>() + size_t(lo) * d.B * d.Hp;
         OpList conv;
-        conv.to_half(src, p->bw.dy_dtype == FLSTM_F32, rows, d.H, size_t(d.H), p->bw.S, dst, rows, size_t(d.Hp));
+        conv.to_half(src, p->bw.dy_dtype == FLSTM_F32, rows, d.H, size_t(d.H), p->bw.k.dy, dst, rows, size_t(d.Hp));
         FL_TRY(run_ops(conv, s));
     }
     RecBwdArgs a;
@@ -800,25 +837,26 @@ int backward_dx(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
     g.M = int(rows); g.N = d.I; g.K = 4 * d.Hp;
     if (p->bw.dx_dtype == FLSTM_F32) g.C32 = static_cast<float*>(p->bw.dx) + row0 * d.I;
     else g.C16 = static_cast<half_t*>(p->bw.dx) + row0 * d.I;
-    g.ldc = size_t(d.I); g.alpha = 1.f / p->bw.S; g.splits = 1; g.split_stride = 0;
+    g.ldc = size_t(d.I); g.alpha = p->bw.k.dx; g.splits = 1; g.split_stride = 0;
     FL_TRY(launch_gemm_nt(g, s));
     return 0;
 }
 
 int backward_rec_once(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_dtype, const void* d_hn,
-                      const void* d_cn, flstm_dtype dstate_dtype, float S, void* dx, flstm_dtype dx_dtype,
+                      const void* d_cn, flstm_dtype dstate_dtype, const BwdScales& k, void* dx, flstm_dtype dx_dtype,
                       hipStream_t s) {
-    int rc = backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, S, dx, dx_dtype, true, s);
+    int rc = backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, true, s);
     if (rc) return rc;
     return backward_recur(p, long(T) - 1, -1, true, s);
 }
 
-// dW_ih = dG^T * X and dW_hh = dG^T * H_prev over the whole sequence, bias gradient and state gradients
+// dW_ih = dG^T * X and dW_hh = dG^T * H_prev over the whole sequence, bias gradient and state gradients (enqueued; the
+// last launch of a pass)
 int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, float* dW_ih, float* dW_hh,
                     float* db_ih, float* db_hh, float* dh0, float* dc0, hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = p->bw.T * size_t(d.B);
-    const float invS = 1.f / p->bw.S;
+    const float invS = p->bw.k.grads;
     // k-major operands exactly as the recurrence left them (H_prev of step t is row block t of the state array,
     // row block 0 = h0), split over K, fp32 partials.  Both gradients come out of ONE launch, dG^T * [X | H_prev]:
     // dG (the large operand) is read once, and the tiles of both products fill the machine together.
@@ -858,11 +896,56 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, floa
     out.reduce_db(d, p->db_part.as<float>(), p->Lb.ng, invS, accumulate, db_ih, db_hh);
     out.unpad(p->dH0.as<float>(), 1, size_t(d.Hp), size_t(d.B), d.H, invS, dh0, 1);
     out.unpad(p->dC.as<float>(), 1, size_t(d.Hp), size_t(d.B), d.H, invS, dc0, 1);
-    int rc = publish_with(p, out, kStampBwdEnd, s);
+    return publish_with(p, out, kStampBwdEnd, s);
+}
+
+// One whole backward pass, enqueued.  dX and the weight gradients follow the recurrence without waiting for its status
+// (one wait per pass); a persistent launch that gave up is found at the end and the pass repeated step-wise over the
+// same outputs.  Only when the caller's gradients are added to (accumulate_grads) the status is checked first
+// (FLSTM_E_STALLED).
+int backward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* dY, flstm_dtype dy_dtype,
+                     const void* d_hn, const void* d_cn, flstm_dtype dstate_dtype, const BwdScales& k, void* dx,
+                     flstm_dtype dx_dtype, float* dW_ih, float* dW_hh, float* db_ih, float* db_hh, float* dh0, float* dc0,
+                     hipStream_t s) {
+    use_tuned(p, T);
+    int rc = backward_rec_once(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, s);
+    if (rc == int(hipErrorCooperativeLaunchTooLarge) && p->Lb.persistent && !p->refused_bwd) {
+        // the grid cannot be co-resident: nothing was launched; this direction runs step-wise from now on
+        p->refused_bwd = true;
+        p->coop_refusals++;
+        replan(p);
+        rc = backward_rec_once(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, s);
+    }
     if (rc) return rc;
-    rc = wait_stream(s);
+    if (p->opt_accumulate) {
+        int st = 0;
+        OpList nothing;
+        rc = wait_status(p, nothing, -1, s, &st);
+        if (rc) return rc;
+        if (st != 0) return FLSTM_E_STALLED;
+    }
+    rc = backward_dx(p, long(T) - 1, 0, s);
     if (rc) return rc;
+    return backward_finish(p, x, x_dtype, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
+}
+// ... once the stream has been waited for (as forward_conclude)
+int backward_conclude(flstm_core_plan* p, bool weight_gradients, hipStream_t s) {
     p->bw.open = false;
+    int st = 0;
+    int rc = take_status(p, s, &st);
+    if (rc) return rc;
+    if (st != 0) {
+        if (p->Lb.persistent) demote(p, false);
+        return FLSTM_E_STALLED;
+    }
+    pass_done(p, false);
+    if (p->opt_profile)
+        FL_TRY(hipMemcpy(p->prof_b, p->prof.as<long long>() + 8, sizeof(p->prof_b), hipMemcpyDeviceToHost));
+    const int dw_start = weight_gradients ? kStampBwdDw : kStampBwdEnd;   // (without that product the dX one ends with the pass)
+    p->ms_bwd[0] = elapsed(p, kStampBwdStart, kStampBwdRecEnd);
+    p->ms_bwd[1] = elapsed(p, kStampBwdRecEnd, dw_start);
+    p->ms_bwd[2] = elapsed(p, dw_start, kStampBwdEnd);
+    p->ms_bwd[3] = elapsed(p, kStampBwdStart, kStampBwdEnd);
     return 0;
 }
 
@@ -880,47 +963,127 @@ extern "C" int flstm_core_backward(flstm_core_plan* p, size_t T, const void* x, 
     if (dW_ih && !x) return FLSTM_E_INVALID;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const float S = grad_scale > 0.f ? grad_scale : 1.f;
-    use_tuned(p, T);
-
-    // dX and the weight gradients follow the recurrence without waiting for its status (one wait per pass); a
-    // persistent launch that gave up is found at the end and the pass repeated step-wise over the same outputs.
-    // Only when the caller's gradients are added to (accumulate_grads) the status is checked first.
+    const BwdScales k = BwdScales::loss_scale(S);
     for (int attempt = 0;; ++attempt) {
-        int rc = backward_rec_once(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, S, dx, dx_dtype, s);
-        if (rc == int(hipErrorCooperativeLaunchTooLarge) && p->Lb.persistent && !p->refused_bwd) {
-            // the grid cannot be co-resident: nothing was launched; this direction runs step-wise from now on
-            p->refused_bwd = true;
-            p->coop_refusals++;
-            replan(p);
-            continue;
-        }
-        if (rc) return rc;
-        int st = 0;
-        if (p->opt_accumulate) {
-            OpList nothing;
-            rc = wait_status(p, nothing, -1, s, &st);
-            if (rc) return rc;
-        }
-        if (st == 0) {
-            rc = backward_dx(p, long(T) - 1, 0, s);
-            if (rc) return rc;
-            rc = backward_finish(p, x, x_dtype, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
-            if (rc) return rc;
-            rc = take_status(p, s, &st);
-            if (rc) return rc;
-            if (st == 0) break;
-        }
-        if (!p->Lb.persistent || attempt > 0) return FLSTM_E_STALLED;
-        demote(p, false);
+        int rc = backward_enqueue(p, T, x, x_dtype, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, dW_ih, dW_hh, db_ih,
+                                  db_hh, dh0, dc0, s);
+        if (rc == 0) rc = wait_stream(s);
+        const bool persistent = p->Lb.persistent != 0;
+        if (rc == 0) rc = backward_conclude(p, dW_ih || dW_hh, s);
+        else if (rc == FLSTM_E_STALLED && persistent) demote(p, false);   // (the check ahead of accumulation)
+        p->bw.open = false;
+        if (rc != FLSTM_E_STALLED || !persistent || attempt > 0) return rc;
     }
-    pass_done(p, false);
-    if (p->opt_profile)
-        FL_TRY(hipMemcpy(p->prof_b, p->prof.as<long long>() + 8, sizeof(p->prof_b), hipMemcpyDeviceToHost));
-    const int dw_start = (dW_ih || dW_hh) ? kStampBwdDw : kStampBwdEnd;   // (without that product the dX one ends with the pass)
-    p->ms_bwd[0] = elapsed(p, kStampBwdStart, kStampBwdRecEnd);
-    p->ms_bwd[1] = elapsed(p, kStampBwdRecEnd, dw_start);
-    p->ms_bwd[2] = elapsed(p, dw_start, kStampBwdEnd);
-    p->ms_bwd[3] = elapsed(p, kStampBwdStart, kStampBwdEnd);
+}
+
+// ---- stacks of layers: the same passes, layer behind layer on one stream with ONE wait at the end
+
+extern "C" int flstm_core_pack(flstm_core_plan* p, const float* w_ih, const float* w_hh, const float* b_ih, const float* b_hh,
+                               void* stream) {
+    int rc = core_pack_weights_async(p, w_ih, w_hh, static_cast<hipStream_t>(stream));
+    if (rc) return rc;
+    return flstm_core_pack_bias(p, b_ih, b_hh, stream);
+}
+
+extern "C" int flstm_stack_forward(flstm_core_plan* const* plans, int layers, size_t T, const void* x, flstm_dtype x_dtype,
+                                   const void* h0, const void* c0, flstm_dtype state_dtype, void* const* ys, flstm_dtype y_dtype,
+                                   void* hy, void* cy, void* stream) {
+    if (!plans || layers < 1 || !ys) return FLSTM_E_INVALID;
+    if (T == 0) return 0;
+    if (!x || T > (size_t(1) << 24)) return FLSTM_E_INVALID;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    for (int l = 0; l < layers; ++l) {
+        const flstm_core_plan* p = plans[l];
+        if (!p || !ys[l] || p->d.B != plans[0]->d.B || p->d.H != plans[0]->d.H || (l > 0 && p->d.I != p->d.H)) return FLSTM_E_INVALID;
+        if (!p->weights_packed || !p->bias_packed) return FLSTM_E_NOT_PACKED;
+    }
+    const size_t state_in = size_t(plans[0]->d.B) * plans[0]->d.H * (state_dtype == FLSTM_F32 ? 4 : 2);
+    const size_t state_out = size_t(plans[0]->d.B) * plans[0]->d.H * (y_dtype == FLSTM_F32 ? 4 : 2);
+    auto at = [](const void* base, size_t off) -> const void* { return base ? static_cast<const char*>(base) + off : nullptr; };
+    auto layer = [&](int l, auto&& pass) -> int {
+        return pass(plans[l], T, l == 0 ? x : ys[l - 1], l == 0 ? x_dtype : y_dtype, at(h0, l * state_in), at(c0, l * state_in),
+                    state_dtype, ys[l], y_dtype, const_cast<void*>(at(hy, l * state_out)), const_cast<void*>(at(cy, l * state_out)), y_dtype, s);
+    };
+    int rc = 0;
+    for (int l = 0; l < layers && rc == 0; ++l) {
+        plans[l]->have_cache = false;
+        rc = layer(l, forward_enqueue);
+    }
+    const int waited = wait_stream(s);
+    if (rc == 0) rc = waited;
+    for (int l = 0; l < layers && rc == 0; ++l) {
+        const bool persistent = plans[l]->Lf.persistent != 0;
+        rc = forward_conclude(plans[l], s);
+        if (rc == FLSTM_E_STALLED && persistent) {   // this layer again, and with it everything that has read its outputs
+            rc = 0;
+            for (int m = l + 1; m < layers && rc == 0; ++m) rc = clear_status(plans[m], s);
+            for (int m = l; m < layers && rc == 0; ++m) {
+                rc = layer(m, forward_pass);
+                if (rc == 0) { plans[m]->have_cache = true; plans[m]->T_cache = T; }
+            }
+            break;
+        }
+        if (rc == 0) { plans[l]->have_cache = true; plans[l]->T_cache = T; }
+    }
+    for (int l = 0; l < layers; ++l) plans[l]->fw.open = false;
+    return rc;
+}
+
+extern "C" int flstm_stack_backward(flstm_core_plan* const* plans, int layers, size_t T, const void* const* xs, flstm_dtype x_dtype,
+                                    const void* dY, flstm_dtype dy_dtype, float dy_scale, const void* const* d_hn,
+                                    const void* const* d_cn, flstm_dtype dstate_dtype, float loss_scale, void* const* dxs,
+                                    flstm_dtype dx_dtype, float* const* dW_ih, float* const* dW_hh, float* const* db_ih,
+                                    float* const* db_hh, float* const* dh0, float* const* dc0, void* stream) {
+    if (!plans || layers < 1 || !xs || !dY || !dxs || !dW_ih || !dW_hh || !db_ih || !dh0 || !dc0) return FLSTM_E_INVALID;
+    if (T == 0) return 0;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    for (int l = 0; l < layers; ++l) {
+        if (!plans[l] || !xs[l] || (l > 0 && !dxs[l])) return FLSTM_E_INVALID;
+        if (!plans[l]->have_cache || plans[l]->T_cache != T) return FLSTM_E_NO_CACHE;
+        if (plans[l]->opt_accumulate) return FLSTM_E_INVALID;
+    }
+    // from layer to layer gradients stay fp16 with the loss scale on them; it is divided out of everything returned
+    const float S = loss_scale > 0.f ? loss_scale : 1.f;
+    auto layer = [&](int l) -> int {
+        const bool top = l == layers - 1;
+        const BwdScales k{top ? dy_scale : 1.f, S, l == 0 ? 1.f / S : 1.f, 1.f / S};
+        return backward_enqueue(plans[l], T, xs[l], l == 0 ? x_dtype : FLSTM_F16, top ? dY : dxs[l + 1], top ? dy_dtype : FLSTM_F16,
+                                d_hn ? d_hn[l] : nullptr, d_cn ? d_cn[l] : nullptr, dstate_dtype, k, dxs[l], l == 0 ? dx_dtype : FLSTM_F16,
+                                dW_ih[l], dW_hh[l], db_ih[l], db_hh ? db_hh[l] : nullptr, dh0[l], dc0[l], s);
+    };
+    int rc = 0, from = layers - 1;
+    for (int attempt = 0;; ++attempt) {   // a layer that gave up is repeated step-wise, and every layer below it with it
+        for (int l = from; l >= 0 && rc == 0; --l) rc = layer(l);
+        const int waited = wait_stream(s);
+        if (rc == 0) rc = waited;
+        bool again = false;
+        for (int l = from; l >= 0 && rc == 0; --l) {
+            const bool persistent = plans[l]->Lb.persistent != 0;
+            rc = backward_conclude(plans[l], true, s);
+            if (rc == FLSTM_E_STALLED && persistent && attempt < layers) {
+                from = l;
+                again = true;
+                for (int m = l - 1; m >= 0; --m) {
+                    const int cleared = clear_status(plans[m], s);
+                    if (cleared) return cleared;
+                }
+            }
+        }
+        for (int l = 0; l < layers; ++l) plans[l]->bw.open = false;
+        if (!again) return rc;
+        rc = 0;
+    }
+}
+
+// The largest |value| of a device tensor (NaN if there is one), on the host: what an automatic loss scale is chosen from.
+extern "C" int flstm_core_absmax(flstm_core_plan* p, const void* t, flstm_dtype dtype, size_t n, float* out, void* stream) {
+    if (!p || !out || (n > 0 && !t)) return FLSTM_E_INVALID;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    *out = 0.f;
+    if (n == 0) return 0;
+    FL_TRY(absmax(t, dtype == FLSTM_F32, n, p->status.as<unsigned>() + kStatusBytes / 4, &p->status_host->absmax, s));
+    FL_TRY(hipStreamSynchronize(s));
+    *out = *static_cast<volatile float*>(&p->status_host->absmax);
     return 0;
 }
 
@@ -975,7 +1138,7 @@ extern "C" int flstm_core_backward_begin(flstm_core_plan* p, size_t T, const voi
     for (float& m : p->ms_bwd) m = -1.f;
     const float S = grad_scale > 0.f ? grad_scale : 1.f;
     use_tuned(p, T);
-    return backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, S, dx, dx_dtype, false, static_cast<hipStream_t>(stream));
+    return backward_setup(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, BwdScales::loss_scale(S), dx, dx_dtype, false, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int flstm_core_backward_steps(flstm_core_plan* p, size_t t_hi, size_t nsteps, void* stream) {
@@ -1015,6 +1178,9 @@ extern "C" int flstm_core_backward_end(flstm_core_plan* p, const void* x, flstm_
     }
     rc = backward_finish(p, x, x_dtype, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
     if (rc) return rc;
+    rc = wait_stream(s);
+    if (rc) return rc;
+    p->bw.open = false;
     pass_done(p, false);
     return 0;
 }

@@ -15,11 +15,15 @@ struct Dims {
 
 // Replaces src/kernels.cu:57-84 (pack_weights_kernel) and :45-55 (combine_bias_kernel): fp32
 // PyTorch-layout weights -> the fp16 operand layouts of the kernels in this library.
+struct FragLayout {   // where a recurrence kernel expects its weight fragments: RecLayout's description of them
+    half8* out = nullptr;
+    int ks = 0, nt = 0, rot_div = 0, nw = 0, unit_major = 0, wide = 0, kq = 0;
+};
+// W_ih twice (as it is for the projection, transposed for dX) and W_hh as forward fragments, backward fragments and (two_d.out
+// set) those of the backward recurrence that splits its product two ways; one launch.
 hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p /*[4Hp][Ip]*/,
-                        half_t* wih_t /*[Ip][4Hp]*/, half8* wfrag_fwd, int ks_fwd, int nt_fwd, int rot_div_fwd, int nw_fwd, int unit_major_fwd, int wide_fwd,
-                        half8* wfrag_bwd, int ks_bwd, int nt_bwd, int rot_div_bwd, int nw_bwd, hipStream_t s);
-// W_hh in the layout of the backward recurrence that splits its product two ways; kq contraction slices.
-hipError_t pack_wfrag_bwd2d(const Dims& d, const float* w_hh, half8* out, int kq, hipStream_t s);
+                        half_t* wih_t /*[Ip][4Hp]*/, const FragLayout& fwd, const FragLayout& bwd, const FragLayout& two_d,
+                        hipStream_t s);
 hipError_t pack_bias(const Dims& d, const float* b_ih, const float* b_hh, float* bias_p, hipStream_t s);
 
 // dst[r][c] (pitch ldc) = sum over z < splits of partial[z * per + r * cols + c]: split-K partials of a plain GEMM.
@@ -32,6 +36,11 @@ hipError_t reduce_partials(const float* partial, int splits, size_t per, int row
 hipError_t checksum_add(const void* p, size_t bytes, u64 salt, u64* out, hipStream_t s);
 
 hipError_t fill_zero(void* p, size_t bytes, hipStream_t s);
+
+// The largest |value| of n elements (NaN if there is one), left in pinned host memory; `partial`: kAbsmaxBlocks words of
+// device memory.
+constexpr int kAbsmaxBlocks = 256;
+hipError_t absmax(const void* t, int f32, size_t n, unsigned* partial, float* host_out, hipStream_t s);
 
 // The layout operations around the GEMMs and the recurrence, up to kMaxOps of them in ONE launch.  A pass starts with
 // half a dozen of them (state rows, rings, counters, operand conversion) and ends with as many (outputs, final states,
@@ -60,7 +69,8 @@ struct LayoutOp {
 enum Stamp : int { kStampFwdStart, kStampFwdRec, kStampFwdRecEnd, kStampBwdStart, kStampBwdRecEnd, kStampBwdDw, kStampBwdEnd, kStampFwdEnd, kStampCount };
 struct HostStatus {
     int status;
-    int pad[15];
+    float absmax;   // (absmax())
+    int pad[14];
     long long stamps[kStampCount];
 };
 struct OpList {

@@ -20,100 +20,127 @@ __device__ __forceinline__ int torch_row(int q, int H) {
     return j < H ? gate * H + j : -1;
 }
 
-__global__ void pack_wih_kernel(Dims d, const float* __restrict__ w_ih, half_t* __restrict__ wih_p,
-                                half_t* __restrict__ wih_t) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    const size_t total = size_t(4) * d.Hp * d.Ip;
-    if (idx >= total) return;
-    const int q = int(idx / d.Ip), i = int(idx % d.Ip);
-    const int row = torch_row(q, d.H);
-    const float v = (row >= 0 && i < d.I) ? w_ih[size_t(row) * d.I + i] : 0.f;
-    wih_p[idx] = (half_t)v;
-    wih_t[size_t(i) * 4 * d.Hp + q] = (half_t)v;
-}
+// Everything that becomes of the weights, one launch; blocks [first[i], first[i + 1]) of the grid make operand i.  A thread
+// makes eight consecutive halfs (one 16-byte store).  One element per thread and one launch per operand took 28 us of
+// kernels and the gaps between them at 650 units, every pass of a training loop.
+struct PackJob {
+    Dims d;
+    const float *w_ih, *w_hh;
+    half_t *wih_p, *wih_t;
+    FragLayout frag[3];     // forward, backward, two-way backward
+    unsigned first[6];
+};
 
-// Forward fragments: B operand of  gates[b][c] += h[b][k] * W_hh[row(c)][k].  The product's columns are local to
-// a workgroup (they only meet the pointwise stage through LDS) and stay gate-major within the slice of JB = 4*NT
-// units: column c = gate * JB + unit.  In the kernels with one cell per thread (rec_fwd_il_kernel,
-// rec_fwd_wide_kernel) they are unit-major, column c = 4 * unit + gate: the four accumulation registers of a lane are then the four gates of one unit.
-// fragment (hs, wave, ks, n): lane l holds column c = n*16 + l%16 of slice hs,
-// k = (ks*nw + wave)*32 + 8*(l/16) + e, e = 0..7 (nw = wavefronts per workgroup, 4 or 8).
-__global__ void pack_wfrag_fwd_kernel(Dims d, const float* __restrict__ w_hh, half_t* __restrict__ out,
-                                      int ks_wave, int nt, int rot_div, int nw, int unit_major, int wide) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;  // one half element
-    const int nh = d.Hp / (4 * nt);
-    const size_t total = size_t(nh) * nw * ks_wave * nt * kWave * 8;
-    if (idx >= total) return;
-    size_t r = idx;
-    const int e = int(r % 8); r /= 8;
+__device__ __forceinline__ half8 frag_values_fwd(const Dims& d, const float* __restrict__ w_hh, const FragLayout& f, size_t item) {
+    // B operand of  gates[b][c] += h[b][k] * W_hh[row(c)][k].  The product's columns are local to a workgroup (they only
+    // meet the pointwise stage through LDS) and stay gate-major within the slice of JB = 4*NT units: column
+    // c = gate * JB + unit.  In the kernels with one cell per thread (rec_fwd_il_kernel, rec_fwd_wide_kernel) they are
+    // unit-major, column c = 4 * unit + gate: the four accumulation registers of a lane are then the four gates of one
+    // unit.  Fragment (hs, wave, ks, n): lane l holds column c = n*16 + l%16 of slice hs, k = (ks*nw + wave)*32 + 8*(l/16)
+    // + e, e = 0..7 (nw = wavefronts per workgroup, 4 or 8).
+    unsigned r = unsigned(item);
     const int lane = int(r % kWave); r /= kWave;
-    const int n = int(r % nt); r /= nt;
-    const int ks = int(r % ks_wave); r /= ks_wave;
-    const int wave = int(r % nw); r /= nw;
-    const int hs = int(r);
-    const int jb = 4 * nt, c = n * 16 + lane % 16;
-    const int gate = unit_major ? c % 4 : c / jb, unit = hs * jb + (unit_major ? c / 4 : c % jb);
+    const int n = int(r % f.nt); r /= f.nt;
+    const int ks = int(r % f.ks); r /= f.ks;
+    const int wave = int(r % f.nw);
+    const int hs = int(r / f.nw);
+    const int jb = 4 * f.nt, c = n * 16 + lane % 16, nh = d.Hp / jb;
+    const int gate = f.unit_major ? c % 4 : c / jb, unit = hs * jb + (f.unit_major ? c / 4 : c % jb);
     // (slot ks of slice hs holds a rotated k-step: recurrent.h, rec_kstep_rotation, rec_wide_rotation)
-    const int kstep = wide ? (ks ^ rec_wide_rotation(ks, hs / 8, ks_wave))
-                           : rec_kstep_of_slot(ks, rec_kstep_rotation(hs, nh, ks_wave, rot_div), ks_wave);
-    const int k = (kstep * nw + wave) * 32 + 8 * (lane / 16) + e;
-    out[idx] = (half_t)((unit < d.H && k < d.H) ? w_hh[size_t(gate * d.H + unit) * d.H + k] : 0.f);
-}
-
-// Backward fragments: B operand of  dh[b][k] += dG[b][q] * W_hh[row(q)][k].
-// fragment (hs, wave, ks, n): lane l holds output column k = hs*16*NT + n*16 + l%16,
-// contraction index q = (ks*nw + wave)*32 + 8*(l/16) + e.
-__global__ void pack_wfrag_bwd_kernel(Dims d, const float* __restrict__ w_hh, half_t* __restrict__ out,
-                                      int ks_wave, int nt, int rot_div, int nw) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    const int nh = d.Hp / (16 * nt);
-    const size_t total = size_t(nh) * nw * ks_wave * nt * kWave * 8;
-    if (idx >= total) return;
-    size_t r = idx;
-    const int e = int(r % 8); r /= 8;
-    const int lane = int(r % kWave); r /= kWave;
-    const int n = int(r % nt); r /= nt;
-    const int ks = int(r % ks_wave); r /= ks_wave;
-    const int wave = int(r % nw); r /= nw;
-    const int hs = int(r);
-    const int k = hs * 16 * nt + n * 16 + lane % 16;
-    const int kstep = rec_kstep_of_slot(ks, rec_kstep_rotation(hs, nh, ks_wave, rot_div), ks_wave);
-    const int q = (kstep * nw + wave) * 32 + 8 * (lane / 16) + e;
-    float v = 0.f;
-    if (q < 4 * d.Hp && k < d.H) {
-        const int row = torch_row(q, d.H);
-        if (row >= 0) v = w_hh[size_t(row) * d.H + k];
+    const int kstep = f.wide ? (ks ^ rec_wide_rotation(ks, hs / 8, f.ks)) : rec_kstep_of_slot(ks, rec_kstep_rotation(hs, nh, f.ks, f.rot_div), f.ks);
+    const int k = (kstep * f.nw + wave) * 32 + 8 * (lane / 16);
+    half8 v{};
+    if (unit < d.H) {
+        const float* row = w_hh + size_t(gate * d.H + unit) * d.H;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (k + e < d.H) v[e] = (half_t)row[k + e];
     }
-    out[idx] = (half_t)v;
+    return v;
 }
 
-// Two-dimensional backward layout: [Hp / 64 column slices s][kq contraction slices q][4 waves][ks k-steps][4 tiles][64 lanes][8],
-// ks = Hp / (32 kq): lane l of tile n holds column 64 s + 16 n + l % 16 of W_hh (hidden unit k of dh = dG * W_hh^T-packed)
-// and the eight packed gate rows (4 Hp / kq) q + 32 (4 ks + wave) + 8 (l / 16) .. +7.
-__global__ void pack_wfrag_bwd2d_kernel(Dims d, const float* __restrict__ w_hh, half_t* __restrict__ out, int kq) {
-    const size_t idx = size_t(blockIdx.x) * kT + threadIdx.x;
-    const bool wide = d.Hp > 2048;
-    const int ksn = wide ? rec_wide_ks(d.Hp) : d.Hp / (32 * kq);   // k-steps per wave: 4 waves * ksn * 32 = 4 Hp / kq packed gate rows (wide: or more, zeros)
-    const size_t total = size_t(d.Hp / 64) * kq * 4 * ksn * 4 * kWave * 8;
-    if (idx >= total) return;
-    size_t r = idx;
-    const int e = int(r % 8); r /= 8;
+// eight consecutive packed gate rows q .. q+7 (two units) of column k of W_hh
+__device__ __forceinline__ half8 gate_rows(const Dims& d, const float* __restrict__ w_hh, int q, int k) {
+    half8 v{};
+    if (k < d.H) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int row = torch_row(q + e, d.H);
+            if (row >= 0) v[e] = (half_t)w_hh[size_t(row) * d.H + k];
+        }
+    }
+    return v;
+}
+
+__device__ __forceinline__ half8 frag_values_bwd(const Dims& d, const float* __restrict__ w_hh, const FragLayout& f, size_t item) {
+    // B operand of  dh[b][k] += dG[b][q] * W_hh[row(q)][k].  Fragment (hs, wave, ks, n): lane l holds output column
+    // k = hs*16*NT + n*16 + l%16, contraction index q = (ks*nw + wave)*32 + 8*(l/16) + e.
+    unsigned r = unsigned(item);
+    const int lane = int(r % kWave); r /= kWave;
+    const int n = int(r % f.nt); r /= f.nt;
+    const int ks = int(r % f.ks); r /= f.ks;
+    const int wave = int(r % f.nw);
+    const int hs = int(r / f.nw), nh = d.Hp / (16 * f.nt);
+    const int k = hs * 16 * f.nt + n * 16 + lane % 16;
+    const int kstep = rec_kstep_of_slot(ks, rec_kstep_rotation(hs, nh, f.ks, f.rot_div), f.ks);
+    const int q = (kstep * f.nw + wave) * 32 + 8 * (lane / 16);
+    return q < 4 * d.Hp ? gate_rows(d, w_hh, q, k) : half8{};
+}
+
+__device__ __forceinline__ half8 frag_values_two_d(const Dims& d, const float* __restrict__ w_hh, const FragLayout& f, size_t item) {
+    // [Hp / 64 column slices s][kq contraction slices q][4 waves][ks k-steps][4 tiles][64 lanes][8]: lane l of tile n holds
+    // column 64 s + 16 n + l % 16 of W_hh (hidden unit k of dh = dG * W_hh^T-packed) and the eight packed gate rows
+    // (4 Hp / kq) q + 32 (4 ks + wave) + 8 (l / 16) .. +7.
+    unsigned r = unsigned(item);
     const int lane = int(r % kWave); r /= kWave;
     const int n = int(r % 4); r /= 4;
-    const int ks = int(r % ksn); r /= ksn;
+    const int ks = int(r % f.ks); r /= f.ks;
     const int wave = int(r % 4); r /= 4;
-    const int qs = int(r % kq); r /= kq;
-    const int sl = int(r);
+    const int qs = int(r % f.kq);
+    const int sl = int(r / f.kq);
     const int k = sl * 64 + n * 16 + lane % 16;
     // (slot ks of a wave holds the k-step the kernel fetches there: rotated per column slice)
-    const int kstep = wide ? (ks ^ rec_wide_rotation(ks, sl / 8, ksn)) : rec_kstep_of_slot(ks, rec_bwd2d_rotation(sl, ksn, kq), ksn);
-    const int in_slice = (kstep * 4 + wave) * 32 + 8 * (lane / 16) + e, q = qs * (4 * d.Hp / kq) + in_slice;
-    float v = 0.f;
-    if (in_slice < 4 * d.Hp / kq && k < d.H) {
-        const int row = torch_row(q, d.H);
-        if (row >= 0) v = w_hh[size_t(row) * d.H + k];
+    const int kstep = f.wide ? (ks ^ rec_wide_rotation(ks, sl / 8, f.ks)) : rec_kstep_of_slot(ks, rec_bwd2d_rotation(sl, f.ks, f.kq), f.ks);
+    const int in_slice = (kstep * 4 + wave) * 32 + 8 * (lane / 16), q = qs * (4 * d.Hp / f.kq) + in_slice;
+    return in_slice < 4 * d.Hp / f.kq ? gate_rows(d, w_hh, q, k) : half8{};
+}
+
+__global__ __launch_bounds__(kT) void pack_kernel(PackJob job) {
+    const Dims& d = job.d;
+    int which = 0;
+    while (blockIdx.x >= job.first[which + 1]) ++which;
+    const size_t item = size_t(blockIdx.x - job.first[which]) * kT + threadIdx.x;
+    if (which == 0) {          // wih_p: eight columns of a packed row
+        const unsigned per_row = unsigned(d.Ip) / 8;
+        if (item >= size_t(4) * d.Hp * per_row) return;
+        const int q = int(unsigned(item) / per_row), i = int(unsigned(item) % per_row) * 8, row = torch_row(q, d.H);
+        half8 v{};
+        if (row >= 0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (i + e < d.I) v[e] = (half_t)job.w_ih[size_t(row) * d.I + i + e];
+        }
+        st_half8(job.wih_p + size_t(q) * d.Ip + i, v);
+    } else if (which == 1) {   // wih_t: eight packed gate columns of a row; 16 rows by 4 chunks per wave, so that reads and writes come in 64-byte pieces
+        const unsigned chunks = unsigned(4 * d.Hp) / 8, lane = unsigned(item) % 64, tile = unsigned(item) / 64, across = chunks / 4;
+        const int i = int(tile / across * 16 + lane % 16), q = int((tile % across) * 4 + lane / 16) * 8;
+        if (i >= d.Ip) return;
+        half8 v{};
+        if (i < d.I) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int row = torch_row(q + e, d.H);
+                if (row >= 0) v[e] = (half_t)job.w_ih[size_t(row) * d.I + i];
+            }
+        }
+        st_half8(job.wih_t + size_t(i) * 4 * d.Hp + q, v);
+    } else {
+        const FragLayout& f = job.frag[which - 2];
+        const size_t n = which == 2 ? size_t(d.Hp / (4 * f.nt)) * f.nw * f.ks * f.nt * kWave
+                       : which == 3 ? size_t(d.Hp / (16 * f.nt)) * f.nw * f.ks * f.nt * kWave : size_t(d.Hp / 64) * f.kq * 4 * f.ks * 4 * kWave;
+        if (item >= n) return;
+        f.out[item] = which == 2 ? frag_values_fwd(d, job.w_hh, f, item) : which == 3 ? frag_values_bwd(d, job.w_hh, f, item) : frag_values_two_d(d, job.w_hh, f, item);
     }
-    out[idx] = (half_t)v;
 }
 
 __global__ void pack_bias_kernel(Dims d, const float* __restrict__ b_ih, const float* __restrict__ b_hh,
@@ -256,26 +283,22 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
 
 }  // namespace
 
-hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p, half_t* wih_t,
-                        half8* wfrag_fwd, int ks_fwd, int nt_fwd, int rot_div_fwd, int nw_fwd, int unit_major_fwd, int wide_fwd, half8* wfrag_bwd, int ks_bwd,
-                        int nt_bwd, int rot_div_bwd, int nw_bwd, hipStream_t s) {
-    const size_t n1 = size_t(4) * d.Hp * d.Ip;
-    hipLaunchKernelGGL(pack_wih_kernel, dim3(grid_for(n1)), dim3(kT), 0, s, d, w_ih, wih_p, wih_t);
-    const size_t n2 = size_t(d.Hp / (4 * nt_fwd)) * nw_fwd * ks_fwd * nt_fwd * kWave * 8;
-    hipLaunchKernelGGL(pack_wfrag_fwd_kernel, dim3(grid_for(n2)), dim3(kT), 0, s, d, w_hh,
-                       reinterpret_cast<half_t*>(wfrag_fwd), ks_fwd, nt_fwd, rot_div_fwd, nw_fwd,
-                       unit_major_fwd, wide_fwd);
-    const size_t n3 = size_t(d.Hp / (16 * nt_bwd)) * nw_bwd * ks_bwd * nt_bwd * kWave * 8;
-    hipLaunchKernelGGL(pack_wfrag_bwd_kernel, dim3(grid_for(n3)), dim3(kT), 0, s, d, w_hh,
-                       reinterpret_cast<half_t*>(wfrag_bwd), ks_bwd, nt_bwd, rot_div_bwd, nw_bwd);
-    return hipGetLastError();
-}
-
-hipError_t pack_wfrag_bwd2d(const Dims& d, const float* w_hh, half8* out, int kq, hipStream_t s) {
-    // Hp / 64 slices of 64 columns, kq slices of 4 Hp / kq packed gate rows, 8 or 16 k-steps per wave
-    if (!((d.Hp == 2048 && (kq == 4 || kq == 8)) || (d.Hp == 1024 && kq == 2) || (d.Hp > 2048 && d.Hp % 64 == 0 && kq == 4))) return hipErrorInvalidValue;
-    const size_t n = rec_bwd_two_d_wfrag_bytes(d.Hp) / sizeof(half_t);
-    hipLaunchKernelGGL(pack_wfrag_bwd2d_kernel, dim3(grid_for(n)), dim3(kT), 0, s, d, w_hh, reinterpret_cast<half_t*>(out), kq);
+hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p, half_t* wih_t, const FragLayout& fwd,
+                        const FragLayout& bwd, const FragLayout& two_d, hipStream_t s) {
+    PackJob job{};
+    job.d = d;
+    job.w_ih = w_ih; job.w_hh = w_hh; job.wih_p = wih_p; job.wih_t = wih_t;
+    job.frag[0] = fwd; job.frag[1] = bwd; job.frag[2] = two_d;
+    // (Hp is a multiple of 32 and Ip of 64: whole chunks of eight, and of four chunks, everywhere)
+    const size_t items[5] = {size_t(4) * d.Hp * d.Ip / 8, size_t(4) * d.Hp * d.Ip / 8,
+                             size_t(d.Hp / (4 * fwd.nt)) * fwd.nw * fwd.ks * fwd.nt * kWave,
+                             size_t(d.Hp / (16 * bwd.nt)) * bwd.nw * bwd.ks * bwd.nt * kWave,
+                             two_d.out ? size_t(d.Hp / 64) * two_d.kq * 4 * two_d.ks * 4 * kWave : 0};
+    for (int i = 0; i < 5; ++i) {
+        if (items[i] >> 32) return hipErrorInvalidValue;
+        job.first[i + 1] = job.first[i] + unsigned(ceil_div(items[i], kT));
+    }
+    hipLaunchKernelGGL(pack_kernel, dim3(job.first[5]), dim3(kT), 0, s, job);
     return hipGetLastError();
 }
 
@@ -438,6 +461,50 @@ hipError_t checksum_add(const void* p, size_t bytes, u64 salt, u64* out, hipStre
     int blocks = grid_for(ceil_div(n, 8));
     if (blocks > 512) blocks = 512;
     hipLaunchKernelGGL(checksum_kernel, dim3(blocks), dim3(kT), 0, s, static_cast<const unsigned short*>(p), n, salt, out);
+    return hipGetLastError();
+}
+
+// |value| as an unsigned word orders like the value, NaN above infinity.
+__global__ __launch_bounds__(kT) void absmax_kernel(const void* t, int f32, size_t n, unsigned* partial) {
+    __shared__ unsigned wave_max[kT / 64];
+    unsigned m = 0;
+    const size_t stride = size_t(gridDim.x) * kT, first = size_t(blockIdx.x) * kT + threadIdx.x;
+    const int V = f32 ? 4 : 8;
+    const size_t nv = reinterpret_cast<uintptr_t>(t) % 16 == 0 ? n / V : 0;
+    for (size_t i = first; i < nv; i += stride) {
+        const uint4 q = static_cast<const uint4*>(t)[i];
+        const unsigned w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (f32) m = max(m, w[e] & 0x7fffffffu);
+            else m = max(m, max(w[e] & 0x7fffu, (w[e] >> 16) & 0x7fffu));
+        }
+    }
+    for (size_t i = nv * V + first; i < n; i += stride)
+        m = max(m, f32 ? static_cast<const unsigned*>(t)[i] & 0x7fffffffu : unsigned(static_cast<const unsigned short*>(t)[i]) & 0x7fffu);
+    for (int off = 32; off > 0; off >>= 1) m = max(m, unsigned(__shfl_down(int(m), off, 64)));
+    if (threadIdx.x % 64 == 0) wave_max[threadIdx.x / 64] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kT / 64; ++w) m = max(m, wave_max[w]);
+        partial[blockIdx.x] = m;
+    }
+}
+__global__ __launch_bounds__(64) void absmax_finish_kernel(const unsigned* partial, int blocks, int f32, float* host_out) {
+    unsigned m = 0;
+    for (int i = threadIdx.x; i < blocks; i += 64) m = max(m, partial[i]);
+    for (int off = 32; off > 0; off >>= 1) m = max(m, unsigned(__shfl_down(int(m), off, 64)));
+    if (threadIdx.x == 0) {
+        const float v = f32 ? __builtin_bit_cast(float, m) : (float)__builtin_bit_cast(half_t, (unsigned short)m);
+        __hip_atomic_store(host_out, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+hipError_t absmax(const void* t, int f32, size_t n, unsigned* partial, float* host_out, hipStream_t s) {
+    int blocks = grid_for(ceil_div(n, 8));
+    if (blocks > kAbsmaxBlocks) blocks = kAbsmaxBlocks;
+    if (blocks < 1) blocks = 1;
+    hipLaunchKernelGGL(absmax_kernel, dim3(blocks), dim3(kT), 0, s, t, f32, n, partial);
+    hipLaunchKernelGGL(absmax_finish_kernel, dim3(1), dim3(64), 0, s, partial, blocks, f32, host_out);
     return hipGetLastError();
 }
 

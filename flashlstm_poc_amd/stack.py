@@ -2,11 +2,36 @@
 pass layer l+1's input gradient is layer l's upstream gradient.  The reference is single-layer only
 (flashlstm_v2/python/flashlstm/streaming_lstm.py:380-430); this is the thin layer loop a multi-layer workload
 needs, with everything resident on the GPU in fp16 between layers."""
+import ctypes
+import math
 from typing import List, Optional, Sequence, Tuple
 
 import torch
 
-from .core import LstmCore
+from .core import F16, F32, LstmCore, _dtype_code, _ptr
+
+
+def _pointers(tensors):
+    """A C array of the device addresses of `tensors` (None: a null pointer)."""
+    return (ctypes.c_void_p * len(tensors))(*[_ptr(t) for t in tensors])
+
+
+def _layer_states(states, shape, name):
+    """Per-layer states -- a (L,B,H) tensor, a sequence of (B,H) tensors or None -- as one contiguous (L,B,H) tensor.  Layers
+    of a sequence may be None (zeros)."""
+    if states is None:
+        return None
+    if not torch.is_tensor(states):
+        states = list(states)
+        if len(states) != shape[0]:
+            raise ValueError(f"{name} must have one entry per layer")
+        like = next((t for t in states if t is not None), None)
+        if like is None:
+            return None
+        states = torch.stack([torch.zeros_like(like) if t is None else t for t in states])
+    if not states.is_cuda or tuple(states.shape) != shape:
+        raise ValueError(f"{name} must hold CUDA tensors of shape {shape[1:]}, one per layer")
+    return states.contiguous()
 
 
 class LstmStack:
@@ -17,6 +42,8 @@ class LstmStack:
             raise ValueError("num_layers must be >= 1")
         self.B, self.I, self.H, self.L = int(batch), int(input_size), int(hidden_size), int(num_layers)
         self.layers: List[LstmCore] = [LstmCore(self.B, self.I if l == 0 else self.H, self.H) for l in range(self.L)]
+        self._lib = self.layers[0].lib
+        self._plans = (ctypes.c_void_p * self.L)(*[layer._h for layer in self.layers])
         self._inputs: List = []
         self.last_loss_scale = 1.0
 
@@ -34,18 +61,31 @@ class LstmStack:
 
     def forward(self, x, h0: Optional[Sequence] = None, c0: Optional[Sequence] = None):
         """x (T,B,I) fp16 on the GPU -> (y of the top layer (T,B,H) fp16, [hy per layer], [cy per layer])."""
-        import torch
+        y, hy, cy = self._forward(x, h0, c0)
+        return y, list(hy.unbind(0)), list(cy.unbind(0))
+
+    def _forward(self, x, h0, c0):
+        """forward() with the final states as (L,B,H) tensors: one library call for the whole stack, one wait."""
         if x.dtype != torch.float16:
             raise ValueError("x must be fp16 (activations travel between layers in fp16)")
-        self._inputs = []
-        hys, cys = [], []
-        cur = x
-        for l, layer in enumerate(self.layers):
-            self._inputs.append(cur)
-            cur, hy, cy = layer.forward(cur, None if h0 is None else h0[l], None if c0 is None else c0[l])
-            hys.append(hy)
-            cys.append(cy)
-        return cur, hys, cys
+        if not x.is_cuda or x.dim() != 3 or x.shape[1] != self.B or x.shape[2] != self.I:
+            raise ValueError(f"x must be a CUDA tensor of shape (T, {self.B}, {self.I})")
+        x = x.contiguous()
+        T, shape = x.shape[0], (self.L, self.B, self.H)
+        h0, c0 = _layer_states(h0, shape, "h0"), _layer_states(c0, shape, "c0")
+        if h0 is not None and c0 is not None and h0.dtype != c0.dtype:
+            raise ValueError("h0 and c0 must share a dtype")
+        state = h0 if h0 is not None else c0
+        ys = [torch.empty((T, self.B, self.H), device=x.device, dtype=torch.float16) for _ in range(self.L)]
+        hy = torch.empty(shape, device=x.device, dtype=torch.float16)
+        cy = torch.empty_like(hy)
+        rc = self._lib.flstm_stack_forward(self._plans, self.L, T, x.data_ptr(), F16, _ptr(h0), _ptr(c0),
+                                           F16 if state is None else _dtype_code(state), _pointers(ys), F16, hy.data_ptr(),
+                                           cy.data_ptr(), LstmCore._stream())
+        if rc != 0:
+            raise RuntimeError(f"flstm_stack_forward failed with status {rc}")
+        self._inputs = [x] + ys[:-1]
+        return ys[-1], hy, cy
 
     def backward(self, dy_top, *, loss_scale="auto", d_hn: Optional[Sequence] = None,
                  d_cn: Optional[Sequence] = None, want_dx: bool = True, dy_factor: float = 1.0):
@@ -60,47 +100,60 @@ class LstmStack:
         2048 output is ~2e-9 per element: with a scale of 2^12 the bottom layer of a 4-layer stack loses all of
         its gradient).  The scale used is kept in self.last_loss_scale.
         Returns (dx of layer 0 (fp32 when a loss scale is in use) or None, [(dW_ih, dW_hh, db) per layer], [dh0 per layer], [dc0 per layer])."""
-        import math
-        import torch
+        return self._backward(dy_top, loss_scale, d_hn, d_cn, want_dx, dy_factor)[:4]
+
+    def _backward(self, dy_top, loss_scale, d_hn, d_cn, want_dx, dy_factor=1.0, dx_dtype=None, both_biases=False):
+        """backward(), one library call for the whole stack with one wait.  dx_dtype: of layer 0's dx (None: as backward()
+        documents); both_biases: a fifth result, the bias gradients again in tensors of their own (for bias_hh)."""
         if not self._inputs:
             raise RuntimeError("backward needs a forward pass first")
+        T, B, H, dev = self._inputs[0].shape[0], self.B, self.H, dy_top.device
+        if tuple(dy_top.shape) != (T, B, H):
+            raise ValueError(f"dy must have shape ({T}, {B}, {H})")
+        dy_top = dy_top.contiguous()
+        if dy_top.dtype not in (torch.float16, torch.float32):
+            dy_top = dy_top.float()
+        dy_code, stream = _dtype_code(dy_top), LstmCore._stream()
         if isinstance(loss_scale, str):
             if loss_scale != "auto":
                 raise ValueError("loss_scale must be a positive number or 'auto'")
-            lo, hi = torch.aminmax(dy_top)
-            amax = max(-float(lo), float(hi)) * abs(float(dy_factor))
+            amax = ctypes.c_float()
+            rc = self._lib.flstm_core_absmax(self._plans[0], dy_top.data_ptr(), dy_code, dy_top.numel(), ctypes.byref(amax), stream)
+            if rc != 0:
+                raise RuntimeError(f"flstm_core_absmax failed with status {rc}")
+            amax = amax.value * abs(float(dy_factor))
             S = 2.0 ** min(60, max(-14, math.floor(math.log2(64.0 / amax)))) if 0.0 < amax < float("inf") else 1.0
         else:
             S = float(loss_scale) if loss_scale and loss_scale > 0 else 1.0
         self.last_loss_scale = S
-        k = S * float(dy_factor)
-        if dy_top.dtype == torch.float16:
-            cur = dy_top * k if k != 1.0 else dy_top     # one pass: the product is formed in fp32 and rounded once
-        else:
-            cur = (dy_top.float() * k).half()
-        grads: List = [None] * self.L
-        dh0s: List = [None] * self.L
-        dc0s: List = [None] * self.L
-        for l in range(self.L - 1, -1, -1):
-            dhn = None if d_hn is None or d_hn[l] is None else (d_hn[l].float() * S)
-            dcn = None if d_cn is None or d_cn[l] is None else (d_cn[l].float() * S)
-            need_dx = want_dx or l > 0
-            dx, dW_ih, dW_hh, db, dh0, dc0 = self.layers[l].backward(self._inputs[l], cur, dhn, dcn, want_dx=need_dx,
-                                                                     dx_dtype=torch.float16)
-            if S != 1.0:
-                for t in (dW_ih, dW_hh, db, dh0, dc0):
-                    t.mul_(1.0 / S)
-            grads[l] = (dW_ih, dW_hh, db)
-            dh0s[l], dc0s[l] = dh0, dc0
-            cur = dx
-        if cur is not None and S != 1.0:
-            cur = cur.float() * (1.0 / S)   # fp32: the unscaled values may lie below the fp16 range
-        return cur, grads, dh0s, dc0s
+        if dx_dtype is None:
+            dx_dtype = torch.float16 if S == 1.0 else torch.float32   # fp32: the unscaled values may lie below the fp16 range
+        ins = [self._inputs[l].shape[2] for l in range(self.L)]
+        f32 = lambda *shape: torch.empty(shape, device=dev, dtype=torch.float32)
+        dxs = [torch.empty((T, B, ins[l]), device=dev, dtype=torch.float16 if l > 0 else dx_dtype) if l > 0 or want_dx else None
+               for l in range(self.L)]
+        dW_ih, dW_hh = [f32(4 * H, ins[l]) for l in range(self.L)], [f32(4 * H, H) for _ in range(self.L)]
+        db = [f32(4 * H) for _ in range(self.L)]
+        db2 = [f32(4 * H) for _ in range(self.L)] if both_biases else None
+        dh0, dc0 = f32(self.L, B, H), f32(self.L, B, H)
+        states = []
+        for grads, name in ((d_hn, "d_hn"), (d_cn, "d_cn")):
+            grads = None if grads is None else [None if g is None else g.float().contiguous() for g in grads]
+            if grads is not None and (len(grads) != self.L or any(g is not None and tuple(g.shape) != (B, H) for g in grads)):
+                raise ValueError(f"{name} must hold one tensor of shape ({B}, {H}) (or None) per layer")
+            states.append(grads)
+        rc = self._lib.flstm_stack_backward(
+            self._plans, self.L, T, _pointers(self._inputs), F16, dy_top.data_ptr(), dy_code, S * float(dy_factor),
+            None if states[0] is None else _pointers(states[0]), None if states[1] is None else _pointers(states[1]), F32, S,
+            _pointers(dxs), F16 if dxs[0] is None else _dtype_code(dxs[0]), _pointers(dW_ih), _pointers(dW_hh), _pointers(db),
+            None if db2 is None else _pointers(db2), _pointers(list(dh0.unbind(0))), _pointers(list(dc0.unbind(0))), stream)
+        if rc != 0:
+            raise RuntimeError(f"flstm_stack_backward failed with status {rc}")
+        return dxs[0], list(zip(dW_ih, dW_hh, db)), list(dh0.unbind(0)), list(dc0.unbind(0)), db2, dh0, dc0
 
     def backward_mse(self, y_top, target, **kwargs):
         """backward() for the loss mean((y_top - target)^2) over all elements: its gradient 2 / N * (y_top - target) is
         handed over as the fp16 difference and the factor 2 / N (see dy_factor).  y_top: what forward() returned."""
-        import torch
         if y_top.dtype != torch.float16 or target.dtype != torch.float16:
             return self.backward((y_top.float() - target.float()), dy_factor=2.0 / y_top.numel(), **kwargs)
         return self.backward(torch.sub(y_top, target), dy_factor=2.0 / y_top.numel(), **kwargs)
@@ -113,36 +166,37 @@ class _StackFunction(torch.autograd.Function):
     def forward(ctx, module, x, h0, c0, y_dtype, loss_scale, *params):
         L = module.num_layers
         stack = module._stack_for(x.shape[1])
-        stack.pack([tuple(p.detach() for p in params[4 * l:4 * l + 4]) for l in range(L)])
-        y, hys, cys = stack.forward(x.detach(), None if h0 is None else list(h0.detach().half()),
-                                    None if c0 is None else list(c0.detach().half()))
+        with torch.no_grad():
+            stream = LstmCore._stream()
+            for l, layer in enumerate(stack.layers):
+                layer._pack_enqueue(*params[4 * l:4 * l + 4], stream)
+            y, hy, cy = stack._forward(x, None if h0 is None else h0.half(), None if c0 is None else c0.half())
+            if y_dtype != y.dtype:
+                y = y.to(y_dtype)
         module._generation += 1
         ctx.module, ctx.stack, ctx.generation, ctx.loss_scale = module, stack, module._generation, loss_scale
         ctx.has_state = (h0 is not None, c0 is not None)
         ctx.x_dtype = x.dtype
-        if y_dtype != y.dtype:
-            y = y.to(y_dtype)
-        return y, torch.stack(hys), torch.stack(cys)
+        ctx.set_materialize_grads(False)   # (a gradient nobody has stays None instead of becoming a tensor of zeros)
+        return y, hy, cy
 
     @staticmethod
     def backward(ctx, dy, dhn, dcn):
         if ctx.generation != ctx.module._generation:
             raise RuntimeError("StackedLSTM keeps the caches of its most recent forward pass only: call backward "
                                "before the next forward pass of the same module")
-        L = ctx.module.num_layers
-        zero_state = lambda g: None if g is None else list(g)
+        stack = ctx.stack
         if dy is None:
-            dy = torch.zeros((ctx.stack._inputs[0].shape[0], ctx.stack.B, ctx.stack.H), device=dhn.device, dtype=torch.float16)
-        dx, grads, dh0s, dc0s = ctx.stack.backward(dy, loss_scale=ctx.loss_scale, d_hn=zero_state(dhn), d_cn=zero_state(dcn),
-                                                   want_dx=ctx.needs_input_grad[1])
+            x = stack._inputs[0]
+            dy = torch.zeros((x.shape[0], stack.B, stack.H), device=x.device, dtype=torch.float16)
+        dx, grads, _, _, db_hh, dh0, dc0 = stack._backward(dy, ctx.loss_scale, dhn, dcn, ctx.needs_input_grad[1],
+                                                           dx_dtype=ctx.x_dtype, both_biases=True)
         flat = []
-        for l in range(L):
-            dW_ih, dW_hh, db = grads[l]
-            flat += [dW_ih, dW_hh, db, db.clone()]
-        gx = None if dx is None else dx.to(ctx.x_dtype)
-        gh0 = torch.stack(dh0s).half() if ctx.has_state[0] and ctx.needs_input_grad[2] else None
-        gc0 = torch.stack(dc0s).half() if ctx.has_state[1] and ctx.needs_input_grad[3] else None
-        return (None, gx, gh0, gc0, None, None, *flat)
+        for (dW_ih, dW_hh, db), db2 in zip(grads, db_hh):
+            flat += [dW_ih, dW_hh, db, db2]
+        gh0 = dh0.half() if ctx.has_state[0] and ctx.needs_input_grad[2] else None
+        gc0 = dc0.half() if ctx.has_state[1] and ctx.needs_input_grad[3] else None
+        return (None, dx, gh0, gc0, None, None, *flat)
 
 
 class StackedLSTM(torch.nn.Module):

@@ -122,6 +122,31 @@ int flstm_core_backward(flstm_core_plan* plan, size_t seq_len,
                         float* dW_ih, float* dW_hh, float* db_ih, float* db_hh,
                         float* dh0, float* dc0, void* stream);
 
+/* Stacks: `layers` plans of one batch and hidden size, plan 0 with its own input size and the others with input size =
+ * hidden size, run as one call per direction: layer behind layer on the stream, ONE wait at the end.  (The reference is
+ * single-layer.)  A layer whose persistent launch gave up is repeated step-wise, with the layers that depend on it.
+ * forward: ys[l] receives layer l's outputs (T, B, H) and is layer l + 1's input; h0, c0, hy, cy are (layers, B, H), h0 / c0
+ *   may be null; ys, hy and cy have y_dtype.  The caches of all layers are kept.
+ * backward: xs[l] is what layer l read in forward (fp16 for l > 0); the gradient of the top layer's outputs is
+ *   dy_scale * dY, where dy_scale contains loss_scale (a power of two) already; d_hn / d_cn may be null, their entries too.
+ *   Gradients travel between layers in fp16 (dxs[l], l > 0) with the loss scale on them; it is divided out of dxs[0]
+ *   (dx_dtype, may be null) and of everything else returned.  db_ih and db_hh receive the same values (db_hh may be null).
+ *   Not with "accumulate_grads". */
+int flstm_stack_forward(flstm_core_plan* const* plans, int layers, size_t seq_len, const void* x, flstm_dtype x_dtype,
+                        const void* h0, const void* c0, flstm_dtype state_dtype, void* const* ys, flstm_dtype y_dtype,
+                        void* hy, void* cy, void* stream);
+int flstm_stack_backward(flstm_core_plan* const* plans, int layers, size_t seq_len, const void* const* xs, flstm_dtype x_dtype,
+                         const void* dY, flstm_dtype dy_dtype, float dy_scale, const void* const* d_hn,
+                         const void* const* d_cn, flstm_dtype dstate_dtype, float loss_scale, void* const* dxs,
+                         flstm_dtype dx_dtype, float* const* dW_ih, float* const* dW_hh, float* const* db_ih,
+                         float* const* db_hh, float* const* dh0, float* const* dc0, void* stream);
+/* Weights and biases in one call that only enqueues (flstm_core_pack_weights waits): for callers whose next pass of the
+ * plan runs on the same stream and who keep the tensors until then. */
+int flstm_core_pack(flstm_core_plan* plan, const float* w_ih, const float* w_hh, const float* b_ih, const float* b_hh,
+                    void* stream);
+/* The largest |value| of n elements of a device tensor, NaN if there is one; waits for the stream. */
+int flstm_core_absmax(flstm_core_plan* plan, const void* tensor, flstm_dtype dtype, size_t n, float* out, void* stream);
+
 /* The same two passes fed in ranges of time steps, for callers that stream a sequence through the device
  * while it is being processed.  (No counterpart in the reference, which walks 32-step chunks inside
  * flashlstm_v2/src/lstm_forward.cu:646-940 and lstm_backward.cu:897-1213; this is the hook its replacement
@@ -150,7 +175,7 @@ int flstm_core_backward_end(flstm_core_plan* plan, const void* x, flstm_dtype x_
 int flstm_core_cache_ptr(const flstm_core_plan* plan, int which, const void** ptr, size_t* ld);
 
 /* Average device time in milliseconds of the phases of the most recent forward / backward,
- * measured with events on the call's stream: names "fwd_proj", "fwd_rec", "fwd_total",
+ * measured by time stamps the kernels leave: names "fwd_proj", "fwd_rec", "fwd_total",
  * "bwd_rec", "bwd_dx", "bwd_dw", "bwd_total".  Negative when not available. */
 double flstm_core_last_ms(const flstm_core_plan* plan, const char* phase);
 
