@@ -340,10 +340,10 @@ extern "C" int flstm_core_set_option(flstm_core_plan* p, const char* name, long 
         // wavefronts per workgroup of the forward recurrence: the weight fragments are packed for it, so a change
         // un-packs them
         if (value != 0 && value != 4 && value != 8) return FLSTM_E_INVALID;
-        const int before = p->Lf.nw;
+        const int before = p->Lf.nw, split_before = p->Lf.split;
         p->opt_waves_f = int(value);
         replan(p);
-        if (p->Lf.nw != before) p->weights_packed = false;
+        if (p->Lf.nw != before || p->Lf.split != split_before) p->weights_packed = false;
         return 0;
     }
     if (!strcmp(name, "inject_stall")) { if (value < 0) return FLSTM_E_INVALID; p->inject_stall = int(value); return 0; }
@@ -415,7 +415,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     const Dims& d = p->d;
     FL_TRY(p->wih_p.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
     FL_TRY(p->wih_t.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
-    FL_TRY(p->wfrag_f.reserve(size_t(p->Lf.nh) * p->Lf.nw * p->ks_f * p->Lf.nt * kWave * sizeof(half8)));
+    FL_TRY(p->wfrag_f.reserve(rec_fwd_fragments(p->Lf, d.Hp) * kWave * sizeof(half8)));
     FL_TRY(p->wfrag_b.reserve(size_t(p->Lb.nh) * p->Lb.nw * p->ks_b * p->Lb.nt * kWave * sizeof(half8)));
     auto layout = [](const DevBuf& out, const RecLayout& L, int ks) {
         FragLayout f;
@@ -423,7 +423,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
         return f;
     };
     FragLayout fwd = layout(p->wfrag_f, p->Lf, p->ks_f), bwd = layout(p->wfrag_b, p->Lb, p->ks_b), two_d;
-    fwd.wide = p->Lf.wide;
+    fwd.wide = p->Lf.wide; fwd.split = p->Lf.split; fwd.fragments = rec_fwd_fragments(p->Lf, d.Hp);
     if (rec_bwd_two_d_possible(d.Hp, p->num_cus)) {   // whether or not the current layout uses them
         FL_TRY(p->wfrag_b2.reserve(rec_bwd_two_d_wfrag_bytes(d.Hp)));
         two_d.out = p->wfrag_b2.as<half8>();

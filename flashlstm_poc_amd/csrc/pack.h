@@ -17,7 +17,8 @@ struct Dims {
 // PyTorch-layout weights -> the fp16 operand layouts of the kernels in this library.
 struct FragLayout {   // where a recurrence kernel expects its weight fragments: RecLayout's description of them
     half8* out = nullptr;
-    int ks = 0, nt = 0, rot_div = 0, nw = 0, unit_major = 0, wide = 0, kq = 0;
+    int ks = 0, nt = 0, rot_div = 0, nw = 0, unit_major = 0, wide = 0, kq = 0, split = 0;
+    size_t fragments = 0;   // forward
 };
 // W_ih twice (as it is for the projection, transposed for dX) and W_hh as forward fragments, backward fragments and (two_d.out
 // set) those of the backward recurrence that splits its product two ways; one launch.

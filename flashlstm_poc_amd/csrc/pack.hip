@@ -38,17 +38,22 @@ __device__ __forceinline__ half8 frag_values_fwd(const Dims& d, const float* __r
     // unit-major, column c = 4 * unit + gate: the four accumulation registers of a lane are then the four gates of one
     // unit.  Fragment (hs, wave, ks, n): lane l holds column c = n*16 + l%16 of slice hs, k = (ks*nw + wave)*32 + 8*(l/16)
     // + e, e = 0..7 (nw = wavefronts per workgroup, 4 or 8).
+    // split (rec_fwd_split_kernel): a wave has two tiles over the whole contraction, column c of tile n is gate c % 4 of
+    // its unit 2 (c / 4) + n.
+    const int tiles = f.split ? 2 : f.nt;
     unsigned r = unsigned(item);
     const int lane = int(r % kWave); r /= kWave;
-    const int n = int(r % f.nt); r /= f.nt;
+    const int n = int(r % tiles); r /= tiles;
     const int ks = int(r % f.ks); r /= f.ks;
-    const int wave = int(r % f.nw);
-    const int hs = int(r / f.nw);
-    const int jb = 4 * f.nt, c = n * 16 + lane % 16, nh = d.Hp / jb;
-    const int gate = f.unit_major ? c % 4 : c / jb, unit = hs * jb + (f.unit_major ? c / 4 : c % jb);
+    const int nw = f.split ? f.split : f.nw;
+    const int wave = int(r % nw);
+    const int hs = int(r / nw);
+    const int jb = f.split ? 8 * f.split : 4 * f.nt, c = n * 16 + lane % 16, nh = d.Hp / jb;
+    const int gate = f.unit_major || f.split ? c % 4 : c / jb;
+    const int unit = hs * jb + (f.split ? wave * 8 + 2 * ((c % 16) / 4) + n : f.unit_major ? c / 4 : c % jb);
     // (slot ks of slice hs holds a rotated k-step: recurrent.h, rec_kstep_rotation, rec_wide_rotation)
     const int kstep = f.wide ? (ks ^ rec_wide_rotation(ks, hs / 8, f.ks)) : rec_kstep_of_slot(ks, rec_kstep_rotation(hs, nh, f.ks, f.rot_div), f.ks);
-    const int k = (kstep * f.nw + wave) * 32 + 8 * (lane / 16);
+    const int k = (f.split ? ks : kstep * f.nw + wave) * 32 + 8 * (lane / 16);
     half8 v{};
     if (unit < d.H) {
         const float* row = w_hh + size_t(gate * d.H + unit) * d.H;
@@ -136,7 +141,7 @@ __global__ __launch_bounds__(kT) void pack_kernel(PackJob job) {
         st_half8(job.wih_t + size_t(i) * 4 * d.Hp + q, v);
     } else {
         const FragLayout& f = job.frag[which - 2];
-        const size_t n = which == 2 ? size_t(d.Hp / (4 * f.nt)) * f.nw * f.ks * f.nt * kWave
+        const size_t n = which == 2 ? f.fragments * kWave
                        : which == 3 ? size_t(d.Hp / (16 * f.nt)) * f.nw * f.ks * f.nt * kWave : size_t(d.Hp / 64) * f.kq * 4 * f.ks * 4 * kWave;
         if (item >= n) return;
         f.out[item] = which == 2 ? frag_values_fwd(d, job.w_hh, f, item) : which == 3 ? frag_values_bwd(d, job.w_hh, f, item) : frag_values_two_d(d, job.w_hh, f, item);
@@ -291,7 +296,7 @@ hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, hal
     job.frag[0] = fwd; job.frag[1] = bwd; job.frag[2] = two_d;
     // (Hp is a multiple of 32 and Ip of 64: whole chunks of eight, and of four chunks, everywhere)
     const size_t items[5] = {size_t(4) * d.Hp * d.Ip / 8, size_t(4) * d.Hp * d.Ip / 8,
-                             size_t(d.Hp / (4 * fwd.nt)) * fwd.nw * fwd.ks * fwd.nt * kWave,
+                             fwd.fragments * kWave,
                              size_t(d.Hp / (16 * bwd.nt)) * bwd.nw * bwd.ks * bwd.nt * kWave,
                              two_d.out ? size_t(d.Hp / 64) * two_d.kq * 4 * two_d.ks * 4 * kWave : 0};
     for (int i = 0; i < 5; ++i) {

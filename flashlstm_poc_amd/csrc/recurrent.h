@@ -30,6 +30,7 @@ struct RecLayout {
                      // launch_persistent's own gate
     int unit_major;  // forward: gate columns of a slice are packed 4 * unit + gate (kernels with one cell per thread), else gate
                      // blocks of jb units
+    int split;       // the kernels for short contractions (rec_fwd_split_kernel, rec_bwd_pair_kernel): waves per workgroup
     int wide;        // more than 2048 hidden units, weights resident (rec_fwd_wide_kernel, rec_bwd_wide_kernel)
     int num_cus;     // of the device the layout was made for
     int rot_div;     // k-step rotation (rec_kstep_rotation): slices rot_div apart run on the same XCD
@@ -194,6 +195,8 @@ int rec_bwd_ring_rows(const RecLayout& L, int B);
 
 // Halfs in one slot of an exchange ring for a [rows][cols] operand (rows padded to 32).
 size_t exchange_slot_halfs(int rows, int cols);
+// Fragments (64 lanes of 16 bytes) of a forward layout.
+size_t rec_fwd_fragments(const RecLayout& L, int Hp);
 // Number of k-steps (32 wide) every wave holds for a layout (sizes the fragment arrays).
 int rec_fwd_ks(const RecLayout& L, int Hp);
 int rec_bwd_ks(const RecLayout& L, int Hp);

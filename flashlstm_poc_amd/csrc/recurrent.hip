@@ -38,6 +38,7 @@
 #include <cstring>
 #include <mutex>
 #include <type_traits>
+#include <utility>
 
 #include "layout_device.h"
 #include "recurrent.h"
@@ -241,6 +242,18 @@ __device__ __forceinline__ void wait_frags(half8 (&a)[8]) {
                  : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7])
                  : "n"(N)
                  : "memory");
+}
+
+// ... for a set of any even size: the count stands in the first statement, the others only name the rest (volatile
+// statements keep their order, so no use moves above them).
+template <int N, int K>
+__device__ __forceinline__ void wait_set(half8 (&a)[K]) {
+    static_assert(K % 2 == 0, "pairs");
+#pragma unroll
+    for (int k = 0; k < K; k += 2) {
+        if (k == 0) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(a[k]), "+v"(a[k + 1]) : "n"(N) : "memory");
+        else asm volatile("" : "+v"(a[k]), "+v"(a[k + 1])::"memory");
+    }
 }
 
 // The same with the count as a value: for callers whose count is a constant only after unrolling.
@@ -1370,6 +1383,206 @@ __global__ __launch_bounds__(8 * kWave) void rec_fwd_il_kernel(RecFwdArgs p, Rec
     clk.flush();
 }
 
+// Phase counters of workgroup 0 (PhaseClock) with everything in LDS.
+struct WideClock {
+    long long* out;
+    __device__ __forceinline__ long long* lds() {
+        __shared__ long long mem[8];   // 0..4 phases, 5 engine clock at the start, 6 wall clock at the start, 7 last lap
+        return mem;
+    }
+    __device__ __forceinline__ void start() {
+        if (out && threadIdx.x == 0) {
+            for (int i = 0; i < 5; ++i) lds()[i] = 0;
+            lds()[6] = lds()[7] = wall_clock64();
+            lds()[5] = clock64();
+        }
+    }
+    __device__ __forceinline__ void lap(int slot) {
+        if (__builtin_expect(out != nullptr, 0)) {
+            if (threadIdx.x == 0) {
+                const long long now = wall_clock64();
+                lds()[slot] += now - lds()[7];
+                lds()[7] = now;
+            }
+        }
+    }
+    __device__ __forceinline__ void flush() {
+        if (out && threadIdx.x == 0) {
+            for (int i = 0; i < 5; ++i) out[i] += lds()[i];
+            out[5] += clock64() - lds()[5];
+            out[6] += wall_clock64() - lds()[6];
+        }
+    }
+};
+
+// ------------------------------------------------------------------- forward, short contractions
+// Up to 512 hidden units the product of a step is short and the kernels above spend their time around it: at 256 units
+// and 8 rows 0.55 of 1.44 us waiting and multiplying, 0.25 turning partial sums through LDS and 0.44 collecting them and
+// updating cells.  Here the waves of a slice split its gate COLUMNS instead of the contraction: each multiplies the
+// whole operand by the 32 columns of its own 8 units and finds the sums of its cells in its accumulators.  Columns are
+// packed so that tile n holds gate c % 4 of unit 2 (c / 4) + n: a lane ends up with all four gates of two neighbouring
+// units of one row, i.e. one 32-bit word of the ring.  Nothing crosses waves, so there is no LDS and no barrier in a
+// step; a wave is a producer and a consumer of its own.  The price is the fetch: every wave loads the whole operand.
+// One 16-row block per group (the layout takes this kernel where all of them run side by side), and as few waves per
+// workgroup as the batch allows: one (8 units), two or four.
+// Measured, us per step, rec_fwd_kernel -> here: 32 units 1.45 -> 0.50, 64 units 1.45 -> 0.53, 128 units 0.63, 256 units
+// and 8 rows 1.44 -> 0.77, 257 units and 70 rows 1.6 -> 1.19, 512 units and 64 rows 1.64 -> 1.34.  What is left at 256
+// units is the exchange: a store's and a load's trip through the L2, then 16 MFMAs and two cells' transcendentals.
+// The x-projection of step t + 1 is requested behind the fragments of step t: it has landed before the fragments of its
+// step, which are younger.  The ring protocol is the one of rec_fwd_kernel, with waves for workgroups: a wave whose product
+// of step t is complete knows that every wave of its group has stored h_{t-1}, i.e. is done reading h_{t-2}, and marks; the
+// mark is acknowledged before the next step's fragments have landed, i.e. before the next h goes out.
+template <int OFF>
+__device__ __forceinline__ void ld_frag_async_off(half8& dst, unsigned lane_off, const half_t* base) {
+    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3 sc1" : "=v"(dst) : "v"(lane_off), "s"(base), "n"(OFF) : "memory");
+}
+template <int KS, int K>
+__device__ __forceinline__ void request_split_one(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off) {
+    if constexpr (K >= KS - 3) ld_frag_async_off<0>(f[K], tail_off[K - (KS - 3)], tile);
+    else ld_frag_async_off<(K % 4) * 1024>(f[K], lane_off[K / 4], tile);
+}
+template <int KS, int... K>
+__device__ __forceinline__ void request_split(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off,
+                                              std::integer_sequence<int, K...>) {
+    (request_split_one<KS, K>(f, tile, lane_off, tail_off), ...);
+}
+__device__ __forceinline__ void ld_stream_at(uintx4& d, const void* base, unsigned off) {
+    asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+template <int KS>
+__global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, RecLayout L, int t_begin, int t_end, int) {
+    static_assert(KS % 2 == 0 && KS <= 16, "up to 512 hidden units");
+    __shared__ int lds_abort;
+    __shared__ int lds_role[2];
+    if (threadIdx.x == 0) lds_abort = 0;
+    __syncthreads();
+    const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
+    if (!role.active) {
+        copy_beside(p.beside, lds_role);
+        return;
+    }
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int hs = role.hs, g = role.g;
+    const int nks = p.Hp / 32;
+    const Poll poll{L.persistent != 0, p.spin_limit, p.spin_ticks, p.status, (lds_int_t*)&lds_abort};
+    WideClock clk{(hs == 0 && g == 0) ? p.prof : nullptr};
+
+    half8 wreg[KS][2];
+    {
+        const half8* wf = p.wfrag + (size_t(hs) * L.split + wave) * size_t(KS) * 2 * kWave;
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) wreg[k][n] = wf[(k * 2 + n) * kWave + lane];
+    }
+    // this lane's two cells: row r, units j and j + 1.  Arrays are addressed as scalar base + 32 bits per lane.
+    const int r = lane % 16, j = hs * L.jb + wave * 8 + 2 * (lane / 16);
+    const int b0 = g * 16;
+    const bool live = b0 + r < p.B;
+    const unsigned row = unsigned(min(r, p.B - 1 - b0)), cell = row * unsigned(p.Hp) + unsigned(j);
+    const unsigned off_ring = unsigned(xch_offset(r, j, nks));          // inside the tile, in halfs
+    const size_t tile_halfs = size_t(nks) * 512;
+    // (a kernel serves contractions up to three k-steps shorter than its own: those hold zero weights and fetch the last
+    // k-step there is)
+    unsigned lane_off[(KS + 3) / 4], tail_off[3];
+#pragma unroll
+    for (int q = 0; q < (KS + 3) / 4; ++q) lane_off[q] = unsigned(lane) * 16u + unsigned(q) * 4096u;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) tail_off[q] = unsigned(lane) * 16u + unsigned(min(max(KS - 3 + q, 0), nks - 1)) * 1024u;
+    float c[2];
+    {
+        const float* src = p.C + (size_t(t_begin) * p.B + b0) * p.Hp + cell;
+        c[0] = src[0];
+        c[1] = src[1];
+    }
+    uintx4 xp[2];   // by parity of the step
+    auto request_xp = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        ld_stream_at(xp[par], p.G + (size_t(t) * p.B + b0) * (size_t(4) * p.Hp), cell * 8u);
+    };
+    if (p.stamps && t_begin == p.t0 && hs == 0 && g == 0 && tid == 0) p.stamps[0] = wall_clock64();
+    loads_landed();
+    clk.start();
+    request_xp(t_begin, std::integral_constant<int, 0>{});
+
+    auto step = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        const half_t* tile = wave_uniform(p.X + size_t(t & 3) * p.x_slot + size_t(g) * tile_halfs);
+        half8 f[KS];
+        auto request = [&]() __attribute__((always_inline)) { request_split(f, tile, lane_off, tail_off, std::make_integer_sequence<int, KS>{}); };
+        request();
+        request_xp(t + 1 < t_end ? t + 1 : t, std::integral_constant<int, 1 - par>{});
+        wait_set<1>(f);
+        auto unwritten = [&]() -> bool {
+            unsigned m = 0u;
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const uint4 ua = __builtin_bit_cast(uint4, f[k]);
+                m = max(m, max(max(ua.x, ua.y), max(ua.z, ua.w)));
+            }
+            return __any(m == kUnwritten) != 0;
+        };
+        if (__builtin_expect(unwritten() && poll.on, 0)) {
+            int spins = 0;
+            long long spin_start = 0;
+            do {
+                if (poll_give_up(poll, spins, spin_start, lane)) leave_kernel();   // (the other waves of the group run into the same bound)
+                request();
+                wait_set<0>(f);
+            } while (unwritten());
+        }
+        floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[k][n], f[k], acc[n], 0, 0, 0);
+        clk.lap(0);
+        settle(xp[par]);
+        half_t* const xout = p.X + size_t((t + 1) & 3) * p.x_slot + size_t(g) * tile_halfs;
+        half_t* const xnext = p.X + size_t((t + 3) & 3) * p.x_slot + size_t(g) * tile_halfs;
+        store_xch(xnext + off_ring, Pack<2>{kUnwritten}, false);
+        float hn[2], gates[2][4];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            float z[4];
+            unpack_h2(n == 0 ? xp[par].x : xp[par].z, z[0], z[1]);
+            unpack_h2(n == 0 ? xp[par].y : xp[par].w, z[2], z[3]);
+#pragma unroll
+            for (int gt = 0; gt < 4; ++gt) z[gt] += acc[n][gt];
+            const float ig = sigmoidf_dev(z[0]), fg = sigmoidf_dev(z[1]), gg = tanhf_dev(z[2]), og = sigmoidf_dev(z[3]);
+            c[n] = fg * c[n] + ig * gg;
+            hn[n] = og * tanhf_dev(c[n]);
+            gates[n][0] = ig; gates[n][1] = fg; gates[n][2] = gg; gates[n][3] = og;
+        }
+        const unsigned h2 = live ? pack_h2(hn[0], hn[1]) : 0u;   // (rows past B travel as zeros)
+        store_xch(xout + off_ring, Pack<2>{h2}, false);
+        clk.lap(2);
+        // caches for the backward pass: off the critical path
+        if (live) {
+            const size_t row0 = size_t(t) * p.B + b0;
+            __builtin_nontemporal_store(floatx2{c[0], c[1]}, reinterpret_cast<floatx2*>(p.C + (row0 + p.B) * p.Hp + cell));
+            __builtin_nontemporal_store(h2, reinterpret_cast<unsigned*>(p.Y + (row0 + p.B) * p.Hp + cell));
+            if (p.y_out) __builtin_nontemporal_store(h2, reinterpret_cast<unsigned*>(p.y_out + row0 * p.Hp + cell));
+            __builtin_nontemporal_store(uintx4{pack_h2(gates[0][0], gates[0][1]), pack_h2(gates[0][2], gates[0][3]),
+                                               pack_h2(gates[1][0], gates[1][1]), pack_h2(gates[1][2], gates[1][3])},
+                                        reinterpret_cast<uintx4*>(p.G + row0 * (size_t(4) * p.Hp) + 4u * cell));
+        }
+        clk.lap(3);
+    };
+    int t = t_begin;
+    for (; t + 1 < t_end; t += 2) {
+        step(t, std::integral_constant<int, 0>{});
+        step(t + 1, std::integral_constant<int, 1>{});
+    }
+    if (t < t_end) step(t, std::integral_constant<int, 0>{});
+    wait_all_vm();
+    settle(xp[0]);   // (the last request is used by nobody, but its registers must not be handed on before it has landed)
+    settle(xp[1]);
+    if (p.stamps && hs == 0 && g == 0 && tid == 0) p.stamps[1] = wall_clock64();
+    clk.flush();
+}
+
 // ---------------------------------------------------------------------- more than 2048 hidden units
 // W_hh of 4096 units is 128 MiB.  Streamed from memory every step that is 27 us forward and 90 us backward at 32 rows;
 // the chip holds 128 MiB of registers and 40 MiB of LDS, so up to 4096 units it can stay resident: 512 KiB per workgroup,
@@ -1531,37 +1744,6 @@ __device__ __forceinline__ void ld_coherent_at(unsigned& d, const void* base, un
 __device__ __forceinline__ void ld_coherent_at(uintx4& d, const void* base, unsigned off) {
     asm volatile("global_load_dwordx4 %0, %1, %2 sc1" : "=v"(d) : "v"(off), "s"(base) : "memory");
 }
-// Phase counters of workgroup 0 (PhaseClock) with everything in LDS.
-struct WideClock {
-    long long* out;
-    __device__ __forceinline__ long long* lds() {
-        __shared__ long long mem[8];   // 0..4 phases, 5 engine clock at the start, 6 wall clock at the start, 7 last lap
-        return mem;
-    }
-    __device__ __forceinline__ void start() {
-        if (out && threadIdx.x == 0) {
-            for (int i = 0; i < 5; ++i) lds()[i] = 0;
-            lds()[6] = lds()[7] = wall_clock64();
-            lds()[5] = clock64();
-        }
-    }
-    __device__ __forceinline__ void lap(int slot) {
-        if (__builtin_expect(out != nullptr, 0)) {
-            if (threadIdx.x == 0) {
-                const long long now = wall_clock64();
-                lds()[slot] += now - lds()[7];
-                lds()[7] = now;
-            }
-        }
-    }
-    __device__ __forceinline__ void flush() {
-        if (out && threadIdx.x == 0) {
-            for (int i = 0; i < 5; ++i) out[i] += lds()[i];
-            out[5] += clock64() - lds()[5];
-            out[6] += wall_clock64() - lds()[6];
-        }
-    }
-};
 // the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
 __device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
 __device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
@@ -2224,6 +2406,224 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
     }
 }
 
+// -------------------------------------------------------------------- backward, short contractions
+// The same for the backward recurrence up to 384 units, with what its four times longer contraction allows: a workgroup of
+// TWO waves owns 16 units (one column tile).  The waves split the contraction, exchange half of their sums through LDS (8
+// bytes per lane, one barrier) and update the cells of two neighbouring units each, one 16-byte chunk of the ring per lane.
+// Against the kernel above: as many fragment loads per CU, half the columns to sum over half the waves.  The operands of
+// step t - 1 (gates, c, dY) are requested behind the fragments of step t.
+// Measured, us per step, rec_bwd_kernel -> here: 64 units 1.62 -> 1.07, 128 units 1.71 -> 1.22, 256 units and 8 rows
+// 1.79 -> 1.54, 257 units and 70 rows 2.13 -> 1.84, 384 units 2.13 -> 1.93.  (Four waves with one cell per lane: 1.65 at
+// 256 units; the longer barrier costs more than the shorter update gives.)
+template <int KS, int K>
+__device__ __forceinline__ void request_pair_one(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off) {
+    if constexpr (K >= KS - 3) ld_frag_async_off<0>(f[K], tail_off[K - (KS - 3)], tile);
+    else ld_frag_async_off<(K % 2) * 2048>(f[K], lane_off[K / 2], tile);
+}
+template <int KS, int... K>
+__device__ __forceinline__ void request_pair(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off,
+                                             std::integer_sequence<int, K...>) {
+    (request_pair_one<KS, K>(f, tile, lane_off, tail_off), ...);
+}
+__device__ __forceinline__ void ld_stream_at(floatx2& d, const void* base, unsigned off) {
+    asm volatile("global_load_dwordx2 %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void ld_stream_at(unsigned& d, const void* base, unsigned off) {
+    asm volatile("global_load_dword %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
+}
+template <int KS>
+__global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, RecLayout L, int t_first, int t_last, int) {
+    static_assert(KS % 4 == 0 && KS <= 24, "up to 384 hidden units");
+    __shared__ int lds_abort;
+    __shared__ int lds_role[2];
+    __shared__ floatx2 swap[2][2][kWave];   // [step parity][receiving wave]
+    __shared__ float red[2 * kWave][8];
+    if (threadIdx.x == 0) lds_abort = 0;
+    __syncthreads();
+    const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
+    if (!role.active) {
+        copy_beside(p.beside, lds_role);
+        return;
+    }
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int hs = role.hs, g = role.g;
+    const int nks = p.Hp / 8;
+    const Poll poll{L.persistent != 0, p.spin_limit, p.spin_ticks, p.status, (lds_int_t*)&lds_abort};
+    const float S = p.dy_scale;
+    WideClock clk{(hs == 0 && g == 0) ? p.prof : nullptr};
+
+    half8 wreg[KS];
+    {
+        const int real = nks / 2;   // k-steps per wave in the packed weights
+        const half8* wf = p.wfrag + (size_t(hs) * 2 + wave) * size_t(real) * kWave;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) wreg[k] = (k < real) ? wf[k * kWave + lane] : half8{};
+    }
+    const size_t gld = size_t(4) * p.Hp;
+    const int r = lane % 16, j = hs * 16 + 4 * (lane / 16) + 2 * wave;   // this lane's cells: row r, units j and j + 1
+    const int b0 = g * 16;
+    const bool live = b0 + r < p.B;
+    const unsigned row = unsigned(min(r, p.B - 1 - b0)), cell = row * unsigned(p.Hp) + unsigned(j);
+    const unsigned off_ring = unsigned(xch_offset(r, 4 * j, nks));
+    const size_t tile_halfs = size_t(nks) * 512;
+    // wave w takes k-steps 2k + w; (a kernel serves contractions up to two k-steps per wave shorter than its own)
+    unsigned lane_off[KS / 2], tail_off[3];
+#pragma unroll
+    for (int q = 0; q < KS / 2; ++q) lane_off[q] = unsigned(lane) * 16u + unsigned(wave) * 1024u + unsigned(q) * 4096u;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) tail_off[q] = unsigned(lane) * 16u + unsigned(min(2 * (KS - 3 + q) + wave, nks - 1)) * 1024u;
+
+    uintx4 gates[2];          // by parity of the steps done
+    floatx2 cprev[2], ccur[2];   // c_{t-1}, c_t
+    unsigned dy2[2];
+    auto request_ops = [&](int t, auto parity) __attribute__((always_inline)) {   // four loads; the closing pass fetches step 0
+        constexpr int par = decltype(parity)::value;
+        const size_t row0 = size_t(max(t, 0)) * p.B + b0;
+        ld_stream_at(gates[par], p.G + row0 * gld, cell * 8u);
+        ld_stream_at(cprev[par], p.C + row0 * p.Hp, cell * 4u);
+        ld_stream_at(ccur[par], p.C + (row0 + p.B) * p.Hp, cell * 4u);
+        ld_stream_at(dy2[par], p.dY + row0 * p.Hp, cell * 2u);
+    };
+    float dc[2];
+    {
+        const float* src = p.dC + size_t(b0) * p.Hp + cell;
+        dc[0] = src[0];
+        dc[1] = src[1];
+    }
+    float dbacc[4][2] = {};
+    __syncthreads();
+    loads_landed();
+    clk.start();
+    auto settle_ops = [&](auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        settle(gates[par]);
+        settle(cprev[par]);
+        settle(ccur[par]);
+        settle(dy2[par]);
+    };
+    auto cell_update = [&](int t, const float (&dh)[2], auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        if (t < 0) {   // closing pass: gradient wrt h0; dc0 is the running dc
+            if (live) {
+                *reinterpret_cast<floatx2*>(p.dH0 + size_t(b0) * p.Hp + cell) = floatx2{dh[0], dh[1]};
+                *reinterpret_cast<floatx2*>(p.dC + size_t(b0) * p.Hp + cell) = floatx2{dc[0], dc[1]};
+            }
+            return;
+        }
+        half_t* const xout = p.X + size_t((t + 8) & 3) * p.x_slot + size_t(g) * tile_halfs;    // dG_t for the peers
+        half_t* const xnext = p.X + size_t((t + 6) & 3) * p.x_slot + size_t(g) * tile_halfs;   // will take dG_{t-2}
+        // (both waves' products are complete: every peer has delivered dG_{t+1}, i.e. is done reading dG_{t+2})
+        store_xch16(xnext + off_ring, uintx4{kUnwritten, kUnwritten, kUnwritten, kUnwritten}, false);
+        float da[4][2], dy[2];
+        unpack_h2(dy2[par], dy[0], dy[1]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            float ig, fg, gg, og;
+            unpack_h2(u == 0 ? gates[par].x : gates[par].z, ig, fg);
+            unpack_h2(u == 0 ? gates[par].y : gates[par].w, gg, og);
+            const float dhu = dh[u] + S * dy[u];
+            const float tc = tanhf_dev(ccur[par][u]);
+            const float dov = dhu * tc;
+            const float d = dc[u] + dhu * og * (1.f - tc * tc);
+            da[0][u] = d * gg * ig * (1.f - ig);
+            da[1][u] = d * cprev[par][u] * fg * (1.f - fg);
+            da[2][u] = d * ig * (1.f - gg * gg);
+            da[3][u] = dov * og * (1.f - og);
+            dc[u] = d * fg;
+        }
+        GateRow<2> out = live ? pack_gates<2>(da) : gates_fill<2>(0u);   // batch rows past B travel as zeros
+        store_xch16(xout + off_ring, out.v[0], false);
+        clk.lap(2);
+        if (live) {
+            float v[4][2];   // db sums the values the weight-gradient GEMMs will see (fp16-rounded)
+            unpack_gates<2>(out, v);
+#pragma unroll
+            for (int gt = 0; gt < 4; ++gt)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) dbacc[gt][u] += v[gt][u];
+            st_gates<2>(p.dG + (size_t(t) * p.B + b0) * gld + 4u * cell, out);
+        }
+        clk.lap(3);
+    };
+    auto step = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        float dh[2];
+        const half_t* tile = wave_uniform(p.X + size_t((t + 9) & 3) * p.x_slot + size_t(g) * tile_halfs);   // dG_{t+1}
+        half8 f[KS];
+        auto request = [&]() __attribute__((always_inline)) { request_pair(f, tile, lane_off, tail_off, std::make_integer_sequence<int, KS>{}); };
+        request();
+        request_ops(t - 1, std::integral_constant<int, 1 - par>{});
+        wait_set<4>(f);
+        auto unwritten = [&]() -> bool {
+            unsigned m = 0u;
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const uint4 ua = __builtin_bit_cast(uint4, f[k]);
+                m = max(m, max(max(ua.x, ua.y), max(ua.z, ua.w)));
+            }
+            return __any(m == kUnwritten) != 0;
+        };
+        if (__builtin_expect(unwritten() && poll.on, 0)) {
+            int spins = 0;
+            long long spin_start = 0;
+            do {
+                if (poll_give_up(poll, spins, spin_start, lane)) break;   // (the workgroup leaves at its barrier)
+                request();
+                wait_set<0>(f);
+            } while (unwritten());
+        }
+        floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) acc[k % 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[k], f[k], acc[k % 2], 0, 0, 0);
+        const floatx4 sum = acc[0] + acc[1];
+        clk.lap(0);
+        swap[par][1 - wave][lane] = wave ? floatx2{sum.x, sum.y} : floatx2{sum.z, sum.w};
+        __syncthreads();
+        if (lds_abort != 0) leave_kernel();
+        const floatx2 other = swap[par][wave][lane];
+        dh[0] = (wave ? sum.z : sum.x) + other.x;
+        dh[1] = (wave ? sum.w : sum.y) + other.y;
+        clk.lap(1);
+        settle_ops(parity);
+        cell_update(t, dh, parity);
+    };
+    int t = t_first;
+    if (t >= p.T - 1) {   // the last step of the sequence: dh comes from the caller
+        const float* src = p.dHn + size_t(b0) * p.Hp + cell;
+        const float dh[2] = {src[0], src[1]};
+        request_ops(t, std::integral_constant<int, 0>{});
+        wait_all_vm();
+        settle_ops(std::integral_constant<int, 0>{});
+        cell_update(t, dh, std::integral_constant<int, 0>{});
+        --t;
+    }
+    request_ops(t, std::integral_constant<int, 0>{});
+    for (; t - 1 >= t_last; t -= 2) {
+        step(t, std::integral_constant<int, 0>{});
+        step(t - 1, std::integral_constant<int, 1>{});
+    }
+    if (t >= t_last) step(t, std::integral_constant<int, 0>{});
+    wait_all_vm();
+    settle_ops(std::integral_constant<int, 0>{});   // (the last request is used by nobody, but its registers must not be handed on before it has landed)
+    settle_ops(std::integral_constant<int, 1>{});
+    if (t_last >= 0 && live) *reinterpret_cast<floatx2*>(p.dC + size_t(b0) * p.Hp + cell) = floatx2{dc[0], dc[1]};   // for the next launch
+    if (p.stamp_end && hs == 0 && g == 0 && tid == 0) *p.stamp_end = wall_clock64();
+    clk.flush();
+    // Bias gradient: fold this launch's sums over the 16 rows (fixed order).
+#pragma unroll
+    for (int gt = 0; gt < 4; ++gt)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) red[tid][gt * 2 + u] = dbacc[gt][u];
+    __syncthreads();
+    if (tid < 64) {
+        const int unit = tid / 4, gt = tid % 4;   // of the slice: lane group unit / 4, wave (unit % 4) / 2
+        float sum = 0.f;
+        for (int k = 0; k < 16; ++k) sum += red[((unit % 4) / 2) * kWave + (unit / 4) * 16 + k][gt * 2 + unit % 2];
+        p.db_part[size_t(g) * gld + size_t(4) * (hs * 16 + unit) + gt] += sum;
+    }
+}
+
 // --------------------------------------------------------------- backward, two-dimensional split
 // For 2048 hidden units the product dG_{t+1} * W_hh^T has 32 MiB of weights.  The kernel above gives a workgroup 16
 // output columns and the whole contraction (8192 packed gate columns), so every workgroup pulls all of dG_{t+1}
@@ -2739,8 +3139,13 @@ void persistent_stream_idle(hipStream_t stream) {
 size_t exchange_slot_halfs(int rows, int cols) { return round_up(size_t(rows), 32) * size_t(cols); }
 
 int rec_fwd_ks(const RecLayout& L, int Hp) {
+    if (L.split) return Hp <= 64 ? 2 : int(round_up(size_t(Hp) / 32, 4));   // (every wave takes the whole contraction)
     const size_t ks = ceil_div(size_t(Hp) / 32, size_t(L.nw));
     return int(L.resident && Hp > 2048 ? round_up(ks, 4) : ks);   // (the wide kernels are built for whole groups of four)
+}
+size_t rec_fwd_fragments(const RecLayout& L, int Hp) {
+    if (L.split) return size_t(Hp) / 8 * rec_fwd_ks(L, Hp) * 2;
+    return size_t(L.nh) * L.nw * rec_fwd_ks(L, Hp) * L.nt;
 }
 int rec_bwd_ks(const RecLayout& L, int Hp) { return int(ceil_div(size_t(Hp) / 8, size_t(L.nw))); }
 
@@ -2762,15 +3167,27 @@ int rec_waves(int B, int Hp, int num_cus, int waves) {
 
 constexpr int kWideMost = 4096;   // hidden units whose W_hh the chip can hold (rec_fwd_wide_kernel)
 
+// Short contractions.  Every wave of rec_fwd_split_kernel fetches the whole operand, so the CU's vector-memory path sets
+// its end: with one or two waves per CU it is the faster kernel up to 512 units (64 rows 1.64 -> 1.34 us per step, 100 rows
+// 1.42), with four up to 256 (200 rows 1.44 -> 1.16; at 288 units equal, at 512 units 1.7 -> 2.3).  rec_bwd_pair_kernel is
+// the faster one up to 384 units (2.13 -> 1.93); at 512 its two waves take as long over the product as the other kernel's
+// four over theirs and its reduction (2.14 -> 2.24).
+constexpr int kFwdSplitMost = 512, kFwdSplitFourMost = 256, kBwdPairMost = 384;
+
+// whether all 16-row blocks of the batch can run side by side
+static bool can_16_rows(int B, int nh, int num_cus) {
+    const bool xcd_mode = (num_cus == 256 && nh <= 32);
+    const int side_by_side = nh > num_cus ? 0 : (xcd_mode ? 8 * (32 / nh) : num_cus / nh);
+    return int(ceil_div(size_t(B), 16)) <= side_by_side;
+}
+
 static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_stepwise, bool fits, int force_mt) {
     L.nh = Hp / L.jb;
     L.resident = fits ? 1 : 0;
     L.rot_div = 0;   // no k-step rotation (plan_rec_bwd turns it on where it pays)
     // Row blocks of 16 rows (one MFMA row tile) when all of them can run side by side: twice the workgroups
     // of 32-row blocks, each with half the product, fetch and cell-update work per step.
-    const bool xcd_mode = (num_cus == 256 && L.nh <= 32);
-    const int side_by_side = L.nh > num_cus ? 0 : (xcd_mode ? 8 * (32 / L.nh) : num_cus / L.nh);
-    const bool can_16 = fits && int(ceil_div(size_t(B), 16)) <= side_by_side;
+    const bool can_16 = fits && can_16_rows(B, L.nh, num_cus);
     L.mt = can_16 ? 1 : 2;
     if (force_mt == 2 || (force_mt == 1 && can_16)) L.mt = force_mt;   // a tuned choice; 16-row blocks only where they fit
     if (fits && Hp > 2048) L.mt = 1;   // the kernels for more than 2048 units take 16-row tiles one after the other
@@ -2809,6 +3226,17 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.unit_major = L.nw == 8 || (fits && Hp > 2048);
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
     L.wide = fits && Hp > 2048;
+    // short contractions: columns split over the waves, where every group has one 16-row block
+    if (L.nw == 4 && Hp <= kFwdSplitMost && num_cus == 256) {
+        for (int per_wg : {1, 2, 4}) {
+            if (per_wg == 4 && Hp > kFwdSplitFourMost) break;
+            if (Hp / (8 * per_wg) > 32 || !can_16_rows(B, Hp / (8 * per_wg), num_cus)) continue;
+            L.split = per_wg;
+            L.jb = 8 * per_wg;
+            finish_layout(L, B, Hp, num_cus, force_stepwise, fits, 1);
+            break;
+        }
+    }
     return L;
 }
 
@@ -2822,6 +3250,15 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.nw = 4;
     L.jb = 16 * L.nt;
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
+    // short contractions: two waves and 16 units per workgroup, where every group has one 16-row block
+    if (Hp <= kBwdPairMost && num_cus == 256 && can_16_rows(B, Hp / 16, num_cus)) {
+        L.split = 2;
+        L.nt = 1;
+        L.nw = 2;
+        L.jb = 16;
+        finish_layout(L, B, Hp, num_cus, force_stepwise, fits, 1);
+        return L;
+    }
     // k-step rotation (recurrent.h): measured, it pays where a group spans the XCDs and a step fetches a lot -- the
     // backward pass at 2048 hidden units, 13.4 -> 12.4 us per step at 128 rows -- and costs a little where the
     // workgroups of an XCD read the same lines in step out of their own L2 (5.33 -> 5.42 us at 1024 units, where
@@ -3030,6 +3467,31 @@ static hipError_t run_fwd_il(const RecLayout& L, const RecFwdArgs& a, hipStream_
                         });
 }
 
+// (next to no LDS in use, but one workgroup per CU: two would share the vector-memory path)
+constexpr size_t kWholeCuLds = size_t(96) << 10;
+
+template <int KS>
+static hipError_t run_fwd_split(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
+    auto kernel = rec_fwd_split_kernel<KS>;
+    const int threads = L.split * kWave;
+    if (L.mt != 1 || !L.resident || L.nrb > L.ng || L.jb != 8 * L.split || rec_fwd_ks(L, a.Hp) != KS || (L.persistent && !L.xcd_local))
+        return hipErrorInvalidValue;
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, kWholeCuLds, kThreads, per_cu, &device);
+    if (e != hipSuccess) return e;
+    if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), kWholeCuLds, stream, a, L, a.t0, a.t1, 0, per_cu[device].load(), device, threads);
+    return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
+                        [&]() -> hipError_t {
+                            for (int t = a.t0; t < a.t1; ++t) {
+                                hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(threads), kWholeCuLds, stream, a, L, t, t + 1, 0);
+                                hipError_t le = hipGetLastError();
+                                if (le != hipSuccess) return le;
+                            }
+                            return hipSuccess;
+                        });
+}
+
 template <int KS, int KL, int NBUF>
 static hipError_t run_fwd_wide(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     constexpr int NW = 4;
@@ -3075,6 +3537,14 @@ hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
         if (ks == 24) return run_fwd_wide<24, 6, 8>(L, a, stream, graphs);
         if (ks == 28) return run_fwd_wide<28, 7, 7>(L, a, stream, graphs);
         return run_fwd_wide<32, 8, 5>(L, a, stream, graphs);
+    }
+    if (L.split) {
+        switch (ks) {
+#define FLSTM_SPLIT_CASE(n) case n: return run_fwd_split<n>(L, a, stream, graphs);
+            FLSTM_SPLIT_CASE(2) FLSTM_SPLIT_CASE(4) FLSTM_SPLIT_CASE(8) FLSTM_SPLIT_CASE(12) FLSTM_SPLIT_CASE(16)
+#undef FLSTM_SPLIT_CASE
+        }
+        return hipErrorInvalidValue;
     }
     if (L.nw == 8) {   // eight waves: the interleaved kernel, 32-row blocks
         if (ks <= 2) return ds ? run_fwd_il<2, true>(L, a, stream, graphs) : run_fwd_il<2, false>(L, a, stream, graphs);
@@ -3145,6 +3615,27 @@ static hipError_t run_bwd2d(const RecLayout& L, const RecBwdArgs& a, hipStream_t
     return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
 }
 
+template <int KS>
+static hipError_t run_bwd_pair(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
+    auto kernel = rec_bwd_pair_kernel<KS>;
+    if (L.nt != 1 || L.nw != 2 || L.jb != 16 || L.mt != 1 || L.nrb > L.ng || a.Hp / 16 > KS || a.Hp / 16 < KS - 2 || (L.persistent && !L.xcd_local))
+        return hipErrorInvalidValue;
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, kWholeCuLds, 2 * kWave, per_cu, &device);
+    if (e != hipSuccess) return e;
+    if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), kWholeCuLds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device, 2 * kWave);
+    return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t_hi, a.t_lo, a.t_hi - a.t_lo + 1, stream,
+                        [&]() -> hipError_t {
+                            for (int t = a.t_hi; t >= a.t_lo; --t) {
+                                hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(2 * kWave), kWholeCuLds, stream, a, L, t, t, 0);
+                                hipError_t le = hipGetLastError();
+                                if (le != hipSuccess) return le;
+                            }
+                            return hipSuccess;
+                        });
+}
+
 template <int KS, int KL, int NBUF>
 static hipError_t run_bwd_wide(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream) {
     const size_t lds = size_t(wide_part_buffers(KL)) * 4 * 16 * (64 + kPartPad) * sizeof(float) + size_t(4) * KL * 4 * kWave * sizeof(half8);
@@ -3198,6 +3689,14 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
     }
     const bool ds = L.persistent && !L.xcd_local;   // (as in launch_rec_fwd)
     if (!L.resident) return run_bwd<2, 1, false, 0, 2, false>(L, a, stream, graphs);
+    if (L.split) {
+        switch ((a.Hp / 16 + 3) / 4) {
+#define FLSTM_PAIR_CASE(n) case n: return run_bwd_pair<4 * n>(L, a, stream, graphs);
+            FLSTM_PAIR_CASE(1) FLSTM_PAIR_CASE(2) FLSTM_PAIR_CASE(3) FLSTM_PAIR_CASE(4) FLSTM_PAIR_CASE(5) FLSTM_PAIR_CASE(6)
+#undef FLSTM_PAIR_CASE
+        }
+        return hipErrorInvalidValue;
+    }
     const int ks = rec_bwd_ks(L, a.Hp);
     if (L.nt == 2) {
         if (L.mt == 1) {

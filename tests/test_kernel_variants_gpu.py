@@ -30,3 +30,17 @@ def test_recurrence_kernels_for_wide_layers(B, H):
     got, info = run_core(p)
     assert info["fallbacks"] == 0 and info["persistent_fwd"] == 1
     check_against(ref, got, label=f"B={B} H={H}")
+
+
+# short contractions: the smallest layer, both sides of the lines (64 | 65, 256 | 257, 384 | 385, 512 | 513 units), batches
+# that take one, two and four waves per workgroup or just miss them, sequences of one, an odd and an even number of steps
+@pytest.mark.parametrize("T,B,H", [(1, 1, 8), (2, 16, 32), (7, 17, 64), (8, 3, 65), (3, 1030, 40), (6, 129, 256), (5, 257, 256),
+                                   (4, 513, 256), (9, 64, 257), (4, 130, 288), (5, 33, 384), (6, 130, 385), (4, 128, 512),
+                                   (3, 129, 500)])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_recurrence_kernels_for_short_contractions(T, B, H, stepwise):
+    p = make_problem(T, B, 20, H, seed=B * 10000 + H)
+    ref, _ = oracle_reference(p)
+    got, info = run_core(p, stepwise=stepwise)
+    assert info["fallbacks"] == 0
+    check_against(ref, got, label=f"T={T} B={B} H={H} stepwise={stepwise}")
