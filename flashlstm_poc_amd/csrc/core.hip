@@ -94,7 +94,6 @@ struct flstm_core_plan {
     int clock_khz = 0;   // maximum engine clock the runtime reports
     Dims d{};
     RecLayout Lf{}, Lb{};
-    int ks_f = 0, ks_b = 0;
     // options
     int opt_stepwise = 0, opt_spin_limit = 1 << 30, opt_spin_ms = 250, opt_dw_splits = 0, opt_accumulate = 0;
     // A persistent launch that gave up (its workgroups were not all running at once, or not spread over the XCDs
@@ -124,7 +123,7 @@ struct flstm_core_plan {
     int seat_sets_left = 0;              // zeroed sets of seat counters in the status block
     int inject_stall = 0;         // test hook: treat the next N passes as if their launches had given up
     // weights
-    DevBuf wih_p, wih_t, wfrag_f, wfrag_b, wfrag_b2, bias_p;
+    DevBuf wih_p, wih_t, wfrag[kFragKinds], bias_p;
     bool weights_packed = false, bias_packed = false;
     // forward state / caches
     DevBuf X16, G, Y, C, status, xch_f, xch_b;
@@ -158,8 +157,6 @@ void replan(flstm_core_plan* p) {
                          p->opt_mt_b ? p->opt_mt_b : p->eff_mt_b,
                          (!p->two_d_explicit && p->eff_two_d >= 0) ? p->eff_two_d : p->opt_two_d);
     p->Lf.cooperative = p->Lb.cooperative = p->opt_cooperative;
-    p->ks_f = rec_fwd_ks(p->Lf, p->d.Hp);
-    p->ks_b = rec_bwd_ks(p->Lb, p->d.Hp);
 }
 
 // Puts the tuned entry for sequence length T in force: the entry tuned at exactly T, else the nearest one within a
@@ -304,7 +301,8 @@ extern "C" int flstm_core_create(size_t batch, size_t input_size, size_t hidden_
 
 extern "C" int flstm_core_destroy(flstm_core_plan* p) {
     if (!p) return FLSTM_E_INVALID;
-    for (DevBuf* b : {&p->wih_p, &p->wih_t, &p->wfrag_f, &p->wfrag_b, &p->wfrag_b2, &p->part_b, &p->bias_p, &p->X16, &p->G, &p->Y, &p->C,
+    for (DevBuf& b : p->wfrag) b.release();
+    for (DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->X16, &p->G, &p->Y, &p->C,
                       &p->status, &p->xch_f, &p->xch_b, &p->dYp, &p->dG, &p->dHn, &p->dC,
                       &p->dH0, &p->db_part, &p->dw_part, &p->prof})
         b->release();
@@ -340,10 +338,10 @@ extern "C" int flstm_core_set_option(flstm_core_plan* p, const char* name, long 
         // wavefronts per workgroup of the forward recurrence: the weight fragments are packed for it, so a change
         // un-packs them
         if (value != 0 && value != 4 && value != 8) return FLSTM_E_INVALID;
-        const int before = p->Lf.nw, split_before = p->Lf.split;
+        const int before = p->Lf.nw;
         p->opt_waves_f = int(value);
         replan(p);
-        if (p->Lf.nw != before || p->Lf.split != split_before) p->weights_packed = false;
+        if (p->Lf.nw != before) p->weights_packed = false;
         return 0;
     }
     if (!strcmp(name, "inject_stall")) { if (value < 0) return FLSTM_E_INVALID; p->inject_stall = int(value); return 0; }
@@ -379,7 +377,8 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
     if (!strcmp(name, "tuned_bwd_two_d")) return p->eff_two_d;
     if (!strcmp(name, "device_bytes")) {
         size_t sum = 0;
-        for (const DevBuf* b : {&p->wih_p, &p->wih_t, &p->wfrag_f, &p->wfrag_b, &p->wfrag_b2, &p->part_b, &p->bias_p, &p->X16, &p->G, &p->Y, &p->C,
+        for (const DevBuf& b : p->wfrag) sum += b.bytes;
+        for (const DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->X16, &p->G, &p->Y, &p->C,
                                 &p->status, &p->xch_f, &p->xch_b, &p->dYp, &p->dG, &p->dHn, &p->dC, &p->dH0, &p->db_part,
                                 &p->dw_part, &p->prof})
             sum += b->bytes;
@@ -415,23 +414,37 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     const Dims& d = p->d;
     FL_TRY(p->wih_p.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
     FL_TRY(p->wih_t.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
-    FL_TRY(p->wfrag_f.reserve(rec_fwd_fragments(p->Lf, d.Hp) * kWave * sizeof(half8)));
-    FL_TRY(p->wfrag_b.reserve(size_t(p->Lb.nh) * p->Lb.nw * p->ks_b * p->Lb.nt * kWave * sizeof(half8)));
-    auto layout = [](const DevBuf& out, const RecLayout& L, int ks) {
-        FragLayout f;
-        f.out = out.as<half8>(); f.ks = ks; f.nt = L.nt; f.rot_div = L.rot_div; f.nw = L.nw; f.unit_major = L.unit_major;
-        return f;
+    // Fragments for every kernel that the options can choose for these sizes, whichever the current ones do: options and
+    // tuned entries change after the weights are packed.  (The one-way kernels have theirs wherever 32-row blocks can be
+    // asked for; those for short contractions, up to 512 units, add at most 2 MiB a direction.)
+    FragLayout frag[kFragKinds];
+    auto want = [&](int kind, const RecLayout& L, int ks, size_t fragments) -> hipError_t {
+        FragLayout& f = frag[kind];
+        const hipError_t e = p->wfrag[kind].reserve(fragments * kWave * sizeof(half8));
+        f.out = p->wfrag[kind].as<half8>(); f.fragments = fragments; f.ks = ks;
+        f.nt = L.nt; f.rot_div = L.rot_div; f.nw = L.nw; f.unit_major = L.unit_major;
+        return e;
     };
-    FragLayout fwd = layout(p->wfrag_f, p->Lf, p->ks_f), bwd = layout(p->wfrag_b, p->Lb, p->ks_b), two_d;
-    fwd.wide = p->Lf.wide; fwd.split = p->Lf.split; fwd.fragments = rec_fwd_fragments(p->Lf, d.Hp);
-    if (rec_bwd_two_d_possible(d.Hp, p->num_cus)) {   // whether or not the current layout uses them
-        FL_TRY(p->wfrag_b2.reserve(rec_bwd_two_d_wfrag_bytes(d.Hp)));
-        two_d.out = p->wfrag_b2.as<half8>();
-        two_d.kq = rec_bwd_two_d_kq(d.B, d.Hp);
-        two_d.wide = d.Hp > 2048;
-        two_d.ks = two_d.wide ? rec_wide_ks(d.Hp) : d.Hp / (32 * two_d.kq);
+    const RecLayout fwd = plan_rec_fwd(d.B, d.Hp, p->num_cus, false, 2, p->opt_waves_f), split = plan_rec_fwd(d.B, d.Hp, p->num_cus, false);
+    const RecLayout bwd = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 2, 0), pair = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 0, 0);
+    FL_TRY(want(kFragFwd, fwd, rec_fwd_ks(fwd, d.Hp), rec_fwd_fragments(fwd, d.Hp)));
+    frag[kFragFwd].wide = fwd.wide;
+    if (split.split) {
+        FL_TRY(want(kFragFwdSplit, split, rec_fwd_ks(split, d.Hp), rec_fwd_fragments(split, d.Hp)));
+        frag[kFragFwdSplit].split = split.split;
     }
-    FL_TRY(pack_weights(d, w_ih, w_hh, p->wih_p.as<half_t>(), p->wih_t.as<half_t>(), fwd, bwd, two_d, s));
+    FL_TRY(want(kFragBwd, bwd, rec_bwd_ks(bwd, d.Hp), rec_bwd_fragments(bwd, d.Hp)));
+    if (pair.split) FL_TRY(want(kFragBwdPair, pair, rec_bwd_ks(pair, d.Hp), rec_bwd_fragments(pair, d.Hp)));
+    if (rec_bwd_two_d_possible(d.Hp, p->num_cus)) {
+        FragLayout& f = frag[kFragBwdTwoD];
+        f.kq = rec_bwd_two_d_kq(d.B, d.Hp);
+        f.wide = d.Hp > 2048;
+        f.ks = f.wide ? rec_wide_ks(d.Hp) : d.Hp / (32 * f.kq);
+        f.fragments = size_t(d.Hp / 64) * f.kq * 4 * f.ks * 4;
+        FL_TRY(p->wfrag[kFragBwdTwoD].reserve(f.fragments * kWave * sizeof(half8)));
+        f.out = p->wfrag[kFragBwdTwoD].as<half8>();
+    }
+    FL_TRY(pack_weights(d, w_ih, w_hh, p->wih_p.as<half_t>(), p->wih_t.as<half_t>(), frag, s));
     p->weights_packed = true;
     return 0;
 }
@@ -539,7 +552,7 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     const Dims& d = p->d;
     RecFwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (padding too: the arguments are the key of a captured graph)
-    a.wfrag = p->wfrag_f.as<half8>();
+    a.wfrag = p->wfrag[p->Lf.split ? kFragFwdSplit : kFragFwd].as<half8>();
     a.Y = p->Y.as<half_t>(); a.G = p->G.as<half_t>(); a.C = p->C.as<float>();
     a.y_out = p->fw.y_direct;
     a.X = p->xch_f.as<half_t>(); a.x_slot = exchange_slot_halfs(d.B, d.Hp);
@@ -784,12 +797,12 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
     }
     RecBwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (as in forward_recur)
-    a.wfrag = p->wfrag_b.as<half8>();
+    a.wfrag = p->wfrag[p->Lb.split ? kFragBwdPair : kFragBwd].as<half8>();
     a.G = p->G.as<half_t>(); a.C = p->C.as<float>(); a.dY = p->bw.dYk; a.dG = p->dG.as<half_t>();
     a.dHn = p->dHn.as<float>(); a.dC = p->dC.as<float>(); a.dH0 = p->dH0.as<float>();
     a.X = p->xch_b.as<half_t>(); a.x_slot = exchange_slot_halfs(rec_bwd_ring_rows(p->Lb, d.B), 4 * d.Hp);
     if (p->Lb.two_d) {
-        a.wfrag2 = p->wfrag_b2.as<half8>();
+        a.wfrag2 = p->wfrag[kFragBwdTwoD].as<half8>();
         a.P = p->part_b.as<float>();
         a.p_slot = rec_bwd_part_slot_floats(p->Lb);
     }

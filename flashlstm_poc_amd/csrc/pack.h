@@ -16,15 +16,16 @@ struct Dims {
 // Replaces src/kernels.cu:57-84 (pack_weights_kernel) and :45-55 (combine_bias_kernel): fp32
 // PyTorch-layout weights -> the fp16 operand layouts of the kernels in this library.
 struct FragLayout {   // where a recurrence kernel expects its weight fragments: RecLayout's description of them
-    half8* out = nullptr;
+    half8* out = nullptr;   // (null: not wanted)
     int ks = 0, nt = 0, rot_div = 0, nw = 0, unit_major = 0, wide = 0, kq = 0, split = 0;
-    size_t fragments = 0;   // forward
+    size_t fragments = 0;   // of 64 lanes
 };
-// W_ih twice (as it is for the projection, transposed for dX) and W_hh as forward fragments, backward fragments and (two_d.out
-// set) those of the backward recurrence that splits its product two ways; one launch.
+// Forward: the one-way kernels' and those of the kernel for short contractions; backward the same; those of the backward
+// recurrence that splits its product two ways.
+enum Frag : int { kFragFwd, kFragFwdSplit, kFragBwd, kFragBwdPair, kFragBwdTwoD, kFragKinds };
+// W_ih twice (as it is for the projection, transposed for dX) and W_hh as every kind of fragments asked for; one launch.
 hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p /*[4Hp][Ip]*/,
-                        half_t* wih_t /*[Ip][4Hp]*/, const FragLayout& fwd, const FragLayout& bwd, const FragLayout& two_d,
-                        hipStream_t s);
+                        half_t* wih_t /*[Ip][4Hp]*/, const FragLayout (&frag)[kFragKinds], hipStream_t s);
 hipError_t pack_bias(const Dims& d, const float* b_ih, const float* b_hh, float* bias_p, hipStream_t s);
 
 // dst[r][c] (pitch ldc) = sum over z < splits of partial[z * per + r * cols + c]: split-K partials of a plain GEMM.

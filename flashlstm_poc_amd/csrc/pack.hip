@@ -27,8 +27,8 @@ struct PackJob {
     Dims d;
     const float *w_ih, *w_hh;
     half_t *wih_p, *wih_t;
-    FragLayout frag[3];     // forward, backward, two-way backward
-    unsigned first[6];
+    FragLayout frag[kFragKinds];
+    unsigned first[kFragKinds + 3];
 };
 
 __device__ __forceinline__ half8 frag_values_fwd(const Dims& d, const float* __restrict__ w_hh, const FragLayout& f, size_t item) {
@@ -141,10 +141,9 @@ __global__ __launch_bounds__(kT) void pack_kernel(PackJob job) {
         st_half8(job.wih_t + size_t(i) * 4 * d.Hp + q, v);
     } else {
         const FragLayout& f = job.frag[which - 2];
-        const size_t n = which == 2 ? f.fragments * kWave
-                       : which == 3 ? size_t(d.Hp / (16 * f.nt)) * f.nw * f.ks * f.nt * kWave : size_t(d.Hp / 64) * f.kq * 4 * f.ks * 4 * kWave;
-        if (item >= n) return;
-        f.out[item] = which == 2 ? frag_values_fwd(d, job.w_hh, f, item) : which == 3 ? frag_values_bwd(d, job.w_hh, f, item) : frag_values_two_d(d, job.w_hh, f, item);
+        if (item >= f.fragments * kWave) return;
+        const int kind = which - 2;
+        f.out[item] = kind <= kFragFwdSplit ? frag_values_fwd(d, job.w_hh, f, item) : kind <= kFragBwdPair ? frag_values_bwd(d, job.w_hh, f, item) : frag_values_two_d(d, job.w_hh, f, item);
     }
 }
 
@@ -288,22 +287,22 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
 
 }  // namespace
 
-hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p, half_t* wih_t, const FragLayout& fwd,
-                        const FragLayout& bwd, const FragLayout& two_d, hipStream_t s) {
+hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p, half_t* wih_t,
+                        const FragLayout (&frag)[kFragKinds], hipStream_t s) {
     PackJob job{};
     job.d = d;
     job.w_ih = w_ih; job.w_hh = w_hh; job.wih_p = wih_p; job.wih_t = wih_t;
-    job.frag[0] = fwd; job.frag[1] = bwd; job.frag[2] = two_d;
     // (Hp is a multiple of 32 and Ip of 64: whole chunks of eight, and of four chunks, everywhere)
-    const size_t items[5] = {size_t(4) * d.Hp * d.Ip / 8, size_t(4) * d.Hp * d.Ip / 8,
-                             fwd.fragments * kWave,
-                             size_t(d.Hp / (16 * bwd.nt)) * bwd.nw * bwd.ks * bwd.nt * kWave,
-                             two_d.out ? size_t(d.Hp / 64) * two_d.kq * 4 * two_d.ks * 4 * kWave : 0};
-    for (int i = 0; i < 5; ++i) {
-        if (items[i] >> 32) return hipErrorInvalidValue;
-        job.first[i + 1] = job.first[i] + unsigned(ceil_div(items[i], kT));
+    for (int i = 0; i < kFragKinds + 2; ++i) {
+        size_t items = size_t(4) * d.Hp * d.Ip / 8;
+        if (i >= 2) {
+            job.frag[i - 2] = frag[i - 2];
+            items = frag[i - 2].out ? frag[i - 2].fragments * kWave : 0;
+        }
+        if (items >> 32) return hipErrorInvalidValue;
+        job.first[i + 1] = job.first[i] + unsigned(ceil_div(items, kT));
     }
-    hipLaunchKernelGGL(pack_kernel, dim3(job.first[5]), dim3(kT), 0, s, job);
+    hipLaunchKernelGGL(pack_kernel, dim3(job.first[kFragKinds + 2]), dim3(kT), 0, s, job);
     return hipGetLastError();
 }
 

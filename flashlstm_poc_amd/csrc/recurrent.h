@@ -170,7 +170,9 @@ constexpr size_t kGraphCacheEntries = 4;
 
 // Picks tile shapes and the group structure for a problem size on the current device.  force_mt: 0 = the rule of
 // thumb (16-row blocks whenever all of them can run side by side), 1 / 2 = that many 16-row tiles per row block
-// (1 only where it fits).  The choice does not change the weight-fragment layout.
+// (1 only where it fits; above 2048 units tiles of 16 rows are taken one after the other whatever it says).  2 is always
+// a one-way kernel: those for short contractions (RecLayout::split) have 16-row blocks.  Each of the two families has its
+// own weight fragments, which depend on the sizes alone (and, one-way forward, on `waves`).
 // waves: 0 = the rule of thumb (rec_waves), 4 or 8 = that many wavefronts per workgroup (8 only up to 1024 units).
 RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt = 0, int waves = 0);
 // two_d: 0 = never the two-way split, 1 = where it is the faster layout, 2 = wherever it can run
@@ -180,14 +182,12 @@ int rec_waves(int B, int Hp, int num_cus, int waves);
 
 // The two-dimensional backward layout: whether a device/size can use it at all (decides whether its weight fragments
 // are packed) and with how many contraction slices (a function of the sizes alone, so that the packed weights fit
-// whatever the options say later), slots of its dG ring, floats per slot of its partial ring and bytes of its weight
-// fragments.
+// whatever the options say later), slots of its dG ring, floats per slot of its partial ring.
 bool rec_bwd_two_d_possible(int Hp, int num_cus);
 int rec_bwd_two_d_kq(int B, int Hp);
 int rec_bwd_dg_slots(const RecLayout& L);
 size_t rec_bwd_part_slot_floats(const RecLayout& L);
 constexpr int kRecBwdPartSlots = 3;
-size_t rec_bwd_two_d_wfrag_bytes(int Hp);
 // Word to fill slot `slot` of the partial ring with before a pass over T steps (see RecBwdArgs::P).
 unsigned rec_bwd_part_fill(int slot, int T);
 // Batch rows the rings of a backward layout are sized for (whole windows where the batch is walked in windows).
@@ -195,8 +195,9 @@ int rec_bwd_ring_rows(const RecLayout& L, int B);
 
 // Halfs in one slot of an exchange ring for a [rows][cols] operand (rows padded to 32).
 size_t exchange_slot_halfs(int rows, int cols);
-// Fragments (64 lanes of 16 bytes) of a forward layout.
+// Fragments (64 lanes of 16 bytes) of a layout.
 size_t rec_fwd_fragments(const RecLayout& L, int Hp);
+size_t rec_bwd_fragments(const RecLayout& L, int Hp);   // (the one-way kernels' and the pair kernel's)
 // Number of k-steps (32 wide) every wave holds for a layout (sizes the fragment arrays).
 int rec_fwd_ks(const RecLayout& L, int Hp);
 int rec_bwd_ks(const RecLayout& L, int Hp);

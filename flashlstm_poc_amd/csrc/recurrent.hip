@@ -3147,6 +3147,7 @@ size_t rec_fwd_fragments(const RecLayout& L, int Hp) {
     if (L.split) return size_t(Hp) / 8 * rec_fwd_ks(L, Hp) * 2;
     return size_t(L.nh) * L.nw * rec_fwd_ks(L, Hp) * L.nt;
 }
+size_t rec_bwd_fragments(const RecLayout& L, int Hp) { return size_t(Hp / (16 * L.nt)) * L.nw * rec_bwd_ks(L, Hp) * L.nt; }
 int rec_bwd_ks(const RecLayout& L, int Hp) { return int(ceil_div(size_t(Hp) / 8, size_t(L.nw))); }
 
 // Wavefronts per workgroup of the forward recurrence: eight (rec_fwd_il_kernel: the two row tiles of a 32-row block
@@ -3226,8 +3227,8 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.unit_major = L.nw == 8 || (fits && Hp > 2048);
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
     L.wide = fits && Hp > 2048;
-    // short contractions: columns split over the waves, where every group has one 16-row block
-    if (L.nw == 4 && Hp <= kFwdSplitMost && num_cus == 256) {
+    // short contractions: columns split over the waves, where every group has one 16-row block (and 32-row blocks are not asked for)
+    if (L.nw == 4 && force_mt != 2 && Hp <= kFwdSplitMost && num_cus == 256) {
         for (int per_wg : {1, 2, 4}) {
             if (per_wg == 4 && Hp > kFwdSplitFourMost) break;
             if (Hp / (8 * per_wg) > 32 || !can_16_rows(B, Hp / (8 * per_wg), num_cus)) continue;
@@ -3250,8 +3251,8 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.nw = 4;
     L.jb = 16 * L.nt;
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
-    // short contractions: two waves and 16 units per workgroup, where every group has one 16-row block
-    if (Hp <= kBwdPairMost && num_cus == 256 && can_16_rows(B, Hp / 16, num_cus)) {
+    // short contractions: two waves and 16 units per workgroup, where every group has one 16-row block (as forward)
+    if (force_mt != 2 && Hp <= kBwdPairMost && num_cus == 256 && can_16_rows(B, Hp / 16, num_cus)) {
         L.split = 2;
         L.nt = 1;
         L.nw = 2;
@@ -3328,10 +3329,6 @@ int rec_bwd_dg_slots(const RecLayout& L) { return L.two_d ? kDgSlots : 4; }
 size_t rec_bwd_part_slot_floats(const RecLayout& L) {
     // [256 workgroups][nm passes][kq senders][rows][64 / kq columns]
     return L.two_d ? size_t(256) * L.nm * 64 * (16 * L.mt) : 0;
-}
-size_t rec_bwd_two_d_wfrag_bytes(int Hp) {
-    if (Hp > 2048) return size_t(Hp / 64) * 4 * 4 * rec_wide_ks(Hp) * 4 * kWave * sizeof(half8);
-    return size_t(Hp) * 4 * Hp * sizeof(half_t);
 }
 int rec_bwd_ring_rows(const RecLayout& L, int B) {
     return (L.two_d && L.win_rows) ? int(ceil_div(size_t(B), size_t(L.win_rows))) * L.win_rows : B;

@@ -47,7 +47,10 @@ int flstm_core_destroy(flstm_core_plan* plan);
  * the weight-gradient GEMM, 0 = automatic), "accumulate_grads" (1 = the backward pass adds dW_ih, dW_hh, db_ih
  * and db_hh to what the caller's buffers hold instead of overwriting them: a sequence processed as several
  * consecutive segments, last segment first, each segment's dh0 / dc0 fed to the next call as d_hn / d_cn),
- * "row_tiles_fwd" / "row_tiles_bwd" (16-row tiles per row block of that recurrence: 1, 2, or 0 = automatic),
+ * "row_tiles_fwd" / "row_tiles_bwd" (16-row tiles per row block of that recurrence: 1, 2, or 0 = automatic; 1 only where
+ * all 16-row blocks run side by side.  The kernels for short contractions, up to 512 units forward and 384 backward, have
+ * 16-row blocks: there 2 chooses the kernel of larger layers, whose sums are in another order.  Above 2048 units batch
+ * rows are taken in tiles of 16, one after the other, and the option changes nothing),
  * "cooperative" (0, the default: persistent launches are plain launches whose grid is checked to be co-resident, and
  * launches to different streams of a device are put one behind the other; 1: hipLaunchCooperativeKernel, which costs
  * 20 us more per launch -- and a process that made a cooperative launch faults inside an attached rocprofiler-sdk tool
@@ -67,8 +70,8 @@ int flstm_core_set_option(flstm_core_plan* plan, const char* name, long value);
  * "fallbacks" (persistent launches that had to be redone step-wise), "demotions_fwd", "demotions_bwd" (how often a
  * direction was demoted to step-wise launches after such a give-up), "hold_fwd", "hold_bwd" (passes a demoted
  * direction still runs step-wise before the persistent kernel is tried again; 0 = not demoted), "slice_fwd", "slice_bwd" (hidden units
- * per workgroup of the recurrence kernels), "row_tiles" (16-row tiles of a 32-row batch block that the
- * recurrence fetches and multiplies: 1 for batches of at most 16 rows, else 2), "hidden_padded",
+ * per workgroup of the recurrence kernels), "row_tiles_fwd", "row_tiles_bwd" (16-row tiles per row block that the
+ * recurrences run with; "row_tiles": the forward one), "hidden_padded",
  * "input_padded", "device_bytes" (device memory the plan holds), "static_scratch_bytes" (size of the fixed scratch
  * array of flstm_core_forward_static), "num_cus" and "clock_khz" (compute units and
  * maximum engine clock of the plan's device).

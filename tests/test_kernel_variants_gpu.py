@@ -44,3 +44,35 @@ def test_recurrence_kernels_for_short_contractions(T, B, H, stepwise):
     got, info = run_core(p, stepwise=stepwise)
     assert info["fallbacks"] == 0
     check_against(ref, got, label=f"T={T} B={B} H={H} stepwise={stepwise}")
+
+
+# 32-row blocks asked for where the rule takes the kernels for short contractions, which have 16-row blocks: the option and
+# a tuned entry are both honoured, after the weights were packed, and taken back without packing again.  One and several row
+# blocks, a partial one, a hidden size per kernel family: both short kernels (256), the forward one alone (385, 512)
+@pytest.mark.parametrize("T,B,H", [(6, 3, 40), (5, 33, 256), (4, 130, 288), (5, 17, 385), (4, 40, 512)])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_row_tile_choice_where_short_contraction_kernels_are_the_rule(T, B, H, stepwise):
+    import numpy as np
+    from flashlstm_poc_amd import LstmCore
+    p = make_problem(T, B, 20, H, seed=B * 10000 + H)
+    ref, _ = oracle_reference(p)
+    core = LstmCore(B, 20, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    by_rule, info = run_core(p, core=core, stepwise=stepwise)
+    assert info["fallbacks"] == 0 and core.info("row_tiles_fwd") == 1
+    for name in ("row_tiles_fwd", "row_tiles_bwd"):
+        core.set_option(name, 2)
+    got, info = run_core(p, core=core, stepwise=stepwise)
+    assert info["fallbacks"] == 0 and core.info("row_tiles_fwd") == 2 and core.info("row_tiles_bwd") == 2
+    check_against(ref, got, label=f"T={T} B={B} H={H} stepwise={stepwise} 32-row blocks")
+    for name in ("row_tiles_fwd", "row_tiles_bwd"):
+        core.set_option(name, 0)
+    assert core.lib.flstm_core_set_tuned(core._h, T, 2, 2, int(stepwise), int(stepwise), 0, -1) == 0
+    tuned, _ = run_core(p, core=core, stepwise=stepwise)
+    assert core.info("row_tiles_fwd") == 2 and core.info("row_tiles_bwd") == 2
+    core.set_option("clear_tuned", 1)
+    again, _ = run_core(p, core=core, stepwise=stepwise)
+    assert core.info("row_tiles_fwd") == 1
+    for k in by_rule:   # the same kernels on the same fragments: the same bits
+        assert np.array_equal(tuned[k], got[k]) and np.array_equal(again[k], by_rule[k]), k
+    core.close()
