@@ -765,7 +765,7 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
         const size_t pslot = rec_bwd_part_slot_floats(p->Lb) * sizeof(float);
         FL_TRY(p->part_b.reserve(kRecBwdPartSlots * pslot));
         for (int i = 0; i < kRecBwdPartSlots; ++i)
-            prep.fill(static_cast<char*>(p->part_b.p) + size_t(i) * pslot, pslot, rec_bwd_part_fill(i, int(T)));
+            prep.fill(static_cast<char*>(p->part_b.p) + size_t(i) * pslot, pslot, rec_bwd_part_fill(p->Lb, i, int(T)));
     }
     prep.to_float(d_hn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, k.state, p->dHn.as<float>(), size_t(d.Hp));
     prep.to_float(d_cn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, k.state, p->dC.as<float>(), size_t(d.Hp));
@@ -829,7 +829,7 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
             const size_t pslot = a.p_slot * sizeof(float);
             const int first_T = t_hi >= long(p->bw.T) - 1 ? int(p->bw.T) : int(t_hi) + 2;   // (its first product step is first_T - 2)
             for (int k = 0; k < kRecBwdPartSlots; ++k)
-                FL_TRY(fill_words(static_cast<char*>(p->part_b.p) + size_t(k) * pslot, pslot, rec_bwd_part_fill(k, first_T), s));
+                FL_TRY(fill_words(static_cast<char*>(p->part_b.p) + size_t(k) * pslot, pslot, rec_bwd_part_fill(p->Lb, k, first_T), s));
         }
         const bool whole = (t_hi == long(p->bw.T) - 1 && t_lo == -1);   // (graphs for whole passes only: see forward_recur)
         hipError_t e = launch_rec_bwd(p->Lb, a, s, (p->opt_graphs && whole) ? &p->graphs_b : nullptr);

@@ -95,8 +95,9 @@ struct RecBwdArgs {
     size_t x_slot;
     const half8* wfrag2; // two-dimensional layout: [32 column slices][kq contraction slices][4 waves][64/kq k-steps][4 tiles][64]
     float* P;            // two-dimensional layout: ring of 3 slots of p_slot floats for the partial sums; before the first
-                         // step the lowest bit of every word of slot (t+3)%3 is the opposite of t&1 for the first step t
-                         // that uses the slot (rec_bwd_part_fill)
+                         // step every word holds what rec_bwd_part_fill says: the 'unwritten' pattern (more than 2048
+                         // units), else a lowest bit in slot (t+3)%3 that is the opposite of t&1 for the first step t
+                         // that uses the slot
     size_t p_slot;
     float* dHn;          // [B][Hp] scaled gradient wrt final h (zeros when absent)
     float* dC;           // [B][Hp] running scaled dc; in: gradient wrt final c, out: dc0
@@ -189,7 +190,7 @@ int rec_bwd_dg_slots(const RecLayout& L);
 size_t rec_bwd_part_slot_floats(const RecLayout& L);
 constexpr int kRecBwdPartSlots = 3;
 // Word to fill slot `slot` of the partial ring with before a pass over T steps (see RecBwdArgs::P).
-unsigned rec_bwd_part_fill(int slot, int T);
+unsigned rec_bwd_part_fill(const RecLayout& L, int slot, int T);
 // Batch rows the rings of a backward layout are sized for (whole windows where the batch is walked in windows).
 int rec_bwd_ring_rows(const RecLayout& L, int B);
 

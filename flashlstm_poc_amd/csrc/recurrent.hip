@@ -1744,6 +1744,10 @@ __device__ __forceinline__ void ld_coherent_at(unsigned& d, const void* base, un
 __device__ __forceinline__ void ld_coherent_at(uintx4& d, const void* base, unsigned off) {
     asm volatile("global_load_dwordx4 %0, %1, %2 sc1" : "=v"(d) : "v"(off), "s"(base) : "memory");
 }
+// (a store addressed the same way)
+__device__ __forceinline__ void st_at(void* base, unsigned off, uintx4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, %2" ::"v"(off), "v"(v), "s"(base) : "memory");
+}
 // the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
 __device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
 __device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
@@ -1869,8 +1873,8 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, Re
 }
 
 // Backward: the product dh = dG_{t+1} * W_hh is split over 64-column slices s and four slices q of the contraction, as in
-// rec_bwd2d_kernel below (whose two rings and their protocol these are: dG through 8 slots with marks, fp32 partial sums
-// through 3 slots tagged with the parity of the step): a workgroup fetches a quarter of dG_{t+1}, forms a partial product
+// rec_bwd2d_kernel below, with its two rings: dG through 8 slots with marks, fp32 partial sums through 3 slots, with marks as
+// well (see mark_inbox): a workgroup fetches a quarter of dG_{t+1}, forms a partial product
 // [16 rows][64], sends 16 columns to each of the four workgroups of its slice -- seated in one XCD -- and finishes 16 units.
 // kWidePipe: (step, tile) items form ONE pipeline that does not stop at the end of a step: the product of item m, then the
 // cells of item m-1, whose partial sums have arrived meanwhile.  What the cells of item m-1 need from memory is requested behind
@@ -1949,13 +1953,9 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
         ld_coherent_at(o_dc, p.dC + size_t(rb) * 16 * p.Hp, cell * 4u);
     };
     auto settle_ops = [&]() __attribute__((always_inline)) { settle(o_gates); settle(o_cp); settle(o_cc); settle(o_dy); settle(o_dc); };
-    // dh of this thread's cell of (t, rb): the four senders' columns, once they carry this step's parity
+    // dh of this thread's cell of (t, rb): the four senders' columns, once none of them shows the mark
     auto collect = [&](int t, int rb) __attribute__((always_inline)) -> float {
-        const unsigned par = unsigned(t) & 1u;
-        auto stale = [&]() -> bool {
-            const unsigned all1 = o_in.x & o_in.y & o_in.z & o_in.w, any1 = o_in.x | o_in.y | o_in.z | o_in.w;
-            return __any(par ? (all1 & 1u) == 0u : (any1 & 1u) != 0u) != 0;
-        };
+        auto stale = [&]() -> bool { return __any(max(max(o_in.x, o_in.y), max(o_in.z, o_in.w)) == kUnwritten) != 0; };
         if (stale()) {
             int spins = 0;
             long long spin_start = 0;
@@ -1970,6 +1970,14 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
         const float a0 = as_float(hi2 ? o_in.z : o_in.x) + as_float(quad_xor2(hi2 ? o_in.x : o_in.z));
         const float a1 = as_float(hi2 ? o_in.w : o_in.y) + as_float(quad_xor2(hi2 ? o_in.y : o_in.w));
         return (hi1 ? a1 : a0) + as_float(quad_xor1(as_bits(hi1 ? a0 : a1)));
+    };
+    // What collect has read is marked for the next use of the slot, step t-3: each lane marks the 16 bytes that it alone reads.
+    // The mark is acknowledged before the wave stores its dG_{t-1} of these rows (every item waits once for its stores), and a
+    // sender's sums of step t-3 wait for dG_{t-2} of one slice of the contraction, whose cells waited for all four senders of step
+    // t-2, who waited for dG_{t-1} of every unit: nobody can overtake the mark.  The sums travel whole; a parity in their
+    // lowest bit, which needs no marks (rec_bwd2d_kernel), would cost them 2^-24.  Behind the cells: off the critical path.
+    auto mark_inbox = [&](int t, int rb) __attribute__((always_inline)) {
+        st_at(part_slot(t) + size_t(inbox0 + unsigned(rb)) * 1024u, in_at * 4u, uintx4{kUnwritten, kUnwritten, kUnwritten, kUnwritten});
     };
     auto cell = [&](int t, int rb, float dh, float dc_in) __attribute__((always_inline)) {
         const int b = rb * 16 + r;
@@ -2036,13 +2044,13 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
         floatx4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += *reinterpret_cast<const floatx4*>(part + (size_t(w) * 16 + r) * PLD + 4 * c);
-        uintx4 tagged = __builtin_bit_cast(uintx4, v);
+        uintx4 sums = __builtin_bit_cast(uintx4, v);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) tagged[e] = (tagged[e] & ~1u) | (unsigned(t) & 1u);
+        for (int e = 0; e < 4; ++e) sums[e] = min(sums[e], kUnwritten - 1u);   // (a NaN that looks like the mark stays a NaN)
         // what the loads behind the fragments brought is here, and everything stored so far is acknowledged (the marks of
         // the items before are in place ahead of what comes next)
         wait_all_vm();
-        *reinterpret_cast<uintx4*>(part_slot(t) + size_t(outbox0 + unsigned(rb)) * 1024u + out_at) = tagged;
+        *reinterpret_cast<uintx4*>(part_slot(t) + size_t(outbox0 + unsigned(rb)) * 1024u + out_at) = sums;
         clk.lap(1);
     };
 
@@ -2081,6 +2089,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
                     const float dh = collect(pt, prb);
                     clk.lap(4);
                     cell(pt, prb, dh, as_float(o_dc));
+                    mark_inbox(pt, prb);
                     clk.lap(2);
                 }
                 have_prev = true;
@@ -2096,6 +2105,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
             settle(o_in);
             const float dh = collect(pt, prb);
             cell(pt, prb, dh, as_float(o_dc));
+            mark_inbox(pt, prb);
         }
     } else {
         for (; t >= t_last; --t) {
@@ -2108,6 +2118,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_wide_kernel(RecBwdArgs p, Re
                 const float dh = collect(t, rb);
                 clk.lap(4);
                 cell(t, rb, dh, ONE ? dc_carried : as_float(o_dc));
+                mark_inbox(t, rb);
                 clk.lap(2);
             }
         }
@@ -3333,7 +3344,8 @@ size_t rec_bwd_part_slot_floats(const RecLayout& L) {
 int rec_bwd_ring_rows(const RecLayout& L, int B) {
     return (L.two_d && L.win_rows) ? int(ceil_div(size_t(B), size_t(L.win_rows))) * L.win_rows : B;
 }
-unsigned rec_bwd_part_fill(int slot, int T) {
+unsigned rec_bwd_part_fill(const RecLayout& L, int slot, int T) {
+    if (L.wide) return kUnwritten;
     // the first product step of a pass is T-2; going down from there, the first step that lands in `slot`
     for (int t = T - 2; t >= -1 && t > T - 2 - kRecBwdPartSlots; --t)
         if ((t + 3) % kRecBwdPartSlots == slot) return (unsigned(t) & 1u) ^ 1u;

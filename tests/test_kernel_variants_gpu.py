@@ -76,3 +76,19 @@ def test_row_tile_choice_where_short_contraction_kernels_are_the_rule(T, B, H, s
     for k in by_rule:   # the same kernels on the same fragments: the same bits
         assert np.array_equal(tuned[k], got[k]) and np.array_equal(again[k], by_rule[k]), k
     core.close()
+
+
+# The partial sums that the workgroups of a column slice exchange keep all of their bits.  With one non-zero weight, a one, in
+# every column of W_hh the closing product gives back single fp16 gate gradients, exactly: one tile, two, several
+@pytest.mark.parametrize("T,B,H", [(1, 16, 2049), (3, 5, 2560), (2, 17, 3072), (4, 40, 3585), (3, 33, 4096)])
+def test_wide_backward_exchanges_whole_sums(T, B, H):
+    import torch
+    p = make_problem(T, B, 24, H, seed=B * 10000 + H)
+    p["w_hh"] = torch.zeros(4 * H, H)
+    p["w_hh"][(torch.arange(H) * 7919 + 13) % (4 * H), torch.arange(H)] = 1.0
+    got, info = run_core(p)
+    assert info["fallbacks"] == 0 and info["bwd_two_d"] == 1
+    dh0 = torch.from_numpy(got["dh0"])
+    normal = dh0.abs() >= 2.0 ** -14
+    assert normal.float().mean() > 0.5
+    assert torch.equal(dh0[normal], dh0[normal].half().double())
