@@ -191,8 +191,7 @@ int publish_with(flstm_core_plan* p, OpList& last, int stamp, hipStream_t s) {
     return 0;
 }
 int wait_stream(hipStream_t s) {
-    FL_TRY(hipStreamSynchronize(s));
-    persistent_stream_idle(s);
+    FL_TRY(wait_for_persistent(s));
     return 0;
 }
 // after the stream has been waited for: the status of the pass; a non-zero one is cleared on the device

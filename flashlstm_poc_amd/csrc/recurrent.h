@@ -206,9 +206,9 @@ int rec_bwd_ks(const RecLayout& L, int Hp);
 // Idle workgroups that a launch with this layout can give to BesideCopies (0: step-wise, or every CU has work).
 int rec_idle_workgroups(const RecLayout& L);
 
-// To be called once a stream that persistent launches went to has been waited for: launches on other streams no longer
-// need to be ordered behind it (launch_persistent).
-void persistent_stream_idle(hipStream_t stream);
+// Waits for a stream that persistent launches went to.  Launches on other streams no longer need to be ordered behind them
+// then (launch_persistent).
+hipError_t wait_for_persistent(hipStream_t stream);
 
 // Runs steps [t0, t1). Persistent layouts use one launch; otherwise one launch per step.
 hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs = nullptr);

@@ -40,6 +40,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "launch_gate.h"
 #include "layout_device.h"
 #include "recurrent.h"
 
@@ -3092,15 +3093,41 @@ hipError_t prepare_kernel(K kernel, size_t lds, int threads, std::atomic<int>* p
 // side on one device (two plans, two streams) could each get half of the CUs and wait for the rest, so launches to
 // different streams are put one behind the other here; launches to one stream are in order anyway.  Only when a launch
 // meets another stream's pass in flight does that cost anything (an event).  hipLaunchCooperativeKernel gives the same
-// guarantee by sending every such kernel through a queue of its own, with a signal from the caller's queue to it and one
-// back: 20 us per launch, 40 of the 400 us of a training pass over 64 steps of 256 units.
+// guarantee, among cooperative launches, by sending every such kernel through a queue of its own, with a signal from the
+// caller's queue to it and one back: 20 us per launch, 40 of the 400 us of a training pass over 64 steps of 256 units.
 struct PersistentGate {
     std::mutex mutex;
-    hipStream_t stream = nullptr;   // where the last launch went
-    bool in_flight = false;         // ... and it has not been waited for yet
+    LaunchGate<hipStream_t> order{hipStreamPerThread};
     hipEvent_t event = nullptr;
 };
 PersistentGate g_gate[kMaxDevices];
+
+// the end of everything `stream` has been given so far, as the gate's event
+hipError_t record_gate(PersistentGate& gate, hipStream_t stream) {
+    if (!gate.event) {
+        const hipError_t e = hipEventCreateWithFlags(&gate.event, hipEventDisableTiming);
+        if (e != hipSuccess) return e;
+    }
+    return hipEventRecord(gate.event, stream);
+}
+
+// Puts what `stream` gets next behind the last persistent launch.  (No stream of the last launch is being captured: the
+// captures of this library hold the gate, see launch_steps.)
+hipError_t wait_for_gate(PersistentGate& gate, hipStream_t stream) {
+    if (!gate.order.must_wait(stream)) return hipSuccess;
+    hipError_t e = hipSuccess;
+    if (!gate.order.recorded()) e = gate.order.wants_event(gate.order.last()) ? hipErrorNotReady : record_gate(gate, gate.order.last());
+    if (e == hipSuccess) e = hipStreamWaitEvent(stream, gate.event, 0);
+    if (e == hipSuccess) return e;
+    // (the other stream is gone, or has no event: nothing of it can be running once the device is idle)
+    (void)hipGetLastError();
+    return hipDeviceSynchronize();
+}
+
+void passed_gate(PersistentGate& gate, hipStream_t stream) {
+    const bool recorded = gate.order.wants_event(stream) && record_gate(gate, stream) == hipSuccess;
+    gate.order.launched(stream, recorded);
+}
 
 // A grid that cannot be co-resident is exactly what a persistent launch must not be given: nothing is launched then
 // (hipErrorCooperativeLaunchTooLarge) and the caller runs the pass step-wise.  Workgroups of OTHER kernels can still keep
@@ -3108,43 +3135,48 @@ PersistentGate g_gate[kMaxDevices];
 template <typename K, typename A>
 hipError_t launch_persistent(K kernel, int grid, size_t lds, hipStream_t stream, A a, RecLayout L, int t_a, int t_b,
                              int ks_wave, int workgroups_per_cu, int device, int threads = kThreads) {
+    PersistentGate& gate = g_gate[device];
+    std::lock_guard<std::mutex> lock(gate.mutex);
     if (L.cooperative) {
+        const hipError_t ordered = wait_for_gate(gate, stream);
+        if (ordered != hipSuccess) return ordered;
         void* params[] = {&a, &L, &t_a, &t_b, &ks_wave};
         hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(grid), dim3(threads), params,
                                                   unsigned(lds), stream);
-        if (e == hipSuccess) return hipSuccess;
+        if (e == hipSuccess) {
+            passed_gate(gate, stream);
+            return hipSuccess;
+        }
         (void)hipGetLastError();
         if (e == hipErrorCooperativeLaunchTooLarge) return e;
         // (any other refusal: no cooperative launch on this runtime)
     }
     if (workgroups_per_cu < 1 || grid > workgroups_per_cu * L.num_cus) return hipErrorCooperativeLaunchTooLarge;
-    PersistentGate& gate = g_gate[device];
-    std::lock_guard<std::mutex> lock(gate.mutex);
-    if (gate.in_flight && gate.stream != stream) {
-        hipError_t e = hipSuccess;
-        if (!gate.event) e = hipEventCreateWithFlags(&gate.event, hipEventDisableTiming);
-        if (e == hipSuccess) e = hipEventRecord(gate.event, gate.stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(stream, gate.event, 0);
-        if (e != hipSuccess) {   // (the other stream is gone: nothing of it can be running once the device is idle)
-            (void)hipGetLastError();
-            e = hipDeviceSynchronize();
-            if (e != hipSuccess) return e;
-        }
-    }
+    hipError_t e = wait_for_gate(gate, stream);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, a, L, t_a, t_b, ks_wave);
-    const hipError_t e = hipGetLastError();
-    if (e == hipSuccess) { gate.stream = stream; gate.in_flight = true; }
+    e = hipGetLastError();
+    if (e == hipSuccess) passed_gate(gate, stream);
     return e;
 }
 
 }  // namespace
 
-void persistent_stream_idle(hipStream_t stream) {
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return;
-    PersistentGate& gate = g_gate[device];
-    std::lock_guard<std::mutex> lock(gate.mutex);
-    if (gate.stream == stream) gate.in_flight = false;
+hipError_t wait_for_persistent(hipStream_t stream) {
+    int device = -1;
+    PersistentGate* gate = nullptr;
+    unsigned long launches = 0;
+    if (hipGetDevice(&device) == hipSuccess && device >= 0 && device < kMaxDevices) {
+        gate = &g_gate[device];
+        std::lock_guard<std::mutex> lock(gate->mutex);
+        launches = gate->order.launches();
+    }
+    const hipError_t e = hipStreamSynchronize(stream);
+    if (e == hipSuccess && gate) {
+        std::lock_guard<std::mutex> lock(gate->mutex);
+        gate->order.waited(stream, launches);
+    }
+    return e;
 }
 
 size_t exchange_slot_halfs(int rows, int cols) { return round_up(size_t(rows), 32) * size_t(cols); }
@@ -3381,7 +3413,13 @@ static hipError_t launch_steps(StepGraphCache* graphs, const void* kernel, const
             graphs->replays++;
             return hipGraphLaunch(e.exec, stream);
         }
-    // not seen before: capture the launches (nothing runs yet), instantiate, launch
+    // Not seen before: capture the launches (nothing runs yet), instantiate, launch.  The gate is held meanwhile: a persistent
+    // launch of another thread that had to wait for this stream would otherwise record its event into the capture.
+    int device = 0;
+    hipError_t de = hipGetDevice(&device);
+    if (de != hipSuccess) return de;
+    if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
+    std::unique_lock<std::mutex> gate_held(g_gate[device].mutex);
     if (hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
         (void)hipGetLastError();
         graphs->disabled = true;
@@ -3390,6 +3428,7 @@ static hipError_t launch_steps(StepGraphCache* graphs, const void* kernel, const
     hipError_t le = launch_all();
     hipGraph_t graph = nullptr;
     hipError_t ce = hipStreamEndCapture(stream, &graph);
+    gate_held.unlock();
     if (le != hipSuccess || ce != hipSuccess || !graph) {
         if (graph) (void)hipGraphDestroy(graph);
         (void)hipGetLastError();
