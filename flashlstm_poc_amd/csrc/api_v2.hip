@@ -385,6 +385,11 @@ void forward_window(Entry& e, const Streams& st, size_t n, const __half* x_host,
         if (!y_host) return;
         check(hipEventRecord(e.chunk_out[k], st.cs), "hipEventRecord");
         check(hipStreamWaitEvent(st.d2h, e.chunk_out[k], 0), "hipStreamWaitEvent");
+        if (y_dev && cp.ldh != H) {   // (the runtime copies rows of a pitch that is not their length one by one, 9 us and more each)
+            check(flstm_hip::gather_from_half(cp.h + (lo + 1) * B * cp.ldh, cp.ldh, (hi - lo) * B, int(H), y_dev + lo * B * H * sizeof(half_t), 0, 0, 0, st.d2h),
+                  "y rows");
+            return;
+        }
         download_rows(y_host, cp.h + B * cp.ldh, cp.ldh, H, sizeof(half_t), lo * B, (hi - lo) * B, st.d2h);
     };
     size_t ck_from = 0;   // checkpoints before this step are on their way

@@ -1198,17 +1198,19 @@ extern "C" int flstm_core_backward_end(flstm_core_plan* p, const void* x, flstm_
 }
 
 bool flstm_hip::core_copy_beside(flstm_core_plan* p, bool forward, const OpList& copies) {
-    // 48 workgroups of 256 threads with one 16-byte load in flight each keep a PCIe link of 57 GB/s busy
-    constexpr int kFewest = 16, kHelpers = 48;
-    const int idle = rec_idle_workgroups(forward ? p->Lf : p->Lb);
-    if (idle < kFewest || copies.count < 1 || copies.count > BesideCopies::kMost) return false;
+    // 48 workgroups of 256 threads with one 16-byte load in flight each keep a PCIe link of 57 GB/s busy.  What counts is the
+    // threads: the kernels for short contractions have workgroups of 64, 128 and 256 of them.
+    constexpr int kFewest = 16 * 256, kThreads = 48 * 256;
+    const RecLayout& L = forward ? p->Lf : p->Lb;
+    const int idle = rec_idle_workgroups(L), threads = rec_threads(L), enough = kThreads / threads;
+    if (idle * threads < kFewest || copies.count < 1 || copies.count > BesideCopies::kMost) return false;
     BesideCopies& b = forward ? p->beside_f : p->beside_b;
     for (int i = 0; i < copies.count; ++i) {
         if (copies.op[i].kind != LayoutOp::kUnpad) return false;
         b.op[i] = copies.op[i];
     }
     b.count = copies.count;
-    b.helpers = idle < kHelpers ? idle : kHelpers;
+    b.helpers = idle < enough ? idle : enough;
     return true;
 }
 

@@ -51,7 +51,7 @@ constexpr int kMaxOps = 12;
 struct LayoutOp {
     enum Kind : int { kFill = 1, kToHalf, kToFloat, kUnpad, kToExchange, kReduceDw, kReduceDb };
     int kind = 0;
-    int in_f32 = 0, out_f32 = 0, vec = 1;   // vec: elements per work item (8, 4 or 2 where alignment allows, else 1)
+    int in_f32 = 0, out_f32 = 0, vec = 1;   // vec: elements per work item (8 or 4 where alignment allows, else 1; kUnpad: 16 bytes of output then)
     void* dst = nullptr;
     void* dst2 = nullptr;
     const void* src = nullptr;              // null reads as zeros (kToHalf, kToFloat, kToExchange)

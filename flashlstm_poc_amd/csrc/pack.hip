@@ -241,7 +241,7 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
             if (o.vec == 8) op_convert<8>(o, first, stride);
             else op_convert<1>(o, first, stride);
         } else if (o.kind == LayoutOp::kUnpad) {
-            op_unpad_any(o, first, stride);
+            op_unpad(o, first, stride);
         } else if (o.kind == LayoutOp::kToExchange) {
             // item i = eight halfs of one lane: [16-row tile][32-wide k-step][lane] (recurrent.hip, xch_offset)
             const unsigned nks = unsigned(o.ld_out) / 32;
@@ -347,14 +347,23 @@ void OpList::to_float(const void* in, int in_f32, size_t rows, int cols, float s
 void OpList::unpad(const void* in, int in_f32, size_t ld_in, size_t rows, int cols, float scale, void* out, int out_f32,
                    size_t rows_per_block, size_t block_stride) {
     if (out == nullptr || rows * size_t(cols) == 0) return;
+    if (rows_per_block >= rows) rows_per_block = 0;
+    if (ld_in == size_t(cols) && rows_per_block == 0 && rows * size_t(cols) <= size_t(1) << 30) {   // contiguous: one row
+        cols = int(rows * size_t(cols));
+        ld_in = round_up(size_t(cols), 8);
+        rows = 1;
+    }
     LayoutOp& o = op[count++];
     o.kind = LayoutOp::kUnpad; o.in_f32 = in_f32; o.out_f32 = out_f32; o.dst = out; o.src = in;
-    o.vec = 1;
-    if (cols % 8 == 0 && ld_in % 8 == 0 && aligned16(in) && aligned16(out)) o.vec = 8;
-    else if (cols % 2 == 0 && ld_in % 2 == 0 && (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 8 == 0) o.vec = 2;
-    o.n = rows * size_t(cols) / o.vec;
+    o.vec = (cols % 8 == 0 && ld_in % 8 == 0 && aligned16(in) && aligned16(out)) ? 8 : 1;
+    if (o.vec == 8) {
+        o.n = rows * size_t(cols) / 8;
+    } else {   // 16 aligned bytes of the output per item (op_unpad_flat)
+        const size_t esz = out_f32 ? 4 : 2;
+        o.n = ceil_div(reinterpret_cast<uintptr_t>(out) % 16 + rows * size_t(cols) * esz, 16);
+    }
     o.rows = rows; o.cols = cols; o.ld_in = ld_in; o.scale = scale;
-    o.rows_per_block = rows_per_block >= rows ? 0 : rows_per_block; o.block_stride = block_stride;
+    o.rows_per_block = rows_per_block; o.block_stride = block_stride;
 }
 
 void OpList::to_exchange(const void* in, int in_f32, size_t rows, int cols, int kcols, half_t* slot) {

@@ -203,8 +203,10 @@ size_t rec_bwd_fragments(const RecLayout& L, int Hp);   // (the one-way kernels'
 int rec_fwd_ks(const RecLayout& L, int Hp);
 int rec_bwd_ks(const RecLayout& L, int Hp);
 
-// Idle workgroups that a launch with this layout can give to BesideCopies (0: step-wise, or every CU has work).
+// Idle workgroups that a launch with this layout can give to BesideCopies (0: step-wise, or every CU has work), and the
+// threads of one.
 int rec_idle_workgroups(const RecLayout& L);
+int rec_threads(const RecLayout& L);
 
 // Waits for a stream that persistent launches went to.  Launches on other streams no longer need to be ordered behind them
 // then (launch_persistent).

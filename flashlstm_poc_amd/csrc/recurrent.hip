@@ -107,7 +107,7 @@ __device__ __forceinline__ void copy_beside(const BesideCopies& c, int* lds_tick
     const int ticket = *lds_ticket;
     if (ticket >= c.helpers) return;
     const size_t stride = size_t(c.helpers) * blockDim.x, first = size_t(ticket) * blockDim.x + threadIdx.x;
-    for (int i = 0; i < c.count; ++i) op_unpad_any(c.op[i], first, stride);
+    for (int i = 0; i < c.count; ++i) op_unpad(c.op[i], first, stride);
 }
 
 // Pattern that marks a not-yet-written pair of halfs in the exchange ring.
@@ -3462,6 +3462,8 @@ int rec_idle_workgroups(const RecLayout& L) {
     const int busy = L.wide && L.two_d ? L.nh * L.jb / 64 * L.kq : L.ng * L.nh;   // (nh, jb: the one-way layout)
     return busy < L.num_cus ? L.num_cus - busy : 0;
 }
+
+int rec_threads(const RecLayout& L) { return (L.split ? L.split : L.nw) * kWave; }
 
 // A launch whose groups sit inside the XCDs always has one workgroup per CU, the others as many as they seat; those
 // get the helpers on top.
