@@ -133,3 +133,33 @@ class SafeTorchLstm(torch.nn.Module):
         """(dW_ih, dW_hh, db) of layer l after backward()."""
         g = self.layers[l].weight_ih_l0.grad
         return g[:, :-1], self.layers[l].weight_hh_l0.grad, g[:, -1]
+
+
+def reference_64(p, device="cuda"):
+    """Forward and backward pass in 64-bit arithmetic on the fp16-rounded weights, from plain matrix products: for layers too
+    large for the CPU oracle.  Same keys as torch_reference, tensors on `device`."""
+    d = {k: v.to(device=device, dtype=torch.float64) for k, v in p.items()}
+    W, U = p["w_ih"].half().to(device).double(), p["w_hh"].half().to(device).double()
+    T, B, I = d["x"].shape
+    h, c = d["h0"], d["c0"]
+    hs, cs, gates = [h], [c], []
+    xp = (d["x"].reshape(T * B, I) @ W.t()).reshape(T, B, -1) + d["b_ih"] + d["b_hh"]
+    for t in range(T):
+        i, f, g, o = (xp[t] + h @ U.t()).chunk(4, 1)
+        i, f, g, o = i.sigmoid(), f.sigmoid(), g.tanh(), o.sigmoid()
+        c = f * c + i * g
+        h = o * c.tanh()
+        hs.append(h); cs.append(c); gates.append((i, f, g, o))
+    dh, dc = d["d_hn"], d["d_cn"]
+    dW, dU, db, dx = torch.zeros_like(W), torch.zeros_like(U), torch.zeros_like(d["b_ih"]), torch.zeros_like(d["x"])
+    for t in range(T - 1, -1, -1):
+        i, f, g, o = gates[t]
+        dh = dh + d["dy"][t]
+        tc = cs[t + 1].tanh()
+        dc = dc + dh * o * (1 - tc * tc)
+        dz = torch.cat([dc * g * i * (1 - i), dc * cs[t] * f * (1 - f), dc * i * (1 - g * g), dh * tc * o * (1 - o)], 1)
+        dc, dh, dx[t] = dc * f, dz @ U, dz @ W
+        dW += dz.t() @ d["x"][t]
+        dU += dz.t() @ hs[t]
+        db += dz.sum(0)
+    return dict(y=torch.stack(hs[1:]), hn=h, cn=cs[-1], dx=dx, dw_ih=dW, dw_hh=dU, db=db, dh0=dh, dc0=dc)

@@ -92,3 +92,60 @@ def test_wide_backward_exchanges_whole_sums(T, B, H):
     normal = dh0.abs() >= 2.0 ** -14
     assert normal.float().mean() > 0.5
     assert torch.equal(dh0[normal], dh0[normal].half().double())
+
+
+# more than 2048 units over enough steps that every slot of the rings is used again and again (eight of dG, three of partial
+# sums): one tile, two, several.  No further from 64-bit arithmetic than one launch per step is; the two differ by which fp16
+# roundings of dG their summation orders flip, 1.3 % in the error at the most over 64 measured pairs, hence 5 %
+@pytest.mark.parametrize("T,B,H", [(24, 1, 2049), (21, 32, 4096), (20, 40, 3072), (22, 70, 2560), (33, 17, 3600)])
+def test_wide_layers_against_64_bits(T, B, H):
+    from helpers import reference_64, rell2
+    p = make_problem(T, B, 24, H, seed=B * 10000 + H)
+    ref = {k: v.cpu().numpy() for k, v in reference_64(p).items()}
+    got, info = run_core(p)
+    assert info["fallbacks"] == 0 and info["persistent_fwd"] == 1 and info["persistent_bwd"] == 1 and info["bwd_two_d"] == 1
+    check_against(ref, got, label=f"T={T} B={B} H={H}")
+    steps, info = run_core(p, stepwise=True)
+    assert info["persistent_bwd"] == 0
+    for k in ref:
+        assert rell2(got[k], ref[k]) <= 1.05 * rell2(steps[k], ref[k]), (k, rell2(got[k], ref[k]), rell2(steps[k], ref[k]))
+
+
+# ... and fed in ranges of steps: what a launch leaves for the next one (the cell state, running dc, both rings, the delay
+# hint) gives the bits of one launch.  Ranges of one step, shorter and longer than the rings
+@pytest.mark.parametrize("T,B,H", [(21, 16, 2049), (23, 30, 3072), (20, 48, 4096), (26, 65, 2600)])
+def test_wide_layers_in_ranges_of_steps(T, B, H):
+    import numpy as np
+    import torch
+    from helpers import rell2, to_np
+    from flashlstm_poc_amd import LstmCore
+    I = 64
+    p = make_problem(T, B, I, H, seed=B * 10000 + H)
+    core = LstmCore(B, I, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    want, info = run_core(p, core=core)
+    lib, s = core.lib, torch.cuda.current_stream().cuda_stream
+    t16 = {k: p[k].cuda().half() for k in ("x", "dy", "h0", "c0", "d_hn", "d_cn")}
+    ptr = {k: v.data_ptr() for k, v in t16.items()}
+    F16 = 1
+    hy, cy = torch.empty(B, H, device="cuda", dtype=torch.float16), torch.empty(B, H, device="cuda", dtype=torch.float16)
+    assert lib.flstm_core_forward_begin(core._h, T, ptr["x"], F16, ptr["h0"], ptr["c0"], F16, s) == 0
+    cuts = [0, 1, 2, 5, 14, T]
+    for a, b in zip(cuts[:-1], cuts[1:]):
+        assert lib.flstm_core_forward_steps(core._h, a, b - a, s) == 0
+    assert lib.flstm_core_forward_end(core._h, hy.data_ptr(), cy.data_ptr(), F16, 1, s) == 0
+    dx = torch.empty(T, B, I, device="cuda", dtype=torch.float16)
+    out = {k: torch.empty(*n, device="cuda") for k, n in (("dw_ih", (4 * H, I)), ("dw_hh", (4 * H, H)), ("db", (4 * H,)),
+                                                        ("db_hh", (4 * H,)), ("dh0", (B, H)), ("dc0", (B, H)))}
+    assert lib.flstm_core_backward_begin(core._h, T, ptr["dy"], F16, ptr["d_hn"], ptr["d_cn"], F16, 1.0, dx.data_ptr(), F16, s) == 0
+    for a, b in reversed(list(zip(cuts[:-1], cuts[1:]))):
+        assert lib.flstm_core_backward_steps(core._h, b - 1, b - a, s) == 0
+    assert lib.flstm_core_backward_end(core._h, ptr["x"], F16, *(out[k].data_ptr() for k in ("dw_ih", "dw_hh", "db", "db_hh", "dh0", "dc0")), s) == 0
+    torch.cuda.synchronize()
+    assert core.info("fallbacks") == 0 and core.info("persistent_bwd") == 1
+    assert np.array_equal(to_np(hy), want["hn"]) and np.array_equal(to_np(cy), want["cn"])
+    for k in ("dh0", "dc0", "dw_ih", "dw_hh"):
+        assert np.array_equal(to_np(out[k]), want[k]), k
+    assert rell2(to_np(dx), want["dx"]) <= 1e-5                # (products of other heights)
+    assert rell2(to_np(out["db"]), want["db"]) <= 1e-6         # (summed range by range)
+    core.close()
