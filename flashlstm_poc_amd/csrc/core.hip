@@ -118,7 +118,7 @@ struct flstm_core_plan {
     StepGraphCache graphs_f, graphs_b;   // captured step-wise launches (only used where the persistent kernels are not)
     int opt_graphs = 1;
     int opt_two_d = 1;   // backward recurrence for 2048 hidden units, two-way split: 0 never, 1 where it is faster, 2 wherever it can run
-    int opt_waves_f = 0;   // wavefronts per workgroup of the forward recurrence: 0 = by size, 4, 8 (the weights are packed for it)
+    int opt_waves_f = 0;   // wavefronts per workgroup of the forward recurrence: 0 = by size, 4, 8 (one-way kernels, whose weights are packed for it)
     HostStatus* status_host = nullptr;   // pinned: the last launch of a pass leaves the status word and the stamps here
     int seat_sets_left = 0;              // zeroed sets of seat counters in the status block
     int inject_stall = 0;         // test hook: treat the next N passes as if their launches had given up
@@ -334,8 +334,8 @@ extern "C" int flstm_core_set_option(flstm_core_plan* p, const char* name, long 
     if (!strcmp(name, "step_graphs")) { p->opt_graphs = value != 0; return 0; }
     if (!strcmp(name, "bwd_two_d")) { if (value < 0 || value > 2) return FLSTM_E_INVALID; p->opt_two_d = int(value); p->two_d_explicit = true; replan(p); return 0; }
     if (!strcmp(name, "waves_fwd")) {
-        // wavefronts per workgroup of the forward recurrence: the weight fragments are packed for it, so a change
-        // un-packs them
+        // wavefronts per workgroup of the forward recurrence: the one-way kernels' weight fragments are packed for 4 or 8
+        // of them, so a change from one to the other un-packs them
         if (value != 0 && value != 4 && value != 8) return FLSTM_E_INVALID;
         const int before = p->Lf.nw;
         p->opt_waves_f = int(value);
@@ -362,7 +362,7 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
     if (!strcmp(name, "row_tiles_bwd")) return p->Lb.mt;
     if (!strcmp(name, "cooperative")) return p->opt_cooperative;
     if (!strcmp(name, "bwd_two_d")) return p->Lb.two_d;
-    if (!strcmp(name, "waves_fwd")) return p->Lf.nw;
+    if (!strcmp(name, "waves_fwd")) return rec_threads(p->Lf) / kWave;
     if (!strcmp(name, "graph_captures")) return p->graphs_f.captures + p->graphs_b.captures;
     if (!strcmp(name, "graph_replays")) return p->graphs_f.replays + p->graphs_b.replays;
     if (!strcmp(name, "graphs_disabled")) return (p->graphs_f.disabled ? 1 : 0) + (p->graphs_b.disabled ? 2 : 0);

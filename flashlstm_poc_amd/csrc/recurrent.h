@@ -174,7 +174,8 @@ constexpr size_t kGraphCacheEntries = 4;
 // (1 only where it fits; above 2048 units tiles of 16 rows are taken one after the other whatever it says).  2 is always
 // a one-way kernel: those for short contractions (RecLayout::split) have 16-row blocks.  Each of the two families has its
 // own weight fragments, which depend on the sizes alone (and, one-way forward, on `waves`).
-// waves: 0 = the rule of thumb (rec_waves), 4 or 8 = that many wavefronts per workgroup (8 only up to 1024 units).
+// waves: 0 = the rule of thumb (rec_waves), 4 or 8 = a one-way kernel with that many wavefronts per workgroup (8 only up to
+// 1024 units).
 RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt = 0, int waves = 0);
 // two_d: 0 = never the two-way split, 1 = where it is the faster layout, 2 = wherever it can run
 RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt = 0, int two_d = 1);

@@ -3270,8 +3270,9 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.unit_major = L.nw == 8 || (fits && Hp > 2048);
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
     L.wide = fits && Hp > 2048;
-    // short contractions: columns split over the waves, where every group has one 16-row block (and 32-row blocks are not asked for)
-    if (L.nw == 4 && force_mt != 2 && Hp <= kFwdSplitMost && num_cus == 256) {
+    // short contractions: columns split over the waves, where every group has one 16-row block (and neither 32-row blocks nor four
+    // waves that split the contraction are asked for)
+    if (L.nw == 4 && waves != 4 && force_mt != 2 && Hp <= kFwdSplitMost && num_cus == 256) {
         for (int per_wg : {1, 2, 4}) {
             if (per_wg == 4 && Hp > kFwdSplitFourMost) break;
             if (Hp / (8 * per_wg) > 32 || !can_16_rows(B, Hp / (8 * per_wg), num_cus)) continue;

@@ -63,6 +63,9 @@ int flstm_core_destroy(flstm_core_plan* plan);
  * batch rows or 1024 and at most 256; 0 = never, 1 = where it measured faster than the one-way layout
  * (2048 units with at most 32 or with 65..128 batch rows), 2 = wherever it can run; default 1, FLASHLSTM_BWD_TWO_D sets
  * the default),
+ * "waves_fwd" (wavefronts per workgroup of the forward recurrence: 0, the default, by size; 4 or 8, which split the
+ * contraction between them, also where the kernel for short contractions would run; 8 up to 1024 units, with 32-row
+ * blocks.  The weights are packed for it: a change between 4 and 8 un-packs them; FLASHLSTM_WAVES_FWD sets the default),
  * "inject_stall" (test hook: the next N passes that use a persistent kernel are treated as if that launch had
  * given up, which exercises the step-wise repeat and the demotion rule without making any kernel wait). */
 int flstm_core_set_option(flstm_core_plan* plan, const char* name, long value);
@@ -70,7 +73,8 @@ int flstm_core_set_option(flstm_core_plan* plan, const char* name, long value);
  * "fallbacks" (persistent launches that had to be redone step-wise), "demotions_fwd", "demotions_bwd" (how often a
  * direction was demoted to step-wise launches after such a give-up), "hold_fwd", "hold_bwd" (passes a demoted
  * direction still runs step-wise before the persistent kernel is tried again; 0 = not demoted), "slice_fwd", "slice_bwd" (hidden units
- * per workgroup of the recurrence kernels), "row_tiles_fwd", "row_tiles_bwd" (16-row tiles per row block that the
+ * per workgroup of the recurrence kernels), "waves_fwd" (wavefronts per workgroup the forward recurrence runs with: 1, 2,
+ * 4 or 8), "row_tiles_fwd", "row_tiles_bwd" (16-row tiles per row block that the
  * recurrences run with; "row_tiles": the forward one), "hidden_padded",
  * "input_padded", "device_bytes" (device memory the plan holds), "static_scratch_bytes" (size of the fixed scratch
  * array of flstm_core_forward_static), "num_cus" and "clock_khz" (compute units and

@@ -149,3 +149,29 @@ def test_wide_layers_in_ranges_of_steps(T, B, H):
     assert rell2(to_np(dx), want["dx"]) <= 1e-5                # (products of other heights)
     assert rell2(to_np(out["db"]), want["db"]) <= 1e-6         # (summed range by range)
     core.close()
+
+
+# four waves asked for where the rule runs the kernel for short contractions with one, two and four: the kernel that splits
+# the contraction between its waves, on weights packed before, and back
+@pytest.mark.parametrize("T,B,H,rule", [(5, 64, 256, 1), (4, 40, 512, 2), (3, 300, 256, 4), (6, 9, 65, 1)])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_four_waves_where_short_contraction_kernels_are_the_rule(T, B, H, rule, stepwise):
+    import numpy as np
+    from flashlstm_poc_amd import LstmCore
+    p = make_problem(T, B, 20, H, seed=B * 10000 + H)
+    ref, _ = oracle_reference(p)
+    core = LstmCore(B, 20, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    assert core.info("waves_fwd") == rule and core.info("slice_fwd") == 8 * rule
+    by_rule, _ = run_core(p, core=core, stepwise=stepwise)
+    core.set_option("waves_fwd", 4)
+    assert core.info("waves_fwd") == 4 and core.info("slice_fwd") == 32 and core.info("row_tiles_fwd") == 1
+    got, info = run_core(p, core=core, stepwise=stepwise)
+    assert info["fallbacks"] == 0
+    check_against(ref, got, label=f"T={T} B={B} H={H} stepwise={stepwise} four waves")
+    core.set_option("waves_fwd", 0)
+    again, _ = run_core(p, core=core, stepwise=stepwise)
+    assert core.info("waves_fwd") == rule
+    for k in by_rule:
+        assert np.array_equal(again[k], by_rule[k]), k
+    core.close()
