@@ -123,8 +123,7 @@ def measured_traffic(workload, phase):
 
 def measured_counters(workload, phase):
     """L2 request and LDS activity counters per launch of a phase's kernel from the same committed summary (rocprofv3
-    --pmc TCC_REQ_sum / SQ_LDS_IDX_ACTIVE / GRBM_GUI_ACTIVE and the kernel trace's duration, taken with plain launches:
-    a profiler tool and cooperative launches do not go together).  None unless the summary was taken from exactly
+    --pmc TCC_REQ_sum / SQ_LDS_IDX_ACTIVE / GRBM_GUI_ACTIVE and the kernel trace's duration).  None unless the summary was taken from exactly
     the kernel sources that are running now."""
     import re
     path = os.path.join(ROOT, "profiles", "hbm_traffic_per_kernel.md")
@@ -370,8 +369,8 @@ def main():
 
 
 def bench_single(args, device):
-    """One single-layer workload: fwd (+ bwd) steps timed with hipEvents, per-phase times from the library's own
-    events on the launch stream, roofline of the dominant kernel, parity on the timed tensors."""
+    """One single-layer workload: fwd (+ bwd) steps timed with hipEvents, per-phase times from the stamps that the
+    library's kernels leave, roofline of the dominant kernel, parity on the timed tensors."""
     import torch
     from flashlstm_poc_amd import LstmCore
     T, B, I, H, backward = WORKLOADS[args.workload]
@@ -396,7 +395,7 @@ def bench_single(args, device):
     e0.record()
     for _ in range(args.steps):
         step()
-        for k in phases:   # device time of each phase of this step (hipEvents on the launch stream)
+        for k in phases:   # device time of each phase of this step (the kernels' stamps)
             acc[k] += core.last_ms(k)
     e1.record()
     torch.cuda.synchronize()
@@ -465,8 +464,7 @@ def bench_single(args, device):
     }
     # What the recurrence moves between workgroups each step.  Measured: requests to the L2 (TCC_REQ, each at most one
     # 128-byte line) and the cycles the LDS address unit was busy (SQ_LDS_IDX_ACTIVE, summed over the CUs), from the
-    # committed counter summary -- taken with plain launches, 5 % slower than the cooperative launches timed here --
-    # divided by that profile's own kernel duration.  Beside them the byte model: every workgroup (16 or 32 batch rows x
+    # committed counter summary, divided by that profile's own kernel duration.  Beside them the byte model: every workgroup (16 or 32 batch rows x
     # one slice of hidden units) fetches the whole h_{t-1} (forward) or dG_{t+1} (backward) of its rows from the L2.
     block = 16 * core.info("row_tiles")   # batch rows per workgroup
     Hp, rows = core.info("hidden_padded"), block * ((B + block - 1) // block)
@@ -488,7 +486,7 @@ def bench_single(args, device):
                 "l2_gb_per_s_at_128B_per_request": round(c["TCC_REQ"] * 128 / (c["ms"] * 1e-3) / 1e9, 1),
                 "lds_busy_cycles_per_step_and_cu": round(c["SQ_LDS_IDX_ACTIVE"] / T / cus, 1),
                 "lds_busy_fraction": round(c["SQ_LDS_IDX_ACTIVE"] / cus / (c["GRBM_GUI_ACTIVE"] / 8), 4),
-                "profile_launch_ms": c["ms"], "launches": "plain (profiler attached)", "source": note}})
+                "profile_launch_ms": c["ms"], "source": note}})
         else:
             entry["measured"] = None
             entry["measured_note"] = note

@@ -7,10 +7,11 @@
 // sequences (or a smaller FLASHLSTM_V2_DEVICE_BUDGET_MB / a forced FLASHLSTM_V2_WINDOW_STEPS) run as several
 // windows with the state carried between them in fp32, which is exact.  Inside a window the work is streamed
 // in CHUNKS: x (dY) goes up in chunks of time steps on the h2d stream, each chunk's projection + recurrence
-// (BPTT steps + dX) is enqueued on the compute stream behind an event, and its y (dx) rows leave on the d2h
-// stream behind another, so the three streams overlap as in the reference's 32-step pipeline
-// (flashlstm_v2/src/lstm_forward.cu:646-940).  FLASHLSTM_V2_CHUNK_STEPS sets the chunk length (default 64;
-// 0 = whole window).
+// (BPTT steps + dX) is enqueued on the compute stream behind an event, and its y (dx) rows leave beside the next
+// chunk's recurrence, written to pinned host memory by workgroups of that launch that have no part in it (where there are
+// none, or the memory is pageable, and for the last chunk: on the d2h stream), so that transfers in both directions and
+// compute overlap as in the reference's 32-step pipeline (flashlstm_v2/src/lstm_forward.cu:646-940).
+// FLASHLSTM_V2_CHUNK_STEPS sets the chunk length (default: chunk_starts(); 0 = whole window).
 //
 // Backward needs the gate cache of the steps it walks.  With one window, forward keeps it on the device in a
 // small registry, and a backward call reuses it when it names the same buffers AND their contents are what
@@ -271,7 +272,7 @@ size_t window_steps_for(Entry& e, size_t T) {
         const long w = atol(v);
         if (w > 0) return size_t(w) < T ? size_t(w) : T;
     }
-    const size_t Hp = (H + 31) / 32 * 32, Ip = (I + 63) / 64 * 64;
+    const size_t Hp = size_t(flstm_core_get_info(e.plan, "hidden_padded")), Ip = size_t(flstm_core_get_info(e.plan, "input_padded"));
     const size_t per_step = B * (4 * I + 2 * Ip + 24 * Hp + 2 * H);
     size_t budget = 0;
     if (const char* v = getenv("FLASHLSTM_V2_DEVICE_BUDGET_MB")) budget = size_t(atol(v) > 0 ? atol(v) : 0) << 20;
@@ -545,7 +546,7 @@ void download_dx(Entry& e, const Streams& st, size_t k, __half* dx_host, size_t 
 void backward_window(Entry& e, const Streams& st, size_t n, const __half* dY_host, const void* d_hn, const void* d_cn,
                      flstm_dtype dstate_dtype, __half* dx_host, bool accumulate, float* dW_ih, float* dW_hh,
                      float* db_ih, float* db_hh, float* dh0, float* dc0) {
-    const size_t B = e.B, I = e.I, H = e.H;
+    const size_t B = e.B, I = e.I;
     const size_t x_bytes = n * B * I * sizeof(half_t);
     if (dx_host) e.dx_dev.reserve(x_bytes);
     check_core(flstm_core_set_option(e.plan, "accumulate_grads", accumulate ? 1 : 0), "flstm_core_set_option");

@@ -280,8 +280,8 @@ extern "C" int flstm_core_create(size_t batch, size_t input_size, size_t hidden_
     p->d.Ip = int(round_up(input_size, 64));
     p->d.Hp = int(round_up(hidden_size, hidden_size > 2048 ? 64 : 32));   // (the wide backward kernel has 64-column slices)
     // Persistent launches go through the gate of launch_persistent; FLASHLSTM_COOPERATIVE_LAUNCH=1 or the option
-    // "cooperative" sends them through hipLaunchCooperativeKernel instead (not under a rocprofiler-sdk tool: with rocprofv3
-    // attached, a process that has made a cooperative launch takes a segmentation fault inside the tool when it exits).
+    // "cooperative" sends them through hipLaunchCooperativeKernel instead (not for use under a rocprofiler-sdk tool: with
+    // rocprofv3 attached, a process that has made a cooperative launch takes a segmentation fault inside the tool when it exits).
     {
         if (const char* v = getenv("FLASHLSTM_COOPERATIVE_LAUNCH")) p->opt_cooperative = atoi(v) != 0;
         if (const char* v = getenv("FLASHLSTM_STEP_GRAPHS")) p->opt_graphs = atoi(v) != 0;

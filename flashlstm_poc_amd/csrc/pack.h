@@ -10,7 +10,7 @@ namespace flstm_hip {
 // neighbours, q = 4 * j + gate.   PyTorch row of (gate, j) is gate*H + j.
 struct Dims {
     int B, I, H;     // caller sizes
-    int Ip, Hp;      // I rounded up to 64, H rounded up to 32
+    int Ip, Hp;      // I rounded up to 64, H to 32 (above 2048: to 64)
 };
 
 // Replaces src/kernels.cu:57-84 (pack_weights_kernel) and :45-55 (combine_bias_kernel): fp32

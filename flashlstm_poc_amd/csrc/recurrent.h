@@ -34,11 +34,13 @@ struct RecLayout {
     int wide;        // more than 2048 hidden units, weights resident (rec_fwd_wide_kernel, rec_bwd_wide_kernel)
     int num_cus;     // of the device the layout was made for
     int rot_div;     // k-step rotation (rec_kstep_rotation): slices rot_div apart run on the same XCD
-    int two_d;       // backward, 2048 hidden units: workgroups split the product over output columns AND the contraction
-                     // (32 column slices x kq contraction slices, partial sums exchanged inside an XCD); nt, jb, nh
-                     // still describe the one-dimensional layout, whose weight fragments the step-wise fallback uses
-    int kq;          // two_d: contraction slices, 8 (one group of 256 workgroups) or 4 (two groups of 128)
-    int nm;          // two_d: passes per step the kernel is built for (row blocks per workgroup, rounded up to 1, 2, 4)
+    int two_d;       // backward, 2048 hidden units and more: workgroups split the product over output columns AND the
+                     // contraction (slices of 64 columns x kq contraction slices, partial sums exchanged inside an XCD); nt,
+                     // jb, nh still describe the one-dimensional layout, whose weight fragments the step-wise fallback uses
+    int kq;          // two_d: contraction slices, 8 (one group of 256 workgroups) or 4 (two groups of 128; above 2048
+                     // units one group)
+    int nm;          // two_d: passes per step the kernel is built for (row blocks per workgroup, rounded up to 1, 2, 4;
+                     // above 2048 units any number of tiles)
     int win_rows;    // two_d: 0, or the batch is walked in windows of this many rows, one persistent launch each (batch
                      // rows are independent sequences); nrb, mt, ng, nm then describe one window
     int nw;          // wavefronts per workgroup of the one-way kernels, which split the contraction between them: 4, or

@@ -32,8 +32,12 @@
 //    No wait for a store acknowledgement and no flag poll sits on the path between one step and the next.
 //    Every retry loop is bounded and reports through `status`.
 //  * Fallback.  The same kernels launched once per step (no waits, kernel boundaries order
-//    memory) serve shapes whose weights do not fit on chip, and are the safe path after a failed
-//    persistent launch.
+//    memory) serve shapes whose weights do not fit on chip (more than 4096 hidden units), and are the
+//    safe path after a failed persistent launch.
+//  * The layout above is that of the one-way kernels.  Up to 512 (forward) and 384 (backward) units the waves of a
+//    workgroup split the columns instead (rec_fwd_split_kernel, rec_bwd_pair_kernel); rec_fwd_il_kernel has eight waves and
+//    two chains; rec_bwd2d_kernel splits the product two ways at 2048 units; above that rec_fwd_wide_kernel and
+//    rec_bwd_wide_kernel hold half a megabyte of weights per workgroup.  Each says why where it stands.
 #include <atomic>
 #include <cstring>
 #include <mutex>
@@ -1799,7 +1803,8 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_wide_kernel(RecFwdArgs p, Re
         const unsigned row = unsigned(min(r, p.B - 1 - rb * 16)), cell = row * unsigned(p.Hp) + unsigned(j);
         const size_t row0 = size_t(t) * p.B + rb * 16;
         ld_at(xp, p.G + row0 * gld, cell * 8u);
-        // (this thread's own store of the step before; another tile's wait has drained it since)
+        // (MANY: this thread's own store of the step before, which another tile's wait has drained since; with one tile only a
+        // launch's first step uses it)
         ld_coherent_at(cp_bits, p.C + row0 * p.Hp, cell * 4u);
     };
     if (p.stamps && t_begin == p.t0 && hs == 0 && g == 0 && tid == 0) p.stamps[0] = wall_clock64();
