@@ -43,7 +43,6 @@ class LstmStack:
         self.B, self.I, self.H, self.L = int(batch), int(input_size), int(hidden_size), int(num_layers)
         self.layers: List[LstmCore] = [LstmCore(self.B, self.I if l == 0 else self.H, self.H) for l in range(self.L)]
         self._lib = self.layers[0].lib
-        self._plans = (ctypes.c_void_p * self.L)(*[layer._h for layer in self.layers])
         self._inputs: List = []
         self.last_loss_scale = 1.0
 
@@ -51,6 +50,11 @@ class LstmStack:
         for layer in self.layers:
             layer.close()
         self._inputs = []
+
+    def _plans(self):
+        """The layers' plans as a C array, read anew for every call: a layer that has been closed is a null pointer, which
+        the library refuses."""
+        return (ctypes.c_void_p * self.L)(*[layer._h for layer in self.layers])
 
     def pack(self, params: Sequence[Tuple]) -> None:
         """params[l] = (w_ih, w_hh, b_ih, b_hh) of layer l (fp32 CUDA tensors, torch.nn.LSTM layout)."""
@@ -79,7 +83,7 @@ class LstmStack:
         ys = [torch.empty((T, self.B, self.H), device=x.device, dtype=torch.float16) for _ in range(self.L)]
         hy = torch.empty(shape, device=x.device, dtype=torch.float16)
         cy = torch.empty_like(hy)
-        rc = self._lib.flstm_stack_forward(self._plans, self.L, T, x.data_ptr(), F16, _ptr(h0), _ptr(c0),
+        rc = self._lib.flstm_stack_forward(self._plans(), self.L, T, x.data_ptr(), F16, _ptr(h0), _ptr(c0),
                                            F16 if state is None else _dtype_code(state), _pointers(ys), F16, hy.data_ptr(),
                                            cy.data_ptr(), LstmCore._stream())
         if rc != 0:
@@ -118,7 +122,7 @@ class LstmStack:
             if loss_scale != "auto":
                 raise ValueError("loss_scale must be a positive number or 'auto'")
             amax = ctypes.c_float()
-            rc = self._lib.flstm_core_absmax(self._plans[0], dy_top.data_ptr(), dy_code, dy_top.numel(), ctypes.byref(amax), stream)
+            rc = self._lib.flstm_core_absmax(self.layers[0]._h, dy_top.data_ptr(), dy_code, dy_top.numel(), ctypes.byref(amax), stream)
             if rc != 0:
                 raise RuntimeError(f"flstm_core_absmax failed with status {rc}")
             amax = amax.value * abs(float(dy_factor))
@@ -143,7 +147,7 @@ class LstmStack:
                 raise ValueError(f"{name} must hold one tensor of shape ({B}, {H}) (or None) per layer")
             states.append(grads)
         rc = self._lib.flstm_stack_backward(
-            self._plans, self.L, T, _pointers(self._inputs), F16, dy_top.data_ptr(), dy_code, S * float(dy_factor),
+            self._plans(), self.L, T, _pointers(self._inputs), F16, dy_top.data_ptr(), dy_code, S * float(dy_factor),
             None if states[0] is None else _pointers(states[0]), None if states[1] is None else _pointers(states[1]), F32, S,
             _pointers(dxs), F16 if dxs[0] is None else _dtype_code(dxs[0]), _pointers(dW_ih), _pointers(dW_hh), _pointers(db),
             None if db2 is None else _pointers(db2), _pointers(list(dh0.unbind(0))), _pointers(list(dc0.unbind(0))), stream)
