@@ -146,6 +146,8 @@ class LstmStack:
             if grads is not None and (len(grads) != self.L or any(g is not None and tuple(g.shape) != (B, H) for g in grads)):
                 raise ValueError(f"{name} must hold one tensor of shape ({B}, {H}) (or None) per layer")
             states.append(grads)
+        for layer in self.layers:   # (a layer used on its own with accumulate_into has left it on, which a stack's pass refuses)
+            layer.set_option("accumulate_grads", 0)
         rc = self._lib.flstm_stack_backward(
             self._plans(), self.L, T, _pointers(self._inputs), F16, dy_top.data_ptr(), dy_code, S * float(dy_factor),
             None if states[0] is None else _pointers(states[0]), None if states[1] is None else _pointers(states[1]), F32, S,
