@@ -81,10 +81,11 @@ def test_gate_bookkeeping(tmp_path):
 
 
 # whole-chip recurrences from three threads, two of them on one stream: none of them may find its workgroups waiting for
-# another's (a launch that did would give up and be counted as a fallback); 96 rows of 1024 units take every CU
+# another's (a launch that did would give up and be counted as a fallback); 96 rows of 1024 units take every CU.  Or all
+# three through the one handle (2) that names another stream in every thread
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,B,H", [(40, 96, 1024), (24, 20, 2560), (30, 16, 2048)])
-def test_persistent_launches_of_several_threads_and_streams(T, B, H):
+@pytest.mark.parametrize("T,B,H,per_thread", [(40, 96, 1024, False), (24, 20, 2560, False), (30, 16, 2048, False), (40, 96, 1024, True)])
+def test_persistent_launches_of_several_threads_and_streams(T, B, H, per_thread, monkeypatch):
     import torch
     from helpers import make_problem
     from flashlstm_poc_amd import LstmCore
@@ -102,6 +103,9 @@ def test_persistent_launches_of_several_threads_and_streams(T, B, H):
     torch.cuda.synchronize()
     assert cores[0].info("persistent_fwd") == 1 and cores[0].info("persistent_bwd") == 1
     shared, other = torch.cuda.Stream(), torch.cuda.Stream()
+    if per_thread:
+        monkeypatch.setattr(LstmCore, "_stream", staticmethod(lambda: 2))
+        shared = other = torch.cuda.default_stream()
     wrong = []
 
     def work(core, stream):
