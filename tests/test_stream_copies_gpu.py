@@ -16,7 +16,8 @@ GUARD = 16   # elements in front of and behind an output
 # odd widths of x and h, single columns, rows shorter than 16 bytes, recurrence workgroups of one, two and four waves, a layer
 # that leaves none idle (128 rows of 1030 units); outputs that start at any element of 16 bytes
 @pytest.mark.parametrize("T,B,I,H,R", [(200, 32, 257, 257, 8), (130, 9, 1, 511, 3), (150, 70, 650, 129, 50), (140, 128, 1023, 40, 1),
-                                       (200, 3, 3, 5, 7), (100, 128, 65, 1030, 8), (96, 5, 33, 2049, 8)])
+                                       (200, 3, 3, 5, 7), (130, 4, 2, 1, 3), (120, 20, 650, 650, 8), (100, 64, 512, 512, 8), (100, 128, 65, 1030, 8),
+                                       (96, 5, 33, 2049, 8)])
 @pytest.mark.parametrize("shift", [0, 1, 5])
 def test_pinned_rows_of_any_width_and_alignment(T, B, I, H, R, shift, monkeypatch):
     p = make_problem(T, B, I, H, seed=T + B)
