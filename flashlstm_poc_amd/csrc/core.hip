@@ -23,10 +23,10 @@
 
 using namespace flstm_hip;
 
-// Scratch memory of flstm_core_forward_static: everything that entry point's kernels need beyond the caller's
-// tensors and the plan's packed weights (status word and seat counters, converted x rows, x-projection / gate rows,
-// state rows, exchange ring).  One array per device, owned by the code object; host code reaches it only through
-// the address hipGetSymbolAddress returns for the device that is current (static_scratch()).
+// Scratch memory of flstm_core_forward_static: what that entry point's kernels need beyond the caller's tensors and what a
+// plan has anyway (packed weights, status block, ring of the whole passes): converted x rows, x-projection / gate rows, state
+// rows, exchange ring.  One array per device, owned by the code object; host code reaches it only through the address
+// hipGetSymbolAddress returns for the device that is current (static_scratch()).
 static constexpr size_t kStaticScratchBytes = size_t(64) << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 static constexpr int kMaxDevices = 64;
@@ -127,11 +127,15 @@ struct flstm_core_plan {
     bool weights_packed = false, bias_packed = false;
     // forward state / caches
     DevBuf X16, G, Y, C, status, xch_f, xch_b;
+    // ring of the whole passes that are one launch (forward_whole): its own, because it stays ready from one to the next
+    DevBuf ring;
+    bool ring_ready = false;   // all slots but ring_base hold the 'unwritten' pattern
+    int ring_base = 0;
     size_t T_cache = 0;
     bool have_cache = false;
     // pass in progress (begin / steps / end)
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
-             half_t* y_direct = nullptr; } fw;   // y_direct: the recurrence writes the caller's y itself
+             half_t* y_direct = nullptr; bool whole = false; } fw;   // y_direct: the recurrence writes the caller's y itself; whole: one launch
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
              BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
     BesideCopies beside_f, beside_b;   // for the next recurrence launch of a pass fed in ranges (core_copy_beside)
@@ -301,7 +305,7 @@ extern "C" int flstm_core_create(size_t batch, size_t input_size, size_t hidden_
 extern "C" int flstm_core_destroy(flstm_core_plan* p) {
     if (!p) return FLSTM_E_INVALID;
     for (DevBuf& b : p->wfrag) b.release();
-    for (DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->X16, &p->G, &p->Y, &p->C,
+    for (DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->ring, &p->X16, &p->G, &p->Y, &p->C,
                       &p->status, &p->xch_f, &p->xch_b, &p->dYp, &p->dG, &p->dHn, &p->dC,
                       &p->dH0, &p->db_part, &p->dw_part, &p->prof})
         b->release();
@@ -377,7 +381,7 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
     if (!strcmp(name, "device_bytes")) {
         size_t sum = 0;
         for (const DevBuf& b : p->wfrag) sum += b.bytes;
-        for (const DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->X16, &p->G, &p->Y, &p->C,
+        for (const DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->ring, &p->X16, &p->G, &p->Y, &p->C,
                                 &p->status, &p->xch_f, &p->xch_b, &p->dYp, &p->dG, &p->dHn, &p->dC, &p->dH0, &p->db_part,
                                 &p->dw_part, &p->prof})
             sum += b->bytes;
@@ -431,6 +435,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     if (split.split) {
         FL_TRY(want(kFragFwdSplit, split, rec_fwd_ks(split, d.Hp), rec_fwd_fragments(split, d.Hp)));
         frag[kFragFwdSplit].split = split.split;
+        FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));   // (here: flstm_core_forward_static allocates nothing)
     }
     FL_TRY(want(kFragBwd, bwd, rec_bwd_ks(bwd, d.Hp), rec_bwd_fragments(bwd, d.Hp)));
     if (pair.split) FL_TRY(want(kFragBwdPair, pair, rec_bwd_ks(pair, d.Hp), rec_bwd_fragments(pair, d.Hp)));
@@ -494,7 +499,6 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     prep.to_exchange(h0, f32, size_t(d.B), d.H, d.Hp, p->xch_f.as<half_t>());
     prep.fill(p->xch_f.as<half_t>() + xslot, 3 * xslot * sizeof(half_t), 0xFFFFFFFFu);
     prep.fill(p->status.as<char>() + kSeatsOffset, kStatusBytes - kSeatsOffset, 0u);
-    if (p->static_call) prep.fill(p->status.p, kStampsOffset, 0u);   // (a borrowed status block holds whatever the last call left)
     if (p->opt_profile) prep.fill(p->prof.p, 8 * sizeof(long long), 0u);
     if (whole_x && !x_in_place(p, x_dtype))
         prep.to_half(x, x_dtype == FLSTM_F32, TB, d.I, size_t(d.I), 1.f, p->X16.as<half_t>(), TB, size_t(d.Ip));
@@ -599,15 +603,96 @@ void final_states(const flstm_core_plan* p, size_t TB, void* hy, void* cy, flstm
     out.unpad(p->C.as<float>() + TB * d.Hp, 1, size_t(d.Hp), size_t(d.B), d.H, 1.f, cy, dtype == FLSTM_F32);
 }
 
+// Whether a pass can be one launch (rec_fwd_whole_kernel): the layout is the one for short contractions.
+bool whole_possible(const flstm_core_plan* p) { return !p->opt_profile && p->ring.p && rec_whole_possible(p->Lf); }
+// ... and whether that launch forms the projection itself: the input rows are short enough for a wave to hold its part of W_ih,
+// fp16 rows used in place are aligned, and it is the faster way.  It saves a launch and G's way through memory (7 us and more)
+// and costs a step what the exchange does not hide.  Measured over 128 steps of 64 rows, us a pass without gradients, projection
+// in front / inside: 256 units 143 / 131 with 64 features, 143 / 134 with 128, 144 / 150 with 256; 384 units 195 / 157, 196 / 169,
+// 198 / 196; 512 units 213 / 194, 211 / 203, 213 / 222; but 64 units, where a step is 0.5 us, 106 / 104, 106 / 109, 107 / 123.
+bool whole_projects(const flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype) {
+    if (p->d.Ip > kRecWholeInput || (x_in_place(p, x_dtype) && reinterpret_cast<uintptr_t>(x) % 16 != 0)) return false;
+    return T <= 32 || (p->d.Ip <= 128 && (p->d.Hp >= 256 || T <= 64));
+}
+
+int forward_whole(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
+                  flstm_dtype state_dtype, void* y, flstm_dtype y_dtype, void* hy, void* cy, flstm_dtype out_state_dtype,
+                  bool save, hipStream_t s) {
+    const Dims& d = p->d;
+    const size_t TB = T * size_t(d.B), xslot = exchange_slot_halfs(d.B, d.Hp);
+    const int f32 = state_dtype == FLSTM_F32;
+    p->fw.T = T; p->fw.x = x; p->fw.x_dtype = x_dtype; p->fw.open = true; p->fw.whole = true;
+    RecWholeArgs a{};
+    OpList prep;   // what there is to do in front of it: converted rows, a ring that is not ready, an h0 no 16-byte load fits
+    const bool projects = whole_projects(p, T, x, x_dtype);
+    if (x_in_place(p, x_dtype)) {
+        a.x = static_cast<const half_t*>(x);
+        a.ldx = d.I;
+    } else {
+        FL_TRY(p->X16.reserve(TB * d.Ip * sizeof(half_t)));
+        prep.to_half(x, x_dtype == FLSTM_F32, TB, d.I, size_t(d.I), 1.f, p->X16.as<half_t>(), TB, size_t(d.Ip));
+        a.x = p->X16.as<half_t>();
+        a.ldx = d.Ip;
+    }
+    if (!p->ring_ready) {
+        p->ring_base = 0;
+        prep.fill(p->ring.as<half_t>() + xslot, 3 * xslot * sizeof(half_t), 0xFFFFFFFFu);
+    }
+    a.base = p->ring_base;
+    a.h0_in_ring = h0 && (d.H % 8 != 0 || reinterpret_cast<uintptr_t>(h0) % 16 != 0);
+    if (a.h0_in_ring) prep.to_exchange(h0, f32, size_t(d.B), d.H, d.Hp, p->ring.as<half_t>() + size_t(a.base) * xslot);
+    p->ring_ready = false;   // (until the pass is known to have gone through)
+    if (save || !projects) FL_TRY(p->G.reserve(TB * 4 * d.Hp * sizeof(half_t)));
+    if (save) {
+        FL_TRY(p->Y.reserve((TB + d.B) * d.Hp * sizeof(half_t)));
+        FL_TRY(p->C.reserve((TB + d.B) * d.Hp * sizeof(float)));
+        a.Y = p->Y.as<half_t>(); a.C = p->C.as<float>();
+    }
+    a.G = p->G.as<half_t>();
+    FL_TRY(run_ops(prep, s));
+    if (!projects) {
+        a.x = nullptr;
+        const int rc = forward_project(p, 0, T, true, s);
+        if (rc) return rc;
+    }
+    a.wfrag = p->wfrag[kFragFwdSplit].as<half8>();
+    a.wih = p->wih_p.as<half_t>(); a.bias = p->bias_p.as<float>(); a.Ip = d.Ip;
+    a.h0 = h0; a.c0 = c0; a.state_f32 = f32;
+    a.ring = p->ring.as<half_t>(); a.x_slot = xslot;
+    a.y = y; a.hy = hy; a.cy = cy;
+    a.y_f32 = y_dtype == FLSTM_F32; a.out_f32 = out_state_dtype == FLSTM_F32;
+    auto pairs = [&](const void* t, int is_f32) { return d.H % 2 == 0 && reinterpret_cast<uintptr_t>(t) % (is_f32 ? 8 : 4) == 0; };
+    a.y_pairs = pairs(y, a.y_f32); a.hy_pairs = pairs(hy, a.out_f32); a.cy_pairs = pairs(cy, a.out_f32);
+    int rc = next_seats(p, &a.seats, s);
+    if (rc) return rc;
+    p->status_host->status = 0;   // (nothing of this plan is running: every pass is waited for)
+    a.status = &p->status_host->status;
+    a.stamps = p->status_host->stamps;
+    a.B = d.B; a.H = d.H; a.Hp = d.Hp; a.T = int(T);
+    a.spin_limit = p->opt_spin_limit;
+    a.spin_ticks = (long long)p->opt_spin_ms * p->wall_khz;
+    FL_TRY(launch_rec_fwd_whole(p->Lf, a, s));
+    return 0;
+}
+
 // One whole forward pass, enqueued: projection, recurrence, outputs, status.  The outputs are written behind the
 // recurrence without waiting for its status: if the persistent launch gave up, the whole pass is repeated step-wise
 // and overwrites them.
 int forward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
                     flstm_dtype state_dtype, void* y, flstm_dtype y_dtype, void* hy, void* cy,
-                    flstm_dtype out_state_dtype, hipStream_t s) {
+                    flstm_dtype out_state_dtype, bool save, hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     use_tuned(p, T);
+    p->fw.whole = false;
+    if (whole_possible(p)) {
+        const int rc = forward_whole(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, save, s);
+        if (rc != int(hipErrorCooperativeLaunchTooLarge)) return rc;
+        p->refused_fwd = true;   // (as in forward_recur)
+        p->coop_refusals++;
+        p->fw.whole = false;
+        replan(p);
+    }
     // An fp16 output whose rows are the state rows is written by the persistent recurrence itself (no copy afterwards).
     // Step-wise launches leave it to the copy: every argument of theirs is then plan-owned, and the graph they were
     // captured into can be replayed on the next pass.
@@ -628,24 +713,29 @@ int forward_conclude(flstm_core_plan* p, hipStream_t s) {
     int st = 0;
     int rc = take_status(p, s, &st);
     if (rc) return rc;
+    if (p->fw.whole && st == 0) {
+        p->ring_base = int((size_t(p->ring_base) + p->fw.T - 1) & 3);
+        p->ring_ready = true;
+    }
     if (st != 0) {
         if (p->Lf.persistent) demote(p, true);   // workgroups not co-resident or not where expected: next time with one launch per step
         return FLSTM_E_STALLED;
     }
     pass_done(p, true);
     if (p->opt_profile) FL_TRY(hipMemcpy(p->prof_f, p->prof.p, sizeof(p->prof_f), hipMemcpyDeviceToHost));
-    p->ms_fwd[0] = elapsed(p, kStampFwdStart, kStampFwdRec);
+    const int first = p->fw.whole ? kStampFwdRec : kStampFwdStart;   // (a pass as one launch is all recurrence)
+    p->ms_fwd[0] = elapsed(p, first, kStampFwdRec);
     p->ms_fwd[1] = elapsed(p, kStampFwdRec, kStampFwdRecEnd);
-    p->ms_fwd[2] = elapsed(p, kStampFwdStart, kStampFwdRecEnd);
+    p->ms_fwd[2] = elapsed(p, first, kStampFwdRecEnd);
     p->fw.open = false;
     return 0;
 }
 
 int forward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
                  flstm_dtype state_dtype, void* y, flstm_dtype y_dtype, void* hy, void* cy,
-                 flstm_dtype out_state_dtype, hipStream_t s) {
+                 flstm_dtype out_state_dtype, bool save, hipStream_t s) {
     for (int attempt = 0;; ++attempt) {
-        int rc = forward_enqueue(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, s);
+        int rc = forward_enqueue(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, save, s);
         if (rc) return rc;
         rc = wait_stream(s);
         if (rc) return rc;
@@ -667,7 +757,7 @@ extern "C" int flstm_core_forward(flstm_core_plan* p, size_t T, const void* x, f
     if (!x || T > (size_t(1) << 24)) return FLSTM_E_INVALID;
     p->have_cache = false;
     int rc = forward_pass(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype,
-                          static_cast<hipStream_t>(stream));
+                          save_for_backward != 0, static_cast<hipStream_t>(stream));
     p->fw.open = false;   // (also when the pass failed: no range of steps may follow it)
     if (rc) return rc;
     if (save_for_backward) { p->have_cache = true; p->T_cache = T; }
@@ -698,29 +788,26 @@ extern "C" int flstm_core_forward_static(flstm_core_plan* p, size_t T, const voi
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     // the same buffers forward_setup() sizes, carved out of the static array instead of allocated
-    const size_t need[6] = {kStatusBytes,
-                            x_in_place(p, x_dtype) ? 0 : TB * d.Ip * sizeof(half_t),
+    const size_t need[5] = {x_in_place(p, x_dtype) ? 0 : TB * d.Ip * sizeof(half_t),
                             TB * 4 * d.Hp * sizeof(half_t),
                             (TB + d.B) * d.Hp * sizeof(half_t),
                             (TB + d.B) * d.Hp * sizeof(float),
                             4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)};
-    size_t off[6], total = 0;
-    for (int i = 0; i < 6; ++i) { off[i] = total; total += align256(need[i]); }
+    size_t off[5], total = align256(kStatusBytes);   // (the limit counts a status block; the plan's own is used)
+    for (int i = 0; i < 5; ++i) { off[i] = total; total += align256(need[i]); }
     if (total > kStaticScratchBytes) return FLSTM_E_TOO_LARGE;
     char* b = static_cast<char*>(base);
-    DevBuf* slot[6] = {&p->status, &p->X16, &p->G, &p->Y, &p->C, &p->xch_f};
-    DevBuf saved[6];
-    for (int i = 0; i < 6; ++i) { saved[i] = *slot[i]; *slot[i] = DevBuf::view(b + off[i], need[i]); }
+    DevBuf* slot[5] = {&p->X16, &p->G, &p->Y, &p->C, &p->xch_f};
+    DevBuf saved[5];
+    for (int i = 0; i < 5; ++i) { saved[i] = *slot[i]; *slot[i] = DevBuf::view(b + off[i], need[i]); }
     const bool had_cache = p->have_cache;
     p->have_cache = false;   // (the plan's own caches are untouched, but no pass may use the borrowed ones later)
-    // (the setup clears the status block: the array keeps whatever the last call left; step-wise launches, if the
-    // pass comes to them, are plain launches: a graph capture allocates)
+    // (step-wise launches, if the pass comes to them, are plain launches: a graph capture allocates)
     p->static_call = true;
-    rc = forward_pass(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, s);
+    rc = forward_pass(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, false, s);
     p->static_call = false;
-    p->seat_sets_left = 0;
     p->fw.open = false;   // (also when the pass failed: the next call must not find a pass in progress)
-    for (int i = 0; i < 6; ++i) *slot[i] = saved[i];
+    for (int i = 0; i < 5; ++i) *slot[i] = saved[i];
     p->have_cache = had_cache;
     return rc;
 }
@@ -1014,7 +1101,7 @@ extern "C" int flstm_stack_forward(flstm_core_plan* const* plans, int layers, si
     auto at = [](const void* base, size_t off) -> const void* { return base ? static_cast<const char*>(base) + off : nullptr; };
     auto layer = [&](int l, auto&& pass) -> int {
         return pass(plans[l], T, l == 0 ? x : ys[l - 1], l == 0 ? x_dtype : y_dtype, at(h0, l * state_in), at(c0, l * state_in),
-                    state_dtype, ys[l], y_dtype, const_cast<void*>(at(hy, l * state_out)), const_cast<void*>(at(cy, l * state_out)), y_dtype, s);
+                    state_dtype, ys[l], y_dtype, const_cast<void*>(at(hy, l * state_out)), const_cast<void*>(at(cy, l * state_out)), y_dtype, true, s);
     };
     int rc = 0;
     for (int l = 0; l < layers && rc == 0; ++l) {

@@ -85,6 +85,36 @@ struct RecFwdArgs {
     long long* prof;     // optional [8] cycle counters of workgroup 0 per phase (null = off)
 };
 
+// A whole forward pass as one launch (rec_fwd_whole_kernel).
+struct RecWholeArgs {
+    const half8* wfrag;   // as rec_fwd_split_kernel's
+    const half_t* wih;    // [4Hp][Ip] packed gate order
+    const float* bias;    // [4Hp] packed gate order
+    const half_t* x;      // [T*B] rows of ldx >= Ip halfs, 16-byte aligned, zero from the input size to Ip; null: the x-projection
+                          // + bias is in G
+    int ldx, Ip;
+    const void* h0;       // [B][H] or null (zeros)
+    const void* c0;
+    int state_f32;
+    int h0_in_ring;       // slot `base` of the ring holds h0 (else it is read from h0: rows of whole, aligned 8-element groups)
+    half_t* ring;         // 4 slots of x_slot halfs; all but slot `base` hold the 'unwritten' pattern.  Afterwards that is true of
+    size_t x_slot;        // slot (base + T - 1) % 4
+    int base;
+    half_t* Y;            // caches as in RecFwdArgs; null: they are not written
+    half_t* G;
+    float* C;
+    void* y;              // [T*B][H] or null
+    void* hy;             // [B][H] or null
+    void* cy;
+    int y_f32, out_f32, y_pairs, hy_pairs, cy_pairs;   // pairs: H is even and the tensor aligned to two elements
+    unsigned* seats;
+    int* status;          // as in RecFwdArgs; these two may be pinned host memory
+    long long* stamps;    // [kStampCount]
+    int B, H, Hp, T;
+    int spin_limit;
+    long long spin_ticks;
+};
+
 struct RecBwdArgs {
     const half8* wfrag;  // [nh][nw waves][ks][nt][64] B-fragments of W_hh^T (rows = hidden k, contraction = packed gate q)
     const half_t* G;     // activated gates cache [T*B][4Hp]
@@ -217,6 +247,11 @@ hipError_t wait_for_persistent(hipStream_t stream);
 
 // Runs steps [t0, t1). Persistent layouts use one launch; otherwise one launch per step.
 hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs = nullptr);
+// Whether a layout can run whole passes as one launch, and the largest padded input size of which that launch forms the
+// projection itself.
+bool rec_whole_possible(const RecLayout& L);
+constexpr int kRecWholeInput = 256;
+hipError_t launch_rec_fwd_whole(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream);
 // Runs steps t_hi .. t_lo (the whole pass is T-1 .. -1: all steps and the final dh0 product).
 hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs = nullptr);
 

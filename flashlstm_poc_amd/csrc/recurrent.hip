@@ -1588,6 +1588,373 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
     clk.flush();
 }
 
+// ---------------------------------------------------------------- forward, short contractions, a whole pass
+// A pass of rec_fwd_split_kernel is four launches: state rows, ring and counters; projection; recurrence; outputs.  Here it is
+// this launch alone, with one in front of it where x has to be converted, or the projection where rows are long.  Measured, us
+// a pass: one step of one row, 128 features and 256 units 37.9 -> 21.7 (6 of them the caller's Python); 128 steps of 256 units without /
+// with caches, 16 rows 142 / 142 -> 127 / 135, 512 rows 326 / 325 -> 189 / 242; of 384 units and 64 rows 205 / 205 -> 157 / 183.
+//  * KI > 0: the x-projection of a wave's 32 gate columns is formed by the wave itself.  Its part of W_ih stays in registers
+//    beside its part of W_hh; one v_mfma_f32_32x32x16 takes the 16 rows of TWO steps, so it fills the instruction, and it runs
+//    in the shadow of the exchange.  x rows are loaded 64 bytes of a row by four lanes (32 bytes by two, as the instruction
+//    wants them, took the path twice as long) and turned into operands, and the sums into this lane's cells, by swapping
+//    16- and 32-lane halves between registers.  The sums have the order and the rounding to fp16 of the GEMMs' (32x32x16,
+//    ascending k, bias last), so a pass gives the same bits as one in ranges of steps or one launch per step.
+//    KI = 0: the projection is in G, as for rec_fwd_split_kernel.
+//  * The ring is left as a pass finds it.  After T steps every slot holds the 'unwritten' pattern except the one that was read
+//    last, (T - 1) % 4, provided the last step stores nothing; the next pass starts with that slot as its own slot 0
+//    (RecWholeArgs::base), which nobody reads, because h0 comes from the caller's tensor.
+//  * Initial states are read, and outputs and final states written, in the caller's layout; the status word and the stamps go
+//    straight to pinned memory.
+// SAVE: the gate, cell and state rows that the backward pass reads are written; a pass without gradients does without them.
+// The cache stores, the output row and the projection stand between the store of h_t and the request for the next step's
+// fragments: requested right behind the store, they come back unwritten and the second request notices them a trip later (256
+// units and 64 rows 0.80 -> 0.95 us per step).
+template <int OFF>
+__device__ __forceinline__ void ld_stream_off(half8& dst, unsigned lane_off, const void* base) {
+    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3 nt" : "=v"(dst) : "v"(lane_off), "s"(base), "n"(OFF) : "memory");
+}
+template <int NR, int K>
+__device__ __forceinline__ void request_rows_one(half8 (&f)[NR], const half_t* const* group, unsigned lane_off) {
+    ld_stream_off<(K % 2) * 64>(f[K], lane_off, group[K / 2]);
+}
+template <int NR, int... K>
+__device__ __forceinline__ void request_rows(half8 (&f)[NR], const half_t* const* group, unsigned lane_off, std::integer_sequence<int, K...>) {
+    (request_rows_one<NR, K>(f, group, lane_off), ...);
+}
+// Two neighbouring values of a row of the caller's tensor; `pairs`: rows have an even number of elements and the tensor is
+// aligned to two of them.
+__device__ __forceinline__ void put_two(void* base, size_t at, int f32, bool pairs, bool first, bool second, float a, float b) {
+    if (f32) {
+        float* dst = static_cast<float*>(base) + at;
+        if (pairs) { if (first) *reinterpret_cast<floatx2*>(dst) = floatx2{a, b}; }
+        else {
+            if (first) dst[0] = a;
+            if (second) dst[1] = b;
+        }
+    } else {
+        half_t* dst = static_cast<half_t*>(base) + at;
+        if (pairs) { if (first) *reinterpret_cast<unsigned*>(dst) = pack_h2(a, b); }
+        else {
+            if (first) dst[0] = (half_t)a;
+            if (second) dst[1] = (half_t)b;
+        }
+    }
+}
+// Element `at` of a tensor of either type, or zero.
+__device__ __forceinline__ float get_one(const void* base, size_t at, int f32, bool there) {
+    if (!base || !there) return 0.f;
+    return f32 ? static_cast<const float*>(base)[at] : (float)static_cast<const half_t*>(base)[at];
+}
+// Rows of 16 lanes (0..3 of a register): a = [a0 a1 a2 a3], b = [b0 b1 b2 b3] -> a = [a0 b0 a1 b1], b = [a2 b2 a3 b3].
+__device__ __forceinline__ void interleave_rows(half8& a, half8& b) {
+    union { half8 h; unsigned u[4]; } x, y;
+    x.h = a;
+    y.h = b;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const auto v = __builtin_amdgcn_permlane16_swap(x.u[e], y.u[e], false, false);   // [a0 b0 a2 b2], [a1 b1 a3 b3]
+        const auto w = __builtin_amdgcn_permlane32_swap(v[0], v[1], false, false);
+        x.u[e] = w[0];
+        y.u[e] = w[1];
+    }
+    a = x.h;
+    b = y.h;
+}
+template <int KS, int KI, bool SAVE>
+__global__ __launch_bounds__(kThreads) void rec_fwd_whole_kernel(RecWholeArgs p, RecLayout L, int, int, int) {
+    static_assert(KS % 2 == 0 && KS <= 16 && KI % 4 == 0, "up to 512 hidden units, rows of whole 64-element groups");
+    constexpr int NG = KI / 4;            // 64-element groups of an input row
+    constexpr int NR = KI ? KI / 2 : 1;   // 32-element groups, one load per step and group
+    __shared__ int lds_abort;
+    __shared__ int lds_role[2];
+    if (threadIdx.x == 0) lds_abort = 0;
+    __syncthreads();
+    const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
+    if (!role.active) return;
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int hs = __builtin_amdgcn_readfirstlane(role.hs), g = __builtin_amdgcn_readfirstlane(role.g);
+    const int nks = p.Hp / 32, groups = p.Ip / 64;
+    const Poll poll{true, p.spin_limit, p.spin_ticks, p.status, (lds_int_t*)&lds_abort};
+    const bool leader = hs == 0 && g == 0 && tid == 0;
+    if (leader) p.stamps[kStampFwdRec] = wall_clock64();
+
+    // this wave's units j0 .. j0 + 7, this lane's two cells: row r, units j and j + 1 (as in rec_fwd_split_kernel)
+    const int j0 = hs * L.jb + wave * 8;
+    const int r = lane % 16, j = j0 + 2 * (lane / 16);
+    const int b0 = g * 16, b = b0 + r;
+    const bool live = b < p.B;
+    const unsigned row = unsigned(min(r, p.B - 1 - b0)), cell = row * unsigned(p.Hp) + unsigned(j);
+
+    half8 xa[NR], xb[NR];   // x rows of a pair of steps: lane l holds row l % 16, elements 8 * (l / 16) .. + 7 of 32
+    const unsigned lane_x = (row * unsigned(p.ldx) + 8u * unsigned(lane / 16)) * 2u;
+    auto request_x = [&](int t) __attribute__((always_inline)) {   // steps t and t + 1, as far as there are such steps
+        const half_t* group[NR];
+        auto of = [&](int tc) __attribute__((always_inline)) {
+            const half_t* base = p.x + (size_t(min(tc, p.T - 1)) * p.B + b0) * p.ldx;
+#pragma unroll
+            for (int q = 0; q < NG; ++q) group[q] = base + 64 * min(q, groups - 1);
+        };
+        of(t);
+        request_rows(xa, group, lane_x, std::make_integer_sequence<int, NR>{});
+        of(t + 1);
+        request_rows(xb, group, lane_x, std::make_integer_sequence<int, NR>{});
+    };
+    uintx4 xp[2];   // by parity of the step: i, f, g, o of this lane's units before the recurrent product
+    auto request_xp = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        ld_stream_at(xp[par], p.G + (size_t(min(t, p.T - 1)) * p.B + b0) * (size_t(4) * p.Hp), cell * 8u);
+    };
+    const std::integral_constant<int, 0> even{};
+    const std::integral_constant<int, 1> odd{};
+
+    // (the first rows through loads the compiler sees: it waits for them beside the weights)
+    if constexpr (KI > 0) {
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const half_t* src = p.x + size_t(b0) * p.ldx + lane_x / 2u + 64 * min(k / 2, groups - 1) + 32 * (k % 2);
+            xa[k] = ld_half8(src);
+            xb[k] = ld_half8(src + (p.T > 1 ? size_t(p.B) * p.ldx : 0));
+        }
+    } else {
+        const half_t* src = p.G + size_t(b0) * (size_t(4) * p.Hp) + 4u * cell;
+        xp[0] = *reinterpret_cast<const uintx4*>(src);
+        xp[1] = *reinterpret_cast<const uintx4*>(src + (p.T > 1 ? size_t(p.B) * 4 * p.Hp : 0));
+    }
+    half8 wreg[KS][2];
+    {
+        const half8* wf = p.wfrag + (size_t(hs) * L.split + wave) * size_t(KS) * 2 * kWave;
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) wreg[k][n] = wf[(k * 2 + n) * kWave + lane];
+    }
+    // W_ih: column c of the 32x32 product is gate c % 4 of unit 4 * (c / 4 % 2) + c / 8, so that lanes 0..31 end up with the
+    // units of lanes 0..31, lanes 32..63 with the others'
+    half8 win[KI ? KI : 1];
+    float bias[4][4];
+    if constexpr (KI > 0) {
+        const int c = lane % 32;
+        const half_t* src = p.wih + size_t(4 * (j0 + 4 * (c / 4 % 2) + c / 8) + c % 4) * p.Ip + 8 * (lane / 32);
+#pragma unroll
+        for (int k = 0; k < KI; ++k) win[k] = k / 4 < groups ? ld_half8(src + 16 * k) : half8{};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const floatx4 v = *reinterpret_cast<const floatx4*>(p.bias + 4 * (j0 + 4 * (lane / 32) + q));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bias[q][e] = v[e];
+        }
+    }
+    const unsigned off_ring = unsigned(xch_offset(r, j, nks));          // inside the tile, in halfs
+    const size_t tile_halfs = size_t(nks) * 512;
+    unsigned lane_off[(KS + 3) / 4], tail_off[3];   // (as in rec_fwd_split_kernel)
+#pragma unroll
+    for (int q = 0; q < (KS + 3) / 4; ++q) lane_off[q] = unsigned(lane) * 16u + unsigned(q) * 4096u;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) tail_off[q] = unsigned(lane) * 16u + unsigned(min(max(KS - 3 + q, 0), nks - 1)) * 1024u;
+
+    half8 f[KS];   // the fragments of h_{t-1}
+    auto request = [&](int t) __attribute__((always_inline)) {
+        const half_t* tile = p.ring + size_t((t + p.base) & 3) * p.x_slot + size_t(g) * tile_halfs;
+        request_split(f, tile, lane_off, tail_off, std::make_integer_sequence<int, KS>{});
+    };
+    auto arrived = [&](int t, auto younger) __attribute__((always_inline)) {   // `younger`: operations issued behind the request, at least
+        wait_set<decltype(younger)::value>(f);
+        auto unwritten = [&]() __attribute__((always_inline)) -> bool {
+            unsigned m = 0u;
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const uint4 ua = __builtin_bit_cast(uint4, f[k]);
+                m = max(m, max(max(ua.x, ua.y), max(ua.z, ua.w)));
+            }
+            return __any(m == kUnwritten) != 0;
+        };
+        if (__builtin_expect(unwritten(), 0)) {
+            int spins = 0;
+            long long spin_start = 0;
+            do {
+                if (poll_give_up(poll, spins, spin_start, lane)) leave_kernel();   // (the other waves of the group run into the same bound)
+                request(t);
+                wait_set<0>(f);
+            } while (unwritten());
+        }
+    };
+
+    // initial states: this lane's cells, and (step 0) the whole operand, rows past B and units past H zero
+    const bool unit0 = live && j < p.H, unit1 = live && j + 1 < p.H;
+    float c[2];
+    {
+        const size_t at = size_t(b) * p.H + j;
+        c[0] = get_one(p.c0, at, p.state_f32, unit0);
+        c[1] = get_one(p.c0, at + 1, p.state_f32, unit1);
+        if (SAVE && live) {
+            const float h[2] = {get_one(p.h0, at, p.state_f32, unit0), get_one(p.h0, at + 1, p.state_f32, unit1)};
+            *reinterpret_cast<floatx2*>(p.C + size_t(b0) * p.Hp + cell) = floatx2{c[0], c[1]};
+            *reinterpret_cast<unsigned*>(p.Y + size_t(b0) * p.Hp + cell) = pack_h2(h[0], h[1]);
+        }
+    }
+    if (p.h0_in_ring) {
+        request(0);
+        wait_set<0>(f);
+    } else {
+        const size_t at = size_t(b) * p.H + 8 * (lane / 16);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            f[k] = half8{};
+            if (p.h0 && live && 32 * k + 8 * (lane / 16) < p.H) {
+                if (p.state_f32) {
+                    const floatx4* src = reinterpret_cast<const floatx4*>(static_cast<const float*>(p.h0) + at + 32 * k);
+                    const floatx4 lo = src[0], hi = src[1];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) { f[k][e] = (half_t)lo[e]; f[k][4 + e] = (half_t)hi[e]; }
+                } else {
+                    f[k] = ld_half8(static_cast<const half_t*>(p.h0) + at + 32 * k);
+                }
+            }
+        }
+    }
+    loads_landed();
+
+    auto project = [&]() __attribute__((always_inline)) {   // of the rows in xa, xb
+        floatx16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+        for (int q = 0; q < NG; ++q)
+            if (q < groups) {   // (a product with the zero weights past the row would turn an infinity into a NaN)
+#pragma unroll
+                for (int k = 2 * q; k < 2 * q + 2; ++k) {
+                    interleave_rows(xa[k], xb[k]);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(win[2 * k], xa[k], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(win[2 * k + 1], xb[k], acc, 0, 0, 0);
+                }
+            }
+        unsigned v[4][2];   // unit 4 * (lane / 32) + q of row lane % 16, step lane / 16 % 2
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float z[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                z[e] = acc[4 * q + e] + bias[q][e];
+                asm volatile("" : "+v"(z[e]));   // (the sum is rounded to fp32 before it is to fp16, as in the GEMMs)
+            }
+            v[q][0] = pack_h2(z[0], z[1]);
+            v[q][1] = pack_h2(z[2], z[3]);
+        }
+        // lanes of an even row of 16 keep units 0 and 1 and take the first step, those of an odd row units 2 and 3 and the second
+        // step: what each has of the other's is swapped
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const auto w = __builtin_amdgcn_permlane16_swap(v[u][e], v[2 + u][e], false, false);
+                xp[0][2 * u + e] = w[0];
+                xp[1][2 * u + e] = w[1];
+            }
+    };
+    if constexpr (KI > 0) {
+        project();
+        request_x(2);
+    }
+
+    // The cells of step t: the product with the fragments in f, the mark for h_{t+2} (see rec_fwd_split_kernel), the update.
+    unsigned h2;
+    uintx4 act;
+    auto cells = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[k][n], f[k], acc[n], 0, 0, 0);
+        if constexpr (KI == 0) settle(xp[par]);
+        store_xch(p.ring + size_t((t + 3 + p.base) & 3) * p.x_slot + size_t(g) * tile_halfs + off_ring, Pack<2>{kUnwritten}, false);
+        float hn[2], gates[2][4];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            float z[4];
+            unpack_h2(xp[par][2 * n], z[0], z[1]);
+            unpack_h2(xp[par][2 * n + 1], z[2], z[3]);
+#pragma unroll
+            for (int gt = 0; gt < 4; ++gt) z[gt] += acc[n][gt];
+            const float ig = sigmoidf_dev(z[0]), fg = sigmoidf_dev(z[1]), og = sigmoidf_dev(z[3]);
+            float gg = tanhf_dev(z[2]);
+            settle(gg);   // (rounded to fp32 before it is to fp16, not by one instruction: the bits of the other kernels)
+            c[n] = __builtin_fmaf(fg, c[n], ig * gg);
+            hn[n] = og * tanhf_dev(c[n]);
+            gates[n][0] = ig; gates[n][1] = fg; gates[n][2] = gg; gates[n][3] = og;
+        }
+        h2 = live ? pack_h2(hn[0], hn[1]) : 0u;   // (rows past B travel as zeros)
+        if constexpr (SAVE)
+            act = uintx4{pack_h2(gates[0][0], gates[0][1]), pack_h2(gates[0][2], gates[0][3]), pack_h2(gates[1][0], gates[1][1]), pack_h2(gates[1][2], gates[1][3])};
+    };
+    auto keep = [&](int t) __attribute__((always_inline)) {   // caches for the backward pass and the output row
+        const size_t row0 = size_t(t) * p.B + b0;
+        if (SAVE && live) {
+            every_wave_here();
+            __builtin_nontemporal_store(floatx2{c[0], c[1]}, reinterpret_cast<floatx2*>(p.C + (row0 + p.B) * p.Hp + cell));
+            __builtin_nontemporal_store(h2, reinterpret_cast<unsigned*>(p.Y + (row0 + p.B) * p.Hp + cell));
+            __builtin_nontemporal_store(act, reinterpret_cast<uintx4*>(p.G + row0 * (size_t(4) * p.Hp) + 4u * cell));
+        }
+        if (p.y) {
+            float h[2];
+            unpack_h2(h2, h[0], h[1]);
+            put_two(p.y, row0 * p.H + row * unsigned(p.H) + unsigned(j), p.y_f32, p.y_pairs, unit0, unit1, h[0], h[1]);
+        }
+    };
+    // h_t goes out; then what is off the path from one step to the next; then the fragments of the next step are requested.
+    auto send = [&](int t) __attribute__((always_inline)) {
+        store_xch(p.ring + size_t((t + 1 + p.base) & 3) * p.x_slot + size_t(g) * tile_halfs + off_ring, Pack<2>{h2}, false);
+        keep(t);
+    };
+    auto publish = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        send(t);
+        if constexpr (KI > 0 && par == 1) project();
+        request(t + 1);
+        if constexpr (KI == 0) request_xp(t + 2, parity);
+        else if constexpr (par == 1) request_x(t + 3);
+    };
+    cells(0, even);
+    int t = 0;   // its cells are updated
+    for (; t + 2 < p.T; t += 2) {
+        publish(t, even);
+        // (what a step has requested beside its fragments has landed when the next step's fragments have, which are younger)
+        arrived(t + 1, std::integral_constant<int, KI == 0 ? 1 : 0>{});
+        if constexpr (KI > 0) {
+#pragma unroll
+            for (int k = 0; k < NR; ++k) { settle(xa[k]); settle(xb[k]); }
+        }
+        cells(t + 1, odd);
+        publish(t + 1, odd);
+        arrived(t + 2, std::integral_constant<int, KI == 0 ? 1 : KI>{});
+        cells(t + 2, even);
+    }
+    wait_all_vm();   // (what the last steps have requested ahead is used by nobody, but its registers must not be handed on before)
+    if constexpr (KI > 0) {
+#pragma unroll
+        for (int k = 0; k < NR; ++k) { settle(xa[k]); settle(xb[k]); }
+    } else {
+        settle(xp[0]);
+        settle(xp[1]);
+    }
+    if (t + 1 < p.T) {
+        send(t);
+        request(t + 1);
+        arrived(t + 1, std::integral_constant<int, 0>{});
+        cells(t + 1, odd);
+    }
+    keep(p.T - 1);
+    {
+        float h[2];
+        unpack_h2(h2, h[0], h[1]);
+        const size_t at = size_t(b0) * p.H + row * unsigned(p.H) + unsigned(j);
+        if (p.hy) put_two(p.hy, at, p.out_f32, p.hy_pairs, unit0, unit1, h[0], h[1]);
+        if (p.cy) put_two(p.cy, at, p.out_f32, p.cy_pairs, unit0, unit1, c[0], c[1]);
+    }
+    if (leader) p.stamps[kStampFwdRecEnd] = p.stamps[kStampFwdEnd] = wall_clock64();
+}
+
 // ---------------------------------------------------------------------- more than 2048 hidden units
 // W_hh of 4096 units is 128 MiB.  Streamed from memory every step that is 27 us forward and 90 us backward at 32 rows;
 // the chip holds 128 MiB of registers and 40 MiB of LDS, so up to 4096 units it can stay resident: 512 KiB per workgroup,
@@ -3546,6 +3913,36 @@ static hipError_t run_fwd_split(const RecLayout& L, const RecFwdArgs& a, hipStre
                             }
                             return hipSuccess;
                         });
+}
+
+template <int KS, int KI, bool SAVE>
+static hipError_t run_fwd_whole(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream) {
+    auto kernel = rec_fwd_whole_kernel<KS, KI, SAVE>;
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, kWholeCuLds, kThreads, per_cu, &device);
+    if (e != hipSuccess) return e;
+    return launch_persistent(kernel, L.grid, kWholeCuLds, stream, a, L, 0, 0, 0, per_cu[device].load(), device, L.split * kWave);
+}
+template <int KS, bool SAVE>
+static hipError_t run_fwd_whole_ki(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream) {
+    if (!a.x) return run_fwd_whole<KS, 0, SAVE>(L, a, stream);
+    if (a.Ip <= 64) return run_fwd_whole<KS, 4, SAVE>(L, a, stream);
+    if (a.Ip <= 128) return run_fwd_whole<KS, 8, SAVE>(L, a, stream);
+    return run_fwd_whole<KS, 16, SAVE>(L, a, stream);
+}
+bool rec_whole_possible(const RecLayout& L) { return L.split && L.persistent && L.xcd_local && L.mt == 1 && L.nrb <= L.ng; }
+hipError_t launch_rec_fwd_whole(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream) {
+    // what the kernel's indexing assumes
+    if (!rec_whole_possible(L) || a.T <= 0 || a.B <= 0 || a.Hp % L.jb != 0 || L.jb != 8 * L.split || L.nrb * 16 < a.B || a.H > a.Hp ||
+        (!a.x && !a.G) || (a.x && (a.Ip <= 0 || a.Ip % 64 != 0 || a.Ip > kRecWholeInput || a.ldx < a.Ip)))
+        return hipErrorInvalidValue;
+    switch (rec_fwd_ks(L, a.Hp)) {
+#define FLSTM_WHOLE_CASE(n) case n: return a.Y ? run_fwd_whole_ki<n, true>(L, a, stream) : run_fwd_whole_ki<n, false>(L, a, stream);
+        FLSTM_WHOLE_CASE(2) FLSTM_WHOLE_CASE(4) FLSTM_WHOLE_CASE(8) FLSTM_WHOLE_CASE(12) FLSTM_WHOLE_CASE(16)
+#undef FLSTM_WHOLE_CASE
+    }
+    return hipErrorInvalidValue;
 }
 
 template <int KS, int KL, int NBUF>

@@ -1,0 +1,73 @@
+"""A whole forward pass as one launch (short contractions) against the same pass as separate launches -- the option "profile"
+takes that path -- bit for bit: outputs, caches, and the gradients made from them."""
+import ctypes
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def cached(core, which, rows, dtype):
+    import torch
+    from flashlstm_poc_amd import load_library
+    ptr, ld = ctypes.c_void_p(), ctypes.c_size_t()
+    assert core.lib.flstm_core_cache_ptr(core._h, which, ctypes.byref(ptr), ctypes.byref(ld)) == 0
+    out = torch.empty(rows, ld.value, device="cuda", dtype=dtype)
+    assert load_library() is core.lib
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipMemcpy(ctypes.c_void_p(out.data_ptr()), ptr, ctypes.c_size_t(out.numel() * out.element_size()), 3) == 0
+    return out
+
+
+# one to five steps (pairs and a single one left), row tiles of 1, 16 and 17 rows, rows of less than and exactly 64, 128 and 256
+# features and of more, every length of the contraction, odd widths; T = 70 crosses the rule for few units, 33 the one for 256 features
+SHAPES = [(1, 1, 128, 256), (2, 16, 64, 64), (3, 17, 65, 33), (4, 3, 1, 1), (5, 40, 256, 512), (33, 20, 200, 130), (32, 20, 200, 130),
+          (70, 5, 128, 96), (64, 5, 128, 96), (9, 100, 300, 512), (12, 512, 20, 256), (7, 128, 64, 257), (6, 64, 129, 384), (37, 33, 100, 384)]
+
+
+@pytest.mark.parametrize("T,B,I,H", SHAPES)
+@pytest.mark.parametrize("dtype,state", [("f16", "f16"), ("f32", "f32"), ("f16", None), ("f32", "f16")])
+def test_whole_pass_gives_the_bits_of_separate_launches(T, B, I, H, dtype, state):
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    types = {"f16": torch.float16, "f32": torch.float32}
+    g = torch.Generator(device="cuda").manual_seed(T * 1000 + H)
+    uniform = lambda *s: (torch.rand(*s, generator=g, device="cuda") * 2 - 1) * H ** -0.5
+    normal = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    core = LstmCore(B, I, H)
+    core.pack(uniform(4 * H, I), uniform(4 * H, H), uniform(4 * H), uniform(4 * H))
+    x, dy = normal(T, B, I).to(types[dtype]), normal(T, B, H).to(types[dtype])
+    h0 = c0 = None
+    if state:
+        h0, c0 = normal(B, H).to(types[state]), normal(B, H).to(types[state])
+
+    def passed(save, want_y=True):
+        out = list(core.forward(x, h0, c0, save_for_backward=save, want_y=want_y))
+        if save:
+            out += [cached(core, 0, (T + 1) * B, torch.float16), cached(core, 1, (T + 1) * B, torch.float32), cached(core, 2, T * B, torch.float16)]
+            out += list(core.backward(x, dy))
+        return out
+
+    core.set_option("profile", 1)
+    want = passed(True)
+    core.set_option("profile", 0)
+    for save, want_y in ((True, True), (False, True), (True, False), (True, True), (False, True)):   # (each leaves the ring to the next)
+        for k, (a, b) in enumerate(zip(passed(save, want_y), want)):
+            assert a is None or torch.equal(a, b), (save, k)
+    assert core.info("fallbacks") == 0
+    core.close()
+
+
+def test_whole_passes_of_a_plan_whose_launch_gave_up():
+    """A pass that gives up leaves the ring in no known state: the next one prepares it anew."""
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    core = LstmCore(16, 64, 128)
+    core.pack(*(torch.randn(*s, device="cuda") * 0.1 for s in ((512, 64), (512, 128), (512,), (512,))))
+    x = torch.randn(11, 16, 64, device="cuda").half()
+    want = core.forward(x)
+    core.set_option("inject_stall", 1)
+    for _ in range(12):   # repeated step-wise, demoted for eight passes, whole again
+        assert all(torch.equal(a, b) for a, b in zip(core.forward(x), want))
+    assert core.info("demotions_fwd") == 1 and core.info("hold_fwd") == 0 and core.info("persistent_fwd") == 1
+    core.close()
