@@ -84,7 +84,7 @@ struct BwdScales {
 // launches several (ranges of steps, windows of rows) takes the sets its setup has zeroed one after the other.
 constexpr size_t kStampsOffset = 64, kSeatsOffset = 256;
 constexpr int kSeatSets = 64;
-constexpr int kSeatWords = 16;   // eight seat counters, the ticket counter of BesideCopies, padding
+constexpr int kSeatWords = 32;   // eight seat counters, the ticket counters of BesideCopies (one) and, from word 16 on, ProjectBeside (eight)
 constexpr size_t kStatusBytes = kSeatsOffset + size_t(kSeatSets) * kSeatWords * sizeof(unsigned);
 static_assert(kStampsOffset + kStampCount * sizeof(long long) <= kSeatsOffset, "stamps fit in front of the seats");
 
@@ -138,6 +138,9 @@ struct flstm_core_plan {
              half_t* y_direct = nullptr; bool whole = false; } fw;   // y_direct: the recurrence writes the caller's y itself; whole: one launch
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
              BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
+    DevBuf tile_words;         // ProjectBeside::ready
+    unsigned tile_mark = 0;    // ... of the last launch
+    ProjectBeside project;     // for the next forward recurrence launch
     BesideCopies beside_f, beside_b;   // for the next recurrence launch of a pass fed in ranges (core_copy_beside)
     // backward scratch
     DevBuf dYp, dG, dHn, dC, dH0, db_part, dw_part, prof, part_b;
@@ -305,7 +308,7 @@ extern "C" int flstm_core_create(size_t batch, size_t input_size, size_t hidden_
 extern "C" int flstm_core_destroy(flstm_core_plan* p) {
     if (!p) return FLSTM_E_INVALID;
     for (DevBuf& b : p->wfrag) b.release();
-    for (DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->ring, &p->X16, &p->G, &p->Y, &p->C,
+    for (DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->ring, &p->tile_words, &p->X16, &p->G, &p->Y, &p->C,
                       &p->status, &p->xch_f, &p->xch_b, &p->dYp, &p->dG, &p->dHn, &p->dC,
                       &p->dH0, &p->db_part, &p->dw_part, &p->prof})
         b->release();
@@ -381,7 +384,7 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
     if (!strcmp(name, "device_bytes")) {
         size_t sum = 0;
         for (const DevBuf& b : p->wfrag) sum += b.bytes;
-        for (const DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->ring, &p->X16, &p->G, &p->Y, &p->C,
+        for (const DevBuf* b : {&p->wih_p, &p->wih_t, &p->part_b, &p->bias_p, &p->ring, &p->tile_words, &p->X16, &p->G, &p->Y, &p->C,
                                 &p->status, &p->xch_f, &p->xch_b, &p->dYp, &p->dG, &p->dHn, &p->dC, &p->dH0, &p->db_part,
                                 &p->dw_part, &p->prof})
             sum += b->bytes;
@@ -509,36 +512,74 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     return 0;
 }
 
-// x rows of steps [t0, t0+n) -> fp16 operand -> x-projection (+ bias) in G
-int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, hipStream_t s) {
+// x rows of steps [t0, t0+n) as the projection's fp16 operand
+int forward_operand(flstm_core_plan* p, size_t t0, size_t n, bool converted, hipStream_t s, const half_t** A, size_t* lda) {
     const Dims& d = p->d;
-    const half_t* A = nullptr;   // first row of step t0
-    size_t lda = 0;
     if (x_in_place(p, p->fw.x_dtype)) {
-        A = static_cast<const half_t*>(p->fw.x) + t0 * d.B * d.I;
-        lda = size_t(d.I);
-    } else {
-        const size_t esz = p->fw.x_dtype == FLSTM_F32 ? 4 : 2;
-        const char* src = static_cast<const char*>(p->fw.x) + t0 * d.B * d.I * esz;
-        half_t* dst = p->X16.as<half_t>() + t0 * d.B * d.Ip;
-        if (!converted) {
-            OpList conv;
-            conv.to_half(src, p->fw.x_dtype == FLSTM_F32, n * d.B, d.I, size_t(d.I), 1.f, dst, n * d.B, size_t(d.Ip));
-            FL_TRY(run_ops(conv, s));
-        }
-        A = dst;
-        lda = size_t(d.Ip);
+        *A = static_cast<const half_t*>(p->fw.x) + t0 * d.B * d.I;
+        *lda = size_t(d.I);
+        return 0;
     }
+    const size_t esz = p->fw.x_dtype == FLSTM_F32 ? 4 : 2;
+    const char* src = static_cast<const char*>(p->fw.x) + t0 * d.B * d.I * esz;
+    half_t* dst = p->X16.as<half_t>() + t0 * d.B * d.Ip;
+    if (!converted) {
+        OpList conv;
+        conv.to_half(src, p->fw.x_dtype == FLSTM_F32, n * d.B, d.I, size_t(d.I), 1.f, dst, n * d.B, size_t(d.Ip));
+        FL_TRY(run_ops(conv, s));
+    }
+    *A = dst;
+    *lda = size_t(d.Ip);
+    return 0;
+}
+
+// Whether the projection of n steps is formed beside their recurrence (ProjectBeside) by the workgroups without a seat there:
+// estimated microseconds of both ways.  A tile of 128 x 128 takes one of them 0.65 us per 64 features (what three slabs in flight
+// bring in) and 2.5, and the recurrence starts a tile later; in front of it the product takes what gemm_nt_cost says, a launch and
+// a gap.  Measured, us a forward pass, in front / beside: 512 steps of 64 rows, 1024 features and units 1275 / 990, of 16 rows of 2048
+// 1443 / 1208, of 64 rows of 640 units and 2048 features 1316 / 956; 128 steps of the first 347 / 292, 32 steps 130 / 116; where the
+// line is drawn: 32 steps of 32 rows of 1536 units, 1024 features (64 workgroups to form it) 128 / 138, 512 steps of them 1439 / 1280.
+bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
+    const Dims& d = p->d;
+    const int helpers = rec_projecting_workgroups(p->Lf);
+    if (helpers < 16 || p->opt_profile || reinterpret_cast<uintptr_t>(A) % 16 != 0) return false;
+    const double tile = d.Ip / 64 * 0.65 + 2.5, rounds = double(ceil_div(ceil_div(n * d.B, 128) * (4 * d.Hp / 128), size_t(helpers)));
+    const double recurrence = (d.Hp <= 1024 ? 1.9 : 2.4) * double(n);
+    const double in_front = recurrence + gemm_nt_cost(int(n * d.B), 4 * d.Hp, d.Ip) + 5.0;
+    return std::fmax(recurrence, rounds * tile) + 1.5 * tile + 2.0 < in_front;
+}
+
+// x rows of steps [t0, t0+n) -> fp16 operand -> x-projection (+ bias) in G, or left to the recurrence's launch
+int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, bool may_leave_it, hipStream_t s) {
+    const Dims& d = p->d;
+    GemmNT g{};
+    int rc = forward_operand(p, t0, n, converted, s, &g.A, &g.lda);
+    if (rc) return rc;
     // The hoisted input projection, one product over all steps.  Cutting it into chunks of time steps (the reference's
     // projchunksz, option "proj_chunk") saves no memory here, where the gate rows of the whole pass are kept, and changes
     // no result; chunks of 64 steps of 32 rows at 1024 units took 32 launches of 24.5 us where one product takes 410 us.
-    GemmNT g{};
-    g.A = A; g.lda = lda;
     g.B = p->wih_p.as<half_t>(); g.ldb = size_t(d.Ip);
     g.M = int(n * d.B); g.N = 4 * d.Hp; g.K = d.Ip;
     g.C16 = p->G.as<half_t>() + t0 * d.B * 4 * d.Hp; g.C32 = nullptr; g.ldc = size_t(4) * d.Hp;
     g.alpha = 1.f; g.splits = 1; g.split_stride = 0;
     g.bias = p->bias_p.as<float>();   // b_ih + b_hh, packed gate order: the recurrence reads x-projection + bias
+    p->project = ProjectBeside{};
+    if (may_leave_it && projects_beside(p, n, g.A)) {
+        const size_t words = ceil_div(size_t(g.M), 128) * (g.N / 128) * sizeof(unsigned);
+        if (words <= p->tile_words.bytes || !p->static_call) {
+            if (words > p->tile_words.bytes || p->tile_mark == ~0u) {
+                FL_TRY(p->tile_words.reserve(words));
+                FL_TRY(fill_zero(p->tile_words.p, p->tile_words.bytes, s));
+                p->tile_mark = 0;
+            }
+            p->project.A = g.A; p->project.lda = g.lda; p->project.B = g.B; p->project.bias = g.bias; p->project.C = g.C16;
+            p->project.M = g.M; p->project.N = g.N; p->project.K = g.K;
+            p->project.ready = p->tile_words.as<unsigned>();
+            p->project.mark = ++p->tile_mark;
+            rec_share_columns(p->Lf, p->project);
+            return 0;
+        }
+    }
     FL_TRY(launch_gemm_nt(g, s));
     return 0;
 }
@@ -565,6 +606,9 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     int rc = next_seats(p, &a.seats, s);
     if (rc) return rc;
     take_beside(p->beside_f, a);
+    a.project = p->project;
+    a.project.ticket = a.seats + 16;
+    p->project = ProjectBeside{};
     a.B = d.B; a.Hp = d.Hp; a.T = int(p->fw.T); a.t0 = int(t0); a.t1 = int(t0 + n);
     a.spin_limit = p->opt_spin_limit;
     a.spin_ticks = (long long)p->opt_spin_ms * p->wall_khz;
@@ -582,6 +626,11 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
         for (int i = 0; i < a.beside.count; ++i) copies.op[copies.count++] = a.beside.op[i];
         a.beside.count = 0;
         FL_TRY(run_ops(copies, s));
+        if (a.project.M != 0) {
+            rc = forward_project(p, t0, n, true, false, s);
+            if (rc) return rc;
+            a.project = ProjectBeside{};
+        }
         e = launch_rec_fwd(p->Lf, a, s, nullptr);
     }
     FL_TRY(e);
@@ -592,7 +641,7 @@ int forward_once(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtyp
                  const void* c0, flstm_dtype state_dtype, hipStream_t s) {
     int rc = forward_setup(p, T, x, x_dtype, h0, c0, state_dtype, true, s);
     if (rc) return rc;
-    rc = forward_project(p, 0, T, true, s);
+    rc = forward_project(p, 0, T, true, true, s);
     if (rc) return rc;
     return forward_recur(p, 0, T, s);
 }
@@ -652,7 +701,7 @@ int forward_whole(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     FL_TRY(run_ops(prep, s));
     if (!projects) {
         a.x = nullptr;
-        const int rc = forward_project(p, 0, T, true, s);
+        const int rc = forward_project(p, 0, T, true, false, s);
         if (rc) return rc;
     }
     a.wfrag = p->wfrag[kFragFwdSplit].as<half8>();
@@ -1203,7 +1252,7 @@ extern "C" int flstm_core_forward_steps(flstm_core_plan* p, size_t t0, size_t ns
     if (!p || !p->fw.open || t0 + nsteps > p->fw.T) return FLSTM_E_INVALID;
     if (nsteps == 0) return 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int rc = forward_project(p, t0, nsteps, false, s);
+    int rc = forward_project(p, t0, nsteps, false, false, s);
     if (rc) return rc;
     return forward_recur(p, t0, nsteps, s);
 }

@@ -41,6 +41,7 @@ int gemm_tn_auto_splits(int M, int N1, int N2, int K, int max_splits);
 // The kernels for products that do not fill the chip with 256 x 256 tiles (gemm_tile.hip): the tile size the launchers
 // above take for a product (64, 128 or 256), and the split count for it (a TN product with fp32 partials).
 int gemm_nt_tile_size(int M, int N, int K);
+double gemm_nt_cost(int M, int N, int K);   // estimated microseconds of an NT product on 256 CUs
 int gemm_tn_tile_size(int M, int N1, int N2, int K, int splits);
 int gemm_tn_plan_splits(int M, int N1, int N2, int K, int max_splits);
 hipError_t launch_gemm_nt_tile(const GemmNT& g, int tile, hipStream_t stream);

@@ -12,31 +12,10 @@
 // slab: wait for this wave's copies of slab k, barrier (everybody's copies have landed and everybody is done with slab
 // k - 1), request slab k + ST - 1 into the buffer of slab k - 1, multiply slab k.  The finished tile is turned through
 // LDS so that rows leave in whole lines whatever their pitch.
-#include "gemm.h"
+#include "gemm_tile_device.h"
 
 namespace flstm_hip {
 namespace {
-
-constexpr int BK = 64;
-constexpr int kTileThreads = 256;
-
-typedef __attribute__((address_space(3))) char lds_char;
-
-// 1 KiB from (base + lane_off) into LDS at lds_block, lane l to byte 16 * l.  Issued by hand, so that the compiler does
-// not wait for it in front of LDS reads of other buffers; the kernels' own waits and barriers order copies and reads.
-__device__ __forceinline__ void copy_1k(const char* base, unsigned lane_off, char* lds_block) {
-    const unsigned m = unsigned(reinterpret_cast<unsigned long>((lds_char*)(lds_block)));
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :: "v"(lane_off), "s"(base), "s"(m) : "m0", "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_copies() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void barrier_here() {
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 
 // Workgroup -> tile.  Workgroups are dealt round-robin to the 8 XCDs; each XCD gets a contiguous run of tiles, walked
 // in bands of four tile rows, so that the workgroups that share an L2 share operand panels.
@@ -73,35 +52,7 @@ __device__ __forceinline__ void store_rows(const T* stage, T* dst, size_t ldc, i
     }
 }
 
-// fma in fp32, then one rounding to fp16 (as in gemm.hip: the same bits whichever kernel forms an element)
-__device__ __forceinline__ half_t round16(float alpha, float acc, float bias) {
-    float v = __builtin_fmaf(alpha, acc, bias);
-    asm volatile("" : "+v"(v));
-    return (half_t)v;
-}
-
-// Accumulators of a wave -> the staged tile.  Register r of MFMA tile (i, j) holds row i*32 + lane%32, column
-// j*32 + 8*(r/4) + 4*(lane/32) + r%4 of the wave's part (operands swapped, D = B * A^T).
-template <int MI, int PITCH>
-__device__ __forceinline__ void stage16(half_t* stage, const floatx16 (&acc)[MI][MI], float alpha, const float* bias, int n0,
-                                        int N, int row, int col, int lane) {
-#pragma unroll
-    for (int j = 0; j < MI; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int c = col + j * 32 + 8 * q + 4 * (lane / 32);
-            float b[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) b[e] = (bias && n0 + c + e < N) ? bias[n0 + c + e] : 0.f;
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                half4 v;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = round16(alpha, acc[i][j][4 * q + e], b[e]);
-                *reinterpret_cast<half4*>(stage + (row + i * 32 + lane % 32) * PITCH + c) = v;
-            }
-        }
-}
+// (stage16's counterpart for fp32 outputs)
 template <int MI, int PITCH>
 __device__ __forceinline__ void stage32(float* stage, const floatx16 (&acc)[MI][MI], float alpha, const float* bias, int n0,
                                         int N, int row, int col, int lane) {
@@ -129,13 +80,10 @@ constexpr size_t tile_lds_bytes() {
     return slabs > stage ? slabs : stage;
 }
 
-// C[M][N] = alpha * A[M][K] * B[N][K]^T (+ bias).  LDS rows of 128 bytes, 16-byte chunk c of row r at c ^ (r/2) % 8 (as
-// in gemm_nt_stream).
+// C[M][N] = alpha * A[M][K] * B[N][K]^T (+ bias), see nt_tile_product.
 template <int TM, int ST>
 __global__ __launch_bounds__(kTileThreads) void gemm_nt_tile(GemmNT g, int tiles_m, int tiles_n) {
     constexpr int MI = TM / 64;                    // 32 x 32 MFMA tiles per wave and direction
-    constexpr int OPERAND = TM * BK * 2, SLAB = 2 * OPERAND;
-    constexpr int CP = TM / 32;                    // copies per wave, operand and slab
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -144,65 +92,9 @@ __global__ __launch_bounds__(kTileThreads) void gemm_nt_tile(GemmNT g, int tiles
     tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * TM, n0 = tn * TM, nk = g.K / BK;
 
-    // copy i of this wave fills rows 8 * (wave * CP + i) .. +7: lane l lands at row l / 8, chunk position l % 8
-    unsigned off_a[CP], off_b[CP];
-#pragma unroll
-    for (int i = 0; i < CP; ++i) {
-        const int r = 8 * (wave * CP + i) + lane / 8;
-        const unsigned chunk = unsigned((lane % 8) ^ ((r >> 1) & 7)) * 16u;
-        off_a[i] = unsigned(min(m0 + r, g.M - 1) - m0) * unsigned(g.lda * 2) + chunk;
-        off_b[i] = unsigned(min(n0 + r, g.N - 1) - n0) * unsigned(g.ldb * 2) + chunk;
-    }
-    const char* src_a = reinterpret_cast<const char*>(g.A + size_t(m0) * g.lda);
-    const char* src_b = reinterpret_cast<const char*>(g.B + size_t(n0) * g.ldb);
-    auto request = [&](int k) {
-        char* dst = lds + (k % ST) * SLAB + wave * CP * 1024;
-#pragma unroll
-        for (int i = 0; i < CP; ++i) {
-            copy_1k(src_a + size_t(k) * (BK * 2), off_a[i], dst + i * 1024);
-            copy_1k(src_b + size_t(k) * (BK * 2), off_b[i], dst + OPERAND + i * 1024);
-        }
-    };
-
     const int wm = wave / 2, wn = wave % 2;
-    const int a_frag = (wm * 32 * MI + lane % 32) * (BK * 2), b_frag = OPERAND + (wn * 32 * MI + lane % 32) * (BK * 2);
-    int pos[BK / 16];
-#pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) pos[kk] = ((2 * kk + lane / 32) ^ ((lane % 32) >> 1 & 7)) * 16;
-
     floatx16 acc[MI][MI];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < MI; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-#pragma unroll
-    for (int k = 0; k < ST - 1; ++k)
-        if (k < nk) request(k);
-    for (int k = 0; k < nk; ++k) {
-        // (near the end fewer slabs are in flight than the count allows for: everything is awaited)
-        if (k + ST - 2 < nk) wait_copies<(ST - 2) * 2 * CP>();
-        else wait_copies<0>();
-        barrier_here();
-        if (k + ST - 1 < nk) request(k + ST - 1);
-        const char* st = lds + (k % ST) * SLAB;
-#pragma unroll
-        for (int kk = 0; kk < BK / 16; ++kk) {
-            half8 af[MI], bf[MI];
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                af[i] = *reinterpret_cast<const half8*>(st + a_frag + i * 32 * BK * 2 + pos[kk]);
-                bf[i] = *reinterpret_cast<const half8*>(st + b_frag + i * 32 * BK * 2 + pos[kk]);
-            }
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < MI; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], acc[i][j], 0, 0, 0);
-        }
-    }
+    nt_tile_product<TM, ST>(acc, lds, g.A + size_t(m0) * g.lda, g.lda, g.M - m0, g.B + size_t(n0) * g.ldb, g.ldb, g.N - n0, nk, wave, lane);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     barrier_here();   // the slabs are done with: their LDS takes the tile
     const int rows = min(TM, g.M - m0), cols = min(TM, g.N - n0);
@@ -391,13 +283,17 @@ static double big_cost(long blocks_of_32, double slabs, bool ragged) {
 }
 static double tiles_of(int M, int N, int T) { return double((M + T - 1) / T) * double((N + T - 1) / T); }
 
-int gemm_nt_tile_size(int M, int N, int K) {
+static double nt_cost(int M, int N, int K, int tile) {
     const double nk = double(K) / BK;
-    const double c64 = tiles_cost(tiles_of(M, N, 64), nk, 2.5, 0.27, 0.22, 0.5);
-    const double c128 = tiles_cost(tiles_of(M, N, 128), nk, 3.0, 0.78, 0.62, 1.6);
-    const double c256 = big_cost(gemm_blocks_of_32(M, N, 0), nk, M % 256 != 0 || N % 256 != 0);
+    if (tile == 64) return tiles_cost(tiles_of(M, N, 64), nk, 2.5, 0.27, 0.22, 0.5);
+    if (tile == 128) return tiles_cost(tiles_of(M, N, 128), nk, 3.0, 0.78, 0.62, 1.6);
+    return big_cost(gemm_blocks_of_32(M, N, 0), nk, M % 256 != 0 || N % 256 != 0);
+}
+int gemm_nt_tile_size(int M, int N, int K) {
+    const double c64 = nt_cost(M, N, K, 64), c128 = nt_cost(M, N, K, 128), c256 = nt_cost(M, N, K, 256);
     return c64 <= c128 && c64 <= c256 ? 64 : (c128 <= c256 ? 128 : 256);
 }
+double gemm_nt_cost(int M, int N, int K) { return nt_cost(M, N, K, gemm_nt_tile_size(M, N, K)); }
 
 static double tn_cost(int M, int N1, int N2, int K, int splits, int tile) {
     const double nk = double(((K + BK - 1) / BK + splits - 1) / splits);

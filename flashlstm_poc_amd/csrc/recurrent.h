@@ -61,6 +61,21 @@ struct BesideCopies {
     unsigned* ticket = nullptr;   // zeroed before the launch
 };
 
+// The x-projection of a forward launch's steps, formed beside them by the workgroups without a seat (project_beside in
+// recurrent.hip): tiles of 128 x 128 in the order of the steps, each announced by a word that the recurrence waits for.
+struct ProjectBeside {
+    const half_t* A = nullptr;   // M rows of K halfs (pitch lda): x from the launch's first step on
+    size_t lda = 0;
+    const half_t* B = nullptr;   // [N][K]: W_ih, packed gate order
+    const float* bias = nullptr; // [N]
+    half_t* C = nullptr;         // [M][N]: the gate rows
+    int M = 0, N = 0, K = 0;     // N a multiple of 128, K of 64; M = 0: nothing to form
+    unsigned* ready = nullptr;   // [N / 128][tiles of 128 rows]: `mark` once the tile is there; holds no such word before the launch
+    unsigned mark = 0;
+    unsigned* ticket = nullptr;  // [8] zeroed before the launch
+    unsigned char first[9] = {}; // columns of tiles [first[x], first[x + 1]) are XCD x's to begin with (rec_share_columns)
+};
+
 struct RecFwdArgs {
     const half8* wfrag;  // [nh][nw waves][ks][nt][64 lanes] MFMA B-fragments of W_hh (packed gate order)
     half_t* Y;           // [(T+1)*B][Hp]; rows [0,B) = h0, rows [(t+1)B, (t+2)B) = h_t (row-major, for later kernels)
@@ -79,6 +94,7 @@ struct RecFwdArgs {
     int B, Hp, T;
     int t0, t1;          // steps [t0, t1) of the sequence are run by this call (state and ring carry over)
     BesideCopies beside;
+    ProjectBeside project;
     long long* stamps;   // optional [2]: when the pass's first launch started and its last one ended (workgroup of group 0, slice 0)
     int spin_limit;      // reloads of a fragment chunk that still shows the 'unwritten' pattern before giving up
     long long spin_ticks;   // the same bound as time: ticks of the device's constant-rate wall clock
@@ -239,6 +255,10 @@ int rec_bwd_ks(const RecLayout& L, int Hp);
 // Idle workgroups that a launch with this layout can give to BesideCopies (0: step-wise, or every CU has work), and the
 // threads of one.
 int rec_idle_workgroups(const RecLayout& L);
+// ... and that it can give to ProjectBeside.
+int rec_projecting_workgroups(const RecLayout& L);
+// Deals the columns of tiles to the XCDs by the workgroups without a seat that each is expected to have.
+void rec_share_columns(const RecLayout& L, ProjectBeside& w);
 int rec_threads(const RecLayout& L);
 
 // Waits for a stream that persistent launches went to.  Launches on other streams no longer need to be ordered behind them

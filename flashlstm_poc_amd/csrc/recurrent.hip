@@ -44,6 +44,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "gemm_tile_device.h"
 #include "launch_gate.h"
 #include "layout_device.h"
 #include "recurrent.h"
@@ -802,6 +803,10 @@ __device__ __forceinline__ void ld_stream(unsigned& d, const void* p) {
 __device__ __forceinline__ void ld_stream(uintx4& d, const void* p) {
     asm volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(d) : "v"(p) : "memory");
 }
+// (past the L2's copies as well: rows that another CU may have written during this launch, see project_beside)
+__device__ __forceinline__ void ld_stream_fresh(uintx4& d, const void* p) {
+    asm volatile("global_load_dwordx4 %0, %1, off sc1 nt" : "=v"(d) : "v"(p) : "memory");
+}
 __device__ __forceinline__ void ld_stream(floatx4& d, const void* p) {
     asm volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(d) : "v"(p) : "memory");
 }
@@ -880,6 +885,72 @@ struct FirstRequestDelay {
     }
 };
 
+// ---------------------------------------------------------------- the x-projection beside the recurrence
+// A forward recurrence that seats half of the CUs (64 rows of 1024 units, 16 of 2048) had the projection in front of it, a fifth
+// of the pass on a chip that was then half idle.  The workgroups without a seat form it while the recurrence runs, in the order
+// of the steps; the recurrence starts when the first tiles are there.  Tiles of 128 x 128 with three slabs requested ahead: a
+// CU that has one workgroup covers a slab's latency by itself.  The tile leaves in device-scope stores, its word behind
+// them; the recurrence reads gate rows past its own L2's copies (sc1), as it reads the ring.
+constexpr int kBesideTile = 128, kBesideSlabs = 4;
+constexpr size_t kBesideLds = size_t(kBesideSlabs) * 2 * kBesideTile * BK * 2;
+__device__ __forceinline__ void project_beside(const ProjectBeside& w, char* lds, int* lds_ticket) {
+    if (w.M == 0) return;
+    constexpr int TM = kBesideTile, MI = TM / 64, PITCH = TM + 8;
+    static_assert(size_t(TM) * PITCH * 2 <= kBesideLds, "the finished tile is turned through the slabs' LDS");
+    const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int tiles_m = (w.M + TM - 1) / TM, home = int(xcc_id()) & 7;
+    for (int turn = 0; turn < 8;) {   // its own XCD's columns, then what is left of the others'
+        const int owner = (home + turn) % 8, columns = w.first[owner + 1] - w.first[owner];
+        __syncthreads();
+        if (tid == 0) *lds_ticket = columns ? int(__hip_atomic_fetch_add(w.ticket + owner, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) : 0;
+        __syncthreads();
+        const int tile = __builtin_amdgcn_readfirstlane(*lds_ticket);
+        if (tile >= tiles_m * columns) {
+            ++turn;
+            continue;
+        }
+        const int tm = tile / columns, tn = w.first[owner] + tile % columns, rows = min(TM, w.M - tm * TM);
+        floatx16 acc[MI][MI];
+        nt_tile_product<TM, kBesideSlabs, true>(acc, lds, w.A + size_t(tm) * TM * w.lda, w.lda, rows, w.B + size_t(tn) * TM * w.K, size_t(w.K), TM,
+                                          w.K / BK, wave, lane);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        barrier_here();   // the slabs are done with: their LDS takes the tile
+        half_t* stage = reinterpret_cast<half_t*>(lds);
+        stage16<MI, PITCH>(stage, acc, 1.f, w.bias, tn * TM, w.N, wave / 2 * 32 * MI, wave % 2 * 32 * MI, lane);
+        __syncthreads();
+        half_t* dst = w.C + size_t(tm) * TM * w.N + size_t(tn) * TM;
+#pragma unroll
+        for (int i = 0; i < TM * TM / 8 / kThreads; ++i) {
+            const int r = (i * kThreads + tid) / (TM / 8), c = tid % (TM / 8) * 8;
+            if (r < rows) store_xch16(dst + size_t(r) * w.N + c, *reinterpret_cast<const uintx4*>(stage + r * PITCH + c), true);
+        }
+        wait_all_vm();
+        __syncthreads();
+        if (tid == 0) __hip_atomic_store(w.ready + size_t(tn) * tiles_m + tm, w.mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+// The recurrence's side of it: rows of the launch, counted from its first, whose gate columns [col, col + 128) are there.
+struct ProjectedRows {
+    int there;
+    __device__ __forceinline__ explicit ProjectedRows(const ProjectBeside& w) : there(w.M == 0 ? 0x7FFFFFFF : 0) {}
+    __device__ __forceinline__ void wait_for(int rows, const ProjectBeside& w, int col, const Poll& poll, int lane) {
+        if (__builtin_expect(rows <= there, 1)) return;
+        const int tiles_m = (w.M + kBesideTile - 1) / kBesideTile;
+        const unsigned* words = w.ready + size_t(col / kBesideTile) * tiles_m;
+        int spins = 0;
+        long long spin_start = 0;
+        for (;;) {   // 64 tiles at a look: the workgroups that form them run ahead, so the looks become rare
+            const int first = there / kBesideTile;
+            const unsigned v = __hip_atomic_load(words + min(first + lane, tiles_m - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const u64 missing = __ballot(v != w.mark);
+            const int more = missing ? __builtin_ctzll(missing) : 64;
+            there = int(min((long long)w.M, (long long)(first + more) * kBesideTile));
+            if (rows <= there) return;
+            if (more == 0 && poll_give_up(poll, spins, spin_start, lane)) return;   // (the workgroup leaves at its next barrier)
+        }
+    }
+};
+
 // ------------------------------------------------------------------------------------ forward
 // Per step and row block: K-split MFMA product on h_{t-1} as it arrives -> partial sums through LDS
 // (two buffers, one barrier per step) -> pointwise cell update -> store h_t -> store c_t and the
@@ -920,6 +991,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
     const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
     if (!role.active) {
         copy_beside(p.beside, lds_role);
+        if constexpr (RESIDENT) project_beside(p.project, reinterpret_cast<char*>(part_all), lds_role);
         return;
     }
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
@@ -961,7 +1033,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
             const int b = min(rb * RB + pr + 16 * ph, p.B - 1);
             const half_t* src = p.G + (size_t(t) * p.B + b) * gld + size_t(4) * j;
 #pragma unroll
-            for (int c = 0; c < UPT / 2; ++c) ld_stream(xp[ph].v[c], src + 8 * c);
+            for (int c = 0; c < UPT / 2; ++c) ld_stream_fresh(xp[ph].v[c], src + 8 * c);
         }
     };
     if (c_in_regs) {
@@ -977,7 +1049,9 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
     loads_landed();
     clk.start();
 
+    ProjectedRows projected(p.project);
     for (int t = t_begin; t < t_end; ++t) {
+        if constexpr (RESIDENT) projected.wait_for((t - p.t0 + 1) * p.B, p.project, hs * NC, poll, lane);
         for (int rb = g; rb < L.nrb; rb += L.ng, ++item) {
             const int row0 = rb * RB;
             float* part = part_all + size_t(item & 1) * NW * kRows * PLD;
@@ -3843,19 +3917,43 @@ int rec_threads(const RecLayout& L) { return (L.split ? L.split : L.nw) * kWave;
 static int grid_with_helpers(const RecLayout& L, const BesideCopies& c) {
     return (L.xcd_local || c.count == 0) ? L.grid : L.grid + c.helpers;
 }
+void rec_share_columns(const RecLayout& L, ProjectBeside& w) {
+    int free_of[8], all = 0;
+    for (int x = 0; x < 8; ++x) {
+        // groups g = x, x + 8, ... sit on XCD x; other layouts seat the first ng * nh workgroups, dealt round-robin
+        const int seated = L.xcd_local ? L.nh * (L.ng > x ? (L.ng - x + 7) / 8 : 0) : (L.ng * L.nh - x + 7) / 8;
+        free_of[x] = L.num_cus / 8 > seated ? L.num_cus / 8 - seated : 0;
+        all += free_of[x];
+    }
+    const int columns = w.N / kBesideTile;
+    int sum = 0;
+    w.first[0] = 0;
+    for (int x = 0; x < 8; ++x) {
+        sum += free_of[x];
+        w.first[x + 1] = (unsigned char)(all > 0 ? (columns * sum + all / 2) / all : columns);
+    }
+}
+int rec_projecting_workgroups(const RecLayout& L) {
+    return (L.persistent && L.resident && !L.split && !L.wide && L.nw == 4) ? rec_idle_workgroups(L) : 0;
+}
 
 template <int NT, int KS, bool RES, int MT, bool DS, bool DEEP = false>
 static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     constexpr int NW = 4;
     auto kernel = rec_fwd_kernel<NT, KS, RES, MT, DS, DEEP>;
     if (L.nw != NW) return hipErrorInvalidValue;   // (the weight fragments are packed for L.nw waves)
-    const size_t lds = size_t(2) * NW * kRows * (16 * NT + kPartPad) * sizeof(float);
+    const size_t parts = size_t(2) * NW * kRows * (16 * NT + kPartPad) * sizeof(float);
+    const size_t lds = RES && parts < kBesideLds ? kBesideLds : parts;   // (one workgroup per CU either way)
+    const ProjectBeside& w = a.project;
+    if (w.M != 0 && (!L.persistent || !RES || w.M != (a.t1 - a.t0) * a.B || w.N != 4 * a.Hp || w.N % kBesideTile != 0 || w.first[8] != w.N / kBesideTile || w.K <= 0 || w.K % BK != 0 ||
+                     w.lda < size_t(w.K) || w.lda >= (size_t(1) << 22) || w.lda % 8 != 0 || reinterpret_cast<uintptr_t>(w.A) % 16 != 0))
+        return hipErrorInvalidValue;
     static std::atomic<int> per_cu[kMaxDevices];
     int device = 0;
     hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
     if (e != hipSuccess) return e;
     const int ks_wave = rec_fwd_ks(L, a.Hp);
-    if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
+    if (L.persistent) return launch_persistent(kernel, w.M != 0 ? L.num_cus : grid_with_helpers(L, a.beside), lds, stream, a, L, a.t0, a.t1, ks_wave, per_cu[device].load(), device, NW * kWave);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
                         [&]() -> hipError_t {
                             for (int t = a.t0; t < a.t1; ++t) {
