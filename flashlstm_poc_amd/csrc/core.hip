@@ -435,13 +435,13 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     const RecLayout bwd = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 2, 0), pair = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 0, 0);
     FL_TRY(want(kFragFwd, fwd, rec_fwd_ks(fwd, d.Hp), rec_fwd_fragments(fwd, d.Hp)));
     frag[kFragFwd].wide = fwd.wide;
-    if (split.split) {
+    if (split.split || split.broad) {
         FL_TRY(want(kFragFwdSplit, split, rec_fwd_ks(split, d.Hp), rec_fwd_fragments(split, d.Hp)));
         frag[kFragFwdSplit].split = split.split;
-        FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));   // (here: flstm_core_forward_static allocates nothing)
+        if (split.split) FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));   // (here: flstm_core_forward_static allocates nothing)
     }
     FL_TRY(want(kFragBwd, bwd, rec_bwd_ks(bwd, d.Hp), rec_bwd_fragments(bwd, d.Hp)));
-    if (pair.split) FL_TRY(want(kFragBwdPair, pair, rec_bwd_ks(pair, d.Hp), rec_bwd_fragments(pair, d.Hp)));
+    if (pair.split || pair.broad) FL_TRY(want(kFragBwdPair, pair, rec_bwd_ks(pair, d.Hp), rec_bwd_fragments(pair, d.Hp)));
     if (rec_bwd_two_d_possible(d.Hp, p->num_cus)) {
         FragLayout& f = frag[kFragBwdTwoD];
         f.kq = rec_bwd_two_d_kq(d.B, d.Hp);
@@ -596,7 +596,7 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     const Dims& d = p->d;
     RecFwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (padding too: the arguments are the key of a captured graph)
-    a.wfrag = p->wfrag[p->Lf.split ? kFragFwdSplit : kFragFwd].as<half8>();
+    a.wfrag = p->wfrag[p->Lf.split || p->Lf.broad ? kFragFwdSplit : kFragFwd].as<half8>();
     a.Y = p->Y.as<half_t>(); a.G = p->G.as<half_t>(); a.C = p->C.as<float>();
     a.y_out = p->fw.y_direct;
     a.X = p->xch_f.as<half_t>(); a.x_slot = exchange_slot_halfs(d.B, d.Hp);
@@ -932,7 +932,7 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
     }
     RecBwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (as in forward_recur)
-    a.wfrag = p->wfrag[p->Lb.split ? kFragBwdPair : kFragBwd].as<half8>();
+    a.wfrag = p->wfrag[p->Lb.split || p->Lb.broad ? kFragBwdPair : kFragBwd].as<half8>();
     a.G = p->G.as<half_t>(); a.C = p->C.as<float>(); a.dY = p->bw.dYk; a.dG = p->dG.as<half_t>();
     a.dHn = p->dHn.as<float>(); a.dC = p->dC.as<float>(); a.dH0 = p->dH0.as<float>();
     a.X = p->xch_b.as<half_t>(); a.x_slot = exchange_slot_halfs(rec_bwd_ring_rows(p->Lb, d.B), 4 * d.Hp);

@@ -20,8 +20,8 @@ struct FragLayout {   // where a recurrence kernel expects its weight fragments:
     int ks = 0, nt = 0, rot_div = 0, nw = 0, unit_major = 0, wide = 0, kq = 0, split = 0;
     size_t fragments = 0;   // of 64 lanes
 };
-// Forward: the one-way kernels' and those of the kernel for short contractions; backward the same; those of the backward
-// recurrence that splits its product two ways.
+// Forward: the one-way kernels' and those of the kernel for short contractions, or with slices of 32 units (RecLayout::broad);
+// backward the same; those of the backward recurrence that splits its product two ways.
 enum Frag : int { kFragFwd, kFragFwdSplit, kFragBwd, kFragBwdPair, kFragBwdTwoD, kFragKinds };
 // W_ih twice (as it is for the projection, transposed for dX) and W_hh as every kind of fragments asked for; one launch.
 hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p /*[4Hp][Ip]*/,

@@ -31,6 +31,7 @@ struct RecLayout {
     int unit_major;  // forward: gate columns of a slice are packed 4 * unit + gate (kernels with one cell per thread), else gate
                      // blocks of jb units
     int split;       // the kernels for short contractions (rec_fwd_split_kernel, rec_bwd_pair_kernel): waves per workgroup
+    int broad;       // 1025 to 1536 units: slices of 32 units instead of 16, 16-row blocks (any number of them)
     int wide;        // more than 2048 hidden units, weights resident (rec_fwd_wide_kernel, rec_bwd_wide_kernel)
     int num_cus;     // of the device the layout was made for
     int rot_div;     // k-step rotation (rec_kstep_rotation): slices rot_div apart run on the same XCD

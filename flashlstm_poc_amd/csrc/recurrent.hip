@@ -951,6 +951,17 @@ struct ProjectedRows {
     }
 };
 
+// 16 rows of partial sums per wave: [wave][16][pld] (spill_partials with one row tile and a 16-row pitch per wave)
+template <int NT>
+__device__ __forceinline__ void spill_partials16(float* part, const floatx4 (&acc)[2][NT], int wave, int lane, int pld) {
+    float* base = part + (size_t(wave) * 16 + size_t(lane % 16)) * pld + 4 * (lane / 16);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) *reinterpret_cast<floatx4*>(base + n * 16) = acc[0][n];
+}
+
+// Rows of a wave's partial sums in the forward kernel: 32, or the one tile's 16 where LDS holds weights as well.
+__host__ __device__ constexpr int fwd_part_rows(int MT, int KL) { return MT == 1 && KL > 0 ? 16 : kRows; }
+
 // ------------------------------------------------------------------------------------ forward
 // Per step and row block: K-split MFMA product on h_{t-1} as it arrives -> partial sums through LDS
 // (two buffers, one barrier per step) -> pointwise cell update -> store h_t -> store c_t and the
@@ -968,13 +979,14 @@ struct ProjectedRows {
 // of the block (two units each) and store that half of h_t, then rows 16..31.  The consumers fetch and multiply
 // tile by tile (wave_product_tiles), so the second phase of a step overlaps the first half of the peers' next
 // product instead of sitting on the path from one step to the next.
-template <int NT, int KS, bool RESIDENT, int MT, bool DS, bool DEEP = false>
+template <int NT, int KS, bool RESIDENT, int MT, bool DS, bool DEEP = false, int KL = 0>
 __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayout L, int t_begin,
                                                            int t_end, int ks_wave) {
     constexpr int NW = 4;
     constexpr int JB = 4 * NT;    // hidden units of this slice
     constexpr int NC = 16 * NT;   // gate columns of this slice (i,f,g,o blocks of JB)
     constexpr int PLD = NC + kPartPad;
+    constexpr int PROWS = fwd_part_rows(MT, KL);   // rows of a wave's partial sums
     constexpr bool SPLIT = RESIDENT && MT == 2 && JB >= 32;
     // cell updates per thread: the slice's units of one batch row are shared by GPR threads; 32 rows x 8 threads,
     // or 16 rows x 16 threads (per phase, or when a block has one row tile) where the slice is wide enough for 2 units each
@@ -983,7 +995,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
     constexpr int NPH = SPLIT ? 2 : 1;   // pointwise phases per step
     static_assert(UPT == 2 || UPT == 4, "2 or 4 hidden units per thread");
     typedef Pack<UPT> PackT;
-    extern __shared__ __attribute__((aligned(16))) float part_all[];  // [2][4][32][PLD]
+    extern __shared__ __attribute__((aligned(16))) float part_all[];  // [2][4][PROWS][PLD] | weight fragments of KL k-steps
     __shared__ int lds_abort;
     __shared__ int lds_role[2];
 
@@ -1006,13 +1018,17 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
     if constexpr (DS) first_request.start_from(p.delay_hint);
 
     const half8* wfrag_wave = p.wfrag + (size_t(hs) * NW + wave) * size_t(ks_wave) * NT * kWave;
-    half8 wreg[KS][NT];
+    half8 wreg[KS - KL][NT];
+    half8* wlds = reinterpret_cast<half8*>(part_all + 2 * NW * PROWS * PLD) + size_t(wave) * KL * NT * kWave;
     if constexpr (RESIDENT) {
 #pragma unroll
         for (int k = 0; k < KS; ++k)
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
-                wreg[k][n] = (k < ks_wave) ? wfrag_wave[(size_t(k) * NT + n) * kWave + lane] : half8{};
+            for (int n = 0; n < NT; ++n) {
+                const half8 w = (k < ks_wave) ? wfrag_wave[(size_t(k) * NT + n) * kWave + lane] : half8{};
+                if (wlds_has(k, KS, KL)) wlds[(wlds_before(k, KS, KL) * NT + n) * kWave + lane] = w;
+                else wreg[wreg_slot(k, KS, KL)][n] = w;
+            }
     }
 
     const size_t gld = size_t(4) * p.Hp;
@@ -1054,7 +1070,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
         if constexpr (RESIDENT) projected.wait_for((t - p.t0 + 1) * p.B, p.project, hs * NC, poll, lane);
         for (int rb = g; rb < L.nrb; rb += L.ng, ++item) {
             const int row0 = rb * RB;
-            float* part = part_all + size_t(item & 1) * NW * kRows * PLD;
+            float* part = part_all + size_t(item & 1) * NW * PROWS * PLD;
             const half_t* xin = p.X + size_t(t & 3) * p.x_slot;          // h_{t-1}, fragment-major
             half_t* xout = p.X + size_t((t + 1) & 3) * p.x_slot;         // h_t
             half_t* xnext = p.X + size_t((t + 3) & 3) * p.x_slot;        // will take h_{t+2}: marked unwritten
@@ -1071,11 +1087,12 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
                 ahead = wave_product_tiles<NT, KS, 0, NPH * UPT / 2, kFwdBufs, false, 0, DS>(acc, wreg, nullptr, a0, a1, wave, lane, nks_total, ks_wave, rotation, poll,
                                                              [&]() { prefetch(t, rb); });
             else
-                ahead = wave_product<NT, KS, RESIDENT, 0, UPT / 2, MT, DEEP ? 4 : 2, DEEP ? 2 : (KS == 12) ? 4 : 0, DEEP, DS && !DEEP>(acc, wreg, nullptr, wfrag_wave, a0, a1, wave, lane, nks_total,
+                ahead = wave_product<NT, KS, RESIDENT, KL, UPT / 2, MT, DEEP ? 4 : 2, DEEP ? 2 : (KS == 12) ? 4 : 0, DEEP, DS && !DEEP>(acc, wreg, wlds, wfrag_wave, a0, a1, wave, lane, nks_total,
                                                                ks_wave, rotation, poll, [&]() { prefetch(t, rb); });
             if constexpr (DS) first_request.learn(ahead);
             clk.lap(0);
-            spill_partials<NT, MT>(part, acc, wave, lane, PLD);
+            if constexpr (PROWS == 16) spill_partials16<NT>(part, acc, wave, lane, PLD);
+            else spill_partials<NT, MT>(part, acc, wave, lane, PLD);
             __syncthreads();
             if (lds_abort != 0) leave_kernel();
             clk.lap(1);
@@ -1113,7 +1130,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
 #pragma unroll
                         for (int w = 0; w < NW; ++w) {
                             float v[UPT];
-                            ld_f32(part + (size_t(w) * kRows + prow) * PLD + gt * JB + pj, v);
+                            ld_f32(part + (size_t(w) * PROWS + prow) * PLD + gt * JB + pj, v);
 #pragma unroll
                             for (int u = 0; u < UPT; ++u) z[gt][u] += v[u];
                         }
@@ -1170,14 +1187,6 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
     clk.flush();
 }
 
-
-// 16 rows of partial sums per wave: [wave][16][pld] (spill_partials with one row tile and a 16-row pitch per wave)
-template <int NT>
-__device__ __forceinline__ void spill_partials16(float* part, const floatx4 (&acc)[2][NT], int wave, int lane, int pld) {
-    float* base = part + (size_t(wave) * 16 + size_t(lane % 16)) * pld + 4 * (lane / 16);
-#pragma unroll
-    for (int n = 0; n < NT; ++n) *reinterpret_cast<floatx4*>(base + n * 16) = acc[0][n];
-}
 
 // ------------------------------------------------------------------- forward, interleaved chains
 // The kernel above walks one dependent chain per row block: product -> partial sums -> cell update -> h_t out -> one
@@ -3663,12 +3672,18 @@ constexpr int kWideMost = 4096;   // hidden units whose W_hh the chip can hold (
 // the faster one up to 384 units (2.13 -> 1.93); at 512 its two waves take as long over the product as the other kernel's
 // four over theirs and its reduction (2.14 -> 2.24).
 constexpr int kFwdSplitMost = 512, kFwdSplitFourMost = 256, kBwdPairMost = 384;
+constexpr int kBroadMost = 1536;   // hidden units of which a workgroup can hold the weights of a slice of 32 (384 KiB)
 
 // whether all 16-row blocks of the batch can run side by side
 static bool can_16_rows(int B, int nh, int num_cus) {
     const bool xcd_mode = (num_cus == 256 && nh <= 32);
     const int side_by_side = nh > num_cus ? 0 : (xcd_mode ? 8 * (32 / nh) : num_cus / nh);
     return int(ceil_div(size_t(B), 16)) <= side_by_side;
+}
+
+// row blocks of `rows` rows that a workgroup takes one after the other per step, slices by nh
+static int turns(int B, int rows, int nh, int num_cus) {
+    return int(ceil_div(ceil_div(size_t(B), size_t(rows)), size_t(num_cus / nh > 0 ? num_cus / nh : 1)));
 }
 
 static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_stepwise, bool fits, int force_mt) {
@@ -3681,6 +3696,7 @@ static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_s
     L.mt = can_16 ? 1 : 2;
     if (force_mt == 2 || (force_mt == 1 && can_16)) L.mt = force_mt;   // a tuned choice; 16-row blocks only where they fit
     if (fits && Hp > 2048) L.mt = 1;   // the kernels for more than 2048 units take 16-row tiles one after the other
+    if (L.broad) L.mt = 1;     // (slices of 32 units above 1024: likewise)
     if (L.nw == 8) L.mt = 2;   // the eight-wave kernels take 32-row blocks (their two row tiles take turns)
     L.nrb = int(ceil_div(size_t(B), size_t(16 * L.mt)));
     L.xcd_local = 0;
@@ -3716,6 +3732,16 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.unit_major = L.nw == 8 || (fits && Hp > 2048);
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
     L.wide = fits && Hp > 2048;
+    // 1025 to 1536 units: slices of 32 units, as backward, where all 16-row blocks run side by side that way or take fewer turns a
+    // step than blocks of 32 with slices of 16.  Measured at 1536 units, us per step: 33 to 64 rows 2.85 -> 2.55, 80 rows 4.8 -> 2.6, 160 rows
+    // 8.4 -> 4.9; with as many turns (100, 161 rows) a tie, at 1280 units and 161 rows 4.6 -> 4.95.
+    if (force_mt != 2 && Hp > 1024 && Hp <= kBroadMost && !can_16_rows(B, Hp / 16, num_cus) && Hp / 32 <= num_cus &&
+        (can_16_rows(B, Hp / 32, num_cus) || turns(B, 16, Hp / 32, num_cus) < turns(B, 32, Hp / 16, num_cus))) {
+        L.broad = 1;
+        L.nt = 8;
+        L.jb = 32;
+        finish_layout(L, B, Hp, num_cus, force_stepwise, fits, 1);
+    }
     // short contractions: columns split over the waves, where every group has one 16-row block (and neither 32-row blocks nor four
     // waves that split the contraction are asked for)
     if (L.nw == 4 && waves != 4 && force_mt != 2 && Hp <= kFwdSplitMost && num_cus == 256) {
@@ -3749,6 +3775,16 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
         L.jb = 16;
         finish_layout(L, B, Hp, num_cus, force_stepwise, fits, 1);
         return L;
+    }
+    // 1025 to 1536 units: slices of 32 where the 16-row blocks do not fit side by side with slices of 16.  A step is bound by the
+    // fetch of dG_{t+1} of a workgroup's rows, whatever its slice, and with half the slices twice the groups run; what a workgroup
+    // holds, 384 KiB, leaves no registers for a second row tile.  Measured at 1536 units, us per step: 33 to 64 rows 5.6 -> 3.8, 80 rows
+    // 9.4 -> 4.2, 100 rows 9.6 -> 7.2, 160 rows 15.0 -> 8.2, 256 rows 20.2 -> 15.6; at 1056 units 64 rows 5.3 -> 3.7, 400 rows 25.3 -> 15.9.
+    if (force_mt != 2 && Hp > 1024 && Hp <= kBroadMost && !can_16_rows(B, Hp / 16, num_cus) && Hp / 32 <= num_cus) {
+        L.broad = 1;
+        L.nt = 2;
+        L.jb = 32;
+        finish_layout(L, B, Hp, num_cus, force_stepwise, fits, 1);
     }
     // k-step rotation (recurrent.h): measured, it pays where a group spans the XCDs and a step fetches a lot -- the
     // backward pass at 2048 hidden units, 13.4 -> 12.4 us per step at 128 rows -- and costs a little where the
@@ -3937,12 +3973,12 @@ int rec_projecting_workgroups(const RecLayout& L) {
     return (L.persistent && L.resident && !L.split && !L.wide && L.nw == 4) ? rec_idle_workgroups(L) : 0;
 }
 
-template <int NT, int KS, bool RES, int MT, bool DS, bool DEEP = false>
+template <int NT, int KS, bool RES, int MT, bool DS, bool DEEP = false, int KL = 0>
 static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     constexpr int NW = 4;
-    auto kernel = rec_fwd_kernel<NT, KS, RES, MT, DS, DEEP>;
+    auto kernel = rec_fwd_kernel<NT, KS, RES, MT, DS, DEEP, KL>;
     if (L.nw != NW) return hipErrorInvalidValue;   // (the weight fragments are packed for L.nw waves)
-    const size_t parts = size_t(2) * NW * kRows * (16 * NT + kPartPad) * sizeof(float);
+    const size_t parts = size_t(2) * NW * fwd_part_rows(MT, KL) * (16 * NT + kPartPad) * sizeof(float) + size_t(NW) * KL * NT * kWave * sizeof(half8);
     const size_t lds = RES && parts < kBesideLds ? kBesideLds : parts;   // (one workgroup per CU either way)
     const ProjectBeside& w = a.project;
     if (w.M != 0 && (!L.persistent || !RES || w.M != (a.t1 - a.t0) * a.B || w.N != 4 * a.Hp || w.N % kBesideTile != 0 || w.first[8] != w.N / kBesideTile || w.K <= 0 || w.K % BK != 0 ||
@@ -4111,7 +4147,10 @@ hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
             if (ks <= 2) return run_fwd_ds<8, 2, 1>(L, a, ds, stream, graphs);
             if (ks <= 4) return run_fwd_ds<8, 4, 1>(L, a, ds, stream, graphs);
             if (ks <= 6) return run_fwd_ds<8, 6, 1>(L, a, ds, stream, graphs);
-            return run_fwd_ds<8, 8, 1>(L, a, ds, stream, graphs);
+            if (ks <= 8) return run_fwd_ds<8, 8, 1>(L, a, ds, stream, graphs);
+            // (RecLayout::broad; step-wise launches of it too)
+            if (ks <= 10) return run_fwd_ds<8, 10, 1>(L, a, ds, stream, graphs);
+            return ds ? run_fwd<8, 12, true, 1, true, false, 2>(L, a, stream, graphs) : run_fwd<8, 12, true, 1, false, false, 2>(L, a, stream, graphs);
         }
         if (ks <= 4) return run_fwd_ds<8, 4, 2>(L, a, ds, stream, graphs);
         return run_fwd_ds<8, 8, 2>(L, a, ds, stream, graphs);
@@ -4254,7 +4293,8 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
             if (ks <= 8) return run_bwd_ds<2, 8, 0, 1>(L, a, ds, stream, graphs);
             if (ks <= 16) return run_bwd_ds<2, 16, 0, 1>(L, a, ds, stream, graphs);
             if (ks <= 24) return run_bwd_ds<2, 24, 0, 1>(L, a, ds, stream, graphs);
-            return run_bwd_ds<2, 32, 8, 1>(L, a, ds, stream, graphs);
+            if (ks <= 32) return run_bwd_ds<2, 32, 8, 1>(L, a, ds, stream, graphs);
+            return run_bwd_ds<2, 48, 14, 1>(L, a, ds, stream, graphs);
         }
         if (ks <= 16) return run_bwd_ds<2, 16, 0, 2>(L, a, ds, stream, graphs);
         return run_bwd_ds<2, 32, 8, 2>(L, a, ds, stream, graphs);
