@@ -1179,7 +1179,10 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
             // poll notices the data a full round trip to the L2 after it went out, whereas a wave that asks once the
             // data is there has it after one trip: measured, the early waves finished their product 0.4 us AFTER the
             // others (2048 units, 16 rows).  So all four waves start a product together.
+            // Likewise where 16 threads share a row and the block has fewer than 16: some waves have no cells (1024 units, one row
+            // 1.80 -> 1.61 us per step, five rows 1.83 -> 1.68, twelve 1.79 -> 1.74; backward 2.53 -> 2.40, 2.65 -> 2.51, 2.65 -> 2.62).
             if constexpr (MT == 1 && GPR == 8) __syncthreads();
+            else if constexpr (MT == 1) { if (p.B - row0 < RB) __syncthreads(); }
         }
     }
     if constexpr (DS) first_request.leave(p.delay_hint);
@@ -2838,7 +2841,8 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
                 }
             }
             clk.lap(3);
-            if constexpr (MT == 1 && GPR == 8) __syncthreads();   // (waves without cells to update: as in the forward kernel)
+            if constexpr (MT == 1 && GPR == 8) __syncthreads();
+            else if constexpr (MT == 1) { if (p.B - row0 < RB) __syncthreads(); }   // (as in the forward kernel)   // (waves without cells to update: as in the forward kernel)
         }
     }
     if (p.stamp_end && hs == 0 && g == 0 && tid == 0) *p.stamp_end = wall_clock64();
