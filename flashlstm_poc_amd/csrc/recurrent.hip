@@ -1543,6 +1543,7 @@ __device__ __forceinline__ void ld_stream_at(uintx4& d, const void* base, unsign
 template <int KS>
 __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, RecLayout L, int t_begin, int t_end, int) {
     static_assert(KS % 2 == 0 && KS <= 16, "up to 512 hidden units");
+    constexpr bool LATE = KS >= 12;   // (when the x-projection is requested: rec_fwd_whole_kernel)
     __shared__ int lds_abort;
     __shared__ int lds_role[2];
     if (threadIdx.x == 0) lds_abort = 0;
@@ -1603,8 +1604,8 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
         half8 f[KS];
         auto request = [&]() __attribute__((always_inline)) { request_split(f, tile, lane_off, tail_off, std::make_integer_sequence<int, KS>{}); };
         request();
-        request_xp(t + 1 < t_end ? t + 1 : t, std::integral_constant<int, 1 - par>{});
-        wait_set<1>(f);
+        if constexpr (!LATE) request_xp(t + 1 < t_end ? t + 1 : t, std::integral_constant<int, 1 - par>{});
+        wait_set<LATE ? 0 : 1>(f);
         auto unwritten = [&]() -> bool {
             unsigned m = 0u;
 #pragma unroll
@@ -1623,6 +1624,7 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
                 wait_set<0>(f);
             } while (unwritten());
         }
+        if constexpr (LATE) request_xp(t + 1 < t_end ? t + 1 : t, std::integral_constant<int, 1 - par>{});
         floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int k = 0; k < KS; ++k)
@@ -1695,6 +1697,11 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
 // The cache stores, the output row and the projection stand between the store of h_t and the request for the next step's
 // fragments: requested right behind the store, they come back unwritten and the second request notices them a trip later (256
 // units and 64 rows 0.80 -> 0.95 us per step).
+// LATE: the rows of the steps to come (x or the x-projection) are requested once the fragments are there, not behind their
+// request.  A wave that finds the fragments unwritten and asks again would wait for those rows as well (loads return in order),
+// a trip to memory; a wave that finds them there loses the head start.  Measured, us per step, behind / once there: 512 units and
+// 64 rows 1.28 / 1.16, 384 and 100 rows 1.18 / 1.02, 256 units and four waves a workgroup (300 rows) 1.25 / 1.14; but 256 units
+// and 8 rows 0.88 / 0.90, 64 units 0.56 / 0.58, 128 units and 200 rows 0.66 / 0.67.
 template <int OFF>
 __device__ __forceinline__ void ld_stream_off(half8& dst, unsigned lane_off, const void* base) {
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3 nt" : "=v"(dst) : "v"(lane_off), "s"(base), "n"(OFF) : "memory");
@@ -1746,7 +1753,7 @@ __device__ __forceinline__ void interleave_rows(half8& a, half8& b) {
     a = x.h;
     b = y.h;
 }
-template <int KS, int KI, bool SAVE>
+template <int KS, int KI, bool SAVE, bool LATE>
 __global__ __launch_bounds__(kThreads) void rec_fwd_whole_kernel(RecWholeArgs p, RecLayout L, int, int, int) {
     static_assert(KS % 2 == 0 && KS <= 16 && KI % 4 == 0, "up to 512 hidden units, rows of whole 64-element groups");
     constexpr int NG = KI / 4;            // 64-element groups of an input row
@@ -1993,27 +2000,35 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_whole_kernel(RecWholeArgs p,
         store_xch(p.ring + size_t((t + 1 + p.base) & 3) * p.x_slot + size_t(g) * tile_halfs + off_ring, Pack<2>{h2}, false);
         keep(t);
     };
+    // the rows that the fragments' wait of step t + 1 leaves in flight: those of step t + 2, or of the pair after the next
+    auto request_rows_of = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        if constexpr (KI == 0) request_xp(t + 2, parity);
+        else if constexpr (par == 1) request_x(t + 3);
+    };
     auto publish = [&](int t, auto parity) __attribute__((always_inline)) {
         constexpr int par = decltype(parity)::value;
+        (void)par;
         send(t);
         if constexpr (KI > 0 && par == 1) project();
         request(t + 1);
-        if constexpr (KI == 0) request_xp(t + 2, parity);
-        else if constexpr (par == 1) request_x(t + 3);
+        if constexpr (!LATE) request_rows_of(t, parity);
     };
     cells(0, even);
     int t = 0;   // its cells are updated
     for (; t + 2 < p.T; t += 2) {
         publish(t, even);
-        // (what a step has requested beside its fragments has landed when the next step's fragments have, which are younger)
-        arrived(t + 1, std::integral_constant<int, KI == 0 ? 1 : 0>{});
+        // (what a step has requested behind its fragments has landed when the next step's fragments have, which are younger)
+        arrived(t + 1, std::integral_constant<int, LATE ? 0 : KI == 0 ? 1 : 0>{});
+        if constexpr (LATE) request_rows_of(t, even);
         if constexpr (KI > 0) {
 #pragma unroll
             for (int k = 0; k < NR; ++k) { settle(xa[k]); settle(xb[k]); }
         }
         cells(t + 1, odd);
         publish(t + 1, odd);
-        arrived(t + 2, std::integral_constant<int, KI == 0 ? 1 : KI>{});
+        arrived(t + 2, std::integral_constant<int, LATE ? 0 : KI == 0 ? 1 : KI>{});
+        if constexpr (LATE) request_rows_of(t + 1, odd);
         cells(t + 2, even);
     }
     wait_all_vm();   // (what the last steps have requested ahead is used by nobody, but its registers must not be handed on before)
@@ -2882,9 +2897,11 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
 // TWO waves owns 16 units (one column tile).  The waves split the contraction, exchange half of their sums through LDS (8
 // bytes per lane, one barrier) and update the cells of two neighbouring units each, one 16-byte chunk of the ring per lane.
 // Against the kernel above: as many fragment loads per CU, half the columns to sum over half the waves.  The operands of
-// step t - 1 (gates, c, dY) are requested behind the fragments of step t.
-// Measured, us per step, rec_bwd_kernel -> here: 64 units 1.62 -> 1.07, 128 units 1.71 -> 1.22, 256 units and 8 rows
-// 1.79 -> 1.54, 257 units and 70 rows 2.13 -> 1.84, 384 units 2.13 -> 1.93.  (Four waves with one cell per lane: 1.65 at
+// step t - 1 (gates, c, dY) are requested once the fragments of step t are there: requested behind them, a wave that finds the
+// fragments unwritten and asks again waits for those operands' trip to memory as well, since loads return in order.
+// Measured, us per step, rec_bwd_kernel -> here with the operands behind the fragments -> once those are there: 64 units 1.62 ->
+// 1.17 -> 0.89, 128 units and 200 rows 1.35 -> 1.09, 256 units and 8 rows 1.79 -> 1.54 -> 1.49, 257 units and 70 rows 2.13 -> 1.79 -> 1.59,
+// 384 units and 100 rows 1.94 -> 1.75.  (Four waves with one cell per lane: 1.65 at
 // 256 units; the longer barrier costs more than the shorter update gives.)
 template <int KS, int K>
 __device__ __forceinline__ void request_pair_one(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off) {
@@ -3024,8 +3041,7 @@ __global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, R
         half8 f[KS];
         auto request = [&]() __attribute__((always_inline)) { request_pair(f, tile, lane_off, tail_off, std::make_integer_sequence<int, KS>{}); };
         request();
-        request_ops(t - 1, std::integral_constant<int, 1 - par>{});
-        wait_set<4>(f);
+        wait_set<0>(f);
         auto unwritten = [&]() -> bool {
             unsigned m = 0u;
 #pragma unroll
@@ -3044,6 +3060,7 @@ __global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, R
                 wait_set<0>(f);
             } while (unwritten());
         }
+        request_ops(t - 1, std::integral_constant<int, 1 - par>{});
         floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int k = 0; k < KS; ++k) acc[k % 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[k], f[k], acc[k % 2], 0, 0, 0);
@@ -4053,21 +4070,29 @@ static hipError_t run_fwd_split(const RecLayout& L, const RecFwdArgs& a, hipStre
                         });
 }
 
-template <int KS, int KI, bool SAVE>
+template <int KS, int KI, bool SAVE, bool LATE>
 static hipError_t run_fwd_whole(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream) {
-    auto kernel = rec_fwd_whole_kernel<KS, KI, SAVE>;
+    auto kernel = rec_fwd_whole_kernel<KS, KI, SAVE, LATE>;
     static std::atomic<int> per_cu[kMaxDevices];
     int device = 0;
     hipError_t e = prepare_kernel(kernel, kWholeCuLds, kThreads, per_cu, &device);
     if (e != hipSuccess) return e;
     return launch_persistent(kernel, L.grid, kWholeCuLds, stream, a, L, 0, 0, 0, per_cu[device].load(), device, L.split * kWave);
 }
-template <int KS, bool SAVE>
+template <int KS, bool SAVE, bool LATE>
 static hipError_t run_fwd_whole_ki(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream) {
-    if (!a.x) return run_fwd_whole<KS, 0, SAVE>(L, a, stream);
-    if (a.Ip <= 64) return run_fwd_whole<KS, 4, SAVE>(L, a, stream);
-    if (a.Ip <= 128) return run_fwd_whole<KS, 8, SAVE>(L, a, stream);
-    return run_fwd_whole<KS, 16, SAVE>(L, a, stream);
+    if (!a.x) return run_fwd_whole<KS, 0, SAVE, LATE>(L, a, stream);
+    if (a.Ip <= 64) return run_fwd_whole<KS, 4, SAVE, LATE>(L, a, stream);
+    if (a.Ip <= 128) return run_fwd_whole<KS, 8, SAVE, LATE>(L, a, stream);
+    return run_fwd_whole<KS, 16, SAVE, LATE>(L, a, stream);
+}
+template <int KS>
+static hipError_t run_fwd_whole_ks(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream) {
+    constexpr bool LATE = KS >= 12;
+    if constexpr (KS == 8) {
+        if (L.split == 4) return a.Y ? run_fwd_whole_ki<KS, true, true>(L, a, stream) : run_fwd_whole_ki<KS, false, true>(L, a, stream);
+    }
+    return a.Y ? run_fwd_whole_ki<KS, true, LATE>(L, a, stream) : run_fwd_whole_ki<KS, false, LATE>(L, a, stream);
 }
 bool rec_whole_possible(const RecLayout& L) { return L.split && L.persistent && L.xcd_local && L.mt == 1 && L.nrb <= L.ng; }
 hipError_t launch_rec_fwd_whole(const RecLayout& L, const RecWholeArgs& a, hipStream_t stream) {
@@ -4076,7 +4101,7 @@ hipError_t launch_rec_fwd_whole(const RecLayout& L, const RecWholeArgs& a, hipSt
         (!a.x && !a.G) || (a.x && (a.Ip <= 0 || a.Ip % 64 != 0 || a.Ip > kRecWholeInput || a.ldx < a.Ip)))
         return hipErrorInvalidValue;
     switch (rec_fwd_ks(L, a.Hp)) {
-#define FLSTM_WHOLE_CASE(n) case n: return a.Y ? run_fwd_whole_ki<n, true>(L, a, stream) : run_fwd_whole_ki<n, false>(L, a, stream);
+#define FLSTM_WHOLE_CASE(n) case n: return run_fwd_whole_ks<n>(L, a, stream);
         FLSTM_WHOLE_CASE(2) FLSTM_WHOLE_CASE(4) FLSTM_WHOLE_CASE(8) FLSTM_WHOLE_CASE(12) FLSTM_WHOLE_CASE(16)
 #undef FLSTM_WHOLE_CASE
     }
