@@ -1087,8 +1087,12 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_kernel(RecFwdArgs p, RecLayo
                 ahead = wave_product_tiles<NT, KS, 0, NPH * UPT / 2, kFwdBufs, false, 0, DS>(acc, wreg, nullptr, a0, a1, wave, lane, nks_total, ks_wave, rotation, poll,
                                                              [&]() { prefetch(t, rb); });
             else
-                ahead = wave_product<NT, KS, RESIDENT, KL, UPT / 2, MT, DEEP ? 4 : 2, DEEP ? 2 : (KS == 12) ? 4 : 0, DEEP, DS && !DEEP>(acc, wreg, wlds, wfrag_wave, a0, a1, wave, lane, nks_total,
-                                                               ks_wave, rotation, poll, [&]() { prefetch(t, rb); });
+                // One row tile and peers on other XCDs: what bounds a step is how long the exchanged fragments take to come,
+                // so two chunks are asked for ahead of the one being multiplied (512 steps of 16 rows x 2048 units 2.20 ->
+                // 2.12 us a step, of 3 rows 2.31 -> 2.22, of 16 rows x 1300 units 2.02 -> 1.95; three chunks ahead give no
+                // more).  The other instances stay at one: within an XCD nothing is gained, two row tiles have no registers.
+                ahead = wave_product<NT, KS, RESIDENT, KL, UPT / 2, MT, DEEP ? 4 : (DS && MT == 1 && (NT == 4 || KS == 10)) ? 3 : 2, DEEP ? 2 : (KS == 12) ? 4 : 0, DEEP,
+                                     DS && !DEEP>(acc, wreg, wlds, wfrag_wave, a0, a1, wave, lane, nks_total, ks_wave, rotation, poll, [&]() { prefetch(t, rb); });
             if constexpr (DS) first_request.learn(ahead);
             clk.lap(0);
             if constexpr (PROWS == 16) spill_partials16<NT>(part, acc, wave, lane, PLD);
