@@ -975,9 +975,8 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
 }
 
 // dX rows of steps [t_lo, t_hi] = dG * W_ih  (contraction over the packed gate columns)
-int backward_dx(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
+GemmNT dx_product(flstm_core_plan* p, long t_hi, long t_lo) {
     const Dims& d = p->d;
-    if (!p->bw.dx || t_hi < t_lo) return 0;
     const size_t row0 = size_t(t_lo) * d.B, rows = size_t(t_hi - t_lo + 1) * d.B;
     GemmNT g{};
     g.A = p->dG.as<half_t>() + row0 * 4 * d.Hp; g.lda = size_t(4) * d.Hp;
@@ -986,7 +985,11 @@ int backward_dx(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
     if (p->bw.dx_dtype == FLSTM_F32) g.C32 = static_cast<float*>(p->bw.dx) + row0 * d.I;
     else g.C16 = static_cast<half_t*>(p->bw.dx) + row0 * d.I;
     g.ldc = size_t(d.I); g.alpha = p->bw.k.dx; g.splits = 1; g.split_stride = 0;
-    FL_TRY(launch_gemm_nt(g, s));
+    return g;
+}
+int backward_dx(flstm_core_plan* p, long t_hi, long t_lo, hipStream_t s) {
+    if (!p->bw.dx || t_hi < t_lo) return 0;
+    FL_TRY(launch_gemm_nt(dx_product(p, t_hi, t_lo), s));
     return 0;
 }
 
@@ -999,8 +1002,9 @@ int backward_rec_once(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype 
 }
 
 // dW_ih = dG^T * X and dW_hh = dG^T * H_prev over the whole sequence, bias gradient and state gradients (enqueued; the
-// last launch of a pass)
-int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, float* dW_ih, float* dW_hh,
+// last launch of a pass).  `with_dx`: a whole pass, whose dX is formed here as well, in the same launch where both products are
+// small (launch_gemm_tn_and_nt).
+int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, bool with_dx, float* dW_ih, float* dW_hh,
                     float* db_ih, float* db_hh, float* dh0, float* dc0, hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = p->bw.T * size_t(d.B);
@@ -1014,6 +1018,8 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, floa
     const int n_ih = dW_ih ? d.Ip : 0, n_hh = dW_hh ? d.Hp : 0, ncols = n_ih + n_hh;
     const bool accumulate = p->opt_accumulate != 0;
     OpList out;   // gradients into the caller's layout, one launch
+    with_dx = with_dx && p->bw.dx;
+    if (with_dx && ncols == 0) FL_TRY(launch_gemm_nt(dx_product(p, long(p->bw.T) - 1, 0), s));
     if (ncols > 0) {
         // automatic: what the kernels' schedules make fastest (gemm_tn_plan_splits), at least two 64-row slabs per split
         int want = p->opt_dw_splits > 0 ? p->opt_dw_splits : p->eff_dw;
@@ -1037,7 +1043,8 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, floa
         g.C16 = nullptr; g.C32 = p->dw_part.as<float>(); g.ldc = size_t(ncols);
         g.alpha = 1.f; g.splits = splits; g.split_stride = per;
         g.stamp = stamps_of(p) + kStampBwdDw;
-        FL_TRY(launch_gemm_tn(g, s));
+        if (with_dx) FL_TRY(launch_gemm_tn_and_nt(g, dx_product(p, long(p->bw.T) - 1, 0), s));
+        else FL_TRY(launch_gemm_tn(g, s));
         out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), 0, d.I, invS, accumulate, dW_ih);
         out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), n_ih, d.H, invS, accumulate, dW_hh);
     }
@@ -1072,9 +1079,7 @@ int backward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_
         if (rc) return rc;
         if (st != 0) return FLSTM_E_STALLED;
     }
-    rc = backward_dx(p, long(T) - 1, 0, s);
-    if (rc) return rc;
-    return backward_finish(p, x, x_dtype, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
+    return backward_finish(p, x, x_dtype, true, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
 }
 // ... once the stream has been waited for (as forward_conclude)
 int backward_conclude(flstm_core_plan* p, bool weight_gradients, hipStream_t s) {
@@ -1089,7 +1094,7 @@ int backward_conclude(flstm_core_plan* p, bool weight_gradients, hipStream_t s) 
     pass_done(p, false);
     if (p->opt_profile)
         FL_TRY(hipMemcpy(p->prof_b, p->prof.as<long long>() + 8, sizeof(p->prof_b), hipMemcpyDeviceToHost));
-    const int dw_start = weight_gradients ? kStampBwdDw : kStampBwdEnd;   // (without that product the dX one ends with the pass)
+    const int dw_start = weight_gradients ? kStampBwdDw : kStampBwdEnd;   // (without that product the dX one ends with the pass; where they share a launch bwd_dw is both)
     p->ms_bwd[0] = elapsed(p, kStampBwdStart, kStampBwdRecEnd);
     p->ms_bwd[1] = elapsed(p, kStampBwdRecEnd, dw_start);
     p->ms_bwd[2] = elapsed(p, dw_start, kStampBwdEnd);
@@ -1324,7 +1329,7 @@ extern "C" int flstm_core_backward_end(flstm_core_plan* p, const void* x, flstm_
         if (p->Lb.persistent) demote(p, false);
         return FLSTM_E_STALLED;
     }
-    rc = backward_finish(p, x, x_dtype, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
+    rc = backward_finish(p, x, x_dtype, false, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
     if (rc) return rc;
     rc = wait_stream(s);
     if (rc) return rc;

@@ -31,6 +31,10 @@ hipError_t launch_gemm_nt(const GemmNT& g, hipStream_t stream);
 // (N % 8 == 0); K is arbitrary.  C[M][N] as above.
 hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream);
 
+// A TN product (fp32 partials) and an NT product that do not depend on each other: the same results as the two launches, in one
+// where both are small.
+hipError_t launch_gemm_tn_and_nt(const GemmNT& tn, const GemmNT& nt, hipStream_t stream);
+
 // Number of K slices the launchers really produce when `wanted` are asked for (every slice gets a
 // whole number of 64-wide K slabs). Size split-K partial buffers with this.
 int gemm_effective_splits(int K, int wanted);
@@ -46,6 +50,9 @@ int gemm_tn_tile_size(int M, int N1, int N2, int K, int splits);
 int gemm_tn_plan_splits(int M, int N1, int N2, int K, int max_splits);
 hipError_t launch_gemm_nt_tile(const GemmNT& g, int tile, hipStream_t stream);
 hipError_t launch_gemm_tn_tile(const GemmNT& g, int tile, int splits, int slabs_per_split, hipStream_t stream);
+bool gemm_pair_possible(const GemmNT& tn, int tn_tile, int splits, const GemmNT& nt, int nt_tile);
+hipError_t launch_gemm_pair_tile(const GemmNT& tn, int tn_tile, int splits, int slabs_per_split, const GemmNT& nt, int nt_tile,
+                                 hipStream_t stream);
 // blocks of 32 tiles of 256 x 256 that the large kernels deal to the XCDs for an M x (N1 + N2) product
 long gemm_blocks_of_32(int M, int N1, int N2);
 

@@ -667,13 +667,19 @@ static TileOrder make_order(int tiles_m, int tiles_n, int splits) {
     return o;
 }
 
-hipError_t launch_gemm_nt(const GemmNT& g, hipStream_t stream) {
-    if (g.M <= 0 || g.N <= 0 || g.K <= 0) return hipSuccess;
+static hipError_t check_nt(const GemmNT& g) {
     if (g.K % BK != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0) return hipErrorInvalidValue;
     // (a copy addresses a tile's 256 rows with 32-bit byte offsets from the tile's first row)
     if (g.lda >= (size_t(1) << 22) || g.ldb >= (size_t(1) << 22)) return hipErrorInvalidValue;
     if ((g.C16 == nullptr) == (g.C32 == nullptr)) return hipErrorInvalidValue;
     if (g.bias && (reinterpret_cast<uintptr_t>(g.bias) % 16 != 0 || g.splits > 1)) return hipErrorInvalidValue;
+    return hipSuccess;
+}
+
+hipError_t launch_gemm_nt(const GemmNT& g, hipStream_t stream) {
+    if (g.M <= 0 || g.N <= 0 || g.K <= 0) return hipSuccess;
+    hipError_t e = check_nt(g);
+    if (e != hipSuccess) return e;
     int splits = g.splits < 1 ? 1 : g.splits;
     if (splits > 1 && g.C32 == nullptr) return hipErrorInvalidValue;
     const int nslab = g.K / BK;
@@ -692,7 +698,7 @@ hipError_t launch_gemm_nt(const GemmNT& g, hipStream_t stream) {
     const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
     const TileOrder order = make_order(tiles_m, tiles_n, splits);
     // (set before every launch: the call is cheap, needs no process-wide flag and holds for whichever device is current)
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_nt_stream),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_nt_stream),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(kLdsBytesStream));
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(gemm_nt_stream, dim3(256), dim3(kThreads), kLdsBytesStream, stream, g, order,
@@ -700,8 +706,7 @@ hipError_t launch_gemm_nt(const GemmNT& g, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream) {
-    if (g.M <= 0 || g.N <= 0 || g.K <= 0) return hipSuccess;
+static hipError_t check_tn(const GemmNT& g) {
     if (g.M % 8 != 0 || g.N % 8 != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0 || g.bias) return hipErrorInvalidValue;
     if ((g.C16 == nullptr) == (g.C32 == nullptr)) return hipErrorInvalidValue;
     if (g.C32 && (reinterpret_cast<uintptr_t>(g.C32) % 16 != 0 || g.split_stride % 4 != 0)) return hipErrorInvalidValue;
@@ -715,14 +720,22 @@ hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream) {
     // (a copy addresses a slab's 64 k-rows with 32-bit byte offsets from the slab's first row)
     if (g.lda >= (size_t(1) << 22) || g.ldb >= (size_t(1) << 22) || (g.B2 && g.ldb2 >= (size_t(1) << 22)))
         return hipErrorInvalidValue;
+    if (g.B2 && (g.C32 == nullptr || g.N1 <= 0 || g.N1 >= g.N || g.N1 % 8 != 0 || g.ldb2 % 8 != 0)) return hipErrorInvalidValue;
+    return hipSuccess;
+}
+
+hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream) {
+    if (g.M <= 0 || g.N <= 0 || g.K <= 0) return hipSuccess;
+    hipError_t e = check_tn(g);
+    if (e != hipSuccess) return e;
+    const int splits = g.splits < 1 ? 1 : g.splits;
     const int nslab = (g.K + BK - 1) / BK;
     const int slabs_per_split = (nslab + splits - 1) / splits;
-    if (g.B2 && (g.C32 == nullptr || g.N1 <= 0 || g.N1 >= g.N || g.N1 % 8 != 0 || g.ldb2 % 8 != 0)) return hipErrorInvalidValue;
     if (g.C32) {
         const int tile = gemm_tn_tile_size(g.M, g.B2 ? g.N1 : g.N, g.B2 ? g.N - g.N1 : 0, g.K, splits);
         if (tile != BM) return launch_gemm_tn_tile(g, tile, splits, slabs_per_split, stream);
     }
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tn_stream),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tn_stream),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(kLdsBytesStream));
     if (e != hipSuccess) return e;
     const int tiles_m = (g.M + BM - 1) / BM;
@@ -731,6 +744,26 @@ hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream) {
     hipLaunchKernelGGL(gemm_tn_stream, dim3(256), dim3(kThreads), kLdsBytesStream, stream, g, order,
                        slabs_per_split);
     return hipGetLastError();
+}
+
+// The kernels for small products leave most of the chip idle at their start and end, and between two launches it is idle for
+// another 2 us, so the two of a backward pass share a launch where both run in those kernels (with two workgroups to a CU: the
+// instances for more than 512 tiles of 64 x 64 keep five there, which they would lose).  A 256 x 256 tile's kernel has the chip to
+// itself.  A training pass, two launches -> one: 64 steps of 8 rows x 256 units 240 -> 234 us, 200 of 70 x 257 units 682 -> 667, 256 of
+// 48 x 1536 units (342 + 121 us of products, both with a last round that is half empty) 2148 -> 2060.
+hipError_t launch_gemm_tn_and_nt(const GemmNT& tn, const GemmNT& nt, hipStream_t stream) {
+    if (tn.M > 0 && tn.N > 0 && tn.K > 0 && nt.M > 0 && nt.N > 0 && nt.K > 0 && tn.C32 && nt.splits <= 1) {
+        hipError_t e = check_tn(tn);
+        if (e == hipSuccess) e = check_nt(nt);
+        if (e != hipSuccess) return e;
+        const int splits = tn.splits < 1 ? 1 : tn.splits, nslab = (tn.K + BK - 1) / BK;
+        const int tn_tile = gemm_tn_tile_size(tn.M, tn.B2 ? tn.N1 : tn.N, tn.B2 ? tn.N - tn.N1 : 0, tn.K, splits);
+        const int nt_tile = gemm_nt_tile_size(nt.M, nt.N, nt.K);
+        if (gemm_pair_possible(tn, tn_tile, splits, nt, nt_tile))
+            return launch_gemm_pair_tile(tn, tn_tile, splits, (nslab + splits - 1) / splits, nt, nt_tile, stream);
+    }
+    hipError_t e = launch_gemm_nt(nt, stream);
+    return e != hipSuccess ? e : launch_gemm_tn(tn, stream);
 }
 
 long gemm_blocks_of_32(int M, int N1, int N2) {

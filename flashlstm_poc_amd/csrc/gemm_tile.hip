@@ -80,16 +80,15 @@ constexpr size_t tile_lds_bytes() {
     return slabs > stage ? slabs : stage;
 }
 
-// C[M][N] = alpha * A[M][K] * B[N][K]^T (+ bias), see nt_tile_product.
+// Tile `lin` of C[M][N] = alpha * A[M][K] * B[N][K]^T (+ bias), see nt_tile_product.
 template <int TM, int ST>
-__global__ __launch_bounds__(kTileThreads) void gemm_nt_tile(GemmNT g, int tiles_m, int tiles_n) {
+__device__ __forceinline__ void nt_tile(const GemmNT& g, char* lds, int lin, int tiles_m, int tiles_n) {
     constexpr int MI = TM / 64;                    // 32 x 32 MFMA tiles per wave and direction
-    extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
-    if (g.stamp && blockIdx.x == 0 && tid == 0) *g.stamp = wall_clock64();
+    if (g.stamp && lin == 0 && tid == 0) *g.stamp = wall_clock64();
     int tm, tn;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    tile_of(lin, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * TM, n0 = tn * TM, nk = g.K / BK;
 
     const int wm = wave / 2, wn = wave % 2;
@@ -116,30 +115,29 @@ __global__ __launch_bounds__(kTileThreads) void gemm_nt_tile(GemmNT g, int tiles
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4v lds_short4;
 
-// C[M][N] = alpha * sum_k A[k][m] * B[k][n] over one K split.  Slabs sit in LDS as they sit in memory, 64 k-rows of TM
+// Tile `lin` of C[M][N] = alpha * sum_k A[k][m] * B[k][n] over K split `split`.  Slabs sit in LDS as they sit in memory, 64 k-rows of TM
 // columns per operand; fragments are read with the transposing LDS load (see gemm_tn_stream).  The four k-rows that 32
 // lanes read together are kept in different quarters of a 256-byte bank row: the 64-byte chunk c of k-row r sits at
 // c ^ (r % 4) where a row is 256 bytes, at c ^ (r / 2 % 2) where it is 128 (two rows share a bank row).
 template <int TM, int ST>
-__global__ __launch_bounds__(kTileThreads) void gemm_tn_tile(GemmNT g, int tiles_m, int tiles_n, int slabs_per_split) {
+__device__ __forceinline__ void tn_tile(const GemmNT& g, char* lds, int lin, int split, int tiles_m, int tiles_n, int slabs_per_split) {
     constexpr int MI = TM / 64;
     constexpr int ROWB = TM * 2;                   // bytes of an LDS row
     constexpr int OPERAND = BK * ROWB, SLAB = 2 * OPERAND;
     constexpr int CP = TM / 32;                    // copies per wave, operand and slab
     constexpr int RPC = 1024 / ROWB;               // k-rows per copy
-    extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
-    if (g.stamp && blockIdx.x == 0 && tid == 0) *g.stamp = wall_clock64();
+    if (g.stamp && lin == 0 && tid == 0) *g.stamp = wall_clock64();
     int tm, tn;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    tile_of(lin, tiles_m, tiles_n, tm, tn);
     const int tiles_n1 = g.B2 ? (g.N1 + TM - 1) / TM : (1 << 30);
     const bool side = tn >= tiles_n1;              // columns [N1, N) of C: the second B operand
     const int m0 = tm * TM, n0 = (tn - (side ? tiles_n1 : 0)) * TM;
     const half_t* B = side ? g.B2 : g.B;
     const size_t ldb = side ? g.ldb2 : g.ldb;
     const int nside = g.B2 ? (side ? g.N - g.N1 : g.N1) : g.N;
-    const int slab0 = blockIdx.y * slabs_per_split;
+    const int slab0 = split * slabs_per_split;
     const int nk = min((g.K + BK - 1) / BK - slab0, slabs_per_split);
     if (nk <= 0) return;
 
@@ -233,8 +231,35 @@ __global__ __launch_bounds__(kTileThreads) void gemm_tn_tile(GemmNT g, int tiles
     float* stage = reinterpret_cast<float*>(lds);
     stage32<MI, PITCH>(stage, acc, g.alpha, nullptr, 0, 0, wm * 32 * MI, wn * 32 * MI, lane);
     __syncthreads();
-    float* dst = g.C32 + size_t(blockIdx.y) * g.split_stride + size_t(m0) * g.ldc + n0 + (side ? g.N1 : 0);
+    float* dst = g.C32 + size_t(split) * g.split_stride + size_t(m0) * g.ldc + n0 + (side ? g.N1 : 0);
     store_rows<TM, TM, PITCH>(stage, dst, g.ldc, min(TM, g.M - m0), min(TM, nside - n0), tid);
+}
+
+template <int TM, int ST>
+__global__ __launch_bounds__(kTileThreads) void gemm_nt_tile(GemmNT g, int tiles_m, int tiles_n) {
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    nt_tile<TM, ST>(g, lds, blockIdx.x, tiles_m, tiles_n);
+}
+
+template <int TM, int ST>
+__global__ __launch_bounds__(kTileThreads) void gemm_tn_tile(GemmNT g, int tiles_m, int tiles_n, int slabs_per_split) {
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    tn_tile<TM, ST>(g, lds, blockIdx.x, blockIdx.y, tiles_m, tiles_n, slabs_per_split);
+}
+
+// A TN and an NT product of the same pass in one launch (launch_gemm_tn_and_nt): workgroups [0, tn_first) and those from
+// tn_first + tn_m * tn_n * splits on have the NT product's tiles, those between the TN product's.  tn_first is 0 or all of the NT
+// product's: the product whose tiles take longer comes first, so that the other's fill up its end (297 rows x 1920 units: 120 slabs
+// an NT tile, 5 a TN one).
+struct PairTiles {
+    int tn_m, tn_n, splits, slabs_per_split, nt_m, nt_n, tn_first;
+};
+template <int TN, int SN, int TT, int SS>
+__global__ __launch_bounds__(kTileThreads) void gemm_pair_tile(GemmNT tn, GemmNT nt, PairTiles t) {
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    const int lin = int(blockIdx.x) - t.tn_first, per_split = t.tn_m * t.tn_n, all = per_split * t.splits;
+    if (lin >= 0 && lin < all) tn_tile<TN, SN>(tn, lds, lin % per_split, lin / per_split, t.tn_m, t.tn_n, t.slabs_per_split);
+    else nt_tile<TT, SS>(nt, lds, t.tn_first ? int(blockIdx.x) : lin - all, t.nt_m, t.nt_n);
 }
 
 template <typename K>
@@ -260,6 +285,24 @@ hipError_t run_tn(const GemmNT& g, int splits, int slabs_per_split, hipStream_t 
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((gemm_tn_tile<TM, ST>), dim3(unsigned(tm) * unsigned(tn), unsigned(splits)), dim3(kTileThreads),
                        (tile_lds_bytes<TM, ST>()), s, g, tm, tn, slabs_per_split);
+    return hipGetLastError();
+}
+
+template <int TN, int SN, int TT, int SS>
+hipError_t run_pair(const GemmNT& tn, const GemmNT& nt, int splits, int slabs_per_split, hipStream_t s) {
+    PairTiles t;
+    t.tn_m = (tn.M + TN - 1) / TN;
+    t.tn_n = tn.B2 ? (tn.N1 + TN - 1) / TN + (tn.N - tn.N1 + TN - 1) / TN : (tn.N + TN - 1) / TN;
+    t.splits = splits;
+    t.slabs_per_split = slabs_per_split;
+    t.nt_m = (nt.M + TT - 1) / TT;
+    t.nt_n = (nt.N + TT - 1) / TT;
+    t.tn_first = (nt.K / BK) * TT > slabs_per_split * TN ? t.nt_m * t.nt_n : 0;   // (a slab of a 128 x 128 tile takes twice as long)
+    constexpr size_t lds = tile_lds_bytes<TN, SN>() > tile_lds_bytes<TT, SS>() ? tile_lds_bytes<TN, SN>() : tile_lds_bytes<TT, SS>();
+    hipError_t e = with_lds(gemm_pair_tile<TN, SN, TT, SS>, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((gemm_pair_tile<TN, SN, TT, SS>), dim3(unsigned(t.tn_m) * unsigned(t.tn_n) * unsigned(splits) + unsigned(t.nt_m) * unsigned(t.nt_n)),
+                       dim3(kTileThreads), lds, s, tn, nt, t);
     return hipGetLastError();
 }
 
@@ -334,6 +377,17 @@ hipError_t launch_gemm_tn_tile(const GemmNT& g, int tile, int splits, int slabs_
     const double tiles = (tiles_of(g.M, g.B2 ? g.N1 : g.N, 64) + (g.B2 ? tiles_of(g.M, g.N - g.N1, 64) : 0.0)) * splits;
     if (tile == 64) return tiles <= 512 ? run_tn<64, 4>(g, splits, slabs_per_split, s) : run_tn<64, 2>(g, splits, slabs_per_split, s);
     return run_tn<128, 2>(g, splits, slabs_per_split, s);
+}
+
+bool gemm_pair_possible(const GemmNT& tn, int tn_tile, int splits, const GemmNT& nt, int nt_tile) {
+    const double tn_tiles = (tiles_of(tn.M, tn.B2 ? tn.N1 : tn.N, 64) + (tn.B2 ? tiles_of(tn.M, tn.N - tn.N1, 64) : 0.0)) * splits;
+    return (tn_tile == 128 || (tn_tile == 64 && tn_tiles <= 512)) && (nt_tile == 128 || (nt_tile == 64 && tiles_of(nt.M, nt.N, 64) <= 512));
+}
+hipError_t launch_gemm_pair_tile(const GemmNT& tn, int tn_tile, int splits, int slabs_per_split, const GemmNT& nt, int nt_tile,
+                                 hipStream_t s) {
+    if (tn_tile == 64)
+        return nt_tile == 64 ? run_pair<64, 4, 64, 4>(tn, nt, splits, slabs_per_split, s) : run_pair<64, 4, 128, 2>(tn, nt, splits, slabs_per_split, s);
+    return nt_tile == 64 ? run_pair<128, 2, 64, 4>(tn, nt, splits, slabs_per_split, s) : run_pair<128, 2, 128, 2>(tn, nt, splits, slabs_per_split, s);
 }
 
 }  // namespace flstm_hip
