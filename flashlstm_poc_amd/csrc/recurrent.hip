@@ -4175,7 +4175,7 @@ hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
         // weights: one built for 1024 units spends the same time per step at 256.  So there is one per 256 units (with
         // two row tiles, where the product is the smaller part, per 512).  Measured, us per step, forward / backward, one kernel for all
         // -> this: 256 units and 8 rows 1.76 / 2.44 -> 1.50 / 1.82, 512 and 64 rows 1.84 / 2.90 -> 1.64 / 2.16, 672
-        // and 20 rows 1.91 / 2.97 -> 1.74 / 2.54, 1536 and 48 rows 3.18 / 6.74 -> 2.90 / 5.73.
+        // and 20 rows 1.91 / 2.97 -> 1.74 / 2.54.
         if (L.mt == 1) {
             if (ks <= 2) return run_fwd_ds<8, 2, 1>(L, a, ds, stream, graphs);
             if (ks <= 4) return run_fwd_ds<8, 4, 1>(L, a, ds, stream, graphs);
