@@ -197,6 +197,7 @@ int publish_with(flstm_core_plan* p, OpList& last, int stamp, hipStream_t s) {
     last.stamps = stamps_of(p);
     last.stamp = stamp;
     last.publish = p->status_host;
+    if (last.only_if_ok && p->inject_stall > 0) FL_TRY(fill_words(p->status.p, sizeof(int), 1u, s));   // (take_status would be too late)
     FL_TRY(run_ops(last, s));
     return 0;
 }
@@ -208,9 +209,9 @@ int wait_stream(hipStream_t s) {
 int take_status(flstm_core_plan* p, hipStream_t s, int* out) {
     *out = *static_cast<volatile int*>(&p->status_host->status);
     if (*out != 0) FL_TRY(fill_zero(p->status.p, sizeof(int), s));
-    if (*out == 0 && p->inject_stall > 0) {   // (2 in a row: the step-wise repeat of a pass fails too, i.e. the call does)
+    if (p->inject_stall > 0) {   // (2 in a row: the step-wise repeat of a pass fails too, i.e. the call does)
         p->inject_stall--;
-        *out = 1;
+        if (*out == 0) *out = 1;
     }
     return 0;
 }
@@ -746,6 +747,7 @@ int forward_outputs(flstm_core_plan* p, size_t TB, void* y, flstm_dtype y_dtype,
                     hipStream_t s) {
     const Dims& d = p->d;
     OpList out;
+    out.only_if_ok = p->fw.behind;
     out.unpad(p->Y.as<half_t>() + size_t(d.B) * d.Hp, 0, size_t(d.Hp), TB, d.H, 1.f, y, y_dtype == FLSTM_F32);
     final_states(p, TB, hy, cy, out_state_dtype, out);
     return publish_with(p, out, kStampFwdEnd, s);
@@ -753,7 +755,8 @@ int forward_outputs(flstm_core_plan* p, size_t TB, void* y, flstm_dtype y_dtype,
 
 // One whole forward pass, enqueued: projection, recurrence, outputs, status.  The outputs are written behind the
 // recurrence without waiting for its status: if the persistent launch gave up, the whole pass is repeated step-wise
-// and overwrites them.
+// and overwrites them -- unless one of them lies in an input, which the repeat will read: then the launch that writes them looks
+// at the status first.
 // A caller may hand over outputs that lie in inputs: the state carried in place (hy is h0, cy is c0), y over x.  Within the
 // recurrence's launch nothing orders one workgroup's outputs behind another's reads of h0 (a single step has no exchange) or of
 // x (rows read by the projection's tiles, or a step ahead), so such a pass writes only the plan's own arrays there, as one that
@@ -1089,8 +1092,8 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, bool
 
 // One whole backward pass, enqueued.  dX and the weight gradients follow the recurrence without waiting for its status
 // (one wait per pass); a persistent launch that gave up is found at the end and the pass repeated step-wise over the
-// same outputs.  Only when the caller's gradients are added to (accumulate_grads) the status is checked first
-// (FLSTM_E_STALLED).
+// same outputs.  Only when the caller's gradients are added to (accumulate_grads), or an output lies in an input of the
+// recurrence (dh0 in d_hn's place, dx in dY's), the status is checked first (FLSTM_E_STALLED).
 int backward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* dY, flstm_dtype dy_dtype,
                      const void* d_hn, const void* d_cn, flstm_dtype dstate_dtype, const BwdScales& k, void* dx,
                      flstm_dtype dx_dtype, float* dW_ih, float* dW_hh, float* db_ih, float* db_hh, float* dh0, float* dc0,
@@ -1105,7 +1108,10 @@ int backward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_
         rc = backward_rec_once(p, T, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, s);
     }
     if (rc) return rc;
-    if (p->opt_accumulate) {
+    const Dims& d = p->d;
+    const size_t TB = T * size_t(d.B), BH = size_t(d.B) * d.H;
+    if (p->opt_accumulate || overlap({bytes_of(dx, TB * d.I, dx_dtype), bytes_of(dh0, BH, FLSTM_F32), bytes_of(dc0, BH, FLSTM_F32)},
+                                     {bytes_of(dY, TB * d.H, dy_dtype), bytes_of(d_hn, BH, dstate_dtype), bytes_of(d_cn, BH, dstate_dtype)})) {
         int st = 0;
         OpList nothing;
         rc = wait_status(p, nothing, -1, s, &st);
@@ -1135,6 +1141,22 @@ int backward_conclude(flstm_core_plan* p, bool weight_gradients, hipStream_t s) 
     return 0;
 }
 
+int backward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* dY, flstm_dtype dy_dtype,
+                  const void* d_hn, const void* d_cn, flstm_dtype dstate_dtype, const BwdScales& k, void* dx,
+                  flstm_dtype dx_dtype, float* dW_ih, float* dW_hh, float* db_ih, float* db_hh, float* dh0, float* dc0,
+                  hipStream_t s) {
+    for (int attempt = 0;; ++attempt) {
+        int rc = backward_enqueue(p, T, x, x_dtype, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, dW_ih, dW_hh, db_ih,
+                                  db_hh, dh0, dc0, s);
+        if (rc == 0) rc = wait_stream(s);
+        const bool persistent = p->Lb.persistent != 0;
+        if (rc == 0) rc = backward_conclude(p, dW_ih || dW_hh, s);
+        else if (rc == FLSTM_E_STALLED && persistent) demote(p, false);   // (the check ahead of accumulation)
+        p->bw.open = false;
+        if (rc != FLSTM_E_STALLED || !persistent || attempt > 0) return rc;
+    }
+}
+
 }  // namespace
 
 extern "C" int flstm_core_backward(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype,
@@ -1148,18 +1170,8 @@ extern "C" int flstm_core_backward(flstm_core_plan* p, size_t T, const void* x, 
     if (!dY) return FLSTM_E_INVALID;
     if (dW_ih && !x) return FLSTM_E_INVALID;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const float S = grad_scale > 0.f ? grad_scale : 1.f;
-    const BwdScales k = BwdScales::loss_scale(S);
-    for (int attempt = 0;; ++attempt) {
-        int rc = backward_enqueue(p, T, x, x_dtype, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, dW_ih, dW_hh, db_ih,
-                                  db_hh, dh0, dc0, s);
-        if (rc == 0) rc = wait_stream(s);
-        const bool persistent = p->Lb.persistent != 0;
-        if (rc == 0) rc = backward_conclude(p, dW_ih || dW_hh, s);
-        else if (rc == FLSTM_E_STALLED && persistent) demote(p, false);   // (the check ahead of accumulation)
-        p->bw.open = false;
-        if (rc != FLSTM_E_STALLED || !persistent || attempt > 0) return rc;
-    }
+    const BwdScales k = BwdScales::loss_scale(grad_scale > 0.f ? grad_scale : 1.f);
+    return backward_pass(p, T, x, x_dtype, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
 }
 
 // ---- stacks of layers: the same passes, layer behind layer on one stream with ONE wait at the end
@@ -1183,17 +1195,33 @@ extern "C" int flstm_stack_forward(flstm_core_plan* const* plans, int layers, si
         if (!p || !ys[l] || p->d.B != plans[0]->d.B || p->d.H != plans[0]->d.H || (l > 0 && p->d.I != p->d.H)) return FLSTM_E_INVALID;
         if (!p->weights_packed || !p->bias_packed) return FLSTM_E_NOT_PACKED;
     }
-    const size_t state_in = size_t(plans[0]->d.B) * plans[0]->d.H * (state_dtype == FLSTM_F32 ? 4 : 2);
-    const size_t state_out = size_t(plans[0]->d.B) * plans[0]->d.H * (y_dtype == FLSTM_F32 ? 4 : 2);
+    const size_t TB = T * size_t(plans[0]->d.B), BH = size_t(plans[0]->d.B) * plans[0]->d.H;
+    const size_t state_in = BH * (state_dtype == FLSTM_F32 ? 4 : 2), state_out = BH * (y_dtype == FLSTM_F32 ? 4 : 2);
     auto at = [](const void* base, size_t off) -> const void* { return base ? static_cast<const char*>(base) + off : nullptr; };
     auto layer = [&](int l, auto&& pass) -> int {
         return pass(plans[l], T, l == 0 ? x : ys[l - 1], l == 0 ? x_dtype : y_dtype, at(h0, l * state_in), at(c0, l * state_in),
                     state_dtype, ys[l], y_dtype, const_cast<void*>(at(hy, l * state_out)), const_cast<void*>(at(cy, l * state_out)), y_dtype, true, s);
     };
     int rc = 0;
+    // Where an output lies in what a layer reads -- the states carried in place, one layer's rows over another's --, a layer that
+    // gave up could not be repeated once the layers above it have run: each is waited for then.
+    bool in_place = overlap({bytes_of(hy, layers * BH, y_dtype), bytes_of(cy, layers * BH, y_dtype)},
+                            {bytes_of(x, TB * plans[0]->d.I, x_dtype), bytes_of(h0, layers * BH, state_dtype), bytes_of(c0, layers * BH, state_dtype)});
+    for (int l = 0; l < layers; ++l) {
+        const Bytes rows = bytes_of(ys[l], TB * plans[0]->d.H, y_dtype);
+        in_place = in_place || overlap({rows}, {bytes_of(x, TB * plans[0]->d.I, x_dtype), bytes_of(h0, layers * BH, state_dtype), bytes_of(c0, layers * BH, state_dtype)});
+        for (int m = 0; m < l; ++m) in_place = in_place || overlap({rows}, {bytes_of(ys[m], TB * plans[0]->d.H, y_dtype)});
+    }
     for (int l = 0; l < layers && rc == 0; ++l) {
         plans[l]->have_cache = false;
-        rc = layer(l, forward_enqueue);
+        rc = in_place ? layer(l, forward_pass) : layer(l, forward_enqueue);
+    }
+    if (in_place) {
+        for (int l = 0; l < layers; ++l) {
+            plans[l]->fw.open = false;
+            if (rc == 0) { plans[l]->have_cache = true; plans[l]->T_cache = T; }
+        }
+        return rc;
     }
     const int waited = wait_stream(s);
     if (rc == 0) rc = waited;
@@ -1230,16 +1258,33 @@ extern "C" int flstm_stack_backward(flstm_core_plan* const* plans, int layers, s
     }
     // from layer to layer gradients stay fp16 with the loss scale on them; it is divided out of everything returned
     const float S = loss_scale > 0.f ? loss_scale : 1.f;
-    auto layer = [&](int l) -> int {
+    auto layer = [&](int l, auto&& pass) -> int {
         const bool top = l == layers - 1;
         const BwdScales k{top ? dy_scale : 1.f, S, l == 0 ? 1.f / S : 1.f, 1.f / S};
-        return backward_enqueue(plans[l], T, xs[l], l == 0 ? x_dtype : FLSTM_F16, top ? dY : dxs[l + 1], top ? dy_dtype : FLSTM_F16,
+        return pass(plans[l], T, xs[l], l == 0 ? x_dtype : FLSTM_F16, top ? dY : dxs[l + 1], top ? dy_dtype : FLSTM_F16,
                                 d_hn ? d_hn[l] : nullptr, d_cn ? d_cn[l] : nullptr, dstate_dtype, k, dxs[l], l == 0 ? dx_dtype : FLSTM_F16,
                                 dW_ih[l], dW_hh[l], db_ih[l], db_hh ? db_hh[l] : nullptr, dh0[l], dc0[l], s);
     };
     int rc = 0, from = layers - 1;
+    // (as forward: gradients over gradients that a layer above has yet to be repeated from, one buffer for the dxs of several layers)
+    bool in_place = false;
+    for (int l = 0; l < layers && !in_place; ++l) {
+        const Dims& d = plans[l]->d;
+        const size_t TB = T * size_t(d.B), BH = size_t(d.B) * d.H;
+        auto dx_of = [&](int m) { return bytes_of(dxs[m], TB * plans[m]->d.I, m == 0 ? dx_dtype : FLSTM_F16); };
+        for (int m = 0; m < layers && !in_place; ++m) {
+            in_place = overlap({dx_of(l), bytes_of(dh0[l], BH, FLSTM_F32), bytes_of(dc0[l], BH, FLSTM_F32)},
+                               {bytes_of(dY, TB * d.H, dy_dtype), bytes_of(xs[m], TB * plans[m]->d.I, m == 0 ? x_dtype : FLSTM_F16), bytes_of(d_hn ? d_hn[m] : nullptr, BH, dstate_dtype),
+                                bytes_of(d_cn ? d_cn[m] : nullptr, BH, dstate_dtype)}) ||
+                       (m < l && overlap({dx_of(l)}, {dx_of(m)}));
+        }
+    }
+    if (in_place) {
+        for (int l = from; l >= 0 && rc == 0; --l) rc = layer(l, backward_pass);
+        return rc;
+    }
     for (int attempt = 0;; ++attempt) {   // a layer that gave up is repeated step-wise, and every layer below it with it
-        for (int l = from; l >= 0 && rc == 0; --l) rc = layer(l);
+        for (int l = from; l >= 0 && rc == 0; --l) rc = layer(l, backward_enqueue);
         const int waited = wait_stream(s);
         if (rc == 0) rc = waited;
         bool again = false;
@@ -1304,6 +1349,7 @@ extern "C" int flstm_core_forward_end(flstm_core_plan* p, void* hy, void* cy, fl
     const size_t TB = p->fw.T * size_t(d.B);
     p->fw.open = false;
     OpList out;
+    out.only_if_ok = true;   // (a window's state may be carried in place, and the repeat reads it)
     final_states(p, TB, hy, cy, out_state_dtype, out);
     int st = 0;
     int rc = wait_status(p, out, kStampFwdEnd, s, &st);

@@ -81,6 +81,7 @@ struct OpList {
     const int* status = nullptr;      // device status word (with `publish`)
     long long* stamps = nullptr;
     HostStatus* publish = nullptr;
+    bool only_if_ok = false;          // (with `status`) the operations are left out if that word is not 0
     LayoutOp op[kMaxOps];
 
     void fill(void* p, size_t bytes, unsigned word);   // bytes: a multiple of 4

@@ -225,7 +225,7 @@ __device__ __forceinline__ void op_reduce_dw(const LayoutOp& o, size_t first, si
 __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
     int which = 0;
     while (which + 1 < list.count && blockIdx.x >= list.op[which + 1].first_block) ++which;
-    if (list.count > 0) {
+    if (list.count > 0 && !(list.only_if_ok && *list.status != 0)) {
         const LayoutOp& o = list.op[which];
         const size_t stride = size_t(o.blocks) * kT;
         const size_t first = size_t(blockIdx.x - o.first_block) * kT + threadIdx.x;

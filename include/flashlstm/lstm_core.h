@@ -90,7 +90,8 @@ int flstm_core_pack_bias(flstm_core_plan* plan, const float* b_ih, const float* 
 
 /* Forward over T steps.  h0/c0 may be null (zeros).  y, hy, cy may be null (not written).
  * Outputs may lie in inputs (hy in h0's place, cy in c0's, y in x's), whole or in part and whatever the element types: the
- * caller's tensors are then written once everything has been read, by one launch more.  Outputs must not lie in each other.
+ * caller's tensors are then written once everything has been read and the pass is known to have gone through, by one launch
+ * more.  Outputs must not lie in each other, but for hy as the last rows of a y of its type.
  * With save_for_backward != 0 the plan keeps the fp16 gate cache (activated i,f,g,o), the fp32
  * cell states and the fp16 outputs of this call for flstm_core_backward. */
 int flstm_core_forward(flstm_core_plan* plan, size_t seq_len,
@@ -122,7 +123,9 @@ int flstm_core_forward_static(flstm_core_plan* plan, size_t seq_len,
 /* BPTT for the last forward of this plan.  d_hn/d_cn may be null (zeros).  Any output may be null.
  * grad_scale (a power of two, 1 if <= 0) multiplies dY on load and is divided out of every
  * output; use it when dY is too small for fp16 pre-activation gradients.
- * db_ih and db_hh receive the same values. */
+ * db_ih and db_hh receive the same values.
+ * dx may lie in dY's place, dh0 and dc0 in those of d_hn and d_cn (the call then waits for the recurrence before it writes);
+ * dx must not lie in x. */
 int flstm_core_backward(flstm_core_plan* plan, size_t seq_len,
                         const void* x, flstm_dtype x_dtype,
                         const void* dY, flstm_dtype dy_dtype,
@@ -141,7 +144,8 @@ int flstm_core_backward(flstm_core_plan* plan, size_t seq_len,
  *   dy_scale * dY, where dy_scale contains loss_scale (a power of two) already; d_hn / d_cn may be null, their entries too.
  *   Gradients travel between layers in fp16 (dxs[l], l > 0) with the loss scale on them; it is divided out of dxs[0]
  *   (dx_dtype, may be null) and of everything else returned.  db_ih and db_hh receive the same values (db_hh may be null).
- *   Not with "accumulate_grads". */
+ *   Not with "accumulate_grads".
+ * Where an output lies in an input, or rows or gradients of several layers in one buffer, the layers are waited for one by one. */
 int flstm_stack_forward(flstm_core_plan* const* plans, int layers, size_t seq_len, const void* x, flstm_dtype x_dtype,
                         const void* h0, const void* c0, flstm_dtype state_dtype, void* const* ys, flstm_dtype y_dtype,
                         void* hy, void* cy, void* stream);
@@ -165,7 +169,8 @@ int flstm_core_absmax(flstm_core_plan* plan, const void* tensor, flstm_dtype dty
  * _steps calls only enqueue work.  forward ranges go from step 0 upwards and must cover [0, T) in order;
  * backward ranges go from step T-1 downwards.  _end waits, returns FLSTM_E_STALLED if a persistent launch
  * gave up (repeat the pass with flstm_core_forward / flstm_core_backward, which fall back to step-wise
- * launches), and otherwise finishes the pass (final states; weight and bias gradients). */
+ * launches), and otherwise finishes the pass (final states; weight and bias gradients).  hy may lie in h0's place, cy in c0's;
+ * dx and dY must be buffers of their own. */
 int flstm_core_forward_begin(flstm_core_plan* plan, size_t seq_len, const void* x, flstm_dtype x_dtype,
                              const void* h0, const void* c0, flstm_dtype state_dtype, void* stream);
 int flstm_core_forward_steps(flstm_core_plan* plan, size_t t0, size_t nsteps, void* stream);
