@@ -1204,13 +1204,14 @@ extern "C" int flstm_stack_forward(flstm_core_plan* const* plans, int layers, si
     };
     int rc = 0;
     // Where an output lies in what a layer reads -- the states carried in place, one layer's rows over another's --, a layer that
-    // gave up could not be repeated once the layers above it have run: each is waited for then.
+    // gave up could not be repeated once the layers above it have run: each is waited for then.  So it is where a plan stands for
+    // several layers (weights that they share): what a plan knows of its pass -- the status, the ring's slot -- is that of one pass.
     bool in_place = overlap({bytes_of(hy, layers * BH, y_dtype), bytes_of(cy, layers * BH, y_dtype)},
                             {bytes_of(x, TB * plans[0]->d.I, x_dtype), bytes_of(h0, layers * BH, state_dtype), bytes_of(c0, layers * BH, state_dtype)});
     for (int l = 0; l < layers; ++l) {
         const Bytes rows = bytes_of(ys[l], TB * plans[0]->d.H, y_dtype);
         in_place = in_place || overlap({rows}, {bytes_of(x, TB * plans[0]->d.I, x_dtype), bytes_of(h0, layers * BH, state_dtype), bytes_of(c0, layers * BH, state_dtype)});
-        for (int m = 0; m < l; ++m) in_place = in_place || overlap({rows}, {bytes_of(ys[m], TB * plans[0]->d.H, y_dtype)});
+        for (int m = 0; m < l; ++m) in_place = in_place || plans[m] == plans[l] || overlap({rows}, {bytes_of(ys[m], TB * plans[0]->d.H, y_dtype)});
     }
     for (int l = 0; l < layers && rc == 0; ++l) {
         plans[l]->have_cache = false;

@@ -145,7 +145,9 @@ int flstm_core_backward(flstm_core_plan* plan, size_t seq_len,
  *   Gradients travel between layers in fp16 (dxs[l], l > 0) with the loss scale on them; it is divided out of dxs[0]
  *   (dx_dtype, may be null) and of everything else returned.  db_ih and db_hh receive the same values (db_hh may be null).
  *   Not with "accumulate_grads".
- * Where an output lies in an input, or rows or gradients of several layers in one buffer, the layers are waited for one by one. */
+ * Where an output lies in an input, or rows or gradients of several layers in one buffer, the layers are waited for one by one.
+ * Forward, a plan may stand for several layers (weights that they share; waited for one by one too).  It keeps the caches of the
+ * last of them alone, so a backward pass wants a plan per layer. */
 int flstm_stack_forward(flstm_core_plan* const* plans, int layers, size_t seq_len, const void* x, flstm_dtype x_dtype,
                         const void* h0, const void* c0, flstm_dtype state_dtype, void* const* ys, flstm_dtype y_dtype,
                         void* hy, void* cy, void* stream);

@@ -157,3 +157,31 @@ def test_stacked_module_trains_like_torch_lstm():
     with pytest.raises(RuntimeError, match="most recent forward"):
         y_old.sum().backward()
     mod.release()
+
+
+def test_layers_that_share_a_plan():
+    """One plan for several layers, forward: an even number of steps (the ring of a whole pass then ends on another slot than it began on),
+    call after call, also with a launch that gives up."""
+    from flashlstm_poc_amd import LstmCore
+    from flashlstm_poc_amd.stack import _pointers
+    T, B, H, L = 6, 20, 64, 3
+    g = torch.Generator(device="cuda").manual_seed(11)
+    normal = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    core = LstmCore(B, H, H)
+    core.pack(normal(4 * H, H) * 0.1, normal(4 * H, H) * 0.1, normal(4 * H) * 0.1, normal(4 * H) * 0.1)
+    lib, s = core.lib, torch.cuda.current_stream().cuda_stream
+    for call in range(5):
+        x, h, c = normal(T, B, H).half(), normal(L, B, H).half(), normal(L, B, H).half()
+        want, rows = [], x
+        for l in range(L):
+            want.append(core.forward(rows, h[l], c[l]))
+            rows = want[-1][0]
+        if call == 3:
+            core.set_option("inject_stall", 1)
+        ys, hy, cy = [torch.empty_like(x) for _ in range(L)], torch.empty_like(h), torch.empty_like(c)
+        assert lib.flstm_stack_forward((type(core._h) * L)(*[core._h] * L), L, T, x.data_ptr(), 1,
+                                       h.data_ptr(), c.data_ptr(), 1, _pointers(ys), 1, hy.data_ptr(), cy.data_ptr(), s) == 0
+        for l in range(L):
+            assert torch.equal(ys[l], want[l][0]) and torch.equal(hy[l], want[l][1]) and torch.equal(cy[l], want[l][2]), (call, l)
+        assert core.info("fallbacks") == (call >= 3)
+    core.close()
