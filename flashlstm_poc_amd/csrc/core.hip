@@ -138,7 +138,8 @@ struct flstm_core_plan {
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
              half_t* y_direct = nullptr;   // the recurrence writes the caller's y itself
              bool whole = false;           // one launch (forward_whole)
-             bool behind = false; } fw;    // the caller's outputs are written by a launch of their own behind the recurrence
+             bool behind = false;          // the caller's final states are written by a launch of their own behind the recurrence ...
+             bool rows_behind = false; } fw;   // ... and y with them
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
              BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
     DevBuf tile_words;         // ProjectBeside::ready
@@ -395,6 +396,7 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
         return long(sum);
     }
     if (!strcmp(name, "outputs_behind")) return p->fw.behind;
+    if (!strcmp(name, "rows_behind")) return p->fw.rows_behind;
     if (!strcmp(name, "slice_fwd")) return p->Lf.jb;
     if (!strcmp(name, "slice_bwd")) return p->Lb.jb;
     if (!strcmp(name, "groups_fwd")) return p->Lf.ng;
@@ -761,7 +763,10 @@ int forward_outputs(flstm_core_plan* p, size_t TB, void* y, flstm_dtype y_dtype,
 // recurrence's launch nothing orders one workgroup's outputs behind another's reads of h0 (a single step has no exchange) or of
 // x (rows read by the projection's tiles, or a step ahead), so such a pass writes only the plan's own arrays there, as one that
 // saves its caches does, and the caller's tensors are written by a launch behind it: one step of a row of 256 units takes 27.8 us
-// with its state in place, 21.5 with outputs of its own, 37 as separate launches throughout.
+// with its state in place, 21.5 with outputs of its own, 37 as separate launches throughout.  A recurrence of separate launches,
+// whose states leave in a launch behind it anyway, goes on writing a y that lies in no input (512 steps of 64 rows of 1024 units
+// with the state in place 976 -> 955 us).  A whole pass does not: 64 steps of 64 rows of 256 units take 84 us with y copied, 88
+// with y and the caches both written from within.
 int forward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
                     flstm_dtype state_dtype, void* y, flstm_dtype y_dtype, void* hy, void* cy,
                     flstm_dtype out_state_dtype, bool save, hipStream_t s) {
@@ -769,10 +774,13 @@ int forward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_d
     const size_t TB = T * size_t(d.B);
     use_tuned(p, T);
     p->fw.whole = false;
-    const bool behind = overlap({bytes_of(y, TB * d.H, y_dtype), bytes_of(hy, size_t(d.B) * d.H, out_state_dtype), bytes_of(cy, size_t(d.B) * d.H, out_state_dtype)},
-                                {bytes_of(x, TB * d.I, x_dtype), bytes_of(h0, size_t(d.B) * d.H, state_dtype), bytes_of(c0, size_t(d.B) * d.H, state_dtype)});
+    const size_t BH = size_t(d.B) * d.H;
+    const auto inputs = {bytes_of(x, TB * d.I, x_dtype), bytes_of(h0, BH, state_dtype), bytes_of(c0, BH, state_dtype)};
+    const bool rows_behind = overlap({bytes_of(y, TB * d.H, y_dtype)}, inputs);
+    const bool behind = rows_behind || overlap({bytes_of(hy, BH, out_state_dtype), bytes_of(cy, BH, out_state_dtype)}, inputs);
     p->fw.behind = behind;
     if (whole_possible(p)) {
+        p->fw.rows_behind = behind;
         const int rc = behind ? forward_whole(p, T, x, x_dtype, h0, c0, state_dtype, nullptr, y_dtype, nullptr, nullptr, out_state_dtype, true, s)
                               : forward_whole(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, save, s);
         if (rc == 0 && behind) return forward_outputs(p, TB, y, y_dtype, hy, cy, out_state_dtype, s);
@@ -786,8 +794,9 @@ int forward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_d
     // Step-wise launches leave it to the copy: every argument of theirs is then plan-owned, and the graph they were
     // captured into can be replayed on the next pass.
     half_t* const y_direct =
-        (y && y_dtype == FLSTM_F16 && d.H == d.Hp && p->Lf.persistent && !behind) ? static_cast<half_t*>(y) : nullptr;
+        (y && y_dtype == FLSTM_F16 && d.H == d.Hp && p->Lf.persistent && !rows_behind) ? static_cast<half_t*>(y) : nullptr;
     p->fw.y_direct = y_direct;
+    p->fw.rows_behind = behind && y && !y_direct;
     int rc = forward_once(p, T, x, x_dtype, h0, c0, state_dtype, s);
     p->fw.y_direct = nullptr;
     if (rc) return rc;
@@ -1329,7 +1338,8 @@ extern "C" int flstm_core_forward_begin(flstm_core_plan* p, size_t T, const void
     p->have_cache = false;
     for (float& m : p->ms_fwd) m = -1.f;
     use_tuned(p, T);
-    p->fw.behind = true;   // (flstm_core_forward_end)
+    p->fw.behind = true;   // (flstm_core_forward_end; the rows are the caller's to fetch)
+    p->fw.rows_behind = false;
     return forward_setup(p, T, x, x_dtype, h0, c0, state_dtype, false, static_cast<hipStream_t>(stream));
 }
 

@@ -77,7 +77,8 @@ int flstm_core_set_option(flstm_core_plan* plan, const char* name, long value);
  * 4 or 8), "row_tiles_fwd", "row_tiles_bwd" (16-row tiles per row block that the
  * recurrences run with; "row_tiles": the forward one), "hidden_padded",
  * "input_padded", "outputs_behind" (the last forward pass wrote the caller's outputs by a launch of its own behind the
- * recurrence, because one of them lay in an input or the pass came in ranges of steps; else 0), "device_bytes" (device memory the plan holds), "static_scratch_bytes" (size of the fixed scratch
+ * recurrence, because one of them lay in an input or the pass came in ranges of steps; else 0), "rows_behind" (the
+ * same, and y was among them), "device_bytes" (device memory the plan holds), "static_scratch_bytes" (size of the fixed scratch
  * array of flstm_core_forward_static), "num_cus" and "clock_khz" (compute units and
  * maximum engine clock of the plan's device).
  * Unknown names give -1. */
@@ -90,8 +91,8 @@ int flstm_core_pack_bias(flstm_core_plan* plan, const float* b_ih, const float* 
 
 /* Forward over T steps.  h0/c0 may be null (zeros).  y, hy, cy may be null (not written).
  * Outputs may lie in inputs (hy in h0's place, cy in c0's, y in x's), whole or in part and whatever the element types: the
- * caller's tensors are then written once everything has been read and the pass is known to have gone through, by one launch
- * more.  Outputs must not lie in each other, but for hy as the last rows of a y of its type.
+ * outputs -- but for a y that lies in no input -- are then written once everything has been read and the pass is known to have gone
+ * through, by one launch more.  Outputs must not lie in each other, but for hy as the last rows of a y of its type.
  * With save_for_backward != 0 the plan keeps the fp16 gate cache (activated i,f,g,o), the fp32
  * cell states and the fp16 outputs of this call for flstm_core_backward. */
 int flstm_core_forward(flstm_core_plan* plan, size_t seq_len,

@@ -181,3 +181,23 @@ def test_stack_in_place(stalled):
     for mine, theirs in zip(grads, want[1]):
         assert all(torch.equal(a, b) for a, b in zip(mine, theirs))
     stack.close()
+
+
+# y apart from the inputs is written by the recurrence of separate launches, whatever becomes of the states
+@pytest.mark.parametrize("T,B,I,H", [(100, 32, 512, 1024), (20, 40, 96, 640)])
+def test_rows_apart_from_the_inputs_are_not_copied(T, B, I, H):
+    import torch
+    core, normal = made(B, I, H, seed=T + H)
+    x, h, c = normal(T, B, I).half(), normal(B, H).half(), normal(B, H).half()
+    empty = lambda *s: torch.empty(*s, device="cuda", dtype=torch.float16)
+    want, y, rows = [empty(T, B, H), empty(B, H), empty(B, H)], empty(T, B, H), empty(T, B, H)
+    core.forward(x, h, c, save_for_backward=False)   # (as in test_outputs_anywhere_in_the_inputs)
+    core.forward_static(x, h, c, *want)
+    assert core.info("outputs_behind") == 0 and core.info("rows_behind") == 0
+    rows[-1].copy_(h)
+    core.forward_static(x, rows[-1], c, rows, empty(B, H), empty(B, H))   # y over h0
+    assert core.info("outputs_behind") == 1 and core.info("rows_behind") == 1 and torch.equal(rows, want[0])
+    core.forward_static(x, h, c, y, h, c)
+    assert core.info("outputs_behind") == 1 and core.info("rows_behind") == 0 and core.info("fallbacks") == 0
+    assert all(torch.equal(a, b) for a, b in zip((y, h, c), want))
+    core.close()
