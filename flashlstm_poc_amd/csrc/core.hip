@@ -138,10 +138,12 @@ struct flstm_core_plan {
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
              half_t* y_direct = nullptr;   // the recurrence writes the caller's y itself
              bool whole = false;           // one launch (forward_whole)
+             int projection = 0;           // where the x-projection is formed: 0 in front of the recurrence, 1 beside it, 2 inside its launch
              bool behind = false;          // the caller's final states are written by a launch of their own behind the recurrence ...
              bool rows_behind = false; } fw;   // ... and y with them
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
-             BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false; } bw;
+             BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false;
+             bool shared = false; } bw;   // dX and the weight gradients in one launch
     DevBuf tile_words;         // ProjectBeside::ready
     unsigned tile_mark = 0;    // ... of the last launch
     ProjectBeside project;     // for the next forward recurrence launch
@@ -395,6 +397,9 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
             sum += b->bytes;
         return long(sum);
     }
+    if (!strcmp(name, "whole_fwd")) return p->fw.whole;
+    if (!strcmp(name, "projection_fwd")) return p->fw.projection;
+    if (!strcmp(name, "products_shared")) return p->bw.shared;
     if (!strcmp(name, "outputs_behind")) return p->fw.behind;
     if (!strcmp(name, "rows_behind")) return p->fw.rows_behind;
     if (!strcmp(name, "slice_fwd")) return p->Lf.jb;
@@ -584,6 +589,7 @@ int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, boo
     g.alpha = 1.f; g.splits = 1; g.split_stride = 0;
     g.bias = p->bias_p.as<float>();   // b_ih + b_hh, packed gate order: the recurrence reads x-projection + bias
     p->project = ProjectBeside{};
+    p->fw.projection = 0;
     if (may_leave_it && projects_beside(p, n, g.A)) {
         const size_t words = ceil_div(size_t(g.M), 128) * (g.N / 128) * sizeof(unsigned);
         if (words <= p->tile_words.bytes || !p->static_call) {
@@ -597,6 +603,7 @@ int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, boo
             p->project.ready = p->tile_words.as<unsigned>();
             p->project.mark = ++p->tile_mark;
             rec_share_columns(p->Lf, p->project);
+            p->fw.projection = 1;
             return 0;
         }
     }
@@ -719,6 +726,7 @@ int forward_whole(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     }
     a.G = p->G.as<half_t>();
     FL_TRY(run_ops(prep, s));
+    p->fw.projection = 2;
     if (!projects) {
         a.x = nullptr;
         const int rc = forward_project(p, 0, T, true, false, s);
@@ -1064,6 +1072,7 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, bool
     const bool accumulate = p->opt_accumulate != 0;
     OpList out;   // gradients into the caller's layout, one launch
     with_dx = with_dx && p->bw.dx;
+    p->bw.shared = false;
     if (with_dx && ncols == 0) FL_TRY(launch_gemm_nt(dx_product(p, long(p->bw.T) - 1, 0), s));
     if (ncols > 0) {
         // automatic: what the kernels' schedules make fastest (gemm_tn_plan_splits), at least two 64-row slabs per split
@@ -1088,7 +1097,7 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, bool
         g.C16 = nullptr; g.C32 = p->dw_part.as<float>(); g.ldc = size_t(ncols);
         g.alpha = 1.f; g.splits = splits; g.split_stride = per;
         g.stamp = stamps_of(p) + kStampBwdDw;
-        if (with_dx) FL_TRY(launch_gemm_tn_and_nt(g, dx_product(p, long(p->bw.T) - 1, 0), s));
+        if (with_dx) FL_TRY(launch_gemm_tn_and_nt(g, dx_product(p, long(p->bw.T) - 1, 0), s, &p->bw.shared));
         else FL_TRY(launch_gemm_tn(g, s));
         out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), 0, d.I, invS, accumulate, dW_ih);
         out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), n_ih, d.H, invS, accumulate, dW_hh);

@@ -32,8 +32,8 @@ hipError_t launch_gemm_nt(const GemmNT& g, hipStream_t stream);
 hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream);
 
 // A TN product (fp32 partials) and an NT product that do not depend on each other: the same results as the two launches, in one
-// where both are small.
-hipError_t launch_gemm_tn_and_nt(const GemmNT& tn, const GemmNT& nt, hipStream_t stream);
+// where both are small (`shared`).
+hipError_t launch_gemm_tn_and_nt(const GemmNT& tn, const GemmNT& nt, hipStream_t stream, bool* shared);
 
 // Number of K slices the launchers really produce when `wanted` are asked for (every slice gets a
 // whole number of 64-wide K slabs). Size split-K partial buffers with this.

@@ -751,7 +751,8 @@ hipError_t launch_gemm_tn(const GemmNT& g, hipStream_t stream) {
 // instances for more than 512 tiles of 64 x 64 keep five there, which they would lose).  A 256 x 256 tile's kernel has the chip to
 // itself.  A training pass, two launches -> one: 64 steps of 8 rows x 256 units 240 -> 234 us, 200 of 70 x 257 units 682 -> 667, 256 of
 // 48 x 1536 units (342 + 121 us of products, both with a last round that is half empty) 2148 -> 2060.
-hipError_t launch_gemm_tn_and_nt(const GemmNT& tn, const GemmNT& nt, hipStream_t stream) {
+hipError_t launch_gemm_tn_and_nt(const GemmNT& tn, const GemmNT& nt, hipStream_t stream, bool* shared) {
+    *shared = false;
     if (tn.M > 0 && tn.N > 0 && tn.K > 0 && nt.M > 0 && nt.N > 0 && nt.K > 0 && tn.C32 && nt.splits <= 1) {
         hipError_t e = check_tn(tn);
         if (e == hipSuccess) e = check_nt(nt);
@@ -759,7 +760,8 @@ hipError_t launch_gemm_tn_and_nt(const GemmNT& tn, const GemmNT& nt, hipStream_t
         const int splits = tn.splits < 1 ? 1 : tn.splits, nslab = (tn.K + BK - 1) / BK;
         const int tn_tile = gemm_tn_tile_size(tn.M, tn.B2 ? tn.N1 : tn.N, tn.B2 ? tn.N - tn.N1 : 0, tn.K, splits);
         const int nt_tile = gemm_nt_tile_size(nt.M, nt.N, nt.K);
-        if (gemm_pair_possible(tn, tn_tile, splits, nt, nt_tile))
+        *shared = gemm_pair_possible(tn, tn_tile, splits, nt, nt_tile);
+        if (*shared)
             return launch_gemm_pair_tile(tn, tn_tile, splits, (nslab + splits - 1) / splits, nt, nt_tile, stream);
     }
     hipError_t e = launch_gemm_nt(nt, stream);

@@ -76,7 +76,10 @@ int flstm_core_set_option(flstm_core_plan* plan, const char* name, long value);
  * per workgroup of the recurrence kernels), "waves_fwd" (wavefronts per workgroup the forward recurrence runs with: 1, 2,
  * 4 or 8), "row_tiles_fwd", "row_tiles_bwd" (16-row tiles per row block that the
  * recurrences run with; "row_tiles": the forward one), "hidden_padded",
- * "input_padded", "outputs_behind" (the last forward pass wrote the caller's outputs by a launch of its own behind the
+ * "input_padded", "whole_fwd" (the last forward pass was one launch, but for what had to be prepared in front of it), "projection_fwd"
+ * (where it formed the x-projection: 0 by a launch in front of the recurrence, 1 beside it by the workgroups of the same launch that
+ * have no share in it, 2 inside it), "products_shared" (the last backward pass formed dX and the weight gradients in one launch),
+ * "outputs_behind" (the last forward pass wrote the caller's outputs by a launch of its own behind the
  * recurrence, because one of them lay in an input or the pass came in ranges of steps; else 0), "rows_behind" (the
  * same, and y was among them), "device_bytes" (device memory the plan holds), "static_scratch_bytes" (size of the fixed scratch
  * array of flstm_core_forward_static), "num_cus" and "clock_khz" (compute units and

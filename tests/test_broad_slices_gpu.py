@@ -13,13 +13,20 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(5, 49, 1025), (6, 112, 1056), (4, 100, 1120), (7, 81, 1280), (3, 97, 1281), (6, 33, 1400), (5, 80, 1536), (4, 81, 1536), (3, 161, 1536)]
 
 
+NARROW_FORWARD = [(97, 1281), (81, 1536), (161, 1536), (165, 1280)]   # slices of 16 forward: as many turns a step with 32-row blocks
+
+
 @pytest.mark.parametrize("T,B,H", SHAPES)
 @pytest.mark.parametrize("stepwise", [False, True])
 def test_slices_of_32_units_against_the_oracle(T, B, H, stepwise):
     p = make_problem(T, B, 24, H, seed=B * 10000 + H)
     ref, _ = oracle_reference(p)
-    got, info = run_core(p, stepwise=stepwise)
-    assert info["fallbacks"] == 0
+    from flashlstm_poc_amd import LstmCore
+    core = LstmCore(B, 24, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    got, info = run_core(p, stepwise=stepwise, core=core)
+    assert info["fallbacks"] == 0 and core.info("slice_bwd") == 32 and core.info("slice_fwd") == (16 if (B, H) in NARROW_FORWARD else 32)
+    core.close()
     check_against(ref, got, label=f"B={B} H={H} stepwise={stepwise}")
 
 
@@ -35,6 +42,7 @@ def test_slices_of_32_units_against_64_bits_and_32_row_blocks(T, B, H):
     core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
     got, info = run_core(p, core=core)
     assert info["fallbacks"] == 0 and core.info("slice_bwd") == 32 and core.info("row_tiles_bwd") == 1
+    assert core.info("slice_fwd") == (16 if (B, H) in NARROW_FORWARD else 32)
     for name in ("row_tiles_fwd", "row_tiles_bwd"):
         core.set_option(name, 2)
     blocks, info = run_core(p, core=core)

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 # dX, for both; tiles that keep a launch to themselves
 SHAPES = [(1, 1, 1, 1), (8, 9, 65, 257), (20, 100, 1000, 64), (33, 9, 456, 950), (200, 70, 65, 257), (260, 50, 300, 72), (128, 100, 512, 256),
           (300, 64, 128, 64), (64, 256, 1024, 256)]
+APART = [(300, 64, 128, 64), (64, 256, 1024, 256)]
 
 
 @pytest.mark.parametrize("T,B,I,H", SHAPES)
@@ -24,7 +25,7 @@ def test_shared_launch_gives_the_bits_of_two(T, B, I, H, half):
     core = LstmCore(B, I, H)
     core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
     want, info = run_core(p, core=core, half=half)
-    assert info["fallbacks"] == 0
+    assert info["fallbacks"] == 0 and core.info("products_shared") == (0 if (T, B, I, H) in APART else 1)
     dt = torch.float16 if half else torch.float32
     code = 1 if half else 0
     dev = {k: p[k].cuda().to(dt) for k in ("x", "h0", "c0", "dy", "d_hn", "d_cn")}
@@ -39,6 +40,7 @@ def test_shared_launch_gives_the_bits_of_two(T, B, I, H, half):
     assert lib.flstm_core_backward_end(core._h, dev["x"].data_ptr(), code,
                                        *(out[k].data_ptr() for k in ("dw_ih", "dw_hh", "db", "db_hh", "dh0", "dc0")), s) == 0
     torch.cuda.synchronize()
+    assert core.info("products_shared") == 0
     for k, v in dict(out, dx=dx).items():
         if k != "db_hh":
             assert np.array_equal(to_np(v), want[k]), k

@@ -7,7 +7,8 @@ pytestmark = pytest.mark.gpu
 # one, two and four groups inside XCDs (what is idle: six whole XCDs, four, ...), groups across XCDs, slices of 16 units (two of them in
 # a column of tiles), two row blocks; rows that end inside a tile, one tile of rows, rows of 64 features and many
 SHAPES = [(600, 32, 1024, 1024), (300, 64, 512, 1024), (255, 33, 448, 640), (400, 7, 1024, 992), (130, 100, 2048, 640),
-          (200, 16, 2048, 2048), (150, 48, 512, 1536), (333, 9, 256, 1400)]
+          (200, 16, 2048, 2048), (150, 48, 512, 1536), (333, 9, 256, 1400), (260, 100, 512, 640)]
+IN_FRONT = [(130, 100, 2048, 640)]   # 116 workgroups would take longer over 2048 features than the recurrence and the product apart
 
 
 @pytest.mark.parametrize("T,B,I,H", SHAPES)
@@ -30,10 +31,12 @@ def test_projection_beside_the_recurrence_gives_the_bits_of_one_in_front(T, B, I
 
     core.set_option("profile", 1)
     want = [passed(x) for x in xs]
+    assert core.info("projection_fwd") == 0
     core.set_option("profile", 0)
     for x, w in zip(xs + xs[:1], want + want[:1]):   # other rows every time: no tile of a pass before may be taken for this one's
         for k, (a, b) in enumerate(zip(passed(x), w)):
             assert torch.equal(a, b), k
+        assert core.info("projection_fwd") == (0 if (T, B, I, H) in IN_FRONT else 1)
     short = xs[0][:T // 2].contiguous()
     core.set_option("profile", 1)
     y, _, _ = core.forward(short, h0, c0)
@@ -51,7 +54,7 @@ def test_recurrence_that_waits_in_vain_for_its_projection_is_repeated():
     core.pack(*(torch.randn(*s, device="cuda") * 0.03 for s in ((4096, 512), (4096, 1024), (4096,), (4096,))))
     x = torch.randn(128, 64, 512, device="cuda").half()
     want = core.forward(x)
-    assert core.info("fallbacks") == 0
+    assert core.info("projection_fwd") == 1 and core.info("fallbacks") == 0
     core.set_option("spin_limit", 0)
     assert all(torch.equal(a, b) for a, b in zip(core.forward(x), want))
     assert core.info("fallbacks") >= 1 and core.info("persistent_fwd") == 0

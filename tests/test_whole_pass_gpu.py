@@ -23,6 +23,7 @@ def cached(core, which, rows, dtype):
 # features and of more, every length of the contraction, odd widths; T = 70 crosses the rule for few units, 33 the one for 256 features
 SHAPES = [(1, 1, 128, 256), (2, 16, 64, 64), (3, 17, 65, 33), (4, 3, 1, 1), (5, 40, 256, 512), (33, 20, 200, 130), (32, 20, 200, 130),
           (70, 5, 128, 96), (64, 5, 128, 96), (9, 100, 300, 512), (12, 512, 20, 256), (7, 128, 64, 257), (6, 64, 129, 384), (37, 33, 100, 384)]
+IN_FRONT = [(33, 20, 200, 130), (70, 5, 128, 96), (9, 100, 300, 512)]   # whose projection has a launch of its own
 
 
 @pytest.mark.parametrize("T,B,I,H", SHAPES)
@@ -50,10 +51,12 @@ def test_whole_pass_gives_the_bits_of_separate_launches(T, B, I, H, dtype, state
 
     core.set_option("profile", 1)
     want = passed(True)
+    assert core.info("whole_fwd") == 0
     core.set_option("profile", 0)
     for save, want_y in ((True, True), (False, True), (True, False), (True, True), (False, True)):   # (each leaves the ring to the next)
         for k, (a, b) in enumerate(zip(passed(save, want_y), want)):
             assert a is None or torch.equal(a, b), (save, k)
+        assert core.info("whole_fwd") == 1 and core.info("projection_fwd") == (0 if (T, B, I, H) in IN_FRONT else 2)
     assert core.info("fallbacks") == 0
     core.close()
 
@@ -69,5 +72,28 @@ def test_whole_passes_of_a_plan_whose_launch_gave_up():
     core.set_option("inject_stall", 1)
     for _ in range(12):   # repeated step-wise, demoted for eight passes, whole again
         assert all(torch.equal(a, b) for a, b in zip(core.forward(x), want))
+    assert core.info("whole_fwd") == 1
     assert core.info("demotions_fwd") == 1 and core.info("hold_fwd") == 0 and core.info("persistent_fwd") == 1
+    core.close()
+
+
+# enough steps for some wave to ask too early: of 11 steps of the first, half the passes went through without a reload
+@pytest.mark.parametrize("T,B,I,H", [(300, 16, 64, 128), (200, 40, 300, 512), (300, 100, 20, 256)])
+def test_whole_pass_that_gives_up_inside(T, B, I, H):
+    """A bound of no reload at all: a wave finds the fragments unwritten and leaves, with the ring half written and the status in the
+    host's memory.  The pass is repeated step-wise; with the bound taken back, whole passes over other rows follow, and their bits."""
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    core = LstmCore(B, I, H)
+    core.pack(*(torch.randn(*s, device="cuda") * 0.1 for s in ((4 * H, I), (4 * H, H), (4 * H,), (4 * H,))))
+    xs = [torch.randn(T, B, I, device="cuda").half() for _ in range(12)]
+    want = [core.forward(x) for x in xs]
+    assert core.info("whole_fwd") == 1 and core.info("fallbacks") == 0
+    core.set_option("spin_limit", 0)
+    assert all(torch.equal(a, b) for a, b in zip(core.forward(xs[0]), want[0]))
+    assert core.info("fallbacks") == 1 and core.info("persistent_fwd") == 0 and core.info("whole_fwd") == 0
+    core.set_option("spin_limit", 1 << 30)
+    for x, w in zip(xs, want):   # seven more of them step-wise
+        assert all(torch.equal(a, b) for a, b in zip(core.forward(x), w))
+    assert core.info("whole_fwd") == 1 and core.info("fallbacks") == 1
     core.close()
