@@ -284,10 +284,13 @@ def bench_stack(args, device):
     torch.cuda.synchronize()
     ms = e0.elapsed_time(e1) / args.steps
     flops = sum(24.0 * T * B * H * ((I if l == 0 else H) + H) for l in range(L))
-    phases = {ph: sum(layer.last_ms(ph) for layer in stack.layers) for ph in ("fwd_proj", "fwd_rec", "bwd_rec", "bwd_dx", "bwd_dw")}
+    # (a time below zero: that layer's projection has no launch of its own, its work is the recurrence's)
+    phases = {ph: sum(max(layer.last_ms(ph), 0.0) for layer in stack.layers) for ph in ("fwd_proj", "fwd_rec", "bwd_rec", "bwd_dx", "bwd_dw")}
     dom = max(phases, key=phases.get)
-    dom_flops = {"fwd_proj": sum(2.0 * T * B * 4 * H * (I if l == 0 else H) for l in range(L)),
-                 "fwd_rec": L * 2.0 * T * B * 4 * H * H, "bwd_rec": L * 2.0 * T * B * 4 * H * H,
+    projected = [2.0 * T * B * 4 * H * (I if l == 0 else H) for l in range(L)]
+    with_rec = sum(f for f, layer in zip(projected, stack.layers) if layer.info("projection_fwd") != 0)
+    dom_flops = {"fwd_proj": sum(projected) - with_rec,
+                 "fwd_rec": L * 2.0 * T * B * 4 * H * H + with_rec, "bwd_rec": L * 2.0 * T * B * 4 * H * H,
                  "bwd_dx": sum(2.0 * T * B * 4 * H * (I if l == 0 else H) for l in range(1, L)),
                  "bwd_dw": sum(2.0 * T * B * 4 * H * ((I if l == 0 else H) + H) for l in range(L))}[dom]
     tf = dom_flops / (phases[dom] * 1e-3) / 1e12
@@ -402,9 +405,16 @@ def bench_single(args, device):
     wall_ms = (time.perf_counter() - t0) * 1e3 / args.steps
     ms = e0.elapsed_time(e1) / args.steps
     phase_ms = {k: v / args.steps for k, v in acc.items()}
+    # Products without a launch of their own are part of the one that formed them (a phase then has no time, or no telling one).
+    projection, whole, shared = core.info("projection_fwd"), core.info("whole_fwd") == 1, backward and core.info("products_shared") == 1
+    if projection != 0:
+        del phase_ms["fwd_proj"]
+    if shared:
+        phase_ms["bwd_dw"] += phase_ms.pop("bwd_dx")
     # Engine clock inside the recurrence kernels, from two untimed passes with the kernels' own counters on: workgroup 0
     # reads the shader clock counter and the constant 100 MHz counter at its first and last step.  (The part lowers its
-    # clock under the GEMMs and raises it again only slowly, so the recurrences that follow them run below 2.4 GHz.)
+    # clock under the GEMMs and raises it again only slowly, so the recurrences that follow them run below 2.4 GHz.  These two passes
+    # have the projection in front of the recurrence, wherever the timed ones form it.)
     engine_mhz = {}
     if not args.no_engine_clock:
         core.set_option("profile", 1)
@@ -423,12 +433,19 @@ def bench_single(args, device):
     kflops = {"fwd_proj": 2.0 * T * B * 4 * H * I, "fwd_rec": 2.0 * T * B * 4 * H * H,
               "bwd_rec": 2.0 * T * B * 4 * H * H, "bwd_dx": 2.0 * T * B * 4 * H * I,
               "bwd_dw": 2.0 * T * B * 4 * H * (I + H)}
-    kname = {"fwd_proj": "gemm_nt_stream (X*W_ih^T + bias)", "fwd_rec": "rec_fwd_kernel (persistent recurrence)",
+    if projection != 0:
+        kflops["fwd_rec"] += kflops["fwd_proj"]
+    if shared:
+        kflops["bwd_dw"] += kflops["bwd_dx"]
+    rec_fwd = "a whole pass" if whole else "persistent recurrence"
+    rec_kernel = "rec_fwd_whole_kernel" if whole else "rec_fwd_il_kernel" if core.info("waves_fwd") == 8 else "rec_fwd_kernel"
+    kname = {"fwd_proj": "gemm_nt_stream (X*W_ih^T + bias)",
+             "fwd_rec": f"{rec_kernel} ({rec_fwd}{', X*W_ih^T + bias with it' if projection else ''})",
              "bwd_rec": ("rec_bwd2d_kernel (persistent BPTT, product split over columns and contraction)"
                          if core.info("bwd_two_d") == 1 else "rec_bwd_kernel (persistent BPTT)"), "bwd_dx": "gemm_nt_stream (dG*W_ih)",
-             "bwd_dw": "gemm_tn_stream split-K x2 (dG^T*X, dG^T*H) + reduce_dw"}
+             "bwd_dw": ("gemm_pair_tile (dG^T*X, dG^T*H, dG*W_ih)" if shared else "gemm_tn_stream split-K x2 (dG^T*X, dG^T*H)") + " + reduce_dw"}
     kernels = []
-    for k in phases:
+    for k in phase_ms:
         tf = kflops[k] / (phase_ms[k] * 1e-3) / 1e12 if phase_ms[k] > 0 else 0.0
         kernels.append({"phase": k, "kernel": kname[k], "ms": round(phase_ms[k], 4), "tflops": round(tf, 1),
                         "frac_of_peak": round(tf / PEAK_FP16_TFLOPS, 4)})

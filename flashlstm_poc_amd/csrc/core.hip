@@ -138,6 +138,7 @@ struct flstm_core_plan {
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
              half_t* y_direct = nullptr;   // the recurrence writes the caller's y itself
              bool whole = false;           // one launch (forward_whole)
+             int begin = kStampFwdBegin;   // the stamp that begins the pass
              int projection = 0;           // where the x-projection is formed: 0 in front of the recurrence, 1 beside it, 2 inside its launch
              bool behind = false;          // the caller's final states are written by a launch of their own behind the recurrence ...
              bool rows_behind = false; } fw;   // ... and y with them
@@ -510,6 +511,7 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     p->fw.T = T; p->fw.x = x; p->fw.x_dtype = x_dtype; p->fw.open = true; p->fw.whole = false;
+    p->fw.begin = kStampFwdBegin;
     p->beside_f.count = 0;
     if (!x_in_place(p, x_dtype)) FL_TRY(p->X16.reserve(TB * d.Ip * sizeof(half_t)));
     FL_TRY(p->G.reserve(TB * 4 * d.Hp * sizeof(half_t)));
@@ -531,6 +533,7 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     if (whole_x && !x_in_place(p, x_dtype))
         prep.to_half(x, x_dtype == FLSTM_F32, TB, d.I, size_t(d.I), 1.f, p->X16.as<half_t>(), TB, size_t(d.Ip));
     prep.stamps = stamps_of(p);
+    prep.begin = kStampFwdBegin;
     prep.stamp = kStampFwdStart;
     FL_TRY(run_ops(prep, s));
     p->seat_sets_left = kSeatSets;
@@ -575,7 +578,8 @@ bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
 }
 
 // x rows of steps [t0, t0+n) -> fp16 operand -> x-projection (+ bias) in G, or left to the recurrence's launch
-int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, bool may_leave_it, hipStream_t s) {
+// (`stamp`: where the product leaves its start, if anywhere)
+int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, bool may_leave_it, hipStream_t s, long long* stamp = nullptr) {
     const Dims& d = p->d;
     GemmNT g{};
     int rc = forward_operand(p, t0, n, converted, s, &g.A, &g.lda);
@@ -588,6 +592,7 @@ int forward_project(flstm_core_plan* p, size_t t0, size_t n, bool converted, boo
     g.C16 = p->G.as<half_t>() + t0 * d.B * 4 * d.Hp; g.C32 = nullptr; g.ldc = size_t(4) * d.Hp;
     g.alpha = 1.f; g.splits = 1; g.split_stride = 0;
     g.bias = p->bias_p.as<float>();   // b_ih + b_hh, packed gate order: the recurrence reads x-projection + bias
+    g.stamp = stamp;
     p->project = ProjectBeside{};
     p->fw.projection = 0;
     if (may_leave_it && projects_beside(p, n, g.A)) {
@@ -725,11 +730,19 @@ int forward_whole(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
         a.Y = p->Y.as<half_t>(); a.C = p->C.as<float>();
     }
     a.G = p->G.as<half_t>();
-    FL_TRY(run_ops(prep, s));
+    a.status = p->fw.behind ? p->status.as<int>() : &p->status_host->status;   // (behind: published by the outputs' launch)
+    a.stamps = p->fw.behind ? stamps_of(p) : p->status_host->stamps;
+    p->fw.begin = prep.count > 0 ? kStampFwdBegin : projects ? kStampFwdRec : kStampFwdStart;   // (of whichever launch comes first)
+    if (prep.count > 0) {
+        prep.stamps = a.stamps;
+        prep.begin = kStampFwdBegin;
+        prep.stamp = kStampFwdStart;
+        FL_TRY(run_ops(prep, s));
+    }
     p->fw.projection = 2;
     if (!projects) {
         a.x = nullptr;
-        const int rc = forward_project(p, 0, T, true, false, s);
+        const int rc = forward_project(p, 0, T, true, false, s, prep.count > 0 ? nullptr : a.stamps + kStampFwdStart);
         if (rc) return rc;
     }
     a.wfrag = p->wfrag[kFragFwdSplit].as<half8>();
@@ -743,8 +756,6 @@ int forward_whole(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     int rc = next_seats(p, &a.seats, s);
     if (rc) return rc;
     p->status_host->status = 0;   // (nothing of this plan is running: every pass is waited for)
-    a.status = p->fw.behind ? p->status.as<int>() : &p->status_host->status;   // (behind: published by the outputs' launch)
-    a.stamps = p->fw.behind ? stamps_of(p) : p->status_host->stamps;
     a.B = d.B; a.H = d.H; a.Hp = d.Hp; a.T = int(T);
     a.spin_limit = p->opt_spin_limit;
     a.spin_ticks = (long long)p->opt_spin_ms * p->wall_khz;
@@ -825,10 +836,9 @@ int forward_conclude(flstm_core_plan* p, hipStream_t s) {
     }
     pass_done(p, true);
     if (p->opt_profile) FL_TRY(hipMemcpy(p->prof_f, p->prof.p, sizeof(p->prof_f), hipMemcpyDeviceToHost));
-    const int first = p->fw.whole ? kStampFwdRec : kStampFwdStart;   // (a pass as one launch is all recurrence)
-    p->ms_fwd[0] = elapsed(p, first, kStampFwdRec);
+    p->ms_fwd[0] = p->fw.projection == 0 ? elapsed(p, kStampFwdStart, kStampFwdRec) : -1.f;
     p->ms_fwd[1] = elapsed(p, kStampFwdRec, kStampFwdRecEnd);
-    p->ms_fwd[2] = elapsed(p, first, kStampFwdRecEnd);
+    p->ms_fwd[2] = elapsed(p, p->fw.begin, kStampFwdEnd);
     p->fw.open = false;
     return 0;
 }
@@ -963,6 +973,7 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     if (whole_dy && p->bw.dYk != dY)
         prep.to_half(dY, dy_dtype == FLSTM_F32, TB, d.H, size_t(d.H), k.dy, p->dYp.as<half_t>(), TB, size_t(d.Hp));
     prep.stamps = stamps_of(p);
+    prep.begin = kStampBwdBegin;
     prep.stamp = kStampBwdStart;
     FL_TRY(run_ops(prep, s));
     p->seat_sets_left = kSeatSets;
@@ -1155,7 +1166,7 @@ int backward_conclude(flstm_core_plan* p, bool weight_gradients, hipStream_t s) 
     p->ms_bwd[0] = elapsed(p, kStampBwdStart, kStampBwdRecEnd);
     p->ms_bwd[1] = elapsed(p, kStampBwdRecEnd, dw_start);
     p->ms_bwd[2] = elapsed(p, dw_start, kStampBwdEnd);
-    p->ms_bwd[3] = elapsed(p, kStampBwdStart, kStampBwdEnd);
+    p->ms_bwd[3] = elapsed(p, kStampBwdBegin, kStampBwdEnd);
     return 0;
 }
 

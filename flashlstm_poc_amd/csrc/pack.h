@@ -68,7 +68,7 @@ struct LayoutOp {
 // Time stamps and status of a pass.  Device side: word 0 of `status` is the recurrence's status, `stamps` hold ticks of
 // the constant-rate clock.  A list with `publish` set copies both to pinned host memory, so that the wait that ends the
 // pass is also the one that makes them readable: no copy command and no second round trip.
-enum Stamp : int { kStampFwdStart, kStampFwdRec, kStampFwdRecEnd, kStampBwdStart, kStampBwdRecEnd, kStampBwdDw, kStampBwdEnd, kStampFwdEnd, kStampCount };
+enum Stamp : int { kStampFwdStart, kStampFwdRec, kStampFwdRecEnd, kStampBwdStart, kStampBwdRecEnd, kStampBwdDw, kStampBwdEnd, kStampFwdEnd, kStampFwdBegin, kStampBwdBegin, kStampCount };
 struct HostStatus {
     int status;
     float absmax;   // (absmax())
@@ -78,6 +78,7 @@ struct HostStatus {
 struct OpList {
     int count = 0;
     int stamp = -1;                   // which stamp block 0 writes when it is done (-1: none)
+    int begin = -1;                   // ... and which when it starts
     const int* status = nullptr;      // device status word (with `publish`)
     long long* stamps = nullptr;
     HostStatus* publish = nullptr;

@@ -223,6 +223,7 @@ __device__ __forceinline__ void op_reduce_dw(const LayoutOp& o, size_t first, si
 // traffic or launch latency: eight elements per thread in 16-byte accesses where the pitches allow (fp32 sequence of
 // 65536 x 1024 from fp16 rows: 2.1 TB/s with one element per thread and 64-bit index arithmetic).
 __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
+    if (blockIdx.x == 0 && threadIdx.x == 0 && list.begin >= 0) list.stamps[list.begin] = wall_clock64();
     int which = 0;
     while (which + 1 < list.count && blockIdx.x >= list.op[which + 1].first_block) ++which;
     if (list.count > 0 && !(list.only_if_ok && *list.status != 0)) {

@@ -195,9 +195,15 @@ int flstm_core_backward_end(flstm_core_plan* plan, const void* x, flstm_dtype x_
  *   which = 2: activated gates fp16 [T*B][4Hp], column 4 * unit + gate (gates i, f, g, o) */
 int flstm_core_cache_ptr(const flstm_core_plan* plan, int which, const void** ptr, size_t* ld);
 
-/* Average device time in milliseconds of the phases of the most recent forward / backward,
- * measured by time stamps the kernels leave: names "fwd_proj", "fwd_rec", "fwd_total",
- * "bwd_rec", "bwd_dx", "bwd_dw", "bwd_total".  Negative when not available. */
+/* Device time in milliseconds of the phases of the most recent forward / backward (one whole pass, not one fed in ranges of
+ * steps), measured by time stamps the kernels leave.  Negative when not available.
+ * "fwd_proj": the x-projection where a launch in front of the recurrence forms it (get_info "projection_fwd" is 0), else negative.
+ * "fwd_rec": the recurrence, with the projection where that is formed beside or inside it; where the pass is one launch
+ *   ("whole_fwd") with the outputs and final states too.
+ * "fwd_total": all launches of the pass, from the setup (converted rows, state rows, ring) to the outputs.
+ * "bwd_rec": the setup's end to the end of the recurrence.  "bwd_dx", "bwd_dw": from there to the start of the weight gradients'
+ *   product, and from that to the end of the pass; where dX shares that launch ("products_shared"), how its time falls to the two
+ *   says nothing, their sum does.  "bwd_total": all launches of the pass. */
 double flstm_core_last_ms(const flstm_core_plan* plan, const char* phase);
 
 /* Tuner (the counterpart of the reference's projection-chunk tuner, src/tune_projchunksz.cu:56-226, and of the
