@@ -7,6 +7,7 @@
 //            -> dW = dG^T * [X ; H_prev] as one split-K GEMM -> reductions into caller layout.
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -109,7 +110,7 @@ struct flstm_core_plan {
     // Tuned launch choices per sequence length (flstm_core_tune): 16- or 32-row blocks and persistent or step-wise
     // launches per direction, split-K count of the weight-gradient GEMM.  eff_* hold the entry in force for the
     // sequence length of the current pass (0 = no tuned value: the rules of thumb decide); explicit options win.
-    struct Tuned { size_t T; int mt_f, mt_b, step_f, step_b, dw_splits, two_d; float ms_f, ms_b, ms_dw; };   // two_d: -1 = not tuned, else the bwd_two_d option
+    struct Tuned { size_t T; int mt_f, mt_b, step_f, step_b, dw_splits, two_d; float ms_f, ms_b, ms_dw, pass_f, products; };   // two_d: -1 = not tuned, else the bwd_two_d option
     std::vector<Tuned> tuned;
     int opt_mt_f = 0, opt_mt_b = 0;
     int eff_mt_f = 0, eff_mt_b = 0, eff_step_f = 0, eff_step_b = 0, eff_dw = 0, eff_two_d = -1;
@@ -1558,9 +1559,9 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
     const size_t TB = T * size_t(d.B);
     // synthetic inputs: varied values (the matrix cores draw more power on them than on constants, and the GEMMs run
     // about a fifth slower: candidates are compared under the clock they will run at)
-    DevBuf x, dy, dwi, dwh;
+    DevBuf x, dy, dwi, dwh, y, dx;
     int rc = 0;
-    auto fail = [&](int code) { x.release(); dy.release(); dwi.release(); dwh.release(); return code; };
+    auto fail = [&](int code) { x.release(); dy.release(); dwi.release(); dwh.release(); y.release(); dx.release(); return code; };
     if (x.reserve(TB * d.I * sizeof(half_t)) != hipSuccess || dy.reserve(TB * d.H * sizeof(half_t)) != hipSuccess ||
         dwi.reserve(size_t(4) * d.H * d.I * sizeof(float)) != hipSuccess ||
         dwh.reserve(size_t(4) * d.H * d.H * sizeof(float)) != hipSuccess)
@@ -1568,6 +1569,12 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
     if (fill_noise(x.as<half_t>(), TB * d.I, 0x1234567u, 1.7f, s) != hipSuccess ||
         fill_noise(dy.as<half_t>(), TB * d.H, 0x89ABCDEu, 1.7f, s) != hipSuccess)
         return fail(int(hipErrorUnknown));
+    // y and dx as passes in use write them (without memory for them, passes that leave them out are compared)
+    if (y.reserve(TB * d.H * sizeof(half_t)) != hipSuccess || dx.reserve(TB * d.I * sizeof(half_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        y.release();
+        dx.release();
+    }
     // the plan's explicit options and tuned state are set aside while candidates run
     const int keep_step = p->opt_stepwise, keep_mtf = p->opt_mt_f, keep_mtb = p->opt_mt_b, keep_dw = p->opt_dw_splits,
               keep_acc = p->opt_accumulate, keep_two_d = p->opt_two_d;
@@ -1586,20 +1593,29 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
         replan(p);
     };
     flstm_core_plan::Tuned best{};
-    best.T = T; best.ms_f = best.ms_b = best.ms_dw = -1.f; best.two_d = -1;
-    auto run = [&](float& f_ms, float& b_ms, float& dw_ms) -> int {
-        f_ms = b_ms = dw_ms = 1e30f;
+    best.T = T; best.ms_f = best.ms_b = best.ms_dw = best.pass_f = best.products = -1.f; best.two_d = -1;
+    // A forward candidate is judged by the whole call: whether its projection and outputs have launches of their own or are part
+    // of the recurrence's depends on the candidate, so the phases do not hold the same work.  A split count by all products, of
+    // which dX may share the launch.
+    struct Times { float pass_f, f, b, products, dw; } ms;
+    auto run = [&]() -> int {
+        ms = Times{1e30f, 1e30f, 1e30f, 1e30f, 1e30f};
+        auto least = [](float& to, float v) { if (v > 0 && v < to) to = v; };
         for (int r = 0; r <= repeats; ++r) {   // first pass is a warm-up
-            int e = flstm_core_forward(p, T, x.p, FLSTM_F16, nullptr, nullptr, FLSTM_F16, nullptr, FLSTM_F16, nullptr, nullptr,
+            const auto before = std::chrono::steady_clock::now();
+            int e = flstm_core_forward(p, T, x.p, FLSTM_F16, nullptr, nullptr, FLSTM_F16, y.p, FLSTM_F16, nullptr, nullptr,
                                        FLSTM_F16, 1, s);
             if (e) return e;
-            e = flstm_core_backward(p, T, x.p, FLSTM_F16, dy.p, FLSTM_F16, nullptr, nullptr, FLSTM_F16, 1.f, nullptr, FLSTM_F16,
+            const float whole = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - before).count();
+            e = flstm_core_backward(p, T, x.p, FLSTM_F16, dy.p, FLSTM_F16, nullptr, nullptr, FLSTM_F16, 1.f, dx.p, FLSTM_F16,
                                     dwi.as<float>(), dwh.as<float>(), nullptr, nullptr, nullptr, nullptr, s);
             if (e) return e;
             if (r == 0) continue;
-            if (p->ms_fwd[1] > 0 && p->ms_fwd[1] < f_ms) f_ms = p->ms_fwd[1];
-            if (p->ms_bwd[0] > 0 && p->ms_bwd[0] < b_ms) b_ms = p->ms_bwd[0];
-            if (p->ms_bwd[2] > 0 && p->ms_bwd[2] < dw_ms) dw_ms = p->ms_bwd[2];
+            least(ms.pass_f, whole);
+            least(ms.f, p->ms_fwd[1]);
+            least(ms.b, p->ms_bwd[0]);
+            least(ms.products, p->ms_bwd[1] + p->ms_bwd[2]);
+            least(ms.dw, p->ms_bwd[2]);
         }
         return 0;
     };
@@ -1611,11 +1627,10 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
             replan(p);
             const bool f_is = (p->Lf.mt == mt), b_is = (p->Lb.mt == mt);   // 16-row blocks may not fit
             if (!f_is && !b_is) continue;
-            float f_ms, b_ms, dw_ms;
-            rc = run(f_ms, b_ms, dw_ms);
+            rc = run();
             if (rc) { restore(); return fail(rc); }
-            if (f_is && (best.ms_f < 0 || f_ms < best.ms_f)) { best.ms_f = f_ms; best.mt_f = mt; best.step_f = step; }
-            if (b_is && (best.ms_b < 0 || b_ms < best.ms_b)) { best.ms_b = b_ms; best.mt_b = mt; best.step_b = step; }
+            if (f_is && (best.pass_f < 0 || ms.pass_f < best.pass_f)) { best.pass_f = ms.pass_f; best.ms_f = ms.f; best.mt_f = mt; best.step_f = step; }
+            if (b_is && (best.ms_b < 0 || ms.b < best.ms_b)) { best.ms_b = ms.b; best.mt_b = mt; best.step_b = step; }
         }
     }
     // 1b) the layout of the backward recurrence where the two-way split can run (2048 and 1024 hidden units): off /
@@ -1629,10 +1644,9 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
             replan(p);
             if (!p->Lb.persistent) continue;
             if (td == 2 && !p->Lb.two_d) continue;   // (nothing new: the split does not fit this batch)
-            float f_ms, b_ms, dw_ms;
-            rc = run(f_ms, b_ms, dw_ms);
+            rc = run();
             if (rc) { restore(); return fail(rc); }
-            if (best_td_ms < 0 || b_ms < best_td_ms) { best_td_ms = b_ms; best.two_d = td; }
+            if (best_td_ms < 0 || ms.b < best_td_ms) { best_td_ms = ms.b; best.two_d = td; }
         }
         // (the entry keeps the better of: the best row-block height under the plan's own setting, the best setting)
         if (best_td_ms >= 0 && best_td_ms < best.ms_b) { best.ms_b = best_td_ms; best.mt_b = 0; best.step_b = 0; }
@@ -1651,10 +1665,9 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
         if (eff == last_eff) continue;
         last_eff = eff;
         p->opt_dw_splits = cand;
-        float f_ms, b_ms, dw_ms;
-        rc = run(f_ms, b_ms, dw_ms);
+        rc = run();
         if (rc) { restore(); return fail(rc); }
-        if (best.ms_dw < 0 || dw_ms < best.ms_dw) { best.ms_dw = dw_ms; best.dw_splits = cand; }
+        if (best.products < 0 || ms.products < best.products) { best.products = ms.products; best.ms_dw = ms.dw; best.dw_splits = cand; }
     }
     restore();
     for (auto it = p->tuned.begin(); it != p->tuned.end();)
@@ -1672,7 +1685,7 @@ extern "C" int flstm_core_set_tuned(flstm_core_plan* p, size_t T, int row_tiles_
         return FLSTM_E_INVALID;
     flstm_core_plan::Tuned t{};
     t.T = T; t.mt_f = row_tiles_fwd; t.mt_b = row_tiles_bwd; t.step_f = stepwise_fwd != 0; t.step_b = stepwise_bwd != 0;
-    t.dw_splits = dw_splits; t.two_d = bwd_two_d; t.ms_f = t.ms_b = t.ms_dw = -1.f;
+    t.dw_splits = dw_splits; t.two_d = bwd_two_d; t.ms_f = t.ms_b = t.ms_dw = t.pass_f = t.products = -1.f;
     for (auto it = p->tuned.begin(); it != p->tuned.end();)
         it = (it->T == T) ? p->tuned.erase(it) : it + 1;
     p->tuned.push_back(t);
@@ -1698,6 +1711,8 @@ extern "C" double flstm_core_tuned_ms(const flstm_core_plan* p, size_t T, const 
     if (!p || !phase) return -1.0;
     for (const auto& t : p->tuned)
         if (t.T == T) {
+            if (!strcmp(phase, "fwd_pass")) return t.pass_f;
+            if (!strcmp(phase, "bwd_products")) return t.products;
             if (!strcmp(phase, "fwd_rec")) return t.ms_f;
             if (!strcmp(phase, "bwd_rec")) return t.ms_b;
             if (!strcmp(phase, "bwd_dw")) return t.ms_dw;

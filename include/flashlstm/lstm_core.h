@@ -217,8 +217,10 @@ double flstm_core_last_ms(const flstm_core_plan* plan, const char* phase);
  * one (explicit options "stepwise", "row_tiles_fwd", "row_tiles_bwd", "dw_splits" still win; option "clear_tuned"
  * forgets everything).  Read back with flstm_core_get_info: "tuned_entries", and for the entry in force for the
  * last pass "tuned_T", "tuned_row_tiles_fwd", "tuned_row_tiles_bwd", "tuned_stepwise_fwd", "tuned_stepwise_bwd",
- * "tuned_dw_splits" (0 = rule of thumb), "tuned_bwd_two_d" (-1 = not tuned); flstm_core_tuned_ms gives the best time
- * found per phase ("fwd_rec", "bwd_rec", "bwd_dw").  The plan's forward cache is invalidated.  Allocates temporary
+ * "tuned_dw_splits" (0 = rule of thumb), "tuned_bwd_two_d" (-1 = not tuned); flstm_core_tuned_ms gives the times the
+ * choices were made by: "fwd_pass" (a whole forward call, since what is part of the recurrence's launch depends on the choice),
+ * "bwd_rec", "bwd_products" (dX and the weight gradients, which may share a launch), and of the same passes "fwd_rec" and
+ * "bwd_dw" as flstm_core_last_ms has them.  The plan's forward cache is invalidated.  Allocates temporary
  * device buffers. */
 int flstm_core_tune(flstm_core_plan* plan, size_t seq_len, int repeats, int try_stepwise, void* stream);
 double flstm_core_tuned_ms(const flstm_core_plan* plan, size_t seq_len, const char* phase);

@@ -125,3 +125,36 @@ def test_tuner_tries_the_layouts_of_the_backward_recurrence_at_2048_units():
     core.forward(p["x"], p["h0"], p["c0"]); core.backward(p["x"], p["dy"])
     assert core.info("bwd_two_d") == 0
     core.close()
+
+
+@pytest.mark.parametrize("T,B,I,H", [(64, 32, 2176, 2048), (64, 128, 1024, 1024), (64, 40, 96, 256)])
+def test_tuner_judges_the_forward_choices_by_whole_calls(T, B, I, H):
+    """What "fwd_rec" holds depends on the candidate (16-row blocks seat every CU here and have the projection in front; 32-row blocks leave
+    idle ones that form it beside the recurrence; whole passes hold their outputs too), so the choice is made by calls."""
+    import time
+    import torch
+    from flashlstm_poc_amd import LstmCore, sweep
+    p = sweep.make_problem(T, B, I, H, seed=9)
+    core = LstmCore(B, I, H)
+    core.pack(p["w_ih"], p["w_hh"], p["b_ih"], p["b_hh"])
+    t = core.tune(T, repeats=6)
+    ms = lambda phase: core.lib.flstm_core_tuned_ms(core._h, T, phase.encode())
+    assert ms("fwd_pass") > ms("fwd_rec") > 0 and ms("bwd_products") >= ms("bwd_dw") > 0
+    x = p["x"].half()
+
+    def least():
+        core.forward(x)
+        times = []
+        for _ in range(12):
+            torch.cuda.synchronize()
+            start = time.perf_counter()
+            core.forward(x)
+            times.append((time.perf_counter() - start) * 1e3)
+        return min(times)
+
+    # (wide bounds: calls of 0.1 to 0.4 ms, timed from Python, on a machine that others use as well)
+    assert 0.5 < least() / ms("fwd_pass") < 2.0
+    core.set_option("row_tiles_fwd", 3 - t["row_tiles_fwd"])
+    if core.info("row_tiles_fwd") != t["row_tiles_fwd"]:
+        assert ms("fwd_pass") < 1.5 * least()
+    core.close()
