@@ -639,9 +639,11 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     int rc = next_seats(p, &a.seats, s);
     if (rc) return rc;
     take_beside(p->beside_f, a);
-    a.project = p->project;
-    a.project.ticket = a.seats + 16;
-    p->project = ProjectBeside{};
+    if (p->project.M != 0) {   // (else all of it stays zero: an assigned struct brings padding of its own into a graph's key)
+        a.project = p->project;
+        a.project.ticket = a.seats + 16;
+        p->project = ProjectBeside{};
+    }
     a.B = d.B; a.Hp = d.Hp; a.T = int(p->fw.T); a.t0 = int(t0); a.t1 = int(t0 + n);
     a.spin_limit = p->opt_spin_limit;
     a.spin_ticks = (long long)p->opt_spin_ms * p->wall_khz;

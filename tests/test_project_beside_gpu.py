@@ -59,3 +59,24 @@ def test_recurrence_that_waits_in_vain_for_its_projection_is_repeated():
     assert all(torch.equal(a, b) for a, b in zip(core.forward(x), want))
     assert core.info("fallbacks") >= 1 and core.info("persistent_fwd") == 0
     core.close()
+
+
+def test_step_wise_passes_between_projections_beside_replay_one_graph():
+    """The arguments of a step-wise launch are the key of its captured graph: what a pass with its projection beside left behind in them
+    must not show."""
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    core = LstmCore(64, 512, 1024)
+    core.pack(*(torch.randn(*s, device="cuda") * 0.03 for s in ((4096, 512), (4096, 1024), (4096,), (4096,))))
+    x = torch.randn(128, 64, 512, device="cuda").half()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):   # (the legacy default stream cannot be captured)
+        want = core.forward(x)
+        for again in range(5):
+            core.set_option("stepwise", 1)
+            assert all(torch.equal(a, b) for a, b in zip(core.forward(x), want))
+            assert core.info("projection_fwd") == 0 and core.info("graph_captures") == 1 and core.info("graph_replays") == again
+            core.set_option("stepwise", 0)
+            assert all(torch.equal(a, b) for a, b in zip(core.forward(x), want))
+            assert core.info("projection_fwd") == 1
+    core.close()
