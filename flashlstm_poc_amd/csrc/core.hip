@@ -568,6 +568,10 @@ int forward_operand(flstm_core_plan* p, size_t t0, size_t n, bool converted, hip
 // a gap.  Measured, us a forward pass, in front / beside: 512 steps of 64 rows, 1024 features and units 1275 / 990, of 16 rows of 2048
 // 1443 / 1208, of 64 rows of 640 units and 2048 features 1316 / 956; 128 steps of the first 347 / 292, 32 steps 130 / 116; where the
 // line is drawn: 32 steps of 32 rows of 1536 units, 1024 features (64 workgroups to form it) 128 / 138, 512 steps of them 1439 / 1280.
+// A step is taken for 1.9 or 2.4 us however many row blocks a workgroup has in it: with two turns a step (100 rows of 1400 units) it
+// lasts twice that, more of the product fits beside it than is reckoned with, and the rule keeps to the launch in front.  Fewer than
+// 16 workgroups are not tried: where 241 and more have seats a step takes 8 tiles or more (17 rows of 2048 units, 113 of 1024), which
+// so few keep up with for a hundred features at most, and that product is short in front, too.
 bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
     const Dims& d = p->d;
     const int helpers = rec_projecting_workgroups(p->Lf);

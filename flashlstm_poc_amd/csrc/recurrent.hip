@@ -1696,7 +1696,8 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
 //    last, (T - 1) % 4, provided the last step stores nothing; the next pass starts with that slot as its own slot 0
 //    (RecWholeArgs::base), which nobody reads, because h0 comes from the caller's tensor.
 //  * Initial states are read, and outputs and final states written, in the caller's layout; the status word and the stamps go
-//    straight to pinned memory.
+//    straight to pinned memory.  (Outputs that lie in inputs are not: no wave knows whether the others have read what it would
+//    write over -- a single step has no exchange.  The launch then has none, and one behind it copies the caches' rows.)
 // SAVE: the gate, cell and state rows that the backward pass reads are written; a pass without gradients does without them.
 // The cache stores, the output row and the projection stand between the store of h_t and the request for the next step's
 // fragments: requested right behind the store, they come back unwritten and the second request notices them a trip later (256
@@ -2860,8 +2861,8 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
                 }
             }
             clk.lap(3);
-            if constexpr (MT == 1 && GPR == 8) __syncthreads();
-            else if constexpr (MT == 1) { if (p.B - row0 < RB) __syncthreads(); }   // (as in the forward kernel)   // (waves without cells to update: as in the forward kernel)
+            if constexpr (MT == 1 && GPR == 8) __syncthreads();   // (waves without cells to update: as in the forward kernel)
+            else if constexpr (MT == 1) { if (p.B - row0 < RB) __syncthreads(); }
         }
     }
     if (p.stamp_end && hs == 0 && g == 0 && tid == 0) *p.stamp_end = wall_clock64();

@@ -66,6 +66,8 @@ int flstm_core_destroy(flstm_core_plan* plan);
  * "waves_fwd" (wavefronts per workgroup of the forward recurrence: 0, the default, by size; 4 or 8, which split the
  * contraction between them, also where the kernel for short contractions would run; 8 up to 1024 units, with 32-row
  * blocks.  The weights are packed for it: a change between 4 and 8 un-packs them; FLASHLSTM_WAVES_FWD sets the default),
+ * "profile" (1: workgroup 0 of the recurrences counts cycles by phase, flstm_core_last_ms "fwd_clk0" .. "bwd_clk7".  Such forward
+ * passes are made of separate launches, with the projection in front of the recurrence: "whole_fwd" and "projection_fwd" are 0),
  * "inject_stall" (test hook: the next N passes that use a persistent kernel are treated as if that launch had
  * given up, which exercises the step-wise repeat and the demotion rule without making any kernel wait). */
 int flstm_core_set_option(flstm_core_plan* plan, const char* name, long value);
@@ -108,9 +110,9 @@ int flstm_core_forward(flstm_core_plan* plan, size_t seq_len,
 /* flstm_core_forward for callers that cannot allocate device memory (tight serving loops, harnesses that forbid
  * hipMalloc, the host code around a HIP graph).  It has no counterpart in the reference.  Same arguments, results
  * and kernels as flstm_core_forward with save_for_backward = 0, but everything the kernels need beyond the caller's
- * tensors and the plan's packed weights -- status word, converted x rows, x-projection / gate rows, state rows,
- * exchange ring -- lives in one fixed 64 MiB array in the library's device image instead of buffers grown by the
- * plan: the call allocates and frees nothing, also not when a persistent launch gives up and the pass is repeated
+ * tensors and what the plan has had since its weights were packed (those, the status block, the exchange ring of passes that are
+ * one launch) -- converted x rows, x-projection / gate rows, state rows, exchange ring -- lives in one fixed 64 MiB array in the
+ * library's device image instead of buffers grown by the plan: the call allocates and frees nothing, also not when a persistent launch gives up and the pass is repeated
  * with one launch per step (those are plain launches here, never a captured graph).  Like flstm_core_forward it is
  * SYNCHRONOUS -- it waits for its stream and reads the status of the pass on the host -- so it cannot itself be
  * recorded into a graph that is being captured.  A pass that needs more (about T*B*(14*Hp + 2*Ip) bytes; the limit
