@@ -223,7 +223,8 @@ __device__ __forceinline__ void op_reduce_dw(const LayoutOp& o, size_t first, si
 // traffic or launch latency: eight elements per thread in 16-byte accesses where the pitches allow (fp32 sequence of
 // 65536 x 1024 from fp16 rows: 2.1 TB/s with one element per thread and 64-bit index arithmetic).
 __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
-    if (blockIdx.x == 0 && threadIdx.x == 0 && list.begin >= 0) list.stamps[list.begin] = wall_clock64();
+    // (stored at the end: a store in front of the operations' loads keeps block 0 waiting for its way to memory, 1 us a pass)
+    const long long begun = blockIdx.x == 0 && list.begin >= 0 ? wall_clock64() : 0;
     int which = 0;
     while (which + 1 < list.count && blockIdx.x >= list.op[which + 1].first_block) ++which;
     if (list.count > 0 && !(list.only_if_ok && *list.status != 0)) {
@@ -277,10 +278,11 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && list.stamps) {
         const long long now = wall_clock64();
+        if (list.begin >= 0) list.stamps[list.begin] = begun;
         if (list.stamp >= 0) list.stamps[list.stamp] = now;
         if (list.publish) {   // (what earlier launches left: this launch writes neither the status nor the other stamps)
             __hip_atomic_store(&list.publish->status, *list.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            for (int i = 0; i < kStampCount; ++i)
+            for (int i = list.stamp == kStampFwdEnd ? kStampFwdBegin : kStampBwdBegin; i <= list.stamp; ++i)
                 __hip_atomic_store(&list.publish->stamps[i], i == list.stamp ? now : list.stamps[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }

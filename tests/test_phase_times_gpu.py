@@ -42,7 +42,8 @@ def test_forward_phases(T, B, I, H, dtype, whole, projection):
     else:
         assert phase["fwd_proj"] < 0
     assert phase["fwd_rec"] > 0
-    assert max(phase["fwd_proj"], 0.0) + phase["fwd_rec"] <= phase["fwd_total"] <= ms
+    # (times are fp32 milliseconds: sums of two of them agree to 1e-6)
+    assert max(phase["fwd_proj"], 0.0) + phase["fwd_rec"] <= phase["fwd_total"] * 1.000001 <= ms
     assert phase["fwd_total"] >= phase["fwd_rec"] + converted + (product if projection == 0 else 0.0)
     core.close()
 
