@@ -563,23 +563,25 @@ int forward_operand(flstm_core_plan* p, size_t t0, size_t n, bool converted, hip
 }
 
 // Whether the projection of n steps is formed beside their recurrence (ProjectBeside) by the workgroups without a seat there:
-// estimated microseconds of both ways.  A tile of 128 x 128 takes one of them 0.65 us per 64 features (what three slabs in flight
-// bring in) and 2.5, and the recurrence starts a tile later; in front of it the product takes what gemm_nt_cost says, a launch and
-// a gap.  Measured, us a forward pass, in front / beside: 512 steps of 64 rows, 1024 features and units 1275 / 990, of 16 rows of 2048
-// 1443 / 1208, of 64 rows of 640 units and 2048 features 1316 / 956; 128 steps of the first 347 / 292, 32 steps 130 / 116; where the
-// line is drawn: 32 steps of 32 rows of 1536 units, 1024 features (64 workgroups to form it) 128 / 138, 512 steps of them 1439 / 1280.
-// A step is taken for 1.9 or 2.4 us however many row blocks a workgroup has in it: with two turns a step (100 rows of 1400 units) it
-// lasts twice that, more of the product fits beside it than is reckoned with, and the rule keeps to the launch in front.  Fewer than
-// 16 workgroups are not tried: where 241 and more have seats a step takes 8 tiles or more (17 rows of 2048 units, 113 of 1024), which
-// so few keep up with for a hundred features at most, and that product is short in front, too.
+// estimated microseconds of both ways.  Where these set the pace a tile of 128 x 128 takes one of them 4.6 us and 0.52 per 64
+// features (1 / 2 / 8 / 16 / 32 slabs 5.1 / 5.7 / 8.8 / 12.8 / 21.2 us, with 16 to 96 of them at work); the recurrence starts a tile
+// later, for which the first ones, with memory to themselves, take 2.5 and 0.65.  In front of it the product takes what
+// gemm_nt_cost says, a launch and a gap.  A step takes 1.9 or 2.4 us for every row block that a workgroup has in it.
+// Measured, us a forward pass, in front / beside: 512 steps of 64 rows, 1024 features and units 1275 / 990, of 16 rows of 2048
+// 1443 / 1208, of 64 rows of 640 units and 2048 features 1316 / 956; 128 steps of the first 347 / 292, 32 steps 130 / 116; 200 steps of
+// 100 rows of 1536 units and 32 features, two turns a step 1036 / 946; the other side of the line: 256 steps of 200 rows of 512 units,
+// 32 features and 48 workgroups to form it 509 / 704, 128 features 513 / 786; 32 steps of 32 rows of 1536 units, 1024 features 128 / 138 (512 steps
+// 1439 / 1280).  Of 570 combinations measured both ways the choice is on average 0.2 % off the faster one, at most 4 % or 4 us.  Fewer than 16 workgroups are not tried: where 241 and more have seats a step takes
+// 8 tiles or more (17 rows of 2048 units, 113 of 1024), which so few do not keep up with.
 bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
     const Dims& d = p->d;
     const int helpers = rec_projecting_workgroups(p->Lf);
     if (helpers < 16 || p->opt_profile || reinterpret_cast<uintptr_t>(A) % 16 != 0) return false;
-    const double tile = d.Ip / 64 * 0.65 + 2.5, rounds = double(ceil_div(ceil_div(n * d.B, 128) * (4 * d.Hp / 128), size_t(helpers)));
-    const double recurrence = (d.Hp <= 1024 ? 1.9 : 2.4) * double(n);
+    const double slabs = d.Ip / 64, tile = slabs * 0.52 + 4.6, first = slabs * 0.65 + 2.5;
+    const double rounds = double(ceil_div(ceil_div(n * d.B, 128) * (4 * d.Hp / 128), size_t(helpers)));
+    const double recurrence = (d.Hp <= 1024 ? 1.9 : 2.4) * double(n * ceil_div(size_t(p->Lf.nrb), size_t(p->Lf.ng)));
     const double in_front = recurrence + gemm_nt_cost(int(n * d.B), 4 * d.Hp, d.Ip) + 5.0;
-    return std::fmax(recurrence, rounds * tile) + 1.5 * tile + 2.0 < in_front;
+    return std::fmax(recurrence, 1.05 * rounds * tile) + 1.5 * first + 2.0 < in_front;
 }
 
 // x rows of steps [t0, t0+n) -> fp16 operand -> x-projection (+ bias) in G, or left to the recurrence's launch
@@ -693,14 +695,41 @@ void final_states(const flstm_core_plan* p, size_t TB, void* hy, void* cy, flstm
 
 // Whether a pass can be one launch (rec_fwd_whole_kernel): the layout is the one for short contractions.
 bool whole_possible(const flstm_core_plan* p) { return !p->opt_profile && p->ring.p && rec_whole_possible(p->Lf); }
+// Microseconds a step that the projection takes inside it (fp16 rows of up to 128 features): what the exchange does not hide.
+// Measured over 64 to 1024 steps, in front / inside, us a pass: 32 units and one row 523 / 627 over 1024 steps; 256 units, 64 rows and 64
+// features 874 / 867, 128 features 871 / 882, with caches 891 / 917; 200 rows (two waves a workgroup) 1207 / 967; 384 units, 64
+// features, one row 973 / 1033, 64 rows 1088 / 1024; 512 units, 16 rows, 128 features and 256 steps 19 / 2 less than separate launches.
+double inside_step(const flstm_core_plan* p, bool save) {
+    const Dims& d = p->d;
+    const bool long_rows = d.Ip > 64;
+    if (d.Hp > 256) return long_rows ? (save ? 0.1 : 0.055) : d.B >= 16 || d.Hp > 384 ? 0.0 : 0.06;
+    if (p->Lf.split > 1) return 0.0;
+    const double short_rows = d.Hp > 128 ? (save ? 0.05 : 0.022) : d.Hp < 128 || save ? 0.1 : 0.06;
+    return short_rows + (long_rows ? 0.03 : 0.0);
+}
 // ... and whether that launch forms the projection itself: the input rows are short enough for a wave to hold its part of W_ih,
-// fp16 rows used in place are aligned, and it is the faster way.  It saves a launch and G's way through memory (7 us and more)
-// and costs a step what the exchange does not hide.  Measured over 128 steps of 64 rows, us a pass without gradients, projection
-// in front / inside: 256 units 143 / 131 with 64 features, 143 / 134 with 128, 144 / 150 with 256; 384 units 195 / 157, 196 / 169,
-// 198 / 196; 512 units 213 / 194, 211 / 203, 213 / 222; but 64 units, where a step is 0.5 us, 106 / 104, 106 / 109, 107 / 123.
-bool whole_projects(const flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype) {
-    if (p->d.Ip > kRecWholeInput || (x_in_place(p, x_dtype) && reinterpret_cast<uintptr_t>(x) % 16 != 0)) return false;
-    return T <= 32 || (p->d.Ip <= 128 && (p->d.Hp >= 256 || T <= 64));
+// fp16 rows used in place are aligned, and it is the faster way: it saves the product, a launch and a gap.  Up to 32 steps always;
+// rows of more than 128 features cost 0.3 us a step.  (Two and four waves a workgroup with 65 to 128 features: up to 192 units only
+// for 64 steps, 192 units and 200 rows 613 / 630 us over 512 with caches.)
+bool whole_projects(const flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, bool save) {
+    const Dims& d = p->d;
+    if (d.Ip > kRecWholeInput || (x_in_place(p, x_dtype) && reinterpret_cast<uintptr_t>(x) % 16 != 0)) return false;
+    if (T <= 32) return true;
+    if (d.Ip > 128 || (p->Lf.split > 1 && d.Hp <= 192 && d.Ip > 64 && T > 64)) return false;
+    return double(T) * inside_step(p, save) < gemm_nt_cost(int(T * size_t(d.B)), 4 * d.Hp, d.Ip) + 3.0;
+}
+// ... and whether one launch is the faster way at all.  It saves two launches and their gaps, 8 us.  With one wave a workgroup and up
+// to 256 units its steps are longer for what they write (caches, the caller's y) between h and the next request, 0.03 us with
+// caches, 0.015 without at 64 to 128 units and 16 to 256 rows.  Separate / one launch, us: 16 rows of 64 units, 32 features, with caches
+// 108 / 103 over 128 steps, 180 / 184 over 256, 601 / 628 over 1024; without 601 / 614.  Two and more waves and more units gain throughout
+// (512 rows of 256 units 2669 -> 998 us over 1024 steps).
+bool whole_pays(const flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, bool save) {
+    const Dims& d = p->d;
+    if (p->Lf.split > 1 || d.Hp > 256 || T <= 32) return true;
+    double loss = double(T) * (save ? 0.03 : d.Hp >= 64 && d.Hp <= 128 && d.B >= 16 && d.B <= 256 ? 0.015 : 0.0);
+    if (whole_projects(p, T, x, x_dtype, save))
+        loss += double(T) * inside_step(p, save) - gemm_nt_cost(int(T * size_t(d.B)), 4 * d.Hp, d.Ip) - 3.0;
+    return loss <= 8.0;
 }
 
 int forward_whole(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, const void* h0, const void* c0,
@@ -712,7 +741,7 @@ int forward_whole(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     p->fw.T = T; p->fw.x = x; p->fw.x_dtype = x_dtype; p->fw.open = true; p->fw.whole = true;
     RecWholeArgs a{};
     OpList prep;   // what there is to do in front of it: converted rows, a ring that is not ready, an h0 no 16-byte load fits
-    const bool projects = whole_projects(p, T, x, x_dtype);
+    const bool projects = whole_projects(p, T, x, x_dtype, save);
     if (x_in_place(p, x_dtype)) {
         a.x = static_cast<const half_t*>(x);
         a.ldx = d.I;
@@ -805,7 +834,7 @@ int forward_enqueue(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_d
     const bool rows_behind = overlap({bytes_of(y, TB * d.H, y_dtype)}, inputs);
     const bool behind = rows_behind || overlap({bytes_of(hy, BH, out_state_dtype), bytes_of(cy, BH, out_state_dtype)}, inputs);
     p->fw.behind = behind;
-    if (whole_possible(p)) {
+    if (whole_possible(p) && whole_pays(p, T, x, x_dtype, save || behind)) {
         p->fw.rows_behind = behind;
         const int rc = behind ? forward_whole(p, T, x, x_dtype, h0, c0, state_dtype, nullptr, y_dtype, nullptr, nullptr, out_state_dtype, true, s)
                               : forward_whole(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, save, s);

@@ -7,8 +7,9 @@ pytestmark = pytest.mark.gpu
 # one, two and four groups inside XCDs (what is idle: six whole XCDs, four, ...), groups across XCDs, slices of 16 units (two of them in
 # a column of tiles), two row blocks; rows that end inside a tile, one tile of rows, rows of 64 features and many
 SHAPES = [(600, 32, 1024, 1024), (300, 64, 512, 1024), (255, 33, 448, 640), (400, 7, 1024, 992), (130, 100, 2048, 640),
-          (200, 16, 2048, 2048), (150, 48, 512, 1536), (333, 9, 256, 1400), (260, 100, 512, 640)]
-IN_FRONT = [(130, 100, 2048, 640)]   # 116 workgroups would take longer over 2048 features than the recurrence and the product apart
+          (200, 16, 2048, 2048), (150, 48, 512, 1536), (333, 9, 256, 1400), (260, 100, 512, 640),
+          (64, 200, 32, 512), (60, 200, 700, 512), (40, 100, 128, 1536)]
+IN_FRONT = [(130, 100, 2048, 640), (64, 200, 32, 512), (60, 200, 700, 512)]   # so few workgroups take longer than the recurrence and the product apart
 
 
 @pytest.mark.parametrize("T,B,I,H", SHAPES)
