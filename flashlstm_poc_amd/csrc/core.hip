@@ -728,13 +728,14 @@ bool whole_projects(const flstm_core_plan* p, size_t T, const void* x, flstm_dty
 }
 // ... and whether one launch is the faster way at all.  It saves two launches and their gaps, 8 us.  With one wave a workgroup and up
 // to 256 units its steps are longer for what they write (caches, the caller's y) between h and the next request, 0.03 us with
-// caches, 0.015 without at 64 to 128 units and 16 to 256 rows.  Separate / one launch, us: 16 rows of 64 units, 32 features, with caches
-// 108 / 103 over 128 steps, 180 / 184 over 256, 601 / 628 over 1024; without 601 / 614.  Two and more waves and more units gain throughout
+// caches, 0.015 without at 64 to 128 units, 16 to 256 rows and up to 128 features.  Separate / one launch, us: 16 rows of 64 units, 32
+// features, with caches 108 / 103 over 128 steps, 180 / 184 over 256, 601 / 628 over 1024; without 601 / 614; 133 rows of 120 units and 1799
+// features over 1292 steps, without, 1930 / 1869.  Two and more waves and more units gain throughout
 // (512 rows of 256 units 2669 -> 998 us over 1024 steps).
 bool whole_pays(const flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dtype, bool save) {
     const Dims& d = p->d;
     if (p->Lf.split > 1 || d.Hp > 256 || T <= 32) return true;
-    double loss = double(T) * (save ? 0.03 : d.Hp >= 64 && d.Hp <= 128 && d.B >= 16 && d.B <= 256 ? 0.015 : 0.0);
+    double loss = double(T) * (save ? 0.03 : d.Hp >= 64 && d.Hp <= 128 && d.Ip <= 128 && d.B >= 16 && d.B <= 256 ? 0.015 : 0.0);
     if (whole_projects(p, T, x, x_dtype, save))
         loss += double(T) * inside_step(p, save) - gemm_nt_cost(int(T * size_t(d.B)), 4 * d.Hp, d.Ip) - 3.0;
     return loss <= 8.0;

@@ -22,7 +22,7 @@ def cached(core, which, rows, dtype):
 # one to five steps (pairs and a single one left), row tiles of 1, 16 and 17 rows, rows of less than and exactly 64, 128 and 256
 # features and of more, every length of the contraction, odd widths; T = 64 crosses the rule for few units, 33 the one for 256 features
 SHAPES = [(1, 1, 128, 256), (2, 16, 64, 64), (3, 17, 65, 33), (4, 3, 1, 1), (5, 40, 256, 512), (33, 20, 200, 130), (32, 20, 200, 130),
-          (70, 5, 128, 96), (64, 5, 128, 96), (50, 5, 128, 96), (9, 100, 300, 512), (12, 512, 20, 256), (7, 128, 64, 257), (6, 64, 129, 384), (37, 33, 100, 384)]
+          (70, 5, 128, 96), (64, 5, 128, 96), (45, 5, 128, 96), (9, 100, 300, 512), (12, 512, 20, 256), (7, 128, 64, 257), (6, 64, 129, 384), (37, 33, 100, 384)]
 IN_FRONT = [(33, 20, 200, 130), (70, 5, 128, 96), (64, 5, 128, 96), (9, 100, 300, 512)]   # whose projection has a launch of its own
 
 
