@@ -3760,8 +3760,11 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.wide = fits && Hp > 2048;
     // 1025 to 1536 units: slices of 32 units, as backward, where all 16-row blocks run side by side that way or take fewer turns a
     // step than blocks of 32 with slices of 16.  Measured at 1536 units, us per step: 33 to 64 rows 2.85 -> 2.55, 80 rows 4.8 -> 2.6, 160 rows
-    // 8.4 -> 4.9; with as many turns (100, 161 rows) a tie, at 1280 units and 161 rows 4.6 -> 4.95.
-    if (force_mt != 2 && Hp > 1024 && Hp <= kBroadMost && !can_16_rows(B, Hp / 16, num_cus) && Hp / 32 <= num_cus &&
+    // 8.4 -> 4.9; with as many turns (100, 161 rows) a tie, at 1280 units and 161 rows 4.6 -> 4.95.  So it is from 33 rows on where slices of
+    // 16 seat them too (up to 1360 units): three groups of those, most of the CUs, fetch over the XCDs twice as often.  A pass of 200 steps,
+    // slices of 16 / 32, us: 33 rows of 1056 units 534 / 483, 48 rows of 1216 605 / 492, with 1024 features 698 / 504; 24 rows of 1300 514 / 514,
+    // 17 rows 472 / 509, 24 rows of 1536 468 / 514.
+    if (force_mt != 2 && Hp > 1024 && Hp <= kBroadMost && (B > 32 || !can_16_rows(B, Hp / 16, num_cus)) && Hp / 32 <= num_cus &&
         (can_16_rows(B, Hp / 32, num_cus) || turns(B, 16, Hp / 32, num_cus) < turns(B, 32, Hp / 16, num_cus))) {
         L.broad = 1;
         L.nt = 8;

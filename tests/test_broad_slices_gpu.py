@@ -57,6 +57,26 @@ def test_slices_of_32_units_against_64_bits_and_32_row_blocks(T, B, H):
     core.close()
 
 
+# 33 to 48 rows where slices of 16 would seat them as well: forward alone; one row fewer keeps those
+@pytest.mark.parametrize("T,B,H,forward", [(22, 33, 1056, 32), (21, 40, 1216, 32), (23, 48, 1344, 32), (21, 32, 1216, 16)])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_forward_slices_where_both_kinds_are_seated(T, B, H, forward, stepwise):
+    from flashlstm_poc_amd import LstmCore
+    from helpers import reference_64, rell2
+    p = make_problem(T, B, 24, H, seed=B * 10000 + H)
+    ref = {k: v.cpu().numpy() for k, v in reference_64(p).items()}
+    core = LstmCore(B, 24, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    got, info = run_core(p, core=core, stepwise=stepwise)
+    assert info["fallbacks"] == 0 and core.info("slice_fwd") == forward and core.info("slice_bwd") == 16
+    core.set_option("row_tiles_fwd", 2)
+    blocks, info = run_core(p, core=core)
+    assert info["fallbacks"] == 0 and core.info("slice_fwd") == 16
+    for k in ref:   # (as above)
+        assert rell2(got[k], ref[k]) <= 1.05 * rell2(blocks[k], ref[k]), (k, rell2(got[k], ref[k]), rell2(blocks[k], ref[k]))
+    core.close()
+
+
 @pytest.mark.parametrize("T,B,H", [(21, 80, 1100), (23, 48, 1536), (20, 90, 1400)])
 def test_slices_of_32_units_in_ranges_of_steps(T, B, H):
     from test_kernel_variants_gpu import test_wide_layers_in_ranges_of_steps as in_ranges
