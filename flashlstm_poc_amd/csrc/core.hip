@@ -710,7 +710,7 @@ bool whole_possible(const flstm_core_plan* p) { return !p->opt_profile && p->rin
 double inside_step(const flstm_core_plan* p, bool save) {
     const Dims& d = p->d;
     const bool long_rows = d.Ip > 64;
-    if (d.Hp > 256) return long_rows ? (save ? 0.1 : 0.05) : d.B >= 16 || d.Hp > 384 ? 0.0 : 0.06;
+    if (d.Hp > 256) return long_rows ? (save ? 0.1 : 0.05) : d.B >= 4 || d.Hp > 384 ? 0.0 : 0.06;
     if (p->Lf.split > 1) return 0.0;
     const double short_rows = d.Hp > 128 ? (save ? 0.05 : 0.022) : d.Hp < 128 || save ? 0.1 : 0.06;
     return short_rows + (long_rows ? (d.Hp > 128 ? 0.03 : 0.035) : 0.0);
@@ -879,6 +879,7 @@ int forward_conclude(flstm_core_plan* p, hipStream_t s) {
         p->ring_ready = true;
     }
     if (st != 0) {
+        p->fw.begin_on_device = false;   // (there are no times of a pass that gave up)
         if (p->Lf.persistent) demote(p, true);   // workgroups not co-resident or not where expected: next time with one launch per step
         return FLSTM_E_STALLED;
     }

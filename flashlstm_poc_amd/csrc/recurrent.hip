@@ -2908,6 +2908,8 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
 // 1.17 -> 0.89, 128 units and 200 rows 1.35 -> 1.09, 256 units and 8 rows 1.79 -> 1.54 -> 1.49, 257 units and 70 rows 2.13 -> 1.79 -> 1.59,
 // 384 units and 100 rows 1.94 -> 1.75.  (Four waves with one cell per lane: 1.65 at
 // 256 units; the longer barrier costs more than the shorter update gives.)
+// LATE = false has them behind the fragments: four rows of 32 units, or two of 64 over a short sequence, find the fragments there and
+// gain the head start (run_bwd_pair).
 template <int KS, int K>
 __device__ __forceinline__ void request_pair_one(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off) {
     if constexpr (K >= KS - 3) ld_frag_async_off<0>(f[K], tail_off[K - (KS - 3)], tile);
@@ -2924,7 +2926,7 @@ __device__ __forceinline__ void ld_stream_at(floatx2& d, const void* base, unsig
 __device__ __forceinline__ void ld_stream_at(unsigned& d, const void* base, unsigned off) {
     asm volatile("global_load_dword %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
 }
-template <int KS>
+template <int KS, bool LATE>
 __global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, RecLayout L, int t_first, int t_last, int) {
     static_assert(KS % 4 == 0 && KS <= 24, "up to 384 hidden units");
     __shared__ int lds_abort;
@@ -3046,7 +3048,8 @@ __global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, R
         half8 f[KS];
         auto request = [&]() __attribute__((always_inline)) { request_pair(f, tile, lane_off, tail_off, std::make_integer_sequence<int, KS>{}); };
         request();
-        wait_set<0>(f);
+        if constexpr (!LATE) request_ops(t - 1, std::integral_constant<int, 1 - par>{});
+        wait_set<LATE ? 0 : 4>(f);
         auto unwritten = [&]() -> bool {
             unsigned m = 0u;
 #pragma unroll
@@ -3065,7 +3068,7 @@ __global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, R
                 wait_set<0>(f);
             } while (unwritten());
         }
-        request_ops(t - 1, std::integral_constant<int, 1 - par>{});
+        if constexpr (LATE) request_ops(t - 1, std::integral_constant<int, 1 - par>{});
         floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int k = 0; k < KS; ++k) acc[k % 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[k], f[k], acc[k % 2], 0, 0, 0);
@@ -4242,9 +4245,9 @@ static hipError_t run_bwd2d(const RecLayout& L, const RecBwdArgs& a, hipStream_t
     return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
 }
 
-template <int KS>
+template <int KS, bool LATE = true>
 static hipError_t run_bwd_pair(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
-    auto kernel = rec_bwd_pair_kernel<KS>;
+    auto kernel = rec_bwd_pair_kernel<KS, LATE>;
     if (L.nt != 1 || L.nw != 2 || L.jb != 16 || L.mt != 1 || L.nrb > L.ng || a.Hp / 16 > KS || a.Hp / 16 < KS - 2 || (L.persistent && !L.xcd_local))
         return hipErrorInvalidValue;
     static std::atomic<int> per_cu[kMaxDevices];
@@ -4317,6 +4320,10 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
     const bool ds = L.persistent && !L.xcd_local;   // (as in launch_rec_fwd)
     if (!L.resident) return run_bwd<2, 1, false, 0, 2, false>(L, a, stream, graphs);
     if (L.split) {
+        // When the next step's operands are requested (rec_bwd_pair_kernel).  Behind the fragments / once those are there, us a pass: 32
+        // units and one row 191 / 199 over 200 steps, 616 / 655 over 800, four rows 193 / 199 and 630 / 666, six 196 / 201 and 811 / 659; 64
+        // units and one row 195 / 203 and 742 / 685, two rows 199 / 206 and 794 / 688, four 226 / 207 and 860 / 692.
+        if (a.Hp <= 64 && a.B * a.Hp <= 128 && (a.Hp <= 32 || a.T <= 256)) return run_bwd_pair<4, false>(L, a, stream, graphs);
         switch ((a.Hp / 16 + 3) / 4) {
 #define FLSTM_PAIR_CASE(n) case n: return run_bwd_pair<4 * n>(L, a, stream, graphs);
             FLSTM_PAIR_CASE(1) FLSTM_PAIR_CASE(2) FLSTM_PAIR_CASE(3) FLSTM_PAIR_CASE(4) FLSTM_PAIR_CASE(5) FLSTM_PAIR_CASE(6)

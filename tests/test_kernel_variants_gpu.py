@@ -46,6 +46,18 @@ def test_recurrence_kernels_for_short_contractions(T, B, H, stepwise):
     check_against(ref, got, label=f"T={T} B={B} H={H} stepwise={stepwise}")
 
 
+# few rows of 32 and 64 units, backward: the two moments at which a step's operands are requested, on both sides of their line, over
+# sequences of one, an odd and an even number of steps and some that reuse every slot of the ring
+@pytest.mark.parametrize("T,B,H", [(1, 1, 32), (2, 4, 32), (3, 5, 32), (21, 4, 17), (40, 1, 64), (33, 2, 60), (34, 3, 64), (256, 2, 64), (257, 2, 64)])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_backward_of_few_rows_of_small_layers(T, B, H, stepwise):
+    p = make_problem(T, B, 20, H, seed=B * 10000 + H)
+    ref, _ = oracle_reference(p)
+    got, info = run_core(p, stepwise=stepwise)
+    assert info["fallbacks"] == 0
+    check_against(ref, got, label=f"T={T} B={B} H={H} stepwise={stepwise}")
+
+
 # 32-row blocks asked for where the rule takes the kernels for short contractions, which have 16-row blocks: the option and
 # a tuned entry are both honoured, after the weights were packed, and taken back without packing again.  One and several row
 # blocks, a partial one, a hidden size per kernel family: both short kernels (256), the forward one alone (385, 512)
