@@ -574,12 +574,14 @@ int forward_operand(flstm_core_plan* p, size_t t0, size_t n, bool converted, hip
 // estimated microseconds of both ways.  Where these set the pace a tile of 128 x 128 takes one of them 4.6 us and 0.52 per 64
 // features (1 / 2 / 8 / 16 / 32 slabs 5.1 / 5.7 / 8.8 / 12.8 / 21.2 us, with 16 to 96 of them at work); the recurrence starts a tile
 // later, for which the first ones, with memory to themselves, take 2.5 and 0.65.  In front of it the product takes what
-// gemm_nt_cost says, a launch and a gap.  A step takes 1.9 or 2.4 us for every row block that a workgroup has in it.
+// gemm_nt_cost says, a launch and a gap.  A step takes 1.65 us (to 768 units), 1.8 (to 1024) or 2.4 for every row block that a
+// workgroup has in it; behind the last tile there are the steps of its 128 rows left.
 // Measured, us a forward pass, in front / beside: 512 steps of 64 rows, 1024 features and units 1275 / 990, of 16 rows of 2048
 // 1443 / 1208, of 64 rows of 640 units and 2048 features 1316 / 956; 128 steps of the first 347 / 292, 32 steps 130 / 116; 200 steps of
 // 100 rows of 1536 units and 32 features, two turns a step 1036 / 946; the other side of the line: 256 steps of 200 rows of 512 units,
 // 32 features and 48 workgroups to form it 509 / 704, 128 features 513 / 786; 32 steps of 32 rows of 1536 units, 1024 features 128 / 138 (512 steps
-// 1439 / 1280).  Of 570 combinations measured both ways the choice is on average 0.2 % off the faster one, at most 4 % or 4 us.  Fewer than 16 workgroups are not tried: where 241 and more have seats a step takes
+// 1439 / 1280); 211 steps of 256 rows of 384 units and 32 features 389 / 438.  Of 570 combinations measured both ways the choice is on
+// average 0.15 % off the faster one, at most 3 us or 2 % where it is beside.  Fewer than 16 workgroups are not tried: where 241 and more have seats a step takes
 // 8 tiles or more (17 rows of 2048 units, 113 of 1024), which so few do not keep up with.
 bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
     const Dims& d = p->d;
@@ -587,9 +589,10 @@ bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
     if (helpers < 16 || p->opt_profile || reinterpret_cast<uintptr_t>(A) % 16 != 0) return false;
     const double slabs = d.Ip / 64, tile = slabs * 0.52 + 4.6, first = slabs * 0.65 + 2.5;
     const double rounds = double(ceil_div(ceil_div(n * d.B, 128) * (4 * d.Hp / 128), size_t(helpers)));
-    const double recurrence = (d.Hp <= 1024 ? 1.9 : 2.4) * double(n * ceil_div(size_t(p->Lf.nrb), size_t(p->Lf.ng)));
+    const double step = (d.Hp <= 768 ? 1.65 : d.Hp <= 1024 ? 1.8 : 2.4) * double(ceil_div(size_t(p->Lf.nrb), size_t(p->Lf.ng)));
+    const double recurrence = step * double(n), last = step * std::fmin(double(n), 128.0 / d.B);
     const double in_front = recurrence + gemm_nt_cost(int(n * d.B), 4 * d.Hp, d.Ip) + 5.0;
-    return std::fmax(recurrence, 1.05 * rounds * tile) + 1.5 * first + 2.0 < in_front;
+    return std::fmax(recurrence + 1.5 * first + 2.0, 1.05 * rounds * tile + last + 4.0) < in_front;
 }
 
 // x rows of steps [t0, t0+n) -> fp16 operand -> x-projection (+ bias) in G, or left to the recurrence's launch
