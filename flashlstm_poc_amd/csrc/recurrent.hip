@@ -2908,8 +2908,8 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
 // 1.17 -> 0.89, 128 units and 200 rows 1.35 -> 1.09, 256 units and 8 rows 1.79 -> 1.54 -> 1.49, 257 units and 70 rows 2.13 -> 1.79 -> 1.59,
 // 384 units and 100 rows 1.94 -> 1.75.  (Four waves with one cell per lane: 1.65 at
 // 256 units; the longer barrier costs more than the shorter update gives.)
-// LATE = false has them behind the fragments: four rows of 32 units, or two of 64 over a short sequence, find the fragments there and
-// gain the head start (run_bwd_pair).
+// LATE = false has them behind the fragments: one to four rows of up to 64 units over a short sequence find the fragments there and gain
+// the head start (launch_rec_bwd).
 template <int KS, int K>
 __device__ __forceinline__ void request_pair_one(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off) {
     if constexpr (K >= KS - 3) ld_frag_async_off<0>(f[K], tail_off[K - (KS - 3)], tile);
@@ -4320,10 +4320,11 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
     const bool ds = L.persistent && !L.xcd_local;   // (as in launch_rec_fwd)
     if (!L.resident) return run_bwd<2, 1, false, 0, 2, false>(L, a, stream, graphs);
     if (L.split) {
-        // When the next step's operands are requested (rec_bwd_pair_kernel).  Behind the fragments / once those are there, us a pass: 32
-        // units and one row 191 / 199 over 200 steps, 616 / 655 over 800, four rows 193 / 199 and 630 / 666, six 196 / 201 and 811 / 659; 64
-        // units and one row 195 / 203 and 742 / 685, two rows 199 / 206 and 794 / 688, four 226 / 207 and 860 / 692.
-        if (a.Hp <= 64 && a.B * a.Hp <= 128 && (a.Hp <= 32 || a.T <= 256)) return run_bwd_pair<4, false>(L, a, stream, graphs);
+        // When the next step's operands are requested (rec_bwd_pair_kernel): behind the fragments while those of the whole pass, 14 bytes
+        // a cell and step, are still in the XCD's L2.  Behind the fragments / once those are there, us a pass: 32 units and one row 189 / 203
+        // over 200 steps, 762 / 830 over 1000, two rows 720 / 750 over 900, 1373 / 1211 over 1500, three 347 / 359 over 400, 983 / 824 over 1000, four 196 / 204
+        // over 200, 571 / 507 over 600; 64 units and one row 191 / 208 over 200, 742 / 685 over 800, two rows 232 / 254 over 256; four 226 / 207 over 200.
+        if (a.Hp <= 64 && a.B * a.Hp <= 128 && (long long)a.T * a.B * a.Hp <= 32768) return run_bwd_pair<4, false>(L, a, stream, graphs);
         switch ((a.Hp / 16 + 3) / 4) {
 #define FLSTM_PAIR_CASE(n) case n: return run_bwd_pair<4 * n>(L, a, stream, graphs);
             FLSTM_PAIR_CASE(1) FLSTM_PAIR_CASE(2) FLSTM_PAIR_CASE(3) FLSTM_PAIR_CASE(4) FLSTM_PAIR_CASE(5) FLSTM_PAIR_CASE(6)

@@ -48,7 +48,7 @@ def test_recurrence_kernels_for_short_contractions(T, B, H, stepwise):
 
 # few rows of 32 and 64 units, backward: the two moments at which a step's operands are requested, on both sides of their line, over
 # sequences of one, an odd and an even number of steps and some that reuse every slot of the ring
-@pytest.mark.parametrize("T,B,H", [(1, 1, 32), (2, 4, 32), (3, 5, 32), (21, 4, 17), (40, 1, 64), (33, 2, 60), (34, 3, 64), (256, 2, 64), (257, 2, 64)])
+@pytest.mark.parametrize("T,B,H", [(1, 1, 32), (2, 4, 32), (3, 5, 32), (21, 4, 17), (40, 1, 64), (33, 2, 60), (34, 3, 64), (256, 2, 64), (257, 2, 64), (257, 4, 32)])
 @pytest.mark.parametrize("stepwise", [False, True])
 def test_backward_of_few_rows_of_small_layers(T, B, H, stepwise):
     p = make_problem(T, B, 20, H, seed=B * 10000 + H)
