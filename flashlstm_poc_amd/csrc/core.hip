@@ -145,6 +145,7 @@ struct flstm_core_plan {
              bool behind = false;          // the caller's final states are written by a launch of their own behind the recurrence ...
              bool rows_behind = false; } fw;   // ... and y with them
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
+             int few = 0;   // RecLayout::few that the exchange ring is laid out for
              BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false;
              bool shared = false; } bw;   // dX and the weight gradients in one launch
     DevBuf tile_words;         // ProjectBeside::ready
@@ -453,7 +454,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
         return e;
     };
     const RecLayout fwd = plan_rec_fwd(d.B, d.Hp, p->num_cus, false, 2, p->opt_waves_f), split = plan_rec_fwd(d.B, d.Hp, p->num_cus, false);
-    const RecLayout bwd = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 2, 0), pair = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 0, 0);
+    const RecLayout bwd = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 2, 0), broad = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 0, 0);
     FL_TRY(want(kFragFwd, fwd, rec_fwd_ks(fwd, d.Hp), rec_fwd_fragments(fwd, d.Hp)));
     frag[kFragFwd].wide = fwd.wide;
     if (split.split || split.broad) {
@@ -462,7 +463,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
         if (split.split) FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));   // (here: flstm_core_forward_static allocates nothing)
     }
     FL_TRY(want(kFragBwd, bwd, rec_bwd_ks(bwd, d.Hp), rec_bwd_fragments(bwd, d.Hp)));
-    if (pair.split || pair.broad) FL_TRY(want(kFragBwdPair, pair, rec_bwd_ks(pair, d.Hp), rec_bwd_fragments(pair, d.Hp)));
+    if (broad.broad) FL_TRY(want(kFragBwdBroad, broad, rec_bwd_ks(broad, d.Hp), rec_bwd_fragments(broad, d.Hp)));
     if (rec_bwd_two_d_possible(d.Hp, p->num_cus)) {
         FragLayout& f = frag[kFragBwdTwoD];
         f.kq = rec_bwd_two_d_kq(d.B, d.Hp);
@@ -1002,7 +1003,8 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     FL_TRY(p->dH0.reserve(st_bytes));
     FL_TRY(p->dG.reserve(TB * 4 * d.Hp * sizeof(half_t)));
     FL_TRY(p->db_part.reserve(size_t(p->Lb.ng) * 4 * d.Hp * sizeof(float)));
-    const size_t xslot = exchange_slot_halfs(rec_bwd_ring_rows(p->Lb, d.B), 4 * d.Hp);
+    const size_t xslot = rec_bwd_slot_halfs(p->Lb, d.B, d.Hp);
+    p->bw.few = p->Lb.few;
     const size_t dg_slots = size_t(rec_bwd_dg_slots(p->Lb));
     FL_TRY(p->xch_b.reserve(dg_slots * xslot * sizeof(half_t)));
     // One launch (see forward_setup): the dG ring 'unwritten', the ring of partial sums in its starting parities, the
@@ -1047,10 +1049,10 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
     }
     RecBwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (as in forward_recur)
-    a.wfrag = p->wfrag[p->Lb.split || p->Lb.broad ? kFragBwdPair : kFragBwd].as<half8>();
+    a.wfrag = p->wfrag[p->Lb.broad ? kFragBwdBroad : kFragBwd].as<half8>();
     a.G = p->G.as<half_t>(); a.C = p->C.as<float>(); a.dY = p->bw.dYk; a.dG = p->dG.as<half_t>();
     a.dHn = p->dHn.as<float>(); a.dC = p->dC.as<float>(); a.dH0 = p->dH0.as<float>();
-    a.X = p->xch_b.as<half_t>(); a.x_slot = exchange_slot_halfs(rec_bwd_ring_rows(p->Lb, d.B), 4 * d.Hp);
+    a.X = p->xch_b.as<half_t>(); a.x_slot = rec_bwd_slot_halfs(p->Lb, d.B, d.Hp);
     if (p->Lb.two_d) {
         a.wfrag2 = p->wfrag[kFragBwdTwoD].as<half8>();
         a.P = p->part_b.as<float>();
@@ -1460,6 +1462,10 @@ extern "C" int flstm_core_backward_steps(flstm_core_plan* p, size_t t_hi, size_t
     if (!p || !p->bw.open || t_hi >= p->bw.T || nsteps == 0 || nsteps > t_hi + 1) return FLSTM_E_INVALID;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const long lo = long(t_hi) - long(nsteps) + 1;
+    if (p->bw.few != p->Lb.few) {   // (an option has changed the layout, and with it the ring: the caller repeats the pass)
+        p->bw.open = false;
+        return FLSTM_E_STALLED;
+    }
     // the range that reaches step 0 also runs the closing product for dh0
     int rc = backward_recur(p, long(t_hi), lo == 0 ? -1 : lo, false, s);
     if (rc == int(hipErrorCooperativeLaunchTooLarge) && p->Lb.persistent && !p->refused_bwd) {

@@ -21,8 +21,9 @@ struct FragLayout {   // where a recurrence kernel expects its weight fragments:
     size_t fragments = 0;   // of 64 lanes
 };
 // Forward: the one-way kernels' and those of the kernel for short contractions, or with slices of 32 units (RecLayout::broad);
-// backward the same; those of the backward recurrence that splits its product two ways.
-enum Frag : int { kFragFwd, kFragFwdSplit, kFragBwd, kFragBwdPair, kFragBwdTwoD, kFragKinds };
+// backward the one-way kernels' (which that for few rows uses as well), with slices of 32 units, and those of the recurrence that splits its
+// product two ways.
+enum Frag : int { kFragFwd, kFragFwdSplit, kFragBwd, kFragBwdBroad, kFragBwdTwoD, kFragKinds };
 // W_ih twice (as it is for the projection, transposed for dX) and W_hh as every kind of fragments asked for; one launch.
 hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p /*[4Hp][Ip]*/,
                         half_t* wih_t /*[Ip][4Hp]*/, const FragLayout (&frag)[kFragKinds], hipStream_t s);

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kT) void pack_kernel(PackJob job) {
         const FragLayout& f = job.frag[which - 2];
         if (item >= f.fragments * kWave) return;
         const int kind = which - 2;
-        f.out[item] = kind <= kFragFwdSplit ? frag_values_fwd(d, job.w_hh, f, item) : kind <= kFragBwdPair ? frag_values_bwd(d, job.w_hh, f, item) : frag_values_two_d(d, job.w_hh, f, item);
+        f.out[item] = kind <= kFragFwdSplit ? frag_values_fwd(d, job.w_hh, f, item) : kind <= kFragBwdBroad ? frag_values_bwd(d, job.w_hh, f, item) : frag_values_two_d(d, job.w_hh, f, item);
     }
 }
 

@@ -34,10 +34,11 @@
 //  * Fallback.  The same kernels launched once per step (no waits, kernel boundaries order
 //    memory) serve shapes whose weights do not fit on chip (more than 4096 hidden units), and are the
 //    safe path after a failed persistent launch.
-//  * The layout above is that of the one-way kernels.  Up to 512 (forward) and 384 (backward) units the waves of a
-//    workgroup split the columns instead (rec_fwd_split_kernel, rec_bwd_pair_kernel); rec_fwd_il_kernel has eight waves and
-//    two chains; rec_bwd2d_kernel splits the product two ways at 2048 units; above that rec_fwd_wide_kernel and
+//  * The layout above is that of the one-way kernels.  Up to 512 units the waves of a forward workgroup split the columns
+//    instead (rec_fwd_split_kernel); rec_bwd_few_kernel takes blocks of fewer rows up to 1024 units;
+//    rec_fwd_il_kernel has eight waves and two chains; rec_bwd2d_kernel splits the product two ways at 2048 units; above that rec_fwd_wide_kernel and
 //    rec_bwd_wide_kernel hold half a megabyte of weights per workgroup.  Each says why where it stands.
+#include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <mutex>
@@ -260,6 +261,19 @@ __device__ __forceinline__ void wait_set(half8 (&a)[K]) {
         if (k == 0) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(a[k]), "+v"(a[k + 1]) : "n"(N) : "memory");
         else asm volatile("" : "+v"(a[k]), "+v"(a[k + 1])::"memory");
     }
+}
+
+// ... of any size, with the count as a value that is a constant once unrolled (loads behind it, a multiple of K).
+template <int K>
+__device__ __forceinline__ void wait_chunk(half8 (&a)[K], int younger) {
+    switch (younger / K) {
+#define FLSTM_WAIT_CASE(n) case n: asm volatile("s_waitcnt vmcnt(%1)" : "+v"(a[0]) : "n"(n * K) : "memory"); break;
+        FLSTM_WAIT_CASE(1) FLSTM_WAIT_CASE(2) FLSTM_WAIT_CASE(3) FLSTM_WAIT_CASE(4) FLSTM_WAIT_CASE(5)
+#undef FLSTM_WAIT_CASE
+        default: asm volatile("s_waitcnt vmcnt(0)" : "+v"(a[0])::"memory"); break;   // (waiting for more is always safe)
+    }
+#pragma unroll
+    for (int k = 1; k < K; ++k) asm volatile("" : "+v"(a[k])::"memory");
 }
 
 // The same with the count as a value: for callers whose count is a constant only after unrolling.
@@ -811,6 +825,9 @@ __device__ __forceinline__ void ld_stream(floatx4& d, const void* p) {
     asm volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(d) : "v"(p) : "memory");
 }
 __device__ __forceinline__ void wait_all_vm() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Weight fragments that stay for the whole launch go to the accumulation registers, which an MFMA reads as well: the sums are then
+// in vector registers, where they are added without being copied first.
+__device__ __forceinline__ void keep_aside(half8& w) { asm volatile("" : "+a"(w)); }
 template <typename T>
 __device__ __forceinline__ void settle(T& x) { asm volatile("" : "+v"(x)); }   // no use of x moves above this point
 __device__ __forceinline__ void to_floats(const F32<2>& r, float (&f)[2]) { f[0] = r.v.x; f[1] = r.v.y; }
@@ -1680,6 +1697,16 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
     clk.flush();
 }
 
+// the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
+__device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
+__device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
+__device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
+__device__ __forceinline__ unsigned as_bits(float v) { return __builtin_bit_cast(unsigned, v); }
+// the value of the lane N rows further on in the same 16
+template <int N>
+__device__ __forceinline__ float row_ahead(float v) {
+    return as_float(unsigned(__builtin_amdgcn_update_dpp(0, int(as_bits(v)), 0x100 | N, 0xF, 0xF, true)));
+}
 // ---------------------------------------------------------------- forward, short contractions, a whole pass
 // A pass of rec_fwd_split_kernel is four launches: state rows, ring and counters; projection; recurrence; outputs.  Here it is
 // this launch alone, with one in front of it where x has to be converted, or the projection where rows are long.  Measured, us
@@ -2226,11 +2253,6 @@ __device__ __forceinline__ void ld_coherent_at(uintx4& d, const void* base, unsi
 __device__ __forceinline__ void st_at(void* base, unsigned off, uintx4 v) {
     asm volatile("global_store_dwordx4 %0, %1, %2" ::"v"(off), "v"(v), "s"(base) : "memory");
 }
-// the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
-__device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
-__device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
-__device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
-__device__ __forceinline__ unsigned as_bits(float v) { return __builtin_bit_cast(unsigned, v); }
 
 // Forward: a workgroup owns the 64 gate columns of 16 units over the whole contraction.  Gate columns are packed
 // unit-major, so a thread finds the four gate sums of its cell in one 16-byte LDS read per wave.
@@ -2897,42 +2919,38 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
     }
 }
 
-// -------------------------------------------------------------------- backward, short contractions
-// The same for the backward recurrence up to 384 units, with what its four times longer contraction allows: a workgroup of
-// TWO waves owns 16 units (one column tile).  The waves split the contraction, exchange half of their sums through LDS (8
-// bytes per lane, one barrier) and update the cells of two neighbouring units each, one 16-byte chunk of the ring per lane.
-// Against the kernel above: as many fragment loads per CU, half the columns to sum over half the waves.  The operands of
-// step t - 1 (gates, c, dY) are requested once the fragments of step t are there: requested behind them, a wave that finds the
-// fragments unwritten and asks again waits for those operands' trip to memory as well, since loads return in order.
-// Measured, us per step, rec_bwd_kernel -> here with the operands behind the fragments -> once those are there: 64 units 1.62 ->
-// 1.17 -> 0.89, 128 units and 200 rows 1.35 -> 1.09, 256 units and 8 rows 1.79 -> 1.54 -> 1.49, 257 units and 70 rows 2.13 -> 1.79 -> 1.59,
-// 384 units and 100 rows 1.94 -> 1.75.  (Four waves with one cell per lane: 1.65 at
-// 256 units; the longer barrier costs more than the shorter update gives.)
-// LATE = false has them behind the fragments: one to four rows of up to 64 units over a short sequence find the fragments there and gain
-// the head start (launch_rec_bwd).
-template <int KS, int K>
-__device__ __forceinline__ void request_pair_one(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off) {
-    if constexpr (K >= KS - 3) ld_frag_async_off<0>(f[K], tail_off[K - (KS - 3)], tile);
-    else ld_frag_async_off<(K % 2) * 2048>(f[K], lane_off[K / 2], tile);
+// -------------------------------------------------------------------- backward, few rows per group
+// 385 to 1024 units where blocks of RB = 8 or 4 rows can all run side by side, each on an XCD's share of workgroups of its own.  A step
+// of rec_bwd_kernel is bound by the fetch of dG_{t+1}: a workgroup owns 32 columns of the product and pulls all 4 Hp gate columns of its 16 rows
+// through the CU's one vector-memory path (128 KiB at 1024 units, 128 loads, 1 us), and the 32 workgroups of an XCD the same lines through
+// one L2.  Fewer rows per group fetch less only if the fragments stay full: an A-fragment has 16 rows whatever the batch has.  Here a
+// fragment holds PK = 16 / RB k-steps of RB rows each -- rows RB*s .. of the tile are k-step s of the pack -- and is multiplied by
+// the weights of each of its k-steps in turn, into an accumulator of its own: of accumulator s only the lanes of rows RB*s .. mean something (the others
+// have met another k-step's operand), and they are added up across the lanes of the tile once, at the end.  As many MFMAs as before, 1 / PK of
+// the loads, and 1 / PK of the cells: wave w updates the 8 units of the slice whose gate columns are k-step w of it, one cell per lane.
+//   ring (halfs): group g, pack P of wave w's k-steps (4 i + w, i = PK*P + s), row r, column q = 32 (4 i + w) + q%32:
+//   g * tile_halfs + (4 P + w) * 512 + (r + RB*s + 16 * (q%32 / 8)) * 8 + q%8
+// k-steps past the contraction that a pack reaches into are written as zeros once per launch, by the last slice's workgroup.
+// The ring protocol is rec_bwd_kernel's.  All fragments of a step are requested at once; the cell operands of step t - 1 (gates, c, dY) once
+// they are there: requested behind them, a wave that finds the fragments unwritten and asks again waits for those operands' trip to
+// memory as well, since loads return in order.  One barrier a step; what a step consists of is the trip of dG through the L2 (0.8 us), then
+// the MFMAs (0.45 us at 1024 units), the partial sums and one cell a lane.
+// Measured, us a step, rec_bwd_kernel (above 384 units) or a kernel of two waves with 16 units each -> blocks of 8 -> of 4 rows: 1024
+// units and 32 rows 2.67 -> 1.71 -> 1.43, 64 rows 2.69 -> 1.74, 650 and 20 rows 2.48 -> 1.49 -> 1.33, 512 and 64 rows 2.10 -> 1.19 ->
+// 1.11, 257 and 70 rows 1.63 -> 1.11 -> 1.06, 256 and 8 rows 1.45 -> 1.00 -> 0.91, 64 and 16 rows 0.89 -> 0.89 -> 0.84.
+template <int RB>
+__device__ __forceinline__ unsigned few_offset(int i, int wave, int row, int chunk, int half) {
+    constexpr int PK = 16 / RB;
+    return unsigned(((i / PK) * 4 + wave) * 512 + ((row + RB * (i % PK)) + 16 * chunk) * 8 + half * 4);
 }
-template <int KS, int... K>
-__device__ __forceinline__ void request_pair(half8 (&f)[KS], const half_t* tile, const unsigned* lane_off, const unsigned* tail_off,
-                                             std::integer_sequence<int, K...>) {
-    (request_pair_one<KS, K>(f, tile, lane_off, tail_off), ...);
-}
-__device__ __forceinline__ void ld_stream_at(floatx2& d, const void* base, unsigned off) {
-    asm volatile("global_load_dwordx2 %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
-}
-__device__ __forceinline__ void ld_stream_at(unsigned& d, const void* base, unsigned off) {
-    asm volatile("global_load_dword %0, %1, %2 nt" : "=v"(d) : "v"(off), "s"(base) : "memory");
-}
-template <int KS, bool LATE>
-__global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, RecLayout L, int t_first, int t_last, int) {
-    static_assert(KS % 4 == 0 && KS <= 24, "up to 384 hidden units");
+template <int KS, int RB, int CH>
+__global__ __launch_bounds__(kThreads) void rec_bwd_few_kernel(RecBwdArgs p, RecLayout L, int t_first, int t_last, int ks_wave) {
+    constexpr int PK = 16 / RB, NP = KS / PK, NCH = NP / CH, PLD = 32 + kPartPad;
+    static_assert(KS % PK == 0 && NP % CH == 0, "whole packs, whole chunks");
+    __shared__ __attribute__((aligned(16))) float part_all[2][4][16][PLD];
+    __shared__ float red[kThreads][4];
     __shared__ int lds_abort;
     __shared__ int lds_role[2];
-    __shared__ floatx2 swap[2][2][kWave];   // [step parity][receiving wave]
-    __shared__ float red[2 * kWave][8];
     if (threadIdx.x == 0) lds_abort = 0;
     __syncthreads();
     const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
@@ -2942,152 +2960,177 @@ __global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, R
     }
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int hs = role.hs, g = role.g;
-    const int nks = p.Hp / 8;
+    const int hs = __builtin_amdgcn_readfirstlane(role.hs), g = __builtin_amdgcn_readfirstlane(role.g);
     const Poll poll{L.persistent != 0, p.spin_limit, p.spin_ticks, p.status, (lds_int_t*)&lds_abort};
     const float S = p.dy_scale;
     WideClock clk{(hs == 0 && g == 0) ? p.prof : nullptr};
 
-    half8 wreg[KS];
+    half8 wreg[KS][2];
     {
-        const int real = nks / 2;   // k-steps per wave in the packed weights
-        const half8* wf = p.wfrag + (size_t(hs) * 2 + wave) * size_t(real) * kWave;
+        const half8* wf = p.wfrag + (size_t(hs) * 4 + wave) * size_t(ks_wave) * 2 * kWave;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) wreg[k] = (k < real) ? wf[k * kWave + lane] : half8{};
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) wreg[k][n] = (k < ks_wave) ? wf[(k * 2 + n) * kWave + lane] : half8{};
+        if constexpr (KS <= 12) {   // (256 units 0.95 -> 0.91 us a step; 1024 units and 8 rows a block 1.72 -> 1.79, 650 units 1.36 -> 1.42)
+            loads_landed();
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) keep_aside(wreg[k][n]);
+        }
     }
     const size_t gld = size_t(4) * p.Hp;
-    const int r = lane % 16, j = hs * 16 + 4 * (lane / 16) + 2 * wave;   // this lane's cells: row r, units j and j + 1
-    const int b0 = g * 16;
-    const bool live = b0 + r < p.B;
-    const unsigned row = unsigned(min(r, p.B - 1 - b0)), cell = row * unsigned(p.Hp) + unsigned(j);
-    const unsigned off_ring = unsigned(xch_offset(r, 4 * j, nks));
-    const size_t tile_halfs = size_t(nks) * 512;
-    // wave w takes k-steps 2k + w; (a kernel serves contractions up to two k-steps per wave shorter than its own)
-    unsigned lane_off[KS / 2], tail_off[3];
+    // this lane's cell: unit 8 wave + 2 chunk + half of the slice (one 8-byte group of the ring; with RB = 4 lanes 32 .. 63 have none)
+    const int half = lane & 1, r = (lane >> 1) % RB, chunk = (lane / (2 * RB)) & 3;
+    const bool cell_lane = RB == 8 || lane < 32;
+    const int unit = 8 * wave + 2 * chunk + half;
+    const int b0 = g * RB;
+    const bool live = cell_lane && b0 + r < p.B;
+    const unsigned row = unsigned(min(r, p.B - 1 - b0)), cell = row * unsigned(p.Hp) + unsigned(hs * 32 + unit);
+    const int packs = (ks_wave + PK - 1) / PK;   // of one wave, at most NP
+    const size_t tile_halfs = size_t(packs) * 4 * 512;
+    const unsigned off_ring = few_offset<RB>(hs, wave, r, chunk, half);
+    if (hs == L.nh - 1 && cell_lane) {
+        for (int i = ks_wave; i < packs * PK; ++i)
+            for (int slot = 0; slot < 4; ++slot)
+                store_xch(p.X + size_t(slot) * p.x_slot + size_t(g) * tile_halfs + few_offset<RB>(i, wave, r, chunk, half), Pack<4>{uintx2{0u, 0u}}, false);
+    }
+    unsigned lane_off[NP];   // (a kernel serves shorter contractions than its own: packs past the last one fetch that again and meet zero weights)
 #pragma unroll
-    for (int q = 0; q < KS / 2; ++q) lane_off[q] = unsigned(lane) * 16u + unsigned(wave) * 1024u + unsigned(q) * 4096u;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) tail_off[q] = unsigned(lane) * 16u + unsigned(min(2 * (KS - 3 + q) + wave, nks - 1)) * 1024u;
+    for (int q = 0; q < NP; ++q) lane_off[q] = unsigned(lane) * 16u + unsigned(wave) * 1024u + unsigned(min(q, packs - 1)) * 4096u;
 
-    uintx4 gates[2];          // by parity of the steps done
-    floatx2 cprev[2], ccur[2];   // c_{t-1}, c_t
-    unsigned dy2[2];
-    auto request_ops = [&](int t, auto parity) __attribute__((always_inline)) {   // four loads; the closing pass fetches step 0
+    uintx2 gates[2];       // by parity of the steps done
+    unsigned cprev[2];     // c_{t-1}; c_t is the last step's
+    unsigned dy1[2];
+    auto request_ops = [&](int t, auto parity) __attribute__((always_inline)) {   // three loads; the closing pass fetches step 0
         constexpr int par = decltype(parity)::value;
         const size_t row0 = size_t(max(t, 0)) * p.B + b0;
-        ld_stream_at(gates[par], p.G + row0 * gld, cell * 8u);
-        ld_stream_at(cprev[par], p.C + row0 * p.Hp, cell * 4u);
-        ld_stream_at(ccur[par], p.C + (row0 + p.B) * p.Hp, cell * 4u);
-        ld_stream_at(dy2[par], p.dY + row0 * p.Hp, cell * 2u);
+        ld_at(gates[par], p.G + row0 * gld, cell * 8u);
+        ld_at(cprev[par], p.C + row0 * p.Hp, cell * 4u);
+        ld_half_at(dy1[par], p.dY + row0 * p.Hp, cell * 2u);
     };
-    float dc[2];
-    {
-        const float* src = p.dC + size_t(b0) * p.Hp + cell;
-        dc[0] = src[0];
-        dc[1] = src[1];
-    }
-    float dbacc[4][2] = {};
-    __syncthreads();
-    loads_landed();
-    clk.start();
     auto settle_ops = [&](auto parity) __attribute__((always_inline)) {
         constexpr int par = decltype(parity)::value;
         settle(gates[par]);
         settle(cprev[par]);
-        settle(ccur[par]);
-        settle(dy2[par]);
+        settle(dy1[par]);
     };
-    auto cell_update = [&](int t, const float (&dh)[2], auto parity) __attribute__((always_inline)) {
+    float dc = p.dC[size_t(b0) * p.Hp + cell];
+    float ccur = p.C[(size_t(max(t_first, 0)) * p.B + p.B + b0) * p.Hp + cell];
+    float dbacc[4] = {};
+    __syncthreads();
+    loads_landed();
+    clk.start();
+    auto cell_update = [&](int t, float dh, auto parity) __attribute__((always_inline)) {
         constexpr int par = decltype(parity)::value;
         if (t < 0) {   // closing pass: gradient wrt h0; dc0 is the running dc
             if (live) {
-                *reinterpret_cast<floatx2*>(p.dH0 + size_t(b0) * p.Hp + cell) = floatx2{dh[0], dh[1]};
-                *reinterpret_cast<floatx2*>(p.dC + size_t(b0) * p.Hp + cell) = floatx2{dc[0], dc[1]};
+                p.dH0[size_t(b0) * p.Hp + cell] = dh;
+                p.dC[size_t(b0) * p.Hp + cell] = dc;
             }
             return;
         }
         half_t* const xout = p.X + size_t((t + 8) & 3) * p.x_slot + size_t(g) * tile_halfs;    // dG_t for the peers
         half_t* const xnext = p.X + size_t((t + 6) & 3) * p.x_slot + size_t(g) * tile_halfs;   // will take dG_{t-2}
-        // (both waves' products are complete: every peer has delivered dG_{t+1}, i.e. is done reading dG_{t+2})
-        store_xch16(xnext + off_ring, uintx4{kUnwritten, kUnwritten, kUnwritten, kUnwritten}, false);
-        float da[4][2], dy[2];
-        unpack_h2(dy2[par], dy[0], dy[1]);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            float ig, fg, gg, og;
-            unpack_h2(u == 0 ? gates[par].x : gates[par].z, ig, fg);
-            unpack_h2(u == 0 ? gates[par].y : gates[par].w, gg, og);
-            const float dhu = dh[u] + S * dy[u];
-            const float tc = tanhf_dev(ccur[par][u]);
-            const float dov = dhu * tc;
-            const float d = dc[u] + dhu * og * (1.f - tc * tc);
-            da[0][u] = d * gg * ig * (1.f - ig);
-            da[1][u] = d * cprev[par][u] * fg * (1.f - fg);
-            da[2][u] = d * ig * (1.f - gg * gg);
-            da[3][u] = dov * og * (1.f - og);
-            dc[u] = d * fg;
-        }
-        GateRow<2> out = live ? pack_gates<2>(da) : gates_fill<2>(0u);   // batch rows past B travel as zeros
-        store_xch16(xout + off_ring, out.v[0], false);
+        // (all four waves' products are complete: every peer has delivered dG_{t+1}, i.e. is done reading dG_{t+2})
+        if (cell_lane) store_xch(xnext + off_ring, Pack<4>{uintx2{kUnwritten, kUnwritten}}, false);
+        float ig, fg, gg, og, dy, unused;
+        unpack_h2(gates[par].x, ig, fg);
+        unpack_h2(gates[par].y, gg, og);
+        unpack_h2(dy1[par], dy, unused);
+        const float cp = as_float(cprev[par]);
+        const float dhu = dh + S * dy;
+        const float tc = tanhf_dev(ccur);
+        const float dov = dhu * tc;
+        const float d = dc + dhu * og * (1.f - tc * tc);
+        uintx2 out{pack_h2(d * gg * ig * (1.f - ig), d * cp * fg * (1.f - fg)),
+                   pack_h2(d * ig * (1.f - gg * gg), dov * og * (1.f - og))};
+        dc = d * fg;
+        ccur = cp;
+        if (!live) out = uintx2{0u, 0u};   // batch rows past B travel as zeros
+        if (cell_lane) store_xch(xout + off_ring, Pack<4>{out}, false);
         clk.lap(2);
         if (live) {
-            float v[4][2];   // db sums the values the weight-gradient GEMMs will see (fp16-rounded)
-            unpack_gates<2>(out, v);
+            float v[4];   // db sums the values the weight-gradient GEMMs will see (fp16-rounded)
+            unpack_h2(out.x, v[0], v[1]);
+            unpack_h2(out.y, v[2], v[3]);
 #pragma unroll
-            for (int gt = 0; gt < 4; ++gt)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) dbacc[gt][u] += v[gt][u];
-            st_gates<2>(p.dG + (size_t(t) * p.B + b0) * gld + 4u * cell, out);
+            for (int gt = 0; gt < 4; ++gt) dbacc[gt] += v[gt];
+            st_pack(p.dG + (size_t(t) * p.B + b0) * gld + size_t(4u * cell), Pack<4>{out});
         }
         clk.lap(3);
     };
     auto step = [&](int t, auto parity) __attribute__((always_inline)) {
         constexpr int par = decltype(parity)::value;
-        float dh[2];
         const half_t* tile = wave_uniform(p.X + size_t((t + 9) & 3) * p.x_slot + size_t(g) * tile_halfs);   // dG_{t+1}
-        half8 f[KS];
-        auto request = [&]() __attribute__((always_inline)) { request_pair(f, tile, lane_off, tail_off, std::make_integer_sequence<int, KS>{}); };
-        request();
-        if constexpr (!LATE) request_ops(t - 1, std::integral_constant<int, 1 - par>{});
-        wait_set<LATE ? 0 : 4>(f);
-        auto unwritten = [&]() -> bool {
-            unsigned m = 0u;
+        half8 f[NCH][CH];
+        auto request = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-            for (int k = 0; k < KS; ++k) {
-                const uint4 ua = __builtin_bit_cast(uint4, f[k]);
-                m = max(m, max(max(ua.x, ua.y), max(ua.z, ua.w)));
-            }
-            return __any(m == kUnwritten) != 0;
+            for (int q = 0; q < CH; ++q) ld_frag_async_at(f[c][q], lane_off[c * CH + q], tile);
         };
-        if (__builtin_expect(unwritten() && poll.on, 0)) {
-            int spins = 0;
-            long long spin_start = 0;
-            do {
-                if (poll_give_up(poll, spins, spin_start, lane)) break;   // (the workgroup leaves at its barrier)
-                request();
-                wait_set<0>(f);
-            } while (unwritten());
-        }
-        if constexpr (LATE) request_ops(t - 1, std::integral_constant<int, 1 - par>{});
-        floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int k = 0; k < KS; ++k) acc[k % 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[k], f[k], acc[k % 2], 0, 0, 0);
-        const floatx4 sum = acc[0] + acc[1];
+        for (int c = 0; c < NCH; ++c) request(c);
+        floatx4 acc[PK][2];
+#pragma unroll
+        for (int s = 0; s < PK; ++s) acc[s][0] = acc[s][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            wait_chunk(f[c], (NCH - 1 - c) * CH);   // (loads return in order)
+            auto unwritten = [&]() -> bool {
+                unsigned m = 0u;
+#pragma unroll
+                for (int q = 0; q < CH; ++q) {
+                    const uint4 ua = __builtin_bit_cast(uint4, f[c][q]);
+                    m = max(m, max(max(ua.x, ua.y), max(ua.z, ua.w)));
+                }
+                return __any(m == kUnwritten) != 0;
+            };
+            if (__builtin_expect(unwritten() && poll.on, 0)) {
+                int spins = 0;
+                long long spin_start = 0;
+                for (;;) {
+#pragma unroll
+                    for (int later = c; later < NCH; ++later) request(later);   // (what was requested behind this chunk is as stale)
+#pragma unroll
+                    for (int later = c; later < NCH; ++later) wait_chunk(f[later], 0);   // (all: the next turn writes over them)
+                    if (!unwritten()) break;
+                    if (poll_give_up(poll, spins, spin_start, lane)) leave_kernel();   // (a wave that has ended does not count at a barrier; the others leave there)
+                }
+            }
+            if (c == NCH - 1) request_ops(t - 1, std::integral_constant<int, 1 - par>{});
+#pragma unroll
+            for (int q = 0; q < CH; ++q)
+#pragma unroll
+                for (int s = 0; s < PK; ++s)
+#pragma unroll
+                    for (int n = 0; n < 2; ++n)
+                        acc[s][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[(c * CH + q) * PK + s][n], f[c][q], acc[s][n], 0, 0, 0);
+        }
         clk.lap(0);
-        swap[par][1 - wave][lane] = wave ? floatx2{sum.x, sum.y} : floatx2{sum.z, sum.w};
+        float (&part)[4][16][PLD] = part_all[par];   // (all 16 rows are stored, those past RB for nothing: without a branch in between an addition is one instruction)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            floatx4 sum = acc[0][n];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sum[e] += row_ahead<RB>(acc[1][n][e]);
+                if constexpr (PK == 4) sum[e] += row_ahead<2 * RB>(acc[2][n][e]) + row_ahead<3 * RB>(acc[3][n][e]);
+            }
+            *reinterpret_cast<floatx4*>(&part[wave][lane % 16][n * 16 + 4 * (lane / 16)]) = sum;
+        }
         __syncthreads();
         if (lds_abort != 0) leave_kernel();
-        const floatx2 other = swap[par][wave][lane];
-        dh[0] = (wave ? sum.z : sum.x) + other.x;
-        dh[1] = (wave ? sum.w : sum.y) + other.y;
+        float dh = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) dh += part[w][r][unit];
         clk.lap(1);
         settle_ops(parity);
         cell_update(t, dh, parity);
     };
     int t = t_first;
     if (t >= p.T - 1) {   // the last step of the sequence: dh comes from the caller
-        const float* src = p.dHn + size_t(b0) * p.Hp + cell;
-        const float dh[2] = {src[0], src[1]};
+        const float dh = p.dHn[size_t(b0) * p.Hp + cell];
         request_ops(t, std::integral_constant<int, 0>{});
         wait_all_vm();
         settle_ops(std::integral_constant<int, 0>{});
@@ -3103,20 +3146,18 @@ __global__ __launch_bounds__(2 * kWave) void rec_bwd_pair_kernel(RecBwdArgs p, R
     wait_all_vm();
     settle_ops(std::integral_constant<int, 0>{});   // (the last request is used by nobody, but its registers must not be handed on before it has landed)
     settle_ops(std::integral_constant<int, 1>{});
-    if (t_last >= 0 && live) *reinterpret_cast<floatx2*>(p.dC + size_t(b0) * p.Hp + cell) = floatx2{dc[0], dc[1]};   // for the next launch
+    if (t_last >= 0 && live) p.dC[size_t(b0) * p.Hp + cell] = dc;   // for the next launch
     if (p.stamp_end && hs == 0 && g == 0 && tid == 0) *p.stamp_end = wall_clock64();
     clk.flush();
-    // Bias gradient: fold this launch's sums over the 16 rows (fixed order).
+    // Bias gradient: fold this launch's sums over the rows (fixed order).
 #pragma unroll
-    for (int gt = 0; gt < 4; ++gt)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) red[tid][gt * 2 + u] = dbacc[gt][u];
+    for (int gt = 0; gt < 4; ++gt) red[tid][gt] = dbacc[gt];
     __syncthreads();
-    if (tid < 64) {
-        const int unit = tid / 4, gt = tid % 4;   // of the slice: lane group unit / 4, wave (unit % 4) / 2
+    if (tid < 128) {
+        const int u = tid / 4, gt = tid % 4;   // unit u of the slice: wave u / 8, chunk u % 8 / 2, half u % 2
         float sum = 0.f;
-        for (int k = 0; k < 16; ++k) sum += red[((unit % 4) / 2) * kWave + (unit / 4) * 16 + k][gt * 2 + unit % 2];
-        p.db_part[size_t(g) * gld + size_t(4) * (hs * 16 + unit) + gt] += sum;
+        for (int k = 0; k < RB; ++k) sum += red[(u / 8) * kWave + (u % 8 / 2) * (2 * RB) + 2 * k + u % 2][gt];
+        p.db_part[size_t(g) * gld + size_t(4) * (hs * 32 + u) + gt] += sum;
     }
 }
 
@@ -3697,10 +3738,8 @@ constexpr int kWideMost = 4096;   // hidden units whose W_hh the chip can hold (
 
 // Short contractions.  Every wave of rec_fwd_split_kernel fetches the whole operand, so the CU's vector-memory path sets
 // its end: with one or two waves per CU it is the faster kernel up to 512 units (64 rows 1.64 -> 1.34 us per step, 100 rows
-// 1.42), with four up to 256 (200 rows 1.44 -> 1.16; at 288 units equal, at 512 units 1.7 -> 2.3).  rec_bwd_pair_kernel is
-// the faster one up to 384 units (2.13 -> 1.93); at 512 its two waves take as long over the product as the other kernel's
-// four over theirs and its reduction (2.14 -> 2.24).
-constexpr int kFwdSplitMost = 512, kFwdSplitFourMost = 256, kBwdPairMost = 384;
+// 1.42), with four up to 256 (200 rows 1.44 -> 1.16; at 288 units equal, at 512 units 1.7 -> 2.3).
+constexpr int kFwdSplitMost = 512, kFwdSplitFourMost = 256;
 constexpr int kBroadMost = 1536;   // hidden units of which a workgroup can hold the weights of a slice of 32 (384 KiB)
 
 // whether all 16-row blocks of the batch can run side by side
@@ -3747,6 +3786,25 @@ static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_s
         L.ng = L.nrb < cap ? L.nrb : cap;
         L.grid = L.ng * L.nh;
     }
+}
+
+// Rows per block of rec_bwd_few_kernel, 0: not for these sizes.  Blocks of 4 where all of them run side by side, else of 8 (us a step, 8 / 4 rows:
+// 1024 units and 32 rows 1.71 / 1.43, 650 and 20 rows 1.49 / 1.33, 257 and 70 rows 1.11 / 1.06, 64 and 16 rows 0.90 / 0.84); but a batch of
+// at most four rows is one block either way, and up to 512 units the shorter sum over the lanes counts (256 units and one row
+// 0.80 / 0.90, 64 and four 0.74 / 0.79; 640 and four 1.34 / 1.26).
+static int few_rows_bwd(int B, int Hp, int num_cus) {
+    if (Hp > 1024 || num_cus != 256) return 0;
+    const int side_by_side = 8 * (32 / (Hp / 32));
+    if (int(ceil_div(size_t(B), 4)) <= side_by_side && (B > 4 || Hp > 512)) return 4;
+    return int(ceil_div(size_t(B), 8)) <= side_by_side ? 8 : 0;
+}
+
+// (step-wise launches too: the same sums in the same order)
+static void few_blocks(RecLayout& L, int B, int rows) {
+    L.few = rows;
+    L.mt = 1;
+    L.nrb = L.ng = int(ceil_div(size_t(B), size_t(rows)));
+    if (!L.persistent) L.grid = L.ng * L.nh;
 }
 
 RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt, int waves) {
@@ -3799,13 +3857,9 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.nw = 4;
     L.jb = 16 * L.nt;
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
-    // short contractions: two waves and 16 units per workgroup, where every group has one 16-row block (as forward)
-    if (force_mt != 2 && Hp <= kBwdPairMost && num_cus == 256 && can_16_rows(B, Hp / 16, num_cus)) {
-        L.split = 2;
-        L.nt = 1;
-        L.nw = 2;
-        L.jb = 16;
-        finish_layout(L, B, Hp, num_cus, force_stepwise, fits, 1);
+    // few rows (rec_bwd_few_kernel): every group has one block, its slices are those of the one-way kernel, and so are its fragments
+    if (force_mt != 2 && !(two_d >= 2 && Hp == 1024) && few_rows_bwd(B, Hp, num_cus)) {
+        few_blocks(L, B, few_rows_bwd(B, Hp, num_cus));
         return L;
     }
     // 1025 to 1536 units: slices of 32 where the 16-row blocks do not fit side by side with slices of 16.  A step is bound by the
@@ -3874,6 +3928,13 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
         }
     }
     return L;
+}
+
+size_t rec_bwd_slot_halfs(const RecLayout& L, int B, int Hp) {
+    const size_t plain = exchange_slot_halfs(rec_bwd_ring_rows(L, B), 4 * Hp);
+    if (!L.few) return plain;
+    const size_t packs = ceil_div(size_t(Hp / 32), size_t(16 / L.few));
+    return std::max(plain, size_t(L.nrb) * packs * 4 * 512);
 }
 
 bool rec_bwd_two_d_possible(int Hp, int num_cus) {
@@ -4245,20 +4306,23 @@ static hipError_t run_bwd2d(const RecLayout& L, const RecBwdArgs& a, hipStream_t
     return launch_persistent(kernel, L.grid, lds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device);
 }
 
-template <int KS, bool LATE = true>
-static hipError_t run_bwd_pair(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
-    auto kernel = rec_bwd_pair_kernel<KS, LATE>;
-    if (L.nt != 1 || L.nw != 2 || L.jb != 16 || L.mt != 1 || L.nrb > L.ng || a.Hp / 16 > KS || a.Hp / 16 < KS - 2 || (L.persistent && !L.xcd_local))
+template <int KS, int RB, int CH>
+static hipError_t run_bwd_few(const RecLayout& L, const RecBwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
+    auto kernel = rec_bwd_few_kernel<KS, RB, CH>;
+    const int ks_wave = rec_bwd_ks(L, a.Hp);
+    // what the kernel's indexing assumes
+    if ((L.persistent && !L.xcd_local) || !L.resident || L.nt != 2 || L.nw != 4 || L.jb != 32 || L.nrb > L.ng || L.nrb * RB < a.B || ks_wave != L.nh || ks_wave > KS ||
+        L.rot_div != 0 || a.x_slot < rec_bwd_slot_halfs(L, a.B, a.Hp))
         return hipErrorInvalidValue;
     static std::atomic<int> per_cu[kMaxDevices];
     int device = 0;
-    hipError_t e = prepare_kernel(kernel, kWholeCuLds, 2 * kWave, per_cu, &device);
+    hipError_t e = prepare_kernel(kernel, kWholeCuLds, kThreads, per_cu, &device);
     if (e != hipSuccess) return e;
-    if (L.persistent) return launch_persistent(kernel, grid_with_helpers(L, a.beside), kWholeCuLds, stream, a, L, a.t_hi, a.t_lo, 0, per_cu[device].load(), device, 2 * kWave);
+    if (L.persistent) return launch_persistent(kernel, L.grid, kWholeCuLds, stream, a, L, a.t_hi, a.t_lo, ks_wave, per_cu[device].load(), device);
     return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t_hi, a.t_lo, a.t_hi - a.t_lo + 1, stream,
                         [&]() -> hipError_t {
                             for (int t = a.t_hi; t >= a.t_lo; --t) {
-                                hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(2 * kWave), kWholeCuLds, stream, a, L, t, t, 0);
+                                hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(kThreads), kWholeCuLds, stream, a, L, t, t, ks_wave);
                                 hipError_t le = hipGetLastError();
                                 if (le != hipSuccess) return le;
                             }
@@ -4319,20 +4383,24 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
     }
     const bool ds = L.persistent && !L.xcd_local;   // (as in launch_rec_fwd)
     if (!L.resident) return run_bwd<2, 1, false, 0, 2, false>(L, a, stream, graphs);
-    if (L.split) {
-        // When the next step's operands are requested (rec_bwd_pair_kernel): behind the fragments while those of the whole pass, 14 bytes
-        // a cell and step, are still in the XCD's L2.  Behind the fragments / once those are there, us a pass: 32 units and one row 189 / 203
-        // over 200 steps, 762 / 830 over 1000, two rows 720 / 750 over 900, 1373 / 1211 over 1500, three 347 / 359 over 400, 983 / 824 over 1000, four 196 / 204
-        // over 200, 571 / 507 over 600; 64 units and one row 191 / 208 over 200, 742 / 685 over 800, two rows 232 / 254 over 256; four 226 / 207 over 200.
-        if (a.Hp <= 64 && a.B * a.Hp <= 128 && (long long)a.T * a.B * a.Hp <= 32768) return run_bwd_pair<4, false>(L, a, stream, graphs);
-        switch ((a.Hp / 16 + 3) / 4) {
-#define FLSTM_PAIR_CASE(n) case n: return run_bwd_pair<4 * n>(L, a, stream, graphs);
-            FLSTM_PAIR_CASE(1) FLSTM_PAIR_CASE(2) FLSTM_PAIR_CASE(3) FLSTM_PAIR_CASE(4) FLSTM_PAIR_CASE(5) FLSTM_PAIR_CASE(6)
-#undef FLSTM_PAIR_CASE
-        }
-        return hipErrorInvalidValue;
-    }
     const int ks = rec_bwd_ks(L, a.Hp);
+    if (L.few) {
+        if (L.few == 8) {
+            if (ks <= 4) return run_bwd_few<4, 8, 2>(L, a, stream, graphs);
+            if (ks <= 8) return run_bwd_few<8, 8, 4>(L, a, stream, graphs);
+            if (ks <= 12) return run_bwd_few<12, 8, 3>(L, a, stream, graphs);
+            if (ks <= 16) return run_bwd_few<16, 8, 4>(L, a, stream, graphs);
+            if (ks <= 24) return run_bwd_few<24, 8, 4>(L, a, stream, graphs);
+            return ks <= 32 ? run_bwd_few<32, 8, 4>(L, a, stream, graphs) : hipErrorInvalidValue;
+        }
+        if (L.few != 4) return hipErrorInvalidValue;
+        if (ks <= 4) return run_bwd_few<4, 4, 1>(L, a, stream, graphs);
+        if (ks <= 8) return run_bwd_few<8, 4, 2>(L, a, stream, graphs);
+        if (ks <= 12) return run_bwd_few<12, 4, 3>(L, a, stream, graphs);
+        if (ks <= 16) return run_bwd_few<16, 4, 4>(L, a, stream, graphs);
+        if (ks <= 24) return run_bwd_few<24, 4, 3>(L, a, stream, graphs);
+        return ks <= 32 ? run_bwd_few<32, 4, 4>(L, a, stream, graphs) : hipErrorInvalidValue;
+    }
     if (L.nt == 2) {
         if (L.mt == 1) {
             if (ks <= 8) return run_bwd_ds<2, 8, 0, 1>(L, a, ds, stream, graphs);

@@ -1,0 +1,76 @@
+"""Recurrences in blocks of few rows, fragments that hold several k-steps of them: against 64-bit arithmetic, the kernels with blocks of 32
+rows, ranges of steps, launches per step, and values that are not finite."""
+import numpy as np
+import pytest
+
+from helpers import make_problem, reference_64, rell2, to_np
+from test_core_gpu import run_core
+
+pytestmark = pytest.mark.gpu
+
+# T, B, H and the groups backward.  Slices that end a pack of two or four and slices that
+# leave 1 to 3 of its k-steps without one; the first and last size of every kernel (4, 8, 12, 16, 24, 32 k-steps a wave); one row, a block that
+# is not full, the last batch of blocks of 4 and the first of 8, of 8 and of another kernel
+SHAPES = [(9, 1, 32, 1), (9, 5, 100, 2), (7, 16, 128, 4), (6, 9, 130, 3), (8, 4, 256, 1), (7, 129, 256, 17),
+          (9, 70, 257, 18), (6, 65, 384, 9), (6, 5, 385, 2), (7, 64, 512, 16), (6, 128, 512, 16), (5, 1, 513, 1),
+          (9, 20, 650, 5), (6, 33, 768, 5), (7, 32, 769, 8), (6, 6, 800, 2), (8, 32, 1024, 8), (5, 33, 1000, 5), (5, 64, 1024, 8)]
+
+
+@pytest.mark.parametrize("T,B,H,backward", SHAPES)
+@pytest.mark.parametrize("half", [True, False])
+def test_few_rows_against_64_bits_and_32_row_blocks(T, B, H, backward, half):
+    from flashlstm_poc_amd import LstmCore
+    p = make_problem(T, B, 24, H, seed=B * 10000 + H)
+    ref = {k: v.cpu().numpy() for k, v in reference_64(p).items()}
+    core = LstmCore(B, 24, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    got, info = run_core(p, core=core, half=half)
+    assert info["fallbacks"] == 0 and core.info("groups_bwd") == backward
+    steps, _ = run_core(p, core=core, half=half, stepwise=True)
+    for name in ("row_tiles_fwd", "row_tiles_bwd"):
+        core.set_option(name, 2)
+    blocks, info = run_core(p, core=core, half=half)
+    assert info["fallbacks"] == 0 and core.info("groups_bwd") == -(-B // 32)
+    # (as between the other layouts a sum's order flips roundings of h and dG; one row over few steps has few of them to average over)
+    for k in ref:
+        worst = 1.05 * max(rell2(blocks[k], ref[k]), rell2(steps[k], ref[k])) + (2e-4 if B * H < 2000 else 0.0)
+        assert rell2(got[k], ref[k]) <= worst, (k, rell2(got[k], ref[k]), worst)
+    for name in ("row_tiles_fwd", "row_tiles_bwd"):
+        core.set_option(name, 0)
+    again, _ = run_core(p, core=core, half=half)
+    for k in got:
+        assert np.array_equal(again[k], got[k]), k
+    core.close()
+
+
+@pytest.mark.parametrize("T,B,H", [(21, 9, 100), (22, 40, 257), (20, 20, 650), (21, 33, 1000), (23, 50, 800)])
+def test_few_rows_in_ranges_of_steps(T, B, H):
+    from test_kernel_variants_gpu import test_wide_layers_in_ranges_of_steps as in_ranges
+    in_ranges(T, B, H)
+
+
+@pytest.mark.parametrize("shape", [(6, 8, 64, 250), (7, 20, 64, 650), (6, 32, 64, 1024)])
+def test_a_row_of_nans_stays_in_its_row(shape):
+    from test_core_gpu import test_a_batch_row_of_nans_stays_in_its_row as stays
+    stays(shape)
+
+
+# a weight beyond fp16: every sum it enters is infinite and its gate saturated, and nothing else changes
+@pytest.mark.parametrize("B,H", [(8, 250), (20, 650), (32, 1024)])
+def test_infinite_weights_give_what_the_other_kernels_give(B, H):
+    from flashlstm_poc_amd import LstmCore
+    p = make_problem(5, B, 24, H, seed=3)
+    p["w_hh"] = p["w_hh"].clone()
+    p["w_hh"][3, 7] = 1e6
+    core = LstmCore(B, 24, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    got, info = run_core(p, core=core)
+    assert info["fallbacks"] == 0
+    for name in ("row_tiles_fwd", "row_tiles_bwd"):
+        core.set_option(name, 2)
+    blocks, _ = run_core(p, core=core)
+    for k in ("y", "hn", "cn", "dx", "dh0", "dc0"):
+        assert np.array_equal(np.isfinite(got[k]), np.isfinite(blocks[k])), k
+        there = np.isfinite(blocks[k])
+        assert rell2(got[k][there], blocks[k][there]) <= 2e-3, k
+    core.close()
