@@ -135,17 +135,19 @@ struct flstm_core_plan {
     int ring_base = 0;
     size_t T_cache = 0;
     bool have_cache = false;
+    bool plain_ring = false;   // a call whose scratch has no room for the ring of RecLayout::few
     // pass in progress (begin / steps / end)
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
              half_t* y_direct = nullptr;   // the recurrence writes the caller's y itself
              bool whole = false;           // one launch (forward_whole)
+             int few = 0;                  // RecLayout::few that the exchange ring is laid out for
              int begin = kStampFwdBegin;   // the stamp that begins the pass
              bool begin_on_device = false;   // ... it and kStampFwdStart are not among the published ones (forward_whole)
              int projection = 0;           // where the x-projection is formed: 0 in front of the recurrence, 1 beside it, 2 inside its launch
              bool behind = false;          // the caller's final states are written by a launch of their own behind the recurrence ...
              bool rows_behind = false; } fw;   // ... and y with them
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
-             int few = 0;   // RecLayout::few that the exchange ring is laid out for
+             int few = 0;   // (as forward)
              BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false;
              bool shared = false; } bw;   // dX and the weight gradients in one launch
     DevBuf tile_words;         // ProjectBeside::ready
@@ -169,7 +171,7 @@ namespace {
 
 void replan(flstm_core_plan* p) {
     p->Lf = plan_rec_fwd(p->d.B, p->d.Hp, p->num_cus, p->opt_stepwise || p->hold_fwd > 0 || p->eff_step_f || p->refused_fwd,
-                         p->opt_mt_f ? p->opt_mt_f : p->eff_mt_f, p->opt_waves_f);
+                         p->plain_ring ? 2 : p->opt_mt_f ? p->opt_mt_f : p->eff_mt_f, p->opt_waves_f);
     p->Lb = plan_rec_bwd(p->d.B, p->d.Hp, p->num_cus, p->opt_stepwise || p->hold_bwd > 0 || p->eff_step_b || p->refused_bwd,
                          p->opt_mt_b ? p->opt_mt_b : p->eff_mt_b,
                          (!p->two_d_explicit && p->eff_two_d >= 0) ? p->eff_two_d : p->opt_two_d);
@@ -444,7 +446,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     FL_TRY(p->wih_t.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
     // Fragments for every kernel that the options can choose for these sizes, whichever the current ones do: options and
     // tuned entries change after the weights are packed.  (The one-way kernels have theirs wherever 32-row blocks can be
-    // asked for; those for short contractions, up to 512 units, add at most 2 MiB a direction.)
+    // asked for; those for short contractions, up to 512 units, add at most 2 MiB, those for few rows, up to 1024, 8 MiB.)
     FragLayout frag[kFragKinds];
     auto want = [&](int kind, const RecLayout& L, int ks, size_t fragments) -> hipError_t {
         FragLayout& f = frag[kind];
@@ -457,7 +459,7 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     const RecLayout bwd = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 2, 0), broad = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 0, 0);
     FL_TRY(want(kFragFwd, fwd, rec_fwd_ks(fwd, d.Hp), rec_fwd_fragments(fwd, d.Hp)));
     frag[kFragFwd].wide = fwd.wide;
-    if (split.split || split.broad) {
+    if (split.split || split.broad || split.few) {
         FL_TRY(want(kFragFwdSplit, split, rec_fwd_ks(split, d.Hp), rec_fwd_fragments(split, d.Hp)));
         frag[kFragFwdSplit].split = split.split;
         if (split.split) FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));   // (here: flstm_core_forward_static allocates nothing)
@@ -519,7 +521,7 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
                   const void* c0, flstm_dtype state_dtype, bool whole_x, hipStream_t s) {
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
-    p->fw.T = T; p->fw.x = x; p->fw.x_dtype = x_dtype; p->fw.open = true; p->fw.whole = false;
+    p->fw.T = T; p->fw.x = x; p->fw.x_dtype = x_dtype; p->fw.open = true; p->fw.whole = false; p->fw.few = p->Lf.few;
     p->fw.begin = kStampFwdBegin;
     p->fw.begin_on_device = false;
     p->beside_f.count = 0;
@@ -527,7 +529,7 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     FL_TRY(p->G.reserve(TB * 4 * d.Hp * sizeof(half_t)));
     FL_TRY(p->Y.reserve((TB + d.B) * d.Hp * sizeof(half_t)));
     FL_TRY(p->C.reserve((TB + d.B) * d.Hp * sizeof(float)));
-    const size_t xslot = exchange_slot_halfs(d.B, d.Hp);
+    const size_t xslot = rec_fwd_slot_halfs(p->Lf, d.B, d.Hp);
     FL_TRY(p->xch_f.reserve(4 * xslot * sizeof(half_t)));
     // One launch: the initial state rows (a null h0 / c0 reads as zeros), the exchange ring -- slot 0 holds h0 (rows past B
     // zero), slots 1 to 3 the 'unwritten' pattern --, the seat and phase counters, and (whole passes) the fp16 operand
@@ -536,7 +538,7 @@ int forward_setup(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
     const int f32 = state_dtype == FLSTM_F32;
     prep.to_half(h0, f32, size_t(d.B), d.H, size_t(d.H), 1.f, p->Y.as<half_t>(), size_t(d.B), size_t(d.Hp));
     prep.to_float(c0, f32, size_t(d.B), d.H, 1.f, p->C.as<float>(), size_t(d.Hp));
-    prep.to_exchange(h0, f32, size_t(d.B), d.H, d.Hp, p->xch_f.as<half_t>());
+    prep.to_exchange(h0, f32, size_t(d.B), d.H, d.Hp, p->xch_f.as<half_t>(), p->Lf.few);
     prep.fill(p->xch_f.as<half_t>() + xslot, 3 * xslot * sizeof(half_t), 0xFFFFFFFFu);
     prep.fill(p->status.as<char>() + kSeatsOffset, kStatusBytes - kSeatsOffset, 0u);
     if (p->opt_profile) prep.fill(p->prof.p, 8 * sizeof(long long), 0u);
@@ -575,8 +577,8 @@ int forward_operand(flstm_core_plan* p, size_t t0, size_t n, bool converted, hip
 // estimated microseconds of both ways.  Where these set the pace a tile of 128 x 128 takes one of them 4.6 us and 0.52 per 64
 // features (1 / 2 / 8 / 16 / 32 slabs 5.1 / 5.7 / 8.8 / 12.8 / 21.2 us, with 16 to 96 of them at work); the recurrence starts a tile
 // later, for which the first ones, with memory to themselves, take 2.5 and 0.65.  In front of it the product takes what
-// gemm_nt_cost says, a launch and a gap.  A step takes 1.65 us (to 768 units), 1.8 (to 1024) or 2.4 for every row block that a
-// workgroup has in it; behind the last tile there are the steps of its 128 rows left.
+// gemm_nt_cost says, a launch and a gap.  A step takes 1.65 us (to 768 units; few rows 1.5), 1.8 (to 1024; few rows 1.7) or 2.4 for every row
+// block that a workgroup has in it; behind the last tile there are the steps of its 128 rows left.
 // Measured, us a forward pass, in front / beside: 512 steps of 64 rows, 1024 features and units 1275 / 990, of 16 rows of 2048
 // 1443 / 1208, of 64 rows of 640 units and 2048 features 1316 / 956; 128 steps of the first 347 / 292, 32 steps 130 / 116; 200 steps of
 // 100 rows of 1536 units and 32 features, two turns a step 1036 / 946; the other side of the line: 256 steps of 200 rows of 512 units,
@@ -590,7 +592,8 @@ bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
     if (helpers < 16 || p->opt_profile || reinterpret_cast<uintptr_t>(A) % 16 != 0) return false;
     const double slabs = d.Ip / 64, tile = slabs * 0.52 + 4.6, first = slabs * 0.65 + 2.5;
     const double rounds = double(ceil_div(ceil_div(n * d.B, 128) * (4 * d.Hp / 128), size_t(helpers)));
-    const double step = (d.Hp <= 768 ? 1.65 : d.Hp <= 1024 ? 1.8 : 2.4) * double(ceil_div(size_t(p->Lf.nrb), size_t(p->Lf.ng)));
+    const double one = d.Hp <= 768 ? (p->Lf.few == 8 ? 1.5 : 1.65) : d.Hp <= 1024 ? (p->Lf.few == 8 ? 1.7 : 1.8) : 2.4;
+    const double step = one * double(ceil_div(size_t(p->Lf.nrb), size_t(p->Lf.ng)));
     const double recurrence = step * double(n), last = step * std::fmin(double(n), 128.0 / d.B);
     const double in_front = recurrence + gemm_nt_cost(int(n * d.B), 4 * d.Hp, d.Ip) + 5.0;
     return std::fmax(recurrence + 1.5 * first + 2.0, 1.05 * rounds * tile + last + 4.0) < in_front;
@@ -643,14 +646,39 @@ void take_beside(BesideCopies& waiting, Args& a) {
     waiting.count = 0;
 }
 
+const half8* forward_fragments(const flstm_core_plan* p) {
+    return p->wfrag[p->Lf.split || p->Lf.broad || p->Lf.few ? kFragFwdSplit : kFragFwd].as<half8>();
+}
+
+// The exchange ring as the steps from t0 on expect it, for a layout that came into force during the pass: h of the last step from its
+// state rows, the other slots 'unwritten'.
+int forward_ring_again(flstm_core_plan* p, size_t t0, hipStream_t s) {
+    const Dims& d = p->d;
+    const size_t xslot = rec_fwd_slot_halfs(p->Lf, d.B, d.Hp);
+    FL_TRY(p->xch_f.reserve(4 * xslot * sizeof(half_t)));
+    OpList ring;
+    for (size_t k = 0; k < 4; ++k) {
+        half_t* const slot = p->xch_f.as<half_t>() + k * xslot;
+        if (k == (t0 & 3)) ring.to_exchange(p->Y.as<half_t>() + t0 * d.B * d.Hp, 0, size_t(d.B), d.Hp, d.Hp, slot, p->Lf.few);
+        else ring.fill(slot, xslot * sizeof(half_t), 0xFFFFFFFFu);
+    }
+    p->fw.few = p->Lf.few;
+    FL_TRY(run_ops(ring, s));
+    return 0;
+}
+
 int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     const Dims& d = p->d;
+    if (p->fw.few != p->Lf.few) {
+        const int changed = forward_ring_again(p, t0, s);
+        if (changed) return changed;
+    }
     RecFwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (padding too: the arguments are the key of a captured graph)
-    a.wfrag = p->wfrag[p->Lf.split || p->Lf.broad ? kFragFwdSplit : kFragFwd].as<half8>();
+    a.wfrag = forward_fragments(p);
     a.Y = p->Y.as<half_t>(); a.G = p->G.as<half_t>(); a.C = p->C.as<float>();
     a.y_out = p->fw.y_direct;
-    a.X = p->xch_f.as<half_t>(); a.x_slot = exchange_slot_halfs(d.B, d.Hp);
+    a.X = p->xch_f.as<half_t>(); a.x_slot = rec_fwd_slot_halfs(p->Lf, d.B, d.Hp);
     a.status = p->status.as<int>();
     a.delay_hint = p->status.as<int>() + 1;
     a.stamps = stamps_of(p) + kStampFwdRec;
@@ -683,6 +711,13 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
             rc = forward_project(p, t0, n, true, false, s);
             if (rc) return rc;
             a.project = ProjectBeside{};
+        }
+        if (p->fw.few != p->Lf.few) {
+            rc = forward_ring_again(p, t0, s);
+            if (rc) return rc;
+            a.wfrag = forward_fragments(p);
+            a.X = p->xch_f.as<half_t>();
+            a.x_slot = rec_fwd_slot_halfs(p->Lf, d.B, d.Hp);
         }
         e = launch_rec_fwd(p->Lf, a, s, nullptr);
     }
@@ -952,14 +987,27 @@ extern "C" int flstm_core_forward_static(flstm_core_plan* p, size_t T, const voi
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     // the same buffers forward_setup() sizes, carved out of the static array instead of allocated
-    const size_t need[5] = {x_in_place(p, x_dtype) ? 0 : TB * d.Ip * sizeof(half_t),
-                            TB * 4 * d.Hp * sizeof(half_t),
-                            (TB + d.B) * d.Hp * sizeof(half_t),
-                            (TB + d.B) * d.Hp * sizeof(float),
-                            4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)};
-    size_t off[5], total = align256(kStatusBytes);   // (the limit counts a status block; the plan's own is used)
-    for (int i = 0; i < 5; ++i) { off[i] = total; total += align256(need[i]); }
-    if (total > kStaticScratchBytes) return FLSTM_E_TOO_LARGE;
+    size_t need[5], off[5], total = 0;
+    auto carve = [&]() {
+        const size_t bytes[5] = {x_in_place(p, x_dtype) ? 0 : TB * d.Ip * sizeof(half_t),
+                                 TB * 4 * d.Hp * sizeof(half_t),
+                                 (TB + d.B) * d.Hp * sizeof(half_t),
+                                 (TB + d.B) * d.Hp * sizeof(float),
+                                 4 * rec_fwd_slot_halfs(p->Lf, d.B, d.Hp) * sizeof(half_t)};
+        total = align256(kStatusBytes);   // (the limit counts a status block; the plan's own is used)
+        for (int i = 0; i < 5; ++i) { need[i] = bytes[i]; off[i] = total; total += align256(need[i]); }
+    };
+    use_tuned(p, T);
+    carve();
+    if (total > kStaticScratchBytes && p->Lf.few) {   // (its ring may be a little larger than the other kernels')
+        p->plain_ring = true;
+        replan(p);
+        carve();
+    }
+    if (total > kStaticScratchBytes) {
+        if (p->plain_ring) { p->plain_ring = false; replan(p); }
+        return FLSTM_E_TOO_LARGE;
+    }
     char* b = static_cast<char*>(base);
     DevBuf* slot[5] = {&p->X16, &p->G, &p->Y, &p->C, &p->xch_f};
     DevBuf saved[5];
@@ -970,6 +1018,7 @@ extern "C" int flstm_core_forward_static(flstm_core_plan* p, size_t T, const voi
     p->static_call = true;
     rc = forward_pass(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, false, s);
     p->static_call = false;
+    if (p->plain_ring) { p->plain_ring = false; replan(p); }
     p->fw.open = false;   // (also when the pass failed: the next call must not find a pass in progress)
     for (int i = 0; i < 5; ++i) *slot[i] = saved[i];
     p->have_cache = had_cache;

@@ -20,9 +20,9 @@ struct FragLayout {   // where a recurrence kernel expects its weight fragments:
     int ks = 0, nt = 0, rot_div = 0, nw = 0, unit_major = 0, wide = 0, kq = 0, split = 0;
     size_t fragments = 0;   // of 64 lanes
 };
-// Forward: the one-way kernels' and those of the kernel for short contractions, or with slices of 32 units (RecLayout::broad);
-// backward the one-way kernels' (which that for few rows uses as well), with slices of 32 units, and those of the recurrence that splits its
-// product two ways.
+// Forward: the one-way kernels' and those of the kernel for short contractions, for few rows, or with slices of 32 units
+// (RecLayout::split, few, broad); backward the one-way kernels' (which those for few rows use as well), with slices of 32 units, and those of
+// the recurrence that splits its product two ways.
 enum Frag : int { kFragFwd, kFragFwdSplit, kFragBwd, kFragBwdBroad, kFragBwdTwoD, kFragKinds };
 // W_ih twice (as it is for the projection, transposed for dX) and W_hh as every kind of fragments asked for; one launch.
 hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p /*[4Hp][Ip]*/,
@@ -62,7 +62,7 @@ struct LayoutOp {
     int cols = 0;
     unsigned word = 0;                      // kFill
     float scale = 1.f;
-    int splits = 0, H = 0, accumulate = 0;  // kReduceDw, kReduceDb
+    int splits = 0, H = 0, accumulate = 0;  // kReduceDw, kReduceDb (kToExchange: splits = rows a block, RecLayout::few)
     size_t per = 0;
     unsigned first_block = 0, blocks = 0;   // set by run_ops
 };
@@ -99,8 +99,8 @@ struct OpList {
     void unpad(const void* in, int in_f32, size_t ld_in, size_t rows, int cols, float scale, void* out, int out_f32,
                size_t rows_per_block = 0, size_t block_stride = 0);
     // rows x cols (pitch cols; null reads as zeros) -> a whole slot of an exchange ring (fragment-major, rows padded to 32, kcols
-    // columns), zero elsewhere
-    void to_exchange(const void* in, int in_f32, size_t rows, int cols, int kcols, half_t* slot);
+    // columns), zero elsewhere.  few: the ring of rec_fwd_few_kernel, blocks of that many rows (RecLayout::few)
+    void to_exchange(const void* in, int in_f32, size_t rows, int cols, int kcols, half_t* slot, int few = 0);
     // Sums columns [col0, col0 + out_cols) of the split-K partials [splits][4Hp][ld] (packed gate rows) into dst
     // [4H][out_cols] (PyTorch row order), times `scale`; `accumulate` adds to dst instead of overwriting it (the beta=1
     // accumulation over chunks of flashlstm_v2/src/lstm_backward.cu:1112-1142).  A null dst adds nothing.

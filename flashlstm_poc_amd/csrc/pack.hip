@@ -245,12 +245,14 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
         } else if (o.kind == LayoutOp::kUnpad) {
             op_unpad(o, first, stride);
         } else if (o.kind == LayoutOp::kToExchange) {
-            // item i = eight halfs of one lane: [16-row tile][32-wide k-step][lane] (recurrent.hip, xch_offset)
-            const unsigned nks = unsigned(o.ld_out) / 32;
+            // item i = eight halfs of one lane: [16-row tile][32-wide k-step][lane] (recurrent.hip, xch_offset); with `splits` rows a block
+            // and pack = 16 / rows: [block][pack of k-steps 4 (pack P + s) + w at 4 P + w][lane], rows * s .. k-step s (rec_fwd_few_kernel)
+            const unsigned rb = o.splits ? unsigned(o.splits) : 16u, pack = 16u / rb, nks = unsigned(o.ld_out) / 32;
+            const unsigned per_tile = o.splits ? (nks + 4 * pack - 1) / (4 * pack) * 4 : nks;
             for (size_t i = first; i < o.n; i += stride) {
-                const unsigned lane = unsigned(i) % 64, ks = (unsigned(i) / 64) % nks, tile = unsigned(i) / 64 / nks;
-                const size_t r = size_t(tile) * 16 + lane % 16;
-                const unsigned k = ks * 32 + (lane / 16) * 8;
+                const unsigned lane = unsigned(i) % 64, at = (unsigned(i) / 64) % per_tile, tile = unsigned(i) / 64 / per_tile;
+                const size_t r = size_t(tile) * rb + lane % rb;
+                const unsigned k = (4 * (at / 4 * pack + lane % 16 / rb) + at % 4) * 32 + (lane / 16) * 8;
                 half8 h{};
                 if (o.src != nullptr && r < o.rows) {
 #pragma unroll
@@ -369,10 +371,11 @@ void OpList::unpad(const void* in, int in_f32, size_t ld_in, size_t rows, int co
     o.rows_per_block = rows_per_block; o.block_stride = block_stride;
 }
 
-void OpList::to_exchange(const void* in, int in_f32, size_t rows, int cols, int kcols, half_t* slot) {
+void OpList::to_exchange(const void* in, int in_f32, size_t rows, int cols, int kcols, half_t* slot, int few) {
     LayoutOp& o = op[count++];
     o.kind = LayoutOp::kToExchange; o.in_f32 = in_f32; o.dst = slot; o.src = in;
-    o.n = exchange_slot_halfs(int(rows), kcols) / 8;
+    o.splits = few;
+    o.n = few ? ceil_div(rows, size_t(few)) * ceil_div(size_t(kcols) / 32, size_t(4 * 16 / few)) * 4 * kWave : exchange_slot_halfs(int(rows), kcols) / 8;
     o.rows = rows; o.cols = cols; o.ld_out = size_t(kcols);
 }
 

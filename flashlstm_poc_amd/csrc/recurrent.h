@@ -31,7 +31,7 @@ struct RecLayout {
     int unit_major;  // forward: gate columns of a slice are packed 4 * unit + gate (kernels with one cell per thread), else gate
                      // blocks of jb units
     int split;       // forward, the kernel for short contractions (rec_fwd_split_kernel): waves per workgroup
-    int few;         // backward: 0, or rows per block (4 or 8) of rec_bwd_few_kernel; nrb counts those blocks
+    int few;         // 0, or rows per block of rec_fwd_few_kernel (8 or 16) / rec_bwd_few_kernel (4 or 8); nrb counts those blocks
     int broad;       // 1025 to 1536 units: slices of 32 units instead of 16, 16-row blocks (any number of them)
     int wide;        // more than 2048 hidden units, weights resident (rec_fwd_wide_kernel, rec_bwd_wide_kernel)
     int num_cus;     // of the device the layout was made for
@@ -245,7 +245,8 @@ unsigned rec_bwd_part_fill(const RecLayout& L, int slot, int T);
 // Batch rows the rings of a backward layout are sized for (whole windows where the batch is walked in windows).
 int rec_bwd_ring_rows(const RecLayout& L, int B);
 
-// Halfs in one slot of the dG ring of a backward layout.
+// Halfs in one slot of the ring of a forward layout, and of the dG ring of a backward one.
+size_t rec_fwd_slot_halfs(const RecLayout& L, int B, int Hp);
 size_t rec_bwd_slot_halfs(const RecLayout& L, int B, int Hp);
 
 // Halfs in one slot of an exchange ring for a [rows][cols] operand (rows padded to 32).

@@ -35,7 +35,7 @@
 //    memory) serve shapes whose weights do not fit on chip (more than 4096 hidden units), and are the
 //    safe path after a failed persistent launch.
 //  * The layout above is that of the one-way kernels.  Up to 512 units the waves of a forward workgroup split the columns
-//    instead (rec_fwd_split_kernel); rec_bwd_few_kernel takes blocks of fewer rows up to 1024 units;
+//    instead (rec_fwd_split_kernel); rec_fwd_few_kernel and rec_bwd_few_kernel take blocks of fewer rows up to 1024 units;
 //    rec_fwd_il_kernel has eight waves and two chains; rec_bwd2d_kernel splits the product two ways at 2048 units; above that rec_fwd_wide_kernel and
 //    rec_bwd_wide_kernel hold half a megabyte of weights per workgroup.  Each says why where it stands.
 #include <algorithm>
@@ -820,6 +820,9 @@ __device__ __forceinline__ void ld_stream(uintx4& d, const void* p) {
 // (past the L2's copies as well: rows that another CU may have written during this launch, see project_beside)
 __device__ __forceinline__ void ld_stream_fresh(uintx4& d, const void* p) {
     asm volatile("global_load_dwordx4 %0, %1, off sc1 nt" : "=v"(d) : "v"(p) : "memory");
+}
+__device__ __forceinline__ void ld_stream_fresh(uintx2& d, const void* p) {
+    asm volatile("global_load_dwordx2 %0, %1, off sc1 nt" : "=v"(d) : "v"(p) : "memory");
 }
 __device__ __forceinline__ void ld_stream(floatx4& d, const void* p) {
     asm volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(d) : "v"(p) : "memory");
@@ -1697,6 +1700,19 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
     clk.flush();
 }
 
+// ------------------------------------------------------------------------------- forward, few rows per group
+// 513 to 1024 units where blocks of RB = 8 rows leave half of the workgroups without a seat, and where blocks of RB = 16 take most of them
+// (few_rows_fwd).  The waves of a slice split the contraction as in rec_fwd_kernel.  What is shorter here:
+//  * a fragment holds PK = 16 / RB k-steps of RB rows each (as in rec_bwd_few_kernel), so that a group of 8 rows fetches half;
+//  * all fragments of a step are requested at once; the x-projection of step t + 1 is requested once they are there, a step ahead;
+//  * columns are packed 4 * unit + gate, so a cell's four sums of a wave are 16 bytes of LDS, and with 8 rows a lane has one cell.
+//   ring (halfs): block g, pack P of wave w's k-steps k = 4 (PK*P + s) + w, row r, column q = 32 k + q%32:
+//   g * tile_halfs + (4 P + w) * 512 + (r + RB*s + 16 * (q%32 / 8)) * 8 + q%8
+// Measured, us a step, rec_fwd_kernel -> here: 1024 units and 32 rows 1.77 -> 1.70 (over 2048 steps, where the other kernel's clock falls,
+// 2.03 -> 1.70), 4 rows 1.66 -> 1.57, 650 and 20 rows 1.61 -> 1.50, 1024 and 80 rows 2.00 -> 1.86, 128 rows 2.23 -> 2.05.  What is left
+// at 1024 units: the trip through the L2 (0.8 us), 64 MFMAs a wave (0.45), partial sums and the cells' five exponentials.
+// K-steps past the contraction are written as zeros once per launch (step-wise by every launch; the first reads none).  The rows of the x-projection that are formed beside (project_beside)
+// are waited for a step ahead as well.
 // the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
 __device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
 __device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
@@ -1707,6 +1723,193 @@ template <int N>
 __device__ __forceinline__ float row_ahead(float v) {
     return as_float(unsigned(__builtin_amdgcn_update_dpp(0, int(as_bits(v)), 0x100 | N, 0xF, 0xF, true)));
 }
+template <int KS, int RB>
+__global__ __launch_bounds__(kThreads) void rec_fwd_few_kernel(RecFwdArgs p, RecLayout L, int t_begin, int t_end, int ks_wave) {
+    constexpr int PK = 16 / RB, NP = (KS + PK - 1) / PK, UPT = RB / 8, PLD = 128 + (RB == 8 ? 28 : 4);   // (pitch: 16 rows', and 16 lanes' cells', 16 bytes lie in different banks)
+    static_assert((RB == 8 || RB == 16) && KS % PK == 0, "whole packs");
+    constexpr int CH = NP % 4 == 0 ? 4 : NP % 3 == 0 ? 3 : 2, NCH = NP / CH;
+    static_assert(NP % CH == 0, "whole chunks");
+    extern __shared__ __attribute__((aligned(16))) float part_all[];   // [2][4][16][PLD], and project_beside's
+    __shared__ int lds_abort;
+    __shared__ int lds_role[2];
+    if (threadIdx.x == 0) lds_abort = 0;
+    __syncthreads();
+    const Role role = make_role(L.nh, L.ng, L.gpx, L.xcd_local, p.seats, p.status, lds_role);
+    if (!role.active) {
+        copy_beside(p.beside, lds_role);
+        project_beside(p.project, reinterpret_cast<char*>(part_all), lds_role);
+        return;
+    }
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int hs = __builtin_amdgcn_readfirstlane(role.hs), g = __builtin_amdgcn_readfirstlane(role.g);
+    const int nks = p.Hp / 32, packs = (ks_wave + PK - 1) / PK;   // packs of one wave
+    const Poll poll{L.persistent != 0, p.spin_limit, p.spin_ticks, p.status, (lds_int_t*)&lds_abort};
+    WideClock clk{(hs == 0 && g == 0) ? p.prof : nullptr};
+
+    half8 wreg[KS][8];
+    {
+        const half8* wf = p.wfrag + (size_t(hs) * 4 + wave) * size_t(ks_wave) * 8 * kWave;
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int n = 0; n < 8; ++n) wreg[k][n] = (k < ks_wave) ? wf[(k * 8 + n) * kWave + lane] : half8{};
+        loads_landed();
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int n = 0; n < 8; ++n) keep_aside(wreg[k][n]);
+    }
+    // this lane's cells: row r, units 8 wave + 2 (lane / 16) + half (RB = 16: both)
+    const int half = RB == 8 ? lane & 1 : 0, r = RB == 8 ? (lane >> 1) % 8 : lane % 16;
+    const int u = 8 * wave + 2 * (lane / 16) + half, j = hs * 32 + u;
+    const int b0 = g * RB;
+    const bool live = b0 + r < p.B, word_lane = half == 0;
+    const unsigned row = unsigned(min(r, p.B - 1 - b0)), cell = row * unsigned(p.Hp) + unsigned(j);
+    auto ring_offset = [&](int k) { return unsigned((k / (4 * PK) * 4 + k % 4) * 512 + ((r + RB * (k / 4 % PK)) + 16 * wave) * 8 + 2 * (lane / 16)); };
+    const unsigned off_ring = ring_offset(hs);
+    const size_t tile_halfs = size_t(packs) * 4 * 512;
+    if (hs == L.nh - 1 && word_lane) {   // k-steps past the contraction
+        for (int k = nks; k < packs * PK * 4; ++k)
+            for (int slot = 0; slot < 4; ++slot)
+                store_xch(p.X + size_t(slot) * p.x_slot + size_t(g) * tile_halfs + ring_offset(k), Pack<2>{0u}, false);
+    }
+    unsigned lane_off[NP];   // (packs past the last one fetch that again and meet zero weights)
+#pragma unroll
+    for (int q = 0; q < NP; ++q) lane_off[q] = unsigned(lane) * 16u + unsigned(wave) * 1024u + unsigned(min(q, packs - 1)) * 4096u;
+    float c[UPT];
+#pragma unroll
+    for (int v = 0; v < UPT; ++v) c[v] = p.C[(size_t(t_begin) * p.B + b0) * p.Hp + cell + v];
+    typedef std::conditional_t<UPT == 1, uintx2, uintx4> gates_t;
+    gates_t xp[2];   // by parity of the step
+    ProjectedRows projected(p.project);
+    auto request_xp = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        projected.wait_for((t - p.t0 + 1) * p.B, p.project, hs * 128, poll, lane);
+        ld_stream_fresh(xp[par], p.G + (size_t(t) * p.B + b0) * (size_t(4) * p.Hp) + size_t(4u * cell));
+    };
+    if (p.stamps && t_begin == p.t0 && hs == 0 && g == 0 && tid == 0) p.stamps[0] = wall_clock64();
+    __syncthreads();
+    loads_landed();
+    clk.start();
+    request_xp(t_begin, std::integral_constant<int, 0>{});
+
+    auto step = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int par = decltype(parity)::value;
+        const half_t* tile = wave_uniform(p.X + size_t(t & 3) * p.x_slot + size_t(g) * tile_halfs);
+        half8 f[NCH][CH];
+        auto request = [&](int ch) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < CH; ++q) ld_frag_async_at(f[ch][q], lane_off[ch * CH + q], tile);
+        };
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) request(ch);
+        floatx4 acc[PK][8];
+#pragma unroll
+        for (int s = 0; s < PK; ++s)
+#pragma unroll
+            for (int n = 0; n < 8; ++n) acc[s][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch) {
+            wait_chunk(f[ch], (NCH - 1 - ch) * CH);   // (loads return in order)
+            auto unwritten = [&]() -> bool {
+                unsigned m = 0u;
+#pragma unroll
+                for (int q = 0; q < CH; ++q) {
+                    const uint4 ua = __builtin_bit_cast(uint4, f[ch][q]);
+                    m = max(m, max(max(ua.x, ua.y), max(ua.z, ua.w)));
+                }
+                return __any(m == kUnwritten) != 0;
+            };
+            if (__builtin_expect(unwritten() && poll.on, 0)) {
+                int spins = 0;
+                long long spin_start = 0;
+                for (;;) {
+#pragma unroll
+                    for (int later = ch; later < NCH; ++later) request(later);   // (what was requested behind this chunk is as stale)
+#pragma unroll
+                    for (int later = ch; later < NCH; ++later) wait_chunk(f[later], 0);   // (all: the next turn writes over them)
+                    if (!unwritten()) break;
+                    if (poll_give_up(poll, spins, spin_start, lane)) leave_kernel();   // (a wave that has ended does not count at a barrier; the others leave there)
+                }
+            }
+            if (ch == NCH - 1) request_xp(t + 1 < t_end ? t + 1 : t, std::integral_constant<int, 1 - par>{});
+#pragma unroll
+            for (int q = 0; q < CH; ++q)
+#pragma unroll
+                for (int s = 0; s < PK; ++s)
+#pragma unroll
+                    for (int n = 0; n < 8; ++n)
+                        acc[s][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[(ch * CH + q) * PK + s][n], f[ch][q], acc[s][n], 0, 0, 0);
+        }
+        clk.lap(0);
+        // (all 16 rows of a tile are stored, those past RB for nothing: without a branch in between an addition is one instruction)
+        float* const part = part_all + size_t(par) * 4 * 16 * PLD;
+        float* const mine = part + (size_t(wave) * 16 + size_t(lane % 16)) * PLD + 4 * (lane / 16);
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            floatx4 sum = acc[0][n];
+            if constexpr (PK == 2) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] += row_ahead<8>(acc[PK - 1][n][e]);
+            }
+            *reinterpret_cast<floatx4*>(mine + n * 16) = sum;
+        }
+        __syncthreads();
+        if (lds_abort != 0) leave_kernel();
+        clk.lap(1);
+        settle(xp[par]);
+        half_t* const xout = p.X + size_t((t + 1) & 3) * p.x_slot + size_t(g) * tile_halfs;
+        half_t* const xnext = p.X + size_t((t + 3) & 3) * p.x_slot + size_t(g) * tile_halfs;
+        // (all four waves' products are complete: every peer has delivered h_{t-1}, i.e. is done reading h_{t-2})
+        if (word_lane) store_xch(xnext + off_ring, Pack<2>{kUnwritten}, false);
+        float h[UPT];
+        gates_t act;
+#pragma unroll
+        for (int v = 0; v < UPT; ++v) {
+            floatx4 sum = *reinterpret_cast<const floatx4*>(part + size_t(r) * PLD + 4 * (u + v));
+#pragma unroll
+            for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const floatx4*>(part + (size_t(w) * 16 + r) * PLD + 4 * (u + v));
+            float z[4];
+            unpack_h2(xp[par][2 * v], z[0], z[1]);
+            unpack_h2(xp[par][2 * v + 1], z[2], z[3]);
+            const float ig = sigmoidf_dev(z[0] + sum[0]), fg = sigmoidf_dev(z[1] + sum[1]), gg = tanhf_dev(z[2] + sum[2]), og = sigmoidf_dev(z[3] + sum[3]);
+            c[v] = fg * c[v] + ig * gg;
+            h[v] = og * tanhf_dev(c[v]);
+            act[2 * v] = pack_h2(ig, fg);
+            act[2 * v + 1] = pack_h2(gg, og);
+        }
+        unsigned h2 = pack_h2(h[0], UPT == 2 ? h[UPT - 1] : as_float(quad_xor1(as_bits(h[0]))));
+        if (!live) h2 = 0u;   // (rows past B travel as zeros)
+        if (word_lane) store_xch(xout + off_ring, Pack<2>{h2}, false);
+        clk.lap(2);
+        // caches for the backward pass: off the critical path
+        if (live) {
+            const size_t row0 = size_t(t) * p.B + b0;
+            float* const to = p.C + (row0 + p.B) * p.Hp + cell;
+            if constexpr (UPT == 1) __builtin_nontemporal_store(c[0], to);
+            else __builtin_nontemporal_store(floatx2{c[0], c[UPT - 1]}, reinterpret_cast<floatx2*>(to));
+            __builtin_nontemporal_store(act, reinterpret_cast<gates_t*>(p.G + row0 * (size_t(4) * p.Hp) + size_t(4u * cell)));
+            if (word_lane) {
+                __builtin_nontemporal_store(h2, reinterpret_cast<unsigned*>(p.Y + (row0 + p.B) * p.Hp + cell));
+                if (p.y_out) __builtin_nontemporal_store(h2, reinterpret_cast<unsigned*>(p.y_out + row0 * p.Hp + cell));
+            }
+        }
+        clk.lap(3);
+    };
+    int t = t_begin;
+    for (; t + 1 < t_end; t += 2) {
+        step(t, std::integral_constant<int, 0>{});
+        step(t + 1, std::integral_constant<int, 1>{});
+    }
+    if (t < t_end) step(t, std::integral_constant<int, 0>{});
+    wait_all_vm();
+    settle(xp[0]);   // (the last request is used by nobody, but its registers must not be handed on before it has landed)
+    settle(xp[1]);
+    if (p.stamps && hs == 0 && g == 0 && tid == 0) p.stamps[1] = wall_clock64();
+    clk.flush();
+}
+
 // ---------------------------------------------------------------- forward, short contractions, a whole pass
 // A pass of rec_fwd_split_kernel is four launches: state rows, ring and counters; projection; recurrence; outputs.  Here it is
 // this launch alone, with one in front of it where x has to be converted, or the projection where rows are long.  Measured, us
@@ -3108,7 +3311,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_few_kernel(RecBwdArgs p, Rec
                         acc[s][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wreg[(c * CH + q) * PK + s][n], f[c][q], acc[s][n], 0, 0, 0);
         }
         clk.lap(0);
-        float (&part)[4][16][PLD] = part_all[par];   // (all 16 rows are stored, those past RB for nothing: without a branch in between an addition is one instruction)
+        float (&part)[4][16][PLD] = part_all[par];   // (rows past RB are stored for nothing, as in rec_fwd_few_kernel)
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
             floatx4 sum = acc[0][n];
@@ -3788,7 +3991,19 @@ static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_s
     }
 }
 
-// Rows per block of rec_bwd_few_kernel, 0: not for these sizes.  Blocks of 4 where all of them run side by side, else of 8 (us a step, 8 / 4 rows:
+// Rows per block of rec_fwd_few_kernel, 0: not for these sizes.  Blocks of 8 as long as half of the workgroups stay without a seat, with
+// which the projection is formed; with more of them seated it stands in front.  Us a call, rec_fwd_kernel / blocks of 8: 512 steps of 32
+// rows of 1024 features and units 951 / 927 (2048 steps 4211 / 3573), 4 rows and 128 features 893 / 848, 20 rows of 650 units 874 /
+// 818, 56 rows of 544 879 / 859; the other side of the line, device time: 48 rows of 1024 features and units 1002 / 1192.  Blocks of 16
+// above 768 units where rec_fwd_kernel seats more than half as well: 80 rows of 1024 1383 / 1301, 128 rows 1692 / 1582; 64 rows 1000 / 1043,
+// 100 rows of 600 units 904 / 908.
+static int few_rows_fwd(int B, int Hp, int num_cus) {
+    const int nh = Hp / 32;
+    if (Hp <= kFwdSplitMost || Hp > 1024 || num_cus != 256) return 0;
+    if (int(ceil_div(size_t(B), 8)) * nh <= num_cus / 2) return 8;
+    return Hp > 768 && B > 64 && B <= 128 ? 16 : 0;
+}
+// Rows per block of rec_bwd_few_kernel, likewise.  Blocks of 4 where all of them run side by side, else of 8 (us a step, 8 / 4 rows:
 // 1024 units and 32 rows 1.71 / 1.43, 650 and 20 rows 1.49 / 1.33, 257 and 70 rows 1.11 / 1.06, 64 and 16 rows 0.90 / 0.84); but a batch of
 // at most four rows is one block either way, and up to 512 units the shorter sum over the lanes counts (256 units and one row
 // 0.80 / 0.90, 64 and four 0.74 / 0.79; 640 and four 1.34 / 1.26).
@@ -3843,6 +4058,11 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
             finish_layout(L, B, Hp, num_cus, force_stepwise, fits, 1);
             break;
         }
+    }
+    // few rows (rec_fwd_few_kernel), likewise
+    if (L.nw == 4 && waves != 4 && force_mt != 2 && few_rows_fwd(B, Hp, num_cus)) {
+        L.unit_major = 1;
+        few_blocks(L, B, few_rows_fwd(B, Hp, num_cus));
     }
     return L;
 }
@@ -3930,6 +4150,11 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     return L;
 }
 
+size_t rec_fwd_slot_halfs(const RecLayout& L, int B, int Hp) {
+    const size_t plain = exchange_slot_halfs(B, Hp);
+    if (!L.few) return plain;
+    return std::max(plain, size_t(L.nrb) * ceil_div(size_t(Hp / 32), size_t(4 * 16 / L.few)) * 4 * 512);
+}
 size_t rec_bwd_slot_halfs(const RecLayout& L, int B, int Hp) {
     const size_t plain = exchange_slot_halfs(rec_bwd_ring_rows(L, B), 4 * Hp);
     if (!L.few) return plain;
@@ -4066,6 +4291,13 @@ int rec_projecting_workgroups(const RecLayout& L) {
     return (L.persistent && L.resident && !L.split && !L.wide && L.nw == 4) ? rec_idle_workgroups(L) : 0;
 }
 
+// what project_beside's indexing assumes
+static bool projection_fits(const RecLayout& L, const RecFwdArgs& a) {
+    const ProjectBeside& w = a.project;
+    return L.persistent && w.M == (a.t1 - a.t0) * a.B && w.N == 4 * a.Hp && w.N % kBesideTile == 0 && w.first[8] == w.N / kBesideTile && w.K > 0 &&
+           w.K % BK == 0 && w.lda >= size_t(w.K) && w.lda < (size_t(1) << 22) && w.lda % 8 == 0 && reinterpret_cast<uintptr_t>(w.A) % 16 == 0;
+}
+
 template <int NT, int KS, bool RES, int MT, bool DS, bool DEEP = false, int KL = 0>
 static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     constexpr int NW = 4;
@@ -4074,9 +4306,7 @@ static hipError_t run_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
     const size_t parts = size_t(2) * NW * fwd_part_rows(MT, KL) * (16 * NT + kPartPad) * sizeof(float) + size_t(NW) * KL * NT * kWave * sizeof(half8);
     const size_t lds = RES && parts < kBesideLds ? kBesideLds : parts;   // (one workgroup per CU either way)
     const ProjectBeside& w = a.project;
-    if (w.M != 0 && (!L.persistent || !RES || w.M != (a.t1 - a.t0) * a.B || w.N != 4 * a.Hp || w.N % kBesideTile != 0 || w.first[8] != w.N / kBesideTile || w.K <= 0 || w.K % BK != 0 ||
-                     w.lda < size_t(w.K) || w.lda >= (size_t(1) << 22) || w.lda % 8 != 0 || reinterpret_cast<uintptr_t>(w.A) % 16 != 0))
-        return hipErrorInvalidValue;
+    if (w.M != 0 && (!RES || !projection_fits(L, a))) return hipErrorInvalidValue;
     static std::atomic<int> per_cu[kMaxDevices];
     int device = 0;
     hipError_t e = prepare_kernel(kernel, lds, NW * kWave, per_cu, &device);
@@ -4213,6 +4443,8 @@ static hipError_t run_fwd_ds(const RecLayout& L, const RecFwdArgs& a, bool ds, h
     return ds ? run_fwd<NT, KS, true, MT, true>(L, a, stream, graphs) : run_fwd<NT, KS, true, MT, false>(L, a, stream, graphs);
 }
 
+static hipError_t launch_fwd_few(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs);
+
 hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
     if (a.T <= 0 || a.B <= 0 || a.t1 <= a.t0) return hipSuccess;
     if (a.Hp % 32 != 0 || a.Hp % L.jb != 0 || a.t0 < 0 || a.t1 > a.T) return hipErrorInvalidValue;
@@ -4234,6 +4466,7 @@ hipError_t launch_rec_fwd(const RecLayout& L, const RecFwdArgs& a, hipStream_t s
         }
         return hipErrorInvalidValue;
     }
+    if (L.few) return launch_fwd_few(L, a, stream, graphs);
     if (L.nw == 8) {   // eight waves: the interleaved kernel, 32-row blocks
         if (ks <= 2) return ds ? run_fwd_il<2, true>(L, a, stream, graphs) : run_fwd_il<2, false>(L, a, stream, graphs);
         return ds ? run_fwd_il<4, true>(L, a, stream, graphs) : run_fwd_il<4, false>(L, a, stream, graphs);
@@ -4416,6 +4649,37 @@ hipError_t launch_rec_bwd(const RecLayout& L, const RecBwdArgs& a, hipStream_t s
         if (L.mt == 1) return ks <= 48 ? run_bwd_ds<1, 48, 12, 1>(L, a, ds, stream, graphs) : run_bwd_ds<1, 64, 24, 1>(L, a, ds, stream, graphs);
         return ks <= 48 ? run_bwd_ds<1, 48, 12, 2>(L, a, ds, stream, graphs) : run_bwd_ds<1, 64, 24, 2>(L, a, ds, stream, graphs);
     }
+    return hipErrorInvalidValue;
+}
+
+template <int KS, int RB>
+static hipError_t run_fwd_few(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
+    auto kernel = rec_fwd_few_kernel<KS, RB>;
+    // what the kernel's indexing assumes
+    const int ks = rec_fwd_ks(L, a.Hp);
+    if ((L.persistent && !L.xcd_local) || !L.resident || L.jb != 32 || L.nw != 4 || L.nt != 8 || !L.unit_major || L.rot_div != 0 || L.nrb > L.ng || L.nrb * RB < a.B || ks > KS ||
+        a.x_slot < rec_fwd_slot_halfs(L, a.B, a.Hp) || (a.project.M != 0 && !projection_fits(L, a)))
+        return hipErrorInvalidValue;
+    static std::atomic<int> per_cu[kMaxDevices];
+    int device = 0;
+    hipError_t e = prepare_kernel(kernel, kBesideLds, kThreads, per_cu, &device);
+    if (e != hipSuccess) return e;
+    if (L.persistent) return launch_persistent(kernel, L.grid, kBesideLds, stream, a, L, a.t0, a.t1, ks, per_cu[device].load(), device);
+    return launch_steps(graphs, reinterpret_cast<const void*>(kernel), &a, sizeof(a), L, a.t0, a.t1, a.t1 - a.t0, stream,
+                        [&]() -> hipError_t {
+                            for (int t = a.t0; t < a.t1; ++t) {
+                                hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(kThreads), kBesideLds, stream, a, L, t, t + 1, ks);
+                                hipError_t le = hipGetLastError();
+                                if (le != hipSuccess) return le;
+                            }
+                            return hipSuccess;
+                        });
+}
+
+static hipError_t launch_fwd_few(const RecLayout& L, const RecFwdArgs& a, hipStream_t stream, StepGraphCache* graphs) {
+    const int ks = rec_fwd_ks(L, a.Hp);
+    if (L.few == 8) return ks <= 6 ? run_fwd_few<6, 8>(L, a, stream, graphs) : run_fwd_few<8, 8>(L, a, stream, graphs);
+    if (L.few == 16) return run_fwd_few<8, 16>(L, a, stream, graphs);
     return hipErrorInvalidValue;
 }
 

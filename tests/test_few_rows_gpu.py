@@ -1,5 +1,5 @@
 """Recurrences in blocks of few rows, fragments that hold several k-steps of them: against 64-bit arithmetic, the kernels with blocks of 32
-rows, ranges of steps, launches per step, and values that are not finite."""
+rows, ranges of steps, launches per step, values that are not finite, and a layout that changes during a pass."""
 import numpy as np
 import pytest
 
@@ -8,24 +8,25 @@ from test_core_gpu import run_core
 
 pytestmark = pytest.mark.gpu
 
-# T, B, H and the groups backward.  Slices that end a pack of two or four and slices that
+# T, B, H and the groups backward and forward (None: another kernel forward).  Slices that end a pack of two or four and slices that
 # leave 1 to 3 of its k-steps without one; the first and last size of every kernel (4, 8, 12, 16, 24, 32 k-steps a wave); one row, a block that
-# is not full, the last batch of blocks of 4 and the first of 8, of 8 and of another kernel
-SHAPES = [(9, 1, 32, 1), (9, 5, 100, 2), (7, 16, 128, 4), (6, 9, 130, 3), (8, 4, 256, 1), (7, 129, 256, 17),
-          (9, 70, 257, 18), (6, 65, 384, 9), (6, 5, 385, 2), (7, 64, 512, 16), (6, 128, 512, 16), (5, 1, 513, 1),
-          (9, 20, 650, 5), (6, 33, 768, 5), (7, 32, 769, 8), (6, 6, 800, 2), (8, 32, 1024, 8), (5, 33, 1000, 5), (5, 64, 1024, 8)]
+# is not full, the last batch of blocks of 4 and the first of 8, of 8 and of another kernel; forward the last batch of 8 rows, the first and last of 16
+SHAPES = [(9, 1, 32, 1, None), (9, 5, 100, 2, None), (7, 16, 128, 4, None), (6, 9, 130, 3, None), (8, 4, 256, 1, None), (7, 129, 256, 17, None),
+          (9, 70, 257, 18, None), (6, 65, 384, 9, None), (6, 5, 385, 2, None), (7, 64, 512, 16, None), (6, 128, 512, 16, None), (5, 1, 513, 1, 1),
+          (9, 20, 650, 5, 3), (6, 33, 768, 5, 5), (7, 32, 769, 8, 4), (6, 6, 800, 2, 1), (8, 32, 1024, 8, 4), (5, 33, 1000, 5, None), (5, 64, 1024, 8, None),
+          (6, 65, 769, 5, 5), (6, 128, 1024, 8, 8), (4, 97, 801, 7, 7)]
 
 
-@pytest.mark.parametrize("T,B,H,backward", SHAPES)
+@pytest.mark.parametrize("T,B,H,backward,forward", SHAPES)
 @pytest.mark.parametrize("half", [True, False])
-def test_few_rows_against_64_bits_and_32_row_blocks(T, B, H, backward, half):
+def test_few_rows_against_64_bits_and_32_row_blocks(T, B, H, backward, forward, half):
     from flashlstm_poc_amd import LstmCore
     p = make_problem(T, B, 24, H, seed=B * 10000 + H)
     ref = {k: v.cpu().numpy() for k, v in reference_64(p).items()}
     core = LstmCore(B, 24, H)
     core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
     got, info = run_core(p, core=core, half=half)
-    assert info["fallbacks"] == 0 and core.info("groups_bwd") == backward
+    assert info["fallbacks"] == 0 and core.info("groups_bwd") == backward and (forward is None or core.info("groups_fwd") == forward)
     steps, _ = run_core(p, core=core, half=half, stepwise=True)
     for name in ("row_tiles_fwd", "row_tiles_bwd"):
         core.set_option(name, 2)
@@ -43,20 +44,20 @@ def test_few_rows_against_64_bits_and_32_row_blocks(T, B, H, backward, half):
     core.close()
 
 
-@pytest.mark.parametrize("T,B,H", [(21, 9, 100), (22, 40, 257), (20, 20, 650), (21, 33, 1000), (23, 50, 800)])
+@pytest.mark.parametrize("T,B,H", [(21, 9, 100), (22, 40, 257), (20, 20, 650), (21, 33, 1000), (23, 80, 800)])
 def test_few_rows_in_ranges_of_steps(T, B, H):
     from test_kernel_variants_gpu import test_wide_layers_in_ranges_of_steps as in_ranges
     in_ranges(T, B, H)
 
 
-@pytest.mark.parametrize("shape", [(6, 8, 64, 250), (7, 20, 64, 650), (6, 32, 64, 1024)])
+@pytest.mark.parametrize("shape", [(6, 8, 64, 250), (7, 20, 64, 650), (6, 32, 64, 1024), (6, 100, 64, 1000)])
 def test_a_row_of_nans_stays_in_its_row(shape):
     from test_core_gpu import test_a_batch_row_of_nans_stays_in_its_row as stays
     stays(shape)
 
 
 # a weight beyond fp16: every sum it enters is infinite and its gate saturated, and nothing else changes
-@pytest.mark.parametrize("B,H", [(8, 250), (20, 650), (32, 1024)])
+@pytest.mark.parametrize("B,H", [(8, 250), (20, 650), (32, 1024), (100, 1000)])
 def test_infinite_weights_give_what_the_other_kernels_give(B, H):
     from flashlstm_poc_amd import LstmCore
     p = make_problem(5, B, 24, H, seed=3)
@@ -73,4 +74,41 @@ def test_infinite_weights_give_what_the_other_kernels_give(B, H):
         assert np.array_equal(np.isfinite(got[k]), np.isfinite(blocks[k])), k
         there = np.isfinite(blocks[k])
         assert rell2(got[k][there], blocks[k][there]) <= 2e-3, k
+    core.close()
+
+
+# an option that changes the layout between two ranges of a pass: forward goes on in the other layout's ring, backward asks for the pass again
+@pytest.mark.parametrize("T,B,H", [(11, 20, 650), (9, 32, 1024)])
+@pytest.mark.parametrize("name,value", [("row_tiles_fwd", 2), ("stepwise", 1)])
+def test_layout_that_changes_during_a_pass(T, B, H, name, value):
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    p = make_problem(T, B, 64, H, seed=5)
+    core = LstmCore(B, 64, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    want, _ = run_core(p, core=core)
+    lib, s = core.lib, torch.cuda.current_stream().cuda_stream
+    t16 = {k: p[k].cuda().half() for k in ("x", "dy", "h0", "c0")}
+    hy, cy = (torch.empty(B, H, device="cuda", dtype=torch.float16) for _ in range(2))
+    for first, then in ((0, value), (value, 0)):
+        core.set_option(name, first)
+        assert lib.flstm_core_forward_begin(core._h, T, t16["x"].data_ptr(), 1, t16["h0"].data_ptr(), t16["c0"].data_ptr(), 1, s) == 0
+        assert lib.flstm_core_forward_steps(core._h, 0, 6, s) == 0
+        core.set_option(name, then)
+        assert lib.flstm_core_forward_steps(core._h, 6, T - 6, s) == 0
+        assert lib.flstm_core_forward_end(core._h, hy.data_ptr(), cy.data_ptr(), 1, 1, s) == 0
+        torch.cuda.synchronize()
+        assert core.info("fallbacks") == 0
+        assert rell2(to_np(hy), want["hn"]) <= 1e-3 and rell2(to_np(cy), want["cn"]) <= 1e-3
+    core.set_option(name, 0)
+    core.forward(t16["x"], t16["h0"], t16["c0"])
+    assert lib.flstm_core_backward_begin(core._h, T, t16["dy"].data_ptr(), 1, None, None, 1, 1.0, None, 1, s) == 0
+    assert lib.flstm_core_backward_steps(core._h, T - 1, 3, s) == 0
+    core.set_option("row_tiles_bwd", 2)
+    stalled = lib.flstm_core_backward_steps(core._h, T - 4, T - 3, s)
+    torch.cuda.synchronize()
+    assert stalled != 0 and core.info("fallbacks") == 0
+    core.set_option("row_tiles_bwd", 0)
+    got = core.backward(t16["x"], t16["dy"])
+    assert bool(torch.isfinite(got[0]).all())
     core.close()
