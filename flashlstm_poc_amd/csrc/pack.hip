@@ -271,7 +271,15 @@ __global__ __launch_bounds__(kT) void layout_ops_kernel(OpList list) {
                 const int row = torch_row(int(q), o.H);
                 if (row < 0) continue;
                 float s = 0.f;
-                for (int g = 0; g < o.splits; ++g) s += part[size_t(g) * o.n + q];
+                int g = 0;
+                for (; g + 8 <= o.splits; g += 8) {   // (eight on their way at a time: small layers have up to 256 groups)
+                    float v[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = part[size_t(g + e) * o.n + q];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) s += v[e];
+                }
+                for (; g < o.splits; ++g) s += part[size_t(g) * o.n + q];
                 s *= o.scale;
                 if (db_ih) db_ih[row] = o.accumulate ? db_ih[row] + s : s;
                 if (db_hh && db_hh != db_ih) db_hh[row] = o.accumulate ? db_hh[row] + s : s;
