@@ -48,8 +48,9 @@ int flstm_core_destroy(flstm_core_plan* plan);
  * and db_hh to what the caller's buffers hold instead of overwriting them: a sequence processed as several
  * consecutive segments, last segment first, each segment's dh0 / dc0 fed to the next call as d_hn / d_cn),
  * "row_tiles_fwd" / "row_tiles_bwd" (16-row tiles per row block of that recurrence: 1, 2, or 0 = automatic; 1 only where
- * all 16-row blocks run side by side.  The kernels for short contractions, up to 512 units forward and 384 backward, have
- * 16-row blocks: there 2 chooses the kernel of larger layers, whose sums are in another order.  Above 2048 units batch
+ * all 16-row blocks run side by side.  The kernels for short contractions, up to 512 units forward, have 16-row blocks, those for
+ * few rows, up to 1024 units, blocks of 4 to 16: there 2 chooses the one-way kernel, whose sums are in another order.  An option that
+ * changes the blocks between two flstm_core_backward_steps of a pass makes the next one return FLSTM_E_STALLED.  Above 2048 units batch
  * rows are taken in tiles of 16, one after the other, and the option changes nothing),
  * "cooperative" (0, the default: persistent launches are plain launches whose grid is checked to be co-resident, and
  * launches to different streams of a device are put one behind the other; 1: hipLaunchCooperativeKernel, which costs
