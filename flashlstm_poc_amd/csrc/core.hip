@@ -147,7 +147,7 @@ struct flstm_core_plan {
              bool behind = false;          // the caller's final states are written by a launch of their own behind the recurrence ...
              bool rows_behind = false; } fw;   // ... and y with them
     struct { size_t T = 0; const half_t* dYk = nullptr; const void* dY = nullptr; flstm_dtype dy_dtype = FLSTM_F16;
-             int few = 0;   // (as forward)
+             RecLayout L{};   // of the whole pass: the ring and the groups of the bias gradient are laid out for it, whatever options change meanwhile
              BwdScales k; float dy_scale = 1.f; void* dx = nullptr; flstm_dtype dx_dtype = FLSTM_F16; bool open = false;
              bool shared = false; } bw;   // dX and the weight gradients in one launch
     DevBuf tile_words;         // ProjectBeside::ready
@@ -1036,9 +1036,10 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     const size_t TB = T * size_t(d.B);
     p->bw.T = T; p->bw.dY = dY; p->bw.dy_dtype = dy_dtype; p->bw.k = k; p->bw.dx = dx; p->bw.dx_dtype = dx_dtype;
     p->bw.open = true;
+    const RecLayout& L = p->bw.L = p->Lb;
     p->beside_b.count = 0;
     // (step-wise launches always read a plan-owned copy, so that their captured graph can be replayed)
-    if (dy_dtype == FLSTM_F16 && d.H == d.Hp && p->Lb.persistent) {
+    if (dy_dtype == FLSTM_F16 && d.H == d.Hp && L.persistent) {
         p->bw.dYk = static_cast<const half_t*>(dY);
         p->bw.dy_scale = k.dy;
     } else {
@@ -1051,25 +1052,24 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
     FL_TRY(p->dC.reserve(st_bytes));
     FL_TRY(p->dH0.reserve(st_bytes));
     FL_TRY(p->dG.reserve(TB * 4 * d.Hp * sizeof(half_t)));
-    FL_TRY(p->db_part.reserve(size_t(p->Lb.ng) * 4 * d.Hp * sizeof(float)));
-    const size_t xslot = rec_bwd_slot_halfs(p->Lb, d.B, d.Hp);
-    p->bw.few = p->Lb.few;
-    const size_t dg_slots = size_t(rec_bwd_dg_slots(p->Lb));
+    FL_TRY(p->db_part.reserve(size_t(L.ng) * 4 * d.Hp * sizeof(float)));
+    const size_t xslot = rec_bwd_slot_halfs(L, d.B, d.Hp);
+    const size_t dg_slots = size_t(rec_bwd_dg_slots(L));
     FL_TRY(p->xch_b.reserve(dg_slots * xslot * sizeof(half_t)));
     // One launch (see forward_setup): the dG ring 'unwritten', the ring of partial sums in its starting parities, the
     // scaled state gradients, the bias-gradient partials, the seat counters, the phase counters.
     static_assert(kRecBwdPartSlots + 7 <= kMaxOps, "what an OpList holds");
     OpList prep;
     prep.fill(p->xch_b.p, dg_slots * xslot * sizeof(half_t), 0xFFFFFFFFu);
-    if (p->Lb.two_d) {
-        const size_t pslot = rec_bwd_part_slot_floats(p->Lb) * sizeof(float);
+    if (L.two_d) {
+        const size_t pslot = rec_bwd_part_slot_floats(L) * sizeof(float);
         FL_TRY(p->part_b.reserve(kRecBwdPartSlots * pslot));
         for (int i = 0; i < kRecBwdPartSlots; ++i)
-            prep.fill(static_cast<char*>(p->part_b.p) + size_t(i) * pslot, pslot, rec_bwd_part_fill(p->Lb, i, int(T)));
+            prep.fill(static_cast<char*>(p->part_b.p) + size_t(i) * pslot, pslot, rec_bwd_part_fill(L, i, int(T)));
     }
     prep.to_float(d_hn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, k.state, p->dHn.as<float>(), size_t(d.Hp));
     prep.to_float(d_cn, dstate_dtype == FLSTM_F32, size_t(d.B), d.H, k.state, p->dC.as<float>(), size_t(d.Hp));
-    prep.fill(p->db_part.p, size_t(p->Lb.ng) * 4 * d.Hp * sizeof(float), 0u);
+    prep.fill(p->db_part.p, size_t(L.ng) * 4 * d.Hp * sizeof(float), 0u);
     prep.fill(p->status.as<char>() + kSeatsOffset, kStatusBytes - kSeatsOffset, 0u);
     if (p->opt_profile) prep.fill(p->prof.as<long long>() + 8, 8 * sizeof(long long), 0u);
     if (whole_dy && p->bw.dYk != dY)
@@ -1086,6 +1086,7 @@ int backward_setup(flstm_core_plan* p, size_t T, const void* dY, flstm_dtype dy_
 // when the caller's dY cannot be used in place
 int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hipStream_t s) {
     const Dims& d = p->d;
+    const RecLayout& L = p->bw.L;
     const long lo = t_lo < 0 ? 0 : t_lo;
     if (!converted && p->bw.dYk != p->bw.dY && t_hi >= lo) {
         const size_t esz = p->bw.dy_dtype == FLSTM_F32 ? 4 : 2;
@@ -1098,14 +1099,14 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
     }
     RecBwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (as in forward_recur)
-    a.wfrag = p->wfrag[p->Lb.broad ? kFragBwdBroad : kFragBwd].as<half8>();
+    a.wfrag = p->wfrag[L.broad ? kFragBwdBroad : kFragBwd].as<half8>();
     a.G = p->G.as<half_t>(); a.C = p->C.as<float>(); a.dY = p->bw.dYk; a.dG = p->dG.as<half_t>();
     a.dHn = p->dHn.as<float>(); a.dC = p->dC.as<float>(); a.dH0 = p->dH0.as<float>();
-    a.X = p->xch_b.as<half_t>(); a.x_slot = rec_bwd_slot_halfs(p->Lb, d.B, d.Hp);
-    if (p->Lb.two_d) {
+    a.X = p->xch_b.as<half_t>(); a.x_slot = rec_bwd_slot_halfs(L, d.B, d.Hp);
+    if (L.two_d) {
         a.wfrag2 = p->wfrag[kFragBwdTwoD].as<half8>();
         a.P = p->part_b.as<float>();
-        a.p_slot = rec_bwd_part_slot_floats(p->Lb);
+        a.p_slot = rec_bwd_part_slot_floats(L);
     }
     a.db_part = p->db_part.as<float>();
     a.status = p->status.as<int>();
@@ -1119,7 +1120,7 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
     // One launch, or one per window of batch rows (RecLayout::win_rows).  The windows share the ring of partial sums,
     // so every launch of a windowed pass starts from a ring prepared for ITS first product step (a single window's
     // launches continue each other's parities instead).
-    const int win = (p->Lb.two_d && p->Lb.win_rows) ? p->Lb.win_rows : d.B;
+    const int win = (L.two_d && L.win_rows) ? L.win_rows : d.B;
     for (int b_lo = 0; b_lo < d.B; b_lo += win) {
         a.b_lo = b_lo;
         a.b_hi = b_lo + win < d.B ? b_lo + win : d.B;
@@ -1130,11 +1131,11 @@ int backward_recur(flstm_core_plan* p, long t_hi, long t_lo, bool converted, hip
             const size_t pslot = a.p_slot * sizeof(float);
             const int first_T = t_hi >= long(p->bw.T) - 1 ? int(p->bw.T) : int(t_hi) + 2;   // (its first product step is first_T - 2)
             for (int k = 0; k < kRecBwdPartSlots; ++k)
-                FL_TRY(fill_words(static_cast<char*>(p->part_b.p) + size_t(k) * pslot, pslot, rec_bwd_part_fill(p->Lb, k, first_T), s));
+                FL_TRY(fill_words(static_cast<char*>(p->part_b.p) + size_t(k) * pslot, pslot, rec_bwd_part_fill(L, k, first_T), s));
         }
         const bool whole = (t_hi == long(p->bw.T) - 1 && t_lo == -1);   // (graphs for whole passes only: see forward_recur)
-        hipError_t e = launch_rec_bwd(p->Lb, a, s, (p->opt_graphs && whole) ? &p->graphs_b : nullptr);
-        if (e == hipErrorCooperativeLaunchTooLarge && p->Lb.persistent) return int(e);   // (handled by the caller: the layout changes)
+        hipError_t e = launch_rec_bwd(L, a, s, (p->opt_graphs && whole) ? &p->graphs_b : nullptr);
+        if (e == hipErrorCooperativeLaunchTooLarge && L.persistent) return int(e);   // (handled by the caller: the layout changes)
         FL_TRY(e);
     }
     return 0;
@@ -1215,7 +1216,7 @@ int backward_finish(flstm_core_plan* p, const void* x, flstm_dtype x_dtype, bool
         out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), 0, d.I, invS, accumulate, dW_ih);
         out.reduce_dw(d, p->dw_part.as<float>(), splits, size_t(ncols), n_ih, d.H, invS, accumulate, dW_hh);
     }
-    out.reduce_db(d, p->db_part.as<float>(), p->Lb.ng, invS, accumulate, db_ih, db_hh);
+    out.reduce_db(d, p->db_part.as<float>(), p->bw.L.ng, invS, accumulate, db_ih, db_hh);
     out.unpad(p->dH0.as<float>(), 1, size_t(d.Hp), size_t(d.B), d.H, invS, dh0, 1);
     out.unpad(p->dC.as<float>(), 1, size_t(d.Hp), size_t(d.B), d.H, invS, dc0, 1);
     return publish_with(p, out, kStampBwdEnd, s);
@@ -1258,7 +1259,7 @@ int backward_conclude(flstm_core_plan* p, bool weight_gradients, hipStream_t s) 
     int rc = take_status(p, s, &st);
     if (rc) return rc;
     if (st != 0) {
-        if (p->Lb.persistent) demote(p, false);
+        if (p->bw.L.persistent) demote(p, false);
         return FLSTM_E_STALLED;
     }
     pass_done(p, false);
@@ -1280,7 +1281,7 @@ int backward_pass(flstm_core_plan* p, size_t T, const void* x, flstm_dtype x_dty
         int rc = backward_enqueue(p, T, x, x_dtype, dY, dy_dtype, d_hn, d_cn, dstate_dtype, k, dx, dx_dtype, dW_ih, dW_hh, db_ih,
                                   db_hh, dh0, dc0, s);
         if (rc == 0) rc = wait_stream(s);
-        const bool persistent = p->Lb.persistent != 0;
+        const bool persistent = p->bw.L.persistent != 0;
         if (rc == 0) rc = backward_conclude(p, dW_ih || dW_hh, s);
         else if (rc == FLSTM_E_STALLED && persistent) demote(p, false);   // (the check ahead of accumulation)
         p->bw.open = false;
@@ -1421,7 +1422,7 @@ extern "C" int flstm_stack_backward(flstm_core_plan* const* plans, int layers, s
         if (rc == 0) rc = waited;
         bool again = false;
         for (int l = from; l >= 0 && rc == 0; --l) {
-            const bool persistent = plans[l]->Lb.persistent != 0;
+            const bool persistent = plans[l]->bw.L.persistent != 0;
             rc = backward_conclude(plans[l], true, s);
             if (rc == FLSTM_E_STALLED && persistent && attempt < layers) {
                 from = l;
@@ -1511,13 +1512,9 @@ extern "C" int flstm_core_backward_steps(flstm_core_plan* p, size_t t_hi, size_t
     if (!p || !p->bw.open || t_hi >= p->bw.T || nsteps == 0 || nsteps > t_hi + 1) return FLSTM_E_INVALID;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const long lo = long(t_hi) - long(nsteps) + 1;
-    if (p->bw.few != p->Lb.few) {   // (an option has changed the layout, and with it the ring: the caller repeats the pass)
-        p->bw.open = false;
-        return FLSTM_E_STALLED;
-    }
     // the range that reaches step 0 also runs the closing product for dh0
     int rc = backward_recur(p, long(t_hi), lo == 0 ? -1 : lo, false, s);
-    if (rc == int(hipErrorCooperativeLaunchTooLarge) && p->Lb.persistent && !p->refused_bwd) {
+    if (rc == int(hipErrorCooperativeLaunchTooLarge) && p->bw.L.persistent && !p->refused_bwd) {
         // the grid cannot be co-resident: step-wise from now on; the rings of this pass were laid out for the persistent
         // kernel, so the caller repeats the pass (as after a launch that gave up)
         p->refused_bwd = true;
@@ -1543,7 +1540,7 @@ extern "C" int flstm_core_backward_end(flstm_core_plan* p, const void* x, flstm_
     if (rc) return rc;
     if (st != 0) {   // the caller repeats the pass through flstm_core_backward
         p->bw.open = false;
-        if (p->Lb.persistent) demote(p, false);
+        if (p->bw.L.persistent) demote(p, false);
         return FLSTM_E_STALLED;
     }
     rc = backward_finish(p, x, x_dtype, false, dW_ih, dW_hh, db_ih, db_hh, dh0, dc0, s);
@@ -1559,7 +1556,7 @@ bool flstm_hip::core_copy_beside(flstm_core_plan* p, bool forward, const OpList&
     // 48 workgroups of 256 threads with one 16-byte load in flight each keep a PCIe link of 57 GB/s busy.  What counts is the
     // threads: the kernels for short contractions have workgroups of 64, 128 and 256 of them.
     constexpr int kFewest = 16 * 256, kThreads = 48 * 256;
-    const RecLayout& L = forward ? p->Lf : p->Lb;
+    const RecLayout& L = forward ? p->Lf : p->bw.L;
     const int idle = rec_idle_workgroups(L), threads = rec_threads(L), enough = kThreads / threads;
     if (idle * threads < kFewest || copies.count < 1 || copies.count > BesideCopies::kMost) return false;
     BesideCopies& b = forward ? p->beside_f : p->beside_b;

@@ -49,9 +49,8 @@ int flstm_core_destroy(flstm_core_plan* plan);
  * consecutive segments, last segment first, each segment's dh0 / dc0 fed to the next call as d_hn / d_cn),
  * "row_tiles_fwd" / "row_tiles_bwd" (16-row tiles per row block of that recurrence: 1, 2, or 0 = automatic; 1 only where
  * all 16-row blocks run side by side.  The kernels for short contractions, up to 512 units forward, have 16-row blocks, those for
- * few rows, up to 1024 units, blocks of 4 to 16: there 2 chooses the one-way kernel, whose sums are in another order.  An option that
- * changes the blocks between two flstm_core_backward_steps of a pass makes the next one return FLSTM_E_STALLED.  Above 2048 units batch
- * rows are taken in tiles of 16, one after the other, and the option changes nothing),
+ * few rows, up to 1024 units, blocks of 4 to 16: there 2 chooses the one-way kernel, whose sums are in another order.   Above
+ * 2048 units batch rows are taken in tiles of 16, one after the other, and the option changes nothing),
  * "cooperative" (0, the default: persistent launches are plain launches whose grid is checked to be co-resident, and
  * launches to different streams of a device are put one behind the other; 1: hipLaunchCooperativeKernel, which costs
  * 20 us more per launch -- and a process that made a cooperative launch faults inside an attached rocprofiler-sdk tool
@@ -179,7 +178,8 @@ int flstm_core_absmax(flstm_core_plan* plan, const void* tensor, flstm_dtype dty
  * backward ranges go from step T-1 downwards.  _end waits, returns FLSTM_E_STALLED if a persistent launch
  * gave up (repeat the pass with flstm_core_forward / flstm_core_backward, which fall back to step-wise
  * launches), and otherwise finishes the pass (final states; weight and bias gradients).  hy may lie in h0's place, cy in c0's;
- * dx and dY must be buffers of their own. */
+ * dx and dY must be buffers of their own.  A backward pass runs to its end with the layout of its _begin: an option that changes
+ * the layout in between ("row_tiles_bwd", "bwd_two_d", "stepwise") counts from the next pass on. */
 int flstm_core_forward_begin(flstm_core_plan* plan, size_t seq_len, const void* x, flstm_dtype x_dtype,
                              const void* h0, const void* c0, flstm_dtype state_dtype, void* stream);
 int flstm_core_forward_steps(flstm_core_plan* plan, size_t t0, size_t nsteps, void* stream);

@@ -77,7 +77,7 @@ def test_infinite_weights_give_what_the_other_kernels_give(B, H):
     core.close()
 
 
-# an option that changes the layout between two ranges of a pass: forward goes on in the other layout's ring, backward asks for the pass again
+# an option that changes the layout between two ranges of a forward pass: it goes on in the other layout's ring
 @pytest.mark.parametrize("T,B,H", [(11, 20, 650), (9, 32, 1024)])
 @pytest.mark.parametrize("name,value", [("row_tiles_fwd", 2), ("stepwise", 1)])
 def test_layout_that_changes_during_a_pass(T, B, H, name, value):
@@ -88,7 +88,7 @@ def test_layout_that_changes_during_a_pass(T, B, H, name, value):
     core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
     want, _ = run_core(p, core=core)
     lib, s = core.lib, torch.cuda.current_stream().cuda_stream
-    t16 = {k: p[k].cuda().half() for k in ("x", "dy", "h0", "c0")}
+    t16 = {k: p[k].cuda().half() for k in ("x", "dy", "h0", "c0", "d_hn", "d_cn")}
     hy, cy = (torch.empty(B, H, device="cuda", dtype=torch.float16) for _ in range(2))
     for first, then in ((0, value), (value, 0)):
         core.set_option(name, first)
@@ -100,15 +100,46 @@ def test_layout_that_changes_during_a_pass(T, B, H, name, value):
         torch.cuda.synchronize()
         assert core.info("fallbacks") == 0
         assert rell2(to_np(hy), want["hn"]) <= 1e-3 and rell2(to_np(cy), want["cn"]) <= 1e-3
-    core.set_option(name, 0)
+        core.set_option(name, 0)
+        grads = core.backward(t16["x"], t16["dy"], t16["d_hn"], t16["d_cn"])   # from the caches of all steps
+        for k, g in zip(("dx", "dw_ih", "dw_hh", "db", "dh0", "dc0"), grads):
+            assert rell2(to_np(g), want[k]) <= 1e-3, k
+    core.close()
+
+
+# ... of a backward pass, or behind the last of them: the pass keeps the layout it began with -- the ring, and the groups whose bias
+# gradients its end adds up (2 to 17 groups become one, and one becomes as many)
+@pytest.mark.parametrize("T,B,H,name,value", [(8, 9, 100, "row_tiles_bwd", 2), (8, 16, 650, "row_tiles_bwd", 2), (8, 32, 1024, "row_tiles_bwd", 2),
+                                              (7, 129, 256, "row_tiles_bwd", 2), (8, 20, 650, "stepwise", 1), (6, 16, 2048, "bwd_two_d", 0)])
+def test_a_backward_pass_keeps_its_layout(T, B, H, name, value):
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    p = make_problem(T, B, 64, H, seed=6)
+    core = LstmCore(B, 64, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    lib, s = core.lib, torch.cuda.current_stream().cuda_stream
+    t16 = {k: p[k].cuda().half() for k in ("x", "dy", "h0", "c0")}
     core.forward(t16["x"], t16["h0"], t16["c0"])
-    assert lib.flstm_core_backward_begin(core._h, T, t16["dy"].data_ptr(), 1, None, None, 1, 1.0, None, 1, s) == 0
-    assert lib.flstm_core_backward_steps(core._h, T - 1, 3, s) == 0
-    core.set_option("row_tiles_bwd", 2)
-    stalled = lib.flstm_core_backward_steps(core._h, T - 4, T - 3, s)
-    torch.cuda.synchronize()
-    assert stalled != 0 and core.info("fallbacks") == 0
-    core.set_option("row_tiles_bwd", 0)
-    got = core.backward(t16["x"], t16["dy"])
-    assert bool(torch.isfinite(got[0]).all())
+
+    def in_two_ranges(first, between, behind):
+        out = [torch.full(shape, float("nan"), device="cuda") for shape in ((T, B, 64), (4 * H, 64), (4 * H, H), (4 * H,), (B, H), (B, H))]
+        dx, dw_ih, dw_hh, db, dh0, dc0 = (t.data_ptr() for t in out)
+        core.set_option(name, first)
+        assert lib.flstm_core_backward_begin(core._h, T, t16["dy"].data_ptr(), 1, None, None, 1, 1.0, dx, 0, s) == 0
+        assert lib.flstm_core_backward_steps(core._h, T - 1, 3, s) == 0
+        core.set_option(name, between)
+        assert lib.flstm_core_backward_steps(core._h, T - 4, T - 3, s) == 0
+        core.set_option(name, behind)
+        assert lib.flstm_core_backward_end(core._h, t16["x"].data_ptr(), 1, dw_ih, dw_hh, db, None, dh0, dc0, s) == 0
+        torch.cuda.synchronize()
+        assert core.info("fallbacks") == 0
+        return [to_np(t) for t in out]
+
+    default = 1 if name == "bwd_two_d" else 0
+    for first, other in ((default, value), (value, default)):
+        want = in_two_ranges(first, first, first)
+        assert all(np.isfinite(w).all() for w in want)
+        for between, behind in ((first, other), (other, other), (other, first)):
+            for w, g in zip(want, in_two_ranges(first, between, behind)):
+                assert np.array_equal(w, g)
     core.close()
