@@ -32,10 +32,15 @@ def test_few_rows_against_64_bits_and_32_row_blocks(T, B, H, backward, forward, 
         core.set_option(name, 2)
     blocks, info = run_core(p, core=core, half=half)
     assert info["fallbacks"] == 0 and core.info("groups_bwd") == -(-B // 32)
-    # (as between the other layouts a sum's order flips roundings of h and dG; one row over few steps has few of them to average over)
+    # What both kernels are off by is the rounding of h, dG and the outputs to fp16, 2^-11 at most and some 2^-12 in the mean, once or twice
+    # in every sum.  Another order of an fp32 sum moves it by some 2^-20, which turns one rounding in a hundred the other way: the errors of
+    # two right kernels differ by that hundredth (0.8 % at most over this table, 1.5 % of hn of five rows), a wrong term is more than all of it.
     for k in ref:
-        worst = 1.05 * max(rell2(blocks[k], ref[k]), rell2(steps[k], ref[k])) + (2e-4 if B * H < 2000 else 0.0)
-        assert rell2(got[k], ref[k]) <= worst, (k, rell2(got[k], ref[k]), worst)
+        assert rell2(blocks[k], ref[k]) <= 1e-3, k
+        assert rell2(got[k], ref[k]) <= 1.05 * rell2(blocks[k], ref[k]), (k, rell2(got[k], ref[k]), rell2(blocks[k], ref[k]))
+    # launches per step run the same kernel: the same bits but for db, whose sums of up to 9 steps and 129 rows a launch adds up by itself
+    for k in ref:
+        assert np.array_equal(steps[k], got[k]) if k != "db" else rell2(steps[k], got[k]) <= 1e-6, k
     for name in ("row_tiles_fwd", "row_tiles_bwd"):
         core.set_option(name, 0)
     again, _ = run_core(p, core=core, half=half)
