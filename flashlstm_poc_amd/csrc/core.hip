@@ -135,7 +135,6 @@ struct flstm_core_plan {
     int ring_base = 0;
     size_t T_cache = 0;
     bool have_cache = false;
-    bool plain_ring = false;   // a call whose scratch has no room for the ring of RecLayout::few
     // pass in progress (begin / steps / end)
     struct { size_t T = 0; const void* x = nullptr; flstm_dtype x_dtype = FLSTM_F16; bool open = false;
              half_t* y_direct = nullptr;   // the recurrence writes the caller's y itself
@@ -171,7 +170,7 @@ namespace {
 
 void replan(flstm_core_plan* p) {
     p->Lf = plan_rec_fwd(p->d.B, p->d.Hp, p->num_cus, p->opt_stepwise || p->hold_fwd > 0 || p->eff_step_f || p->refused_fwd,
-                         p->plain_ring ? 2 : p->opt_mt_f ? p->opt_mt_f : p->eff_mt_f, p->opt_waves_f);
+                         p->opt_mt_f ? p->opt_mt_f : p->eff_mt_f, p->opt_waves_f);
     p->Lb = plan_rec_bwd(p->d.B, p->d.Hp, p->num_cus, p->opt_stepwise || p->hold_bwd > 0 || p->eff_step_b || p->refused_bwd,
                          p->opt_mt_b ? p->opt_mt_b : p->eff_mt_b,
                          (!p->two_d_explicit && p->eff_two_d >= 0) ? p->eff_two_d : p->opt_two_d);
@@ -462,7 +461,9 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     if (split.split || split.broad || split.few) {
         FL_TRY(want(kFragFwdSplit, split, rec_fwd_ks(split, d.Hp), rec_fwd_fragments(split, d.Hp)));
         frag[kFragFwdSplit].split = split.split;
-        if (split.split) FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));   // (here: flstm_core_forward_static allocates nothing)
+        // (the rings here: flstm_core_forward_static allocates nothing)
+        if (split.split) FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));
+        if (split.few) FL_TRY(p->xch_f.reserve(4 * rec_fwd_slot_halfs(split, d.B, d.Hp) * sizeof(half_t)));
     }
     FL_TRY(want(kFragBwd, bwd, rec_bwd_ks(bwd, d.Hp), rec_bwd_fragments(bwd, d.Hp)));
     if (broad.broad) FL_TRY(want(kFragBwdBroad, broad, rec_bwd_ks(broad, d.Hp), rec_bwd_fragments(broad, d.Hp)));
@@ -987,40 +988,29 @@ extern "C" int flstm_core_forward_static(flstm_core_plan* p, size_t T, const voi
     const Dims& d = p->d;
     const size_t TB = T * size_t(d.B);
     // the same buffers forward_setup() sizes, carved out of the static array instead of allocated
-    size_t need[5], off[5], total = 0;
-    auto carve = [&]() {
-        const size_t bytes[5] = {x_in_place(p, x_dtype) ? 0 : TB * d.Ip * sizeof(half_t),
-                                 TB * 4 * d.Hp * sizeof(half_t),
-                                 (TB + d.B) * d.Hp * sizeof(half_t),
-                                 (TB + d.B) * d.Hp * sizeof(float),
-                                 4 * rec_fwd_slot_halfs(p->Lf, d.B, d.Hp) * sizeof(half_t)};
-        total = align256(kStatusBytes);   // (the limit counts a status block; the plan's own is used)
-        for (int i = 0; i < 5; ++i) { need[i] = bytes[i]; off[i] = total; total += align256(need[i]); }
-    };
-    use_tuned(p, T);
-    carve();
-    if (total > kStaticScratchBytes && p->Lf.few) {   // (its ring may be a little larger than the other kernels')
-        p->plain_ring = true;
-        replan(p);
-        carve();
-    }
-    if (total > kStaticScratchBytes) {
-        if (p->plain_ring) { p->plain_ring = false; replan(p); }
-        return FLSTM_E_TOO_LARGE;
-    }
+    const size_t need[5] = {x_in_place(p, x_dtype) ? 0 : TB * d.Ip * sizeof(half_t),
+                            TB * 4 * d.Hp * sizeof(half_t),
+                            (TB + d.B) * d.Hp * sizeof(half_t),
+                            (TB + d.B) * d.Hp * sizeof(float),
+                            4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)};
+    size_t off[5], total = align256(kStatusBytes);   // (the limit counts a status block; the plan's own is used)
+    for (int i = 0; i < 5; ++i) { off[i] = total; total += align256(need[i]); }
+    if (total > kStaticScratchBytes) return FLSTM_E_TOO_LARGE;
     char* b = static_cast<char*>(base);
     DevBuf* slot[5] = {&p->X16, &p->G, &p->Y, &p->C, &p->xch_f};
+    // (the ring of RecLayout::few may be larger than the one that the limit counts: where the rule takes that layout, packing has reserved
+    // it in the plan, and the pass sums in the order of flstm_core_forward up to the limit)
+    const int carved = plan_rec_fwd(d.B, d.Hp, p->num_cus, false).few ? 4 : 5;
     DevBuf saved[5];
-    for (int i = 0; i < 5; ++i) { saved[i] = *slot[i]; *slot[i] = DevBuf::view(b + off[i], need[i]); }
+    for (int i = 0; i < carved; ++i) { saved[i] = *slot[i]; *slot[i] = DevBuf::view(b + off[i], need[i]); }
     const bool had_cache = p->have_cache;
     p->have_cache = false;   // (the plan's own caches are untouched, but no pass may use the borrowed ones later)
     // (step-wise launches, if the pass comes to them, are plain launches: a graph capture allocates)
     p->static_call = true;
     rc = forward_pass(p, T, x, x_dtype, h0, c0, state_dtype, y, y_dtype, hy, cy, out_state_dtype, false, s);
     p->static_call = false;
-    if (p->plain_ring) { p->plain_ring = false; replan(p); }
     p->fw.open = false;   // (also when the pass failed: the next call must not find a pass in progress)
-    for (int i = 0; i < 5; ++i) *slot[i] = saved[i];
+    for (int i = 0; i < carved; ++i) *slot[i] = saved[i];
     p->have_cache = had_cache;
     return rc;
 }

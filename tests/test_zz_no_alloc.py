@@ -155,3 +155,27 @@ def test_static_forward_allocates_nothing_on_the_step_wise_path_and_after_a_give
         assert torch.equal(g, w), ("after a failed call", what)
     for h in (plan, ref, plan2):
         assert lib.flstm_core_destroy(h) == 0
+
+
+# The last length that the array holds, where the ring of a kernel for few rows (blocks of 8, of 16) is larger than the one that the limit
+# counts and would not fit beside the rest: that kernel runs all the same, and the next length is refused
+@pytest.mark.parametrize("T,B,H", [(162, 54, 544), (51, 115, 800)])
+def test_static_forward_at_the_limit_sums_as_the_allocating_forward(T, B, H):
+    from flashlstm_poc_amd import load_library
+    lib = load_library()
+    p = make_problem(T + 1, B, 64, H, seed=44)
+    cvh = lambda t: t.cuda().half().contiguous()
+    x, h0, c0 = cvh(p["x"]), cvh(p["h0"]), cvh(p["c0"])
+    plan, keep = _plan(lib, p)
+    ref, keep_r = _plan(lib, p)
+    rc, want, _ = _call(lib, False, ref, x[:T].contiguous(), h0, c0, F16, torch.float16)
+    assert rc == 0
+    for call in range(2):
+        rc, got, grew = _call(lib, True, plan, x[:T].contiguous(), h0, c0, F16, torch.float16)
+        assert rc == 0 and (grew == 0 or call == 0)
+        for g, w, what in zip(got, want, ("y", "hy", "cy")):
+            assert torch.equal(g, w), (call, what)
+    rc, _, _ = _call(lib, True, plan, x, h0, c0, F16, torch.float16)
+    assert rc == 2004
+    for h in (plan, ref):
+        assert lib.flstm_core_destroy(h) == 0
