@@ -713,14 +713,7 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
             if (rc) return rc;
             a.project = ProjectBeside{};
         }
-        if (p->fw.few != p->Lf.few) {
-            rc = forward_ring_again(p, t0, s);
-            if (rc) return rc;
-            a.wfrag = forward_fragments(p);
-            a.X = p->xch_f.as<half_t>();
-            a.x_slot = rec_fwd_slot_halfs(p->Lf, d.B, d.Hp);
-        }
-        e = launch_rec_fwd(p->Lf, a, s, nullptr);
+        e = launch_rec_fwd(p->Lf, a, s, nullptr);   // (a plan's blocks are the same step-wise: the ring and the fragments stand)
     }
     FL_TRY(e);
     return 0;
