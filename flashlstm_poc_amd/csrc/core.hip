@@ -127,6 +127,7 @@ struct flstm_core_plan {
     // weights
     DevBuf wih_p, wih_t, wfrag[kFragKinds], bias_p;
     bool weights_packed = false, bias_packed = false;
+    bool one_way_packed = false;   // kFragFwd is there (else it is made from the other forward fragments: forward_fragments)
     // forward state / caches
     DevBuf X16, G, Y, C, status, xch_f, xch_b;
     // ring of the whole passes that are one launch (forward_whole): its own, because it stays ready from one to the next
@@ -445,7 +446,9 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     FL_TRY(p->wih_t.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
     // Fragments for every kernel that the options can choose for these sizes, whichever the current ones do: options and
     // tuned entries change after the weights are packed.  (The one-way kernels have theirs wherever 32-row blocks can be
-    // asked for; those for short contractions, up to 512 units, add at most 2 MiB, those for few rows, up to 1024, 8 MiB.)
+    // asked for; those for short contractions, up to 512 units, add at most 2 MiB, those for few rows, up to 1024, 8 MiB.  Where few
+    // rows are the rule, the one-way kernel's wait for an option that asks for them: packed with the others each time they
+    // took 8 us of the 70 of a packing of 1024 units, and a training step packs its weights.)
     FragLayout frag[kFragKinds];
     auto want = [&](int kind, const RecLayout& L, int ks, size_t fragments) -> hipError_t {
         FragLayout& f = frag[kind];
@@ -458,6 +461,8 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     const RecLayout bwd = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 2, 0), broad = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 0, 0);
     FL_TRY(want(kFragFwd, fwd, rec_fwd_ks(fwd, d.Hp), rec_fwd_fragments(fwd, d.Hp)));
     frag[kFragFwd].wide = fwd.wide;
+    p->one_way_packed = !(split.few && fwd.nw == 4);
+    if (!p->one_way_packed) frag[kFragFwd].fragments = 0;   // (the memory is there: flstm_core_forward_static allocates nothing)
     if (split.split || split.broad || split.few) {
         FL_TRY(want(kFragFwdSplit, split, rec_fwd_ks(split, d.Hp), rec_fwd_fragments(split, d.Hp)));
         frag[kFragFwdSplit].split = split.split;
@@ -647,8 +652,15 @@ void take_beside(BesideCopies& waiting, Args& a) {
     waiting.count = 0;
 }
 
-const half8* forward_fragments(const flstm_core_plan* p) {
-    return p->wfrag[p->Lf.split || p->Lf.broad || p->Lf.few ? kFragFwdSplit : kFragFwd].as<half8>();
+// The fragments of the forward layout; the one-way kernel's are made here the first time that a plan whose rule is few rows needs them.
+int forward_fragments(flstm_core_plan* p, const half8** fragments, hipStream_t s) {
+    const int kind = p->Lf.split || p->Lf.broad || p->Lf.few ? kFragFwdSplit : kFragFwd;
+    if (kind == kFragFwd && !p->one_way_packed) {
+        FL_TRY(gate_major_fragments(p->wfrag[kFragFwdSplit].as<half8>(), p->wfrag[kFragFwd].as<half8>(), rec_fwd_fragments(p->Lf, p->d.Hp), s));
+        p->one_way_packed = true;
+    }
+    *fragments = p->wfrag[kind].as<half8>();
+    return 0;
 }
 
 // The exchange ring as the steps from t0 on expect it, for a layout that came into force during the pass: h of the last step from its
@@ -676,14 +688,15 @@ int forward_recur(flstm_core_plan* p, size_t t0, size_t n, hipStream_t s) {
     }
     RecFwdArgs a;
     memset(static_cast<void*>(&a), 0, sizeof(a));   // (padding too: the arguments are the key of a captured graph)
-    a.wfrag = forward_fragments(p);
+    int rc = forward_fragments(p, &a.wfrag, s);
+    if (rc) return rc;
     a.Y = p->Y.as<half_t>(); a.G = p->G.as<half_t>(); a.C = p->C.as<float>();
     a.y_out = p->fw.y_direct;
     a.X = p->xch_f.as<half_t>(); a.x_slot = rec_fwd_slot_halfs(p->Lf, d.B, d.Hp);
     a.status = p->status.as<int>();
     a.delay_hint = p->status.as<int>() + 1;
     a.stamps = stamps_of(p) + kStampFwdRec;
-    int rc = next_seats(p, &a.seats, s);
+    rc = next_seats(p, &a.seats, s);
     if (rc) return rc;
     take_beside(p->beside_f, a);
     if (p->project.M != 0) {   // (else all of it stays zero: an assigned struct brings padding of its own into a graph's key)

@@ -147,6 +147,15 @@ __global__ __launch_bounds__(kT) void pack_kernel(PackJob job) {
     }
 }
 
+// Fragment `tile` of a slice's 128 columns 32 * gate + unit from those of columns 4 * unit + gate: lane l of it, column 16 tile + l % 16, is a lane
+// of the other order's tile that holds the same column and the same eight k.
+__global__ __launch_bounds__(kT) void gate_major_kernel(const half8* __restrict__ in, half8* __restrict__ out, unsigned items) {
+    const unsigned i = blockIdx.x * kT + threadIdx.x;
+    if (i >= items) return;
+    const unsigned lane = i % kWave, tile = i / kWave % 8, column = 16 * tile + lane % 16, other = column % 32 * 4 + column / 32;
+    out[i] = in[(i / (8 * kWave) * 8 + other / 16) * kWave + lane / 16 * 16 + other % 16];
+}
+
 __global__ void pack_bias_kernel(Dims d, const float* __restrict__ b_ih, const float* __restrict__ b_hh,
                                  float* __restrict__ out) {
     const int q = blockIdx.x * kT + threadIdx.x;
@@ -316,6 +325,13 @@ hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, hal
         job.first[i + 1] = job.first[i] + unsigned(ceil_div(items, kT));
     }
     hipLaunchKernelGGL(pack_kernel, dim3(job.first[kFragKinds + 2]), dim3(kT), 0, s, job);
+    return hipGetLastError();
+}
+
+hipError_t gate_major_fragments(const half8* unit_major, half8* out, size_t fragments, hipStream_t s) {
+    const size_t items = fragments * kWave;
+    if (items == 0 || fragments % 8 != 0 || items >> 32) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gate_major_kernel, dim3(unsigned(ceil_div(items, kT))), dim3(kT), 0, s, unit_major, out, unsigned(items));
     return hipGetLastError();
 }
 

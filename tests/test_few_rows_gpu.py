@@ -148,3 +148,33 @@ def test_a_backward_pass_keeps_its_layout(T, B, H, name, value):
             for w, g in zip(want, in_two_ranges(first, between, behind)):
                 assert np.array_equal(w, g)
     core.close()
+
+
+# The one-way kernel's weights, made when an option first asks for that kernel: those of the last packing, as a plan of more rows packs them
+# (its blocks of 32 rows sum a row as these do)
+@pytest.mark.parametrize("B,H", [(20, 650), (32, 1024), (5, 513), (70, 800)])
+def test_weights_of_the_one_way_kernel_follow_the_packing(B, H):
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    few, other = LstmCore(B, 64, H), LstmCore(250, 64, H)
+    for core in (few, other):
+        core.set_option("waves_fwd", 4)
+        core.set_option("row_tiles_fwd", 2)
+    for k, (name, value) in enumerate((("row_tiles_fwd", 2), ("row_tiles_fwd", 0), ("waves_fwd", 0), ("row_tiles_fwd", 2))):
+        p = make_problem(6, 250, 64, H, seed=80 + k)
+        weights = [p[n].cuda() for n in ("w_ih", "w_hh", "b_ih", "b_hh")]
+        x, h0, c0 = (p[n].cuda().half() for n in ("x", "h0", "c0"))
+        small = [x[:, :B].contiguous(), h0[:B].contiguous(), c0[:B].contiguous()]
+        few.pack(*weights)
+        other.pack(*weights)
+        want = other.forward(x, h0, c0)
+        few.set_option(name, value)
+        for again in range(2):
+            got = few.forward(*small)
+            if few.info("row_tiles_fwd") == 2:
+                for g, w in zip(got, (want[0][:, :B], want[1][:B], want[2][:B])):
+                    assert torch.equal(g, w)
+            else:
+                assert rell2(to_np(got[0]), to_np(want[0][:, :B])) <= 1e-3
+    few.close()
+    other.close()
