@@ -127,7 +127,8 @@ struct flstm_core_plan {
     // weights
     DevBuf wih_p, wih_t, wfrag[kFragKinds], bias_p;
     bool weights_packed = false, bias_packed = false;
-    bool one_way_packed = false;   // kFragFwd is there (else it is made from the other forward fragments: forward_fragments)
+    bool frag_there[2] = {false, false};   // kFragFwd, kFragFwdSplit (one that is not is made from the other: forward_fragments)
+    bool many_steps = false;   // of the pass that use_tuned was told of (many_steps())
     // forward state / caches
     DevBuf X16, G, Y, C, status, xch_f, xch_b;
     // ring of the whole passes that are one launch (forward_whole): its own, because it stays ready from one to the next
@@ -171,15 +172,17 @@ namespace {
 
 void replan(flstm_core_plan* p) {
     p->Lf = plan_rec_fwd(p->d.B, p->d.Hp, p->num_cus, p->opt_stepwise || p->hold_fwd > 0 || p->eff_step_f || p->refused_fwd,
-                         p->opt_mt_f ? p->opt_mt_f : p->eff_mt_f, p->opt_waves_f);
+                         p->opt_mt_f ? p->opt_mt_f : p->eff_mt_f, p->opt_waves_f, p->many_steps);
     p->Lb = plan_rec_bwd(p->d.B, p->d.Hp, p->num_cus, p->opt_stepwise || p->hold_bwd > 0 || p->eff_step_b || p->refused_bwd,
                          p->opt_mt_b ? p->opt_mt_b : p->eff_mt_b,
                          (!p->two_d_explicit && p->eff_two_d >= 0) ? p->eff_two_d : p->opt_two_d);
     p->Lf.cooperative = p->Lb.cooperative = p->opt_cooperative;
 }
 
+bool many_steps(const flstm_core_plan* p, size_t T);
+
 // Puts the tuned entry for sequence length T in force: the entry tuned at exactly T, else the nearest one within a
-// factor of two, else none.
+// factor of two, else none; and the forward layout for as many steps.
 void use_tuned(flstm_core_plan* p, size_t T) {
     const flstm_core_plan::Tuned* best = nullptr;
     double best_d = 1.0;   // |log2(T / T')| <= 1
@@ -191,7 +194,9 @@ void use_tuned(flstm_core_plan* p, size_t T) {
               sb = best ? best->step_b : 0, td = best ? best->two_d : -1;
     p->eff_dw = best ? best->dw_splits : 0;
     p->eff_T = best ? best->T : 0;
-    if (mt_f != p->eff_mt_f || mt_b != p->eff_mt_b || sf != p->eff_step_f || sb != p->eff_step_b || td != p->eff_two_d) {
+    const bool many = many_steps(p, T);
+    if (many != p->many_steps || mt_f != p->eff_mt_f || mt_b != p->eff_mt_b || sf != p->eff_step_f || sb != p->eff_step_b || td != p->eff_two_d) {
+        p->many_steps = many;
         p->eff_mt_f = mt_f; p->eff_mt_b = mt_b; p->eff_step_f = sf; p->eff_step_b = sb; p->eff_two_d = td;
         replan(p);
     }
@@ -418,6 +423,8 @@ extern "C" long flstm_core_get_info(const flstm_core_plan* p, const char* name) 
     if (!strcmp(name, "slice_bwd")) return p->Lb.jb;
     if (!strcmp(name, "groups_fwd")) return p->Lf.ng;
     if (!strcmp(name, "groups_bwd")) return p->Lb.ng;
+    if (!strcmp(name, "few_rows_fwd")) return p->Lf.few;
+    if (!strcmp(name, "few_rows_bwd")) return p->Lb.few;
     if (!strcmp(name, "fallbacks")) return p->fallbacks;
     if (!strcmp(name, "demotions_fwd")) return p->demotions_fwd;
     if (!strcmp(name, "demotions_bwd")) return p->demotions_bwd;
@@ -446,9 +453,9 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
     FL_TRY(p->wih_t.reserve(size_t(4) * d.Hp * d.Ip * sizeof(half_t)));
     // Fragments for every kernel that the options can choose for these sizes, whichever the current ones do: options and
     // tuned entries change after the weights are packed.  (The one-way kernels have theirs wherever 32-row blocks can be
-    // asked for; those for short contractions, up to 512 units, add at most 2 MiB, those for few rows, up to 1024, 8 MiB.  Where few
-    // rows are the rule, the one-way kernel's wait for an option that asks for them: packed with the others each time they
-    // took 8 us of the 70 of a packing of 1024 units, and a training step packs its weights.)
+    // asked for; those for short contractions, up to 512 units, add at most 2 MiB, those for few rows, up to 1024, 8 MiB.  Of these
+    // last and the one-way kernel's, those that the rule reads are packed, and the others wait for a pass that needs them: packed
+    // with them each time they took 8 us of the 70 of a packing of 1024 units, and a training step packs its weights.)
     FragLayout frag[kFragKinds];
     auto want = [&](int kind, const RecLayout& L, int ks, size_t fragments) -> hipError_t {
         FragLayout& f = frag[kind];
@@ -457,18 +464,23 @@ int flstm_hip::core_pack_weights_async(flstm_core_plan* p, const float* w_ih, co
         f.nt = L.nt; f.rot_div = L.rot_div; f.nw = L.nw; f.unit_major = L.unit_major;
         return e;
     };
-    const RecLayout fwd = plan_rec_fwd(d.B, d.Hp, p->num_cus, false, 2, p->opt_waves_f), split = plan_rec_fwd(d.B, d.Hp, p->num_cus, false);
+    const RecLayout fwd = plan_rec_fwd(d.B, d.Hp, p->num_cus, false, 2, p->opt_waves_f), split = plan_rec_fwd(d.B, d.Hp, p->num_cus, false, 0, 0, true);
+    const bool few_by_rule = plan_rec_fwd(d.B, d.Hp, p->num_cus, false).few != 0;
     const RecLayout bwd = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 2, 0), broad = plan_rec_bwd(d.B, d.Hp, p->num_cus, false, 0, 0);
     FL_TRY(want(kFragFwd, fwd, rec_fwd_ks(fwd, d.Hp), rec_fwd_fragments(fwd, d.Hp)));
     frag[kFragFwd].wide = fwd.wide;
-    p->one_way_packed = !(split.few && fwd.nw == 4);
-    if (!p->one_way_packed) frag[kFragFwd].fragments = 0;   // (the memory is there: flstm_core_forward_static allocates nothing)
-    if (split.split || split.broad || split.few) {
+    if (split.split || split.broad || (split.few && fwd.nw == 4)) {
         FL_TRY(want(kFragFwdSplit, split, rec_fwd_ks(split, d.Hp), rec_fwd_fragments(split, d.Hp)));
         frag[kFragFwdSplit].split = split.split;
         // (the rings here: flstm_core_forward_static allocates nothing)
         if (split.split) FL_TRY(p->ring.reserve(4 * exchange_slot_halfs(d.B, d.Hp) * sizeof(half_t)));
-        if (split.few) FL_TRY(p->xch_f.reserve(4 * rec_fwd_slot_halfs(split, d.B, d.Hp) * sizeof(half_t)));
+        if (few_by_rule) FL_TRY(p->xch_f.reserve(4 * rec_fwd_slot_halfs(split, d.B, d.Hp) * sizeof(half_t)));
+    }
+    p->frag_there[kFragFwd] = p->frag_there[kFragFwdSplit] = true;
+    if (split.few && fwd.nw == 4) {   // (the memory is there: flstm_core_forward_static allocates nothing)
+        const int later = few_by_rule ? kFragFwd : kFragFwdSplit;
+        frag[later].fragments = 0;
+        p->frag_there[later] = false;
     }
     FL_TRY(want(kFragBwd, bwd, rec_bwd_ks(bwd, d.Hp), rec_bwd_fragments(bwd, d.Hp)));
     if (broad.broad) FL_TRY(want(kFragBwdBroad, broad, rec_bwd_ks(broad, d.Hp), rec_bwd_fragments(broad, d.Hp)));
@@ -592,17 +604,31 @@ int forward_operand(flstm_core_plan* p, size_t t0, size_t n, bool converted, hip
 // 1439 / 1280); 211 steps of 256 rows of 384 units and 32 features 389 / 438.  Of 570 combinations measured both ways the choice is on
 // average 0.15 % off the faster one, at most 3 us or 2 % where it is beside.  Fewer than 16 workgroups are not tried: where 241 and more have seats a step takes
 // 8 tiles or more (17 rows of 2048 units, 113 of 1024), which so few do not keep up with.
-bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
-    const Dims& d = p->d;
-    const int helpers = rec_projecting_workgroups(p->Lf);
-    if (helpers < 16 || p->opt_profile || reinterpret_cast<uintptr_t>(A) % 16 != 0) return false;
+bool beside_pays(const Dims& d, const RecLayout& L, size_t n) {
+    const int helpers = rec_projecting_workgroups(L);
+    if (helpers < 16) return false;
     const double slabs = d.Ip / 64, tile = slabs * 0.52 + 4.6, first = slabs * 0.65 + 2.5;
     const double rounds = double(ceil_div(ceil_div(n * d.B, 128) * (4 * d.Hp / 128), size_t(helpers)));
-    const double one = d.Hp <= 768 ? (p->Lf.few == 8 ? 1.5 : 1.65) : d.Hp <= 1024 ? (p->Lf.few == 8 ? 1.7 : 1.8) : 2.4;
-    const double step = one * double(ceil_div(size_t(p->Lf.nrb), size_t(p->Lf.ng)));
+    const double one = d.Hp <= 768 ? (L.few == 8 ? 1.5 : 1.65) : d.Hp <= 1024 ? (L.few == 8 ? 1.7 : 1.8) : 2.4;
+    const double step = one * double(ceil_div(size_t(L.nrb), size_t(L.ng)));
     const double recurrence = step * double(n), last = step * std::fmin(double(n), 128.0 / d.B);
     const double in_front = recurrence + gemm_nt_cost(int(n * d.B), 4 * d.Hp, d.Ip) + 5.0;
     return std::fmax(recurrence + 1.5 * first + 2.0, 1.05 * rounds * tile + last + 4.0) < in_front;
+}
+bool projects_beside(const flstm_core_plan* p, size_t n, const half_t* A) {
+    return !p->opt_profile && reinterpret_cast<uintptr_t>(A) % 16 == 0 && beside_pays(p->d, p->Lf, n);
+}
+
+// Whether the 16-row blocks of a pass run in rec_fwd_few_kernel (plan_rec_fwd; 65 to 128 rows of 769 to 1024 units): from 512 steps on with the
+// projection in front, from 2048 on with it beside.  That kernel's step is the shorter one once the clock has fallen under the load; at the clock
+// that a short pass runs at, its stores of four bytes cost more than it gains.  Time with it over that with rec_fwd_kernel, 66 to 128 rows,
+// 800 to 1024 units, 64 to 1024 features, forward alone / forward of a training step: in front 2048 steps 0.83-0.94 / 0.87-0.93, 1024 steps 0.83-0.95 /
+// 0.89-0.98, 512 steps 0.86-1.00 / 0.89-1.03, 256 steps 0.98-1.05 / 0.97-1.04, 128 steps 0.99-1.08 / 1.01-1.07; beside 2048 steps 0.85-1.00 / 0.92-1.07,
+// 1024 steps 0.92-1.08 / 0.99-1.13, 512 steps 0.99-1.08 / 0.99-1.09, 16 steps 0.99-1.04.  (The bits are the same either way.)
+bool many_steps(const flstm_core_plan* p, size_t T) {
+    const Dims& d = p->d;
+    if (T < 512 || plan_rec_fwd(d.B, d.Hp, p->num_cus, false, 0, 0, true).few != 16) return false;
+    return T >= 2048 || !beside_pays(d, plan_rec_fwd(d.B, d.Hp, p->num_cus, false), T);
 }
 
 // x rows of steps [t0, t0+n) -> fp16 operand -> x-projection (+ bias) in G, or left to the recurrence's launch
@@ -652,12 +678,13 @@ void take_beside(BesideCopies& waiting, Args& a) {
     waiting.count = 0;
 }
 
-// The fragments of the forward layout; the one-way kernel's are made here the first time that a plan whose rule is few rows needs them.
+// The fragments of the forward layout; those that packing left out are made here the first time that a pass needs them.
 int forward_fragments(flstm_core_plan* p, const half8** fragments, hipStream_t s) {
     const int kind = p->Lf.split || p->Lf.broad || p->Lf.few ? kFragFwdSplit : kFragFwd;
-    if (kind == kFragFwd && !p->one_way_packed) {
-        FL_TRY(gate_major_fragments(p->wfrag[kFragFwdSplit].as<half8>(), p->wfrag[kFragFwd].as<half8>(), rec_fwd_fragments(p->Lf, p->d.Hp), s));
-        p->one_way_packed = true;
+    if (!p->frag_there[kind]) {
+        const int other = kind == kFragFwd ? kFragFwdSplit : kFragFwd;
+        FL_TRY(reorder_fragments(p->wfrag[other].as<half8>(), p->wfrag[kind].as<half8>(), rec_fwd_fragments(p->Lf, p->d.Hp), kind == kFragFwd, s));
+        p->frag_there[kind] = true;
     }
     *fragments = p->wfrag[kind].as<half8>();
     return 0;

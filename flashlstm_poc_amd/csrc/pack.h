@@ -27,8 +27,9 @@ enum Frag : int { kFragFwd, kFragFwdSplit, kFragBwd, kFragBwdBroad, kFragBwdTwoD
 // W_ih twice (as it is for the projection, transposed for dX) and W_hh as every kind of fragments asked for; one launch.
 hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, half_t* wih_p /*[4Hp][Ip]*/,
                         half_t* wih_t /*[Ip][4Hp]*/, const FragLayout (&frag)[kFragKinds], hipStream_t s);
-// The one-way forward kernel's fragments of slices of 32 units, up to 1024 units (columns 32 * gate + unit), from those of columns 4 * unit + gate.
-hipError_t gate_major_fragments(const half8* unit_major, half8* out, size_t fragments, hipStream_t s);
+// Forward fragments of slices of 32 units, up to 1024 units: those of columns 32 * gate + unit (gate_major, the one-way kernel's) from those of
+// columns 4 * unit + gate, or the other way round.
+hipError_t reorder_fragments(const half8* in, half8* out, size_t fragments, bool gate_major, hipStream_t s);
 hipError_t pack_bias(const Dims& d, const float* b_ih, const float* b_hh, float* bias_p, hipStream_t s);
 
 // dst[r][c] (pitch ldc) = sum over z < splits of partial[z * per + r * cols + c]: split-K partials of a plain GEMM.

@@ -147,12 +147,13 @@ __global__ __launch_bounds__(kT) void pack_kernel(PackJob job) {
     }
 }
 
-// Fragment `tile` of a slice's 128 columns 32 * gate + unit from those of columns 4 * unit + gate: lane l of it, column 16 tile + l % 16, is a lane
-// of the other order's tile that holds the same column and the same eight k.
-__global__ __launch_bounds__(kT) void gate_major_kernel(const half8* __restrict__ in, half8* __restrict__ out, unsigned items) {
+// Fragment `tile` of a slice's 128 columns in one order, 32 * gate + unit or 4 * unit + gate, from those in the other: lane l of it, column
+// 16 tile + l % 16, is a lane of the other order's tile that holds the same column and the same eight k.
+__global__ __launch_bounds__(kT) void reorder_kernel(const half8* __restrict__ in, half8* __restrict__ out, unsigned items, int gate_major) {
     const unsigned i = blockIdx.x * kT + threadIdx.x;
     if (i >= items) return;
-    const unsigned lane = i % kWave, tile = i / kWave % 8, column = 16 * tile + lane % 16, other = column % 32 * 4 + column / 32;
+    const unsigned lane = i % kWave, tile = i / kWave % 8, column = 16 * tile + lane % 16;
+    const unsigned other = gate_major ? column % 32 * 4 + column / 32 : column % 4 * 32 + column / 4;
     out[i] = in[(i / (8 * kWave) * 8 + other / 16) * kWave + lane / 16 * 16 + other % 16];
 }
 
@@ -328,10 +329,10 @@ hipError_t pack_weights(const Dims& d, const float* w_ih, const float* w_hh, hal
     return hipGetLastError();
 }
 
-hipError_t gate_major_fragments(const half8* unit_major, half8* out, size_t fragments, hipStream_t s) {
+hipError_t reorder_fragments(const half8* in, half8* out, size_t fragments, bool gate_major, hipStream_t s) {
     const size_t items = fragments * kWave;
     if (items == 0 || fragments % 8 != 0 || items >> 32) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(gate_major_kernel, dim3(unsigned(ceil_div(items, kT))), dim3(kT), 0, s, unit_major, out, unsigned(items));
+    hipLaunchKernelGGL(reorder_kernel, dim3(unsigned(ceil_div(items, kT))), dim3(kT), 0, s, in, out, unsigned(items), int(gate_major));
     return hipGetLastError();
 }
 

@@ -226,7 +226,8 @@ constexpr size_t kGraphCacheEntries = 4;
 // own weight fragments, which depend on the sizes alone (and, one-way forward, on `waves`).
 // waves: 0 = the rule of thumb (rec_waves), 4 or 8 = a one-way kernel with that many wavefronts per workgroup (8 only up to
 // 1024 units).
-RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt = 0, int waves = 0);
+// many_steps: a pass over which 16-row blocks of 769 to 1024 units run faster in rec_fwd_few_kernel (the bits are rec_fwd_kernel's).
+RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt = 0, int waves = 0, bool many_steps = false);
 // two_d: 0 = never the two-way split, 1 = where it is the faster layout, 2 = wherever it can run
 RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt = 0, int two_d = 1);
 // Wavefronts per workgroup the forward kernel runs with for these sizes (a function of the sizes alone).

@@ -1867,12 +1867,20 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_few_kernel(RecFwdArgs p, Rec
         gates_t act;
 #pragma unroll
         for (int v = 0; v < UPT; ++v) {
-            floatx4 sum = *reinterpret_cast<const floatx4*>(part + size_t(r) * PLD + 4 * (u + v));
-#pragma unroll
-            for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const floatx4*>(part + (size_t(w) * 16 + r) * PLD + 4 * (u + v));
+            floatx4 sum;   // (blocks of 16 sum in the order of rec_fwd_kernel)
             float z[4];
             unpack_h2(xp[par][2 * v], z[0], z[1]);
             unpack_h2(xp[par][2 * v + 1], z[2], z[3]);
+            if constexpr (PK == 1) {
+                sum = floatx4{z[0], z[1], z[2], z[3]};
+                z[0] = z[1] = z[2] = z[3] = 0.f;
+            }
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const floatx4 p_w = *reinterpret_cast<const floatx4*>(part + (size_t(w) * 16 + r) * PLD + 4 * (u + v));
+                if (PK == 1 || w > 0) sum += p_w;
+                else sum = p_w;
+            }
             const float ig = sigmoidf_dev(z[0] + sum[0]), fg = sigmoidf_dev(z[1] + sum[1]), gg = tanhf_dev(z[2] + sum[2]), og = sigmoidf_dev(z[3] + sum[3]);
             c[v] = fg * c[v] + ig * gg;
             h[v] = og * tanhf_dev(c[v]);
@@ -3992,16 +4000,17 @@ static void finish_layout(RecLayout& L, int B, int Hp, int num_cus, bool force_s
 }
 
 // Rows per block of rec_fwd_few_kernel, 0: not for these sizes.  Blocks of 8 as long as half of the workgroups stay without a seat, with
-// which the projection is formed; with more of them seated it stands in front.  Us a call, rec_fwd_kernel / blocks of 8: 512 steps of 32
-// rows of 1024 features and units 951 / 927 (2048 steps 4211 / 3573), 4 rows and 128 features 893 / 848, 20 rows of 650 units 874 /
-// 818, 56 rows of 544 879 / 859; the other side of the line, device time: 48 rows of 1024 features and units 1002 / 1192.  Blocks of 16
-// above 768 units where rec_fwd_kernel seats more than half as well: 80 rows of 1024 1383 / 1301, 128 rows 1692 / 1582; 64 rows 1000 / 1043,
-// 100 rows of 600 units 904 / 908.
-static int few_rows_fwd(int B, int Hp, int num_cus) {
+// which the projection is formed.  Us a call, rec_fwd_kernel / blocks of 8: 512 steps of 32 rows of 1024 features and units 948 / 926, 4 rows
+// and 64 features 896 / 849, 20 rows of 650 units 872 / 814, 32 rows of 544 864 / 848; the other side of the line, device time: 48 rows of 1024
+// features and units 1002 / 1192, where the projection comes to stand in front.  (Where it stands there either way, or little of it is to be formed,
+// the line could be further on: 48 rows of 700 units and 512 features 903 / 840, 64 rows and 128 features 875 / 838.)  One to four steps take 1 to
+// 2 us longer (twice the workgroups fetch the weights: 32 rows of 1024 units 54 / 56).
+// Blocks of 16, the rows of rec_fwd_kernel, only over many steps (many_steps in core.hip).
+static int few_rows_fwd(int B, int Hp, int num_cus, bool many_steps) {
     const int nh = Hp / 32;
     if (Hp <= kFwdSplitMost || Hp > 1024 || num_cus != 256) return 0;
     if (int(ceil_div(size_t(B), 8)) * nh <= num_cus / 2) return 8;
-    return Hp > 768 && B > 64 && B <= 128 ? 16 : 0;
+    return many_steps && Hp > 768 && B > 64 && B <= 128 ? 16 : 0;
 }
 // Rows per block of rec_bwd_few_kernel, likewise.  Blocks of 4 where all of them run side by side, else of 8 (us a step, 8 / 4 rows:
 // 1024 units and 32 rows 1.71 / 1.43, 650 and 20 rows 1.49 / 1.33, 257 and 70 rows 1.11 / 1.06, 64 and 16 rows 0.90 / 0.84); but a batch of
@@ -4022,7 +4031,7 @@ static void few_blocks(RecLayout& L, int B, int rows) {
     if (!L.persistent) L.grid = L.ng * L.nh;
 }
 
-RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt, int waves) {
+RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int force_mt, int waves, bool many_steps) {
     RecLayout L{};
     L.num_cus = num_cus;
     bool fits = true;
@@ -4060,9 +4069,10 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
         }
     }
     // few rows (rec_fwd_few_kernel), likewise
-    if (L.nw == 4 && waves != 4 && force_mt != 2 && few_rows_fwd(B, Hp, num_cus)) {
+    const int rows = few_rows_fwd(B, Hp, num_cus, many_steps);
+    if (L.nw == 4 && waves != 4 && force_mt != 2 && rows) {
         L.unit_major = 1;
-        few_blocks(L, B, few_rows_fwd(B, Hp, num_cus));
+        few_blocks(L, B, rows);
     }
     return L;
 }

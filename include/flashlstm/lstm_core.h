@@ -49,7 +49,7 @@ int flstm_core_destroy(flstm_core_plan* plan);
  * consecutive segments, last segment first, each segment's dh0 / dc0 fed to the next call as d_hn / d_cn),
  * "row_tiles_fwd" / "row_tiles_bwd" (16-row tiles per row block of that recurrence: 1, 2, or 0 = automatic; 1 only where
  * all 16-row blocks run side by side.  The kernels for short contractions, up to 512 units forward, have 16-row blocks, those for
- * few rows, up to 1024 units, blocks of 4 to 16: there 2 chooses the one-way kernel, whose sums are in another order.   Above
+ * few rows, up to 1024 units, blocks of 4 to 16: there 2 chooses the one-way kernel, whose sums are in another order.  Above
  * 2048 units batch rows are taken in tiles of 16, one after the other, and the option changes nothing),
  * "cooperative" (0, the default: persistent launches are plain launches whose grid is checked to be co-resident, and
  * launches to different streams of a device are put one behind the other; 1: hipLaunchCooperativeKernel, which costs
@@ -77,7 +77,8 @@ int flstm_core_set_option(flstm_core_plan* plan, const char* name, long value);
  * direction still runs step-wise before the persistent kernel is tried again; 0 = not demoted), "slice_fwd", "slice_bwd" (hidden units
  * per workgroup of the recurrence kernels), "waves_fwd" (wavefronts per workgroup the forward recurrence runs with: 1, 2,
  * 4 or 8), "row_tiles_fwd", "row_tiles_bwd" (16-row tiles per row block that the
- * recurrences run with; "row_tiles": the forward one), "hidden_padded",
+ * recurrences run with; "row_tiles": the forward one), "few_rows_fwd", "few_rows_bwd" (rows per block of the kernels for few rows, 0: the
+ * recurrence runs in another kernel), "hidden_padded",
  * "input_padded", "whole_fwd" (the last forward pass was one launch, but for what had to be prepared in front of it), "projection_fwd"
  * (where it formed the x-projection: 0 by a launch in front of the recurrence, 1 beside it by the workgroups of the same launch that
  * have no share in it, 2 inside it), "products_shared" (the last backward pass formed dX and the weight gradients in one launch),

@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 # T, B, H and the groups backward and forward (None: another kernel forward).  Slices that end a pack of two or four and slices that
 # leave 1 to 3 of its k-steps without one; the first and last size of every kernel (4, 8, 12, 16, 24, 32 k-steps a wave); one row, a block that
-# is not full, the last batch of blocks of 4 and the first of 8, of 8 and of another kernel; forward the last batch of 8 rows, the first and last of 16
+# is not full, the last batch of blocks of 4 and the first of 8, of 8 and of another kernel; forward the last batch of 8 rows (the last three are
+# another kernel's over so few steps)
 SHAPES = [(9, 1, 32, 1, None), (9, 5, 100, 2, None), (7, 16, 128, 4, None), (6, 9, 130, 3, None), (8, 4, 256, 1, None), (7, 129, 256, 17, None),
           (9, 70, 257, 18, None), (6, 65, 384, 9, None), (6, 5, 385, 2, None), (7, 64, 512, 16, None), (6, 128, 512, 16, None), (5, 1, 513, 1, 1),
           (9, 20, 650, 5, 3), (6, 33, 768, 5, 5), (7, 32, 769, 8, 4), (6, 6, 800, 2, 1), (8, 32, 1024, 8, 4), (5, 33, 1000, 5, None), (5, 64, 1024, 8, None),
@@ -177,4 +178,32 @@ def test_weights_of_the_one_way_kernel_follow_the_packing(B, H):
             else:
                 assert rell2(to_np(got[0]), to_np(want[0][:, :B])) <= 1e-3
     few.close()
+    other.close()
+
+
+# Blocks of 16 rows: from 512 steps on where the projection stands in front, from 2048 on beside it, and the bits of the one-way kernel, which
+# takes the others.  The weights that the other kernel reads are made from the packed ones, for each packing anew.  (8 blocks of 7 and of 8
+# k-steps a wave, the last one not full; 6 and 5 of 8)
+@pytest.mark.parametrize("first,B,I,H,beside", [(512, 128, 24, 769, 0), (512, 113, 24, 1024, 0), (512, 90, 520, 1000, 0), (2048, 66, 24, 1000, 1)])
+def test_many_steps_in_blocks_of_16(first, B, I, H, beside):
+    import torch
+    from flashlstm_poc_amd import LstmCore
+    core, other = LstmCore(B, I, H), LstmCore(B, I, H)
+    other.set_option("waves_fwd", 4)
+    for seed, lengths in ((90, (first, first - 1)), (91, (5, first))):
+        p = make_problem(first, B, I, H, seed=seed)
+        weights = [p[n].cuda() for n in ("w_ih", "w_hh", "b_ih", "b_hh")]
+        x, h0, c0 = (p[n].cuda().half() for n in ("x", "h0", "c0"))
+        core.pack(*weights)
+        other.pack(*weights)
+        for T in lengths:
+            got, want = core.forward(x[:T], h0, c0), other.forward(x[:T], h0, c0)
+            assert core.info("few_rows_fwd") == (16 if T == first else 0) and other.info("few_rows_fwd") == 0
+            assert core.info("fallbacks") == 0 and (T < first or core.info("projection_fwd") == beside)
+            for g, w in zip(got, want):
+                assert torch.equal(g, w)
+    core.set_option("stepwise", 1)
+    got = core.forward(x, h0, c0)
+    assert core.info("few_rows_fwd") == 16 and all(torch.equal(g, w) for g, w in zip(got, want))
+    core.close()
     other.close()

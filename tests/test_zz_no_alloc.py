@@ -157,8 +157,8 @@ def test_static_forward_allocates_nothing_on_the_step_wise_path_and_after_a_give
         assert lib.flstm_core_destroy(h) == 0
 
 
-# The last length that the array holds, where the ring of a kernel for few rows (blocks of 8, of 16) is larger than the one that the limit
-# counts and would not fit beside the rest: that kernel runs all the same, and the next length is refused
+# The last length that the array holds, where the ring of the kernel for few rows (blocks of 8; of 16 it is another kernel over so few steps) is larger
+# than the one that the limit counts and would not fit beside the rest: that kernel runs all the same, and the next length is refused
 @pytest.mark.parametrize("T,B,H", [(162, 54, 544), (51, 115, 800)])
 def test_static_forward_at_the_limit_sums_as_the_allocating_forward(T, B, H):
     from flashlstm_poc_amd import load_library
