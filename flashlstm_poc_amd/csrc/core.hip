@@ -1717,6 +1717,7 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
     const bool keep_cache = p->have_cache;
     const std::vector<flstm_core_plan::Tuned> keep_tuned = p->tuned;
     p->tuned.clear();
+    use_tuned(p, T);
     p->opt_accumulate = 0;
     auto restore = [&]() {
         p->opt_stepwise = keep_step; p->opt_mt_f = keep_mtf; p->opt_mt_b = keep_mtb; p->opt_dw_splits = keep_dw;
@@ -1757,10 +1758,12 @@ extern "C" int flstm_core_tune(flstm_core_plan* p, size_t T, int repeats, int tr
     // 1) row-block height and launch mode of the two recurrences (independent of each other and of the GEMMs)
     p->opt_dw_splits = 0;
     for (int step = 0; step <= (try_stepwise ? 1 : 0); ++step) {
-        for (int mt = 1; mt <= 2; ++mt) {
+        bool rule_f = false, rule_b = false;   // whether the rule is neither
+        for (int mt : {1, 2, 0}) {
             p->opt_stepwise = step; p->opt_mt_f = mt; p->opt_mt_b = mt;
             replan(p);
-            const bool f_is = (p->Lf.mt == mt), b_is = (p->Lb.mt == mt);   // 16-row blocks may not fit
+            const bool f_is = mt ? p->Lf.mt == mt : rule_f && p->Lf.few, b_is = mt ? p->Lb.mt == mt : rule_b && p->Lb.few;   // 16-row blocks may not fit
+            if (mt == 1) { rule_f = !p->Lf.few; rule_b = !p->Lb.few; }
             if (!f_is && !b_is) continue;
             rc = run();
             if (rc) { restore(); return fail(rc); }

@@ -3951,6 +3951,7 @@ constexpr int kWideMost = 4096;   // hidden units whose W_hh the chip can hold (
 // its end: with one or two waves per CU it is the faster kernel up to 512 units (64 rows 1.64 -> 1.34 us per step, 100 rows
 // 1.42), with four up to 256 (200 rows 1.44 -> 1.16; at 288 units equal, at 512 units 1.7 -> 2.3).
 constexpr int kFwdSplitMost = 512, kFwdSplitFourMost = 256;
+constexpr int kBwdSmallMost = 384;   // hidden units up to which asking for blocks of 16 rows backward changes nothing (plan_rec_bwd)
 constexpr int kBroadMost = 1536;   // hidden units of which a workgroup can hold the weights of a slice of 32 (384 KiB)
 
 // whether all 16-row blocks of the batch can run side by side
@@ -4068,9 +4069,9 @@ RecLayout plan_rec_fwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
             break;
         }
     }
-    // few rows (rec_fwd_few_kernel), likewise
+    // few rows (rec_fwd_few_kernel), unless blocks of 16 or 32 rows are asked for
     const int rows = few_rows_fwd(B, Hp, num_cus, many_steps);
-    if (L.nw == 4 && waves != 4 && force_mt != 2 && rows) {
+    if (L.nw == 4 && waves != 4 && force_mt == 0 && rows) {
         L.unit_major = 1;
         few_blocks(L, B, rows);
     }
@@ -4087,8 +4088,10 @@ RecLayout plan_rec_bwd(int B, int Hp, int num_cus, bool force_stepwise, int forc
     L.nw = 4;
     L.jb = 16 * L.nt;
     finish_layout(L, B, Hp, num_cus, force_stepwise, fits, force_mt);
-    // few rows (rec_bwd_few_kernel): every group has one block, its slices are those of the one-way kernel, and so are its fragments
-    if (force_mt != 2 && !(two_d >= 2 && Hp == 1024) && few_rows_bwd(B, Hp, num_cus)) {
+    // few rows (rec_bwd_few_kernel): every group has one block, its slices are those of the one-way kernel, and so are its fragments.  Blocks of
+    // 16 rows are the one-way kernel's where they are worth asking for (us a step, blocks of 16 / the rule: 1024 units and 32 rows 2.67 / 1.43,
+    // 512 and 64 rows 2.10 / 1.11); up to 384 units its step is twice as long and they mean the rule's blocks, as forward up to 512 units.
+    if ((force_mt == 0 || (force_mt == 1 && Hp <= kBwdSmallMost)) && !(two_d >= 2 && Hp == 1024) && few_rows_bwd(B, Hp, num_cus)) {
         few_blocks(L, B, few_rows_bwd(B, Hp, num_cus));
         return L;
     }

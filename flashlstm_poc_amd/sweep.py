@@ -151,7 +151,7 @@ def format_row(r: Dict) -> str:
               f"fwd+bwd {r['torch_fwd_bwd_ms']:9.3f} ms (x{r['speedup_fwd_bwd']:.2f})")
     if "tuned" in r:
         t = r["tuned"]
-        s += (f"  | tuned: rows/block fwd {16 * t['row_tiles_fwd']} bwd {16 * t['row_tiles_bwd']}, "
+        s += (f"  | tuned: rows/block fwd {16 * t['row_tiles_fwd'] or 'by rule'} bwd {16 * t['row_tiles_bwd'] or 'by rule'}, "
               f"{'step-wise' if t['stepwise_fwd'] else 'persistent'}/{'step-wise' if t['stepwise_bwd'] else 'persistent'}, "
               f"dW split-K {t['dw_splits']}")
     if "parity_ok" in r:

@@ -48,8 +48,9 @@ int flstm_core_destroy(flstm_core_plan* plan);
  * and db_hh to what the caller's buffers hold instead of overwriting them: a sequence processed as several
  * consecutive segments, last segment first, each segment's dh0 / dc0 fed to the next call as d_hn / d_cn),
  * "row_tiles_fwd" / "row_tiles_bwd" (16-row tiles per row block of that recurrence: 1, 2, or 0 = automatic; 1 only where
- * all 16-row blocks run side by side.  The kernels for short contractions, up to 512 units forward, have 16-row blocks, those for
- * few rows, up to 1024 units, blocks of 4 to 16: there 2 chooses the one-way kernel, whose sums are in another order.  Above
+ * all 16-row blocks run side by side.  Automatic may be the kernels for short contractions, up to 512 units forward, with 16-row blocks, or
+ * those for few rows, up to 1024 units, with blocks of 4 to 16: 2 chooses the one-way kernel instead, and so does 1 above 512 units
+ * forward and 384 backward (below it is as 0 wherever 0 is one of these); its sums are in another order.  Above
  * 2048 units batch rows are taken in tiles of 16, one after the other, and the option changes nothing),
  * "cooperative" (0, the default: persistent launches are plain launches whose grid is checked to be co-resident, and
  * launches to different streams of a device are put one behind the other; 1: hipLaunchCooperativeKernel, which costs
@@ -214,7 +215,7 @@ double flstm_core_last_ms(const flstm_core_plan* plan, const char* phase);
  * autotune loop of python/benchmark_lstm.py:203-301, for the launch choices that matter in this library).  For
  * sequence length seq_len it times, on synthetic data of varied values (the matrix cores run slower on those than
  * on constants) in the plan's own buffers, `repeats` passes of every candidate: 16- or 32-row blocks for each
- * recurrence (where both fit), persistent or -- with try_stepwise -- one launch per step, the layout of the
+ * recurrence (where both fit) and the rule's own where they are neither, persistent or -- with try_stepwise -- one launch per step, the layout of the
  * backward recurrence where the two-way split can run (option "bwd_two_d" 0 / 1 / 2, unless that option was set
  * explicitly), and the split-K count of the weight-gradient GEMM around the rule of thumb; the fastest choice
  * per phase is cached in the plan and used by every later pass whose length is within a factor of two of a tuned

@@ -207,3 +207,61 @@ def test_many_steps_in_blocks_of_16(first, B, I, H, beside):
     assert core.info("few_rows_fwd") == 16 and all(torch.equal(g, w) for g, w in zip(got, want))
     core.close()
     other.close()
+
+
+# Blocks of 16 rows asked for where the rule takes blocks of fewer: the one-way kernel above 512 units forward and 384 backward, by an option and by a
+# tuned entry, step-wise as well; below, where 16-row blocks never were that kernel's, the rule's.  (First and last sizes of that kernel's
+# instantiations; a block that is not full, one row, all rows that have blocks of 8)
+@pytest.mark.parametrize("T,B,H", [(6, 65, 384), (6, 5, 385), (7, 64, 512), (5, 1, 513), (9, 20, 650), (7, 32, 769), (5, 33, 1000), (8, 32, 1024)])
+@pytest.mark.parametrize("stepwise", [False, True])
+def test_blocks_of_16_rows_where_fewer_are_the_rule(T, B, H, stepwise):
+    from flashlstm_poc_amd import LstmCore
+    p = make_problem(T, B, 24, H, seed=B * 10000 + H)
+    ref = {k: v.cpu().numpy() for k, v in reference_64(p).items()}
+    core = LstmCore(B, 24, H)
+    core.pack(*(p[k].cuda() for k in ("w_ih", "w_hh", "b_ih", "b_hh")))
+    runs = {}
+    for tiles in (0, 2, 1):
+        for name in ("row_tiles_fwd", "row_tiles_bwd"):
+            core.set_option(name, tiles)
+        runs[tiles], info = run_core(p, core=core, stepwise=stepwise)
+        assert info["fallbacks"] == 0
+    assert core.info("few_rows_fwd") == 0 and core.info("row_tiles_fwd") == 1 and core.info("row_tiles_bwd") == 1
+    one_way = H > 384
+    assert (core.info("few_rows_bwd") == 0) == one_way and (not one_way or core.info("groups_bwd") == -(-B // 16))
+    assert H <= 512 or core.info("groups_fwd") == -(-B // 16)
+    # (the error of blocks of 32 and the allowance for flipped roundings: test_few_rows_against_64_bits_and_32_row_blocks)
+    for k in ref:
+        assert rell2(runs[1][k], ref[k]) <= 1.05 * rell2(runs[2][k], ref[k]) <= 1.05e-3, k
+        assert one_way or np.array_equal(runs[1][k], runs[0][k]), k
+    # a tuned entry says the same, and one without a choice leaves the rule in force
+    for name in ("row_tiles_fwd", "row_tiles_bwd"):
+        core.set_option(name, 0)
+    for tiles in (1, 0):
+        assert core.lib.flstm_core_set_tuned(core._h, T, tiles, tiles, int(stepwise), int(stepwise), 0, -1) == 0
+        tuned, _ = run_core(p, core=core, stepwise=stepwise)
+        for k in tuned:
+            assert np.array_equal(tuned[k], runs[tiles][k]), (tiles, k)
+    core.close()
+
+
+# The tuner has all three: what it keeps is a choice that can be put back, and no slower than either of the others
+def test_tuner_tries_the_rule_beside_blocks_of_16_and_32_rows():
+    from flashlstm_poc_amd import LstmCore, sweep
+    T, B, I, H = 64, 20, 64, 650
+    p = sweep.make_problem(T, B, I, H, seed=9)
+    core = LstmCore(B, I, H)
+    core.pack(p["w_ih"], p["w_hh"], p["b_ih"], p["b_hh"])
+    least = {}
+    for tiles in (0, 1, 2):
+        core.set_option("row_tiles_bwd", tiles)
+        core.forward(p["x"])
+        for _ in range(8):
+            core.backward(p["x"], p["dy"])
+            least[tiles] = min(least.get(tiles, 1e9), core.last_ms("bwd_rec"))
+    core.set_option("row_tiles_bwd", 0)
+    t = core.tune(T, repeats=6)
+    # (bwd_rec_ms is the device's own time; the three differ by more than a third: 1.3 us a step, 2.5 and more)
+    assert t["row_tiles_bwd"] == min(least, key=least.get) == 0 and t["bwd_rec_ms"] < 1.2 * least[0]
+    assert core.info("few_rows_bwd") == 4
+    core.close()
