@@ -1700,6 +1700,17 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
     clk.flush();
 }
 
+// the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
+__device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
+__device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
+__device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
+__device__ __forceinline__ unsigned as_bits(float v) { return __builtin_bit_cast(unsigned, v); }
+// the value of the lane N rows further on in the same 16
+template <int N>
+__device__ __forceinline__ float row_ahead(float v) {
+    return as_float(unsigned(__builtin_amdgcn_update_dpp(0, int(as_bits(v)), 0x100 | N, 0xF, 0xF, true)));
+}
+
 // ------------------------------------------------------------------------------- forward, few rows per group
 // 513 to 1024 units where blocks of RB = 8 rows leave half of the workgroups without a seat, and where blocks of RB = 16 take most of them
 // (few_rows_fwd).  The waves of a slice split the contraction as in rec_fwd_kernel.  What is shorter here:
@@ -1711,18 +1722,9 @@ __global__ __launch_bounds__(kThreads) void rec_fwd_split_kernel(RecFwdArgs p, R
 // Measured, us a step, rec_fwd_kernel -> here: 1024 units and 32 rows 1.77 -> 1.70 (over 2048 steps, where the other kernel's clock falls,
 // 2.03 -> 1.70), 4 rows 1.66 -> 1.57, 650 and 20 rows 1.61 -> 1.50, 1024 and 80 rows 2.00 -> 1.86, 128 rows 2.23 -> 2.05.  What is left
 // at 1024 units: the trip through the L2 (0.8 us), 64 MFMAs a wave (0.45), partial sums and the cells' five exponentials.
-// K-steps past the contraction are written as zeros once per launch (step-wise by every launch; the first reads none).  The rows of the x-projection that are formed beside (project_beside)
-// are waited for a step ahead as well.
-// the value of another lane of the same four: quad_perm(1, 0, 3, 2) and (2, 3, 0, 1)
-__device__ __forceinline__ unsigned quad_xor1(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)); }
-__device__ __forceinline__ unsigned quad_xor2(unsigned v) { return unsigned(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)); }
-__device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
-__device__ __forceinline__ unsigned as_bits(float v) { return __builtin_bit_cast(unsigned, v); }
-// the value of the lane N rows further on in the same 16
-template <int N>
-__device__ __forceinline__ float row_ahead(float v) {
-    return as_float(unsigned(__builtin_amdgcn_update_dpp(0, int(as_bits(v)), 0x100 | N, 0xF, 0xF, true)));
-}
+// K-steps past the contraction that a pack reaches into are zeros: in the slot that the first step reads because OpList::to_exchange has
+// written that whole slot, in all four because the last slice's workgroup writes them at the start of every launch.  The rows of the
+// x-projection that are formed beside (project_beside) are waited for a step ahead as well.
 template <int KS, int RB>
 __global__ __launch_bounds__(kThreads) void rec_fwd_few_kernel(RecFwdArgs p, RecLayout L, int t_begin, int t_end, int ks_wave) {
     constexpr int PK = 16 / RB, NP = (KS + PK - 1) / PK, UPT = RB / 8, PLD = 128 + (RB == 8 ? 28 : 4);   // (pitch: 16 rows', and 16 lanes' cells', 16 bytes lie in different banks)
@@ -3131,7 +3133,7 @@ __global__ __launch_bounds__(kThreads) void rec_bwd_kernel(RecBwdArgs p, RecLayo
 }
 
 // -------------------------------------------------------------------- backward, few rows per group
-// 385 to 1024 units where blocks of RB = 8 or 4 rows can all run side by side, each on an XCD's share of workgroups of its own.  A step
+// Up to 1024 units where blocks of RB = 8 or 4 rows can all run side by side, each on an XCD's share of workgroups of its own.  A step
 // of rec_bwd_kernel is bound by the fetch of dG_{t+1}: a workgroup owns 32 columns of the product and pulls all 4 Hp gate columns of its 16 rows
 // through the CU's one vector-memory path (128 KiB at 1024 units, 128 loads, 1 us), and the 32 workgroups of an XCD the same lines through
 // one L2.  Fewer rows per group fetch less only if the fragments stay full: an A-fragment has 16 rows whatever the batch has.  Here a
