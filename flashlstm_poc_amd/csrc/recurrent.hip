@@ -4018,7 +4018,10 @@ static int few_rows_fwd(int B, int Hp, int num_cus, bool many_steps) {
 // Rows per block of rec_bwd_few_kernel, likewise.  Blocks of 4 where all of them run side by side, else of 8 (us a step, 8 / 4 rows:
 // 1024 units and 32 rows 1.71 / 1.43, 650 and 20 rows 1.49 / 1.33, 257 and 70 rows 1.11 / 1.06, 64 and 16 rows 0.90 / 0.84); but a batch of
 // at most four rows is one block either way, and up to 512 units the shorter sum over the lanes counts (256 units and one row
-// 0.80 / 0.90, 64 and four 0.74 / 0.79; 640 and four 1.34 / 1.26).
+// 0.80 / 0.90, 64 and four 0.74 / 0.79; 640 and four 1.34 / 1.26).  (Five to eight rows of 32 units: a training step of 200 steps 369 with blocks
+// of 4, 361 of 8, of 1000 steps 1411 and 1460.)  A launch begins 1 to 2 us later than with blocks of 16 rows, for the zeroed k-steps and the cells'
+// operands behind the weights: 5 steps of 128 rows of 32 units are a training step of 114 us instead of 112, and from 10 steps on the steps
+// make up for it but for 32 units.
 static int few_rows_bwd(int B, int Hp, int num_cus) {
     if (Hp > 1024 || num_cus != 256) return 0;
     const int side_by_side = 8 * (32 / (Hp / 32));
